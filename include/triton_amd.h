@@ -169,6 +169,18 @@ int tamd_routing(const void *logits, int dtype, int64_t stride, int n_rows, int 
                  void *stream);
 
 /*
+ * tamd_routing that also leaves the softmax values in expert-sorted order: sorted_vals[i] (the type of y_vals, which is
+ * the type of the logits) is the value of the flat (token, slot) entry col_sorted_indx[i] -- the per-row factors of
+ * the down projection (gammas, tests/test_distributed.py:201-208), written where the entry is placed instead of by
+ * an indexing pass afterwards.  sorted_vals may be null.
+ */
+int tamd_routing_gates(const void *logits, int dtype, int64_t stride, int n_rows, int n_cols, int k, void *y_vals,
+                       int16_t *y_indx, uint32_t *bits, int64_t bits_stride_row, int64_t bits_stride_word, int32_t *col_sum,
+                       int32_t *col_sorted_indx, int32_t *row_sorted_indx, int32_t *gather_indx, void *sorted_vals,
+                       int32_t *offs, int64_t offs_pitch, int32_t *schedule, int64_t sched_pitch, int max_n_blocks,
+                       int32_t *workspace, void *stream);
+
+/*
  * tamd_routing_metadata for callers that cannot allocate (code under HIP graph capture, serving loops and
  * harnesses that forbid hipMalloc).  No counterpart in the reference, where every workspace is a torch allocation
  * made per call.  Same arguments and results as tamd_routing_metadata without `workspace`: the intermediate

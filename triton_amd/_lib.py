@@ -124,6 +124,8 @@ _SIGNATURES = {
                                       _INT, _PTR], C.c_int),
     "tamd_routing": ([_PTR, _INT, _I64, _INT, _INT, _INT, _PTR, _PTR, _PTR, _I64, _I64, _PTR, _PTR, _PTR, _PTR, _PTR,
                       _I64, _PTR, _I64, _INT, _PTR, _PTR], C.c_int),
+    "tamd_routing_gates": ([_PTR, _INT, _I64, _INT, _INT, _INT, _PTR, _PTR, _PTR, _I64, _I64, _PTR, _PTR, _PTR, _PTR, _PTR,
+                            _PTR, _I64, _PTR, _I64, _INT, _PTR, _PTR], C.c_int),
     "tamd_matmul": ([C.POINTER(MatmulArgs), _PTR], C.c_int),
     "tamd_reduce": ([_PTR, _INT, _I64, _I64, _I64, _I64, _I64, _I64, _PTR, _I64, _I64, _I64, _PTR, _I64, _I64, _I64,
                      _PTR, _INT, _I64, _I64, _PTR], C.c_int),

@@ -73,12 +73,14 @@ TAMD_DEVICE float group_max_f32(float v) {
 
 // L lanes cooperate on one row; EPL > 0 keeps ceil(n_cols/L) <= EPL keys in registers.  `row` is the row of this
 // thread's group of L lanes (any row >= n_rows: a group that only takes part in the shuffles); lds_indx, when given,
-// also receives the picked columns ([row][k] ints) for a kernel that goes on to use them.
+// also receives the picked columns ([row][k] ints) for a kernel that goes on to use them, and lds_gate the bits of the
+// stored values.
 template <int DT, int L, int EPL>
 TAMD_DEVICE void topk_row(const void *__restrict__ x, int64_t x_stride, int n_rows, int n_cols, int k,
                           int apply_softmax, int use_provided, void *__restrict__ y_vals,
                           int16_t *__restrict__ y_indx, int64_t y_stride, uint32_t *__restrict__ bits,
-                          int64_t bits_stride_row, int64_t bits_stride_word, int64_t row, int32_t *lds_indx) {
+                          int64_t bits_stride_row, int64_t bits_stride_word, int64_t row, int32_t *lds_indx,
+                          uint32_t *lds_gate = nullptr) {
   const int sub = threadIdx.x % L;
   const bool live = row < n_rows;
   const int64_t rrow = live ? row : 0;
@@ -145,6 +147,7 @@ TAMD_DEVICE void topk_row(const void *__restrict__ x, int64_t x_stride, int n_ro
     store_from_f32<DT>(y_vals, rrow * y_stride + sub, v);
     if (!use_provided) y_indx[rrow * y_stride + sub] = (int16_t)my_idx;
     if (lds_indx) lds_indx[rrow * k + sub] = my_idx;
+    if (lds_gate) lds_gate[rrow * k + sub] = DT == TAMD_F32 ? f32_to_bits(v) : DT == TAMD_BF16 ? f32_to_bf16_bits(v) : f32_to_f16_bits(v);
   }
   const int n_words = (n_cols + 31) / 32;
   const int base_lane = (threadIdx.x % kWave) - sub;
@@ -200,6 +203,24 @@ int launch_topk(const void *x, int64_t xs, int n_rows, int n_cols, int k, int sm
 
 TAMD_DEVICE int load_indx(const void *p, int is16, int64_t i) {
   return is16 ? (int)((const int16_t *)p)[i] : ((const int32_t *)p)[i];
+}
+
+// Gate weights in expert-sorted order (what the down projection takes as its per-row factors): entry i of the flat
+// (token, slot) array goes to the place its index goes to.  Bits are moved as they are; `esz` is 4 or 2, 0 when no
+// sorted copy is asked for.
+struct Gates {
+  const void *vals;
+  void *sorted;
+  int esz;
+};
+TAMD_DEVICE uint32_t load_gate(const Gates &g, int64_t i) {
+  if (g.esz == 4) return ((const uint32_t *)g.vals)[i];
+  if (g.esz == 2) return ((const uint16_t *)g.vals)[i];
+  return 0;
+}
+TAMD_DEVICE void store_gate(const Gates &g, int64_t pos, uint32_t bits) {
+  if (g.esz == 4) ((uint32_t *)g.sorted)[pos] = bits;
+  else if (g.esz == 2) ((uint16_t *)g.sorted)[pos] = (uint16_t)bits;
 }
 
 TAMD_DEVICE uint64_t same_id_mask(int e, bool valid, int nbits) {
@@ -325,7 +346,7 @@ __global__ __launch_bounds__(1024) void order_kernel(const void *__restrict__ in
                                                     const int32_t *__restrict__ col_offs,
                                                     const int32_t *__restrict__ n_valid,
                                                     int32_t *__restrict__ col_sorted, int32_t *__restrict__ row_sorted,
-                                                    int32_t *__restrict__ gather) {
+                                                    int32_t *__restrict__ gather, Gates gates) {
   const int blk = blockIdx.x;
   const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
   const int nv = *n_valid;
@@ -341,6 +362,7 @@ __global__ __launch_bounds__(1024) void order_kernel(const void *__restrict__ in
       row_sorted[i] = pos;
       col_sorted[pos] = (int32_t)i;
       if (gather) gather[pos] = (int32_t)(i / k);
+      store_gate(gates, pos, load_gate(gates, i));
     } else if (i < n) {
       row_sorted[i] = -1;
     }
@@ -379,7 +401,7 @@ inline MetaPlan make_meta_plan(int64_t n_indx, int E) {
 }
 
 inline int launch_bitmatrix_metadata(const void *indx, int is16, int64_t n, int E, int k, int32_t *col_sum,
-                                     int32_t *col_sorted, int32_t *row_sorted, int32_t *gather, int32_t *ws,
+                                     int32_t *col_sorted, int32_t *row_sorted, int32_t *gather, Gates gates, int32_t *ws,
                                      hipStream_t st, bool before_order(void *), void *ctx) {
   MetaPlan p = make_meta_plan(n, E);
   size_t lds = (size_t)p.CH * E * 4;
@@ -390,7 +412,7 @@ inline int launch_bitmatrix_metadata(const void *indx, int is16, int64_t n, int 
   if (before_order && !before_order(ctx)) return launch_status();
   order_kernel<<<dim3((unsigned)p.n_blocks), 1024, 0, st>>>(indx, is16, n, E, p.CH, p.nbits, k, ws + p.off_chunk_pref,
                                                           ws + p.off_block_tot, ws + p.off_col_offs,
-                                                          ws + p.off_n_valid, col_sorted, row_sorted, gather);
+                                                          ws + p.off_n_valid, col_sorted, row_sorted, gather, gates);
   return launch_status();
 }
 
@@ -536,7 +558,7 @@ __global__ __launch_bounds__(1024) void order_scan_kernel(const void *__restrict
                                                           int32_t *__restrict__ col_sorted, int32_t *__restrict__ row_sorted,
                                                           int32_t *__restrict__ gather, int32_t *__restrict__ offs,
                                                           int64_t offs_pitch, int32_t *__restrict__ sched,
-                                                          int64_t sched_pitch, int max_blocks) {
+                                                          int64_t sched_pitch, int max_blocks, Gates gates) {
   extern __shared__ int32_t sm[];
   int32_t *hist = sm;                          // [CH][E]  counts of this block's chunks, then their exclusive prefix
   int32_t *tot = hist + (int64_t)CH * E;       // [E]      entries per expert
@@ -551,7 +573,11 @@ __global__ __launch_bounds__(1024) void order_scan_kernel(const void *__restrict
   const int i = (blk * CH + wave) * 64 + lane;
   const bool has = orders && wave < CH && i < n;
   int ev = 0;
-  if (n > 0) ev = load_indx(indx, is16, has ? i : 0);
+  uint32_t gate = 0;
+  if (n > 0) {
+    ev = load_indx(indx, is16, has ? i : 0);
+    gate = load_gate(gates, has ? i : 0);
+  }
   if (orders)
     for (int j = tid; j < CH * E; j += 1024) hist[j] = 0;
   // 1. partial sums of the table: thread (part, e) takes the blocks [part * per, (part + 1) * per)
@@ -566,7 +592,7 @@ __global__ __launch_bounds__(1024) void order_scan_kernel(const void *__restrict
       pbel[part * E + e] = below;
     }
   }
-  asm volatile("" : "+v"(ev));
+  asm volatile("" : "+v"(ev), "+v"(gate));
   ev = has ? ev : -1;
   __syncthreads();
   // 2. totals per expert; counts of this wave's chunk
@@ -605,6 +631,7 @@ __global__ __launch_bounds__(1024) void order_scan_kernel(const void *__restrict
       row_sorted[i] = pos;
       col_sorted[pos] = i;
       if (gather) gather[pos] = i / k;
+      store_gate(gates, pos, gate);
     } else if (wave < CH && i < n) {
       row_sorted[i] = -1;
     }
@@ -634,7 +661,7 @@ inline bool order_scan_applicable(int64_t n, int E, int CH, int64_t nb) {
 inline int launch_order_scan(const void *indx, int is16, int64_t n, int E, int CH, int nbits, int k, const int32_t *block_tot,
                              int64_t nb, int32_t *col_sum, int32_t *col_sorted, int32_t *row_sorted, int32_t *gather,
                              int32_t *offs, int64_t offs_pitch, int32_t *sched, int64_t sched_pitch, int max_blocks,
-                             hipStream_t st) {
+                             Gates gates, hipStream_t st) {
   int P = 1024 / E;
   P = P > 16 ? 16 : P;
   P = P > nb ? (int)nb : P;
@@ -644,7 +671,7 @@ inline int launch_order_scan(const void *indx, int is16, int64_t n, int E, int C
   if (int rc = raise_lds_limit_once((const void *)order_scan_kernel)) return rc;
   order_scan_kernel<<<dim3((unsigned)(nb + shares)), 1024, (size_t)ints * 4, st>>>(
       indx, is16, (int)n, E, CH, nbits, k, block_tot, (int)nb, P, col_sum, col_sorted, row_sorted, gather, offs, offs_pitch,
-      sched, sched_pitch, max_blocks);
+      sched, sched_pitch, max_blocks, gates);
   return launch_status();
 }
 
@@ -703,11 +730,12 @@ int launch_topk_hist(const void *x, int64_t xs, int n_rows, int E, int k, void *
 // the three prefix sums, the ordering and the ragged tables without leaving the workgroup --
 // one launch instead of four, which is what the cost of routing is made of at these sizes.
 // lidx: the index array in LDS (a kernel that has just computed it), or null to read `indx` from memory.
-TAMD_DEVICE void meta_fused_body(int32_t *sm, bool zeroed, const int32_t *lidx, const void *__restrict__ indx, int is16,
+// lgate: the gate weights' bits in LDS beside it, or null likewise.
+TAMD_DEVICE void meta_fused_body(int32_t *sm, bool zeroed, const int32_t *lidx, const uint32_t *lgate, const void *__restrict__ indx, int is16,
                                  int n, int E, int k, int nbits, int NC, int P, int32_t *__restrict__ col_sum,
                                  int32_t *__restrict__ col_sorted, int32_t *__restrict__ row_sorted,
                                  int32_t *__restrict__ gather, int32_t *__restrict__ offs, int64_t offs_pitch,
-                                 int32_t *__restrict__ sched, int64_t sched_pitch, int max_blocks) {
+                                 int32_t *__restrict__ sched, int64_t sched_pitch, int max_blocks, Gates gates) {
   int32_t *hist = sm;                         // [NC][E]  counts, then exclusive prefix over chunks
   int32_t *csum = hist + (int64_t)NC * E;     // [E]
   int32_t *psum = csum + E;                   // [P][E]   partial sums of chunk ranges
@@ -816,6 +844,7 @@ TAMD_DEVICE void meta_fused_body(int32_t *sm, bool zeroed, const int32_t *lidx, 
         row_sorted[i] = pos;
         col_sorted[pos] = i;
         if (gather) gather[pos] = i / k;
+        store_gate(gates, pos, lgate ? lgate[i] : load_gate(gates, i));
       } else if (i < n) {
         row_sorted[i] = -1;
       }
@@ -834,10 +863,10 @@ __global__ __launch_bounds__(1024) void meta_fused_kernel(const void *__restrict
                                                           int32_t *__restrict__ col_sorted, int32_t *__restrict__ row_sorted,
                                                           int32_t *__restrict__ gather, int32_t *__restrict__ offs,
                                                           int64_t offs_pitch, int32_t *__restrict__ sched,
-                                                          int64_t sched_pitch, int max_blocks) {
+                                                          int64_t sched_pitch, int max_blocks, Gates gates) {
   extern __shared__ int32_t sm[];
-  meta_fused_body(sm, false, nullptr, indx, is16, n, E, k, nbits, NC, P, col_sum, col_sorted, row_sorted, gather, offs,
-                  offs_pitch, sched, sched_pitch, max_blocks);
+  meta_fused_body(sm, false, nullptr, nullptr, indx, is16, n, E, k, nbits, NC, P, col_sum, col_sorted, row_sorted, gather, offs,
+                  offs_pitch, sched, sched_pitch, max_blocks, gates);
 }
 
 // ---------------------------------------------------------------------------
@@ -856,26 +885,27 @@ __global__ __launch_bounds__(1024) void routing_fused_kernel(const void *__restr
                                                              int32_t *__restrict__ row_sorted, int32_t *__restrict__ gather,
                                                              int32_t *__restrict__ offs, int64_t offs_pitch,
                                                              int32_t *__restrict__ sched, int64_t sched_pitch,
-                                                             int max_blocks) {
+                                                             int max_blocks, Gates gates) {
   extern __shared__ int32_t sm[];
-  const int n = n_rows * k;
+  const int n = n_rows * k, n4 = (n + 3) / 4 * 4;
   int32_t *lidx = sm;                        // [n] picked columns
-  int32_t *meta = sm + (n + 3) / 4 * 4;
+  uint32_t *lgate = (uint32_t *)sm + n4;     // [n] gate weights
+  int32_t *meta = sm + 2 * n4;
   constexpr int ROWS = 1024 / L;
   for (int i = threadIdx.x; i < NC * E; i += 1024) meta[i] = 0;  // the histograms (the barrier below covers them)
   for (int row0 = 0; row0 < n_rows; row0 += ROWS)
     topk_row<DT, L, EPL>(x, x_stride, n_rows, E, k, 1, 0, y_vals, y_indx, k, bits, bits_stride_row, bits_stride_word,
-                         (int64_t)row0 + threadIdx.x / L, lidx);
+                         (int64_t)row0 + threadIdx.x / L, lidx, lgate);
   __syncthreads();
-  meta_fused_body(meta, true, lidx, nullptr, 0, n, E, k, nbits, NC, P, col_sum, col_sorted, row_sorted, gather, offs,
-                  offs_pitch, sched, sched_pitch, max_blocks);
+  meta_fused_body(meta, true, lidx, lgate, nullptr, 0, n, E, k, nbits, NC, P, col_sum, col_sorted, row_sorted, gather, offs,
+                  offs_pitch, sched, sched_pitch, max_blocks, gates);
 }
 
 template <int DT>
 int launch_routing_fused(const void *x, int64_t xs, int n_rows, int E, int k, void *yv, int16_t *yi, uint32_t *bits,
                          int64_t bsr, int64_t bsw, int nbits, int NC, int P, size_t lds, int32_t *col_sum,
                          int32_t *col_sorted, int32_t *row_sorted, int32_t *gather, int32_t *offs, int64_t offs_pitch,
-                         int32_t *sched, int64_t sched_pitch, int max_blocks, hipStream_t st) {
+                         int32_t *sched, int64_t sched_pitch, int max_blocks, Gates gates, hipStream_t st) {
   int need = (E + 7) / 8;
   if (need < k) need = k;
 #define TAMD_RF(LL, EE)                                                                                              \
@@ -883,7 +913,7 @@ int launch_routing_fused(const void *x, int64_t xs, int n_rows, int E, int k, vo
     auto kern = routing_fused_kernel<DT, LL, EE>;                                                                    \
     if (int rc = raise_lds_limit_once((const void *)kern)) return rc;                                                \
     kern<<<1, 1024, lds, st>>>(x, xs, n_rows, E, k, yv, yi, bits, bsr, bsw, nbits, NC, P, col_sum, col_sorted,        \
-                               row_sorted, gather, offs, offs_pitch, sched, sched_pitch, max_blocks);                \
+                               row_sorted, gather, offs, offs_pitch, sched, sched_pitch, max_blocks, gates);         \
   } while (0)
   if (need <= 8) TAMD_RF(8, 8);
   else if (need <= 16) TAMD_RF(16, 8);
@@ -931,7 +961,7 @@ extern "C" int tamd_bitmatrix_metadata(const void *indx, int indx_is_int16, int6
   if (n_indx < 0 || n_cols <= 0 || n_cols > 16384 || n_indx > 0x7FFFFFFF) return TAMD_E_INVALID;
   if (!col_sum || !workspace || (n_indx > 0 && (!indx || !col_sorted_indx || !row_sorted_indx))) return TAMD_E_INVALID;
   return launch_bitmatrix_metadata(indx, indx_is_int16, n_indx, n_cols, 1, col_sum, col_sorted_indx, row_sorted_indx,
-                                   nullptr, workspace, (hipStream_t)stream, nullptr, nullptr);
+                                   nullptr, Gates{nullptr, nullptr, 0}, workspace, (hipStream_t)stream, nullptr, nullptr);
 }
 
 static int ragged_launch(const int32_t *slice_sizes, int n_slices, int32_t *offs, int64_t offs_pitch,
@@ -977,7 +1007,7 @@ bool ragged_between(void *p) {
 static int routing_metadata_impl(const void *indx, int indx_is_int16, int64_t n_indx, int n_cols, int k,
                                  int32_t *col_sum, int32_t *col_sorted_indx, int32_t *row_sorted_indx,
                                  int32_t *gather_indx, int32_t *offs, int64_t offs_pitch, int32_t *schedule,
-                                 int64_t sched_pitch, int max_n_blocks, int32_t *workspace, void *stream) {
+                                 int64_t sched_pitch, int max_n_blocks, int32_t *workspace, Gates gates, void *stream) {
   if (n_indx < 0 || n_cols <= 0 || n_cols > 16384 || n_indx > 0x7FFFFFFF || k < 1) return TAMD_E_INVALID;
   if (max_n_blocks < 0 || offs_pitch < n_cols + 1 || sched_pitch < max_n_blocks) return TAMD_E_INVALID;
   if (!col_sum || !workspace || !offs || (max_n_blocks > 0 && !schedule)) return TAMD_E_INVALID;
@@ -994,7 +1024,7 @@ static int routing_metadata_impl(const void *indx, int indx_is_int16, int64_t n_
       if (int rc = raise_lds_limit_once((const void *)meta_fused_kernel)) return rc;
       meta_fused_kernel<<<1, 1024, (size_t)ints * 4, (hipStream_t)stream>>>(
           indx, indx_is_int16, (int)n_indx, n_cols, k, nbits, (int)NC, (int)P, col_sum, col_sorted_indx, row_sorted_indx,
-          gather_indx, offs, offs_pitch, schedule, sched_pitch, max_n_blocks);
+          gather_indx, offs, offs_pitch, schedule, sched_pitch, max_n_blocks, gates);
       return launch_status();
     }
   }
@@ -1007,7 +1037,7 @@ static int routing_metadata_impl(const void *indx, int indx_is_int16, int64_t n_
           indx, indx_is_int16, n_indx, n_cols, p.CH, p.nbits, nullptr, workspace + p.off_block_tot);
       return launch_order_scan(indx, indx_is_int16, n_indx, n_cols, p.CH, p.nbits, k, workspace + p.off_block_tot, p.n_blocks,
                                col_sum, col_sorted_indx, row_sorted_indx, gather_indx, offs, offs_pitch, schedule, sched_pitch,
-                               max_n_blocks, st);
+                               max_n_blocks, gates, st);
     }
   }
   const size_t sr_lds = ((size_t)n_cols + 6 * ((size_t)n_cols + 1) + 17) * 4;
@@ -1025,12 +1055,12 @@ static int routing_metadata_impl(const void *indx, int indx_is_int16, int64_t n_
         workspace + p.off_col_offs, workspace + p.off_n_valid, offs, offs_pitch, schedule, sched_pitch, max_n_blocks);
     order_kernel<<<dim3((unsigned)p.n_blocks), 1024, 0, st>>>(
         indx, indx_is_int16, n_indx, n_cols, p.CH, p.nbits, k, workspace + p.off_chunk_pref, workspace + p.off_block_off,
-        workspace + p.off_col_offs, workspace + p.off_n_valid, col_sorted_indx, row_sorted_indx, gather_indx);
+        workspace + p.off_col_offs, workspace + p.off_n_valid, col_sorted_indx, row_sorted_indx, gather_indx, gates);
     return launch_status();
   }
   RaggedCtx ctx{col_sum, n_cols, offs, offs_pitch, schedule, sched_pitch, max_n_blocks, (hipStream_t)stream};
   return launch_bitmatrix_metadata(indx, indx_is_int16, n_indx, n_cols, k, col_sum, col_sorted_indx,
-                                   row_sorted_indx, gather_indx, workspace, (hipStream_t)stream, ragged_between, &ctx);
+                                   row_sorted_indx, gather_indx, gates, workspace, (hipStream_t)stream, ragged_between, &ctx);
 }
 
 extern "C" int tamd_routing_metadata(const void *indx, int indx_is_int16, int64_t n_indx, int n_cols, int k,
@@ -1038,7 +1068,8 @@ extern "C" int tamd_routing_metadata(const void *indx, int indx_is_int16, int64_
                                      int32_t *gather_indx, int32_t *offs, int64_t offs_pitch, int32_t *schedule,
                                      int64_t sched_pitch, int max_n_blocks, int32_t *workspace, void *stream) {
   return routing_metadata_impl(indx, indx_is_int16, n_indx, n_cols, k, col_sum, col_sorted_indx, row_sorted_indx,
-                               gather_indx, offs, offs_pitch, schedule, sched_pitch, max_n_blocks, workspace, stream);
+                               gather_indx, offs, offs_pitch, schedule, sched_pitch, max_n_blocks, workspace,
+                               Gates{nullptr, nullptr, 0}, stream);
 }
 
 extern "C" int tamd_routing(const void *logits, int dtype, int64_t stride, int n_rows, int n_cols, int k, void *y_vals,
@@ -1046,6 +1077,17 @@ extern "C" int tamd_routing(const void *logits, int dtype, int64_t stride, int n
                             int32_t *col_sum, int32_t *col_sorted_indx, int32_t *row_sorted_indx, int32_t *gather_indx,
                             int32_t *offs, int64_t offs_pitch, int32_t *schedule, int64_t sched_pitch, int max_n_blocks,
                             int32_t *workspace, void *stream) {
+  return tamd_routing_gates(logits, dtype, stride, n_rows, n_cols, k, y_vals, y_indx, bits, bits_stride_row, bits_stride_word,
+                            col_sum, col_sorted_indx, row_sorted_indx, gather_indx, nullptr, offs, offs_pitch, schedule,
+                            sched_pitch, max_n_blocks, workspace, stream);
+}
+
+extern "C" int tamd_routing_gates(const void *logits, int dtype, int64_t stride, int n_rows, int n_cols, int k, void *y_vals,
+                                  int16_t *y_indx, uint32_t *bits, int64_t bits_stride_row, int64_t bits_stride_word,
+                                  int32_t *col_sum, int32_t *col_sorted_indx, int32_t *row_sorted_indx, int32_t *gather_indx,
+                                  void *sorted_vals, int32_t *offs, int64_t offs_pitch, int32_t *schedule,
+                                  int64_t sched_pitch, int max_n_blocks, int32_t *workspace, void *stream) {
+  const Gates gates{y_vals, sorted_vals, sorted_vals ? dtype_size(dtype) : 0};
   // a few rows (at most two passes of the workgroup's 1024 threads over them), at most 512 columns, and the
   // metadata workspace of one workgroup fits LDS: one launch for everything
   if (n_rows > 0 && n_cols > 0 && n_cols <= 512 && k >= 1 && k <= 64 && k <= n_cols && logits && y_vals && y_indx && bits &&
@@ -1059,7 +1101,7 @@ extern "C" int tamd_routing(const void *logits, int dtype, int64_t stride, int n
     const int64_t NC = (n + 63) / 64;
     int64_t P = 1024 / n_cols;
     P = P < 1 ? 1 : (P > NC ? NC : P);
-    const int64_t ints = (n + 3) / 4 * 4 + NC * n_cols + (int64_t)n_cols + P * n_cols + 6 * (int64_t)(n_cols + 1);
+    const int64_t ints = 2 * ((n + 3) / 4 * 4) + NC * n_cols + (int64_t)n_cols + P * n_cols + 6 * (int64_t)(n_cols + 1);
     if (n_rows <= 2 * (1024 / L) && NC <= 64 && ints * 4 <= 156 * 1024) {
       int nbits = 0;
       while ((1 << nbits) < n_cols) ++nbits;
@@ -1067,7 +1109,7 @@ extern "C" int tamd_routing(const void *logits, int dtype, int64_t stride, int n
 #define TAMD_RFD(DT)                                                                                                  \
   return launch_routing_fused<DT>(logits, stride, n_rows, n_cols, k, y_vals, y_indx, bits, bits_stride_row,            \
                                   bits_stride_word, nbits, (int)NC, (int)P, (size_t)ints * 4, col_sum, col_sorted_indx,  \
-                                  row_sorted_indx, gather_indx, offs, offs_pitch, schedule, sched_pitch, max_n_blocks, st)
+                                  row_sorted_indx, gather_indx, offs, offs_pitch, schedule, sched_pitch, max_n_blocks, gates, st)
       if (dtype == TAMD_F32) TAMD_RFD(TAMD_F32);
       if (dtype == TAMD_BF16) TAMD_RFD(TAMD_BF16);
       TAMD_RFD(TAMD_F16);
@@ -1094,14 +1136,14 @@ extern "C" int tamd_routing(const void *logits, int dtype, int64_t stride, int n
                                         bits_stride_word, nbits, L, CH, workspace, st);
       if (rc != 0) return rc;
       return launch_order_scan(y_indx, 1, n, n_cols, CH, nbits, k, workspace, nb, col_sum, col_sorted_indx, row_sorted_indx,
-                               gather_indx, offs, offs_pitch, schedule, sched_pitch, max_n_blocks, st);
+                               gather_indx, offs, offs_pitch, schedule, sched_pitch, max_n_blocks, gates, st);
     }
   }
   const int rc = tamd_topk_forward(logits, dtype, stride, n_rows, n_cols, k, 1, 0, y_vals, y_indx, k, bits, bits_stride_row,
                                    bits_stride_word, stream);
   if (rc != 0) return rc;
   return routing_metadata_impl(y_indx, 1, (int64_t)n_rows * k, n_cols, k, col_sum, col_sorted_indx, row_sorted_indx,
-                               gather_indx, offs, offs_pitch, schedule, sched_pitch, max_n_blocks, workspace, stream);
+                               gather_indx, offs, offs_pitch, schedule, sched_pitch, max_n_blocks, workspace, gates, stream);
 }
 
 // Device address of `scratch` on the current device.  In host code the array's name only stands for the symbol: its
@@ -1151,5 +1193,6 @@ extern "C" int tamd_routing_metadata_static(const void *indx, int indx_is_int16,
   // every entry of the workspace that a launch reads is written earlier by the same call (per-chunk prefixes and
   // per-workgroup totals by the histogram kernel, the prefix tables by the scan kernel): nothing has to start at zero
   return routing_metadata_impl(indx, indx_is_int16, n_indx, n_cols, k, col_sum, col_sorted_indx, row_sorted_indx,
-                               gather_indx, offs, offs_pitch, schedule, sched_pitch, max_n_blocks, ws, stream);
+                               gather_indx, offs, offs_pitch, schedule, sched_pitch, max_n_blocks, ws,
+                               Gates{nullptr, nullptr, 0}, stream);
 }
