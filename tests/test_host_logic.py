@@ -205,3 +205,15 @@ def test_turned_gate_weights_are_cached_per_tensor_and_version():
     del w
     gc.collect()
     assert key not in mm._TURNED
+
+
+def test_native_tile_choice_follows_make_opt_flags():
+    """The native host path chooses row blocks by the rule of make_opt_flags (no constraints set)."""
+    from triton_amd import _native
+    OF.reset_opt_flags_constraints()
+    for m in (1, 15, 16, 17, 64, 65, 255, 256, 1000, 4097, 65536):
+        for slices in (1, 7, 32, 128):
+            for ragged, expected in ((False, None), (True, None), (True, 1), (True, 9), (True, 40), (True, 1000)):
+                for fp8 in (False, True):
+                    want = OF.make_opt_flags(m, 64, 64, slices, ragged, expected, fp8).block_m
+                    assert _native.choose_block_m(m, slices, ragged, -1 if expected is None else expected, fp8) == want

@@ -11,6 +11,7 @@ from concurrent.futures import ThreadPoolExecutor
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libtriton_amd.so")
+HOST = os.path.join(HERE, "_host.so")  # the native host path (csrc/host.cpp), a CPython extension
 SOURCES = ["api.cpp", "mxfp.hip", "routing.hip", "elementwise.hip", "moe_matmul.hip", "moe_matmul_bf16.hip", "moe_matmul_f16.hip",
            "moe_matmul_fp8.hip", "moe_matmul_bf16_swiglu.hip", "moe_matmul_f16_swiglu.hip", "moe_matmul_fp8_swiglu.hip",
            "moe_matmul_fp8e5m2.hip", "moe_matmul_fp8e5m2_swiglu.hip", "moe_matmul_stream_fp8e5m2.hip",
@@ -83,6 +84,22 @@ def _compile(src, obj):
         raise RuntimeError(f"{src}: kernels using scratch memory: " + ", ".join(f"{n} ({b} B/lane)" for n, b in spilled))
 
 
+def _build_host():
+    """The CPython extension: host code only, against torch's headers and libraries."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths
+    libs = os.path.join(os.path.dirname(torch.__file__), "lib")
+    inc = [f for p in (*include_paths("cuda"), sysconfig.get_paths()["include"]) for f in ("-isystem", p)]
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *inc, os.path.join(CSRC, "host.cpp"), "-o", HOST,
+           f"-L{libs}", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"g++ failed for host.cpp:\n{res.stdout}\n{res.stderr}")
+
+
 def build(force=True, verbose=False):
     """Compiles every source and links the shared library. Returns its path."""
     objdir = os.path.join(HERE, "build")
@@ -96,15 +113,19 @@ def build(force=True, verbose=False):
         newest = max(os.path.getmtime(p) for p in [os.path.join(CSRC, s), *deps])
         if force or not os.path.exists(o) or os.path.getmtime(o) < newest:
             todo.append((s, o))
+    host_src = [os.path.join(CSRC, "host.cpp"), os.path.join(HERE, "..", "include", "triton_amd.h")]
+    host = force or not os.path.exists(HOST) or os.path.getmtime(HOST) < max(map(os.path.getmtime, host_src))
     with ThreadPoolExecutor(max_workers=min(8, max(1, len(todo)))) as ex:
-        list(ex.map(lambda so: _compile(*so), todo))
+        jobs = [ex.submit(_compile, s, o) for s, o in todo] + ([ex.submit(_build_host)] if host else [])
+        for job in jobs:
+            job.result()
     if todo or not os.path.exists(LIB):
         cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB, *objs]
         res = subprocess.run(cmd, capture_output=True, text=True)
         if res.returncode != 0:
             raise RuntimeError(f"link failed:\n{res.stdout}\n{res.stderr}")
     if verbose:
-        print(f"built {LIB} ({len(todo)} objects recompiled)")
+        print(f"built {LIB} ({len(todo)} objects recompiled){' and ' + HOST if host else ''}")
     return LIB
 
 

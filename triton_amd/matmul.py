@@ -10,7 +10,7 @@ from typing import Callable, Optional
 
 import torch
 
-from . import _lib
+from . import _lib, _native
 from .matmul_details import opt_flags as _opt_flags
 from .matmul_details.opt_flags import (InapplicableConstraint, OptFlags, make_opt_flags, scoped_opt_flags,
                                        scoped_opt_flags_constraints)
@@ -128,6 +128,13 @@ def matmul(a, b, bias, a_ragged_metadata: Optional[RaggedTensorMetadata] = None,
     a_ragged_metadata: rows of `a` (after gather) are grouped by slice.
     gather_indx / scatter_indx: int32 row maps (scatter -1 drops the row).
     """
+    if type(a) is torch.Tensor and a.is_cuda and b_ragged_metadata is None and fused_comm is None and c_acc_in is None:
+        done = _native.matmul(a, b, bias, a_ragged_metadata, gather_indx, scatter_indx, precision_config, betas, gammas,
+                              out_alpha, c, fused_activation, epilogue)
+        if done is not None:
+            if type(done) is int:
+                _lib.check(done, "matmul")
+            return done
     if precision_config is None:
         precision_config = _DEFAULT_PRECISION
     if fused_activation is None:

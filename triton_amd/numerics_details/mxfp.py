@@ -4,7 +4,7 @@ from enum import Enum
 
 import torch
 
-from .. import _lib
+from .. import _lib, _native
 from ..tensor import FP4, Tensor, empty, torch_dtype_to_dtype, wrap_torch_tensor
 from ..tensor_details.dtype import UINT8
 from ..tensor_details.layout import StridedLayout
@@ -50,6 +50,13 @@ def downcast_to_mxfp(x, out_dtype, axis: int, scale_dtype: torch.dtype = torch.u
     """Quantises `x` along `axis` in groups of 32: returns (values, scales) as torch
     tensors whose storage is contiguous along `axis`; FP4 values pack two codes per
     byte along it (even index in the low nibble)."""
+    if type(x) is torch.Tensor and x.is_cuda and scale_dtype is torch.uint8 and microblock_size == MXFP_BLOCK_SIZE \
+            and type(out_dtype) is torch.dtype:
+        done = _native.downcast(x, out_dtype, axis, DEQUANT_SCALE_ROUNDING_MODE.value)
+        if done is not None:
+            if type(done) is int:
+                _lib.check(done, "downcast_to_mxfp")
+            return done
     if isinstance(x, Tensor):
         x = x.storage.data
     assert scale_dtype == torch.uint8 or scale_dtype == torch.float8_e4m3fn, f"Invalid scale dtype {scale_dtype=}"
@@ -101,6 +108,12 @@ def downcast_to_mxfp(x, out_dtype, axis: int, scale_dtype: torch.dtype = torch.u
 def upcast_from_mxfp(tensor: torch.Tensor, scale: torch.Tensor, target_dtype: torch.dtype, axis: int,
                      tensor_scale=None):
     """Inverse of downcast_to_mxfp; the result is contiguous in the logical axis order."""
+    if tensor_scale is None and type(tensor) is torch.Tensor and tensor.is_cuda and type(target_dtype) is torch.dtype:
+        done = _native.upcast(tensor, scale, target_dtype, axis)
+        if done is not None:
+            if type(done) is int:
+                _lib.check(done, "upcast_from_mxfp")
+            return done
     ndim = tensor.ndim
     assert -ndim <= axis < ndim, f"Invalid axis {axis=}"
     axis = axis % ndim

@@ -7,11 +7,14 @@ from typing import Optional
 
 import torch
 
-from . import _lib
+from . import _lib, _native
 from .numerics import InFlexData, OutFlexData
 from .specialize import FnSpecs
 
 MXFP_BLOCK_SIZE = 32
+
+
+_NO_IN, _NO_OUT = InFlexData(), OutFlexData()
 
 
 @dataclass(frozen=True)
@@ -66,9 +69,9 @@ def _postprocess_code(fn: Optional[PostprocessFn]):
 
 
 def reduce(x: torch.Tensor, dim: int, mask: Optional[torch.Tensor] = None, scale: Optional[torch.Tensor] = None,
-           x_mxscale: Optional[torch.Tensor] = None, x_flex: Optional[InFlexData] = InFlexData(),
+           x_mxscale: Optional[torch.Tensor] = None, x_flex: Optional[InFlexData] = _NO_IN,
            x_global_scale: Optional[torch.Tensor] = None, y: Optional[torch.Tensor] = None,
-           y_dtype: Optional[torch.dtype] = None, y_flex: Optional[OutFlexData] = OutFlexData(),
+           y_dtype: Optional[torch.dtype] = None, y_flex: Optional[OutFlexData] = _NO_OUT,
            y_flex_saturate_inf: bool = False, y_has_mx: Optional[bool] = None, y_mx_scale_dtype=None,
            y_microblock_size: int = MXFP_BLOCK_SIZE, y_value_pack_factor: int = 1,
            postprocess_fn1: Optional[PostprocessFn] = None, postprocess_fn2: Optional[PostprocessFn] = None,
@@ -76,6 +79,15 @@ def reduce(x: torch.Tensor, dim: int, mask: Optional[torch.Tensor] = None, scale
     """Returns (y, y_mxscale).  y = postprocess(sum over `dim` of where(mask, x * scale, 0)), accumulated in float32 in
     index order; then the output's flexpoint scales or its MXFP8 quantisation along the last axis (when the input is
     microscaled, as in the reference, reduce.py:1185-1206); cast to y_dtype (default x.dtype)."""
+    if (mask is None and scale is None and y is None and y_dtype is None and x_mxscale is None and x_flex is _NO_IN
+            and y_flex is _NO_OUT and x_global_scale is None and postprocess_fn1 is None and postprocess_fn2 is None
+            and not y_has_mx and unpadded_batch_size is None and y_microblock_size == MXFP_BLOCK_SIZE
+            and y_value_pack_factor == 1 and x.is_cuda):
+        done = _native.reduce(x, dim)  # the top-k combine of 16-bit rows
+        if done is not None:
+            if type(done) is int:
+                _lib.check(done, "reduce")
+            return done, None
     if unpadded_batch_size is not None:
         # a device-side count of the rows of the first kept axis that hold data (reduce.py:694-695, 550-555): the rest
         # of y is left as it is.  Read by the kernel, never on the host.
