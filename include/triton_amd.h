@@ -296,6 +296,9 @@ typedef struct tamd_matmul_args {
    * K and N padded with zero codes; in a block, column 2c + f of the strip is position 32 f + c (64 bytes), its
    * 16-byte part p in slot p ^ ((c >> 2) & 3) ^ 2 f.  Only w_stride_e is used (bytes); w 16-byte aligned. */
   int w_layout;
+  /* rows of y (of one batch entry) that dst(r) can name; with a span y_rows * y_stride_m below 2 GB the results are
+   * stored through 32-bit offsets.  0: unknown, the general (slower) stores are used. */
+  int64_t y_rows;
 } tamd_matmul_args;
 
 int tamd_matmul(const tamd_matmul_args *args, void *stream);

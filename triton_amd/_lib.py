@@ -55,7 +55,7 @@ class MatmulArgs(C.Structure):
         ("w_mx_layout", C.c_int),
         ("x_mx_scale", C.c_void_p), ("x_mx_stride_m", C.c_int64), ("x_mx_stride_z", C.c_int64),
         ("y_mx_scale", C.c_void_p), ("y_mx_stride_m", C.c_int64), ("y_mx_stride_z", C.c_int64),
-        ("w_layout", C.c_int),
+        ("w_layout", C.c_int), ("y_rows", C.c_int64),
     ]
 
 

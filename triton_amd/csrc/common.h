@@ -36,18 +36,18 @@ TAMD_DEVICE uint32_t f32_to_f16_bits(float f) {
 // largest finite code when `saturate`, NaN otherwise (what a plain cast does); NaN stays NaN.
 TAMD_DEVICE uint32_t f32_to_e4m3_bits(float f, bool saturate) {
   const uint32_t u = f32_to_bits(f), sign = (u >> 24) & 0x80u, mag = u & 0x7FFFFFFFu;
-  if (mag > 0x7F800000u) return sign | 0x7Fu;
-  if (mag >= 0x43E80000u) return sign | (saturate ? 0x7Eu : 0x7Fu);  // 464.0f
-  return (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(f, f, 0, false) & 0xFFu;
+  const uint32_t in_range = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(f, f, 0, false) & 0xFFu;
+  const uint32_t beyond = sign | (saturate && mag <= 0x7F800000u ? 0x7Eu : 0x7Fu);
+  return mag >= 0x43E80000u ? beyond : in_range;  // 464.0f (selections: no branch per value)
 }
 
 // float32 -> OCP e5m2 byte, round to nearest even.  Magnitudes that round beyond 57344 (>= 61440) give infinity
 // (or the largest finite code when saturating); NaN stays NaN.
 TAMD_DEVICE uint32_t f32_to_e5m2_bits(float f, bool saturate) {
   const uint32_t u = f32_to_bits(f), sign = (u >> 24) & 0x80u, mag = u & 0x7FFFFFFFu;
-  if (mag > 0x7F800000u) return sign | 0x7Fu;
-  if (mag >= 0x47700000u) return sign | (saturate ? 0x7Bu : 0x7Cu);  // 61440.0f
-  return (uint32_t)__builtin_amdgcn_cvt_pk_bf8_f32(f, f, 0, false) & 0xFFu;
+  const uint32_t in_range = (uint32_t)__builtin_amdgcn_cvt_pk_bf8_f32(f, f, 0, false) & 0xFFu;
+  const uint32_t beyond = sign | (mag > 0x7F800000u ? 0x7Fu : (saturate ? 0x7Bu : 0x7Cu));
+  return mag >= 0x47700000u ? beyond : in_range;  // 61440.0f
 }
 TAMD_DEVICE uint32_t f32_to_fp8_bits(float f, int dt) {
   return dt == TAMD_FP8_E5M2 ? f32_to_e5m2_bits(f, false) : f32_to_e4m3_bits(f, false);

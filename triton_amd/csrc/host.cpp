@@ -448,6 +448,7 @@ PyObject *py_matmul(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
     g.x_stride_m = a.stride(0);
     g.x_rows = a_rows;
     g.y = out.data_ptr();
+    g.y_rows = rows_out;
     g.M = (int)M, g.N = (int)N, g.K = (int)K, g.n_experts = (int)n_slices;
     g.gather_indx = gather ? (const int32_t *)gather->data_ptr() : nullptr;
     g.scatter_indx = scatter ? (const int32_t *)scatter->data_ptr() : nullptr;

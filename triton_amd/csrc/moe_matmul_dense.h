@@ -146,7 +146,8 @@ TAMD_DEVICE void run_tile_w16(const tamd_matmul_args &a, const Tile &t, uint8_t 
     rd = rd == 2 ? 0 : rd + 1;
   }
   wait_dma();
-  tile_epilogue<NFR, ACT, XDT, false>(a, t, acc, lds);
+  __syncthreads();  // every wave is done with the stages: the epilogue's tables go there
+  tile_epilogue<NFR, ACT, XDT, false>(a, t, acc, lds + wave * 4096);
 }
 
 template <int XDT, int BM, int ACT, bool WKC>
@@ -170,7 +171,6 @@ int launch_w16(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
   constexpr int LDS_ROWS = 32 * MF;
   constexpr int PIPE = 3 * LDS_ROWS * A_ROW_BYTES + 3 * W16_STAGE;
   static_assert(PIPE <= 160 * 1024, "one workgroup per CU");
-  constexpr int OUT_BYTES = LDS_ROWS * 256 * 2;
   const int grid_n = (a.N + BLOCK_N - 1) / BLOCK_N;
   const int64_t total = (int64_t)grid_m * grid_n;
   if (total <= 0) return 0;
@@ -178,7 +178,7 @@ int launch_w16(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
   if (launch > 0x7FFFFFFF) return TAMD_E_UNSUPPORTED;
   auto kern = mm_x16_w16_kernel<XDT, BM, ACT, WKC>;
   if (int rc = raise_lds_limit_once((const void *)kern)) return rc;
-  kern<<<dim3((unsigned)launch), 256, PIPE > OUT_BYTES ? PIPE : OUT_BYTES, st>>>(a, grid_n, total);
+  kern<<<dim3((unsigned)launch), 256, PIPE, st>>>(a, grid_n, total);
   return launch_status();
 }
 

@@ -36,6 +36,7 @@ typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef int i32x8_t __attribute__((ext_vector_type(8)));
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
 
 constexpr bool is_fp8(int dt) { return dt == TAMD_FP8_E4M3 || dt == TAMD_FP8_E5M2; }
 
@@ -424,127 +425,147 @@ static_assert(ring_outstanding(4, 2, 1, 4, false) == 6 && ring_outstanding(4, 2,
 static_assert(ring_outstanding(3, 2, 2, 4, false) == 6 && ring_outstanding(3, 2, 2, 4, true) == 6, "ring bookkeeping");
 static_assert(ring_outstanding(3, 1, 1, 4, false) == 1 && ring_outstanding(3, 1, 1, 4, true) == 5, "ring bookkeeping");
 
+// Flexpoint actual scale: the wave's max|result| by one atomic; positive floats order like their bit patterns.
+TAMD_DEVICE void store_actual_scale(float *actual, uint32_t amax, float out_max, int lane) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    const uint32_t other = (uint32_t)__shfl_xor((int)amax, o);
+    amax = other > amax ? other : amax;
+  }
+  if (lane == 0) {
+    amax = amax < 0x7F800000u ? amax : 0x7F800000u;  // NaN counts as +inf
+    atomicMax((unsigned int *)actual, f32_to_bits(__builtin_fmaf(bits_to_f32(amax), 1.0f / out_max, 1.0e-30f)));
+  }
+}
+
 // Epilogue of one output tile (shared by every tiled kernel).  The accumulators hold, for fragment
 // (i, f), element j: row 32i + 8(j/4) + 4h + j%4, column t.n0 + wave*64 + c32*NF + f.
 //
-// YDT: output type fixed at compile time, or -1 to read a.y_dtype; ROWSC: per-row betas / gammas may be
-// present; FLEX: flexpoint output (expected / actual scale) may be present; MXO: MXFP8 output (a.y_mx_scale).
-// Everything that is false or fixed here is a branch less per output element, and a tile has up to
-// 160 x 256 of them.  The element loops must unroll completely (the accumulators are indexed by them and
-// would otherwise live in scratch memory), and the compiler gives up on that above a body size that one
-// variant holding every feature exceeds: hence MXO and FLEX exclude each other.
+// A wave finishes its 64 columns by itself: the destination of each of the tile's rows (a byte offset into y; out of
+// range for a row that is not stored) and the rows' factors go into a table of the wave's own in LDS, from which four
+// consecutive rows are read at a time by a broadcast; every element is then computed and stored from registers, a row's
+// 32 lanes writing 32 consecutive outputs (one half or whole line of a 16-bit type).  Nothing is masked by control flow:
+// a store whose offset is out of range is dropped by the buffer descriptor.  There is no barrier either, so waves
+// leave the tile one by one.  (Staging the tile through LDS for 16-byte stores, as before, took a fifth to a
+// quarter of a tile's time: two barriers, a pass of narrow LDS writes and a copy-out between them.)
+//
+// YDT: output type; ROWSC: per-row betas / gammas may be present; FLEX: flexpoint output (expected / actual scale) may be
+// present; MXO: MXFP8 output (a.y_mx_scale).  The element loops must unroll completely (the accumulators are indexed by
+// them and would otherwise live in scratch memory).
 // Args: tamd_matmul_args, or the same structure read in place from the kernel-argument segment (see kernel_args_late).
+// tab: LDS that belongs to the wave alone, epilogue_table_bytes(NFR).
+constexpr int epilogue_table_bytes(int nfr) { return nfr * 32 * 12; }
+
 template <int NFR, int ACT, int YDT, bool ROWSC, bool FLEX, bool MXO = false, typename Args = tamd_matmul_args>
-TAMD_DEVICE void tile_epilogue_t(const Args &a, const Tile &t, f32x16_t (&acc)[NFR][NF], uint8_t *lds) {
-  const int tid = threadIdx.x;
-  const int wave = tid / kWave, lane = tid % kWave;
+TAMD_DEVICE void tile_epilogue_t(const Args &a, const Tile &t, f32x16_t (&acc)[NFR][NF], uint8_t *tab) {
+  const int wave = (threadIdx.x / kWave) & 3, lane = threadIdx.x % kWave;
   const int c32 = lane % 32, h = lane / 32;
   const int N = a.N;
   const int col0 = t.n0 + wave * 64 + c32 * NF;
-  const int ydt = YDT < 0 ? a.y_dtype : YDT;
-  // 16-bit and 8-bit outputs are staged through LDS (the K stages are dead by now) so that the global
-  // stores are 16 bytes per lane and whole rows of the tile are contiguous.
+  constexpr uint32_t kDrop = 0x80000000u;                   // an offset that no descriptor here covers
+  constexpr int ydt = YDT;
+  constexpr int NO = ACT == TAMD_ACT_SWIGLU ? NF / 2 : NF;  // outputs per lane per row
+  const int n_out = ACT == TAMD_ACT_SWIGLU ? N / 2 : N;
+  const int out_col0 = ACT == TAMD_ACT_SWIGLU ? col0 / 2 : col0;
+  static_assert(YDT != TAMD_F32, "float32 results take the general epilogue");
+  constexpr int osz = is_fp8(YDT) ? 1 : 2;                  // bytes per output
+  if (t.n0 + wave * 64 >= N) return;
+  // ---- the wave's row table: [rows] destinations, [rows] betas, [rows] gammas
+  uint32_t *tab_dst = (uint32_t *)tab;
+  float *tab_beta = (float *)tab + NFR * 32, *tab_gamma = (float *)tab + NFR * 64;
+#pragma unroll
+  for (int u = 0; u < (NFR + 1) / 2; ++u) {
+    const int r = u * kWave + lane;
+    if (NFR % 2 == 0 || r < NFR * 32) {
+      const int erow = t.start_m + t.off_m + (r < t.rows ? r : t.rows - 1);  // expert-sorted row
+      const int dst = a.scatter_indx ? a.scatter_indx[erow] : erow;
+      float beta = 1.0f, gamma = 1.0f;
+      if constexpr (ROWSC) {
+        if (a.betas) beta = a.betas[erow];
+        if (a.gammas) gamma = a.gammas[erow];
+      }
+      const bool keep = r < t.rows && dst >= 0;
+      if constexpr (MXO) tab_dst[r] = keep ? (uint32_t)dst : kDrop;
+      else tab_dst[r] = keep ? (uint32_t)dst * (uint32_t)(a.y_stride_m * osz) : kDrop;
+      if constexpr (ROWSC) {
+        tab_beta[r] = beta;
+        tab_gamma[r] = gamma;
+      }
+    }
+  }
   float flex = 1.0f;
   if (a.x_scale) flex *= *a.x_scale;
   if (a.w_scale) flex *= *a.w_scale;
   flex *= a.out_alpha;
-  float bias[NF];
+  // without per-row factors bias * beta * out_alpha is one value per column
+  float bias_a[NF];
 #pragma unroll
   for (int f = 0; f < NF; ++f)
-    bias[f] = (a.bias && col0 + f < N) ? load_any_f32(a.bias, a.bias_dtype, (int64_t)t.expert * a.bias_stride_e + col0 + f)
-                                       : 0.f;
-  constexpr int NO = ACT == TAMD_ACT_SWIGLU ? NF / 2 : NF;  // outputs per lane per row
-  constexpr int OUT_COLS = 128 * NO;                        // output columns of the tile
-  const int n_out = ACT == TAMD_ACT_SWIGLU ? N / 2 : N;
-  const int out_col0 = ACT == TAMD_ACT_SWIGLU ? col0 / 2 : col0;
-  const int tile_out0 = ACT == TAMD_ACT_SWIGLU ? t.n0 / 2 : t.n0;
+    bias_a[f] = ((a.bias && col0 + f < N) ? load_any_f32(a.bias, a.bias_dtype, (int64_t)t.expert * a.bias_stride_e + col0 + f)
+                                          : 0.f) * a.out_alpha;
   const bool has_limit = a.act_has_limit != 0;
-  const int osz = ydt == TAMD_F32 ? 4 : (is_fp8(ydt) ? 1 : 2);  // bytes per output
-  const bool staged = osz < 4;
   // flexpoint output: scale by 1 / expected, optionally clamp, and track max|result| for the actual scale
   const float inv_expected = (FLEX && a.y_expected_scale) ? 1.0f / *a.y_expected_scale : 1.0f;
   const bool clamp_out = FLEX && a.y_expected_scale != nullptr && a.y_saturate_inf != 0;
   const float out_max = max_finite_of(ydt);
   const bool track_max = FLEX && a.y_actual_scale != nullptr;
+  const uint32_t track_mask = track_max ? 0x7FFFFFFFu : 0u;
   uint32_t amax = 0;
   auto narrow = [&](float v) -> uint32_t {  // one output value as 8 / 16 bits
     return ydt == TAMD_BF16 ? f32_to_bf16_bits(v) : (ydt == TAMD_F16 ? f32_to_f16_bits(v) : f32_to_fp8_bits(v, ydt));
   };
   auto narrow2 = [&](float lo, float hi) -> uint32_t {  // two 16-bit outputs in one word (one packed conversion)
-    typedef float f32x2_t __attribute__((ext_vector_type(2)));
     if (ydt == TAMD_BF16) return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{lo, hi}, bf16x2_t));
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{lo, hi}, f16x2_t));
   };
-  // without per-row factors bias * beta * out_alpha is one value per column
-  float bias_a[NF];
-#pragma unroll
-  for (int f = 0; f < NF; ++f) bias_a[f] = bias[f] * a.out_alpha;
-  uint8_t *ob = lds;  // [rows][OUT_COLS] outputs of osz bytes
-  // per-row factors: lane L fetches those of row L % 32 of every fragment up front (one round trip to memory);
-  // an element then takes its row's pair from that lane
-  float beta_of[NFR], gamma_of[NFR];
-  const bool has_beta = ROWSC && a.betas != nullptr, has_gamma = ROWSC && a.gammas != nullptr;
+  const __amdgpu_buffer_rsrc_t ry = __builtin_amdgcn_make_buffer_rsrc((uint8_t *)a.y + (int64_t)t.z * a.y_stride_z * osz, 0,
+                                                                     0x7FFFFFFF, 0x00020000);
+  const uint32_t col_off = (uint32_t)out_col0 * (uint32_t)osz, col_kill = out_col0 < n_out ? 0u : kDrop;
+  const __amdgpu_buffer_rsrc_t rsc = __builtin_amdgcn_make_buffer_rsrc(
+      MXO ? a.y_mx_scale + (int64_t)t.z * a.y_mx_stride_z : nullptr, 0, MXO ? 0x7FFFFFFF : 0, 0x00020000);
+  // one lane per row and group of 32 outputs stores the group's scale
+  const uint32_t sc_kill = ((c32 & (32 / NO - 1)) == 0 && out_col0 < n_out) ? 0u : kDrop;
+  // four rows of the table at a time, read one step ahead; the scheduling barrier keeps the compiler from reading the
+  // whole table up front (registers)
+  uint4 next_dst = *(const uint4 *)(tab_dst + h * 4);
+  f32x4_t next_beta = f32x4_t{1.f, 1.f, 1.f, 1.f}, next_gamma = next_beta;
   if constexpr (ROWSC) {
-#pragma unroll
-    for (int i = 0; i < NFR; ++i) {
-      const int r = i * 32 + c32;
-      const int erow = t.start_m + t.off_m + (r < t.rows ? r : t.rows - 1);  // expert-sorted row
-      beta_of[i] = has_beta ? a.betas[erow] : 1.0f;
-      gamma_of[i] = has_gamma ? a.gammas[erow] : 1.0f;
-    }
+    next_beta = *(const f32x4_t *)(tab_beta + h * 4);
+    next_gamma = *(const f32x4_t *)(tab_gamma + h * 4);
   }
-  // destination rows of the 16-byte chunks this thread copies out at the end (chunk id = tid + 256 u): fetched
-  // now, so that the scatter indices arrive while the values are computed
-  constexpr bool PRE = YDT >= 0 && YDT != TAMD_F32;
-  constexpr int OSZ_C = YDT == TAMD_FP8_E4M3 || YDT == TAMD_FP8_E5M2 ? 1 : 2;
-  constexpr int CPR_C = OUT_COLS * OSZ_C / 16;          // chunks per tile row
-  constexpr int MAXU = PRE ? NFR * 32 * CPR_C / 256 : 1;  // chunks per thread
-  int dst_row[MAXU];
-  if constexpr (PRE) {
-#pragma unroll
-    for (int u = 0; u < MAXU; ++u) {
-      const int r = (tid + u * 256) / CPR_C;
-      const int erow = t.start_m + t.off_m + (r < t.rows ? r : t.rows - 1);
-      dst_row[u] = a.scatter_indx ? a.scatter_indx[erow] : erow;
-    }
-  }
-  __syncthreads();
 #pragma unroll
   for (int i = 0; i < NFR; ++i) {
 #pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      const int r = i * 32 + (j >> 2) * 8 + h * 4 + (j & 3);
-      float v[NF];
-      float gamma = 1.0f;
-      if constexpr (ROWSC) {
-        // the factors of row 32 i + l sit in lane l: lanes of half h need l = 8 (j / 4) + 4 h + j % 4
-        const int l0 = (j >> 2) * 8 + (j & 3);
-        // (an absent factor was loaded as 1.0: no branch inside the element loop)
-        const float b0 = bits_to_f32(__builtin_amdgcn_readlane((int)f32_to_bits(beta_of[i]), l0));
-        const float b1 = bits_to_f32(__builtin_amdgcn_readlane((int)f32_to_bits(beta_of[i]), l0 + 4));
-        const float beta = h ? b1 : b0;
-        const float g0 = bits_to_f32(__builtin_amdgcn_readlane((int)f32_to_bits(gamma_of[i]), l0));
-        const float g1 = bits_to_f32(__builtin_amdgcn_readlane((int)f32_to_bits(gamma_of[i]), l0 + 4));
-        gamma = h ? g1 : g0;
-#pragma unroll
-        for (int f = 0; f < NF; ++f) v[f] = __builtin_fmaf(acc[i][f][j], flex, bias_a[f] * beta);
-      } else {
-#pragma unroll
-        for (int f = 0; f < NF; ++f) v[f] = __builtin_fmaf(acc[i][f][j], flex, bias_a[f]);
+    for (int jq = 0; jq < 4; ++jq) {
+      const uint32_t dst4[4] = {next_dst.x, next_dst.y, next_dst.z, next_dst.w};
+      const f32x4_t beta4 = next_beta, gamma4 = next_gamma;
+      if (i * 4 + jq + 1 < NFR * 4) {
+        const int r1 = (i * 4 + jq + 1) * 8 + h * 4;
+        next_dst = *(const uint4 *)(tab_dst + r1);
+        if constexpr (ROWSC) {
+          next_beta = *(const f32x4_t *)(tab_beta + r1);
+          next_gamma = *(const f32x4_t *)(tab_gamma + r1);
+        }
       }
-      float o[NO];
-      if constexpr (ACT == TAMD_ACT_SWIGLU) {
-        o[0] = swiglu_fast(v[0], v[1], a.act_alpha, a.act_limit, has_limit);
-      } else {
 #pragma unroll
-        for (int p = 0; p < NO; ++p) o[p] = v[p];
-      }
-      if constexpr (ROWSC) {
+      for (int jj = 0; jj < 4; ++jj) {
+        const int j = jq * 4 + jj;
+        float v[NF];
 #pragma unroll
-        for (int p = 0; p < NO; ++p) o[p] *= gamma;
-      }
-      if constexpr (MXO) {
-        {
+        for (int f = 0; f < NF; ++f) v[f] = __builtin_fmaf(acc[i][f][j], flex, ROWSC ? bias_a[f] * beta4[jj] : bias_a[f]);
+        float o[NO];
+        if constexpr (ACT == TAMD_ACT_SWIGLU) {
+          o[0] = swiglu_fast(v[0], v[1], a.act_alpha, a.act_limit, has_limit);
+        } else {
+#pragma unroll
+          for (int p = 0; p < NO; ++p) o[p] = v[p];
+        }
+        if constexpr (ROWSC) {
+#pragma unroll
+          for (int p = 0; p < NO; ++p) o[p] *= gamma4[jj];
+        }
+        const uint32_t dst = dst4[jj];
+        if constexpr (MXO) {
           // MXFP8 output: a group is 32 consecutive output columns of a row = the outputs of one half wave (of
           // half of it when a lane holds two columns).  max |o| over the group, scale = 2^ceil(log2(max / 448)),
           // o / scale clamped to +-448; the cast below rounds to nearest even (as tamd_downcast_mxfp does).
@@ -561,167 +582,164 @@ TAMD_DEVICE void tile_epilogue_t(const Args &a, const Tile &t, f32x16_t (&acc)[N
             const float q = o[p] * qs;
             o[p] = q != q ? q : __builtin_fminf(__builtin_fmaxf(q, -448.0f), 448.0f);
           }
-          // one lane per group leaves the scale byte behind the staged tile; the copy-out below places it
-          if ((c32 & (32 / NO - 1)) == 0) ob[NFR * 32 * OUT_COLS + r * (OUT_COLS / 32) + wave * NO + c32 * NO / 32] = (uint8_t)(sb >> 23);
+          __builtin_amdgcn_raw_buffer_store_b8((uint8_t)(sb >> 23), rsc,
+                                               (int)((dst & kDrop) | sc_kill | (dst * (uint32_t)a.y_mx_stride_m + out_col0 / 32)), 0, 0);
         }
-      }
-      if constexpr (FLEX) {
-        if (track_max && r < t.rows) {
+        if constexpr (FLEX) {
+          // (selections, no branches: a branch per element breaks the fragment into hundreds of blocks)
+          const uint32_t amask = (dst | col_kill) & kDrop ? 0u : track_mask;
 #pragma unroll
-          for (int p = 0; p < NO; ++p)
-            if (out_col0 + p < n_out) amax = absmax_bits(amax, o[p]);
+          for (int p = 0; p < NO; ++p) {
+            const uint32_t b = f32_to_bits(o[p]) & amask;
+            amax = b > amax ? b : amax;
+            o[p] *= inv_expected;
+            const float oc = __builtin_fminf(__builtin_fmaxf(o[p], -out_max), out_max);
+            o[p] = clamp_out ? oc : o[p];
+          }
         }
-#pragma unroll
-        for (int p = 0; p < NO; ++p) {
-          o[p] *= inv_expected;
-          if (clamp_out) o[p] = __builtin_fminf(__builtin_fmaxf(o[p], -out_max), out_max);
-        }
-      }
-      if (staged) {
-        uint8_t *dstl = ob + (r * OUT_COLS + wave * 32 * NO + c32 * NO) * osz;
-        if (osz == 2) {
-          if constexpr (NO == 2) *(uint32_t *)dstl = narrow2(o[0], o[NO - 1]);
-          else *(uint16_t *)dstl = (uint16_t)narrow(o[0]);
+        const int off = MXO ? (int)((dst & kDrop) | col_kill | (dst * (uint32_t)a.y_stride_m + col_off)) : (int)((dst + col_off) | col_kill);
+        if constexpr (osz == 2) {
+          if constexpr (NO == 2) __builtin_amdgcn_raw_buffer_store_b32(narrow2(o[0], o[NO - 1]), ry, off, 0, 0);
+          else __builtin_amdgcn_raw_buffer_store_b16((uint16_t)narrow(o[0]), ry, off, 0, 0);
         } else {
-          if constexpr (NO == 2) *(uint16_t *)dstl = (uint16_t)(narrow(o[0]) | (narrow(o[NO - 1]) << 8));
-          else *dstl = (uint8_t)narrow(o[0]);
-        }
-      } else if (r < t.rows) {
-        int64_t dst = t.start_m + t.off_m + r;
-        if (a.scatter_indx) dst = a.scatter_indx[dst];
-        if (dst >= 0) {
-          const int64_t base = (int64_t)t.z * a.y_stride_z + dst * a.y_stride_m;
-#pragma unroll
-          for (int p = 0; p < NO; ++p)
-            if (out_col0 + p < n_out) ((float *)a.y)[base + out_col0 + p] = o[p];
+          if constexpr (NO == 2)
+            __builtin_amdgcn_raw_buffer_store_b16((uint16_t)(narrow(o[0]) | (narrow(o[NO - 1]) << 8)), ry, off, 0, 0);
+          else __builtin_amdgcn_raw_buffer_store_b8((uint8_t)narrow(o[0]), ry, off, 0, 0);
         }
       }
+      // (the running maximum is taken here and not after the last row, with every result kept until then)
+      if constexpr (FLEX) asm volatile("" : "+v"(amax));
+      __builtin_amdgcn_sched_barrier(0);
     }
   }
   if constexpr (FLEX) {
-    if (track_max) {
-      // wave maximum, then one atomic per wave; positive floats order like their bit patterns
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) {
-        const uint32_t other = (uint32_t)__shfl_xor((int)amax, o);
-        amax = other > amax ? other : amax;
-      }
-      if (lane == 0) {
-        amax = amax < 0x7F800000u ? amax : 0x7F800000u;  // NaN counts as +inf
-        const float sc = __builtin_fmaf(bits_to_f32(amax), 1.0f / out_max, 1.0e-30f);
-        atomicMax((unsigned int *)a.y_actual_scale, f32_to_bits(sc));
-      }
-    }
-  }
-  if (staged) {
-    __syncthreads();
-    if constexpr (MXO) {
-      // scale bytes of the tile: OUT_COLS / 32 per row, to the row's (possibly scattered) place
-      constexpr int GPR = OUT_COLS / 32;
-      for (int id = tid; id < t.rows * GPR; id += 256) {
-        const int r = id / GPR, g = id - r * GPR;
-        const int gcol = tile_out0 + g * 32;
-        if (gcol >= n_out) continue;
-        int64_t dst = t.start_m + t.off_m + r;
-        if (a.scatter_indx) dst = a.scatter_indx[dst];
-        if (dst >= 0) a.y_mx_scale[(int64_t)t.z * a.y_mx_stride_z + dst * a.y_mx_stride_m + gcol / 32] = ob[NFR * 32 * OUT_COLS + id];
-      }
-    }
-    const int epc = 16 / osz;                 // outputs per 16-byte chunk
-    const int cpr = OUT_COLS / epc;           // chunks per tile row
-    const int n_chunks = t.rows * cpr;
-    if constexpr (PRE) {
-      // Usual case -- every chunk of the tile lies wholly inside or wholly outside the output's columns and lands on a
-      // 16-byte boundary: the staged chunks are read first, then each is stored under one predicate and no other
-      // control flow (the general loop below compiles to a state machine per chunk that takes several times longer).
-      constexpr int EPC_C = 16 / OSZ_C;
-      const bool whole_chunks =
-          n_out % EPC_C == 0 &&
-          ((((uintptr_t)a.y) | (uintptr_t)(a.y_stride_m * OSZ_C) | (uintptr_t)(a.y_stride_z * OSZ_C)) & 15) == 0;
-      if (whole_chunks) {
-        uint4 staged_chunk[MAXU];
-#pragma unroll
-        for (int u = 0; u < MAXU; ++u) staged_chunk[u] = *(const uint4 *)(ob + (size_t)(tid + u * 256) * 16);
-#pragma unroll
-        for (int u = 0; u < MAXU; ++u) {
-          const int id = tid + u * 256;
-          const int r = id / CPR_C, c = (id - r * CPR_C) * EPC_C;
-          const int gcol = tile_out0 + c;
-          if (id < n_chunks && dst_row[u] >= 0 && gcol < n_out) {
-            uint8_t *yp = (uint8_t *)a.y + ((int64_t)t.z * a.y_stride_z + (int64_t)dst_row[u] * a.y_stride_m + gcol) * OSZ_C;
-            *(uint4 *)yp = staged_chunk[u];
-          }
-        }
-        return;
-      }
-#pragma unroll
-      for (int u = 0; u < MAXU; ++u) {
-        const int id = tid + u * 256;
-        if (id >= n_chunks) break;
-        const int r = id / CPR_C, c = (id - r * CPR_C) * (16 / OSZ_C);
-        const int64_t dst = dst_row[u];
-        if (dst < 0) continue;
-        const int gcol = tile_out0 + c;
-        if (gcol >= n_out) continue;
-        uint8_t *yp = (uint8_t *)a.y + ((int64_t)t.z * a.y_stride_z + dst * a.y_stride_m + gcol) * OSZ_C;
-        const uint8_t *sp = ob + (r * OUT_COLS + c) * OSZ_C;
-        if (gcol + 16 / OSZ_C <= n_out && ((uintptr_t)yp & 15) == 0) {
-          *(uint4 *)yp = *(const uint4 *)sp;
-        } else {
-          const int n_b = (n_out - gcol < 16 / OSZ_C ? n_out - gcol : 16 / OSZ_C) * OSZ_C;
-          for (int e = 0; e < n_b; ++e) yp[e] = sp[e];
-        }
-      }
-      return;
-    }
-    // eight chunks per thread at a time, so that the scatter indices of a batch are fetched together
-    for (int id0 = tid; id0 < n_chunks; id0 += 256 * 8) {
-      int64_t dsts[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int id = id0 + u * 256;
-        const int r = id / cpr;
-        dsts[u] = t.start_m + t.off_m + (r < t.rows ? r : t.rows - 1);
-        if (a.scatter_indx) dsts[u] = a.scatter_indx[dsts[u]];
-      }
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int id = id0 + u * 256;
-        if (id >= n_chunks) break;
-        const int r = id / cpr, c = (id - r * cpr) * epc;
-        const int64_t dst = dsts[u];
-        if (dst < 0) continue;
-        const int gcol = tile_out0 + c;
-        if (gcol >= n_out) continue;
-        uint8_t *yp = (uint8_t *)a.y + ((int64_t)t.z * a.y_stride_z + dst * a.y_stride_m + gcol) * osz;
-        const uint8_t *sp = ob + (r * OUT_COLS + c) * osz;
-        if (gcol + epc <= n_out && ((uintptr_t)yp & 15) == 0) {
-          *(uint4 *)yp = *(const uint4 *)sp;
-        } else {
-          const int n_b = (n_out - gcol < epc ? n_out - gcol : epc) * osz;
-          for (int e = 0; e < n_b; ++e) yp[e] = sp[e];
-        }
-      }
-    }
+    if (track_max) store_actual_scale(a.y_actual_scale, amax, out_max, lane);
   }
 }
 
+// The general epilogue: any output type, alignment and size, every feature read at run time, stores through 64-bit
+// addresses.  A row fragment's accumulators are taken four at a time in a rolled loop and move up by four after each
+// step, so that the loop indexes registers with constants.
+template <int NFR, int ACT, typename Args>
+TAMD_DEVICE void tile_epilogue_general(const Args &a, const Tile &t, f32x16_t (&acc)[NFR][NF], uint8_t *tab) {
+  const int wave = (threadIdx.x / kWave) & 3, lane = threadIdx.x % kWave;
+  const int c32 = lane % 32, h = lane / 32;
+  const int N = a.N;
+  const int col0 = t.n0 + wave * 64 + c32 * NF;
+  constexpr int NO = ACT == TAMD_ACT_SWIGLU ? NF / 2 : NF;
+  const int n_out = ACT == TAMD_ACT_SWIGLU ? N / 2 : N;
+  const int out_col0 = ACT == TAMD_ACT_SWIGLU ? col0 / 2 : col0;
+  if (t.n0 + wave * 64 >= N) return;
+  int32_t *tab_dst = (int32_t *)tab;
+  float *tab_beta = (float *)tab + NFR * 32, *tab_gamma = (float *)tab + NFR * 64;
+  for (int r = lane; r < NFR * 32; r += kWave) {
+    const int erow = t.start_m + t.off_m + (r < t.rows ? r : t.rows - 1);
+    const int dst = a.scatter_indx ? a.scatter_indx[erow] : erow;
+    tab_dst[r] = r < t.rows ? dst : -1;
+    tab_beta[r] = a.betas ? a.betas[erow] : 1.0f;
+    tab_gamma[r] = a.gammas ? a.gammas[erow] : 1.0f;
+  }
+  float flex = 1.0f;
+  if (a.x_scale) flex *= *a.x_scale;
+  if (a.w_scale) flex *= *a.w_scale;
+  flex *= a.out_alpha;
+  float bias_a[NF];
+#pragma unroll
+  for (int f = 0; f < NF; ++f)
+    bias_a[f] = ((a.bias && col0 + f < N) ? load_any_f32(a.bias, a.bias_dtype, (int64_t)t.expert * a.bias_stride_e + col0 + f)
+                                          : 0.f) * a.out_alpha;
+  const bool has_limit = a.act_has_limit != 0;
+  const int ydt = a.y_dtype;
+  const float inv_expected = a.y_expected_scale ? 1.0f / *a.y_expected_scale : 1.0f;
+  const bool clamp_out = a.y_expected_scale != nullptr && a.y_saturate_inf != 0;
+  const float out_max = max_finite_of(ydt);
+  uint32_t amax = 0;
+#pragma unroll
+  for (int i = 0; i < NFR; ++i)
+#pragma unroll 1
+  for (int q = 0; q < 4; ++q) {
+    const int r0 = i * 32 + q * 8 + h * 4;
+#pragma unroll
+    for (int jj = 0; jj < 4; ++jj) {
+      const int dst = tab_dst[r0 + jj];
+      const float beta = tab_beta[r0 + jj], gamma = tab_gamma[r0 + jj];
+      float v[NF], o[NO];
+#pragma unroll
+      for (int f = 0; f < NF; ++f) v[f] = __builtin_fmaf(acc[i][f][jj], flex, bias_a[f] * beta);
+      if constexpr (ACT == TAMD_ACT_SWIGLU) {
+        o[0] = swiglu_fast(v[0], v[1], a.act_alpha, a.act_limit, has_limit);
+      } else {
+#pragma unroll
+        for (int p = 0; p < NO; ++p) o[p] = v[p];
+      }
+#pragma unroll
+      for (int p = 0; p < NO; ++p) o[p] *= gamma;
+      if (a.y_mx_scale) {  // MXFP8 output, as in tile_epilogue_t
+        float m = 0.f;
+#pragma unroll
+        for (int p = 0; p < NO; ++p) m = __builtin_fmaxf(m, out_col0 + p < n_out ? __builtin_fabsf(o[p]) : 0.f);
+        for (int sh = 16 / NO; sh > 0; sh >>= 1) m = __builtin_fmaxf(m, __shfl_xor(m, sh));
+        const uint32_t sb = (f32_to_bits(m / 448.0f) + 0x007FFFFFu) & 0x7F800000u;
+        const float ds = bits_to_f32(sb);
+        const float qs = ds == 0.f ? 0.f : 1.0f / ds;
+#pragma unroll
+        for (int p = 0; p < NO; ++p) {
+          const float w = o[p] * qs;
+          o[p] = w != w ? w : __builtin_fminf(__builtin_fmaxf(w, -448.0f), 448.0f);
+        }
+        if (dst >= 0 && (c32 & (32 / NO - 1)) == 0 && out_col0 < n_out)
+          a.y_mx_scale[(int64_t)t.z * a.y_mx_stride_z + (int64_t)dst * a.y_mx_stride_m + out_col0 / 32] = (uint8_t)(sb >> 23);
+      }
+      if (dst >= 0) {
+        const int64_t at = (int64_t)t.z * a.y_stride_z + (int64_t)dst * a.y_stride_m + out_col0;
+#pragma unroll
+        for (int p = 0; p < NO; ++p) {
+          if (out_col0 + p < n_out) {
+            if (a.y_actual_scale) amax = absmax_bits(amax, o[p]);
+            float w = o[p] * inv_expected;
+            if (clamp_out) w = __builtin_fminf(__builtin_fmaxf(w, -out_max), out_max);
+            if (ydt == TAMD_F32) ((float *)a.y)[at + p] = w;
+            else if (ydt == TAMD_BF16) ((uint16_t *)a.y)[at + p] = (uint16_t)f32_to_bf16_bits(w);
+            else if (ydt == TAMD_F16) ((uint16_t *)a.y)[at + p] = (uint16_t)f32_to_f16_bits(w);
+            else ((uint8_t *)a.y)[at + p] = (uint8_t)f32_to_fp8_bits(w, ydt);
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+#pragma unroll
+      for (int j = 0; j < 12; ++j) acc[i][f][j] = acc[i][f][j + 4];
+  }
+  if (a.y_actual_scale) store_actual_scale(a.y_actual_scale, amax, out_max, lane);
+}
+
 // FAST_YDT: the 16-bit output type that gets the specialised epilogues (the activations' type; bf16 for fp8
-// activations); any other combination takes the general one.
-// FP8_ROWS: the kernel's activations are fp8; then a plain float8_e4m3fn output (the rows the next matmul of an
-// MoE layer consumes) is specialised as well.
+// activations); FP8_ROWS: the kernel's activations are fp8, then float8_e4m3fn output (the rows the next matmul of an
+// MoE layer consumes, usually with a flexpoint scale) is specialised as well.  Any other type takes the general
+// epilogue, and so does an output whose column pairs do not lie whole on aligned words or that spans 2 GB or more.
+template <int ACT, typename Args>
+TAMD_DEVICE bool epilogue_is_regular(const Args &a) {
+  const int osz = a.y_dtype == TAMD_F32 ? 4 : (is_fp8(a.y_dtype) ? 1 : 2);
+  const int64_t lim = 0x7FFFFF00;
+  if (a.y_rows <= 0 || a.y_stride_m < 0 || a.y_rows * a.y_stride_m * osz >= lim) return false;
+  if (a.y_mx_scale && a.y_rows * a.y_mx_stride_m >= lim) return false;
+  if (ACT == TAMD_ACT_SWIGLU) return true;   // one output per lane
+  return ((a.N | (int)a.y_stride_m | (int)a.y_stride_z) & 1) == 0 && ((uintptr_t)a.y & (2 * osz - 1)) == 0;
+}
 template <int NFR, int ACT, int FAST_YDT, bool FP8_ROWS, typename Args>
-TAMD_DEVICE void tile_epilogue(const Args &a, const Tile &t, f32x16_t (&acc)[NFR][NF], uint8_t *lds) {
+TAMD_DEVICE void tile_epilogue(const Args &a, const Tile &t, f32x16_t (&acc)[NFR][NF], uint8_t *tab) {
   const bool flexo = a.y_expected_scale != nullptr || a.y_actual_scale != nullptr;
-  if (a.y_mx_scale) {  // always e4m3 values and no flexpoint output (checked by the entry point)
-    tile_epilogue_t<NFR, ACT, TAMD_FP8_E4M3, true, false, true, Args>(a, t, acc, lds);
-  } else if (FP8_ROWS && a.y_dtype == TAMD_FP8_E4M3 && !flexo) {
-    if constexpr (FP8_ROWS) tile_epilogue_t<NFR, ACT, TAMD_FP8_E4M3, true, false, false, Args>(a, t, acc, lds);
-  } else if (a.y_dtype == FAST_YDT && !flexo) {
-    if (a.betas || a.gammas) tile_epilogue_t<NFR, ACT, FAST_YDT, true, false, false, Args>(a, t, acc, lds);
-    else tile_epilogue_t<NFR, ACT, FAST_YDT, false, false, false, Args>(a, t, acc, lds);
+  const bool fast = epilogue_is_regular<ACT>(a);
+  if (fast && a.y_mx_scale) {  // always e4m3 values and no flexpoint output (checked by the entry point)
+    tile_epilogue_t<NFR, ACT, TAMD_FP8_E4M3, true, false, true, Args>(a, t, acc, tab);
+  } else if (FP8_ROWS && fast && a.y_dtype == TAMD_FP8_E4M3) {
+    if constexpr (FP8_ROWS) tile_epilogue_t<NFR, ACT, TAMD_FP8_E4M3, true, true, false, Args>(a, t, acc, tab);
+  } else if (fast && a.y_dtype == FAST_YDT && !flexo) {
+    if (a.betas || a.gammas) tile_epilogue_t<NFR, ACT, FAST_YDT, true, false, false, Args>(a, t, acc, tab);
+    else tile_epilogue_t<NFR, ACT, FAST_YDT, false, false, false, Args>(a, t, acc, tab);
   } else {
-    tile_epilogue_t<NFR, ACT, -1, true, true, false, Args>(a, t, acc, lds);
+    tile_epilogue_general<NFR, ACT, Args>(a, t, acc, tab);
   }
 }
 
@@ -1319,9 +1337,12 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
 #pragma unroll
           for (int e = 0; e < 4; ++e) acc[0][f][4 * j + e] += v[e];
         }
-    __syncthreads();   // the epilogue stages its output through the same memory
+    __syncthreads();   // the epilogue's tables take the same memory
   }
-  tile_epilogue<NFR, ACT, FP8 ? TAMD_BF16 : XDT, FP8>(kernel_args_late(), t, acc, lds_wg);
+  // (the wave's own weight region is free by now: its table goes there)
+  uint8_t *tab = KS > 1 ? lds_wg + wave * 4096 : lds + DA * A_STAGE + wave * (PAIRED ? 8192 : 4096);
+  static_assert(epilogue_table_bytes(NFR) <= 4096, "a wave's table fits its weight region");
+  tile_epilogue<NFR, ACT, FP8 ? TAMD_BF16 : XDT, FP8>(kernel_args_late(), t, acc, tab);
 }
 
 // Row fragments a workgroup can hold: a 128-row block of 16-bit activations also takes a remainder of
@@ -1378,7 +1399,6 @@ int launch_x16_act(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
   constexpr bool DEEP = deep_mode(is_fp8(XDT), LDS_ROWS);   // (kernels with the scales in LDS)
   constexpr int PIPE_BYTES = pipe_shape(is_fp8(XDT), false, LDS_ROWS, DEEP).bytes;
   constexpr int RING_BYTES = pipe_shape(is_fp8(XDT), true, LDS_ROWS).bytes;
-  constexpr int OUT_BYTES = LDS_ROWS * (ACT == TAMD_ACT_SWIGLU ? 128 : 256) * 2;  // epilogue staging
   int grid_n = (a.N + BLOCK_N - 1) / BLOCK_N;
   int64_t total = (int64_t)grid_m * grid_n;
   if (total <= 0) return 0;
@@ -1396,7 +1416,6 @@ int launch_x16_act(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
   const int sc_in_lds = dense_sc && PIPE_BYTES + sc_bytes <= (DEEP ? 156 : 80) * 1024 && !(is_fp8(XDT) && cdna4);
   constexpr int PLAIN_BYTES = pipe_shape(is_fp8(XDT), false, LDS_ROWS).bytes;   // 16-bit path, scales read from memory
   size_t lds_bytes = sc_in_lds ? PIPE_BYTES + sc_bytes : (is_fp8(XDT) ? RING_BYTES : PLAIN_BYTES);
-  if (lds_bytes < (size_t)OUT_BYTES) lds_bytes = OUT_BYTES;
   void (*kern)(tamd_matmul_args, int, int64_t, int);
   if constexpr (is_fp8(XDT))
     kern = sc_in_lds ? mm_x8_mxfp4_kernel<XDT, BM, ACT, true> : mm_x8_mxfp4_kernel<XDT, BM, ACT, false>;

@@ -393,6 +393,7 @@ def matmul(a, b, bias, a_ragged_metadata: Optional[RaggedTensorMetadata] = None,
     args.y_stride_m, args.y_stride_z = out.stride(1), out.stride(0)
     args.M, args.N, args.K, args.n_experts = M, N, K, n_slices
     args.x_rows = a.shape[-2]
+    args.y_rows = rows_out
     if flex.out_data.expected_scale is not None:
         args.y_expected_scale = flex.out_data.expected_scale.data_ptr()
     if flex.out_data.actual_scale is not None:
@@ -480,6 +481,7 @@ def _matmul_split_k(args, split_k, a, wd, w_is_fp4, out, fused_activation, bias,
             bias_s[0] = bias.reshape(-1)
             part.bias, part.bias_dtype, part.bias_stride_e = bias_s.data_ptr(), _lib.F32, N
         part.activation = _lib.ACT_NONE
+        part.y_rows = rows
         part.y, part.y_dtype = scratch.data_ptr(), _lib.F32
         part.y_stride_m, part.y_stride_z = scratch.stride(2), scratch.stride(0)
         part.y_expected_scale = part.y_actual_scale = None
