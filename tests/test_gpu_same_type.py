@@ -1,0 +1,66 @@
+"""GPU: products of two operands of one type, both contiguous along K (16-bit weights, fp8 x fp8), at the edges of the
+kernel's tiles: row remainders (a lone row, one more than a fragment, the absorbed remainder of a 128-row block), column
+remainders and K remainders, against float32 products of the same values."""
+import pytest
+import torch
+
+from triton_amd.matmul import FlexCtx, InFlexData, PrecisionConfig, matmul
+from triton_amd.matmul_details.opt_flags import scoped_opt_flags_constraints
+from triton_amd.tensor import make_ragged_tensor_metadata
+
+pytestmark = pytest.mark.gpu
+TYPES = [torch.bfloat16, torch.float16, torch.float8_e4m3fn, torch.float8_e5m2]
+
+
+def operands(shape_x, shape_w, dtype, device):
+    x, w = torch.randn(shape_x).to(dtype), (torch.randn(shape_w) * 0.1).to(dtype)
+    return x, w, x.to(device), w.to(device).transpose(-1, -2).contiguous().transpose(-1, -2)
+
+
+def config(dtype, device):
+    if dtype.itemsize > 1:
+        return None, 1.0, 1.0
+    sx, sw = torch.tensor([0.5]), torch.tensor([0.25])
+    flex = FlexCtx(InFlexData(dtype, sx.to(device)), InFlexData(dtype, sw.to(device)))
+    return PrecisionConfig(flex_ctx=flex, out_dtype=torch.bfloat16), 0.5, 0.25
+
+
+@pytest.mark.parametrize("M,K,N", [(1, 16, 136), (33, 144, 264), (160, 1040, 520), (161, 64, 256), (300, 2064, 1000)])
+@pytest.mark.parametrize("block_m", [None, 32, 64, 128])
+@pytest.mark.parametrize("dtype", TYPES)
+def test_dense(M, K, N, block_m, dtype, device):
+    torch.manual_seed(0)
+    x, w, xd, wd = operands((M, K), (K, N), dtype, device)
+    bias = torch.randn(N)
+    pc, sx, sw = config(dtype, device)
+    with scoped_opt_flags_constraints({} if block_m is None else {"block_m": block_m}):
+        y = matmul(xd, wd, bias.to(device), precision_config=pc)
+    ref = (x.float() @ w.float()) * (sx * sw) + bias
+    torch.testing.assert_close(y.cpu().float(), ref, rtol=1e-2, atol=2e-2)
+
+
+@pytest.mark.parametrize("block_m", [16, 32, 64, 128])
+@pytest.mark.parametrize("dtype", TYPES)
+def test_ragged_with_gather_scatter_and_gate_weights(block_m, dtype, device):
+    torch.manual_seed(1)
+    K, N = 208, 264
+    sizes = torch.tensor([0, 1, 16, 33, 160, 161, 300, 129], dtype=torch.int32)
+    E, M = len(sizes), int(sizes.sum())
+    x, w, xd, wd = operands((M, K), (E, K, N), dtype, device)
+    gather, scatter = torch.randperm(M).int(), torch.randperm(M).int()
+    scatter[::7] = -1
+    gammas = torch.rand(M)
+    pc, sx, sw = config(dtype, device)
+    md = make_ragged_tensor_metadata(sizes.to(device), M)
+    y = torch.zeros((M, N), dtype=torch.bfloat16 if dtype.itemsize == 1 else dtype, device=device)
+    with scoped_opt_flags_constraints({"block_m": block_m}):
+        matmul(xd, wd, None, md, gather_indx=gather.to(device), scatter_indx=scatter.to(device), precision_config=pc,
+               gammas=gammas.to(device), c=y)
+    ref = torch.zeros(M, N)
+    rows, e0 = x.float()[gather.long()], 0
+    for e, n in enumerate(sizes.tolist()):
+        out = (rows[e0:e0 + n] @ w[e].float()) * (sx * sw) * gammas[e0:e0 + n, None]
+        at = scatter[e0:e0 + n]
+        ref[at[at >= 0].long()] = out[at >= 0]
+        e0 += n
+    torch.testing.assert_close(y.cpu().float(), ref, rtol=1e-2, atol=2e-2)

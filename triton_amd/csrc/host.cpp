@@ -215,6 +215,7 @@ PyObject *py_matmul(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
     bool mx_out = false, a_mx = false;
     at::ScalarType out_type = a_type;
     bool out_type_set = false;
+    int rhs_type = -1;
     Ref b_scale_o(pc == Py_None ? (Py_INCREF(Py_None), Py_None) : attr(pc, nm.b_mx_scale));
     if (pc != Py_None) {
       Ref r1(attr(pc, nm.a_mx_tensor_scale)), r2(attr(pc, nm.b_mx_tensor_scale)), r3(attr(pc, nm.acc_scale));
@@ -248,8 +249,8 @@ PyObject *py_matmul(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
       need(ld.none() || !a8 || dtype_of(ld.p) == a_type);  // (another 8-bit type: reinterpreted by the general path)
       g.x_scale = scalar_ptr(ls.p, dev);
       g.w_scale = scalar_ptr(rs.p, dev);
-      Ref rd(attr(rhs.p, nm.dtype));
-      need(rd.none());
+      Ref rd(attr(rhs.p, nm.dtype));  // (weights of another 8-bit type: reinterpreted by the general path)
+      if (!rd.none()) rhs_type = (int)dtype_of(rd.p);
       Ref es(attr(outd.p, nm.expected_scale)), acs(attr(outd.p, nm.actual_scale)), cks(attr(outd.p, nm.checksum_scale));
       need(cks.none());
       g.y_expected_scale = scalar_ptr(es.p, dev);
@@ -301,7 +302,7 @@ PyObject *py_matmul(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
       Ref dt(attr(b_o, nm.dtype)), st(attr(b_o, nm.storage)), sh(attr(b_o, nm.shape));
       need(dt.p == obj_fp4 && PyList_Check(sh.p) && PyList_GET_SIZE(sh.p) == 3);
       Ref lay(attr(st.p, nm.layout)), data(attr(st.p, nm.data));
-      need(Py_TYPE(lay.p) == (PyTypeObject *)cls_value_layout);
+      need(Py_TYPE(lay.p) == (PyTypeObject *)cls_value_layout && rhs_type < 0);
       n_mat = as_int(PyList_GET_ITEM(sh.p, 0)), K_W = as_int(PyList_GET_ITEM(sh.p, 1)), N = as_int(PyList_GET_ITEM(sh.p, 2));
       const at::Tensor &w = gpu_tensor(data.p, dev);
       need(w.dim() == 3 && w.is_contiguous() && w.scalar_type() == at::kByte && w.size(0) == n_mat &&
@@ -314,7 +315,11 @@ PyObject *py_matmul(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
       const at::Tensor &w = gpu_tensor(b_o, dev);
       need((w.dim() == 3 || w.dim() == 2) && w.stride(-2) == 1 && w.size(-2) > 1);
       w_fp4 = w.scalar_type() == at::kByte;
-      need(w_fp4 || (w.scalar_type() == a_type && !a8 && w.stride(-1) != 1));
+      need(w_fp4 || w.scalar_type() == a_type);
+      if (a8 && !w_fp4)  // fp8 x fp8: whole, aligned 16-byte chunks along K (otherwise widened by the general path)
+        need(!a_mx && K % 16 == 0 && w.stride(-1) % 16 == 0 && (w.dim() == 2 || w.stride(0) % 16 == 0) && a.stride(0) % 16 == 0 &&
+             ((uintptr_t)w.data_ptr() | (uintptr_t)a.data_ptr()) % 16 == 0);
+      need(rhs_type < 0 || (at::ScalarType)rhs_type == w.scalar_type());
       need(w.stride(-1) != 1);
       n_mat = w.dim() == 3 ? w.size(0) : 1;
       K_W = w.size(-2) * (w_fp4 ? 2 : 1), N = w.size(-1);

@@ -10,6 +10,8 @@ int dispatch_mm_fp8e4m3(const tamd_matmul_args &a, int block_m, int grid_m, hipS
 int dispatch_mm_fp8e5m2(const tamd_matmul_args &a, int block_m, int grid_m, hipStream_t st);
 int dispatch_mm_w16_bf16(const tamd_matmul_args &a, int block_m, int grid_m, hipStream_t st);
 int dispatch_mm_w16_f16(const tamd_matmul_args &a, int block_m, int grid_m, hipStream_t st);
+int dispatch_mm_kk_fp8e4m3(const tamd_matmul_args &a, int block_m, int grid_m, hipStream_t st);
+int dispatch_mm_kk_fp8e5m2(const tamd_matmul_args &a, int block_m, int grid_m, hipStream_t st);
 }  // namespace tamd
 
 using namespace tamd;
@@ -78,8 +80,9 @@ extern "C" int tamd_matmul(const tamd_matmul_args *args, void *stream) {
     if (a.x_dtype == TAMD_FP8_E5M2) return dispatch_mm_fp8e5m2(a, block_m, grid_m, st);
     return dispatch_mm_fp8e4m3(a, block_m, grid_m, st);
   }
-  if ((a.x_dtype == TAMD_BF16 || a.x_dtype == TAMD_F16) && a.w_dtype == a.x_dtype) {
-    // unquantised weights of the activations' type
+  if ((a.x_dtype == TAMD_BF16 || a.x_dtype == TAMD_F16 || x8) && a.w_dtype == a.x_dtype) {
+    // weights of the activations' type: unquantised, or fp8 with per-tensor scales on both sides
+    if (x8 && (a.x_mx_scale || a.w_stride_k != 1)) return TAMD_E_UNSUPPORTED;
     int block_m, grid_m;
     if (ragged) {
       block_m = a.block_m;
@@ -88,6 +91,8 @@ extern "C" int tamd_matmul(const tamd_matmul_args *args, void *stream) {
       block_m = a.force_variant;
       grid_m = block_m ? ((a.M + block_m - 1) / block_m) * a.n_experts : 0;
     }
+    if (a.x_dtype == TAMD_FP8_E4M3) return dispatch_mm_kk_fp8e4m3(a, block_m, grid_m, st);
+    if (a.x_dtype == TAMD_FP8_E5M2) return dispatch_mm_kk_fp8e5m2(a, block_m, grid_m, st);
     if (a.x_dtype == TAMD_BF16) return dispatch_mm_w16_bf16(a, block_m, grid_m, st);
     return dispatch_mm_w16_f16(a, block_m, grid_m, st);
   }

@@ -1,25 +1,20 @@
-// Grouped / dense matmul with unquantised 16-bit weights (bf16 x bf16, f16 x f16): the gate matmul and
-// every caller of `matmul` that passes plain weights.  Same tile decomposition, activation staging and
-// epilogue as the MXFP4 kernel of moe_matmul_impl.h; only the weight path differs:
+// Grouped / dense matmul with unquantised 16-bit weights (bf16 x bf16, f16 x f16): the narrow products (the gate matmul),
+// and weights with unit stride along N; K-contiguous weights go to moe_matmul_kk.h.
 //
-//   * K-contiguous weights (w_stride_k == 1, the layout of the quantised weights): a stage holds
-//     [256 columns][64 K] = 128 bytes per column, copied by DMA exactly like activation rows and read
-//     as 16-byte MFMA fragments;
-//   * N-contiguous weights (w_stride_n == 1, the usual row-major [K, N]): a stage holds
-//     [64 K][256 columns] as it lies in memory (512 bytes per K row); a lane gathers the 8 K values of
-//     its column with 2-byte LDS reads.  The MFMA wants K-contiguous operands on both sides, so one of
-//     the two has to be transposed somewhere; doing it on the LDS read costs no extra pass.
+// N-contiguous weights (w_stride_n == 1, the usual row-major [K, N]): same tile decomposition, activation staging and
+// epilogue as the MXFP4 kernel of moe_matmul_impl.h.  A stage holds [64 K][256 columns] as it lies in memory (512 bytes
+// per K row); a lane gathers the 8 K values of its column with 2-byte LDS reads.  The MFMA wants K-contiguous operands
+// on both sides, so one of the two has to be transposed somewhere; doing it on the LDS read costs no extra pass.
 //
-// One workgroup per CU (three 32 KB weight stages); not a tuned kernel -- the unquantised
-// products on this path are small next to the expert matmuls.
+// One workgroup per CU (three 32 KB weight stages); not a tuned kernel.
 #pragma once
 #include "moe_matmul_impl.h"
 
 namespace tamd {
 
-constexpr int W16_STAGE = 256 * 128;  // bytes of one weight stage in either layout
+constexpr int W16_STAGE = 256 * 128;  // bytes of one weight stage
 
-template <int XDT, int NFR, int LDS_ROWS, int ACT, bool WKC>
+template <int XDT, int NFR, int LDS_ROWS, int ACT>
 TAMD_DEVICE void run_tile_w16(const tamd_matmul_args &a, const Tile &t, uint8_t *lds) {
   typedef Mma<XDT> M;
   typedef typename M::frag_t frag_t;
@@ -34,7 +29,7 @@ TAMD_DEVICE void run_tile_w16(const tamd_matmul_args &a, const Tile &t, uint8_t 
   const v4i_t rx = make_rsrc((const uint8_t *)a.x + (int64_t)t.z * a.x_stride_z * 2, kOob);
   // the descriptor ends with the expert's weights: a copy that starts inside and runs past the end
   // (partial last chunk of columns) delivers zeros for the part outside
-  const int64_t w_span = (WKC ? (int64_t)N * a.w_stride_n : (int64_t)K * a.w_stride_k) * 2;
+  const int64_t w_span = (int64_t)K * a.w_stride_k * 2;
   const v4i_t rw = make_rsrc((const uint8_t *)a.w + (int64_t)t.expert * a.w_stride_e * 2, (uint32_t)w_span);
   const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds;
   constexpr int RING = 3;  // stages: one consumed, two in flight (the K loop of a small tile is latency bound)
@@ -56,21 +51,12 @@ TAMD_DEVICE void run_tile_w16(const tamd_matmul_args &a, const Tile &t, uint8_t 
   int w_chunk[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
-    if constexpr (WKC) {
-      // LDS row p = wave*64 + j*8 + lane/8 holds tile column wave*64 + 2*(q%32) + q/32 (q = p%64) so that a lane's
-      // two fragments are a gate / linear pair; 16-byte chunks swizzled like activation rows
-      const int q = j * 8 + lane / 8;
-      const int col = t.n0 + wave * 64 + 2 * (q % 32) + q / 32;
-      w_chunk[j] = (lane % 8) ^ (((wave * 64 + q) >> 1) & 7);
-      w_off[j] = col < N ? (uint32_t)col * (uint32_t)(a.w_stride_n * 2) + w_chunk[j] * 16 : kOob;
-    } else {
-      // K rows 16w + 2j, 16w + 2j + 1 of the stage, 32 chunks of 8 columns each
-      const int col = t.n0 + 8 * (lane % 32);
-      w_chunk[j] = wave * 16 + 2 * j + lane / 32;  // K row inside the stage
-      // N is a multiple of 8 here; the lane's half (lane/32) of the K row pair goes into the vector offset, the
-      // pair's first row into the wave-uniform scalar offset
-      w_off[j] = col + 8 <= N ? (uint32_t)col * 2u + (uint32_t)(lane / 32) * (uint32_t)(a.w_stride_k * 2) : kOob;
-    }
+    // K rows 16w + 2j, 16w + 2j + 1 of the stage, 32 chunks of 8 columns each
+    const int col = t.n0 + 8 * (lane % 32);
+    w_chunk[j] = wave * 16 + 2 * j + lane / 32;  // K row inside the stage
+    // N is a multiple of 8 here; the lane's half (lane/32) of the K row pair goes into the vector offset, the
+    // pair's first row into the wave-uniform scalar offset
+    w_off[j] = col + 8 <= N ? (uint32_t)col * 2u + (uint32_t)(lane / 32) * (uint32_t)(a.w_stride_k * 2) : kOob;
   }
 
   f32x16_t acc[NFR][NF];
@@ -92,15 +78,10 @@ TAMD_DEVICE void run_tile_w16(const tamd_matmul_args &a, const Tile &t, uint8_t 
     const uint32_t sb = lds_b + slot * W16_STAGE;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      if constexpr (WKC) {
-        const uint32_t kill = kb + w_chunk[j] * 8 < K ? 0u : kOob;
-        dma16(rw, sb + (wave * 64 + j * 8) * 128, w_off[j] | kill, kb * 2);
-      } else {
-        const int k = kb + w_chunk[j];
-        const uint32_t kill = k < K ? 0u : kOob;
-        dma16(rw, sb + (wave * 16 + 2 * j) * 512, w_off[j] | kill,
-              (uint32_t)((int64_t)(kb + wave * 16 + 2 * j) * a.w_stride_k * 2));
-      }
+      const int k = kb + w_chunk[j];
+      const uint32_t kill = k < K ? 0u : kOob;
+      dma16(rw, sb + (wave * 16 + 2 * j) * 512, w_off[j] | kill,
+            (uint32_t)((int64_t)(kb + wave * 16 + 2 * j) * a.w_stride_k * 2));
     }
   };
 
@@ -115,20 +96,14 @@ TAMD_DEVICE void run_tile_w16(const tamd_matmul_args &a, const Tile &t, uint8_t 
       for (int i = 0; i < NFR; ++i) af[i] = *(const frag_t *)(abuf + (i * 32 + c32) * A_ROW_BYTES + aslot * 16);
 #pragma unroll
       for (int f = 0; f < NF; ++f) {
-        frag_t bf;
-        if constexpr (WKC) {
-          const int p = wave * 64 + f * 32 + c32;
-          bf = *(const frag_t *)(bbuf + p * 128 + (((h * 4 + s) ^ ((p >> 1) & 7)) * 16));
-        } else {
-          const uint16_t *colp = (const uint16_t *)bbuf + (wave * 64 + c32 * NF + f);
-          uint32_t w[4];
+        const uint16_t *colp = (const uint16_t *)bbuf + (wave * 64 + c32 * NF + f);
+        uint32_t w[4];
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int k = (h * 4 + s) * 8 + 2 * e;
-            w[e] = (uint32_t)colp[k * 256] | ((uint32_t)colp[(k + 1) * 256] << 16);
-          }
-          bf = __builtin_bit_cast(frag_t, make_uint4(w[0], w[1], w[2], w[3]));
+        for (int e = 0; e < 4; ++e) {
+          const int k = (h * 4 + s) * 8 + 2 * e;
+          w[e] = (uint32_t)colp[k * 256] | ((uint32_t)colp[(k + 1) * 256] << 16);
         }
+        const frag_t bf = __builtin_bit_cast(frag_t, make_uint4(w[0], w[1], w[2], w[3]));
 #pragma unroll
         for (int i = 0; i < NFR; ++i) acc[i][f] = M::mma(af[i], bf, acc[i][f]);
       }
@@ -150,7 +125,7 @@ TAMD_DEVICE void run_tile_w16(const tamd_matmul_args &a, const Tile &t, uint8_t 
   tile_epilogue<NFR, ACT, XDT, false>(a, t, acc, lds + wave * 4096);
 }
 
-template <int XDT, int BM, int ACT, bool WKC>
+template <int XDT, int BM, int ACT>
 __global__ __launch_bounds__(256, 1) void mm_x16_w16_kernel(tamd_matmul_args a, int grid_n, int64_t grid_total) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   constexpr int MF = BM <= 32 ? 1 : BM / 32;
@@ -159,13 +134,13 @@ __global__ __launch_bounds__(256, 1) void mm_x16_w16_kernel(tamd_matmul_args a, 
   const int nfr = (t.rows + 31) / 32;
 #define TAMD_CASE(n)                                                            \
   case n:                                                                       \
-    if constexpr (n <= MF) run_tile_w16<XDT, n, 32 * MF, ACT, WKC>(a, t, lds);  \
+    if constexpr (n <= MF) run_tile_w16<XDT, n, 32 * MF, ACT>(a, t, lds);       \
     break;
   switch (nfr) { TAMD_CASE(1) TAMD_CASE(2) TAMD_CASE(3) TAMD_CASE(4) }
 #undef TAMD_CASE
 }
 
-template <int XDT, int BM, int ACT, bool WKC>
+template <int XDT, int BM, int ACT>
 int launch_w16(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
   constexpr int MF = BM <= 32 ? 1 : BM / 32;
   constexpr int LDS_ROWS = 32 * MF;
@@ -176,7 +151,7 @@ int launch_w16(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
   if (total <= 0) return 0;
   const int64_t launch = ((total + 7) / 8) * 8;
   if (launch > 0x7FFFFFFF) return TAMD_E_UNSUPPORTED;
-  auto kern = mm_x16_w16_kernel<XDT, BM, ACT, WKC>;
+  auto kern = mm_x16_w16_kernel<XDT, BM, ACT>;
   if (int rc = raise_lds_limit_once((const void *)kern)) return rc;
   kern<<<dim3((unsigned)launch), 256, PIPE, st>>>(a, grid_n, total);
   return launch_status();
@@ -343,29 +318,29 @@ int launch_skinny16(const tamd_matmul_args &a, hipStream_t st) {
   return launch_status();
 }
 
+int dispatch_mm_kk_bf16(const tamd_matmul_args &a, int block_m, int grid_m, hipStream_t st);
+int dispatch_mm_kk_f16(const tamd_matmul_args &a, int block_m, int grid_m, hipStream_t st);
+
 // 16-bit activations x 16-bit weights of the same type.  Returns TAMD_E_UNSUPPORTED / _ALIGNMENT for layouts
 // the kernel does not cover.
 template <int XDT>
 int dispatch_w16(const tamd_matmul_args &a, int block_m, int grid_m, hipStream_t st) {
   if (skinny16_applicable(a)) return launch_skinny16<XDT>(a, st);
+  if (a.w_stride_k == 1)
+    return XDT == TAMD_BF16 ? dispatch_mm_kk_bf16(a, block_m, grid_m, st) : dispatch_mm_kk_f16(a, block_m, grid_m, st);
   dense_grid(a, block_m, grid_m);
-  const bool kc = a.w_stride_k == 1, nc = a.w_stride_n == 1;
-  if (!kc && !nc) return TAMD_E_UNSUPPORTED;
-  if (a.K % 8 != 0) return TAMD_E_UNSUPPORTED;  // whole 16-byte chunks along K
-  if (!kc && a.N % 8 != 0) return TAMD_E_UNSUPPORTED;  // whole 16-byte chunks along N
-  const int64_t pitch = kc ? a.w_stride_n : a.w_stride_k;
-  if (!aligned(a.w, 16) || (pitch * 2) % 16 != 0 || (a.w_stride_e * 2) % 16 != 0) return TAMD_E_ALIGNMENT;
+  if (a.w_stride_n != 1) return TAMD_E_UNSUPPORTED;
+  if (a.K % 8 != 0 || a.N % 8 != 0) return TAMD_E_UNSUPPORTED;  // whole 16-byte chunks along K and N
+  if (!aligned(a.w, 16) || (a.w_stride_k * 2) % 16 != 0 || (a.w_stride_e * 2) % 16 != 0) return TAMD_E_ALIGNMENT;
   if (!aligned(a.x, 16) || (a.x_stride_m * 2) % 16 != 0 || (a.x_stride_z * 2) % 16 != 0) return TAMD_E_ALIGNMENT;
   const int64_t x_rows = a.x_rows > 0 ? a.x_rows : a.M;
-  const int64_t w_span = (kc ? (int64_t)a.N * a.w_stride_n : (int64_t)a.K * a.w_stride_k) * 2;
+  const int64_t w_span = (int64_t)a.K * a.w_stride_k * 2;
   if (x_rows * a.x_stride_m * 2 >= (int64_t)0x7FFFFF00 || w_span >= (int64_t)0x7FFFFF00) return TAMD_E_UNSUPPORTED;
   const bool sw = a.activation == TAMD_ACT_SWIGLU;
 #define TAMD_W16(BMV)                                                                                           \
   case BMV:                                                                                                     \
-    if (kc) return sw ? launch_w16<XDT, BMV, TAMD_ACT_SWIGLU, true>(a, grid_m, st)                               \
-                      : launch_w16<XDT, BMV, TAMD_ACT_NONE, true>(a, grid_m, st);                                 \
-    return sw ? launch_w16<XDT, BMV, TAMD_ACT_SWIGLU, false>(a, grid_m, st)                                      \
-              : launch_w16<XDT, BMV, TAMD_ACT_NONE, false>(a, grid_m, st);
+    return sw ? launch_w16<XDT, BMV, TAMD_ACT_SWIGLU>(a, grid_m, st)                                             \
+              : launch_w16<XDT, BMV, TAMD_ACT_NONE>(a, grid_m, st);
   switch (block_m) {
     TAMD_W16(16) TAMD_W16(32) TAMD_W16(64) TAMD_W16(128)
     default: return TAMD_E_UNSUPPORTED;

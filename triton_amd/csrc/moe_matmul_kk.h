@@ -1,0 +1,264 @@
+// Grouped / dense matmul of two operands of the same element type that are both contiguous along K: unquantised 16-bit
+// weights (bf16 x bf16, f16 x f16) and fp8 x fp8 with per-tensor scales.
+//
+// A tile is up to 128 rows (160 with 16-bit operands: a remainder of up to 32 rows is absorbed, as in moe_matmul_impl.h)
+// x 256 columns; a workgroup of eight waves owns a CU.  Both operands travel HBM -> LDS by 16-byte DMA in stages of 128
+// bytes per row and column (64 K of 16-bit values, 128 K of fp8), through a ring of three or four stages that is two or
+// three ahead of the matrix cores; rows and columns are 128-byte lines, requested whole.
+//
+// What bounds it.  With few rows per expert: HBM (the ring holds 64 KB or more of weights in flight per CU).  With full
+// tiles the LDS: per stage a wave of 128 x 64 reads 24 KB for 16 KB x 64 columns of products, and four such waves and
+// the copies take 1152 cycles at 128 bytes per cycle against 1024 of MFMA.  Hence the two K groups: waves 0-3 and 4-7
+// share the tile's four 64-column strips, each group multiplying one half of every stage, so that a SIMD holds two
+// waves for the LDS traffic of one (waves of 64 x 64 would read a third more).  Group 0 requests the next stage's copies
+// before its products and group 1 after them: a copy instruction holds its wave for about a hundred cycles, and with
+// both groups issuing at the same time the matrix cores idled meanwhile.  The groups' partial sums meet in LDS after the
+// loop, each group finishing one half of the row fragments.
+#pragma once
+#include "moe_matmul_impl.h"
+
+namespace tamd {
+
+template <int XDT>
+struct KK {
+  static constexpr bool FP8 = is_fp8(XDT);
+  static constexpr int ESZ = FP8 ? 1 : 2;
+  static constexpr int KS = 128 / ESZ;                 // K per stage
+};
+template <int XDT, int BM>
+struct KKShape {
+  typedef TileShape<XDT, BM> T;
+  static constexpr int STAGE = (T::LDS_ROWS + BLOCK_N) * 128;
+  static constexpr int RING = T::LDS_ROWS <= 32 ? 4 : 3;
+  static constexpr int EXCHANGE = T::MF * 4 * kWave * NF * 16 * 4;   // partial sums of MF row fragments
+  static constexpr int LDS = RING * STAGE > EXCHANGE ? RING * STAGE : EXCHANGE;
+  static_assert(LDS <= 160 * 1024, "one workgroup per CU");
+};
+
+template <int XDT, int NFR, int BM, int ACT>
+TAMD_DEVICE void run_tile_kk(const tamd_matmul_args &a, const Tile &t, uint8_t *lds) {
+  typedef Mma<XDT> M;
+  typedef KKShape<XDT, BM> S;
+  constexpr bool FP8 = KK<XDT>::FP8;
+  constexpr int ESZ = KK<XDT>::ESZ, KS = KK<XDT>::KS, EPC = 16 / ESZ;
+  constexpr int LDS_ROWS = S::T::LDS_ROWS, STAGE = S::STAGE, RING = S::RING;
+  constexpr uint32_t kOob = 0x7FFFFFFFu;
+  const int wave8 = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
+  const int grp = wave8 >> 2, wave = wave8 & 3;        // K group, column strip
+  const int c32 = lane % 32, h = lane / 32;
+  const int K = a.K, N = a.N;
+  const v4i_t rx = make_rsrc((const uint8_t *)a.x + (int64_t)t.z * a.x_stride_z * ESZ, kOob);
+  const v4i_t rw = make_rsrc((const uint8_t *)a.w + (int64_t)t.expert * a.w_stride_e * ESZ, kOob);
+  const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds;
+
+  // ---- copies: instruction q of an operand moves its LDS rows 8q .. 8q + 7, lane -> (row 8q + lane / 8, slot lane % 8),
+  // slot s of row r holding chunk s ^ ((r >> 1) & 7); wave w takes the instructions w, w + 8, ... of both operands
+  const int rin = lane / 8;
+  const int chunk = (lane % 8) ^ ((wave8 & 1) * 4 + (rin >> 1));
+  constexpr int NA0 = (NFR + 1) / 2, NA1 = NFR / 2, NB = 4;   // copies per wave and stage: group 0, group 1; columns
+  uint32_t a_off[NA0], b_off[NB];
+#pragma unroll
+  for (int u = 0; u < NA0; ++u) {
+    const int r = (wave8 + 8 * u) * 8 + rin;
+    const int rr = t.off_m + (r < t.rows ? r : t.rows - 1);
+    const uint32_t src = a.gather_indx ? (uint32_t)a.gather_indx[t.start_m + rr] : (uint32_t)(t.start_m + rr);
+    a_off[u] = r < t.rows ? src * (uint32_t)(a.x_stride_m * ESZ) + chunk * 16 : kOob;
+  }
+#pragma unroll
+  for (int u = 0; u < NB; ++u) {
+    const int p = (wave8 + 8 * u) * 8 + rin;                  // position 64 strip + 32 f + c holds column 64 strip + 2 c + f
+    const int col = t.n0 + (p & ~63) + 2 * (p % 32) + (p % 64) / 32;
+    b_off[u] = col < N ? (uint32_t)col * (uint32_t)(a.w_stride_n * ESZ) + chunk * 16 : kOob;
+  }
+  auto issue = [&](int it, int slot) {   // (chunks past K are not read: zeros)
+    const int kb = it * KS;
+    const uint32_t kill = kb + chunk * EPC < K ? 0u : kOob;
+    const uint32_t sa = lds_base + slot * STAGE + wave8 * 1024;
+#pragma unroll
+    for (int u = 0; u < NA0; ++u)
+      if (u < NA1 || grp == 0) dma16(rx, sa + u * 8192, a_off[u] | kill, kb * ESZ);
+    const uint32_t sb = sa + LDS_ROWS * 128;
+#pragma unroll
+    for (int u = 0; u < NB; ++u) dma16(rw, sb + u * 8192, b_off[u] | kill, kb * ESZ);
+  };
+
+  f32x16_t acc[NFR][NF];
+#pragma unroll
+  for (int i = 0; i < NFR; ++i)
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+#pragma unroll
+      for (int j = 0; j < 16; ++j) acc[i][f][j] = 0.f;
+
+  const bool live = t.n0 + wave * 64 < N;
+  const int swz = (c32 >> 1) & 7;
+  // the group's two 16-byte chunks of a row or column: 16-bit values take two MFMA steps, fp8 one
+  const int slot0 = (FP8 ? (4 * grp + h) : (h * 4 + 2 * grp)) ^ swz, slot1 = (FP8 ? (4 * grp + 2 + h) : (h * 4 + 2 * grp + 1)) ^ swz;
+  const int a_lane = c32 * 128, b_lane = LDS_ROWS * 128 + (wave * 64 + c32) * 128;
+  const int n_k = (K + KS - 1) / KS;
+#pragma unroll
+  for (int s = 0; s < RING - 1; ++s) issue(s, s);
+  int rd = 0, wr = RING - 1;
+  for (int it = 0; it < n_k; ++it) {
+    // copies complete in the order of their requests: all but those of the newest RING - 2 stages have landed
+    if (grp == 0) wait_vmcnt<(RING - 2) * (NA0 + NB)>(); else wait_vmcnt<(RING - 2) * (NA1 + NB)>();
+    __syncthreads();   // stage `it` is visible; every wave is done with the slot that is refilled now
+    const uint8_t *buf = lds + rd * STAGE;
+    uint4 av[NFR][2], bv[NF][2];
+    if (live) {
+#pragma unroll
+      for (int f = 0; f < NF; ++f) {
+        bv[f][0] = *(const uint4 *)(buf + b_lane + f * 4096 + slot0 * 16);
+        bv[f][1] = *(const uint4 *)(buf + b_lane + f * 4096 + slot1 * 16);
+      }
+#pragma unroll
+      for (int i = 0; i < NFR; ++i) {
+        av[i][0] = *(const uint4 *)(buf + a_lane + i * 4096 + slot0 * 16);
+        av[i][1] = *(const uint4 *)(buf + a_lane + i * 4096 + slot1 * 16);
+      }
+    }
+    if (grp == 0) issue(it + RING - 1, wr);
+    if (live) {
+      if constexpr (FP8) {
+        constexpr int CBSZ = XDT == TAMD_FP8_E5M2 ? 1 : 0;
+        auto frag = [](const uint4 &lo, const uint4 &hi) {
+          return i32x8_t{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
+        };
+#pragma unroll
+        for (int i = 0; i < NFR; ++i)
+#pragma unroll
+          for (int f = 0; f < NF; ++f)
+            acc[i][f] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(frag(av[i][0], av[i][1]), frag(bv[f][0], bv[f][1]),
+                                                                      acc[i][f], CBSZ, CBSZ, 0, 0x7F7F7F7F, 0, 0x7F7F7F7F);
+      } else {
+        typedef typename M::frag_t frag_t;
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+          for (int i = 0; i < NFR; ++i)
+#pragma unroll
+            for (int f = 0; f < NF; ++f)
+              acc[i][f] = M::mma(__builtin_bit_cast(frag_t, av[i][s]), __builtin_bit_cast(frag_t, bv[f][s]), acc[i][f]);
+      }
+    }
+    if (grp == 1) issue(it + RING - 1, wr);
+    rd = rd + 1 == RING ? 0 : rd + 1;
+    wr = wr + 1 == RING ? 0 : wr + 1;
+  }
+  wait_dma();
+  __syncthreads();
+
+  // ---- the groups' partial sums: group 0 finishes the row fragments [0, N0), group 1 the rest.  Plane (fragment,
+  // strip) of the exchange is [NF x 4][64 lanes] of four accumulators; a wave reads only what its partner left for it.
+  constexpr int N0 = (NFR + 1) / 2, N1 = NFR / 2;
+  f32x4_t *ex = (f32x4_t *)lds;
+  constexpr int PLANE = NF * 4 * kWave;
+  auto put = [&](int i) {
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        ex[(i * 4 + wave) * PLANE + (f * 4 + j) * kWave + lane] =
+            f32x4_t{acc[i][f][4 * j], acc[i][f][4 * j + 1], acc[i][f][4 * j + 2], acc[i][f][4 * j + 3]};
+  };
+  auto take = [&](int i, f32x16_t (&to)[NF]) {   // (group 0's part first, whichever group adds)
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const f32x4_t v = ex[(i * 4 + wave) * PLANE + (f * 4 + j) * kWave + lane];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) to[f][4 * j + e] += v[e];
+      }
+  };
+  constexpr int FAST = FP8 ? TAMD_BF16 : XDT;
+  if (grp == 0) {
+#pragma unroll
+    for (int i = N0; i < NFR; ++i) put(i);
+  } else {
+#pragma unroll
+    for (int i = 0; i < N0; ++i) put(i);
+  }
+  __syncthreads();
+  if (grp == 0) {
+    f32x16_t mine[N0][NF];
+#pragma unroll
+    for (int i = 0; i < N0; ++i) {
+#pragma unroll
+      for (int f = 0; f < NF; ++f) mine[i][f] = acc[i][f];
+      take(i, mine[i]);
+    }
+    Tile t0 = t;
+    t0.rows = t.rows < 32 * N0 ? t.rows : 32 * N0;
+    tile_epilogue<N0, ACT, FAST, FP8>(kernel_args_late(), t0, mine, lds + wave * PLANE * 16);   // (its plane has been read)
+  } else {
+    if constexpr (N1 > 0) {
+      f32x16_t mine[N1][NF];
+#pragma unroll
+      for (int i = 0; i < N1; ++i) {
+#pragma unroll
+        for (int f = 0; f < NF; ++f) mine[i][f] = acc[N0 + i][f];
+        take(N0 + i, mine[i]);
+      }
+      Tile t1 = t;
+      t1.off_m = t.off_m + 32 * N0;
+      t1.rows = t.rows - 32 * N0;
+      tile_epilogue<N1, ACT, FAST, FP8>(kernel_args_late(), t1, mine, lds + (N0 * 4 + wave) * PLANE * 16);
+    }
+  }
+}
+
+template <int XDT, int BM, int ACT>
+__global__ __launch_bounds__(512, 1) void mm_kk_kernel(tamd_matmul_args a, int grid_n, int64_t grid_total, int group_m) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  typedef TileShape<XDT, BM> S;
+  Tile t;
+  if (!locate_tile<BM, S::EXTRA>(a, grid_n, grid_total, group_m, t)) return;
+  const int nfr = (t.rows + 31) / 32;
+#define TAMD_CASE(n)                                                      \
+  case n:                                                                 \
+    if constexpr (n <= S::MF) run_tile_kk<XDT, n, BM, ACT>(a, t, lds);    \
+    break;
+  switch (nfr) { TAMD_CASE(1) TAMD_CASE(2) TAMD_CASE(3) TAMD_CASE(4) TAMD_CASE(5) }
+#undef TAMD_CASE
+}
+
+template <int XDT, int BM, int ACT>
+int launch_kk(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
+  const int grid_n = (a.N + BLOCK_N - 1) / BLOCK_N;
+  const int64_t total = (int64_t)grid_m * grid_n;
+  if (total <= 0) return 0;
+  const int64_t launch = ((total + 7) / 8) * 8;
+  if (launch > 0x7FFFFFFF) return TAMD_E_UNSUPPORTED;
+  // row blocks walked together (see launch_x16_act)
+  const int64_t rows_per_slice = a.block_schedule ? a.M / a.n_experts : a.M;
+  int64_t group_m = (rows_per_slice + BM - 1) / BM;
+  group_m = group_m < 1 ? 1 : (group_m > 8 ? 8 : group_m);
+  auto kern = mm_kk_kernel<XDT, BM, ACT>;
+  if (int rc = raise_lds_limit_once((const void *)kern)) return rc;
+  kern<<<dim3((unsigned)launch), 512, KKShape<XDT, BM>::LDS, st>>>(a, grid_n, total, (int)group_m);
+  return launch_status();
+}
+
+// Both operands contiguous along K, 16-byte aligned rows and columns, whole 16-byte chunks along K, and offsets inside
+// an operand below 2 GB: anything else is refused (TAMD_E_UNSUPPORTED / _ALIGNMENT).
+template <int XDT>
+int dispatch_kk(const tamd_matmul_args &a, int block_m, int grid_m, hipStream_t st) {
+  constexpr int ESZ = KK<XDT>::ESZ;
+  dense_grid(a, block_m, grid_m);
+  if (a.w_stride_k != 1 || a.K % (16 / ESZ) != 0) return TAMD_E_UNSUPPORTED;
+  if (!aligned(a.w, 16) || (a.w_stride_n * ESZ) % 16 != 0 || (a.w_stride_e * ESZ) % 16 != 0) return TAMD_E_ALIGNMENT;
+  if (!aligned(a.x, 16) || (a.x_stride_m * ESZ) % 16 != 0 || (a.x_stride_z * ESZ) % 16 != 0) return TAMD_E_ALIGNMENT;
+  const int64_t x_rows = a.x_rows > 0 ? a.x_rows : a.M, lim = 0x7FFFFF00;
+  if (x_rows * a.x_stride_m * ESZ >= lim || (int64_t)a.N * a.w_stride_n * ESZ >= lim) return TAMD_E_UNSUPPORTED;
+  const bool sw = a.activation == TAMD_ACT_SWIGLU;
+  switch (block_m) {
+    case 16: return sw ? launch_kk<XDT, 16, TAMD_ACT_SWIGLU>(a, grid_m, st) : launch_kk<XDT, 16, TAMD_ACT_NONE>(a, grid_m, st);
+    case 32: return sw ? launch_kk<XDT, 32, TAMD_ACT_SWIGLU>(a, grid_m, st) : launch_kk<XDT, 32, TAMD_ACT_NONE>(a, grid_m, st);
+    case 64: return sw ? launch_kk<XDT, 64, TAMD_ACT_SWIGLU>(a, grid_m, st) : launch_kk<XDT, 64, TAMD_ACT_NONE>(a, grid_m, st);
+    case 128: return sw ? launch_kk<XDT, 128, TAMD_ACT_SWIGLU>(a, grid_m, st) : launch_kk<XDT, 128, TAMD_ACT_NONE>(a, grid_m, st);
+    default: return TAMD_E_UNSUPPORTED;
+  }
+}
+
+}  // namespace tamd

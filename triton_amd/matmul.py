@@ -96,6 +96,14 @@ def _widen_mxfp4_activations(a_raw):
     return out
 
 
+def _fp8_direct(a, w):
+    """fp8 operands that the fp8 x fp8 kernel reads as they are: one type, both contiguous along K in whole, aligned 16-byte
+    chunks."""
+    whole = lambda t, *strides: t.data_ptr() % 16 == 0 and all(s % 16 == 0 for s in strides)
+    return (a.dtype == w.dtype and a.stride(-1) == 1 and w.stride(-2) == 1 and a.shape[-1] % 16 == 0
+            and whole(a, *a.stride()[:-1]) and whole(w, w.stride(-1), *w.stride()[:-2]))
+
+
 _TURNED = {}  # id(weights) -> (weak reference to them, their version counter, the copy with unit stride along K)
 
 
@@ -240,10 +248,11 @@ def matmul(a, b, bias, a_ragged_metadata: Optional[RaggedTensorMetadata] = None,
     w = flex.rhs_data.reinterpret(b_data)
     a_dtype = a.dtype  # the type the output defaults to
     fp8_types = (torch.float8_e4m3fn, torch.float8_e5m2)
-    if not b_fp4 and w.dtype in fp8_types and a.dtype in fp8_types and a_mx_scale is None:
-        # fp8 x fp8 with per-tensor scales (tests/test_matmul.py:150-154 of the reference): every fp8 number is a
-        # bfloat16 number, so both operands are widened (exactly) and multiplied by the kernel for 16-bit weights; the
-        # flex scales enter in its epilogue as they do for any other pair of types
+    if not b_fp4 and w.dtype in fp8_types and a.dtype in fp8_types and a_mx_scale is None and not _fp8_direct(a, w):
+        # fp8 x fp8 with per-tensor scales (tests/test_matmul.py:150-154 of the reference) of two types, or in a layout that
+        # the kernel for fp8 operands does not read: every fp8 number is a bfloat16 number, so both operands are widened
+        # (exactly) and multiplied by a kernel for 16-bit weights; the flex scales enter in its epilogue as they do for
+        # any other pair of types
         a, w = a.to(torch.bfloat16), w.to(torch.bfloat16)
     if not b_fp4 and w.stride(-1) == 1 and (w.shape[-1] * w.element_size()) % 16 != 0 \
             and (w.shape[-2] * w.element_size()) % 16 == 0:
