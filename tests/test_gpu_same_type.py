@@ -64,3 +64,31 @@ def test_ragged_with_gather_scatter_and_gate_weights(block_m, dtype, device):
         ref[at[at >= 0].long()] = out[at >= 0]
         e0 += n
     torch.testing.assert_close(y.cpu().float(), ref, rtol=1e-2, atol=2e-2)
+
+
+@pytest.mark.parametrize("sizes", [
+    [160] * 20 + [1] * 20,            # equal shares of the work would need more workgroups on an XCD than there are
+    [0, 33, 0, 128, 96, 1, 161, 64],  # every number of fragments, an absorbed remainder and one row more than that
+    [5], [129],
+])
+@pytest.mark.parametrize("quantised", [False, True])
+def test_tiles_shared_out_by_their_time(sizes, quantised, device):
+    torch.manual_seed(2)
+    K, N = 64, 264
+    sizes = torch.tensor(sizes, dtype=torch.int32)
+    E, M = len(sizes), int(sizes.sum())
+    x, w, xd, wd = operands((M, K), (E, K, N), torch.bfloat16, device)
+    pc = None
+    if quantised:
+        from triton_amd.numerics_details.mxfp import downcast_to_mxfp, upcast_from_mxfp
+        v, s = downcast_to_mxfp(wd, torch.uint8, axis=-2)
+        w, wd = upcast_from_mxfp(v, s, torch.bfloat16, axis=-2).cpu(), v
+        pc = PrecisionConfig(b_mx_scale=s, b_microblock_size=32)
+    md = make_ragged_tensor_metadata(sizes.to(device), M)
+    with scoped_opt_flags_constraints({"block_m": 128}):
+        y = matmul(xd, wd, None, md, precision_config=pc)
+    at, ref = 0, torch.zeros(M, N)
+    for e, n in enumerate(sizes.tolist()):
+        ref[at:at + n] = x.float()[at:at + n] @ w[e].float()
+        at += n
+    torch.testing.assert_close(y.cpu().float(), ref, rtol=1e-2, atol=2e-2)

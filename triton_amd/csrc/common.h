@@ -97,6 +97,18 @@ TAMD_DEVICE void store_from_f32(void *p, int64_t i, float v) {
 
 __host__ __device__ inline bool is_fp8_type(int dt) { return dt == TAMD_FP8_E4M3 || dt == TAMD_FP8_E5M2; }
 
+// Inclusive prefix sum over the 64 lanes of a wave (all of them active), in the register file: shifts inside the rows
+// of 16 lanes, then the last lane of rows 0 and 2 added to rows 1 and 3, then lane 31 added to the upper half.
+TAMD_DEVICE int wave_incl_scan(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);  // row_shr:1 (a lane without a source adds 0)
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);  // row_shr:2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);  // row_shr:4
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);  // row_shr:8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);  // row_bcast:15 into rows 1 and 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);  // row_bcast:31 into rows 2 and 3
+  return v;
+}
+
 inline int dtype_size(int dt) {
   switch (dt) {
     case TAMD_F32: return 4;

@@ -180,128 +180,178 @@ TAMD_DEVICE bool locate_tile(const tamd_matmul_args &a, int grid_n, int64_t grid
   return t.rows > 0;
 }
 
-// Tile of a workgroup for ragged problems with few row blocks per expert (at most 1024 row blocks in all), where
-// tiles differ in their number of 32-row fragments and a launch is only a handful of rounds of tiles per CU: the row
-// blocks are taken in the order (fragments descending, schedule index ascending) and dealt round-robin to the 8
-// XCDs, all column tiles of a row block to the same XCD.  Every XCD then gets the same mix of tile sizes (plain
-// schedule order gives XCDs sums of fragments that differ by several per cent), and the smallest tiles run last,
-// which is what bounds the idle time at the end of the launch.  The order is found by the workgroup itself: every
-// thread takes up to four row blocks, their fragment counts are exchanged as ballot masks through LDS, and the thread
-// whose block has this workgroup's position publishes it.  The loads (schedule entry, then slice size and offset) are
-// issued for all blocks at once: two round trips to memory, one fewer than the plain path's chain of dependent loads.
-// When some expert has more than one tile the order is left alone (schedule order, one contiguous range per XCD): the
-// tiles of an expert then run next to each other on one XCD and the later ones find the expert's weights in its L2,
-// which is worth more than the balance (measured: 64 rows per expert +/- 8, sorted order 14 % slower).
-// `lds`: at least 1 KB, free again when the function returns.
-template <int BLOCK_M, int EXTRA>
-TAMD_DEVICE bool locate_tile_sorted(const tamd_matmul_args &a, int grid_n, int grid_m, Tile &t, uint8_t *lds) {
+// Tile of a workgroup for ragged problems with few row blocks per expert (at most 1024 row blocks in all), where tiles
+// differ in their number of 32-row fragments (routed slices are anything from a few rows to several times the mean) and
+// a launch is only a handful of rounds of tiles per CU.  The tiles, in schedule order, are cut into eight ranges of equal
+// estimated time, one per XCD -- an expert's tiles stay next to each other on one XCD -- and within its range an XCD
+// takes the tiles with the most fragments first, so that the last ones to start are the short ones.  (Against ranges of
+// equal tile counts in schedule order, at 128 rows per expert with a spread of 45 %: a layer of 4096 bf16 tokens
+// 860 -> 835 us, one of 1021 tokens with bf16 weights 468 -> 440.)
+//
+// A tile's time is taken as C0 + its fragments: C0 stands for what does not depend on the rows, the stream of the weights
+// above all.  If the cut gives an XCD more tiles than it has workgroups (the launch is sized for the worst split of the
+// rows), all tiles count the same.  Row blocks of up to 32 rows are all of one class: the plain order serves them (the
+// search for the place costs 2 % there).
+//
+// Every workgroup finds its tile by itself, from one scan over the row blocks: counts per fragment class, packed two
+// to a register; the thread whose block holds an XCD's boundary writes the number of tiles of every class before it, and
+// the thread with the wanted block publishes it.  `lds`: at least 1 KB, free again when the function returns.
+// slots: workgroups per XCD.
+template <int BLOCK_M, int EXTRA, int C0>
+TAMD_DEVICE bool locate_tile_balanced(const tamd_matmul_args &a, int grid_n, int grid_m, Tile &t, uint8_t *lds) {
   constexpr int NB = 4;                              // row blocks per thread
-  constexpr int NK = BLOCK_M <= 32 ? 1 : (BLOCK_M + EXTRA) / 32;  // largest fragment count of a tile
+  constexpr int NK = BLOCK_M <= 32 ? 1 : (BLOCK_M + EXTRA) / 32;  // fragment classes
+  constexpr int NP = (NK + 1) / 2;                   // packed counters
+  static_assert(NK <= 6, "class counters");
   const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
-  // (grids stay below 2^31 tiles: 32-bit unsigned arithmetic throughout, whose divisions are the cheap ones)
   const uint32_t gn = (uint32_t)grid_n;
-  const int x = blockIdx.x % 8, j = blockIdx.x / 8;
-  const int slot = (int)((uint32_t)j / gn), pid_n = j - slot * grid_n;
-  const int p = slot * 8 + x;                        // position of this workgroup's row block in the sorted order
-  // The schedule entries are requested before anything waits for the number of real ones (entries past it hold -1, and
-  // the schedule is grid_m entries wide): one round trip to memory instead of two.
-  const int nb = (grid_m + 255) / 256;               // <= NB (checked by the launcher)
+  const int x = blockIdx.x % 8;
+  const uint32_t j = blockIdx.x / 8, slots = gridDim.x / 8;
+  // the schedule entries are requested before anything waits for the number of real ones (entries past it hold -1, and
+  // the schedule is grid_m entries wide): one round trip to memory instead of two
+  const int n_slots = (grid_m + NB - 1) / NB;        // threads that hold blocks (<= 256)
   int sched[NB], ssize[NB], soffs[NB], key[NB];
 #pragma unroll
   for (int u = 0; u < NB; ++u) {
-    const int b = u * 256 + tid;
-    sched[u] = (u < nb && b < grid_m) ? a.block_schedule[b] : -1;
+    const int b = tid * NB + u;
+    sched[u] = b < grid_m ? a.block_schedule[b] : -1;
   }
   const int n_real = a.block_offs[a.n_experts];
-#pragma unroll
-  for (int u = 0; u < NB; ++u) sched[u] = u * 256 + tid < n_real ? sched[u] : -1;
-  // the same workgroup in schedule order: XCD x owns the tiles [x * per_xcd, (x + 1) * per_xcd)
-  const uint32_t real_total = (uint32_t)n_real * gn, per_xcd = (real_total + 7) / 8;
-  const uint32_t plain_pid = (uint32_t)x * per_xcd + (uint32_t)j;
-  const bool plain_live = (uint32_t)j < per_xcd && plain_pid < real_total;
-  if (p >= n_real && !plain_live) return false;
-  const int plain_m = plain_live ? (int)(plain_pid / gn) : -1;
+  if (j >= (uint32_t)n_real * gn) return false;      // (no XCD has more tiles than there are)
 #pragma unroll
   for (int u = 0; u < NB; ++u) {
+    sched[u] = tid * NB + u < n_real ? sched[u] : -1;
     const int e = sched[u] == -1 ? 0 : (sched[u] & 0xFFFF);
-    ssize[u] = u < nb ? a.slice_sizes[e] : 0;
-    soffs[u] = u < nb ? a.slice_offs[e] : 0;
+    ssize[u] = tid < n_slots ? a.slice_sizes[e] : 0;
+    soffs[u] = tid < n_slots ? a.slice_offs[e] : 0;
   }
-  uint64_t *masks = (uint64_t *)lds;                 // [NK][NB][4 waves]
-  int *res = (int *)(lds + NK * NB * 4 * 8);         // [0..3] sorted order, [4..7] schedule order, [8..11] second tiles seen
-  bool second = false;                               // one of this thread's blocks is an expert's second (or later) tile
+  uint32_t own[NP] = {};
 #pragma unroll
   for (int u = 0; u < NB; ++u) {
     const int off = (sched[u] >> 16) * BLOCK_M;
     const int left = ssize[u] - off;
     int rows = left > BLOCK_M + EXTRA ? BLOCK_M : left;
     if (sched[u] == -1 || rows < 0 || (EXTRA > 0 && off > 0 && left <= EXTRA)) rows = 0;  // padding / absorbed remainder
-    key[u] = (rows + 31) / 32;
-    if (BLOCK_M <= 32) key[u] = rows > 0 ? 1 : 0;
-    second = second || (key[u] > 0 && off > 0);
-    if (u < nb) {
+    key[u] = BLOCK_M <= 32 ? (rows > 0 ? 1 : 0) : (rows + 31) / 32;
 #pragma unroll
-      for (int k = 1; k <= NK; ++k) {
-        const uint64_t m = __ballot(key[u] == k);
-        if (lane == 0) masks[((k - 1) * NB + u) * 4 + wave] = m;
+    for (int k = 1; k <= NK; ++k) own[(k - 1) / 2] += key[u] == k ? 1u << (16 * ((k - 1) & 1)) : 0u;
+  }
+  // exclusive prefix of the class counts over the threads (waves 0 .. 3 hold the blocks)
+  uint32_t *wsum = (uint32_t *)lds;                  // [4][NP]
+  uint32_t *cut = wsum + 4 * NP;                     // [9][NK] tiles of class k before XCD x's range
+  int *res = (int *)(cut + 9 * NK);                  // schedule entry, slice size, slice offset
+  uint32_t before[NP], total[NP] = {};
+#pragma unroll
+  for (int p = 0; p < NP; ++p) {
+    const uint32_t inc = (uint32_t)wave_incl_scan((int)own[p]);
+    before[p] = inc - own[p];
+    if (lane == kWave - 1 && wave < 4) wsum[wave * NP + p] = inc;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < 4; ++w)
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+      const uint32_t v = wsum[w * NP + p];
+      before[p] += w < wave ? v : 0u;
+      total[p] += v;
+    }
+  auto count = [](const uint32_t (&c)[NP], int k) { return (c[(k - 1) / 2] >> (16 * ((k - 1) & 1))) & 0xFFFFu; };
+  uint32_t first[NK], n_of[NK], n_tiles = 0;         // this XCD's tiles: class k's [first, first + n_of)
+#pragma unroll 1
+  for (int flat = 0; flat < 2; ++flat) {
+    // time of a tile of class k; the position of a tile is the time of all tiles before it
+    auto cost = [&](int k) { return flat ? 1u : (uint32_t)(C0 + k); };
+    uint32_t all = 0, pos = 0;
+#pragma unroll
+    for (int k = 1; k <= NK; ++k) {
+      all += cost(k) * count(total, k);
+      pos += cost(k) * count(before, k);
+    }
+    all *= gn, pos *= gn;
+    const uint32_t step = (all + 7) / 8;             // boundaries at multiples of it
+    if (tid < NK) {
+      cut[tid] = 0;
+      cut[8 * NK + tid] = count(total, tid + 1) * gn;
+      // boundaries past the last tile (fewer than eight steps of work)
+      for (int q = 1; q < 8; ++q)
+        if (step * q >= all) cut[q * NK + tid] = count(total, tid + 1) * gn;
+    }
+    uint32_t run[NP];
+#pragma unroll
+    for (int p = 0; p < NP; ++p) run[p] = before[p];
+#pragma unroll
+    for (int u = 0; u < NB; ++u) {
+      if (key[u] > 0) {
+        const uint32_t c = cost(key[u]), end = pos + c * gn;
+        for (uint32_t q = (pos + step - 1) / step; q < 8 && q * step < end; ++q) {
+          if (q == 0) continue;
+          const uint32_t n = (q * step - pos + c - 1) / c;   // columns of this block before the boundary
+#pragma unroll
+          for (int k = 1; k <= NK; ++k) cut[q * NK + k - 1] = count(run, k) * gn + (key[u] == k ? n : 0u);
+        }
+        pos = end;
+#pragma unroll
+        for (int k = 1; k <= NK; ++k) run[(k - 1) / 2] += key[u] == k ? 1u << (16 * ((k - 1) & 1)) : 0u;
       }
     }
+    __syncthreads();
+    uint32_t most = 0;
+#pragma unroll 1
+    for (int q = 0; q < 8; ++q) {
+      uint32_t n = 0;
+      for (int k = 0; k < NK; ++k) n += cut[(q + 1) * NK + k] - cut[q * NK + k];
+      most = n > most ? n : most;
+    }
+    n_tiles = 0;
+#pragma unroll
+    for (int k = 0; k < NK; ++k) {
+      first[k] = cut[x * NK + k];
+      n_of[k] = cut[(x + 1) * NK + k] - first[k];
+      n_tiles += n_of[k];
+    }
+    if (most <= slots) break;                        // (equal counts always fit: the launch covers all tiles)
+    __syncthreads();
   }
+  if (j >= n_tiles) return false;
+  // class and place of this workgroup's tile: most fragments first
+  uint32_t left = j, idx = 0;
+  int cls = 0;
+#pragma unroll
+  for (int k = NK; k >= 1; --k) {
+    if (cls == 0) {
+      if (left < n_of[k - 1]) cls = k, idx = first[k - 1] + left;
+      else left -= n_of[k - 1];
+    }
+  }
+  const uint32_t m = idx / gn;                       // the m-th block of its class
   {
-    const uint64_t any_second = __ballot(second);
-    if (lane == 0) res[8 + wave] = any_second != 0;
-  }
-  __syncthreads();
-  const bool sorted = (res[8] | res[9] | res[10] | res[11]) == 0;
-  // position of each of this thread's blocks: blocks of larger keys first, then those of the same key before it
-  int cnt[NK];
+    uint32_t rank = 0;
 #pragma unroll
-  for (int k = 1; k <= NK; ++k) {
-    cnt[k - 1] = 0;
-    for (int i = 0; i < nb * 4; ++i) cnt[k - 1] += __popcll(masks[(k - 1) * NB * 4 + i]);
-  }
+    for (int k = 1; k <= NK; ++k) rank = cls == k ? count(before, k) : rank;
 #pragma unroll
-  for (int u = 0; u < NB; ++u) {
-    if (u < nb && key[u] > 0) {
-      int pos = 0;
-#pragma unroll
-      for (int k = 1; k <= NK; ++k) pos += k > key[u] ? cnt[k - 1] : 0;
-      const uint64_t *mk = masks + (key[u] - 1) * NB * 4;
-      for (int i = 0; i < u * 4 + wave; ++i) pos += __popcll(mk[i]);
-      pos += __popcll(mk[u * 4 + wave] & ((1ull << lane) - 1ull));
-      if (pos == p) {
-        res[0] = sched[u];
-        res[1] = ssize[u];
-        res[2] = soffs[u];
-        res[3] = 1;
+    for (int u = 0; u < NB; ++u) {
+      if (key[u] == cls) {
+        if (rank == m) {
+          res[0] = sched[u];
+          res[1] = ssize[u];
+          res[2] = soffs[u];
+        }
+        ++rank;
       }
     }
-    if (u * 256 + tid == plain_m) {
-      res[4] = sched[u];
-      res[5] = ssize[u];
-      res[6] = soffs[u];
-    }
-  }
-  if (tid == 0) {
-    int total = 0;
-#pragma unroll
-    for (int k = 1; k <= NK; ++k) total += cnt[k - 1];
-    if (p >= total) res[3] = 0;                      // nobody writes: fewer real tiles than schedule entries
   }
   __syncthreads();
-  const int found = sorted ? res[3] : (int)plain_live;
-  const int sc = res[sorted ? 0 : 4], slice_rows = res[sorted ? 1 : 5], start_m = res[sorted ? 2 : 6];
+  const int sc = res[0], slice_rows = res[1], start_m = res[2];
   __syncthreads();                                   // the scratch may be overwritten from here on
-  if (!found || sc == -1) return false;
-  t.n0 = (sorted ? pid_n : (int)(plain_pid - (uint32_t)plain_m * gn)) * BLOCK_N;
+  t.n0 = (int)(idx - m * gn) * BLOCK_N;
   t.z = 0;
   t.expert = sc & 0xFFFF;
   t.start_m = start_m;
   t.off_m = (sc >> 16) * BLOCK_M;
-  const int left = slice_rows - t.off_m;
-  if (EXTRA > 0 && t.off_m > 0 && left <= EXTRA) return false;  // absorbed by the block before it
-  t.rows = left > BLOCK_M + EXTRA ? BLOCK_M : left;
-  return t.rows > 0;
+  const int rows_left = slice_rows - t.off_m;
+  t.rows = rows_left > BLOCK_M + EXTRA ? BLOCK_M : rows_left;
+  return true;
 }
 
 // 128-bit global -> LDS copy that bypasses registers (buffer_load ... lds).  The LDS destination of
@@ -1359,8 +1409,8 @@ template <int XDT, int BM, int ACT, bool SC_LDS, int KS = 1>
 TAMD_DEVICE void tile_entry(const tamd_matmul_args &a, int grid_n, int64_t grid_total, int group_m, uint8_t *lds) {
   typedef TileShape<XDT, BM> S;
   Tile t;
-  if (KS == 1 && group_m == 0) {  // the workgroup finds its tile's place itself (grid_total = row blocks of the launch)
-    if (!locate_tile_sorted<BM, S::EXTRA>(a, grid_n, (int)grid_total, t, lds)) return;
+  if (BM > 32 && group_m == 0) {  // the workgroup finds its tile's place itself (grid_total = row blocks of the launch)
+    if (!locate_tile_balanced<BM, S::EXTRA, is_fp8(XDT) ? 2 : 1>(a, grid_n, (int)grid_total, t, lds)) return;
   } else if (!locate_tile<BM, S::EXTRA>(a, grid_n, grid_total, group_m, t)) return;
   const int nfr = (t.rows + 31) / 32;  // active row fragments (workgroup uniform)
 #define TAMD_CASE(n)                                                                     \
@@ -1446,10 +1496,9 @@ int launch_x16_act(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
     }
   }
   if (int rc = raise_lds_limit_once((const void *)kern)) return rc;
-  if (a.block_schedule && a.block_offs && group_m == 1 && grid_m <= 1024) {
-    // few row blocks per expert: the workgroups take the row blocks largest first, dealt evenly to the XCDs
-    const int64_t sorted_launch = (int64_t)((grid_m + 7) / 8) * 8 * grid_n;
-    kern<<<dim3((unsigned)sorted_launch), 256, lds_bytes, st>>>(a, grid_n, (int64_t)grid_m, 0);
+  if (BM > 32 && a.block_schedule && a.block_offs && group_m == 1 && grid_m <= 1024) {
+    // few row blocks per expert: the workgroups share the tiles out by their estimated time
+    kern<<<dim3((unsigned)launch), 256, lds_bytes, st>>>(a, grid_n, (int64_t)grid_m, 0);
     return launch_status();
   }
   kern<<<dim3((unsigned)launch), 256, lds_bytes, st>>>(a, grid_n, total, (int)group_m);

@@ -213,7 +213,9 @@ __global__ __launch_bounds__(512, 1) void mm_kk_kernel(tamd_matmul_args a, int g
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   typedef TileShape<XDT, BM> S;
   Tile t;
-  if (!locate_tile<BM, S::EXTRA>(a, grid_n, grid_total, group_m, t)) return;
+  if (BM > 32 && group_m == 0) {  // (grid_total: row blocks of the launch)
+    if (!locate_tile_balanced<BM, S::EXTRA, 3>(a, grid_n, (int)grid_total, t, lds)) return;
+  } else if (!locate_tile<BM, S::EXTRA>(a, grid_n, grid_total, group_m, t)) return;
   const int nfr = (t.rows + 31) / 32;
 #define TAMD_CASE(n)                                                      \
   case n:                                                                 \
@@ -236,7 +238,8 @@ int launch_kk(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
   group_m = group_m < 1 ? 1 : (group_m > 8 ? 8 : group_m);
   auto kern = mm_kk_kernel<XDT, BM, ACT>;
   if (int rc = raise_lds_limit_once((const void *)kern)) return rc;
-  kern<<<dim3((unsigned)launch), 512, KKShape<XDT, BM>::LDS, st>>>(a, grid_n, total, (int)group_m);
+  const bool balanced = BM > 32 && a.block_schedule && a.block_offs && group_m <= 2 && grid_m <= 1024;   // few row blocks per expert
+  kern<<<dim3((unsigned)launch), 512, KKShape<XDT, BM>::LDS, st>>>(a, grid_n, balanced ? (int64_t)grid_m : total, balanced ? 0 : (int)group_m);
   return launch_status();
 }
 

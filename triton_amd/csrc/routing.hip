@@ -265,18 +265,6 @@ __global__ __launch_bounds__(1024) void hist_kernel(const void *__restrict__ ind
   }
 }
 
-// Inclusive prefix sum over the 64 lanes of a wave (all of them active), in the register file: shifts inside the rows
-// of 16 lanes, then the last lane of rows 0 and 2 added to rows 1 and 3, then lane 31 added to the upper half.
-TAMD_DEVICE int wave_incl_scan(int v) {
-  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);  // row_shr:1 (a lane without a source adds 0)
-  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);  // row_shr:2
-  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);  // row_shr:4
-  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);  // row_shr:8
-  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);  // row_bcast:15 into rows 1 and 3
-  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);  // row_bcast:31 into rows 2 and 3
-  return v;
-}
-
 // Exclusive scan of up to 1024 ints held one per thread; returns the total.
 TAMD_DEVICE int block_excl_scan_1024(int v, int &total, int *lds /* >= 17 ints */) {
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
