@@ -183,6 +183,70 @@ __global__ __launch_bounds__((NCW + NC + 2) * 64, 1) void mm_stream16_kernel(tam
                                                            : (a.bias_dtype == TAMD_BF16 ? bits_to_f32(raw << 16)
                                                                                         : f16_bits_to_f32((uint16_t)raw)));
     };
+    // Outputs of the usual 16-bit type without flexpoint scales, stored through 32-bit offsets (an offset out of range drops
+    // the row).  The finishing waves share their SIMDs with compute waves and every wave meets at the barrier of each
+    // unit: with every output type decided per element their code was what a unit of two outputs per lane waited for
+    // (2880 x 2880, 105 experts: 94 -> 77 us; SwiGLU 2880 x 5760: 146 -> 140 us).
+    constexpr int FAST = A8 ? TAMD_BF16 : XDT;
+    const bool fast = a.y_dtype == FAST && !a.y_expected_scale && !a.y_actual_scale && epilogue_is_regular<ACT>(a) &&
+                      (a.block_schedule || (int64_t)a.n_experts * a.y_stride_z * 2 < (int64_t)0x7FFFFF00);
+    if (fast) {
+      constexpr uint32_t kDrop = 0x80000000u;
+      uint32_t r_off = kDrop, q_off = kDrop;   // byte offset of the row: current block, unit being finished
+      const uint32_t z_pitch = (uint32_t)a.y_stride_z * 2u, m_pitch = (uint32_t)a.y_stride_m * 2u;
+      const float alpha = a.out_alpha, act_alpha = a.act_alpha, act_limit = a.act_limit;
+      const bool scattered = a.scatter_indx != nullptr, has_beta = a.betas != nullptr, has_gamma = a.gammas != nullptr;
+      const __amdgpu_buffer_rsrc_t ry = __builtin_amdgcn_make_buffer_rsrc(a.y, 0, 0x7FFFFFFF, 0x00020000);
+      auto finish_fast = [&](int buf) {
+        const float *rbuf = red + buf * (NCW * 256) + red_idx;
+        float s0 = (rbuf[0] + rbuf[256]) + (rbuf[512] + rbuf[768]);
+        float s1 = (rbuf[4] + rbuf[260]) + (rbuf[516] + rbuf[772]);
+        if constexpr (NCW == 8) {
+          s0 += (rbuf[1024] + rbuf[1280]) + (rbuf[1536] + rbuf[1792]);
+          s1 += (rbuf[1028] + rbuf[1284]) + (rbuf[1540] + rbuf[1796]);
+        }
+        const float v0 = (s0 * flex + p_bias0 * p_beta) * alpha;
+        const float v1 = (s1 * flex + p_bias1 * p_beta) * alpha;
+        if constexpr (SW) {
+          const float o = swiglu_fast(v0, v1, act_alpha, act_limit, has_limit) * p_gamma;
+          const uint32_t bits = FAST == TAMD_BF16 ? f32_to_bf16_bits(o) : f32_to_f16_bits(o);
+          __builtin_amdgcn_raw_buffer_store_b16((uint16_t)bits, ry, (int)(q_off + (uint32_t)p_col0 + (uint32_t)pc * 2u), 0, 0);
+        } else {
+          const f32x2_t o = {v0 * p_gamma, v1 * p_gamma};
+          uint32_t bits;
+          if constexpr (FAST == TAMD_BF16) bits = __builtin_bit_cast(uint32_t, __builtin_convertvector(o, bf16x2_t));
+          else bits = __builtin_bit_cast(uint32_t, __builtin_convertvector(o, f16x2_t));
+          __builtin_amdgcn_raw_buffer_store_b32(bits, ry, (int)(q_off + (uint32_t)p_col0 * 2u + (uint32_t)pc * 4u), 0, 0);
+        }
+      };
+      int slot = 0;
+#pragma unroll 1
+      for (int s = 0; s < total_stages; ++s) {
+        __syncthreads();  // the partial sums of stage s - 1 and the bias of stage s are visible
+        if (s > 0) finish_fast((s - 1) & 1);
+        if (c_blk < blk0 || c_cg == n_cg) {
+          if (c_cg == n_cg) c_cg = 0;
+          Block cb;
+          get_block(++c_blk, cb);
+          const bool rv = er < cb.rows;
+          const int erow = cb.row0 + (rv ? er : 0);
+          row_beta = (has_beta && rv) ? a.betas[erow] : 1.0f;
+          row_gamma = (has_gamma && rv) ? a.gammas[erow] : 1.0f;
+          const int dst = scattered ? a.scatter_indx[erow] : erow;
+          r_off = rv && dst >= 0 ? (uint32_t)cb.z * z_pitch + (uint32_t)dst * m_pitch : kDrop;
+        }
+        // this unit's bias and row data travel to the next iteration
+        const uint2 braw = *(const uint2 *)(lds + slot * S::STAGE + S::CODE_BYTES + S::SC_BYTES + pc * 8);
+        p_bias0 = to_f32(braw.x), p_bias1 = to_f32(braw.y);
+        p_beta = row_beta, p_gamma = row_gamma, q_off = r_off;
+        p_col0 = c_cg * 16;
+        ++c_cg;
+        slot = slot + 1 == S::RING ? 0 : slot + 1;
+      }
+      __syncthreads();
+      finish_fast((total_stages - 1) & 1);
+      return;
+    }
     const int osz = a.y_dtype == TAMD_F32 ? 4 : (is_fp8(a.y_dtype) ? 1 : 2);
     auto narrow = [&](float v) -> uint32_t {  // one output value as 8 / 16 bits
       return a.y_dtype == TAMD_BF16 ? f32_to_bf16_bits(v) & 0xFFFFu
