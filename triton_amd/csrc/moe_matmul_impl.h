@@ -189,17 +189,19 @@ TAMD_DEVICE bool locate_tile(const tamd_matmul_args &a, int grid_n, int64_t grid
 // 860 -> 835 us, one of 1021 tokens with bf16 weights 468 -> 440.)
 //
 // A tile's time is taken as C0 + its fragments: C0 stands for what does not depend on the rows, the stream of the weights
-// above all.  If the cut gives an XCD more tiles than it has workgroups (the launch is sized for the worst split of the
-// rows), all tiles count the same.  Row blocks of up to 32 rows are all of one class: the plain order serves them (the
+// above all.  All tiles count the same if the cut gives an XCD more tiles than it has workgroups (the launch is sized for
+// the worst split of the rows), and where the tiles are at most 1.5 times the places on the chip (256 CUs x PER_CU): an
+// XCD with a tile more than its places then takes a round more (450 rows over 16 f16 experts: 186 us by time, 176 by
+// number).  Row blocks of up to 32 rows are all of one class: the plain order serves them (the
 // search for the place costs 2 % there).
 //
 // Every workgroup finds its tile by itself, from one scan over the row blocks: counts per fragment class, packed two
 // to a register; the thread whose block holds an XCD's boundary writes the number of tiles of every class before it, and
 // the thread with the wanted block publishes it.  `lds`: at least 1 KB, free again when the function returns.
 // slots: workgroups per XCD.
-template <int BLOCK_M, int EXTRA, int C0>
+template <int BLOCK_M, int EXTRA, int C0, int PER_CU>
 TAMD_DEVICE bool locate_tile_balanced(const tamd_matmul_args &a, int grid_n, int grid_m, Tile &t, uint8_t *lds) {
-  constexpr int NB = 4;                              // row blocks per thread
+  constexpr int NB = 4;                              // row blocks per thread, at most
   constexpr int NK = BLOCK_M <= 32 ? 1 : (BLOCK_M + EXTRA) / 32;  // fragment classes
   constexpr int NP = (NK + 1) / 2;                   // packed counters
   static_assert(NK <= 6, "class counters");
@@ -209,21 +211,21 @@ TAMD_DEVICE bool locate_tile_balanced(const tamd_matmul_args &a, int grid_n, int
   const uint32_t j = blockIdx.x / 8, slots = gridDim.x / 8;
   // the schedule entries are requested before anything waits for the number of real ones (entries past it hold -1, and
   // the schedule is grid_m entries wide): one round trip to memory instead of two
-  const int n_slots = (grid_m + NB - 1) / NB;        // threads that hold blocks (<= 256)
+  const int nb = (grid_m + 255) / 256;               // thread t < 256 holds the blocks nb t .. nb t + nb - 1
   int sched[NB], ssize[NB], soffs[NB], key[NB];
 #pragma unroll
   for (int u = 0; u < NB; ++u) {
-    const int b = tid * NB + u;
-    sched[u] = b < grid_m ? a.block_schedule[b] : -1;
+    const int b = tid * nb + u;
+    sched[u] = u < nb && tid < 256 && b < grid_m ? a.block_schedule[b] : -1;
   }
   const int n_real = a.block_offs[a.n_experts];
   if (j >= (uint32_t)n_real * gn) return false;      // (no XCD has more tiles than there are)
 #pragma unroll
   for (int u = 0; u < NB; ++u) {
-    sched[u] = tid * NB + u < n_real ? sched[u] : -1;
+    sched[u] = tid * nb + u < n_real ? sched[u] : -1;
     const int e = sched[u] == -1 ? 0 : (sched[u] & 0xFFFF);
-    ssize[u] = tid < n_slots ? a.slice_sizes[e] : 0;
-    soffs[u] = tid < n_slots ? a.slice_offs[e] : 0;
+    ssize[u] = u < nb ? a.slice_sizes[e] : 0;
+    soffs[u] = u < nb ? a.slice_offs[e] : 0;
   }
   uint32_t own[NP] = {};
 #pragma unroll
@@ -258,8 +260,11 @@ TAMD_DEVICE bool locate_tile_balanced(const tamd_matmul_args &a, int grid_n, int
     }
   auto count = [](const uint32_t (&c)[NP], int k) { return (c[(k - 1) / 2] >> (16 * ((k - 1) & 1))) & 0xFFFFu; };
   uint32_t first[NK], n_of[NK], n_tiles = 0;         // this XCD's tiles: class k's [first, first + n_of)
+  uint32_t live = 0;
+#pragma unroll
+  for (int k = 1; k <= NK; ++k) live += count(total, k);
 #pragma unroll 1
-  for (int flat = 0; flat < 2; ++flat) {
+  for (int flat = 2 * live * gn <= 3u * 256u * PER_CU ? 1 : 0; flat < 2; ++flat) {
     // time of a tile of class k; the position of a tile is the time of all tiles before it
     auto cost = [&](int k) { return flat ? 1u : (uint32_t)(C0 + k); };
     uint32_t all = 0, pos = 0;
@@ -282,13 +287,15 @@ TAMD_DEVICE bool locate_tile_balanced(const tamd_matmul_args &a, int grid_n, int
     for (int p = 0; p < NP; ++p) run[p] = before[p];
 #pragma unroll
     for (int u = 0; u < NB; ++u) {
-      if (key[u] > 0) {
+      if (u < nb && key[u] > 0) {
         const uint32_t c = cost(key[u]), end = pos + c * gn;
-        for (uint32_t q = (pos + step - 1) / step; q < 8 && q * step < end; ++q) {
-          if (q == 0) continue;
-          const uint32_t n = (q * step - pos + c - 1) / c;   // columns of this block before the boundary
+#pragma unroll 1
+        for (uint32_t q = 1; q < 8; ++q) {
+          if (q * step >= pos && q * step < end) {
+            const uint32_t n = (q * step - pos + c - 1) / c;   // columns of this block before the boundary
 #pragma unroll
-          for (int k = 1; k <= NK; ++k) cut[q * NK + k - 1] = count(run, k) * gn + (key[u] == k ? n : 0u);
+            for (int k = 1; k <= NK; ++k) cut[q * NK + k - 1] = count(run, k) * gn + (key[u] == k ? n : 0u);
+          }
         }
         pos = end;
 #pragma unroll
@@ -331,7 +338,7 @@ TAMD_DEVICE bool locate_tile_balanced(const tamd_matmul_args &a, int grid_n, int
     for (int k = 1; k <= NK; ++k) rank = cls == k ? count(before, k) : rank;
 #pragma unroll
     for (int u = 0; u < NB; ++u) {
-      if (key[u] == cls) {
+      if (u < nb && key[u] == cls) {
         if (rank == m) {
           res[0] = sched[u];
           res[1] = ssize[u];
@@ -1410,7 +1417,7 @@ TAMD_DEVICE void tile_entry(const tamd_matmul_args &a, int grid_n, int64_t grid_
   typedef TileShape<XDT, BM> S;
   Tile t;
   if (BM > 32 && group_m == 0) {  // the workgroup finds its tile's place itself (grid_total = row blocks of the launch)
-    if (!locate_tile_balanced<BM, S::EXTRA, is_fp8(XDT) ? 2 : 1>(a, grid_n, (int)grid_total, t, lds)) return;
+    if (!locate_tile_balanced<BM, S::EXTRA, is_fp8(XDT) ? 2 : 1, 2>(a, grid_n, (int)grid_total, t, lds)) return;
   } else if (!locate_tile<BM, S::EXTRA>(a, grid_n, grid_total, group_m, t)) return;
   const int nfr = (t.rows + 31) / 32;  // active row fragments (workgroup uniform)
 #define TAMD_CASE(n)                                                                     \
@@ -1496,8 +1503,10 @@ int launch_x16_act(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
     }
   }
   if (int rc = raise_lds_limit_once((const void *)kern)) return rc;
-  if (BM > 32 && a.block_schedule && a.block_offs && group_m == 1 && grid_m <= 1024) {
-    // few row blocks per expert: the workgroups share the tiles out by their estimated time
+  if (BM > 32 && group_m == 1 && a.block_schedule && a.block_offs && grid_m <= 1024 && a.K >= 1536) {
+    // few row blocks per expert: the workgroups share the tiles out by their estimated time.  (The search for a tile's place
+    // takes about 2 us, which a tile of a short K does not win back: 2482 fp8 rows over 60 experts, K 1024 and 800,
+    // 51.3 us in plain order, 53.9 shared out; K 5152 and 2624, 1728 rows over 32 experts: 266 and 258 us.)
     kern<<<dim3((unsigned)launch), 256, lds_bytes, st>>>(a, grid_n, (int64_t)grid_m, 0);
     return launch_status();
   }

@@ -214,7 +214,7 @@ __global__ __launch_bounds__(512, 1) void mm_kk_kernel(tamd_matmul_args a, int g
   typedef TileShape<XDT, BM> S;
   Tile t;
   if (BM > 32 && group_m == 0) {  // (grid_total: row blocks of the launch)
-    if (!locate_tile_balanced<BM, S::EXTRA, 3>(a, grid_n, (int)grid_total, t, lds)) return;
+    if (!locate_tile_balanced<BM, S::EXTRA, 3, 1>(a, grid_n, (int)grid_total, t, lds)) return;
   } else if (!locate_tile<BM, S::EXTRA>(a, grid_n, grid_total, group_m, t)) return;
   const int nfr = (t.rows + 31) / 32;
 #define TAMD_CASE(n)                                                      \
@@ -238,7 +238,10 @@ int launch_kk(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
   group_m = group_m < 1 ? 1 : (group_m > 8 ? 8 : group_m);
   auto kern = mm_kk_kernel<XDT, BM, ACT>;
   if (int rc = raise_lds_limit_once((const void *)kern)) return rc;
-  const bool balanced = BM > 32 && a.block_schedule && a.block_offs && group_m <= 2 && grid_m <= 1024;   // few row blocks per expert
+  // few row blocks per expert, and tiles enough to even out (2.5 per CU of the worst split): shared out by their time.
+  // With one workgroup on a CU nothing hides the search: 450 rows over 16 f16 experts, 1.5 tiles per CU, 176 us in plain
+  // order and 182 shared out.
+  const bool balanced = BM > 32 && group_m <= 2 && a.block_schedule && a.block_offs && grid_m <= 1024 && total >= 640;
   kern<<<dim3((unsigned)launch), 512, KKShape<XDT, BM>::LDS, st>>>(a, grid_n, balanced ? (int64_t)grid_m : total, balanced ? 0 : (int)group_m);
   return launch_status();
 }
