@@ -932,8 +932,9 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
   // LDS, one byte-sized copy per group (64 rows per instruction, waves 0 and 1; groups past K/32 are not read at
   // all, so nothing beyond a row's own scales is touched)
   const bool x_mx = FP8 && a.x_mx_scale != nullptr;
-  const uint32_t lds_as = lds_base + DA * A_STAGE + DB * B_BYTES;
-  const uint32_t *as_buf = (const uint32_t *)(lds + DA * A_STAGE + DB * B_BYTES);
+  constexpr int AS_AT = DA * A_STAGE + DB * B_BYTES + PS.scr_bytes;
+  const uint32_t lds_as = lds_base + AS_AT;
+  const uint32_t *as_buf = (const uint32_t *)(lds + AS_AT);
   v4i_t ras = rx;
   uint32_t as_off = kOob;
   if (x_mx) {
@@ -1073,8 +1074,8 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
   // stage's 4 as 256 contiguous bytes each (lanes 0-15 / 16-31; the other lanes copy nothing).  Strided layout:
   // one byte-sized copy per group, lane L fetching column L of the strip into dword [group][L]; slow (64 lines
   // touched per copy) and only used when the scales of a tile do not fit LDS.
-  const uint32_t lds_scr = lds_base + DA * A_STAGE + DB * B_BYTES + AS_BYTES;
-  const uint8_t *scr_buf = lds + DA * A_STAGE + DB * B_BYTES + AS_BYTES;
+  const uint32_t lds_scr = lds_base + DA * A_STAGE + DB * B_BYTES;
+  const uint8_t *scr_buf = lds + DA * A_STAGE + DB * B_BYTES;
   uint32_t scr_voff = kOob;
   v4i_t rsc = rw;
   if constexpr (RING) {
@@ -1472,7 +1473,10 @@ int launch_x16_act(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
   // (deep mode is worth a CU to itself: up to 156 KB; otherwise two workgroups have to fit)
   const int sc_in_lds = dense_sc && PIPE_BYTES + sc_bytes <= (DEEP ? 156 : 80) * 1024 && !(is_fp8(XDT) && cdna4);
   constexpr int PLAIN_BYTES = pipe_shape(is_fp8(XDT), false, LDS_ROWS).bytes;   // 16-bit path, scales read from memory
-  size_t lds_bytes = sc_in_lds ? PIPE_BYTES + sc_bytes : (is_fp8(XDT) ? RING_BYTES : PLAIN_BYTES);
+  // (ring mode: the block scales of the activations are the pipeline's last region, left out when there are none)
+  constexpr int RING_AS_BYTES = pipe_shape(is_fp8(XDT), true, LDS_ROWS).as_bytes;
+  size_t lds_bytes = sc_in_lds ? PIPE_BYTES + sc_bytes
+                               : (is_fp8(XDT) ? RING_BYTES - (a.x_mx_scale ? 0 : RING_AS_BYTES) : PLAIN_BYTES);
   void (*kern)(tamd_matmul_args, int, int64_t, int);
   if constexpr (is_fp8(XDT))
     kern = sc_in_lds ? mm_x8_mxfp4_kernel<XDT, BM, ACT, true> : mm_x8_mxfp4_kernel<XDT, BM, ACT, false>;
