@@ -92,3 +92,38 @@ def test_tiles_shared_out_by_their_time(sizes, quantised, device):
         ref[at:at + n] = x.float()[at:at + n] @ w[e].float()
         at += n
     torch.testing.assert_close(y.cpu().float(), ref, rtol=1e-2, atol=2e-2)
+
+
+@pytest.mark.parametrize("M,K,N", [(1, 2064, 72), (8, 4112, 64), (9, 48, 328), (16, 1104, 200), (27, 2096, 136), (70, 6912, 608)])
+@pytest.mark.parametrize("dtype", TYPES)
+def test_few_rows(M, K, N, dtype, device):
+    """Narrow tiles: 8, 16 and 32 row lines, K quarters that end early or hold nothing, a partial strip of columns."""
+    torch.manual_seed(2)
+    x, w, xd, wd = operands((M, K), (K, N), dtype, device)
+    bias = torch.randn(N)
+    pc, sx, sw = config(dtype, device)
+    y = matmul(xd, wd, bias.to(device), precision_config=pc)
+    ref = (x.float() @ w.float()) * (sx * sw) + bias
+    torch.testing.assert_close(y.cpu().float(), ref, rtol=1e-2, atol=2e-2)
+
+
+@pytest.mark.parametrize("M,K,N,ragged", [(13, 4960, 72, False), (59, 5312, 264, False), (40, 8064, 136, False), (1613, 2336, 136, False),
+                                          (6, 5184, 264, True), (40, 4256, 72, True)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_few_rows_of_mxfp4(M, K, N, ragged, dtype, device):
+    """MXFP4 weights and few tiles with a K or N that the streaming kernel does not take: groups of waves share a tile."""
+    from triton_amd.numerics_details.mxfp import downcast_to_mxfp, upcast_from_mxfp
+    torch.manual_seed(3)
+    E = 4 if ragged else 1
+    x = torch.randn(M, K).to(dtype)
+    codes, scales = downcast_to_mxfp((torch.randn(E, K, N, device=device) * 0.1), torch.uint8, axis=1)
+    w = upcast_from_mxfp(codes, scales, torch.float32, axis=1).cpu()
+    pc = PrecisionConfig(b_mx_scale=scales if ragged else scales[0], b_microblock_size=32)
+    if not ragged:
+        y, ref = matmul(x.to(device), codes[0], None, precision_config=pc), x.float() @ w[0]
+    else:
+        sizes = torch.tensor([M - 4, 0, 1, 3], dtype=torch.int32)
+        md = make_ragged_tensor_metadata(sizes.to(device), M)
+        y = matmul(x.to(device), codes, None, md, precision_config=pc)
+        ref = torch.cat([part.float() @ w[e] for e, part in enumerate(x.split(sizes.tolist()))])
+    torch.testing.assert_close(y.cpu().float(), ref, rtol=1e-2, atol=3e-2)

@@ -225,6 +225,150 @@ __global__ __launch_bounds__(512, 1) void mm_kk_kernel(tamd_matmul_args a, int g
 #undef TAMD_CASE
 }
 
+// ---- Few tiles: 32 rows x 64 columns, K split over the workgroup's four waves.
+// A problem of few rows has ceil(N / 256) tiles per row block; with fewer tiles than CUs the chip idles while each tile's
+// K loop streams 256 columns through one CU (10 x 6496 x 3096: 13 tiles of 3.3 MB each, 54 us).  Here a tile is one 64-column
+// strip, and a wave has a quarter of K to itself: its copies go through a ring of its own (three stages of up to 12 KB), so
+// the loop has no barrier; the partial sums meet in LDS, added in the order of the waves.  Bound by the copies a wave can
+// issue (one per 8 lines, about 100 cycles each): NA, the row copies of a stage, follows the tile's rows.
+template <int NA>
+struct NarrowShape {
+  static constexpr int A_LINES = 8 * NA, STAGE = (A_LINES + 64) * 128, RING = 3;
+};
+constexpr int kNarrowLds = 4 * NarrowShape<4>::RING * NarrowShape<4>::STAGE;
+static_assert(kNarrowLds <= 160 * 1024, "one workgroup per CU");
+
+template <int XDT, int NA, int ACT>
+TAMD_DEVICE void run_tile_narrow(const tamd_matmul_args &a, const Tile &t, uint8_t *lds) {
+  typedef Mma<XDT> M;
+  typedef NarrowShape<NA> S;
+  constexpr bool FP8 = KK<XDT>::FP8;
+  constexpr int ESZ = KK<XDT>::ESZ, KS = KK<XDT>::KS, EPC = 16 / ESZ;
+  constexpr int RING = S::RING, STAGE = S::STAGE, NB = 8;
+  constexpr uint32_t kOob = 0x7FFFFFFFu;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
+  const int c32 = lane % 32, h = lane / 32;
+  const int K = a.K, N = a.N;
+  const v4i_t rx = make_rsrc((const uint8_t *)a.x + (int64_t)t.z * a.x_stride_z * ESZ, kOob);
+  const v4i_t rw = make_rsrc((const uint8_t *)a.w + (int64_t)t.expert * a.w_stride_e * ESZ, kOob);
+  uint8_t *ring = lds + wave * (RING * STAGE);
+  const uint32_t ring_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)ring;
+  // the wave's stages: [first, first + n_w) of the problem's n_k, the same number for every wave
+  const int n_k = (K + KS - 1) / KS, n_w = (n_k + 3) / 4, first = wave * n_w;
+  // copy u of an operand moves its lines 8u .. 8u + 7, lane -> (line 8u + lane / 8, slot lane % 8); slot s of line r holds
+  // chunk s ^ ((r >> 1) & 7)
+  const int rin = lane / 8;
+  const int chunk[2] = {(lane % 8) ^ (rin >> 1), (lane % 8) ^ (4 + (rin >> 1))};   // even, odd copies
+  uint32_t a_off[NA], b_off[NB];
+#pragma unroll
+  for (int u = 0; u < NA; ++u) {
+    const int r = u * 8 + rin;
+    const int rr = t.off_m + (r < t.rows ? r : t.rows - 1);
+    const uint32_t src = a.gather_indx ? (uint32_t)a.gather_indx[t.start_m + rr] : (uint32_t)(t.start_m + rr);
+    a_off[u] = r < t.rows ? src * (uint32_t)(a.x_stride_m * ESZ) + chunk[u & 1] * 16 : kOob;
+  }
+#pragma unroll
+  for (int u = 0; u < NB; ++u) {
+    const int p = u * 8 + rin;                          // position 32 f + c holds column 2 c + f
+    const int col = t.n0 + 2 * (p % 32) + p / 32;
+    b_off[u] = col < N ? (uint32_t)col * (uint32_t)(a.w_stride_n * ESZ) + chunk[u & 1] * 16 : kOob;
+  }
+  auto issue = [&](int it, int slot) {   // (chunks past K, and stages past the wave's own, are not read: zeros)
+    const int kb = (first + it) * KS;
+    const uint32_t kill[2] = {it < n_w && kb + chunk[0] * EPC < K ? 0u : kOob, it < n_w && kb + chunk[1] * EPC < K ? 0u : kOob};
+    const uint32_t sa = ring_base + slot * STAGE, sb = sa + S::A_LINES * 128;
+#pragma unroll
+    for (int u = 0; u < NA; ++u) dma16(rx, sa + u * 1024, a_off[u] | kill[u & 1], kb * ESZ);
+#pragma unroll
+    for (int u = 0; u < NB; ++u) dma16(rw, sb + u * 1024, b_off[u] | kill[u & 1], kb * ESZ);
+  };
+  f32x16_t acc[1][NF];
+#pragma unroll
+  for (int f = 0; f < NF; ++f)
+#pragma unroll
+    for (int j = 0; j < 16; ++j) acc[0][f][j] = 0.f;
+  // (rows past the tile's lines repeat earlier ones: their results are not stored)
+  const int a_line = c32 & (S::A_LINES - 1), a_swz = (a_line >> 1) & 7, b_swz = (c32 >> 1) & 7;
+  const int a_lane = a_line * 128, b_lane = (S::A_LINES + c32) * 128;
+#pragma unroll
+  for (int s = 0; s < RING - 1; ++s) issue(s, s);
+  int rd = 0, wr = RING - 1;
+#pragma unroll 1
+  for (int it = 0; it < n_w; ++it) {
+    wait_vmcnt<(RING - 2) * (NA + NB)>();   // copies complete in the order of their requests: stage `it` has landed
+    const uint8_t *buf = ring + rd * STAGE;
+    uint4 av[4], bv[NF][4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      // 16-bit: step c takes chunks c (lanes 0-31) and 4 + c; fp8: steps of two chunks, 4 g + h and 4 g + 2 + h
+      const int ch = FP8 ? 4 * (c >> 1) + 2 * (c & 1) + h : 4 * h + c;
+      av[c] = *(const uint4 *)(buf + a_lane + (ch ^ a_swz) * 16);
+#pragma unroll
+      for (int f = 0; f < NF; ++f) bv[f][c] = *(const uint4 *)(buf + b_lane + f * 4096 + (ch ^ b_swz) * 16);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // everything read so far is in registers: the slot of stage it - 1 is free
+    issue(it + RING - 1, wr);
+    if constexpr (FP8) {
+      constexpr int CBSZ = XDT == TAMD_FP8_E5M2 ? 1 : 0;
+      auto frag = [](const uint4 &lo, const uint4 &hi) {
+        return i32x8_t{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
+      };
+#pragma unroll
+      for (int g = 0; g < 2; ++g)
+#pragma unroll
+        for (int f = 0; f < NF; ++f)
+          acc[0][f] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(frag(av[2 * g], av[2 * g + 1]), frag(bv[f][2 * g], bv[f][2 * g + 1]),
+                                                                    acc[0][f], CBSZ, CBSZ, 0, 0x7F7F7F7F, 0, 0x7F7F7F7F);
+    } else {
+      typedef typename M::frag_t frag_t;
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int f = 0; f < NF; ++f)
+          acc[0][f] = M::mma(__builtin_bit_cast(frag_t, av[c]), __builtin_bit_cast(frag_t, bv[f][c]), acc[0][f]);
+    }
+    rd = rd + 1 == RING ? 0 : rd + 1;
+    wr = wr + 1 == RING ? 0 : wr + 1;
+  }
+  wait_dma();
+  __syncthreads();   // every ring is dead
+  f32x4_t *ex = (f32x4_t *)lds;
+  constexpr int PLANE = NF * 4 * kWave;
+  if (wave > 0) {
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        ex[wave * PLANE + (f * 4 + j) * kWave + lane] =
+            f32x4_t{acc[0][f][4 * j], acc[0][f][4 * j + 1], acc[0][f][4 * j + 2], acc[0][f][4 * j + 3]};
+  }
+  __syncthreads();
+  if (wave > 0) return;
+#pragma unroll
+  for (int w = 1; w < 4; ++w)
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const f32x4_t v = ex[w * PLANE + (f * 4 + j) * kWave + lane];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[0][f][4 * j + e] += v[e];
+      }
+  constexpr int FAST = FP8 ? TAMD_BF16 : XDT;
+  tile_epilogue<1, ACT, FAST, FP8>(kernel_args_late(), t, acc, lds);   // (plane 0 was not used)
+}
+
+template <int XDT, int BM, int ACT>
+__global__ __launch_bounds__(256, 1) void mm_kk_narrow_kernel(tamd_matmul_args a, int grid_n, int64_t grid_total, int group_m) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  Tile t;
+  if (!locate_tile<BM, 0>(a, grid_n, grid_total, group_m, t)) return;
+  t.n0 /= 4;   // 64-column tiles
+  if (t.rows <= 8) run_tile_narrow<XDT, 1, ACT>(a, t, lds);
+  else if (t.rows <= 16) run_tile_narrow<XDT, 2, ACT>(a, t, lds);
+  else run_tile_narrow<XDT, 4, ACT>(a, t, lds);
+}
+
 template <int XDT, int BM, int ACT>
 int launch_kk(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
   const int grid_n = (a.N + BLOCK_N - 1) / BLOCK_N;
@@ -236,6 +380,18 @@ int launch_kk(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
   const int64_t rows_per_slice = a.block_schedule ? a.M / a.n_experts : a.M;
   int64_t group_m = (rows_per_slice + BM - 1) / BM;
   group_m = group_m < 1 ? 1 : (group_m > 8 ? 8 : group_m);
+  if constexpr (BM <= 32) {
+    int cus = 0;
+    if (int rc = cu_count(cus)) return rc;
+    if (total < cus) {
+      const int grid64 = (a.N + 63) / 64;
+      auto narrow = mm_kk_narrow_kernel<XDT, BM, ACT>;
+      if (int rc = raise_lds_limit_once((const void *)narrow)) return rc;
+      const int64_t tiles = (int64_t)grid_m * grid64;
+      narrow<<<dim3((unsigned)((tiles + 7) / 8 * 8)), 256, kNarrowLds, st>>>(a, grid64, tiles, 1);
+      return launch_status();
+    }
+  }
   auto kern = mm_kk_kernel<XDT, BM, ACT>;
   if (int rc = raise_lds_limit_once((const void *)kern)) return rc;
   // few row blocks per expert, and tiles enough to even out (2.5 per CU of the worst split): shared out by their time.
