@@ -1489,7 +1489,7 @@ int launch_x16_act(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
   const int64_t fit = (int64_t)(2.5 * 1024 * 1024) / ((int64_t)BM * a.K * (is_fp8(XDT) ? 1 : 2));
   group_m = group_m > fit ? fit : group_m;
   group_m = group_m < 1 ? 1 : (group_m > 16 ? 16 : group_m);
-  if constexpr (!is_fp8(XDT) && BM == 32) {
+  if constexpr (!is_fp8(XDT) && BM <= 32) {
     // Fewer tiles than CUs: K groups, so that every SIMD of the CUs that do get a tile holds two to four waves
     // (at least two 128-K pairs per group; the groups' pipelines and the tile's scales have to fit one CU's LDS)
     int cus = 0;
@@ -1523,10 +1523,10 @@ int launch_x16_act(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
 // rows -- 256 x 2048 x 4096 runs 55 us as 2 x 16 tiles of 128 rows and 27 us as 8 x 16 tiles of 32.
 inline int dense_block_m(const tamd_matmul_args &a) {
   const int64_t cols = (int64_t)((a.N + BLOCK_N - 1) / BLOCK_N) * a.n_experts;
-  const int cand[3] = {128, 64, 32};
+  const int cand[2] = {128, 64};
   for (int bm : cand)
     if (a.M > bm / 2 && (a.M + bm - 1) / bm * cols >= 256) return bm;
-  return 16;  // too few tiles either way: the smallest block gives the most
+  return 32;  // (one 32-row fragment either way: a block of 16 rows only doubles the tiles)
 }
 // A dense / batched problem of 161 to 256 rows whose 32-row tiles number at most half the CUs and whose K holds at
 // least eight 128-K pairs: faster as 32-row tiles with four K groups each (256 x 2048 x 4096: 13.8 us) than as 16-row
