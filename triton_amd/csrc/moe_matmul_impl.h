@@ -935,6 +935,10 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
   constexpr int AS_AT = DA * A_STAGE + DB * B_BYTES + PS.scr_bytes;
   const uint32_t lds_as = lds_base + AS_AT;
   const uint32_t *as_buf = (const uint32_t *)(lds + AS_AT);
+  // (bytes per copy and row: all four of a stage where rows and K allow aligned dwords, two, or one.  A copy of 64 rows
+  // touches up to 64 lines whatever its width; a layer of 2048 MXFP4 tokens, K 2880, 553 us byte by byte, 544 in pairs)
+  const uint64_t as_at = (uint64_t)(uintptr_t)a.x_mx_scale | (uint64_t)a.x_mx_stride_m | (uint64_t)a.x_mx_stride_z | (uint64_t)G;
+  const int as_w = (as_at & 3) == 0 ? 4 : ((as_at & 1) == 0 ? 2 : 1);
   v4i_t ras = rx;
   uint32_t as_off = kOob;
   if (x_mx) {
@@ -950,16 +954,24 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
   // Copies per request, as the counted waits of the ring loops below see them (a wave's copies complete in the order
   // of their requests): the loops of the issue_* functions run to these numbers and the waits are written in them.
   constexpr int CP_A = NFR;        // issue_a: one copy per row fragment
-  constexpr int CP_AS = 4;         // issue_as: one per 32-K group of the stage (waves that hold rows only)
+  constexpr int CP_AS = 4;         // issue_as: 4 / as_w, one per 32-K group of the stage at most (waves that hold rows only)
   constexpr int CP_B = 4;          // issue_b: four 1 KB pieces
   constexpr int CP_BPAIR = 8;      // issue_b_pair: eight
   constexpr int CP_SC_STRIDED = 4; // issue_sc: one per group with strided scales, one in all when pre-shuffled
   auto issue_as = [&](int it) {
     if (x_mx && wave * 64 < LDS_ROWS) {
+      const uint32_t at = lds_as + a_slot(it) * 4 * AS_ROWS * 4 + wave * 256;   // plane 0; planes are AS_ROWS dwords apart
+      if (as_w == 4) {
+        dma4(ras, at, it * 4 < G ? as_off : kOob, (uint32_t)(it * 4));
+      } else if (as_w == 2) {
 #pragma unroll
-      for (int g4 = 0; g4 < CP_AS; ++g4)
-        dma1(ras, lds_as + (a_slot(it) * 4 + g4) * AS_ROWS * 4 + wave * 256, it * 4 + g4 < G ? as_off : kOob,
-             (uint32_t)(it * 4 + g4));
+        for (int p = 0; p < 2; ++p)
+          dma2(ras, at + p * AS_ROWS * 4, it * 4 + 2 * p < G ? as_off : kOob, (uint32_t)(it * 4 + 2 * p));
+      } else {
+#pragma unroll
+        for (int g4 = 0; g4 < CP_AS; ++g4)
+          dma1(ras, at + g4 * AS_ROWS * 4, it * 4 + g4 < G ? as_off : kOob, (uint32_t)(it * 4 + g4));
+      }
     }
   };
 
@@ -1166,11 +1178,20 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
       const uint8_t *buf = lds + a_slot(it) * A_STAGE;
       fp8_read_frags(buf, 0, af8[0]);
       // A scale operand: lane half h supplies K block h of an MFMA; byte 0 is the group of s = 0, byte 2 of s = 1
+      const uint32_t *as = as_buf + a_slot(it) * 4 * AS_ROWS + c32;
+      if (!x_mx) {
 #pragma unroll
-      for (int i = 0; i < NFR; ++i)
-        sa8[i] = x_mx ? (int)(as_buf[(a_slot(it) * 4 + h) * AS_ROWS + i * 32 + c32] |
-                              (as_buf[(a_slot(it) * 4 + 2 + h) * AS_ROWS + i * 32 + c32] << 16))
-                      : 0x7F7F7F7F;
+        for (int i = 0; i < NFR; ++i) sa8[i] = 0x7F7F7F7F;
+      } else if (as_w == 4) {
+#pragma unroll
+        for (int i = 0; i < NFR; ++i) sa8[i] = (int)(as[i * 32] >> (8 * h));
+      } else if (as_w == 2) {
+#pragma unroll
+        for (int i = 0; i < NFR; ++i) sa8[i] = (int)(((as[i * 32] & 0xFFFFu) | (as[AS_ROWS + i * 32] << 16)) >> (8 * h));
+      } else {
+#pragma unroll
+        for (int i = 0; i < NFR; ++i) sa8[i] = (int)(as[h * AS_ROWS + i * 32] | (as[(2 + h) * AS_ROWS + i * 32] << 16));
+      }
     }
   };
 
@@ -1239,7 +1260,15 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
   if constexpr (RING) {
     // Copies complete in the order of their requests, so a stage waits by count for what it needs and leaves the
     // later requests in flight.
-    const bool as_wave = x_mx && wave * 64 < LDS_ROWS;
+    // copies of activation scales in a request of this wave, and the wait that leaves `base` other copies and them in flight
+    const int n_as = x_mx && wave * 64 < LDS_ROWS ? CP_AS / as_w : 0;
+    auto wait_with_as = [&](auto base_c) {
+      constexpr int base = decltype(base_c)::value;
+      if (n_as == 0) wait_vmcnt<base>();
+      else if (n_as == 1) wait_vmcnt<base + 1>();
+      else if (n_as == 2) wait_vmcnt<base + 2>();
+      else wait_vmcnt<base + CP_AS>();
+    };
     constexpr int NSC = CP_SC_STRIDED;  // scale copies of a stage with strided scales (1 when pre-shuffled)
     if constexpr (PAIRED) {
       // Three activation stages; an even stage s moves the weights of s and s + 1 into registers and requests those of
@@ -1249,7 +1278,7 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
       issue_a(1), issue_as(1);
       for (int it = 0; it < n_ka; it += 2) {
         // in flight at most: the activations of stage it + 1
-        if (as_wave) wait_vmcnt<CP_A + CP_AS>(); else wait_vmcnt<CP_A>();
+        wait_with_as(std::integral_constant<int, CP_A>{});
         __syncthreads();
         load_b(it, Set0{});
         load_b(it + 1, Set1{});
@@ -1262,8 +1291,8 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
         compute(it, Set0{}, Set0{});
         if (it + 1 < n_ka) {
           // in flight at most: everything the even stage requested
-          if (cdna4) { if (as_wave) wait_vmcnt<CP_A + CP_AS + CP_BPAIR + 2>(); else wait_vmcnt<CP_A + CP_BPAIR + 2>(); }
-          else { if (as_wave) wait_vmcnt<CP_A + CP_AS + CP_BPAIR + 2 * NSC>(); else wait_vmcnt<CP_A + CP_BPAIR + 2 * NSC>(); }
+          if (cdna4) wait_with_as(std::integral_constant<int, CP_A + CP_BPAIR + 2>{});
+          else wait_with_as(std::integral_constant<int, CP_A + CP_BPAIR + 2 * NSC>{});
           __syncthreads();
           fp8_read0(it + 1);
           issue_a(it + 3);

@@ -227,7 +227,7 @@ __global__ __launch_bounds__(512, 1) void mm_kk_kernel(tamd_matmul_args a, int g
 
 // ---- Few tiles: 32 rows x 64 columns, K split over the workgroup's four waves.
 // A problem of few rows has ceil(N / 256) tiles per row block; with fewer tiles than CUs the chip idles while each tile's
-// K loop streams 256 columns through one CU (10 x 6496 x 3096: 13 tiles of 3.3 MB each, 54 us).  Here a tile is one 64-column
+// K loop streams 256 columns through one CU (10 x 6496 x 3096: 13 tiles of 3.3 MB each, 54 us; now 19).  Here a tile is one 64-column
 // strip, and a wave has a quarter of K to itself: its copies go through a ring of its own (three stages of up to 12 KB), so
 // the loop has no barrier; the partial sums meet in LDS, added in the order of the waves.  Bound by the copies a wave can
 // issue (one per 8 lines, about 100 cycles each): NA, the row copies of a stage, follows the tile's rows.
@@ -381,10 +381,15 @@ int launch_kk(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
   int64_t group_m = (rows_per_slice + BM - 1) / BM;
   group_m = group_m < 1 ? 1 : (group_m > 8 ? 8 : group_m);
   if constexpr (BM <= 32) {
+    // Narrow tiles where their rounds of a quarter of K, and about eight stages of start and finish each, are less than the
+    // K loop of a wide tile.  (5472 x 5760 and 2880 x 5472, one row for each of 3 experts: layer 132 us wide, 78 narrow; K of
+    // 576, four rows x 7752 columns: 8.3 us wide, 10.2 narrow.)
     int cus = 0;
     if (int rc = cu_count(cus)) return rc;
-    if (total < cus) {
-      const int grid64 = (a.N + 63) / 64;
+    const int grid64 = (a.N + 63) / 64;
+    const int64_t n_k = (a.K + KK<XDT>::KS - 1) / KK<XDT>::KS;
+    const int64_t rounds = ((int64_t)grid_m * grid64 + cus - 1) / cus;
+    if (total < cus && rounds * (n_k + 32) < 4 * n_k) {
       auto narrow = mm_kk_narrow_kernel<XDT, BM, ACT>;
       if (int rc = raise_lds_limit_once((const void *)narrow)) return rc;
       const int64_t tiles = (int64_t)grid_m * grid64;
