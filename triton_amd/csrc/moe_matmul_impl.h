@@ -511,7 +511,28 @@ TAMD_DEVICE void store_actual_scale(float *actual, uint32_t amax, float out_max,
 // them and would otherwise live in scratch memory).
 // Args: tamd_matmul_args, or the same structure read in place from the kernel-argument segment (see kernel_args_late).
 // tab: LDS that belongs to the wave alone, epilogue_table_bytes(NFR).
-constexpr int epilogue_table_bytes(int nfr) { return nfr * 32 * 12; }
+constexpr int epilogue_table_bytes(int nfr) { return nfr * 32 * 16; }
+// Largest magnitude of a group of 32 e4m3 outputs -> its e8m0 byte, the exponent of 2^ceil(log2(m / 448)), without the
+// division: 448 = 1.75 * 2^8, and a float32 above 1.75 * 2^k never rounds down to it when divided, so the exponent goes up
+// where the mantissa exceeds .75.  (Quotients below 2^-126 give 2^-126, those that round to zero give zero, infinity
+// stays; compared with the division for every float32 from zero to infinity.)
+TAMD_DEVICE uint32_t e4m3_group_scale(float m) {
+  const uint32_t b = f32_to_bits(m), e = (b + 0x1FFFFFu) >> 23;
+  const uint32_t finite = b > 224u ? (e > 9u ? e - 8u : 1u) : 0u;
+  return b >= 0x7F800000u ? 255u : finite;
+}
+// Maximum over a lane's aligned group of 32 / NO lanes: inside 16 lanes by moves in the register file (mirrored lanes
+// serve once the blocks of four and eight hold one value), across them through the LDS crossbar.
+template <int NO>
+TAMD_DEVICE float group_max_lanes(float m) {
+  auto with = [&](uint32_t other) { m = __builtin_fmaxf(m, bits_to_f32(other)); };
+  with((uint32_t)__builtin_amdgcn_update_dpp(0, (int)f32_to_bits(m), 0xB1, 0xF, 0xF, true));    // quad_perm [1,0,3,2]
+  with((uint32_t)__builtin_amdgcn_update_dpp(0, (int)f32_to_bits(m), 0x4E, 0xF, 0xF, true));    // quad_perm [2,3,0,1]
+  with((uint32_t)__builtin_amdgcn_update_dpp(0, (int)f32_to_bits(m), 0x141, 0xF, 0xF, true));   // row_half_mirror
+  with((uint32_t)__builtin_amdgcn_update_dpp(0, (int)f32_to_bits(m), 0x140, 0xF, 0xF, true));   // row_mirror
+  if constexpr (NO == 1) with((uint32_t)__shfl_xor((int)f32_to_bits(m), 16));
+  return m;
+}
 
 template <int NFR, int ACT, int YDT, bool ROWSC, bool FLEX, bool MXO = false, typename Args = tamd_matmul_args>
 TAMD_DEVICE void tile_epilogue_t(const Args &a, const Tile &t, f32x16_t (&acc)[NFR][NF], uint8_t *tab) {
@@ -527,7 +548,7 @@ TAMD_DEVICE void tile_epilogue_t(const Args &a, const Tile &t, f32x16_t (&acc)[N
   static_assert(YDT != TAMD_F32, "float32 results take the general epilogue");
   constexpr int osz = is_fp8(YDT) ? 1 : 2;                  // bytes per output
   if (t.n0 + wave * 64 >= N) return;
-  // ---- the wave's row table: [rows] destinations, [rows] betas, [rows] gammas
+  // ---- the wave's row table: [rows] destinations, [rows] betas, [rows] gammas, [rows] destinations of the scales (MXO)
   uint32_t *tab_dst = (uint32_t *)tab;
   float *tab_beta = (float *)tab + NFR * 32, *tab_gamma = (float *)tab + NFR * 64;
 #pragma unroll
@@ -542,8 +563,8 @@ TAMD_DEVICE void tile_epilogue_t(const Args &a, const Tile &t, f32x16_t (&acc)[N
         if (a.gammas) gamma = a.gammas[erow];
       }
       const bool keep = r < t.rows && dst >= 0;
-      if constexpr (MXO) tab_dst[r] = keep ? (uint32_t)dst : kDrop;
-      else tab_dst[r] = keep ? (uint32_t)dst * (uint32_t)(a.y_stride_m * osz) : kDrop;
+      tab_dst[r] = keep ? (uint32_t)dst * (uint32_t)(a.y_stride_m * osz) : kDrop;
+      if constexpr (MXO) tab_dst[NFR * 96 + r] = keep ? (uint32_t)dst * (uint32_t)a.y_mx_stride_m : kDrop;
       if constexpr (ROWSC) {
         tab_beta[r] = beta;
         tab_gamma[r] = gamma;
@@ -580,8 +601,8 @@ TAMD_DEVICE void tile_epilogue_t(const Args &a, const Tile &t, f32x16_t (&acc)[N
   const uint32_t col_off = (uint32_t)out_col0 * (uint32_t)osz, col_kill = out_col0 < n_out ? 0u : kDrop;
   const __amdgpu_buffer_rsrc_t rsc = __builtin_amdgcn_make_buffer_rsrc(
       MXO ? a.y_mx_scale + (int64_t)t.z * a.y_mx_stride_z : nullptr, 0, MXO ? 0x7FFFFFFF : 0, 0x00020000);
-  // one lane per row and group of 32 outputs stores the group's scale
-  const uint32_t sc_kill = ((c32 & (32 / NO - 1)) == 0 && out_col0 < n_out) ? 0u : kDrop;
+  // the scales of four rows go out together: in a group's lanes, lane jj takes row jj's
+  const uint32_t sc_off = ((c32 & (32 / NO - 1)) < 4 && (out_col0 & ~31) < n_out) ? (uint32_t)(out_col0 / 32) : kDrop;
   // four rows of the table at a time, read one step ahead; the scheduling barrier keeps the compiler from reading the
   // whole table up front (registers)
   uint4 next_dst = *(const uint4 *)(tab_dst + h * 4);
@@ -604,13 +625,11 @@ TAMD_DEVICE void tile_epilogue_t(const Args &a, const Tile &t, f32x16_t (&acc)[N
           next_gamma = *(const f32x4_t *)(tab_gamma + r1);
         }
       }
-#pragma unroll
-      for (int jj = 0; jj < 4; ++jj) {
+      auto result = [&](int jj, float (&o)[NO]) {
         const int j = jq * 4 + jj;
         float v[NF];
 #pragma unroll
         for (int f = 0; f < NF; ++f) v[f] = __builtin_fmaf(acc[i][f][j], flex, ROWSC ? bias_a[f] * beta4[jj] : bias_a[f]);
-        float o[NO];
         if constexpr (ACT == TAMD_ACT_SWIGLU) {
           o[0] = swiglu_fast(v[0], v[1], a.act_alpha, a.act_limit, has_limit);
         } else {
@@ -621,27 +640,44 @@ TAMD_DEVICE void tile_epilogue_t(const Args &a, const Tile &t, f32x16_t (&acc)[N
 #pragma unroll
           for (int p = 0; p < NO; ++p) o[p] *= gamma4[jj];
         }
-        const uint32_t dst = dst4[jj];
-        if constexpr (MXO) {
-          // MXFP8 output: a group is 32 consecutive output columns of a row = the outputs of one half wave (of
-          // half of it when a lane holds two columns).  max |o| over the group, scale = 2^ceil(log2(max / 448)),
-          // o / scale clamped to +-448; the cast below rounds to nearest even (as tamd_downcast_mxfp does).
-          float m = 0.f;
+      };
+      float out4[4][NO];
+      if constexpr (MXO) {
+        // MXFP8 output: a group is 32 consecutive output columns of a row = the outputs of one half wave (of
+        // half of it when a lane holds two columns).  max |o| over the group, scale = 2^ceil(log2(max / 448)),
+        // o / scale clamped to +-448; the cast below rounds to nearest even (as tamd_downcast_mxfp does).  Four rows at a
+        // time, so that their maxima overlap (67218 rows x 736 -> 544 outputs: 213 us row by row with shuffles through
+        // LDS and two divisions each, 165 now).
+        float m4[4];
 #pragma unroll
-          for (int p = 0; p < NO; ++p) m = __builtin_fmaxf(m, out_col0 + p < n_out ? __builtin_fabsf(o[p]) : 0.f);
+        for (int jj = 0; jj < 4; ++jj) {
+          result(jj, out4[jj]);
+          m4[jj] = 0.f;
 #pragma unroll
-          for (int sh = 16 / NO; sh > 0; sh >>= 1) m = __builtin_fmaxf(m, __shfl_xor(m, sh));
-          const uint32_t sb = (f32_to_bits(m / 448.0f) + 0x007FFFFFu) & 0x7F800000u;
-          const float ds = bits_to_f32(sb);
-          const float qs = ds == 0.f ? 0.f : 1.0f / ds;
+          for (int p = 0; p < NO; ++p) m4[jj] = __builtin_fmaxf(m4[jj], out_col0 + p < n_out ? __builtin_fabsf(out4[jj][p]) : 0.f);
+        }
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj) m4[jj] = group_max_lanes<NO>(m4[jj]);
+        uint32_t my_scale = 0;
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj) {
+          const uint32_t se = e4m3_group_scale(m4[jj]);
+          const float qs = bits_to_f32(se == 0u || se == 255u ? 0u : (254u - se) << 23);   // 1 / 2^(se - 127)
 #pragma unroll
           for (int p = 0; p < NO; ++p) {
-            const float q = o[p] * qs;
-            o[p] = q != q ? q : __builtin_fminf(__builtin_fmaxf(q, -448.0f), 448.0f);
+            const float q = out4[jj][p] * qs;
+            out4[jj][p] = q != q ? q : __builtin_fminf(__builtin_fmaxf(q, -448.0f), 448.0f);
           }
-          __builtin_amdgcn_raw_buffer_store_b8((uint8_t)(sb >> 23), rsc,
-                                               (int)((dst & kDrop) | sc_kill | (dst * (uint32_t)a.y_mx_stride_m + out_col0 / 32)), 0, 0);
+          my_scale = (c32 & 3) == jj ? se : my_scale;
         }
+        const uint32_t sdst = tab_dst[NFR * 96 + (i * 4 + jq) * 8 + h * 4 + (c32 & 3)];
+        __builtin_amdgcn_raw_buffer_store_b8((uint8_t)my_scale, rsc, (int)(((sdst | sc_off) & kDrop) ? kDrop : sdst + sc_off), 0, 0);
+      }
+#pragma unroll
+      for (int jj = 0; jj < 4; ++jj) {
+        float (&o)[NO] = out4[jj];
+        if constexpr (!MXO) result(jj, o);
+        const uint32_t dst = dst4[jj];
         if constexpr (FLEX) {
           // (selections, no branches: a branch per element breaks the fragment into hundreds of blocks)
           const uint32_t amask = (dst | col_kill) & kDrop ? 0u : track_mask;
@@ -654,7 +690,7 @@ TAMD_DEVICE void tile_epilogue_t(const Args &a, const Tile &t, f32x16_t (&acc)[N
             o[p] = clamp_out ? oc : o[p];
           }
         }
-        const int off = MXO ? (int)((dst & kDrop) | col_kill | (dst * (uint32_t)a.y_stride_m + col_off)) : (int)((dst + col_off) | col_kill);
+        const int off = (int)((dst + col_off) | col_kill);
         if constexpr (osz == 2) {
           if constexpr (NO == 2) __builtin_amdgcn_raw_buffer_store_b32(narrow2(o[0], o[NO - 1]), ry, off, 0, 0);
           else __builtin_amdgcn_raw_buffer_store_b16((uint16_t)narrow(o[0]), ry, off, 0, 0);
