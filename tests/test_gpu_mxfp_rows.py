@@ -62,3 +62,19 @@ def test_widen_rows(rows, row_bytes, device):
                                           _lib.stream_ptr(d.device))
     assert rc == 0
     assert torch.equal(wide.cpu(), want)
+
+
+@pytest.mark.parametrize("shape", [(5, 2080, 1160), (1, 1664, 2616), (2, 96, 264)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_columns_by_tiles_and_one_by_one(shape, dtype, device):
+    """A strided quantised axis: 150 / 125 tiles with partly filled ones, and two sizes with too few tiles; any finite values."""
+    torch.manual_seed(6)
+    x = torch.randn(shape)
+    odd = torch.randint(-2**31, 2**31 - 1, shape, dtype=torch.int64).to(torch.int32).view(torch.float32)
+    x = torch.where(torch.rand(shape) < 0.02, odd, x).to(dtype)
+    x = torch.where(torch.isfinite(x), x, torch.ones((), dtype=dtype))
+    ref_v, ref_s = downcast_to_mxfp_ref(x, torch.uint8, -2, "up")
+    v, s = downcast_to_mxfp(x.to(device), torch.uint8, -2)
+    assert torch.equal(s.cpu(), ref_s) and torch.equal(v.cpu(), ref_v)
+    back = upcast_from_mxfp(v, s, dtype, -2).cpu().float()
+    assert torch.equal(back, upcast_from_mxfp_ref(ref_v, ref_s, dtype, -2).float())

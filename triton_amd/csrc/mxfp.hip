@@ -646,6 +646,18 @@ __global__ __launch_bounds__(256) void upcast_cols_tile_kernel(
   }
 }
 
+// Up to how many tiles a tensor whose quantised axis is strided goes to the kernels of one column per thread instead of the tile
+// kernels.  A tile is 131072 elements to a workgroup whose passes follow one another, so that one round of tiles takes the
+// same time for few of them as for 256: 15 to 22 us to quantise, 8 to 11 to dequantise; the column kernels have 64 times the
+// workgroups and take about 4 us and 1 us per million elements.  Quantising float32 [1, 1760, 3000] (48 tiles) 18.6 us by
+// tiles, 9.2 by columns, [1, 2880, 5760] (135) 22.0 and 18.7; bf16 [2, 1184, 4328] (102) 16.6 and 13.4, [1, 2880, 5760]
+// (138) 17.5 and 19.0.  Dequantising to bf16 [2, 1024, 648] (12) 7.9 and 5.2, [1, 1664, 2616] (44) 8.4 and 9.4; to float32
+// [1, 1760, 3000] (48) 10.9 and 9.7, [5, 1248, 1232] (100) 10.9 and 11.6.
+template <int DT>
+constexpr int64_t kColumnsUpToDown = DT == TAMD_F32 ? 136 : 104;
+template <int DT>
+constexpr int64_t kColumnsUpToUp = DT == TAMD_F32 ? 48 : 24;
+
 // Groups from which a thread of the row kernels takes two: below, the grid would no longer give every SIMD a few waves.
 constexpr int64_t kRowsUnrolled = 64 * 2048;
 
@@ -671,9 +683,10 @@ int launch_downcast(const void *src, int64_t nb, int64_t L, int64_t nr, int64_t 
   if constexpr (QK != QK_E2M1) return TAMD_E_UNSUPPORTED;  // fp8 values: quantised axis contiguous only
   constexpr int NV = 16 / ES;
   bool vec = nr % NV == 0 && aligned(src, 16) && (ssb * ES) % 16 == 0 && (ssl * ES) % 16 == 0;
-  if (vec) {
-    constexpr int CW = kTileCols<DT>, GT = kTileGroups<DT>;
-    int64_t blocks = ((nr + CW - 1) / CW) * ((G + GT - 1) / GT) * nb;
+  constexpr int CW = kTileCols<DT>, GT = kTileGroups<DT>;
+  const int64_t tiles = ((nr + CW - 1) / CW) * ((G + GT - 1) / GT) * nb;
+  if (vec && tiles > kColumnsUpToDown<DT>) {
+    const int64_t blocks = tiles;
     if (blocks > 0x7FFFFFFF) return TAMD_E_UNSUPPORTED;
     if (int rc = raise_lds_limit_once((const void *)downcast_cols_tile_kernel<DT>)) return rc;
     downcast_cols_tile_kernel<DT><<<dim3((unsigned)blocks), 256, kTileLds<DT>, st>>>(src, nb, G, nr, ssb, ssl, vals, vsb, vsr,
@@ -707,9 +720,10 @@ int launch_upcast(const uint8_t *vals, int64_t vsb, int64_t vsr, const uint8_t *
   if constexpr (QK != QK_E2M1) return TAMD_E_UNSUPPORTED;  // fp8 values: quantised axis contiguous only
   constexpr int NV = 16 / ES;
   bool vec = nr % NV == 0 && aligned(dst, 16) && (dsb * ES) % 16 == 0 && (dsl * ES) % 16 == 0;
-  if (vec) {
-    constexpr int CW = kTileCols<DT>, GT = kTileGroups<DT>;
-    int64_t blocks = ((nr + CW - 1) / CW) * ((G + GT - 1) / GT) * nb;
+  constexpr int CW = kTileCols<DT>, GT = kTileGroups<DT>;
+  const int64_t tiles = ((nr + CW - 1) / CW) * ((G + GT - 1) / GT) * nb;
+  if (vec && tiles > kColumnsUpToUp<DT>) {
+    const int64_t blocks = tiles;
     if (blocks > 0x7FFFFFFF) return TAMD_E_UNSUPPORTED;
     if (int rc = raise_lds_limit_once((const void *)upcast_cols_tile_kernel<DT>)) return rc;
     upcast_cols_tile_kernel<DT><<<dim3((unsigned)blocks), 256, kTileLds<DT>, st>>>(vals, vsb, vsr, scales, csb, csr, dst, nb, G,
