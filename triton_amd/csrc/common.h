@@ -53,6 +53,21 @@ TAMD_DEVICE uint32_t f32_to_fp8_bits(float f, int dt) {
   return dt == TAMD_FP8_E5M2 ? f32_to_e5m2_bits(f, false) : f32_to_e4m3_bits(f, false);
 }
 
+// Largest magnitude m of a group of microscaled values -> its e8m0 byte, the exponent of 2^ceil(log2(m / largest value)),
+// without the division: the largest values are 1.5 * 2^2 (e2m1), 1.75 * 2^8 (e4m3) and 1.75 * 2^15 (e5m2), and a float32
+// above 1.5 * 2^k or 1.75 * 2^k never rounds down to 2^k' when divided, so the exponent goes up where the mantissa exceeds
+// .5 or .75.  (Quotients below 2^-126 give 2^-126, those that round to zero -- LEAST is the last such bit pattern -- give
+// zero, infinity stays; compared with the division for every float32 from zero to infinity.)
+template <int DT>
+TAMD_DEVICE uint32_t ceil_scale_byte(float m) {
+  constexpr uint32_t CARRY = DT == TAMD_MXFP4 ? 0x3FFFFFu : 0x1FFFFFu;
+  constexpr uint32_t SHIFT = DT == TAMD_MXFP4 ? 2u : (DT == TAMD_FP8_E4M3 ? 8u : 15u);
+  constexpr uint32_t LEAST = DT == TAMD_MXFP4 ? 3u : (DT == TAMD_FP8_E4M3 ? 224u : 28672u);
+  const uint32_t b = f32_to_bits(m), e = (b + CARRY) >> 23;
+  const uint32_t finite = b > LEAST ? (e > SHIFT + 1u ? e - SHIFT : 1u) : 0u;
+  return b >= 0x7F800000u ? 255u : finite;
+}
+
 // Largest finite value of an output type, and the running |x| maximum kept as float bits so that NaN
 // (above +inf as an integer) survives the maximum (flexpoint.py:119-146 of the reference).
 TAMD_DEVICE float max_finite_of(int dt) {

@@ -512,15 +512,6 @@ TAMD_DEVICE void store_actual_scale(float *actual, uint32_t amax, float out_max,
 // Args: tamd_matmul_args, or the same structure read in place from the kernel-argument segment (see kernel_args_late).
 // tab: LDS that belongs to the wave alone, epilogue_table_bytes(NFR).
 constexpr int epilogue_table_bytes(int nfr) { return nfr * 32 * 16; }
-// Largest magnitude of a group of 32 e4m3 outputs -> its e8m0 byte, the exponent of 2^ceil(log2(m / 448)), without the
-// division: 448 = 1.75 * 2^8, and a float32 above 1.75 * 2^k never rounds down to it when divided, so the exponent goes up
-// where the mantissa exceeds .75.  (Quotients below 2^-126 give 2^-126, those that round to zero give zero, infinity
-// stays; compared with the division for every float32 from zero to infinity.)
-TAMD_DEVICE uint32_t e4m3_group_scale(float m) {
-  const uint32_t b = f32_to_bits(m), e = (b + 0x1FFFFFu) >> 23;
-  const uint32_t finite = b > 224u ? (e > 9u ? e - 8u : 1u) : 0u;
-  return b >= 0x7F800000u ? 255u : finite;
-}
 // Maximum over a lane's aligned group of 32 / NO lanes: inside 16 lanes by moves in the register file (mirrored lanes
 // serve once the blocks of four and eight hold one value), across them through the LDS crossbar.
 template <int NO>
@@ -661,7 +652,7 @@ TAMD_DEVICE void tile_epilogue_t(const Args &a, const Tile &t, f32x16_t (&acc)[N
         uint32_t my_scale = 0;
 #pragma unroll
         for (int jj = 0; jj < 4; ++jj) {
-          const uint32_t se = e4m3_group_scale(m4[jj]);
+          const uint32_t se = ceil_scale_byte<TAMD_FP8_E4M3>(m4[jj]);
           const float qs = bits_to_f32(se == 0u || se == 255u ? 0u : (254u - se) << 23);   // 1 / 2^(se - 127)
 #pragma unroll
           for (int p = 0; p < NO; ++p) {

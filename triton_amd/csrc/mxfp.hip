@@ -69,13 +69,8 @@ constexpr float kInvPow2Q = QK == QK_E2M1 ? 0.25f : (QK == QK_E4M3 ? 1.0f / 256.
 // Returns the multiplier 1/scale and writes the e8m0 byte.
 template <int QK = QK_E2M1>
 TAMD_DEVICE float group_scale(float gmax, int mode, uint32_t &scale_byte) {
-  uint32_t sb;
-  if (mode == TAMD_ROUND_UP) {
-    sb = (f32_to_bits(gmax / kMaxQ<QK>) + 0x007FFFFFu) & 0x7F800000u;
-  } else {
-    sb = f32_to_bits(gmax * kInvPow2Q<QK>) & 0x7F800000u;
-  }
-  scale_byte = sb >> 23;
+  constexpr int DT = QK == QK_E2M1 ? TAMD_MXFP4 : (QK == QK_E4M3 ? TAMD_FP8_E4M3 : TAMD_FP8_E5M2);
+  scale_byte = mode == TAMD_ROUND_UP ? ceil_scale_byte<DT>(gmax) : f32_to_bits(gmax * kInvPow2Q<QK>) >> 23;
   // 1 / 2^(e-127): 2^(127-e), of which the one for e = 254 is a subnormal; 0 for e = 0 (an empty group) and for infinity
   const uint32_t e = scale_byte;
   return bits_to_f32(e == 0u || e == 255u ? 0u : (e == 254u ? 0x00400000u : (254u - e) << 23));
