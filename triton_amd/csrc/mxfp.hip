@@ -66,14 +66,21 @@ constexpr float kMaxQ = QK == QK_E2M1 ? 6.0f : (QK == QK_E4M3 ? 448.0f : 57344.0
 template <int QK>
 constexpr float kInvPow2Q = QK == QK_E2M1 ? 0.25f : (QK == QK_E4M3 ? 1.0f / 256.0f : 1.0f / 32768.0f);
 
+// e8m0 byte of a group with the largest magnitude gmax.
+template <int QK>
+TAMD_DEVICE uint32_t group_scale_byte(float gmax, int mode) {
+  constexpr int DT = QK == QK_E2M1 ? TAMD_MXFP4 : (QK == QK_E4M3 ? TAMD_FP8_E4M3 : TAMD_FP8_E5M2);
+  return mode == TAMD_ROUND_UP ? ceil_scale_byte<DT>(gmax) : f32_to_bits(gmax * kInvPow2Q<QK>) >> 23;
+}
+// 1 / 2^(e-127): 2^(127-e), of which the one for e = 254 is a subnormal; 0 for e = 0 (an empty group) and for infinity
+TAMD_DEVICE float scale_reciprocal(uint32_t e) {
+  return bits_to_f32(e == 0u || e == 255u ? 0u : (e == 254u ? 0x00400000u : (254u - e) << 23));
+}
 // Returns the multiplier 1/scale and writes the e8m0 byte.
 template <int QK = QK_E2M1>
 TAMD_DEVICE float group_scale(float gmax, int mode, uint32_t &scale_byte) {
-  constexpr int DT = QK == QK_E2M1 ? TAMD_MXFP4 : (QK == QK_E4M3 ? TAMD_FP8_E4M3 : TAMD_FP8_E5M2);
-  scale_byte = mode == TAMD_ROUND_UP ? ceil_scale_byte<DT>(gmax) : f32_to_bits(gmax * kInvPow2Q<QK>) >> 23;
-  // 1 / 2^(e-127): 2^(127-e), of which the one for e = 254 is a subnormal; 0 for e = 0 (an empty group) and for infinity
-  const uint32_t e = scale_byte;
-  return bits_to_f32(e == 0u || e == 255u ? 0u : (e == 254u ? 0x00400000u : (254u - e) << 23));
+  scale_byte = group_scale_byte<QK>(gmax, mode);
+  return scale_reciprocal(scale_byte);
 }
 
 TAMD_DEVICE float e2m1_value(uint32_t code) {
@@ -358,8 +365,7 @@ __global__ __launch_bounds__(256) void downcast_cols_tile_kernel(
       bool has_nan = false;
 #pragma unroll
       for (int l = 0; l < 32; l += 2) has_nan |= __builtin_isunordered(elem(l, c), elem(l + 1, c));
-      uint32_t sbyte;
-      float qs = group_scale(mx[c], mode, sbyte);
+      const uint32_t sbyte = group_scale_byte<QK_E2M1>(mx[c], mode);
       uint32_t w[4] = {0, 0, 0, 0};
       if (!has_nan && sbyte - 2u <= 251u) {
         // the usual case: the instruction divides by the scale and packs, 1.5 operations per element
@@ -371,6 +377,7 @@ __global__ __launch_bounds__(256) void downcast_cols_tile_kernel(
           w[j] = e2m1_word_scaled(v, ds);
         }
       } else {
+        const float qs = scale_reciprocal(sbyte);
 #pragma unroll
         for (int l = 0; l < 32; l += 2)
           w[l >> 3] |= e2m1_pair(elem(l, c) * qs, elem(l + 1, c) * qs) << (4 * (l & 7));
