@@ -107,7 +107,7 @@ def test_few_rows(M, K, N, dtype, device):
     torch.testing.assert_close(y.cpu().float(), ref, rtol=1e-2, atol=2e-2)
 
 
-@pytest.mark.parametrize("M,K,N,ragged", [(13, 4960, 72, False), (59, 5312, 264, False), (40, 8064, 136, False), (1613, 2336, 136, False),
+@pytest.mark.parametrize("M,K,N,ragged", [(13, 4960, 72, False), (59, 5312, 264, False), (40, 8064, 136, False), (2, 5856, 1072, False), (1613, 2336, 136, False),
                                           (6, 5184, 264, True), (40, 4256, 72, True)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_few_rows_of_mxfp4(M, K, N, ragged, dtype, device):

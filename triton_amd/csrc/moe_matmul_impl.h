@@ -1551,9 +1551,12 @@ int launch_x16_act(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
     int cus = 0;
     if (int rc = cu_count(cus)) return rc;
     const int64_t pairs = (a.K + KB - 1) / KB;
-    const int ks = total * 2 <= cus && pairs >= 8 ? 4 : (total <= cus && pairs >= 4 ? 2 : 1);
-    const size_t pipe = ks == 4 ? 4 * (size_t)pipe_shape(false, false, LDS_ROWS, true, 4).bytes
-                                : 2 * (size_t)pipe_shape(false, false, LDS_ROWS, true, 2).bytes;
+    // (four groups where they fit beside the scales -- K up to 5632 --, else two)
+    constexpr size_t PIPE4 = 4 * (size_t)pipe_shape(false, false, LDS_ROWS, true, 4).bytes;
+    constexpr size_t PIPE2 = 2 * (size_t)pipe_shape(false, false, LDS_ROWS, true, 2).bytes;
+    const bool four = total * 2 <= cus && pairs >= 8 && PIPE4 + sc_bytes <= 156 * 1024;
+    const int ks = four ? 4 : (total <= cus && pairs >= 4 ? 2 : 1);
+    const size_t pipe = four ? PIPE4 : PIPE2;
     if (ks > 1 && dense_sc && pipe + sc_bytes <= 156 * 1024) {
       void (*kk)(tamd_matmul_args, int, int64_t, int) =
           ks == 4 ? mm_x16_mxfp4_kgroups_kernel<XDT, BM, ACT, 4> : mm_x16_mxfp4_kgroups_kernel<XDT, BM, ACT, 2>;
