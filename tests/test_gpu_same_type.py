@@ -127,3 +127,22 @@ def test_few_rows_of_mxfp4(M, K, N, ragged, dtype, device):
         y = matmul(x.to(device), codes, None, md, precision_config=pc)
         ref = torch.cat([part.float() @ w[e] for e, part in enumerate(x.split(sizes.tolist()))])
     torch.testing.assert_close(y.cpu().float(), ref, rtol=1e-2, atol=3e-2)
+
+
+@pytest.mark.parametrize("M,K,N", [(64, 512, 768), (300, 8208, 264), (7, 4096, 72), (27, 2064, 136)])
+@pytest.mark.parametrize("binades", [0, 6])
+@pytest.mark.parametrize("dtype", [torch.float8_e4m3fn, torch.float8_e5m2])
+def test_fp8_products_are_exact(M, K, N, binades, dtype, device):
+    """fp8 x fp8 as precise as the product of the widened operands: exact products, float32 sums.  Each of at most K additions
+    is off by at most half a unit in the last place of a partial sum, 2^-24 of it, in either direction: sqrt(K) 2^-24 of the
+    result (the MFMAs that take fp8 operands drop parts of the products: 1.5e-5 and 6e-5 at every K)."""
+    torch.manual_seed(4)
+
+    def values(*shape):
+        v = torch.randn(shape) * torch.exp2(torch.randint(-binades, binades + 1, shape).float())
+        return (v * (torch.finfo(dtype).max / v.abs().max())).to(dtype)
+
+    x, w = values(M, K), values(N, K)
+    y = matmul(x.to(device), w.to(device).t(), None, precision_config=PrecisionConfig(out_dtype=torch.float32)).cpu().double()
+    ref = x.double() @ w.double().t()
+    assert float((y - ref).norm() / ref.norm()) <= K ** 0.5 * 2.0 ** -24

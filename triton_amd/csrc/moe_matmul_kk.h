@@ -14,6 +14,13 @@
 // before its products and group 1 after them: a copy instruction holds its wave for about a hundred cycles, and with
 // both groups issuing at the same time the matrix cores idled meanwhile.  The groups' partial sums meet in LDS after the
 // loop, each group finishing one half of the row fragments.
+//
+// fp8 operands stay fp8 up to the registers and are widened there, so that the products are those of the widened operands:
+// exact, with float32 sums.  The MFMAs that take fp8 directly (32x32x16 and the scaled 32x32x64 alike) align the products of a
+// step at the largest one and drop what falls below: measured against 64-bit sums over K 512 .. 8192, they are off by 0.9 to
+// 1.5e-5 of the result (normal operands) and 6e-5 (operands over twelve binades) at every K, the bf16 MFMA by 0.2 to 3e-7.
+// 1024 x 8192 x 8192: 110 us, 1.25 PFLOP/s, which is the rate of large bf16 products on this part; 348 widened in a pass of its
+// own, 67 with the fp8 MFMA.
 #pragma once
 #include "moe_matmul_impl.h"
 
@@ -24,6 +31,29 @@ struct KK {
   static constexpr bool FP8 = is_fp8(XDT);
   static constexpr int ESZ = FP8 ? 1 : 2;
   static constexpr int KS = 128 / ESZ;                 // K per stage
+  typedef Mma<FP8 ? TAMD_BF16 : XDT> M;                // (every fp8 number is a bf16 number)
+  typedef typename M::frag_t frag_t;
+  // MFMA steps that a 16-byte chunk of a row or column feeds, and the operand of step s
+  static constexpr int STEPS = FP8 ? 2 : 1;
+  static TAMD_DEVICE frag_t operand(const uint4 &v, int s) {
+    if constexpr (!FP8) {
+      return __builtin_bit_cast(frag_t, v);
+    } else {
+      const uint32_t w[2] = {s ? v.z : v.x, s ? v.w : v.y};
+      bf16x2_t p[4];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        if constexpr (XDT == TAMD_FP8_E5M2) {
+          p[2 * i] = __builtin_amdgcn_cvt_scalef32_pk_bf16_bf8(w[i], 1.0f, false);
+          p[2 * i + 1] = __builtin_amdgcn_cvt_scalef32_pk_bf16_bf8(w[i], 1.0f, true);
+        } else {
+          p[2 * i] = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w[i], 1.0f, false);
+          p[2 * i + 1] = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w[i], 1.0f, true);
+        }
+      }
+      return frag_t{p[0][0], p[0][1], p[1][0], p[1][1], p[2][0], p[2][1], p[3][0], p[3][1]};
+    }
+  }
 };
 template <int XDT, int BM>
 struct KKShape {
@@ -37,7 +67,8 @@ struct KKShape {
 
 template <int XDT, int NFR, int BM, int ACT>
 TAMD_DEVICE void run_tile_kk(const tamd_matmul_args &a, const Tile &t, uint8_t *lds) {
-  typedef Mma<XDT> M;
+  typedef KK<XDT> O;
+  typedef typename O::frag_t frag_t;
   typedef KKShape<XDT, BM> S;
   constexpr bool FP8 = KK<XDT>::FP8;
   constexpr int ESZ = KK<XDT>::ESZ, KS = KK<XDT>::KS, EPC = 16 / ESZ;
@@ -92,8 +123,8 @@ TAMD_DEVICE void run_tile_kk(const tamd_matmul_args &a, const Tile &t, uint8_t *
 
   const bool live = t.n0 + wave * 64 < N;
   const int swz = (c32 >> 1) & 7;
-  // the group's two 16-byte chunks of a row or column: 16-bit values take two MFMA steps, fp8 one
-  const int slot0 = (FP8 ? (4 * grp + h) : (h * 4 + 2 * grp)) ^ swz, slot1 = (FP8 ? (4 * grp + 2 + h) : (h * 4 + 2 * grp + 1)) ^ swz;
+  // the group's two 16-byte chunks of a row or column
+  const int slot0 = (h * 4 + 2 * grp) ^ swz, slot1 = (h * 4 + 2 * grp + 1) ^ swz;
   const int a_lane = c32 * 128, b_lane = LDS_ROWS * 128 + (wave * 64 + c32) * 128;
   const int n_k = (K + KS - 1) / KS;
 #pragma unroll
@@ -119,27 +150,20 @@ TAMD_DEVICE void run_tile_kk(const tamd_matmul_args &a, const Tile &t, uint8_t *
     }
     if (grp == 0) issue(it + RING - 1, wr);
     if (live) {
-      if constexpr (FP8) {
-        constexpr int CBSZ = XDT == TAMD_FP8_E5M2 ? 1 : 0;
-        auto frag = [](const uint4 &lo, const uint4 &hi) {
-          return i32x8_t{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
-        };
 #pragma unroll
-        for (int i = 0; i < NFR; ++i)
+      for (int c = 0; c < 2; ++c)
 #pragma unroll
-          for (int f = 0; f < NF; ++f)
-            acc[i][f] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(frag(av[i][0], av[i][1]), frag(bv[f][0], bv[f][1]),
-                                                                      acc[i][f], CBSZ, CBSZ, 0, 0x7F7F7F7F, 0, 0x7F7F7F7F);
-      } else {
-        typedef typename M::frag_t frag_t;
+        for (int s = 0; s < O::STEPS; ++s) {
+          frag_t b[NF];
 #pragma unroll
-        for (int s = 0; s < 2; ++s)
+          for (int f = 0; f < NF; ++f) b[f] = O::operand(bv[f][c], s);
 #pragma unroll
-          for (int i = 0; i < NFR; ++i)
+          for (int i = 0; i < NFR; ++i) {
+            const frag_t ai = O::operand(av[i][c], s);
 #pragma unroll
-            for (int f = 0; f < NF; ++f)
-              acc[i][f] = M::mma(__builtin_bit_cast(frag_t, av[i][s]), __builtin_bit_cast(frag_t, bv[f][s]), acc[i][f]);
-      }
+            for (int f = 0; f < NF; ++f) acc[i][f] = O::M::mma(ai, b[f], acc[i][f]);
+          }
+        }
     }
     if (grp == 1) issue(it + RING - 1, wr);
     rd = rd + 1 == RING ? 0 : rd + 1;
@@ -240,7 +264,8 @@ static_assert(kNarrowLds <= 160 * 1024, "one workgroup per CU");
 
 template <int XDT, int NA, int ACT>
 TAMD_DEVICE void run_tile_narrow(const tamd_matmul_args &a, const Tile &t, uint8_t *lds) {
-  typedef Mma<XDT> M;
+  typedef KK<XDT> O;
+  typedef typename O::frag_t frag_t;
   typedef NarrowShape<NA> S;
   constexpr bool FP8 = KK<XDT>::FP8;
   constexpr int ESZ = KK<XDT>::ESZ, KS = KK<XDT>::KS, EPC = 16 / ESZ;
@@ -300,33 +325,21 @@ TAMD_DEVICE void run_tile_narrow(const tamd_matmul_args &a, const Tile &t, uint8
     uint4 av[4], bv[NF][4];
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
-      // 16-bit: step c takes chunks c (lanes 0-31) and 4 + c; fp8: steps of two chunks, 4 g + h and 4 g + 2 + h
-      const int ch = FP8 ? 4 * (c >> 1) + 2 * (c & 1) + h : 4 * h + c;
+      const int ch = 4 * h + c;   // (lanes 0-31 take chunks 0 .. 3, the others 4 .. 7)
       av[c] = *(const uint4 *)(buf + a_lane + (ch ^ a_swz) * 16);
 #pragma unroll
       for (int f = 0; f < NF; ++f) bv[f][c] = *(const uint4 *)(buf + b_lane + f * 4096 + (ch ^ b_swz) * 16);
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // everything read so far is in registers: the slot of stage it - 1 is free
     issue(it + RING - 1, wr);
-    if constexpr (FP8) {
-      constexpr int CBSZ = XDT == TAMD_FP8_E5M2 ? 1 : 0;
-      auto frag = [](const uint4 &lo, const uint4 &hi) {
-        return i32x8_t{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
-      };
 #pragma unroll
-      for (int g = 0; g < 2; ++g)
+    for (int c = 0; c < 4; ++c)
 #pragma unroll
-        for (int f = 0; f < NF; ++f)
-          acc[0][f] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(frag(av[2 * g], av[2 * g + 1]), frag(bv[f][2 * g], bv[f][2 * g + 1]),
-                                                                    acc[0][f], CBSZ, CBSZ, 0, 0x7F7F7F7F, 0, 0x7F7F7F7F);
-    } else {
-      typedef typename M::frag_t frag_t;
+      for (int s = 0; s < O::STEPS; ++s) {
+        const frag_t ai = O::operand(av[c], s);
 #pragma unroll
-      for (int c = 0; c < 4; ++c)
-#pragma unroll
-        for (int f = 0; f < NF; ++f)
-          acc[0][f] = M::mma(__builtin_bit_cast(frag_t, av[c]), __builtin_bit_cast(frag_t, bv[f][c]), acc[0][f]);
-    }
+        for (int f = 0; f < NF; ++f) acc[0][f] = O::M::mma(ai, O::operand(bv[f][c], s), acc[0][f]);
+      }
     rd = rd + 1 == RING ? 0 : rd + 1;
     wr = wr + 1 == RING ? 0 : wr + 1;
   }
