@@ -94,6 +94,36 @@ def test_tiles_shared_out_by_their_time(sizes, quantised, device):
     torch.testing.assert_close(y.cpu().float(), ref, rtol=1e-2, atol=2e-2)
 
 
+@pytest.mark.parametrize("n_experts,most", [(1, 700), (7, 700), (64, 330), (65, 330), (200, 200), (512, 40), (513, 40)])
+@pytest.mark.parametrize("kind", ["bf16", "mxfp4", "fp8 x mxfp4"])
+def test_tiles_of_uneven_experts(n_experts, most, kind, device):
+    """Experts of none to several row blocks, some of them absorbed, one to eight experts per lane and more than fit."""
+    from triton_amd.numerics_details.mxfp import downcast_to_mxfp, upcast_from_mxfp
+    g = torch.Generator().manual_seed(n_experts)
+    K, N = 64, 520
+    sizes = torch.randint(0, most + 1, (n_experts,), generator=g, dtype=torch.int32)
+    sizes[::5] = torch.tensor([0, 128, 160, 161, 32], dtype=torch.int32).repeat(n_experts)[:len(sizes[::5])]
+    M = int(sizes.sum())
+    if M == 0:
+        sizes[0] = M = 129
+    x = torch.randn(M, K, generator=g).to(torch.float8_e4m3fn if kind[0] == "f" else torch.bfloat16)
+    w = (torch.randn(n_experts, K, N, generator=g) * 0.1).to(torch.bfloat16).to(device).transpose(-1, -2).contiguous().transpose(-1, -2)
+    pc = PrecisionConfig(out_dtype=torch.bfloat16)
+    if kind != "bf16":
+        v, s = downcast_to_mxfp(w, torch.uint8, axis=-2)
+        pc.b_mx_scale, pc.b_microblock_size = s, 32
+        dense, w = upcast_from_mxfp(v, s, torch.bfloat16, axis=-2), v
+    else:
+        dense = w
+    md = make_ragged_tensor_metadata(sizes.to(device), M)
+    with scoped_opt_flags_constraints({"block_m": 128}):
+        y = matmul(x.to(device), w, None, md, precision_config=pc).cpu().float()
+    dense, at = dense.cpu().float(), 0
+    for e, n in enumerate(sizes.tolist()):
+        torch.testing.assert_close(y[at:at + n], x[at:at + n].float() @ dense[e], rtol=1e-2, atol=2e-2)
+        at += n
+
+
 @pytest.mark.parametrize("M,K,N", [(1, 2064, 72), (8, 4112, 64), (9, 48, 328), (16, 1104, 200), (27, 2096, 136), (70, 6912, 608)])
 @pytest.mark.parametrize("dtype", TYPES)
 def test_few_rows(M, K, N, dtype, device):

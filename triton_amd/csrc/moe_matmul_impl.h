@@ -180,184 +180,62 @@ TAMD_DEVICE bool locate_tile(const tamd_matmul_args &a, int grid_n, int64_t grid
   return t.rows > 0;
 }
 
-// Tile of a workgroup for ragged problems with few row blocks per expert (at most 1024 row blocks in all), where tiles
-// differ in their number of 32-row fragments (routed slices are anything from a few rows to several times the mean) and
-// a launch is only a handful of rounds of tiles per CU.  The tiles, in schedule order, are cut into eight ranges of equal
-// estimated time, one per XCD -- an expert's tiles stay next to each other on one XCD -- and within its range an XCD
-// takes the tiles with the most fragments first, so that the last ones to start are the short ones.  (Against ranges of
-// equal tile counts in schedule order, at 128 rows per expert with a spread of 45 %: a layer of 4096 bf16 tokens
-// 860 -> 835 us, one of 1021 tokens with bf16 weights 468 -> 440.)
+// Tile of a workgroup for ragged problems whose row blocks absorb remainders (EXTRA > 0) and whose experts have a block or two.
+// The schedule's absorbed blocks do nothing: at 128 rows per expert they are a third of it, and XCD ranges of equal
+// numbers of its tiles leave the XCDs with unequal work (32 experts, 2880 x 2880, 128 bf16 rows each: 98 us, 76 so).  Here the
+// ranges are cut from the blocks that have rows, in expert order; up to `group` blocks of an expert run next to each other on
+// a column tile.  (XCD ranges of equal estimated time with the longest tiles first take 2 us to find and read an expert's
+// weights once per block: 128 experts, 200 rows each, 2880 x 2880: 462 us against 414, fp8 rows 387 against 293 in plain order.
+// Where a launch is one to three rounds of tiles they win up to 7 % (32 experts of 160 bf16 rows, 2880 x 5760: 179 against 190),
+// but over 16 to 128 experts of 40 to 250 rows they lose 6 %.)
 //
-// A tile's time is taken as C0 + its fragments: C0 stands for what does not depend on the rows, the stream of the weights
-// above all.  All tiles count the same if the cut gives an XCD more tiles than it has workgroups (the launch is sized for
-// the worst split of the rows), and where the tiles are at most 1.5 times the places on the chip (256 CUs x PER_CU): an
-// XCD with a tile more than its places then takes a round more (450 rows over 16 f16 experts: 186 us by time, 176 by
-// number).  Row blocks of up to 32 rows are all of one class: the plain order serves them (the
-// search for the place costs 2 % there).
-//
-// Every workgroup finds its tile by itself, from one scan over the row blocks: counts per fragment class, packed two
-// to a register; the thread whose block holds an XCD's boundary writes the number of tiles of every class before it, and
-// the thread with the wanted block publishes it.  `lds`: at least 1 KB, free again when the function returns.
-// slots: workgroups per XCD.
-template <int BLOCK_M, int EXTRA, int C0, int PER_CU>
-TAMD_DEVICE bool locate_tile_balanced(const tamd_matmul_args &a, int grid_n, int grid_m, Tile &t, uint8_t *lds) {
-  constexpr int NB = 4;                              // row blocks per thread, at most
-  constexpr int NK = BLOCK_M <= 32 ? 1 : (BLOCK_M + EXTRA) / 32;  // fragment classes
-  constexpr int NP = (NK + 1) / 2;                   // packed counters
-  static_assert(NK <= 6, "class counters");
-  const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
+// Every wave finds the tile by itself, without LDS or barriers and with one round trip to memory: lane l holds the experts
+// [l n, (l + 1) n), n = ceil(experts / 64) up to kLivePerLane, and a scan over the lanes counts the blocks before them.
+constexpr int kLivePerLane = 8;
+template <int BLOCK_M, int EXTRA>
+TAMD_DEVICE bool locate_tile_live(const tamd_matmul_args &a, int grid_n, int group, Tile &t) {
+  const int lane = threadIdx.x % kWave, E = a.n_experts, n_lane = (E + kWave - 1) / kWave;
   const uint32_t gn = (uint32_t)grid_n;
-  const int x = blockIdx.x % 8;
-  const uint32_t j = blockIdx.x / 8, slots = gridDim.x / 8;
-  // the schedule entries are requested before anything waits for the number of real ones (entries past it hold -1, and
-  // the schedule is grid_m entries wide): one round trip to memory instead of two
-  const int nb = (grid_m + 255) / 256;               // thread t < 256 holds the blocks nb t .. nb t + nb - 1
-  int sched[NB], ssize[NB], soffs[NB], key[NB];
+  int rows[kLivePerLane], offs[kLivePerLane];
 #pragma unroll
-  for (int u = 0; u < NB; ++u) {
-    const int b = tid * nb + u;
-    sched[u] = u < nb && tid < 256 && b < grid_m ? a.block_schedule[b] : -1;
+  for (int u = 0; u < kLivePerLane; ++u) {
+    const int e = lane * n_lane + u;
+    const bool in = u < n_lane && e < E;
+    rows[u] = in ? a.slice_sizes[e] : 0;
+    offs[u] = in ? a.slice_offs[e] : 0;
   }
-  const int n_real = a.block_offs[a.n_experts];
-  if (j >= (uint32_t)n_real * gn) return false;      // (no XCD has more tiles than there are)
+  // (a block that starts past the first needs more than EXTRA rows)
+  auto blocks = [](int n) { return n > BLOCK_M ? (n - EXTRA + BLOCK_M - 1) / BLOCK_M : (n > 0 ? 1 : 0); };
+  int own = 0;
 #pragma unroll
-  for (int u = 0; u < NB; ++u) {
-    sched[u] = tid * nb + u < n_real ? sched[u] : -1;
-    const int e = sched[u] == -1 ? 0 : (sched[u] & 0xFFFF);
-    ssize[u] = u < nb ? a.slice_sizes[e] : 0;
-    soffs[u] = u < nb ? a.slice_offs[e] : 0;
+  for (int u = 0; u < kLivePerLane; ++u) own += blocks(rows[u]);
+  const int incl = wave_incl_scan(own);
+  const uint32_t total = (uint32_t)__builtin_amdgcn_readlane(incl, kWave - 1) * gn;
+  const uint32_t per_xcd = (total + 7) / 8, bx = blockIdx.x;
+  const uint32_t idx = (bx % 8) * per_xcd + bx / 8;
+  if (bx / 8 >= per_xcd || idx >= total) return false;
+  const int m = (int)(idx / gn);                     // the m-th block that has rows
+  int first = incl - own, e = 0, n = 0, off = 0, before = 0;
+  bool here = false;
+#pragma unroll
+  for (int u = 0; u < kLivePerLane; ++u) {
+    const int c = blocks(rows[u]);
+    if (m >= first && m < first + c) here = true, e = lane * n_lane + u, n = rows[u], off = offs[u], before = first;
+    first += c;
   }
-  uint32_t own[NP] = {};
-#pragma unroll
-  for (int u = 0; u < NB; ++u) {
-    const int off = (sched[u] >> 16) * BLOCK_M;
-    const int left = ssize[u] - off;
-    int rows = left > BLOCK_M + EXTRA ? BLOCK_M : left;
-    if (sched[u] == -1 || rows < 0 || (EXTRA > 0 && off > 0 && left <= EXTRA)) rows = 0;  // padding / absorbed remainder
-    key[u] = BLOCK_M <= 32 ? (rows > 0 ? 1 : 0) : (rows + 31) / 32;
-#pragma unroll
-    for (int k = 1; k <= NK; ++k) own[(k - 1) / 2] += key[u] == k ? 1u << (16 * ((k - 1) & 1)) : 0u;
-  }
-  // exclusive prefix of the class counts over the threads (waves 0 .. 3 hold the blocks)
-  uint32_t *wsum = (uint32_t *)lds;                  // [4][NP]
-  uint32_t *cut = wsum + 4 * NP;                     // [9][NK] tiles of class k before XCD x's range
-  int *res = (int *)(cut + 9 * NK);                  // schedule entry, slice size, slice offset
-  uint32_t before[NP], total[NP] = {};
-#pragma unroll
-  for (int p = 0; p < NP; ++p) {
-    const uint32_t inc = (uint32_t)wave_incl_scan((int)own[p]);
-    before[p] = inc - own[p];
-    if (lane == kWave - 1 && wave < 4) wsum[wave * NP + p] = inc;
-  }
-  __syncthreads();
-#pragma unroll
-  for (int w = 0; w < 4; ++w)
-#pragma unroll
-    for (int p = 0; p < NP; ++p) {
-      const uint32_t v = wsum[w * NP + p];
-      before[p] += w < wave ? v : 0u;
-      total[p] += v;
-    }
-  auto count = [](const uint32_t (&c)[NP], int k) { return (c[(k - 1) / 2] >> (16 * ((k - 1) & 1))) & 0xFFFFu; };
-  uint32_t first[NK], n_of[NK], n_tiles = 0;         // this XCD's tiles: class k's [first, first + n_of)
-  uint32_t live = 0;
-#pragma unroll
-  for (int k = 1; k <= NK; ++k) live += count(total, k);
-#pragma unroll 1
-  for (int flat = 2 * live * gn <= 3u * 256u * PER_CU ? 1 : 0; flat < 2; ++flat) {
-    // time of a tile of class k; the position of a tile is the time of all tiles before it
-    auto cost = [&](int k) { return flat ? 1u : (uint32_t)(C0 + k); };
-    uint32_t all = 0, pos = 0;
-#pragma unroll
-    for (int k = 1; k <= NK; ++k) {
-      all += cost(k) * count(total, k);
-      pos += cost(k) * count(before, k);
-    }
-    all *= gn, pos *= gn;
-    const uint32_t step = (all + 7) / 8;             // boundaries at multiples of it
-    if (tid < NK) {
-      cut[tid] = 0;
-      cut[8 * NK + tid] = count(total, tid + 1) * gn;
-      // boundaries past the last tile (fewer than eight steps of work)
-      for (int q = 1; q < 8; ++q)
-        if (step * q >= all) cut[q * NK + tid] = count(total, tid + 1) * gn;
-    }
-    uint32_t run[NP];
-#pragma unroll
-    for (int p = 0; p < NP; ++p) run[p] = before[p];
-#pragma unroll
-    for (int u = 0; u < NB; ++u) {
-      if (u < nb && key[u] > 0) {
-        const uint32_t c = cost(key[u]), end = pos + c * gn;
-#pragma unroll 1
-        for (uint32_t q = 1; q < 8; ++q) {
-          if (q * step >= pos && q * step < end) {
-            const uint32_t n = (q * step - pos + c - 1) / c;   // columns of this block before the boundary
-#pragma unroll
-            for (int k = 1; k <= NK; ++k) cut[q * NK + k - 1] = count(run, k) * gn + (key[u] == k ? n : 0u);
-          }
-        }
-        pos = end;
-#pragma unroll
-        for (int k = 1; k <= NK; ++k) run[(k - 1) / 2] += key[u] == k ? 1u << (16 * ((k - 1) & 1)) : 0u;
-      }
-    }
-    __syncthreads();
-    uint32_t most = 0;
-#pragma unroll 1
-    for (int q = 0; q < 8; ++q) {
-      uint32_t n = 0;
-      for (int k = 0; k < NK; ++k) n += cut[(q + 1) * NK + k] - cut[q * NK + k];
-      most = n > most ? n : most;
-    }
-    n_tiles = 0;
-#pragma unroll
-    for (int k = 0; k < NK; ++k) {
-      first[k] = cut[x * NK + k];
-      n_of[k] = cut[(x + 1) * NK + k] - first[k];
-      n_tiles += n_of[k];
-    }
-    if (most <= slots) break;                        // (equal counts always fit: the launch covers all tiles)
-    __syncthreads();
-  }
-  if (j >= n_tiles) return false;
-  // class and place of this workgroup's tile: most fragments first
-  uint32_t left = j, idx = 0;
-  int cls = 0;
-#pragma unroll
-  for (int k = NK; k >= 1; --k) {
-    if (cls == 0) {
-      if (left < n_of[k - 1]) cls = k, idx = first[k - 1] + left;
-      else left -= n_of[k - 1];
-    }
-  }
-  const uint32_t m = idx / gn;                       // the m-th block of its class
-  {
-    uint32_t rank = 0;
-#pragma unroll
-    for (int k = 1; k <= NK; ++k) rank = cls == k ? count(before, k) : rank;
-#pragma unroll
-    for (int u = 0; u < NB; ++u) {
-      if (u < nb && key[u] == cls) {
-        if (rank == m) {
-          res[0] = sched[u];
-          res[1] = ssize[u];
-          res[2] = soffs[u];
-        }
-        ++rank;
-      }
-    }
-  }
-  __syncthreads();
-  const int sc = res[0], slice_rows = res[1], start_m = res[2];
-  __syncthreads();                                   // the scratch may be overwritten from here on
-  t.n0 = (int)(idx - m * gn) * BLOCK_N;
+  const int src = __builtin_ctzll(__ballot(here));   // (exactly one lane)
+  t.expert = __builtin_amdgcn_readlane(e, src);
+  t.start_m = __builtin_amdgcn_readlane(off, src);
+  const int slice_rows = __builtin_amdgcn_readlane(n, src);
+  const uint32_t local = idx - (uint32_t)__builtin_amdgcn_readlane(before, src) * gn;   // tile of the expert
+  const uint32_t b = (uint32_t)blocks(slice_rows), g = b < (uint32_t)group ? b : (uint32_t)group;
+  const uint32_t gi = local / (g * gn), r = local - gi * g * gn;
+  const uint32_t size = b - gi * g < g ? b - gi * g : g, col = r / size;
+  t.n0 = (int)col * BLOCK_N;
   t.z = 0;
-  t.expert = sc & 0xFFFF;
-  t.start_m = start_m;
-  t.off_m = (sc >> 16) * BLOCK_M;
-  const int rows_left = slice_rows - t.off_m;
-  t.rows = rows_left > BLOCK_M + EXTRA ? BLOCK_M : rows_left;
+  t.off_m = (int)(gi * g + r - col * size) * BLOCK_M;
+  const int left = slice_rows - t.off_m;
+  t.rows = left > BLOCK_M + EXTRA ? BLOCK_M : left;
   return true;
 }
 
@@ -1473,8 +1351,8 @@ template <int XDT, int BM, int ACT, bool SC_LDS, int KS = 1>
 TAMD_DEVICE void tile_entry(const tamd_matmul_args &a, int grid_n, int64_t grid_total, int group_m, uint8_t *lds) {
   typedef TileShape<XDT, BM> S;
   Tile t;
-  if (BM > 32 && group_m == 0) {  // the workgroup finds its tile's place itself (grid_total = row blocks of the launch)
-    if (!locate_tile_balanced<BM, S::EXTRA, is_fp8(XDT) ? 2 : 1, 2>(a, grid_n, (int)grid_total, t, lds)) return;
+  if (S::EXTRA > 0 && group_m < 0) {  // absorbed blocks left out of the count; -group_m blocks of an expert together
+    if (!locate_tile_live<BM, S::EXTRA>(a, grid_n, -group_m, t)) return;
   } else if (!locate_tile<BM, S::EXTRA>(a, grid_n, grid_total, group_m, t)) return;
   const int nfr = (t.rows + 31) / 32;  // active row fragments (workgroup uniform)
 #define TAMD_CASE(n)                                                                     \
@@ -1505,6 +1383,12 @@ __global__ __launch_bounds__(256, 2) void mm_x8_mxfp4_kernel(tamd_matmul_args a,
                                                                  int group_m) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   tile_entry<XDT, BM, ACT, SC_LDS>(a, grid_n, grid_total, group_m, lds);
+}
+
+// Whether a ragged problem takes locate_tile_live: absorbed blocks exist and the experts fit its lanes.
+template <int XDT, int BM>
+bool counts_live_blocks(const tamd_matmul_args &a) {
+  return TileShape<XDT, BM>::EXTRA > 0 && a.block_schedule && a.n_experts <= kWave * kLivePerLane;
 }
 
 template <int XDT, int BM, int ACT>
@@ -1566,13 +1450,8 @@ int launch_x16_act(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
     }
   }
   if (int rc = raise_lds_limit_once((const void *)kern)) return rc;
-  if (BM > 32 && group_m == 1 && a.block_schedule && a.block_offs && grid_m <= 1024 && a.K >= 1536) {
-    // few row blocks per expert: the workgroups share the tiles out by their estimated time.  (The search for a tile's place
-    // takes about 2 us, which a tile of a short K does not win back: 2482 fp8 rows over 60 experts, K 1024 and 800,
-    // 51.3 us in plain order, 53.9 shared out; K 5152 and 2624, 1728 rows over 32 experts: 266 and 258 us.)
-    kern<<<dim3((unsigned)launch), 256, lds_bytes, st>>>(a, grid_n, (int64_t)grid_m, 0);
-    return launch_status();
-  }
+  // (an expert's blocks one after the other: with two workgroups per CU an XCD holds 64 tiles, its column tiles of both)
+  if (counts_live_blocks<XDT, BM>(a) && group_m == 1) group_m = -1;
   kern<<<dim3((unsigned)launch), 256, lds_bytes, st>>>(a, grid_n, total, (int)group_m);
   return launch_status();
 }
