@@ -5,9 +5,11 @@ import torch
 
 from oracle import matmul_ref as MR
 from oracle.mxfp_ref import downcast_to_mxfp_ref
-from triton_amd.matmul import PrecisionConfig, matmul
+from triton_amd import _lib
+from triton_amd.matmul import (FlexCtx, FnSpecs, FusedActivation, InFlexData, OutFlexData, PrecisionConfig, matmul)
 from triton_amd.matmul_details.opt_flags import scoped_opt_flags_constraints
 from triton_amd.numerics_details.mxfp import downcast_to_mxfp
+from triton_amd.swiglu import swiglu_fn
 
 pytestmark = pytest.mark.gpu
 
@@ -30,3 +32,60 @@ def test_output_alignment(block_m, M, N, first, pitch, out_dtype, device):
     untouched = torch.ones_like(flat, dtype=torch.bool)
     untouched[first:first + M * pitch].view(M, pitch)[:, :N] = False
     assert (flat[untouched] == -7.0).all()
+
+
+# half a unit in the last place: 2^-(m + 1) of the value with m stored mantissa bits, and at the smallest exponent
+ROUNDING = {torch.float32: (2.0 ** -24, 0.0), torch.bfloat16: (2.0 ** -8, 0.0), torch.float16: (2.0 ** -11, 2.0 ** -25),
+            torch.float8_e4m3fn: (2.0 ** -4, 2.0 ** -10), torch.float8_e5m2: (2.0 ** -3, 2.0 ** -17)}
+
+
+@pytest.mark.parametrize("M,N,pad", [(33, 202, 0), (160, 201, 0), (97, 202, 1), (5, 66, 2)])
+@pytest.mark.parametrize("swiglu,flex,known", [(False, False, True), (False, True, True), (True, True, True), (False, True, False)])
+@pytest.mark.parametrize("out_dtype", list(ROUNDING))
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float8_e4m3fn])
+def test_output_types(M, N, pad, swiglu, flex, known, out_dtype, dtype, device, monkeypatch):
+    """Every output type, with and without flexpoint scales, in whole and in cut pairs of columns, rows that are dropped, and
+    an output whose number of rows is not given (64-bit addresses)."""
+    if swiglu and N % 2:
+        N += 1
+    if not known:
+        pack = _lib.MatmulArgBag.pack
+
+        def without_rows(bag):
+            bag.y_rows = 0
+            return pack(bag)
+        monkeypatch.setattr(_lib.MatmulArgBag, "pack", without_rows)
+    g = torch.Generator().manual_seed(5)
+    K, n_out = 96, N // 2 if swiglu else N
+    x = torch.randn(M, K, generator=g).to(dtype)
+    bias, gammas = torch.randn(N, generator=g), torch.rand(M, generator=g) + 0.5
+    rv, rs = downcast_to_mxfp_ref(torch.randn(K, N, generator=g) * 0.1, torch.uint8, 0)
+    v, s = (t.to(device).t().contiguous().t() for t in (rv, rs))
+    scatter = torch.randperm(M, generator=g).int()
+    scatter[::9] = -1
+    expected, actual = (torch.full((1,), f, device=device) for f in (0.05, 0.0))
+    fc = FlexCtx(lhs_data=InFlexData(dtype, torch.ones(1, device=device)) if dtype.itemsize == 1 else InFlexData(),
+                 out_data=OutFlexData(out_dtype, expected, actual) if flex else OutFlexData())
+    flat = torch.zeros(M * (n_out + pad), dtype=out_dtype, device=device)
+    flat.view(torch.uint8).fill_(0x35)
+    y = flat.view(M, n_out + pad)[:, :n_out]
+    act = FusedActivation(FnSpecs("swiglu", swiglu_fn, ("alpha", "limit"), reduction_n=2), (1.702, 7.0)) if swiglu else None
+    with scoped_opt_flags_constraints({"block_m": 128 if M > 64 else 32}):
+        matmul(x.to(device), v, bias.to(device), scatter_indx=scatter.to(device), gammas=gammas.to(device), c=y, fused_activation=act,
+               precision_config=PrecisionConfig(b_mx_scale=s, b_microblock_size=32, flex_ctx=fc, out_dtype=out_dtype,
+                                                flexpoint_saturate_inf=True))
+    ref = MR.matmul_ref(x.double(), rv, bias, b_mx_scale=rs, fused_swiglu=(1.702, 7.0) if swiglu else None).double() * gammas[:, None]
+    kept = scatter >= 0
+    if flex:
+        top = torch.finfo(out_dtype).max
+        torch.testing.assert_close(actual.cpu().double(), (ref[kept].abs().max() / top + 1e-30)[None], rtol=1e-3, atol=0.0)
+        ref = (ref / 0.05).clamp(-top, top)
+    rel, least = ROUNDING[out_dtype]
+    got = y.cpu().double()[scatter[kept].long()]
+    # (the sums of 96 products: 2e-4 with the fp8 MFMA, whose products are not exact)
+    bound = (rel + 2e-4) * ref[kept].abs() + least + 2e-4 * ref[kept].abs().mean()
+    assert ((got - ref[kept]).abs() <= bound).all()
+    bytes_ = flat.cpu().view(torch.uint8).view(M, -1)
+    named = torch.zeros(M, dtype=torch.bool)
+    named[scatter[kept].long()] = True
+    assert (bytes_[~named] == 0x35).all() and (bytes_[:, n_out * out_dtype.itemsize:] == 0x35).all()

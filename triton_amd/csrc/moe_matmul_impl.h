@@ -37,6 +37,7 @@ typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef int i32x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x2_t __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 
 constexpr bool is_fp8(int dt) { return dt == TAMD_FP8_E4M3 || dt == TAMD_FP8_E5M2; }
 
@@ -384,9 +385,12 @@ TAMD_DEVICE void store_actual_scale(float *actual, uint32_t amax, float out_max,
 // leave the tile one by one.  (Staging the tile through LDS for 16-byte stores, as before, took a fifth to a
 // quarter of a tile's time: two barriers, a pass of narrow LDS writes and a copy-out between them.)
 //
-// YDT: output type; ROWSC: per-row betas / gammas may be present; FLEX: flexpoint output (expected / actual scale) may be
-// present; MXO: MXFP8 output (a.y_mx_scale).  The element loops must unroll completely (the accumulators are indexed by
-// them and would otherwise live in scratch memory).
+// YDT: output type, or a width whose type is read at run time (kAny8, kAny16; float32 is one of its own); ROWSC: per-row
+// betas / gammas may be present; FLEX: flexpoint output (expected / actual scale) may be present; MXO: MXFP8 output
+// (a.y_mx_scale).  The element loops must unroll completely (the accumulators are indexed by them and would otherwise live in
+// scratch memory).
+// pairs: a lane's two outputs lie whole on one aligned word, which is stored at once (only read by the forms of one width;
+// the others are entered with such outputs).
 // Args: tamd_matmul_args, or the same structure read in place from the kernel-argument segment (see kernel_args_late).
 // tab: LDS that belongs to the wave alone, epilogue_table_bytes(NFR).
 constexpr int epilogue_table_bytes(int nfr) { return nfr * 32 * 16; }
@@ -403,19 +407,20 @@ TAMD_DEVICE float group_max_lanes(float m) {
   return m;
 }
 
+constexpr int kAny16 = 0x100, kAny8 = 0x101;
 template <int NFR, int ACT, int YDT, bool ROWSC, bool FLEX, bool MXO = false, typename Args = tamd_matmul_args>
-TAMD_DEVICE void tile_epilogue_t(const Args &a, const Tile &t, f32x16_t (&acc)[NFR][NF], uint8_t *tab) {
+TAMD_DEVICE void tile_epilogue_t(const Args &a, const Tile &t, f32x16_t (&acc)[NFR][NF], uint8_t *tab, bool pairs = true) {
   const int wave = (threadIdx.x / kWave) & 3, lane = threadIdx.x % kWave;
   const int c32 = lane % 32, h = lane / 32;
   const int N = a.N;
   const int col0 = t.n0 + wave * 64 + c32 * NF;
   constexpr uint32_t kDrop = 0x80000000u;                   // an offset that no descriptor here covers
-  constexpr int ydt = YDT;
+  constexpr bool ANY = YDT == kAny16 || YDT == kAny8 || YDT == TAMD_F32;   // one width
+  const int ydt = ANY ? a.y_dtype : YDT;
   constexpr int NO = ACT == TAMD_ACT_SWIGLU ? NF / 2 : NF;  // outputs per lane per row
   const int n_out = ACT == TAMD_ACT_SWIGLU ? N / 2 : N;
   const int out_col0 = ACT == TAMD_ACT_SWIGLU ? col0 / 2 : col0;
-  static_assert(YDT != TAMD_F32, "float32 results take the general epilogue");
-  constexpr int osz = is_fp8(YDT) ? 1 : 2;                  // bytes per output
+  constexpr int osz = YDT == TAMD_F32 ? 4 : (is_fp8(YDT) || YDT == kAny8 ? 1 : 2);   // bytes per output
   if (t.n0 + wave * 64 >= N) return;
   // ---- the wave's row table: [rows] destinations, [rows] betas, [rows] gammas, [rows] destinations of the scales (MXO)
   uint32_t *tab_dst = (uint32_t *)tab;
@@ -468,6 +473,7 @@ TAMD_DEVICE void tile_epilogue_t(const Args &a, const Tile &t, f32x16_t (&acc)[N
   const __amdgpu_buffer_rsrc_t ry = __builtin_amdgcn_make_buffer_rsrc((uint8_t *)a.y + (int64_t)t.z * a.y_stride_z * osz, 0,
                                                                      0x7FFFFFFF, 0x00020000);
   const uint32_t col_off = (uint32_t)out_col0 * (uint32_t)osz, col_kill = out_col0 < n_out ? 0u : kDrop;
+  const uint32_t col_kill1 = out_col0 + 1 < n_out ? 0u : kDrop;   // (the second output of a pair that N cuts)
   const __amdgpu_buffer_rsrc_t rsc = __builtin_amdgcn_make_buffer_rsrc(
       MXO ? a.y_mx_scale + (int64_t)t.z * a.y_mx_stride_z : nullptr, 0, MXO ? 0x7FFFFFFF : 0, 0x00020000);
   // the scales of four rows go out together: in a group's lanes, lane jj takes row jj's
@@ -482,11 +488,11 @@ TAMD_DEVICE void tile_epilogue_t(const Args &a, const Tile &t, f32x16_t (&acc)[N
   }
 #pragma unroll
   for (int i = 0; i < NFR; ++i) {
-#pragma unroll
+#pragma unroll (ANY ? 1 : 4)
     for (int jq = 0; jq < 4; ++jq) {
       const uint32_t dst4[4] = {next_dst.x, next_dst.y, next_dst.z, next_dst.w};
       const f32x4_t beta4 = next_beta, gamma4 = next_gamma;
-      if (i * 4 + jq + 1 < NFR * 4) {
+      if (ANY || i * 4 + jq + 1 < NFR * 4) {   // (one row past the last: still the table)
         const int r1 = (i * 4 + jq + 1) * 8 + h * 4;
         next_dst = *(const uint4 *)(tab_dst + r1);
         if constexpr (ROWSC) {
@@ -495,7 +501,7 @@ TAMD_DEVICE void tile_epilogue_t(const Args &a, const Tile &t, f32x16_t (&acc)[N
         }
       }
       auto result = [&](int jj, float (&o)[NO]) {
-        const int j = jq * 4 + jj;
+        const int j = ANY ? jj : jq * 4 + jj;
         float v[NF];
 #pragma unroll
         for (int f = 0; f < NF; ++f) v[f] = __builtin_fmaf(acc[i][f][j], flex, ROWSC ? bias_a[f] * beta4[jj] : bias_a[f]);
@@ -549,9 +555,9 @@ TAMD_DEVICE void tile_epilogue_t(const Args &a, const Tile &t, f32x16_t (&acc)[N
         const uint32_t dst = dst4[jj];
         if constexpr (FLEX) {
           // (selections, no branches: a branch per element breaks the fragment into hundreds of blocks)
-          const uint32_t amask = (dst | col_kill) & kDrop ? 0u : track_mask;
 #pragma unroll
           for (int p = 0; p < NO; ++p) {
+            const uint32_t amask = (dst | (ANY && p == 1 ? col_kill1 : col_kill)) & kDrop ? 0u : track_mask;
             const uint32_t b = f32_to_bits(o[p]) & amask;
             amax = b > amax ? b : amax;
             o[p] *= inv_expected;
@@ -560,7 +566,9 @@ TAMD_DEVICE void tile_epilogue_t(const Args &a, const Tile &t, f32x16_t (&acc)[N
           }
         }
         const int off = (int)((dst + col_off) | col_kill);
-        if constexpr (osz == 2) {
+        if constexpr (ANY) {
+          // stored below, four rows at a time
+        } else if constexpr (osz == 2) {
           if constexpr (NO == 2) __builtin_amdgcn_raw_buffer_store_b32(narrow2(o[0], o[NO - 1]), ry, off, 0, 0);
           else __builtin_amdgcn_raw_buffer_store_b16((uint16_t)narrow(o[0]), ry, off, 0, 0);
         } else {
@@ -569,8 +577,53 @@ TAMD_DEVICE void tile_epilogue_t(const Args &a, const Tile &t, f32x16_t (&acc)[N
           else __builtin_amdgcn_raw_buffer_store_b8((uint8_t)narrow(o[0]), ry, off, 0, 0);
         }
       }
+      if constexpr (ANY) {
+        // the type and the way to store are the same for the whole launch: one branch each for four rows
+        uint32_t w[4][NO];
+        auto all = [&](auto f) {
+#pragma unroll
+          for (int jj = 0; jj < 4; ++jj)
+#pragma unroll
+            for (int p = 0; p < NO; ++p) w[jj][p] = f(out4[jj][p]);
+        };
+        if constexpr (osz == 4) {
+          all([](float v) { return f32_to_bits(v); });
+        } else if constexpr (osz == 2) {
+          if (ydt == TAMD_BF16) all([](float v) { return f32_to_bf16_bits(v); });
+          else all([](float v) { return f32_to_f16_bits(v); });
+        } else {
+          if (ydt == TAMD_FP8_E5M2) all([](float v) { return f32_to_e5m2_bits(v, false); });
+          else all([](float v) { return f32_to_e4m3_bits(v, false); });
+        }
+        auto store1 = [&](uint32_t v, int off) {
+          if constexpr (osz == 4) __builtin_amdgcn_raw_buffer_store_b32(v, ry, off, 0, 0);
+          else if constexpr (osz == 2) __builtin_amdgcn_raw_buffer_store_b16((uint16_t)v, ry, off, 0, 0);
+          else __builtin_amdgcn_raw_buffer_store_b8((uint8_t)v, ry, off, 0, 0);
+        };
+        if (NO == 1 || !pairs) {
+#pragma unroll
+          for (int jj = 0; jj < 4; ++jj) {
+            store1(w[jj][0], (int)((dst4[jj] + col_off) | col_kill));
+            if constexpr (NO == 2) store1(w[jj][NO - 1], (int)((dst4[jj] + col_off + osz) | col_kill1));
+          }
+        } else {
+#pragma unroll
+          for (int jj = 0; jj < 4; ++jj) {
+            const int off = (int)((dst4[jj] + col_off) | col_kill);
+            if constexpr (osz == 4) __builtin_amdgcn_raw_buffer_store_b64(u32x2_t{w[jj][0], w[jj][NO - 1]}, ry, off, 0, 0);
+            else if constexpr (osz == 2) __builtin_amdgcn_raw_buffer_store_b32(w[jj][0] | (w[jj][NO - 1] << 16), ry, off, 0, 0);
+            else __builtin_amdgcn_raw_buffer_store_b16((uint16_t)(w[jj][0] | (w[jj][NO - 1] << 8)), ry, off, 0, 0);
+          }
+        }
+      }
       // (the running maximum is taken here and not after the last row, with every result kept until then)
       if constexpr (FLEX) asm volatile("" : "+v"(amax));
+      if constexpr (ANY) {   // a rolled loop: the next four rows move to where it looks for them
+#pragma unroll
+        for (int f = 0; f < NF; ++f)
+#pragma unroll
+          for (int e = 0; e < 12; ++e) acc[i][f][e] = acc[i][f][e + 4];
+      }
       __builtin_amdgcn_sched_barrier(0);
     }
   }
@@ -676,32 +729,51 @@ TAMD_DEVICE void tile_epilogue_general(const Args &a, const Tile &t, f32x16_t (&
   if (a.y_actual_scale) store_actual_scale(a.y_actual_scale, amax, out_max, lane);
 }
 
-// FAST_YDT: the 16-bit output type that gets the specialised epilogues (the activations' type; bf16 for fp8
-// activations); FP8_ROWS: the kernel's activations are fp8, then float8_e4m3fn output (the rows the next matmul of an
-// MoE layer consumes, usually with a flexpoint scale) is specialised as well.  Any other type takes the general
-// epilogue, and so does an output whose column pairs do not lie whole on aligned words or that spans 2 GB or more.
-template <int ACT, typename Args>
-TAMD_DEVICE bool epilogue_is_regular(const Args &a) {
+// Whether 32-bit offsets reach every output of a batch entry, and whether a lane's two outputs lie whole on one aligned word
+// (float32 pairs are stored as two words, which need no more than their own alignment).
+template <typename Args>
+TAMD_DEVICE bool epilogue_spans_32_bits(const Args &a) {
   const int osz = a.y_dtype == TAMD_F32 ? 4 : (is_fp8(a.y_dtype) ? 1 : 2);
   const int64_t lim = 0x7FFFFF00;
   if (a.y_rows <= 0 || a.y_stride_m < 0 || a.y_rows * a.y_stride_m * osz >= lim) return false;
-  if (a.y_mx_scale && a.y_rows * a.y_mx_stride_m >= lim) return false;
+  return !a.y_mx_scale || a.y_rows * a.y_mx_stride_m < lim;
+}
+template <int ACT, typename Args>
+TAMD_DEVICE bool epilogue_stores_pairs(const Args &a) {
   if (ACT == TAMD_ACT_SWIGLU) return true;   // one output per lane
+  if (a.y_dtype == TAMD_F32) return (a.N & 1) == 0;
+  const int osz = is_fp8(a.y_dtype) ? 1 : 2;
   return ((a.N | (int)a.y_stride_m | (int)a.y_stride_z) & 1) == 0 && ((uintptr_t)a.y & (2 * osz - 1)) == 0;
 }
+template <int ACT, typename Args>
+TAMD_DEVICE bool epilogue_is_regular(const Args &a) {
+  return epilogue_spans_32_bits(a) && epilogue_stores_pairs<ACT>(a);
+}
+// FAST_YDT: the 16-bit output type that gets epilogues of its own (the activations' type; bf16 for fp8 activations); FP8_ROWS:
+// the kernel's activations are fp8, then float8_e4m3fn output (the rows the next matmul of an MoE layer consumes, usually with
+// a flexpoint scale) has one as well.  Everything else -- another type, flexpoint scales, odd sizes or strides -- takes the form of
+// its width, and only an output of 2 GB or more (or of unknown rows) and MXFP8 output in odd rows the general epilogue.  The
+// general one, a branch and a 64-bit address per element, is slower by (4096 x 2880, MXFP4 weights): fp8 rows, 5759 columns of
+// bf16 116 us against 88; bf16 rows, 5760 columns of float32 145 against 128, of e4m3 with a flexpoint scale 161 against 126.
 template <int NFR, int ACT, int FAST_YDT, bool FP8_ROWS, typename Args>
 TAMD_DEVICE void tile_epilogue(const Args &a, const Tile &t, f32x16_t (&acc)[NFR][NF], uint8_t *tab) {
   const bool flexo = a.y_expected_scale != nullptr || a.y_actual_scale != nullptr;
-  const bool fast = epilogue_is_regular<ACT>(a);
-  if (fast && a.y_mx_scale) {  // always e4m3 values and no flexpoint output (checked by the entry point)
+  const bool spans = epilogue_spans_32_bits(a), pairs = epilogue_stores_pairs<ACT>(a);
+  if (spans && pairs && a.y_mx_scale) {  // always e4m3 values and no flexpoint output (checked by the entry point)
     tile_epilogue_t<NFR, ACT, TAMD_FP8_E4M3, true, false, true, Args>(a, t, acc, tab);
-  } else if (FP8_ROWS && fast && a.y_dtype == TAMD_FP8_E4M3) {
+  } else if (!spans || a.y_mx_scale) {
+    tile_epilogue_general<NFR, ACT, Args>(a, t, acc, tab);
+  } else if (FP8_ROWS && pairs && a.y_dtype == TAMD_FP8_E4M3) {
     if constexpr (FP8_ROWS) tile_epilogue_t<NFR, ACT, TAMD_FP8_E4M3, true, true, false, Args>(a, t, acc, tab);
-  } else if (fast && a.y_dtype == FAST_YDT && !flexo) {
+  } else if (pairs && a.y_dtype == FAST_YDT && !flexo) {
     if (a.betas || a.gammas) tile_epilogue_t<NFR, ACT, FAST_YDT, true, false, false, Args>(a, t, acc, tab);
     else tile_epilogue_t<NFR, ACT, FAST_YDT, false, false, false, Args>(a, t, acc, tab);
+  } else if (a.y_dtype == TAMD_F32) {
+    tile_epilogue_t<NFR, ACT, TAMD_F32, true, true, false, Args>(a, t, acc, tab, pairs);
+  } else if (is_fp8(a.y_dtype)) {
+    tile_epilogue_t<NFR, ACT, kAny8, true, true, false, Args>(a, t, acc, tab, pairs);
   } else {
-    tile_epilogue_general<NFR, ACT, Args>(a, t, acc, tab);
+    tile_epilogue_t<NFR, ACT, kAny16, true, true, false, Args>(a, t, acc, tab, pairs);
   }
 }
 
@@ -1329,6 +1401,9 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
 #pragma unroll
           for (int e = 0; e < 4; ++e) acc[0][f][4 * j + e] += v[e];
         }
+    // (added here: left for the epilogue, which has several forms, the planes would not fit the registers until then)
+#pragma unroll
+    for (int f = 0; f < NF; ++f) asm volatile("" : "+v"(acc[0][f]));
     __syncthreads();   // the epilogue's tables take the same memory
   }
   // (the wave's own weight region is free by now: its table goes there)
