@@ -22,3 +22,26 @@ def test_expert_sorted_gate_weights(T, E, k, dtype, device):
     assert torch.equal(r.scatter_indx.cpu(), ref["scatter_indx"])
     gates = r.expert_sorted_gate_weights
     assert gates.dtype == dtype and torch.equal(gates.cpu(), r.vals.cpu().flatten()[ref["scatter_indx"].long()])
+
+
+@pytest.mark.parametrize("inference", [False, True])
+def test_gate_weights_are_the_callers_own(inference, device):
+    """Scaling the gate weights in place changes neither later accesses nor vals; scaling vals changes later accesses."""
+    with torch.inference_mode(inference):
+        torch.manual_seed(3)
+        logits = torch.randn(65, 32, device=device)
+        r = routing(logits, 4)
+        want = r.vals.clone().reshape(-1)[r.scatter_indx.long()]
+        first = routing(logits, 4).expert_sorted_gate_weights   # (vals not touched before: the kernel's own copy)
+        assert torch.equal(first, want)
+        g = r.expert_sorted_gate_weights
+        g.mul_(3.0)
+        assert torch.equal(r.expert_sorted_gate_weights, want)
+        r.vals.mul_(2.0)
+        assert torch.equal(r.expert_sorted_gate_weights, want * 2)
+        q = routing(logits, 4)
+        q.vals.mul_(2.0)
+        assert torch.equal(q.expert_sorted_gate_weights, want * 2)
+        q = routing(logits, 4)
+        q.expert_sorted_gate_weights.zero_()
+        assert torch.equal(q.expert_sorted_gate_weights, want)

@@ -101,18 +101,19 @@ class RoutingResult:
 
     @property
     def expert_sorted_gate_weights(self):
-        """vals in expert-sorted row order: the `gammas` of the down projection.  The routing kernels write them where they
-        place an entry (two indexing kernels and their launches fewer: 11 us at 256 rows, 13 at 16384)."""
-        g = self._cache.get("gates")
-        if g is None:
-            if "gates" in self._lay:
-                T, k = self._lay["shape"]
-                off = self._lay["gates"][0] * 4 // self._lay["vals_dtype"].itemsize
-                g = _native.view(self._arena, self._lay["vals_dtype"], off, T * k, 1, -1, 0)
-            else:
-                g = self.vals.reshape(-1)[self.scatter_indx.long()]
-            self._cache["gates"] = g
-        return g
+        """vals in expert-sorted row order: the `gammas` of the down projection.  A tensor of its own on every access: a caller
+        may scale it in place.  The routing kernels write one copy where they place an entry (two indexing kernels and their
+        launches fewer: 11 us at 256 rows, 13 at 16384); the first access hands it out if vals cannot have been written to."""
+        mine = object()  # (of several threads one gets the kernels' copy)
+        if "gates" in self._lay and self._vals_as_routed() and self._cache.setdefault("gates", mine) is mine:
+            T, k = self._lay["shape"]
+            off = self._lay["gates"][0] * 4 // self._lay["vals_dtype"].itemsize
+            return _native.view(self._arena, self._lay["vals_dtype"], off, T * k, 1, -1, 0)
+        return self.vals.reshape(-1)[self.scatter_indx.long()]
+
+    def _vals_as_routed(self):
+        # (inference tensors do not count their versions)
+        return self._vals is None or (not self._vals.is_inference() and self._vals._version == 0)
 
 
 @functools.lru_cache(maxsize=512)
