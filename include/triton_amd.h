@@ -20,13 +20,15 @@
 #ifndef TRITON_AMD_H
 #define TRITON_AMD_H
 
+#include <stddef.h>
 #include <stdint.h>
 
 #ifdef __cplusplus
 extern "C" {
 #endif
 
-#define TAMD_VERSION 1
+/* 2: tamd_matmul_args ends with y_rows; tamd_matmul_sized, tamd_routing_gates */
+#define TAMD_VERSION 2
 
 /* error codes (negative) */
 #define TAMD_E_INVALID (-1)     /* bad shape / stride / pointer / enum */
@@ -297,10 +299,16 @@ typedef struct tamd_matmul_args {
    * 16-byte part p in slot p ^ ((c >> 2) & 3) ^ 2 f.  Only w_stride_e is used (bytes); w 16-byte aligned. */
   int w_layout;
   /* rows of y (of one batch entry) that dst(r) can name; with a span y_rows * y_stride_m below 2 GB the results are
-   * stored through 32-bit offsets.  0: unknown, the general (slower) stores are used. */
+   * stored through 32-bit offsets.  0: M without scatter_indx, with it unknown (slower stores through 64-bit
+   * addresses). */
   int64_t y_rows;
 } tamd_matmul_args;
 
+/* args_size = sizeof(tamd_matmul_args) as the caller was compiled: fields that the caller's structure does not have
+ * are taken as zero (a smaller structure than version 1's is TAMD_E_INVALID, a larger one than the library's
+ * TAMD_E_UNSUPPORTED). */
+int tamd_matmul_sized(const tamd_matmul_args *args, size_t args_size, void *stream);
+/* The same for version 1's structure, which ends with w_layout: fields after it are not read. */
 int tamd_matmul(const tamd_matmul_args *args, void *stream);
 
 /*

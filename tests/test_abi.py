@@ -112,6 +112,33 @@ def test_matmul_rejects_degenerate_problems_before_any_launch(lib):
     assert lib.tamd_matmul(C.byref(a), None) == _lib.E_INVALID
 
 
+def test_matmul_reads_no_more_than_the_callers_structure(lib):
+    """A caller compiled against version 1's header hands over a structure that ends with w_layout: here it ends where the
+    next page cannot be read.  (K == 0 is refused before any launch.)"""
+    code = """
+import ctypes as C, mmap
+from triton_amd import _lib
+lib, page = _lib.lib(), mmap.PAGESIZE
+libc = C.CDLL(None, use_errno=True)
+libc.mmap.restype, libc.mmap.argtypes = C.c_void_p, [C.c_void_p, C.c_size_t, C.c_int, C.c_int, C.c_int, C.c_long]
+libc.mprotect.argtypes = [C.c_void_p, C.c_size_t, C.c_int]
+base = libc.mmap(None, 2 * page, 3, mmap.MAP_PRIVATE | mmap.MAP_ANONYMOUS, -1, 0)
+assert libc.mprotect(base + page, page, 0) == 0
+old = _lib.MatmulArgs.y_rows.offset
+a = _lib.MatmulArgs(x=0x1000, w=0x2000, y=0x3000, M=16, N=256, K=0, n_experts=1)
+C.memmove(base + page - old, C.byref(a), old)
+p = C.cast(base + page - old, C.POINTER(_lib.MatmulArgs))
+assert lib.tamd_matmul(p, None) == _lib.E_UNSUPPORTED
+assert lib.tamd_matmul_sized(p, old, None) == _lib.E_UNSUPPORTED
+assert lib.tamd_matmul_sized(p, old - 8, None) == _lib.E_INVALID
+a.K = -32
+assert lib.tamd_matmul_sized(C.byref(a), C.sizeof(a), None) == _lib.E_INVALID
+assert lib.tamd_matmul_sized(C.byref(a), C.sizeof(a) + 8, None) == _lib.E_UNSUPPORTED
+"""
+    subprocess.run([sys.executable, "-c", code], cwd=ROOT, check=True)
+    assert lib.tamd_version() >= 2
+
+
 def test_no_cpu_fallback_in_product():
     """The package never imports the oracle and refuses CPU tensors."""
     import torch

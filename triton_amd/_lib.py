@@ -126,6 +126,7 @@ _SIGNATURES = {
                       _I64, _PTR, _I64, _INT, _PTR, _PTR], C.c_int),
     "tamd_routing_gates": ([_PTR, _INT, _I64, _INT, _INT, _INT, _PTR, _PTR, _PTR, _I64, _I64, _PTR, _PTR, _PTR, _PTR, _PTR,
                             _PTR, _I64, _PTR, _I64, _INT, _PTR, _PTR], C.c_int),
+    "tamd_matmul_sized": ([C.POINTER(MatmulArgs), C.c_size_t, _PTR], C.c_int),
     "tamd_matmul": ([C.POINTER(MatmulArgs), _PTR], C.c_int),
     "tamd_reduce": ([_PTR, _INT, _I64, _I64, _I64, _I64, _I64, _I64, _PTR, _I64, _I64, _I64, _PTR, _I64, _I64, _I64,
                      _PTR, _INT, _I64, _I64, _PTR], C.c_int),

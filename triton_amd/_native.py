@@ -25,7 +25,7 @@ def load():
     host = importlib.util.module_from_spec(importlib.util.spec_from_file_location("triton_amd._host", HOST_PATH, loader=loader))
     loader.exec_module(host)
     addresses = {n: ctypes.cast(getattr(lib, n), ctypes.c_void_p).value
-                 for n in ("tamd_matmul", "tamd_routing_gates", "tamd_reduce", "tamd_downcast_mxfp", "tamd_upcast_mxfp")}
+                 for n in ("tamd_matmul_sized", "tamd_routing_gates", "tamd_reduce", "tamd_downcast_mxfp", "tamd_upcast_mxfp")}
     host.init(addresses, Tensor, CDNA4MXValueLayout, CDNA4MXScaleLayout, FP4, opt_flags._opt_flags_constraints,
               opt_flags._opt_flags)
     for name in _FUNCTIONS:

@@ -27,7 +27,7 @@ namespace {
 
 // ------------------------------------------------------------------ addresses and Python objects handed over by init()
 struct Abi {
-  int (*matmul)(const tamd_matmul_args *, void *);
+  int (*matmul)(const tamd_matmul_args *, size_t, void *);
   int (*routing)(const void *, int, int64_t, int, int, int, void *, int16_t *, uint32_t *, int64_t, int64_t, int32_t *,
                  int32_t *, int32_t *, int32_t *, void *, int32_t *, int64_t, int32_t *, int64_t, int, int32_t *, void *);
   int (*reduce)(const void *, int, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, const void *, int64_t, int64_t,
@@ -458,7 +458,7 @@ PyObject *py_matmul(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
     g.gather_indx = gather ? (const int32_t *)gather->data_ptr() : nullptr;
     g.scatter_indx = scatter ? (const int32_t *)scatter->data_ptr() : nullptr;
     void *st = stream_of(dev);
-    const int rc = without_gil([&] { return abi.matmul(&g, st); });
+    const int rc = without_gil([&] { return abi.matmul(&g, sizeof g, st); });
     if (rc != 0) return PyLong_FromLong(rc);
     if (c_o != Py_None) {
       Py_INCREF(c_o);
@@ -655,7 +655,7 @@ PyObject *py_init(PyObject *, PyObject *args) {
     std::memcpy(slot, &p, sizeof p);
     return p != nullptr;
   };
-  if (!take("tamd_matmul", &abi.matmul) || !take("tamd_routing_gates", &abi.routing) || !take("tamd_reduce", &abi.reduce) ||
+  if (!take("tamd_matmul_sized", &abi.matmul) || !take("tamd_routing_gates", &abi.routing) || !take("tamd_reduce", &abi.reduce) ||
       !take("tamd_downcast_mxfp", &abi.downcast) || !take("tamd_upcast_mxfp", &abi.upcast)) {
     PyErr_SetString(PyExc_RuntimeError, "an entry point of the library is missing");
     return nullptr;

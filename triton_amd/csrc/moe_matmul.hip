@@ -3,6 +3,9 @@
 // (separate translation units so that they compile in parallel).
 #include "common.h"
 
+#include <stddef.h>
+#include <string.h>
+
 namespace tamd {
 int dispatch_mm_bf16(const tamd_matmul_args &a, int block_m, int grid_m, hipStream_t st);
 int dispatch_mm_f16(const tamd_matmul_args &a, int block_m, int grid_m, hipStream_t st);
@@ -16,9 +19,12 @@ int dispatch_mm_kk_fp8e5m2(const tamd_matmul_args &a, int block_m, int grid_m, h
 
 using namespace tamd;
 
-extern "C" int tamd_matmul(const tamd_matmul_args *args, void *stream) {
-  if (!args) return TAMD_E_INVALID;
-  tamd_matmul_args a = *args;
+extern "C" int tamd_matmul_sized(const tamd_matmul_args *args, size_t args_size, void *stream) {
+  if (!args || args_size < offsetof(tamd_matmul_args, y_rows)) return TAMD_E_INVALID;
+  if (args_size > sizeof(tamd_matmul_args)) return TAMD_E_UNSUPPORTED;
+  tamd_matmul_args a = {};
+  memcpy(&a, args, args_size);
+  if (a.y_rows == 0 && !a.scatter_indx) a.y_rows = a.M;
   if (a.M < 0 || a.N < 0 || a.K < 0 || a.n_experts < 1) return TAMD_E_INVALID;
   if (a.n_experts == 1) a.w_stride_e = a.w_mx_stride_e = a.bias_stride_e = 0;  // never used; keeps the alignment checks honest
   if (a.M == 0 || a.N == 0) return 0;
@@ -97,4 +103,8 @@ extern "C" int tamd_matmul(const tamd_matmul_args *args, void *stream) {
     return dispatch_mm_w16_f16(a, block_m, grid_m, st);
   }
   return TAMD_E_UNSUPPORTED;
+}
+
+extern "C" int tamd_matmul(const tamd_matmul_args *args, void *stream) {
+  return tamd_matmul_sized(args, offsetof(tamd_matmul_args, y_rows), stream);
 }

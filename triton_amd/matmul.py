@@ -444,9 +444,13 @@ def matmul(a, b, bias, a_ragged_metadata: Optional[RaggedTensorMetadata] = None,
         _matmul_split_k(args.pack(), flags.split_k, a, wd, b_fp4, out, fused_activation, bias, flex.out_data,
                         precision_config.flexpoint_saturate_inf)
         return finish()
-    rc = _lib.lib().tamd_matmul(ctypes.byref(args.pack()), _lib.stream_ptr(a.device))
+    rc = _launch(args.pack(), a.device)
     _lib.check(rc, "matmul")
     return finish()
+
+
+def _launch(args, device):
+    return _lib.lib().tamd_matmul_sized(ctypes.byref(args), ctypes.sizeof(args), _lib.stream_ptr(device))
 
 
 def _matmul_split_k(args, split_k, a, wd, w_is_fp4, out, fused_activation, bias, out_flex, saturate_inf):
@@ -495,7 +499,7 @@ def _matmul_split_k(args, split_k, a, wd, w_is_fp4, out, fused_activation, bias,
         part.y_stride_m, part.y_stride_z = scratch.stride(2), scratch.stride(0)
         part.y_expected_scale = part.y_actual_scale = None
         part.force_variant = 0
-        rc = _lib.lib().tamd_matmul(ctypes.byref(part), _lib.stream_ptr(out.device))
+        rc = _launch(part, out.device)
         _lib.check(rc, "matmul (split_k ranges as a batch)")
     for s in range(0 if one_launch else n_split):
         k0 = s * chunk
@@ -513,7 +517,7 @@ def _matmul_split_k(args, split_k, a, wd, w_is_fp4, out, fused_activation, bias,
         part.y, part.y_dtype = scratch[s].data_ptr(), _lib.F32
         part.y_stride_m, part.y_stride_z = scratch.stride(2), scratch.stride(1)
         part.y_expected_scale = part.y_actual_scale = None
-        rc = _lib.lib().tamd_matmul(ctypes.byref(part), _lib.stream_ptr(out.device))
+        rc = _launch(part, out.device)
         _lib.check(rc, "matmul (split_k range)")
     # one finalising launch, as in the reference (matmul.py:711-737): sum of the partial results, the fused activation
     # as the reduction's post-processing function, the output's flexpoint scales, the cast
