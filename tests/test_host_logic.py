@@ -217,3 +217,12 @@ def test_native_tile_choice_follows_make_opt_flags():
                 for fp8 in (False, True):
                     want = OF.make_opt_flags(m, 64, 64, slices, ragged, expected, fp8).block_m
                     assert _native.choose_block_m(m, slices, ragged, -1 if expected is None else expected, fp8) == want
+
+
+def test_native_host_path_is_tied_to_its_torch(monkeypatch):
+    """The extension reads tensors in place: one built for another torch is refused when it is loaded, not when it misreads."""
+    from triton_amd import _native
+    assert _native.load().built_for == str(torch.__version__)
+    monkeypatch.setattr(torch, "__version__", "1.0.0")
+    with pytest.raises(RuntimeError, match="was built for torch"):
+        _native.load()

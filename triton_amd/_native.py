@@ -5,13 +5,16 @@ first call does.  Each answers None for a call it does not cover; the caller the
 import ctypes
 import os
 
+import torch
+
 from . import _lib
 
 HOST_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_host.so")
 
 
 def load():
-    """Loads the extension and hands it the library's addresses; raises if it has not been built."""
+    """Loads the extension and hands it the library's addresses; raises if it has not been built, or for another torch: it is
+    compiled against torch's headers and reads tensors in place."""
     import importlib.machinery
     import importlib.util
 
@@ -23,7 +26,14 @@ def load():
         raise RuntimeError(f"{HOST_PATH} is missing: build it with `python -m triton_amd.build`")
     loader = importlib.machinery.ExtensionFileLoader("triton_amd._host", HOST_PATH)
     host = importlib.util.module_from_spec(importlib.util.spec_from_file_location("triton_amd._host", HOST_PATH, loader=loader))
-    loader.exec_module(host)
+    try:
+        loader.exec_module(host)
+        built_for = host.built_for
+    except (ImportError, AttributeError) as e:  # (a symbol of another torch is missing, or a file from before the check)
+        built_for = f"another torch ({e})"
+    if built_for != str(torch.__version__):
+        raise RuntimeError(f"{HOST_PATH} was built for torch {built_for}, this is {torch.__version__}: build it again with "
+                           "`python -m triton_amd.build`")
     addresses = {n: ctypes.cast(getattr(lib, n), ctypes.c_void_p).value
                  for n in ("tamd_matmul_sized", "tamd_routing_gates", "tamd_reduce", "tamd_downcast_mxfp", "tamd_upcast_mxfp")}
     host.init(addresses, Tensor, CDNA4MXValueLayout, CDNA4MXScaleLayout, FP4, opt_flags._opt_flags_constraints,

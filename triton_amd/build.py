@@ -94,7 +94,7 @@ def _build_host():
     libs = os.path.join(os.path.dirname(torch.__file__), "lib")
     inc = [f for p in (*include_paths("cuda"), sysconfig.get_paths()["include"]) for f in ("-isystem", p)]
     cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
-           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *inc, os.path.join(CSRC, "host.cpp"), "-o", HOST,
+           f'-DTAMD_TORCH_VERSION="{torch.__version__}"', f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *inc, os.path.join(CSRC, "host.cpp"), "-o", HOST,
            f"-L{libs}", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip"]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:

@@ -687,4 +687,10 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, methods, null
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__host() { return PyModule_Create(&module); }
+// `built_for`: the torch whose headers and libraries this file was compiled against; the loader compares it before anything
+// here touches a tensor
+PyMODINIT_FUNC PyInit__host() {
+  PyObject *m = PyModule_Create(&module);
+  if (m && PyModule_AddStringConstant(m, "built_for", TAMD_TORCH_VERSION) != 0) Py_CLEAR(m);
+  return m;
+}
