@@ -1,8 +1,10 @@
-"""GPU: what the routing kernels leave in expert-sorted order, on every launch form of the routing, against the oracle."""
+"""GPU: what the routing kernels leave in expert-sorted order, on every launch form of the routing, against the oracle; what the
+host code of the entry points hands out and keeps."""
 import pytest
 import torch
 
 from oracle import routing_ref as RR
+from triton_amd.matmul import matmul
 from triton_amd.routing import routing
 
 pytestmark = pytest.mark.gpu
@@ -45,3 +47,55 @@ def test_gate_weights_are_the_callers_own(inference, device):
         q = routing(logits, 4)
         q.expert_sorted_gate_weights.zero_()
         assert torch.equal(q.expert_sorted_gate_weights, want)
+
+
+def gate(device, seed):
+    """A gate product whose weights have unit stride along N: they are turned, and the copy is kept."""
+    g = torch.Generator().manual_seed(seed)
+    x, w = torch.randn(48, 256, generator=g).bfloat16(), (torch.randn(256, 32, generator=g) * 0.1).bfloat16()
+    return x.to(device), w.to(device), x.float() @ w.float()
+
+
+def close(y, ref):
+    torch.testing.assert_close(y.cpu().float(), ref, rtol=1e-2, atol=1e-2)
+
+
+def test_turned_weights_on_another_stream(device):
+    x, w, ref = gate(device, 0)
+    first, second = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(first):
+        torch.cuda._sleep(200_000_000)      # the copy is made about 0.1 s from now
+        y1 = matmul(x, w, None)
+    with torch.cuda.stream(second):
+        y2 = matmul(x, w, None)
+    torch.cuda.synchronize()
+    close(y1, ref)
+    close(y2, ref)
+
+
+def test_turned_weights_in_a_graph(device):
+    x, w, ref = gate(device, 1)
+    warm = gate(device, 2)
+    matmul(warm[0], warm[1], None)
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        y = matmul(x, w, None)              # the first call on these weights is only recorded
+    close(matmul(x, w, None), ref)          # ... and leaves nothing behind
+    for scale in (1.0, 2.0, 0.5):
+        w.mul_(scale)
+        ref = x.cpu().float() @ w.cpu().float()
+        graph.replay()
+        torch.cuda.synchronize()
+        close(y, ref)
+        close(matmul(x, w, None), ref)
+
+
+def test_turned_weights_in_inference_mode(device):
+    with torch.inference_mode():
+        x, w, ref = gate(device, 3)
+        close(matmul(x, w, None), ref)
+        w.mul_(2.0)
+        close(matmul(x, w, None), 2 * ref)

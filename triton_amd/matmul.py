@@ -104,18 +104,32 @@ def _fp8_direct(a, w):
             and whole(a, *a.stride()[:-1]) and whole(w, w.stride(-1), *w.stride()[:-2]))
 
 
-_TURNED = {}  # id(weights) -> (weak reference to them, their version counter, the copy with unit stride along K)
+# id(weights) -> (weak reference to them, their version counter, the copy with unit stride along K, the stream that makes it,
+# the event after it)
+_TURNED = {}
 
 
 def _k_contiguous_cached(w):
+    if w.is_inference() or (w.is_cuda and torch.cuda.is_current_stream_capturing()):
+        # no version to tell a write by; a copy that only a graph's replay makes, in memory that the graph owns
+        return w.transpose(-1, -2).contiguous().transpose(-1, -2)
     key = id(w)
     hit = _TURNED.get(key)
     if hit is not None and hit[0]() is w and hit[1] == w._version:
-        return hit[2]
+        turned, stream = hit[2], hit[3]
+        if stream is not None and (_lib.stream_ptr(w.device).value or 0) != stream:
+            now = torch.cuda.current_stream(w.device)
+            now.wait_event(hit[4])
+            turned.record_stream(now)
+        return turned
     turned = w.transpose(-1, -2).contiguous().transpose(-1, -2)
+    stream = done = None
+    if w.is_cuda:
+        now = torch.cuda.current_stream(w.device)
+        stream, done = _lib.stream_ptr(w.device).value or 0, now.record_event()
     if len(_TURNED) >= 64:
         _TURNED.clear()
-    _TURNED[key] = (weakref.ref(w, lambda _, key=key: _TURNED.pop(key, None)), w._version, turned)
+    _TURNED[key] = (weakref.ref(w, lambda _, key=key: _TURNED.pop(key, None)), w._version, turned, stream, done)
     return turned
 
 
