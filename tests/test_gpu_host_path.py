@@ -4,8 +4,14 @@ import pytest
 import torch
 
 from oracle import routing_ref as RR
-from triton_amd.matmul import matmul
+from triton_amd import _native
+from triton_amd.matmul import (Epilogue, FlexCtx, FnSpecs, FusedActivation, InFlexData, OutFlexData, PrecisionConfig, matmul)
+from triton_amd.numerics_details.mxfp import downcast_to_mxfp, upcast_from_mxfp
+from triton_amd.reduce import reduce
 from triton_amd.routing import routing
+from triton_amd.swiglu import swiglu_fn
+from triton_amd.tensor import FP4, convert_layout, wrap_torch_tensor
+from triton_amd.tensor_details.layout import CDNA4MXScaleLayout, CDNA4MXValueLayout
 
 pytestmark = pytest.mark.gpu
 
@@ -99,3 +105,154 @@ def test_turned_weights_in_inference_mode(device):
         close(matmul(x, w, None), ref)
         w.mul_(2.0)
         close(matmul(x, w, None), 2 * ref)
+
+
+class BothPaths:
+    """Runs a call as it is and with the native function switched off, says which path the first took, compares the results
+    bit for bit."""
+
+    def __init__(self, monkeypatch, name):
+        _native.load()
+        self.mp, self.name, self.fn, self.covered = monkeypatch, name, getattr(_native, name), None
+
+    def __call__(self, call):
+        def spy(*args):
+            done = self.fn(*args)
+            if self.covered is None:   # (the general path may call itself with a form that is covered)
+                self.covered = done is not None and type(done) is not int
+            return done
+        self.mp.setattr(_native, self.name, spy)
+        native = call()
+        self.mp.setattr(_native, self.name, lambda *args: None)
+        general = call()
+        for a, b in zip(native, general):
+            assert a.dtype == b.dtype and a.shape == b.shape and a.stride() == b.stride()
+            assert torch.equal(a.contiguous().view(torch.uint8), b.contiguous().view(torch.uint8))
+        return self.covered
+
+
+SWIGLU = FusedActivation(FnSpecs("swiglu", swiglu_fn, ("alpha", "limit"), reduction_n=2), (1.702, 7.0))
+F8 = torch.float8_e4m3fn
+# rows, weights, weight layout, options, whether the native path takes the call
+FORMS = [(a, w, lay, opts, True) for a, w, lays in (("bf16", "mxfp4", ("strided", "blocks")), ("f16", "mxfp4", ("strided", "blocks")),
+                                                   ("fp8", "mxfp4", ("strided", "blocks")), ("mxfp8", "mxfp4", ("strided", "blocks")),
+                                                   ("bf16", "bf16", ("strided", )), ("f16", "f16", ("strided", )),
+                                                   ("fp8", "fp8", ("strided", )))
+         for lay in lays for opts in ((), ("gather", "swiglu"), ("scatter", "gammas"), ("dense", ), ("pitch", "c"))] + [
+    ("bf16", "mxfp4", "strided", ("betas", "bias f32"), True), ("bf16", "mxfp4", "strided", ("no bias", "f32 out"), True),
+    ("fp8", "mxfp4", "strided", ("swiglu", "flex out"), True), ("fp8", "mxfp4", "blocks", ("dense", "flex out"), True),
+    ("mxfp8", "mxfp4", "blocks", ("swiglu", "mx out"), True), ("bf16", "mxfp4", "strided", ("out_alpha", "expected"), True),
+    ("bf16", "bf16", "strided", ("2-D", "dense"), True), ("bf16", "mxfp4", "strided", ("2-D", "dense"), True),
+    # conversions, other layouts and long splits are the general path's
+    ("mxfp4", "mxfp4", "strided", ("gather", "swiglu"), False), ("bf16", "mxfp8", "strided", (), False),
+    ("bf16", "mxfp4", "strided", ("scatter", "gammas bf16"), False), ("bf16", "bf16", "along N", (), False),
+    ("fp8", "fp8", "along N", (), False), ("bf16", "mxfp4", "strided", ("dense", "long K"), False),
+    ("bf16", "mxfp4", "strided", ("int64 indices", "gather"), False), ("bf16", "mxfp4", "strided", ("no rows", ), False)]
+
+
+@pytest.mark.parametrize("acts,weights,layout,opts,covered", FORMS)
+def test_native_matmul_is_the_general_path(acts, weights, layout, opts, covered, device, monkeypatch):
+    g = torch.Generator(device=device).manual_seed(7)
+    rnd = lambda *s: torch.randn(s, generator=g, device=device)
+    T, E, k, K, N = (0 if "no rows" in opts else 37), 8, 4, 8192 if "long K" in opts else 160, 192
+    dense = "dense" in opts
+    E = 1 if dense else E
+    r = None if dense else routing(rnd(T, E), k)
+    gathered = "gather" in opts
+    rows = T if dense or gathered else T * k
+    one = lambda v: torch.full((1,), v, device=device)
+    # ---- weights
+    w = rnd(E, N, K) * 0.1
+    pw, lhs, rhs = {}, InFlexData(), InFlexData()
+    if weights[:2] == "mx":
+        v, s = downcast_to_mxfp(w.bfloat16(), torch.uint8 if weights == "mxfp4" else F8, axis=-1)
+        w, s = v.transpose(-1, -2), s.transpose(-1, -2)
+        if layout == "blocks":
+            w, s = (convert_layout(wrap_torch_tensor(w, dtype=FP4), CDNA4MXValueLayout()),
+                    convert_layout(wrap_torch_tensor(s), CDNA4MXScaleLayout()))
+        pw = {"b_mx_scale": s, "b_microblock_size": 32}
+    else:
+        w = w.to({"bf16": torch.bfloat16, "f16": torch.float16, "fp8": F8}[weights]).transpose(-1, -2)
+        if layout == "along N":
+            w = w.contiguous()
+        if weights == "fp8":
+            rhs = InFlexData(F8, one(0.5))
+    if "2-D" in opts:
+        w = w[0]
+        if pw:
+            pw["b_mx_scale"] = pw["b_mx_scale"][0]
+    # ---- rows
+    x = rnd(rows, K + (32 if "pitch" in opts else 0))[:, :K]
+    if acts[:2] == "mx":
+        x, xs = downcast_to_mxfp(x.bfloat16().contiguous(), torch.uint8 if acts == "mxfp4" else F8, axis=-1)
+        pw.update(a_mx_scale=xs, a_microblock_size=32)
+    else:
+        dt = {"bf16": torch.bfloat16, "f16": torch.float16, "fp8": F8}[acts]
+        full = rnd(rows, K + 32).to(dt)
+        x = full[:, :K] if "pitch" in opts else x.to(dt)
+        if acts == "fp8":
+            lhs = InFlexData(F8, one(0.25))
+    # ---- the rest
+    red = 2 if "swiglu" in opts else 1
+    M = T if dense else T * k
+    out_type = torch.float32 if "f32 out" in opts else F8 if "flex out" in opts or "mx out" in opts else None
+    out = OutFlexData(F8, one(0.1), one(0.0)) if "flex out" in opts else OutFlexData(torch.bfloat16, one(0.1)) if "expected" in opts else OutFlexData()
+    if acts == "fp8" and out_type is None:
+        out_type = torch.bfloat16
+    bias = rnd(E, N) if not dense else rnd(N)
+    if "no bias" in opts:
+        bias = None
+    elif "bias f32" not in opts:
+        bias = bias.bfloat16()
+    gammas = torch.rand(M, generator=g, device=device) if "gammas" in opts else torch.rand(M, generator=g, device=device).bfloat16() if "gammas bf16" in opts else None
+    betas = torch.rand(M, generator=g, device=device) if "betas" in opts else None
+    gather = r.gather_indx if gathered else None
+    if "int64 indices" in opts:
+        gather = gather.long()
+
+    def call():
+        if "flex out" in opts:
+            out.actual_scale.zero_()
+        extra = {}
+        if "mx out" in opts:
+            extra["c_mx_scale"] = torch.zeros((M, N // red // 32), dtype=torch.uint8, device=device)
+        pc = PrecisionConfig(flex_ctx=FlexCtx(lhs, rhs, out), out_dtype=out_type, c_microblock_size=32 if extra else None,
+                             flexpoint_saturate_inf="flex out" in opts, **pw, **extra)
+        c = torch.zeros((M, N // red + 8), dtype=out_type or x.dtype, device=device)[:, :N // red] if "c" in opts and acts != "mxfp8" else None
+        y = matmul(x, w, bias, None if dense else r.ragged_metadata, gather_indx=gather,
+                   scatter_indx=r.scatter_indx if "scatter" in opts else None, precision_config=pc, betas=betas, gammas=gammas,
+                   out_alpha=0.5 if "out_alpha" in opts else None, c=c, fused_activation=SWIGLU if red == 2 else None,
+                   epilogue=Epilogue(FnSpecs("QUANTIZE_MXFP8", None, (), ()), (), (), 6.0) if extra else None)
+        return [y, *extra.values(), *([out.actual_scale.clone()] if "flex out" in opts else [])]
+
+    assert BothPaths(monkeypatch, "matmul")(call) == covered
+
+
+@pytest.mark.parametrize("shape,axis,values,covered", [
+    ((33, 96), -1, torch.uint8, True), ((33, 96), 1, F8, True), ((3, 40, 64), 2, torch.float8_e5m2, True),
+    ((2, 64, 24), -2, torch.uint8, True), ((64, 24), 0, torch.uint8, True),
+    ((2, 64, 24), 1, F8, False), ((2, 64, 24), 0, torch.uint8, False), ((64, 24, 2), 0, torch.uint8, False), ((2, 3, 5, 32), -1, F8, False)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_native_conversions_are_the_general_path(shape, axis, values, covered, dtype, device, monkeypatch):
+    torch.manual_seed(8)
+    if shape[axis] % 32:
+        shape = tuple(64 if d == axis % len(shape) else n for d, n in enumerate(shape))
+    x = torch.randn(shape, device=device).to(dtype)
+    assert BothPaths(monkeypatch, "downcast")(lambda: downcast_to_mxfp(x, values, axis=axis)) == covered
+    monkeypatch.undo()
+    v, s = downcast_to_mxfp(x, values, axis=axis)
+    assert BothPaths(monkeypatch, "upcast")(lambda: [upcast_from_mxfp(v, s, dtype, axis=axis)]) == covered
+    monkeypatch.undo()
+    part = x[..., :-1] if axis % x.ndim != x.ndim - 1 else x[..., :-32]     # rows with gaps between them
+    if part.shape[axis] and part.numel():
+        assert BothPaths(monkeypatch, "downcast")(lambda: downcast_to_mxfp(part, values, axis=axis)) in (False, part.is_contiguous())
+
+
+@pytest.mark.parametrize("shape,dim", [((5, 4, 24), 1), ((4, 7, 9), 0), ((3, 5, 33), -1), ((2, 600, 8), 1)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_native_reduce_is_the_general_path(shape, dim, dtype, device, monkeypatch):
+    torch.manual_seed(9)
+    x = torch.randn(shape, device=device).to(dtype)
+    for t in (x, x.transpose(0, 2).contiguous().transpose(0, 2)):
+        assert BothPaths(monkeypatch, "reduce")(lambda: [reduce(t, dim=dim)[0]]) == (shape[dim] < 512)
+        monkeypatch.undo()
