@@ -650,15 +650,18 @@ __global__ __launch_bounds__(256) void upcast_cols_tile_kernel(
 
 // Up to how many tiles a tensor whose quantised axis is strided goes to the kernels of one column per thread instead of the tile
 // kernels.  A tile is 131072 elements to a workgroup whose passes follow one another, so that one round of tiles takes the
-// same time for few of them as for 256: 15 to 22 us to quantise, 8 to 11 to dequantise; the column kernels have 64 times the
-// workgroups and take about 4 us and 1 us per million elements.  Quantising float32 [1, 1760, 3000] (48 tiles) 18.6 us by
-// tiles, 9.2 by columns, [1, 2880, 5760] (135) 22.0 and 18.7; bf16 [2, 1184, 4328] (102) 16.6 and 13.4, [1, 2880, 5760]
-// (138) 17.5 and 19.0.  Dequantising to bf16 [2, 1024, 648] (12) 7.9 and 5.2, [1, 1664, 2616] (44) 8.4 and 9.4; to float32
-// [1, 1760, 3000] (48) 10.9 and 9.7, [5, 1248, 1232] (100) 10.9 and 11.6.
+// same time for few of them as for one per CU: 13 to 23 us to quantise, 8 to 12 to dequantise; the column kernels have 64 times
+// the workgroups and take about 4 us and 1 us per million elements.  Measured over 95 shapes [1 .. 8, 512 .. 2880, 512 .. 5760] of
+// 5 to 300 tiles on 256 CUs, the lines with the least time lost to the wrong kernel (us, by tiles / by columns):
+//   quantising    float32  152 tiles 17.4 / 15.2, 168: 22.1 / 19.3, 192: 22.7 / 19.9, 195: 16.1 / 17.5, 216: 26.0 / 26.8
+//                 16-bit    96 tiles 16.3 / 13.5, 105: 17.3 / 15.5, 114: 17.0 / 15.5, 120: 17.8 / 18.2, 126: 17.2 / 19.1
+//   dequantising  float32   44 tiles 10.8 / 10.0,  48: 11.6 / 10.3,  52: 12.3 / 12.1,  56: 10.7 / 12.4,  64: 11.9 / 12.4
+//                 16-bit    26 tiles  8.2 /  6.8,  32:  8.8 /  8.1,  35:  8.9 /  8.1,  39:  8.9 / 10.0,  48:  9.1 / 11.7
+// Fewer CUs hold a round of fewer tiles: the lines are shares of their number, given for 256.
 template <int DT>
-constexpr int64_t kColumnsUpToDown = DT == TAMD_F32 ? 136 : 104;
+constexpr int64_t kColumnsUpToDown = DT == TAMD_F32 ? 192 : 116;
 template <int DT>
-constexpr int64_t kColumnsUpToUp = DT == TAMD_F32 ? 48 : 24;
+constexpr int64_t kColumnsUpToUp = DT == TAMD_F32 ? 52 : 36;
 
 // Groups from which a thread of the row kernels takes two: below, the grid would no longer give every SIMD a few waves.
 constexpr int64_t kRowsUnrolled = 64 * 2048;
@@ -687,7 +690,9 @@ int launch_downcast(const void *src, int64_t nb, int64_t L, int64_t nr, int64_t 
   bool vec = nr % NV == 0 && aligned(src, 16) && (ssb * ES) % 16 == 0 && (ssl * ES) % 16 == 0;
   constexpr int CW = kTileCols<DT>, GT = kTileGroups<DT>;
   const int64_t tiles = ((nr + CW - 1) / CW) * ((G + GT - 1) / GT) * nb;
-  if (vec && tiles > kColumnsUpToDown<DT>) {
+  int cus = 0;
+  if (int rc = cu_count(cus)) return rc;
+  if (vec && tiles * 256 > kColumnsUpToDown<DT> * cus) {
     const int64_t blocks = tiles;
     if (blocks > 0x7FFFFFFF) return TAMD_E_UNSUPPORTED;
     if (int rc = raise_lds_limit_once((const void *)downcast_cols_tile_kernel<DT>)) return rc;
@@ -724,7 +729,9 @@ int launch_upcast(const uint8_t *vals, int64_t vsb, int64_t vsr, const uint8_t *
   bool vec = nr % NV == 0 && aligned(dst, 16) && (dsb * ES) % 16 == 0 && (dsl * ES) % 16 == 0;
   constexpr int CW = kTileCols<DT>, GT = kTileGroups<DT>;
   const int64_t tiles = ((nr + CW - 1) / CW) * ((G + GT - 1) / GT) * nb;
-  if (vec && tiles > kColumnsUpToUp<DT>) {
+  int cus = 0;
+  if (int rc = cu_count(cus)) return rc;
+  if (vec && tiles * 256 > kColumnsUpToUp<DT> * cus) {
     const int64_t blocks = tiles;
     if (blocks > 0x7FFFFFFF) return TAMD_E_UNSUPPORTED;
     if (int rc = raise_lds_limit_once((const void *)upcast_cols_tile_kernel<DT>)) return rc;
