@@ -419,7 +419,7 @@ def cpu_baseline(x_cpu, vals, scales, bias_cpu, ref, experts, K, N, act, fc2=Non
 
 
 def sample_experts(args, rows, E, K, N):
-    """Experts in the CPU sample: as asked, or about 0.6 TFLOP of oracle work (10-15 s on the box's host cores)."""
+    """Experts in the CPU sample: as asked, or about 0.6 TFLOP of oracle work (10-15 s on 16 host cores)."""
     if args.cpu_experts > 0:
         return min(args.cpu_experts, E)
     return max(1, min(E, int(6e11 * args.cpu_work / (2.0 * rows / E * K * N))))

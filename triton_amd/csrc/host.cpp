@@ -2,7 +2,7 @@
 // ABI, without going through Python objects, ctypes structures and the dispatcher for every field.
 //
 // What bounds it: at decode sizes a layer's kernels take 35 us and the Python host code of its five calls took 120
-// (matmul 19 us, routing 14, reduce 10, ... on the box's host): the GPU waited for the host.  Here a call costs the
+// (matmul 19 us, routing 14, reduce 10, ...): the GPU waited for the host.  Here a call costs the
 // reading of its arguments (about 50 ns per attribute), one caching-allocator request and the launch.
 //
 // Every function covers the calls that need no conversion and no error message -- GPU tensors of the types, layouts

@@ -1559,7 +1559,7 @@ inline void dense_grid(const tamd_matmul_args &a, int &block_m, int &grid_m) {
 
 // The tiled kernels of one activation type and one epilogue activation.  The two activations are compiled in
 // translation units of their own (moe_matmul_<type>.hip: none, moe_matmul_<type>_swiglu.hip: SwiGLU), which
-// is all that separates them: each unit holds 16 kernels of up to 20 unrolled epilogues.
+// is all that separates them: each unit holds 16 kernels of up to five tile sizes with all the forms of their epilogue.
 template <int XDT, int ACT>
 int dispatch_x16_act(const tamd_matmul_args &a, int block_m, int grid_m, hipStream_t st) {
   dense_grid(a, block_m, grid_m);

@@ -6,21 +6,21 @@
 // bytes per row and column (64 K of 16-bit values, 128 K of fp8), through a ring of three or four stages that is two or
 // three ahead of the matrix cores; rows and columns are 128-byte lines, requested whole.
 //
-// What bounds it.  With few rows per expert: HBM (the ring holds 64 KB or more of weights in flight per CU).  With full
-// tiles the LDS: per stage a wave of 128 x 64 reads 24 KB for 16 KB x 64 columns of products, and four such waves and
-// the copies take 1152 cycles at 128 bytes per cycle against 1024 of MFMA.  Hence the two K groups: waves 0-3 and 4-7
-// share the tile's four 64-column strips, each group multiplying one half of every stage, so that a SIMD holds two
-// waves for the LDS traffic of one (waves of 64 x 64 would read a third more).  Group 0 requests the next stage's copies
-// before its products and group 1 after them: a copy instruction holds its wave for about a hundred cycles, and with
-// both groups issuing at the same time the matrix cores idled meanwhile.  The groups' partial sums meet in LDS after the
-// loop, each group finishing one half of the row fragments.
+// What bounds it.  With few rows per expert: HBM (the ring holds 64 KB or more of weights in flight per CU).  With full tiles
+// the stages themselves: a stage's copies (one holds its wave for about a hundred cycles), its barrier and its LDS reads
+// follow one another.  In the layer of 1021 tokens over 32 experts (K 2880) the matrix cores are busy 25 % of the cycles, the
+// address units 63 %, LDS 11 %; at 1024 x 8192 x 8192 of fp8 53, 27 and 11 %.  Hence the two K groups: waves 0-3 and 4-7 share
+// the tile's four 64-column strips, each group multiplying one half of every stage, so that a SIMD holds two waves for the
+// operand reads of one (waves of 64 x 64 would read a third more), and group 0 requests the next stage's copies before its
+// products and group 1 after them: with both groups issuing at the same time the matrix cores idled meanwhile.  The groups'
+// partial sums meet in LDS after the loop, each group finishing one half of the row fragments.
 //
 // fp8 operands stay fp8 up to the registers and are widened there, so that the products are those of the widened operands:
 // exact, with float32 sums.  The MFMAs that take fp8 directly (32x32x16 and the scaled 32x32x64 alike) align the products of a
 // step at the largest one and drop what falls below: measured against 64-bit sums over K 512 .. 8192, they are off by 0.9 to
 // 1.5e-5 of the result (normal operands) and 6e-5 (operands over twelve binades) at every K, the bf16 MFMA by 0.2 to 3e-7.
-// 1024 x 8192 x 8192: 110 us, 1.25 PFLOP/s, which is the rate of large bf16 products on this part; 348 widened in a pass of its
-// own, 67 with the fp8 MFMA.
+// 1024 x 8192 x 8192: 110 us, 1.25 PFLOP/s (large bf16 products of the library reach 1.14 on this part; matrix cores busy 53 % of
+// the cycles, a stage holds 2048 cycles of MFMA then); 348 widened in a pass of its own, 67 with the fp8 MFMA.
 #pragma once
 #include "moe_matmul_impl.h"
 
@@ -254,7 +254,8 @@ __global__ __launch_bounds__(512, 1) void mm_kk_kernel(tamd_matmul_args a, int g
 // K loop streams 256 columns through one CU (10 x 6496 x 3096: 13 tiles of 3.3 MB each, 54 us; now 19).  Here a tile is one 64-column
 // strip, and a wave has a quarter of K to itself: its copies go through a ring of its own (three stages of up to 12 KB), so
 // the loop has no barrier; the partial sums meet in LDS, added in the order of the waves.  Bound by the copies a wave can
-// issue (one per 8 lines, about 100 cycles each): NA, the row copies of a stage, follows the tile's rows.
+// issue (27 x 6912 x 8192: twelve copies of 8 lines per stage, 157 cycles of a wave's life for each; the address units of the CUs
+// at work are busy 57 % of the time, their matrix cores 9 %): NA, the row copies of a stage, follows the tile's rows.
 template <int NA>
 struct NarrowShape {
   static constexpr int A_LINES = 8 * NA, STAGE = (A_LINES + 64) * 128, RING = 3;

@@ -651,7 +651,7 @@ __global__ __launch_bounds__(256) void upcast_cols_tile_kernel(
 // Up to how many tiles a tensor whose quantised axis is strided goes to the kernels of one column per thread instead of the tile
 // kernels.  A tile is 131072 elements to a workgroup whose passes follow one another, so that one round of tiles takes the
 // same time for few of them as for one per CU: 13 to 23 us to quantise, 8 to 12 to dequantise; the column kernels have 64 times
-// the workgroups and take about 4 us and 1 us per million elements.  Measured over 95 shapes [1 .. 8, 512 .. 2880, 512 .. 5760] of
+// the workgroups and take about 4 us and 1 us per million elements.  Measured over 97 shapes [1 .. 8, 512 .. 2880, 512 .. 5760] of
 // 5 to 300 tiles on 256 CUs, the lines with the least time lost to the wrong kernel (us, by tiles / by columns):
 //   quantising    float32  152 tiles 17.4 / 15.2, 168: 22.1 / 19.3, 192: 22.7 / 19.9, 195: 16.1 / 17.5, 216: 26.0 / 26.8
 //                 16-bit    96 tiles 16.3 / 13.5, 105: 17.3 / 15.5, 114: 17.0 / 15.5, 120: 17.8 / 18.2, 126: 17.2 / 19.1
