@@ -67,7 +67,7 @@ def test_ragged_with_gather_scatter_and_gate_weights(block_m, dtype, device):
 
 
 @pytest.mark.parametrize("sizes", [
-    [160] * 20 + [1] * 20,            # equal shares of the work would need more workgroups on an XCD than there are
+    [160] * 20 + [1] * 20,            # tiles of five row fragments and of one, twenty experts each
     [0, 33, 0, 128, 96, 1, 161, 64],  # every number of fragments, an absorbed remainder and one row more than that
     [5], [129],
 ])
