@@ -181,10 +181,12 @@ TAMD_DEVICE bool locate_tile(const tamd_matmul_args &a, int grid_n, int64_t grid
   return t.rows > 0;
 }
 
-// Tile of a workgroup for ragged problems whose row blocks absorb remainders (EXTRA > 0) and whose experts have a block or two.
-// The schedule's absorbed blocks do nothing: at 128 rows per expert they are a third of it, and XCD ranges of equal
-// numbers of its tiles leave the XCDs with unequal work (32 experts, 2880 x 2880, 128 bf16 rows each: 98 us, 76 so).  Here the
-// ranges are cut from the blocks that have rows, in expert order; up to `group` blocks of an expert run next to each other on
+// Tile of a workgroup of a ragged problem, from the slices' sizes alone: one round trip to memory where the schedule takes three
+// (its length, the entry, the slice), each about 0.8 us of a tile that may last 10 (with the row indices requested before the
+// first weights, see run_tile: 333 tokens over 32 experts, 2016 -> 2112, f16, layer 83.4 us -> 81.3).
+// Blocks that absorb remainders (EXTRA > 0) leave the absorbed ones out: at 128 rows per expert they are a third of the schedule,
+// and XCD ranges of equal numbers of its entries leave the XCDs with unequal work (32 experts, 2880 x 2880, 128 bf16 rows
+// each: 98 us, 76 so).  The ranges are in expert order; up to `group` blocks of an expert run next to each other on
 // a column tile.  (XCD ranges of equal estimated time with the longest tiles first take 2 us to find and read an expert's
 // weights once per block: 128 experts, 200 rows each, 2880 x 2880: 462 us against 414, fp8 rows 387 against 293 in plain order.
 // Where a launch is one to three rounds of tiles they win up to 7 % (32 experts of 160 bf16 rows, 2880 x 5760: 179 against 190),
@@ -200,10 +202,11 @@ TAMD_DEVICE bool locate_tile_live(const tamd_matmul_args &a, int grid_n, int gro
   int rows[kLivePerLane], offs[kLivePerLane];
 #pragma unroll
   for (int u = 0; u < kLivePerLane; ++u) {
-    const int e = lane * n_lane + u;
-    const bool in = u < n_lane && e < E;
-    rows[u] = in ? a.slice_sizes[e] : 0;
-    offs[u] = in ? a.slice_offs[e] : 0;
+    rows[u] = offs[u] = 0;
+    if (u == 0 || u < n_lane) {   // (wave uniform)
+      const int e = lane * n_lane + u;
+      if (e < E) rows[u] = a.slice_sizes[e], offs[u] = a.slice_offs[e];
+    }
   }
   // (a block that starts past the first needs more than EXTRA rows)
   auto blocks = [](int n) { return n > BLOCK_M ? (n - EXTRA + BLOCK_M - 1) / BLOCK_M : (n > 0 ? 1 : 0); };
@@ -229,7 +232,9 @@ TAMD_DEVICE bool locate_tile_live(const tamd_matmul_args &a, int grid_n, int gro
   t.start_m = __builtin_amdgcn_readlane(off, src);
   const int slice_rows = __builtin_amdgcn_readlane(n, src);
   const uint32_t local = idx - (uint32_t)__builtin_amdgcn_readlane(before, src) * gn;   // tile of the expert
-  const uint32_t b = (uint32_t)blocks(slice_rows), g = b < (uint32_t)group ? b : (uint32_t)group;
+  const uint32_t b = (uint32_t)blocks(slice_rows);
+  uint32_t g = b < (uint32_t)group ? b : (uint32_t)group;
+  if (g > 1) g = (b + (b + g - 1) / g - 1) / ((b + g - 1) / g);   // (groups of about one size)
   const uint32_t gi = local / (g * gn), r = local - gi * g * gn;
   const uint32_t size = b - gi * g < g ? b - gi * g : g, col = r / size;
   t.n0 = (int)col * BLOCK_N;
@@ -299,6 +304,21 @@ TAMD_DEVICE void wait_vmcnt() {
   static_assert(N >= 0 && N < 64, "vmcnt is a 6-bit counter");
   __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N >> 4) << 14) | (0x7 << 4) | (0xF << 8));
   asm volatile("" ::: "memory");
+}
+
+// A dword from memory into a register, requested through inline asm as well: the compiler would wait for an ordinary load with a
+// count that takes in the LDS copies requested after it, which it does not see.  `v` must not be touched before
+// await_dwords<N>, which waits until at most the N newest requests of the wave are outstanding.
+TAMD_DEVICE uint32_t request_dword(v4i_t rsrc, uint32_t voff) {
+  uint32_t v;
+  asm volatile("s_nop 4\n\tbuffer_load_dword %0, %1, %2, 0 offen" : "=v"(v) : "v"(voff), "s"(rsrc) : "memory");
+  return v;
+}
+template <int N, int COUNT>
+TAMD_DEVICE void await_dwords(uint32_t (&v)[COUNT]) {
+  asm volatile("s_waitcnt vmcnt(%1)" : "+v"(v[0]) : "n"(N) : "memory");
+#pragma unroll
+  for (int i = 1; i < COUNT; ++i) asm volatile("" : "+v"(v[i]));
 }
 
 TAMD_DEVICE v4i_t make_rsrc(const void *base, uint32_t num_records) {
@@ -858,6 +878,7 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
   const int KSP = (G + 7) / 8 * 8;
   const int tile_cols = N - t.n0 < BLOCK_N ? N - t.n0 : BLOCK_N;
   const int64_t sc_tile_off = cdna4 ? (int64_t)(t.n0 / 32) * KSP * 32 : (int64_t)t.n0 * G;
+  auto stage_scales = [&]() {
   if constexpr (SC_LDS) {
     const uint8_t *sc_src = s_base + sc_tile_off;
     const int sc_tile_bytes = BLOCK_N * (cdna4 ? KSP : G);
@@ -889,6 +910,7 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
       }
     }
   }
+  };
   // offset of a column's scales inside the tile's image (LDS) or, without staging, from the expert's first scale
   int sc_col_off[NF];
 #pragma unroll
@@ -917,16 +939,10 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
   const uint64_t as_at = (uint64_t)(uintptr_t)a.x_mx_scale | (uint64_t)a.x_mx_stride_m | (uint64_t)a.x_mx_stride_z | (uint64_t)G;
   const int as_w = (as_at & 3) == 0 ? 4 : ((as_at & 1) == 0 ? 2 : 1);
   v4i_t ras = rx;
-  uint32_t as_off = kOob;
+  uint32_t as_off = kOob;   // (set below, with the rows' offsets)
   if (x_mx) {
     const int64_t xr = a.x_rows > 0 ? a.x_rows : a.M;
     ras = make_rsrc(a.x_mx_scale + (int64_t)t.z * a.x_mx_stride_z, (uint32_t)(xr * a.x_mx_stride_m));
-    const int r = wave * 64 + lane;
-    if (wave * 64 < LDS_ROWS && r < LDS_ROWS) {
-      const int rr = t.off_m + (r < t.rows ? r : t.rows - 1);
-      const uint32_t src = a.gather_indx ? (uint32_t)a.gather_indx[t.start_m + rr] : (uint32_t)(t.start_m + rr);
-      as_off = src * (uint32_t)a.x_mx_stride_m;
-    }
   }
   // Copies per request, as the counted waits of the ring loops below see them (a wave's copies complete in the order
   // of their requests): the loops of the issue_* functions run to these numbers and the waits are written in them.
@@ -955,16 +971,52 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
   // ---- activation DMA: one instruction per 32-row fragment, lane -> (row 8w + lane/8, slot lane%8)
   const int a_rin = wave * 8 + lane / 8;
   const int a_chunk = (lane % 8) ^ ((a_rin >> 1) & 7);
-  uint32_t a_off[NFR];
+  uint32_t a_off[NFR];   // (set below)
+  // The rows' indices are the first thing requested: the first weights, which do not depend on them, are requested while they
+  // come.  (One fragment's lane holds a row of each fragment, then the row whose block scales it copies.)
+  constexpr bool AS = FP8;
+  const v4i_t rg = make_rsrc(a.gather_indx ? a.gather_indx + t.start_m + t.off_m : nullptr, a.gather_indx ? (uint32_t)__builtin_amdgcn_readfirstlane(t.rows) * 4u : 0u);
+  uint32_t row_idx[NFR + (AS ? 1 : 0)];
 #pragma unroll
-  for (int i = 0; i < NFR; ++i) {
-    const int r = i * 32 + a_rin;
-    // rows past the end of the slice are never stored: they are copied as zeros (out-of-range offset), which
-    // keeps the matrix cores' inputs quiet for the padding of a ragged tile
-    const int rr = t.off_m + (r < t.rows ? r : t.rows - 1);
-    const uint32_t src = a.gather_indx ? (uint32_t)a.gather_indx[t.start_m + rr] : (uint32_t)(t.start_m + rr);
-    a_off[i] = r < t.rows ? src * (uint32_t)(a.x_stride_m * ESZ) + a_chunk * 16 : kOob;
+  for (int i = 0; i < NFR; ++i) row_idx[i] = request_dword(rg, (uint32_t)(i * 32 + a_rin) * 4u);
+  if constexpr (AS) row_idx[NFR] = request_dword(rg, (uint32_t)(wave * 64 + lane) * 4u);
+  // One byte per line of what only the epilogue reads -- the bias of the wave's columns, the rows' destinations and factors, the
+  // scales -- so that it finds them in the caches (a tile of few stages spent 1 us of its 10 waiting for them).  The
+  // byte lands in a register that nothing else may take before the K loop has waited for it.
+  uint32_t warm = 0;
+  {
+    const uint8_t *p = (const uint8_t *)a.x;
+    const int col = t.n0 + wave * 64 + lane * 16, row = (lane & 7) * 32;
+    const int64_t erow = t.start_m + t.off_m + (row < t.rows ? row : t.rows - 1);
+    const int kind = lane >> 3;
+    if (kind == 0 && a.bias && lane < 4)
+      p = (const uint8_t *)a.bias + ((int64_t)t.expert * a.bias_stride_e + (col < N ? col : N - 1)) * (a.bias_dtype == TAMD_F32 ? 4 : 2);
+    if (kind == 1 && a.scatter_indx) p = (const uint8_t *)(a.scatter_indx + erow);
+    if (kind == 2 && a.gammas) p = (const uint8_t *)(a.gammas + erow);
+    if (kind == 3 && a.betas) p = (const uint8_t *)(a.betas + erow);
+    if (lane == 32 && a.x_scale) p = (const uint8_t *)a.x_scale;
+    if (lane == 33 && a.w_scale) p = (const uint8_t *)a.w_scale;
+    if (lane == 34 && a.y_expected_scale) p = (const uint8_t *)a.y_expected_scale;
+    asm volatile("global_load_ubyte %0, %1, off" : "+v"(warm) : "v"(p) : "memory");
   }
+  // (after `newer` further requests of the wave)
+  auto rows_known = [&](auto newer) {
+    await_dwords<decltype(newer)::value + 1>(row_idx);   // (and the byte above)
+    const int row0 = t.start_m + t.off_m;
+#pragma unroll
+    for (int i = 0; i < NFR; ++i) {
+      // rows past the end of the slice are never stored: they are copied as zeros (out-of-range offset), which
+      // keeps the matrix cores' inputs quiet for the padding of a ragged tile
+      const int r = i * 32 + a_rin;
+      const uint32_t src = a.gather_indx ? row_idx[i] : (uint32_t)(row0 + r);
+      a_off[i] = r < t.rows ? src * (uint32_t)(a.x_stride_m * ESZ) + a_chunk * 16 : kOob;
+    }
+    if constexpr (AS) {
+      const int r = wave * 64 + lane;
+      const uint32_t src = a.gather_indx ? row_idx[NFR] : (uint32_t)(row0 + r);
+      if (x_mx && r < t.rows) as_off = src * (uint32_t)a.x_mx_stride_m;
+    }
+  };
   // ---- weight DMA: instruction j copies LDS positions j*16 + lane/4, part slot lane%4
   // Codes in the block layout (TAMD_W_CDNA4_BLOCKS): a stage of this wave's strip is one 4 KB block that already has
   // the LDS image's order, so the four copies are linear (whole, aligned lines) and the K stage enters through the
@@ -1233,7 +1285,6 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
 
   typedef std::integral_constant<int, 0> Set0;
   typedef std::integral_constant<int, 1> Set1;
-  uint32_t warm = 0;   // (K groups: a byte fetched only to warm the caches, see below)
   if constexpr (RING) {
     // Copies complete in the order of their requests, so a stage waits by count for what it needs and leaves the
     // later requests in flight.
@@ -1250,8 +1301,10 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
     if constexpr (PAIRED) {
       // Three activation stages; an even stage s moves the weights of s and s + 1 into registers and requests those of
       // s + 2 and s + 3 (one pair), the odd stage requests only activations.
+      issue_b_pair(0);
+      rows_known(std::integral_constant<int, CP_BPAIR>{});
       issue_a(0), issue_as(0);
-      issue_b_pair(0), issue_sc(0), issue_sc(1);
+      issue_sc(0), issue_sc(1);
       issue_a(1), issue_as(1);
       for (int it = 0; it < n_ka; it += 2) {
         // in flight at most: the activations of stage it + 1
@@ -1281,8 +1334,9 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
       // Stage s requests the activations of stage s + 1 and then the weights and scales of stage s + 2 (the weight
       // buffer of stage s is free as soon as its contents are in registers): in flight at the top of a stage are at
       // most the weights and scales the stage before requested (5 copies, or 8 with strided scales).
-      issue_b(0), issue_sc(0);
-      issue_a(0), issue_as(0), issue_b(1), issue_sc(1);
+      issue_b(0);
+      rows_known(std::integral_constant<int, CP_B>{});
+      issue_sc(0), issue_a(0), issue_as(0), issue_b(1), issue_sc(1);
       for (int it = 0; it < n_ka; ++it) {
         if (cdna4) wait_vmcnt<CP_B + 1>(); else wait_vmcnt<CP_B + NSC>();
         __syncthreads();
@@ -1297,8 +1351,11 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
       }
     }
   } else {
-  issue_a(0);
+  // (the scales of the whole tile are first read in stage 0: requested behind that stage's own copies, before any later one)
   issue_b(0);
+  rows_known(std::integral_constant<int, CP_B>{});
+  issue_a(0);
+  if constexpr (SC_LDS) stage_scales();
   if constexpr (FP8) {
     issue_as(0);
     for (int it = 0; it < n_ka; ++it) {  // activation and weight stages coincide (128 K each)
@@ -1313,26 +1370,17 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
       compute(it, Set0{}, Set0{});
     }
   } else if constexpr (DEEP) {
-    if constexpr (KS > 1) {
-      // A K-group tile's fixed costs are a third of its time, so the first thing its epilogue fetches -- the bias of the
-      // lane's columns -- is requested here already.  The request is older than every copy (the counted waits cover
-      // it) and only warms the caches: the byte is dropped after the loop.
-      if (a.bias && grp == 0) {
-        const int esz = a.bias_dtype == TAMD_F32 ? 4 : 2;
-        const uint8_t *bp = (const uint8_t *)a.bias + (col0 < N ? ((int64_t)t.expert * a.bias_stride_e + col0) * esz : 0);
-        asm volatile("global_load_ubyte %0, %1, off" : "=v"(warm) : "v"(bp) : "memory");
-      }
-    }
     // Stage s requests the activations of stage s + DA - 1, an even stage after them the weights of pair s/2 + DB
     // (a weight region is free once its pair's weights are in registers).  Copies complete in the order of their
     // requests: a stage waits until only the requests made after the ones it needs are outstanding
     // (ring_outstanding).  The requests before the loop are those of the stages before 0, in the same order, so the
     // counts hold from the first stage on.
+    // (The first stage's own copies, and the tile's scales, have been requested above.)
     constexpr int PRE = DA - 1 > 2 * DB ? DA - 1 : 2 * DB;
 #pragma unroll
     for (int j = -PRE; j < 0; ++j) {
-      if (j + DA - 1 >= 0) issue_a(j + DA - 1);
-      if (j % 2 == 0 && j / 2 + DB >= 0) issue_b(j / 2 + DB);
+      if (j + DA - 1 > 0) issue_a(j + DA - 1);
+      if (j % 2 == 0 && j / 2 + DB > 0) issue_b(j / 2 + DB);
     }
     const int n_stage = KS > 1 ? 2 * n_sup : n_ka;   // (K groups: the same trip count, and barriers, for every group)
     for (int it = 0; it < n_stage; it += 2) {
@@ -1371,7 +1419,7 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
   }
   }
   wait_dma();
-  if constexpr (KS > 1) asm volatile("" ::"v"(warm));
+  asm volatile("" ::"v"(warm));
 
   if constexpr (KS > 1) {
     // The groups' partial sums meet in LDS (the pipelines are dead: after the barrier every copy has landed and every
@@ -1426,7 +1474,7 @@ template <int XDT, int BM, int ACT, bool SC_LDS, int KS = 1>
 TAMD_DEVICE void tile_entry(const tamd_matmul_args &a, int grid_n, int64_t grid_total, int group_m, uint8_t *lds) {
   typedef TileShape<XDT, BM> S;
   Tile t;
-  if (S::EXTRA > 0 && group_m < 0) {  // absorbed blocks left out of the count; -group_m blocks of an expert together
+  if (group_m < 0) {  // from the slices' sizes; up to -group_m blocks of an expert together
     if (!locate_tile_live<BM, S::EXTRA>(a, grid_n, -group_m, t)) return;
   } else if (!locate_tile<BM, S::EXTRA>(a, grid_n, grid_total, group_m, t)) return;
   const int nfr = (t.rows + 31) / 32;  // active row fragments (workgroup uniform)
@@ -1460,11 +1508,8 @@ __global__ __launch_bounds__(256, 2) void mm_x8_mxfp4_kernel(tamd_matmul_args a,
   tile_entry<XDT, BM, ACT, SC_LDS>(a, grid_n, grid_total, group_m, lds);
 }
 
-// Whether a ragged problem takes locate_tile_live: absorbed blocks exist and the experts fit its lanes.
-template <int XDT, int BM>
-bool counts_live_blocks(const tamd_matmul_args &a) {
-  return TileShape<XDT, BM>::EXTRA > 0 && a.block_schedule && a.n_experts <= kWave * kLivePerLane;
-}
+// Whether a problem takes locate_tile_live: it is ragged and the experts fit the lanes.
+inline bool counts_live_blocks(const tamd_matmul_args &a) { return a.block_schedule && a.n_experts <= kWave * kLivePerLane; }
 
 template <int XDT, int BM, int ACT>
 int launch_x16_act(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
@@ -1504,6 +1549,7 @@ int launch_x16_act(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
   const int64_t fit = (int64_t)(2.5 * 1024 * 1024) / ((int64_t)BM * a.K * (is_fp8(XDT) ? 1 : 2));
   group_m = group_m > fit ? fit : group_m;
   group_m = group_m < 1 ? 1 : (group_m > 16 ? 16 : group_m);
+  if (counts_live_blocks(a)) group_m = -group_m;
   if constexpr (!is_fp8(XDT) && BM <= 32) {
     // Fewer tiles than CUs: K groups, so that every SIMD of the CUs that do get a tile holds two to four waves
     // (at least two 128-K pairs per group; the groups' pipelines and the tile's scales have to fit one CU's LDS)
@@ -1525,8 +1571,6 @@ int launch_x16_act(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
     }
   }
   if (int rc = raise_lds_limit_once((const void *)kern)) return rc;
-  // (an expert's blocks one after the other: with two workgroups per CU an XCD holds 64 tiles, its column tiles of both)
-  if (counts_live_blocks<XDT, BM>(a) && group_m == 1) group_m = -1;
   kern<<<dim3((unsigned)launch), 256, lds_bytes, st>>>(a, grid_n, total, (int)group_m);
   return launch_status();
 }

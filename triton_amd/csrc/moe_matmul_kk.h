@@ -415,7 +415,7 @@ int launch_kk(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
   if (int rc = raise_lds_limit_once((const void *)kern)) return rc;
   // (one workgroup per CU: an XCD holds 32 tiles, and an expert's blocks share a column tile only side by side; 32 experts
   // of 250 bf16 rows, 2880 x 2880: 181 us in fours, 199 one after the other, 217 in schedule order)
-  if (counts_live_blocks<XDT, BM>(a) && group_m <= 2) group_m = -4;
+  if (TileShape<XDT, BM>::EXTRA > 0 && counts_live_blocks(a) && group_m <= 2) group_m = -4;
   kern<<<dim3((unsigned)launch), 512, KKShape<XDT, BM>::LDS, st>>>(a, grid_n, total, (int)group_m);
   return launch_status();
 }
