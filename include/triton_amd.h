@@ -223,8 +223,8 @@ int tamd_routing_metadata_static(const void *indx, int indx_is_int16, int64_t n_
 typedef struct tamd_matmul_args {
   /* activations: [M_x, K], unit stride along K */
   const void *x;
-  int x_dtype; /* TAMD_BF16 / TAMD_F16 / TAMD_FP8_E4M3 / TAMD_FP8_E5M2 */
-  int64_t x_stride_m;
+  int x_dtype; /* TAMD_BF16 / TAMD_F16 / TAMD_FP8_E4M3 / TAMD_FP8_E5M2; TAMD_MXFP4: packed e2m1 codes with x_mx_scale, K >= 256 */
+  int64_t x_stride_m; /* in elements (bytes for TAMD_MXFP4) */
   const float *x_scale; /* per-tensor flex scale (device scalar) or NULL */
   /* weights: n_experts x [K, N]; MXFP4: packed bytes, K/2 bytes contiguous per column.  TAMD_BF16 / TAMD_F16
    * weights must have the activations' type, unit stride along K or along N, and K % 8 == 0 (N % 8 == 0 too when
@@ -281,7 +281,7 @@ typedef struct tamd_matmul_args {
    * tensor_details/layout_details/cdna4_scale.py:32-68 (per expert: ceil(N/32) blocks of ceil(K/256)*8*32 bytes,
    * 16-byte aligned; only w_mx_stride_e is used) */
   int w_mx_layout;
-  /* microscaled activations (MXFP8: x_dtype TAMD_FP8_E4M3 with one e8m0 byte per 32 elements of a row, the
+  /* microscaled activations (x_dtype TAMD_FP8_E4M3 or TAMD_MXFP4 with one e8m0 byte per 32 elements of a row, the
    * a_mx_scale of matmul.py:131-136): [x_rows, K/32] bytes, unit stride along K/32, indexed by the same (gathered)
    * row as x; NULL = no block scales.  x_mx_stride_z is the batch pitch. */
   const uint8_t *x_mx_scale;

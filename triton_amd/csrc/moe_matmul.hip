@@ -11,6 +11,7 @@ int dispatch_mm_bf16(const tamd_matmul_args &a, int block_m, int grid_m, hipStre
 int dispatch_mm_f16(const tamd_matmul_args &a, int block_m, int grid_m, hipStream_t st);
 int dispatch_mm_fp8e4m3(const tamd_matmul_args &a, int block_m, int grid_m, hipStream_t st);
 int dispatch_mm_fp8e5m2(const tamd_matmul_args &a, int block_m, int grid_m, hipStream_t st);
+int dispatch_mm_fp4(const tamd_matmul_args &a, int block_m, int grid_m, hipStream_t st);
 int dispatch_mm_w16_bf16(const tamd_matmul_args &a, int block_m, int grid_m, hipStream_t st);
 int dispatch_mm_w16_f16(const tamd_matmul_args &a, int block_m, int grid_m, hipStream_t st);
 int dispatch_mm_kk_fp8e4m3(const tamd_matmul_args &a, int block_m, int grid_m, hipStream_t st);
@@ -44,8 +45,9 @@ extern "C" int tamd_matmul_sized(const tamd_matmul_args *args, size_t args_size,
   hipStream_t st = (hipStream_t)stream;
 
   const bool x8 = a.x_dtype == TAMD_FP8_E4M3 || a.x_dtype == TAMD_FP8_E5M2;
-  if (a.w_dtype == TAMD_MXFP4 && (a.x_dtype == TAMD_BF16 || a.x_dtype == TAMD_F16 || x8)) {
-    const int esz = x8 ? 1 : 2;
+  const bool x4 = a.x_dtype == TAMD_MXFP4;   // packed e2m1 rows: x strides in bytes
+  if (a.w_dtype == TAMD_MXFP4 && (a.x_dtype == TAMD_BF16 || a.x_dtype == TAMD_F16 || x8 || x4)) {
+    const int esz = x8 || x4 ? 1 : 2;
     if (!a.w_mx_scale) return TAMD_E_INVALID;
     if (a.K % 32 != 0) return TAMD_E_INVALID;
     // weights / scales must be contiguous along K ("column-major" mxfp weights)
@@ -68,10 +70,11 @@ extern "C" int tamd_matmul_sized(const tamd_matmul_args *args, size_t args_size,
         (int64_t)a.N * (cdna4_sc ? (int64_t)(a.K / 32 + 7) : a.w_mx_stride_n) >= (int64_t)0x7FFFFF00)
       return TAMD_E_UNSUPPORTED;
     if (a.x_mx_scale) {
-      // block scales of the activations: MXFP8 (e4m3 values) through the scaled MFMA only
-      if (!x8) return TAMD_E_UNSUPPORTED;
+      // block scales of the activations: MXFP8 (e4m3 values) and MXFP4 through the scaled MFMA only
+      if (!x8 && !x4) return TAMD_E_UNSUPPORTED;
       if (a.x_mx_stride_m < a.K / 32 || x_rows * a.x_mx_stride_m >= (int64_t)0x7FFFFF00) return TAMD_E_UNSUPPORTED;
     }
+    if (x4 && !a.x_mx_scale) return TAMD_E_INVALID;
     int block_m, grid_m;
     if (ragged) {
       block_m = a.block_m;
@@ -81,6 +84,7 @@ extern "C" int tamd_matmul_sized(const tamd_matmul_args *args, size_t args_size,
       block_m = a.force_variant;
       grid_m = block_m ? ((a.M + block_m - 1) / block_m) * a.n_experts : 0;
     }
+    if (x4) return dispatch_mm_fp4(a, block_m, grid_m, st);
     if (a.x_dtype == TAMD_BF16) return dispatch_mm_bf16(a, block_m, grid_m, st);
     if (a.x_dtype == TAMD_F16) return dispatch_mm_f16(a, block_m, grid_m, st);
     if (a.x_dtype == TAMD_FP8_E5M2) return dispatch_mm_fp8e5m2(a, block_m, grid_m, st);

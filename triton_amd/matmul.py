@@ -81,10 +81,19 @@ def _data(t):
     return t.storage.data if isinstance(t, Tensor) else t
 
 
+def _packed_rows_direct(a_raw, flex, ragged):
+    """MXFP4 activations (packed e2m1 codes along K with one e8m0 byte per 32, matmul.py:131-136 of the reference) that
+    the kernel for them reads as they are: whole, aligned 16-byte chunks, K of at least a stage, no split of K (whose
+    ranges are cut in elements), no other type asked for."""
+    split = _opt_flags._constraints().get("split_k") is not None or _opt_flags._opt_flags.get() is not None
+    auto_split = not ragged and a_raw.ndim == 2 and a_raw.shape[0] <= 256 and 2 * a_raw.shape[-1] >= 8192
+    return (not split and not auto_split and flex.lhs_data.dtype is None and a_raw.is_cuda and a_raw.stride(-1) == 1
+            and a_raw.shape[-1] >= 128 and a_raw.data_ptr() % 16 == 0 and all(s % 16 == 0 for s in a_raw.stride()[:-1]))
+
+
 def _widen_mxfp4_activations(a_raw):
-    """MXFP4 activations (packed e2m1 codes along K with one e8m0 byte per 32, matmul.py:131-136 of the reference)
-    against MXFP4 weights: the codes are widened -- exactly: every e2m1 number is a float8_e4m3fn number -- and take
-    the MXFP8 path of the kernels with the same scales."""
+    """MXFP4 activations that the kernel for them does not take: the codes are widened -- exactly: every e2m1 number is
+    a float8_e4m3fn number -- and take the MXFP8 path of the kernels with the same scales."""
     _lib.require_gpu(a_raw, "a")
     assert a_raw.stride(-1) == 1, "packed activations must be contiguous along K"
     rows = a_raw.numel() // a_raw.shape[-1]
@@ -196,6 +205,8 @@ def matmul(a, b, bias, a_ragged_metadata: Optional[RaggedTensorMetadata] = None,
     if precision_config.acc_scale != 1.0:
         raise NotImplementedError("acc_scale other than 1.0 is not built")
     a_mx_scale = precision_config.a_mx_scale
+    flex = precision_config.flex_ctx
+    a_packed = False   # packed e2m1 rows handed to the kernel as they are
     if a_mx_scale is not None:
         a_mx_scale = _data(a_mx_scale)
         a_raw = a.storage.data if isinstance(a, Tensor) else a
@@ -217,8 +228,8 @@ def matmul(a, b, bias, a_ragged_metadata: Optional[RaggedTensorMetadata] = None,
                                  axis=-1)
             a_mx_scale = None
         elif a_fp4:
-            a = _widen_mxfp4_activations(a_raw)
-    flex = precision_config.flex_ctx
+            a_packed = _packed_rows_direct(a_raw, flex, a_ragged_metadata is not None)
+            a = a_raw if a_packed else _widen_mxfp4_activations(a_raw)
     if flex.acc_data.scale is not None:
         raise NotImplementedError("accumulator flex scale is not built")
     if flex.out_data.checksum_scale is not None:
@@ -284,7 +295,7 @@ def matmul(a, b, bias, a_ragged_metadata: Optional[RaggedTensorMetadata] = None,
     _lib.require_gpu(w, "b")
     assert a.stride(-1) == 1 or a.shape[-1] == 1, "a must be contiguous along K"
     # ---- shapes
-    K = a.shape[-1]
+    K = a.shape[-1] * (2 if a_packed else 1)
     K_W, N = b_shape[-2:]
     assert K == K_W, f"inner dimensions differ: {K} vs {K_W}"
     ragged = a_ragged_metadata is not None
@@ -340,9 +351,9 @@ def matmul(a, b, bias, a_ragged_metadata: Optional[RaggedTensorMetadata] = None,
     # ---- tile choice
     flags = make_opt_flags(M, N, K, n_slices, ragged,
                            a_ragged_metadata.expected_slice_size if ragged else None,
-                           fp8_rows=a.dtype in fp8_types and b_fp4)
+                           fp8_rows=(a_packed or a.dtype in fp8_types) and b_fp4)
     args = _lib.MatmulArgBag()
-    args.x, args.x_dtype = a.data_ptr(), _lib.dtype_code(a.dtype)
+    args.x, args.x_dtype = a.data_ptr(), _lib.MXFP4 if a_packed else _lib.dtype_code(a.dtype)
     args.x_stride_m = a.stride(-2)
     args.x_stride_z = a.stride(0) if a.ndim == 3 else 0
     args.x_scale = None if flex.lhs_data.scale is None else flex.lhs_data.scale.data_ptr()
