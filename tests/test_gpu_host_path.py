@@ -256,3 +256,50 @@ def test_native_reduce_is_the_general_path(shape, dim, dtype, device, monkeypatc
     for t in (x, x.transpose(0, 2).contiguous().transpose(0, 2)):
         assert BothPaths(monkeypatch, "reduce")(lambda: [reduce(t, dim=dim)[0]]) == (shape[dim] < 512)
         monkeypatch.undo()
+
+
+@pytest.mark.parametrize("layout", ["strided", "blocks"])
+@pytest.mark.parametrize("form,covered", [("gather swiglu", True), ("scatter", True), ("dense", True), ("out type", True), ("c", True),
+                                          ("lhs type", False), ("pitch", False), ("short", False), ("split_k", False)])
+def test_native_matmul_of_packed_rows(form, covered, layout, device, monkeypatch):
+    """Packed e2m1 rows: what their kernel reads as it is goes the native way."""
+    g = torch.Generator(device=device).manual_seed(11)
+    T, E, k, K, N = 37, 1 if form in ("dense", "split_k") else 8, 4, {"short": 224, "split_k": 8192}.get(form, 288), 192
+    rnd = lambda *s: torch.randn(s, generator=g, device=device).bfloat16()
+    v, s = downcast_to_mxfp(rnd(E, N, K) * 0.1, torch.uint8, axis=-1)
+    w, s = v.transpose(-1, -2), s.transpose(-1, -2)
+    if layout == "blocks":
+        w, s = (convert_layout(wrap_torch_tensor(w, dtype=FP4), CDNA4MXValueLayout()),
+                convert_layout(wrap_torch_tensor(s), CDNA4MXScaleLayout()))
+    r = None if E == 1 else routing(torch.randn((T, E), generator=g, device=device), k)
+    gathered = form == "gather swiglu"
+    x, xs = downcast_to_mxfp(rnd(T if r is None or gathered else T * k, K), torch.uint8, axis=-1)
+    if form == "pitch":
+        x = torch.cat([x, x[:, :8]], dim=1)[:, :K // 2]
+    bias, M = rnd(E, N), T if r is None else T * k
+    lhs = InFlexData(F8) if form == "lhs type" else InFlexData()
+
+    def call():
+        pc = PrecisionConfig(flex_ctx=FlexCtx(lhs_data=lhs), a_mx_scale=xs, a_microblock_size=32, b_mx_scale=s, b_microblock_size=32,
+                             out_dtype=torch.float32 if form == "out type" else None)
+        c = torch.zeros((M, N), dtype=torch.bfloat16, device=device) if form == "c" else None
+        return [matmul(x, w, bias if r is not None else bias[0], r.ragged_metadata if r is not None else None,
+                       gather_indx=r.gather_indx if gathered else None, scatter_indx=r.scatter_indx if form == "scatter" else None,
+                       precision_config=pc, c=c, fused_activation=SWIGLU if gathered else None)]
+
+    assert BothPaths(monkeypatch, "matmul")(call) == covered
+
+
+def test_native_matmul_fills_in_the_output_block_size(device, monkeypatch):
+    torch.manual_seed(12)
+    x, xs = downcast_to_mxfp(torch.randn(5, 64, device=device).bfloat16(), F8, axis=-1)
+    v, s = downcast_to_mxfp(torch.randn(96, 64, device=device).bfloat16(), torch.uint8, axis=-1)
+
+    def call():
+        ys = torch.zeros((5, 3), dtype=torch.uint8, device=device)
+        pc = PrecisionConfig(a_mx_scale=xs, a_microblock_size=32, b_mx_scale=s.t(), b_microblock_size=32, c_mx_scale=ys)
+        y = matmul(x, v.t(), None, precision_config=pc, epilogue=Epilogue(FnSpecs("QUANTIZE_MXFP8", None, (), ()), (), (), 6.0))
+        assert pc.c_microblock_size == 32
+        return [y, ys]
+
+    assert BothPaths(monkeypatch, "matmul")(call)

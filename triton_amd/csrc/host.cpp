@@ -203,13 +203,16 @@ PyObject *py_matmul(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
     const at::Tensor &a = gpu_tensor(a_o, dev);
     need(a.dim() == 2);
     const at::ScalarType a_type = a.scalar_type();
-    const int64_t K = a.size(1), a_rows = a.size(0);
-    need(a.stride(1) == 1 && K > 1);
+    const bool a4 = a_type == at::kByte;  // packed e2m1 rows (with block scales)
+    const int64_t K = a.size(1) * (a4 ? 2 : 1), a_rows = a.size(0);
+    need(a.stride(1) == 1 && a.size(1) > 1);
     tamd_matmul_args g;
     std::memset(&g, 0, sizeof g);
-    g.x_dtype = type_code(a_type);
+    g.x_dtype = a4 ? TAMD_MXFP4 : type_code(a_type);
     need(g.x_dtype != TAMD_F32);
     const bool a8 = is_fp8_code(g.x_dtype);
+    if (a4)  // what the kernel for them reads as it is (_packed_rows_direct; anything else is widened by the general path)
+      need(K >= 256 && a.stride(0) % 16 == 0 && (uintptr_t)a.data_ptr() % 16 == 0);
 
     // ---- precision options
     bool mx_out = false, a_mx = false;
@@ -225,7 +228,7 @@ PyObject *py_matmul(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
       Ref ams(attr(pc, nm.a_mx_scale));
       if (!ams.none()) {
         a_mx = true;
-        need(g.x_dtype == TAMD_FP8_E4M3);
+        need(g.x_dtype == TAMD_FP8_E4M3 || a4);
         const at::Tensor &s = gpu_tensor(ams.p, dev);
         need(s.scalar_type() == at::kByte && s.dim() == 2 && s.size(0) == a_rows && s.size(1) == K / 32 &&
              (s.stride(1) == 1 || s.size(1) == 1));
@@ -239,14 +242,23 @@ PyObject *py_matmul(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
       mx_out = !cms.none();
       if (mx_out) {
         Ref pf(attr(pc, nm.c_value_pack_factor)), mb(attr(pc, nm.c_microblock_size));
-        need(as_int(pf.p) == 1 && !mb.none() && as_int(mb.p) == 32);  // (left out: filled in by the general path)
+        need(as_int(pf.p) == 1);
+        if (mb.none()) {  // left out: filled in for the caller, as the general path does
+          Ref size(PyLong_FromLong(32));
+          if (!size.p || PyObject_SetAttr(pc, nm.c_microblock_size, size.p) != 0) {
+            PyErr_Clear();
+            throw Miss{};
+          }
+        } else {
+          need(as_int(mb.p) == 32);
+        }
       }
       Ref fc(attr(pc, nm.flex_ctx));
       Ref lhs(attr(fc.p, nm.lhs_data)), rhs(attr(fc.p, nm.rhs_data)), outd(attr(fc.p, nm.out_data)), accd(attr(fc.p, nm.acc_data));
       Ref ls(attr(lhs.p, nm.scale)), rs(attr(rhs.p, nm.scale)), as(attr(accd.p, nm.scale));
       need(as.none());
       Ref ld(attr(lhs.p, nm.dtype));
-      need(ld.none() || !a8 || dtype_of(ld.p) == a_type);  // (another 8-bit type: reinterpreted by the general path)
+      need(ld.none() || (!a8 && !a4) || (a8 && dtype_of(ld.p) == a_type));  // (another 8-bit type: reinterpreted by the general path)
       g.x_scale = scalar_ptr(ls.p, dev);
       g.w_scale = scalar_ptr(rs.p, dev);
       Ref rd(attr(rhs.p, nm.dtype));  // (weights of another 8-bit type: reinterpreted by the general path)
@@ -259,6 +271,7 @@ PyObject *py_matmul(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
       need(PyBool_Check(si.p));
       g.y_saturate_inf = si.p == Py_True;
     }
+    need(!a4 || a_mx);
     // ---- epilogue and activation
     if (ep != Py_None) {
       Ref sp(attr(ep, nm.specs));
@@ -315,7 +328,7 @@ PyObject *py_matmul(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
       const at::Tensor &w = gpu_tensor(b_o, dev);
       need((w.dim() == 3 || w.dim() == 2) && w.stride(-2) == 1 && w.size(-2) > 1);
       w_fp4 = w.scalar_type() == at::kByte;
-      need(w_fp4 || w.scalar_type() == a_type);
+      need(w_fp4 || (w.scalar_type() == a_type && !a4));
       if (a8 && !w_fp4)  // fp8 x fp8: whole, aligned 16-byte chunks along K (otherwise widened by the general path)
         need(!a_mx && K % 16 == 0 && w.stride(-1) % 16 == 0 && (w.dim() == 2 || w.stride(0) % 16 == 0) && a.stride(0) % 16 == 0 &&
              ((uintptr_t)w.data_ptr() | (uintptr_t)a.data_ptr()) % 16 == 0);
@@ -409,7 +422,7 @@ PyObject *py_matmul(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
       n_slices = tss.size(0);
       need(n_slices > 0 && n_slices <= n_mat && (!g.bias || tensor(bias_o).dim() == 2));
       const int64_t expected = ex.none() ? -1 : as_int(ex.p);
-      const int bm = choose_block_m(M, n_slices, true, expected, a8 && w_fp4);
+      const int bm = choose_block_m(M, n_slices, true, expected, (a8 || a4) && w_fp4);
       const int row = bm == 16 ? 0 : bm == 32 ? 1 : bm == 64 ? 2 : 3;
       g.slice_sizes = (const int32_t *)tss.data_ptr(), g.slice_offs = (const int32_t *)tso.data_ptr();
       g.block_offs = (const int32_t *)tbo.data_ptr() + row * tbo.stride(0);
@@ -421,6 +434,7 @@ PyObject *py_matmul(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
     } else {
       need(n_mat == 1);
       // (a long K over few rows is split by the general path)
+      need(!a4 || M > 256 || K < 8192);
       need(!(M <= 256 && K >= 8192 && !scatter && !w_blocks && g.w_mx_layout != TAMD_SCALE_CDNA4));
     }
     // ---- output
