@@ -186,7 +186,7 @@ TAMD_DEVICE bool locate_tile(const tamd_matmul_args &a, int grid_n, int64_t grid
 // first weights, see run_tile: 333 tokens over 32 experts, 2016 -> 2112, f16, layer 83.4 us -> 81.3).
 // Blocks that absorb remainders (EXTRA > 0) leave the absorbed ones out: at 128 rows per expert they are a third of the schedule,
 // and XCD ranges of equal numbers of its entries leave the XCDs with unequal work (32 experts, 2880 x 2880, 128 bf16 rows
-// each: 98 us, 76 so).  The ranges are in expert order; up to `group` blocks of an expert run next to each other on
+// each: 98 us, 76 so).  fp8 rows take the schedule: 13 tokens over 64 experts, 2528 -> 1024, layer 34.2 us against 34.7.  The ranges are in expert order; up to `group` blocks of an expert run next to each other on
 // a column tile.  (XCD ranges of equal estimated time with the longest tiles first take 2 us to find and read an expert's
 // weights once per block: 128 experts, 200 rows each, 2880 x 2880: 462 us against 414, fp8 rows 387 against 293 in plain order.
 // Where a launch is one to three rounds of tiles they win up to 7 % (32 experts of 160 bf16 rows, 2880 x 5760: 179 against 190),
@@ -210,9 +210,10 @@ TAMD_DEVICE bool locate_tile_live(const tamd_matmul_args &a, int grid_n, int gro
   }
   // (a block that starts past the first needs more than EXTRA rows)
   auto blocks = [](int n) { return n > BLOCK_M ? (n - EXTRA + BLOCK_M - 1) / BLOCK_M : (n > 0 ? 1 : 0); };
-  int own = 0;
+  int own = blocks(rows[0]);
 #pragma unroll
-  for (int u = 0; u < kLivePerLane; ++u) own += blocks(rows[u]);
+  for (int u = 1; u < kLivePerLane; ++u)
+    if (u < n_lane) own += blocks(rows[u]);
   const int incl = wave_incl_scan(own);
   const uint32_t total = (uint32_t)__builtin_amdgcn_readlane(incl, kWave - 1) * gn;
   const uint32_t per_xcd = (total + 7) / 8, bx = blockIdx.x;
@@ -223,6 +224,7 @@ TAMD_DEVICE bool locate_tile_live(const tamd_matmul_args &a, int grid_n, int gro
   bool here = false;
 #pragma unroll
   for (int u = 0; u < kLivePerLane; ++u) {
+    if (u > 0 && u >= n_lane) continue;
     const int c = blocks(rows[u]);
     if (m >= first && m < first + c) here = true, e = lane * n_lane + u, n = rows[u], off = offs[u], before = first;
     first += c;
@@ -233,13 +235,20 @@ TAMD_DEVICE bool locate_tile_live(const tamd_matmul_args &a, int grid_n, int gro
   const int slice_rows = __builtin_amdgcn_readlane(n, src);
   const uint32_t local = idx - (uint32_t)__builtin_amdgcn_readlane(before, src) * gn;   // tile of the expert
   const uint32_t b = (uint32_t)blocks(slice_rows);
-  uint32_t g = b < (uint32_t)group ? b : (uint32_t)group;
-  if (g > 1) g = (b + (b + g - 1) / g - 1) / ((b + g - 1) / g);   // (groups of about one size)
-  const uint32_t gi = local / (g * gn), r = local - gi * g * gn;
-  const uint32_t size = b - gi * g < g ? b - gi * g : g, col = r / size;
+  uint32_t g = b < (uint32_t)group ? b : (uint32_t)group, blk, col;
+  if (g > 1) {
+    g = (b + (b + g - 1) / g - 1) / ((b + g - 1) / g);   // (groups of about one size)
+    const uint32_t gi = local / (g * gn), r = local - gi * g * gn;
+    const uint32_t size = b - gi * g < g ? b - gi * g : g;
+    col = r / size;
+    blk = gi * g + (r - col * size);
+  } else {
+    blk = local / gn;
+    col = local - blk * gn;
+  }
   t.n0 = (int)col * BLOCK_N;
   t.z = 0;
-  t.off_m = (int)(gi * g + r - col * size) * BLOCK_M;
+  t.off_m = (int)blk * BLOCK_M;
   const int left = slice_rows - t.off_m;
   t.rows = left > BLOCK_M + EXTRA ? BLOCK_M : left;
   return true;
@@ -939,10 +948,16 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
   const uint64_t as_at = (uint64_t)(uintptr_t)a.x_mx_scale | (uint64_t)a.x_mx_stride_m | (uint64_t)a.x_mx_stride_z | (uint64_t)G;
   const int as_w = (as_at & 3) == 0 ? 4 : ((as_at & 1) == 0 ? 2 : 1);
   v4i_t ras = rx;
-  uint32_t as_off = kOob;   // (set below, with the rows' offsets)
+  uint32_t as_off = kOob;
   if (x_mx) {
     const int64_t xr = a.x_rows > 0 ? a.x_rows : a.M;
     ras = make_rsrc(a.x_mx_scale + (int64_t)t.z * a.x_mx_stride_z, (uint32_t)(xr * a.x_mx_stride_m));
+    const int r = wave * 64 + lane;
+    if (wave * 64 < LDS_ROWS && r < LDS_ROWS) {
+      const int rr = t.off_m + (r < t.rows ? r : t.rows - 1);
+      const uint32_t src = a.gather_indx ? (uint32_t)a.gather_indx[t.start_m + rr] : (uint32_t)(t.start_m + rr);
+      as_off = src * (uint32_t)a.x_mx_stride_m;
+    }
   }
   // Copies per request, as the counted waits of the ring loops below see them (a wave's copies complete in the order
   // of their requests): the loops of the issue_* functions run to these numbers and the waits are written in them.
@@ -971,51 +986,32 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
   // ---- activation DMA: one instruction per 32-row fragment, lane -> (row 8w + lane/8, slot lane%8)
   const int a_rin = wave * 8 + lane / 8;
   const int a_chunk = (lane % 8) ^ ((a_rin >> 1) & 7);
-  uint32_t a_off[NFR];   // (set below)
-  // The rows' indices are the first thing requested: the first weights, which do not depend on them, are requested while they
-  // come.  (One fragment's lane holds a row of each fragment, then the row whose block scales it copies.)
-  constexpr bool AS = FP8;
-  const v4i_t rg = make_rsrc(a.gather_indx ? a.gather_indx + t.start_m + t.off_m : nullptr, a.gather_indx ? (uint32_t)__builtin_amdgcn_readfirstlane(t.rows) * 4u : 0u);
-  uint32_t row_idx[NFR + (AS ? 1 : 0)];
+  // Rows past the end of the slice are never stored: they are copied as zeros (out-of-range offset), which keeps the matrix
+  // cores' inputs quiet for the padding of a ragged tile.
+  uint32_t a_off[NFR];
+  const int row0 = t.start_m + t.off_m;
+  auto row_off = [&](int r, uint32_t src) { return r < t.rows ? src * (uint32_t)(a.x_stride_m * ESZ) + a_chunk * 16 : kOob; };
+  // 16-bit rows: their indices are the first thing requested, and the first weights, which do not depend on them, are requested while
+  // they come.  (fp8 rows: the paired copies of their weights are twice as long and the tile starts later, 158 x 640 x 1080 7.6 us
+  // against 7.3.)
+  uint32_t row_idx[NFR];
+  if constexpr (!FP8) {
+    const v4i_t rg = make_rsrc(a.gather_indx + row0, (uint32_t)__builtin_amdgcn_readfirstlane(t.rows) * 4u);
+    if (a.gather_indx) {
 #pragma unroll
-  for (int i = 0; i < NFR; ++i) row_idx[i] = request_dword(rg, (uint32_t)(i * 32 + a_rin) * 4u);
-  if constexpr (AS) row_idx[NFR] = request_dword(rg, (uint32_t)(wave * 64 + lane) * 4u);
-  // One byte per line of what only the epilogue reads -- the bias of the wave's columns, the rows' destinations and factors, the
-  // scales -- so that it finds them in the caches (a tile of few stages spent 1 us of its 10 waiting for them).  The
-  // byte lands in a register that nothing else may take before the K loop has waited for it.
-  uint32_t warm = 0;
-  {
-    const uint8_t *p = (const uint8_t *)a.x;
-    const int col = t.n0 + wave * 64 + lane * 16, row = (lane & 7) * 32;
-    const int64_t erow = t.start_m + t.off_m + (row < t.rows ? row : t.rows - 1);
-    const int kind = lane >> 3;
-    if (kind == 0 && a.bias && lane < 4)
-      p = (const uint8_t *)a.bias + ((int64_t)t.expert * a.bias_stride_e + (col < N ? col : N - 1)) * (a.bias_dtype == TAMD_F32 ? 4 : 2);
-    if (kind == 1 && a.scatter_indx) p = (const uint8_t *)(a.scatter_indx + erow);
-    if (kind == 2 && a.gammas) p = (const uint8_t *)(a.gammas + erow);
-    if (kind == 3 && a.betas) p = (const uint8_t *)(a.betas + erow);
-    if (lane == 32 && a.x_scale) p = (const uint8_t *)a.x_scale;
-    if (lane == 33 && a.w_scale) p = (const uint8_t *)a.w_scale;
-    if (lane == 34 && a.y_expected_scale) p = (const uint8_t *)a.y_expected_scale;
-    asm volatile("global_load_ubyte %0, %1, off" : "+v"(warm) : "v"(p) : "memory");
-  }
-  // (after `newer` further requests of the wave)
-  auto rows_known = [&](auto newer) {
-    await_dwords<decltype(newer)::value + 1>(row_idx);   // (and the byte above)
-    const int row0 = t.start_m + t.off_m;
+      for (int i = 0; i < NFR; ++i) row_idx[i] = request_dword(rg, (uint32_t)(i * 32 + a_rin) * 4u);
+    }
+  } else {
 #pragma unroll
     for (int i = 0; i < NFR; ++i) {
-      // rows past the end of the slice are never stored: they are copied as zeros (out-of-range offset), which
-      // keeps the matrix cores' inputs quiet for the padding of a ragged tile
-      const int r = i * 32 + a_rin;
-      const uint32_t src = a.gather_indx ? row_idx[i] : (uint32_t)(row0 + r);
-      a_off[i] = r < t.rows ? src * (uint32_t)(a.x_stride_m * ESZ) + a_chunk * 16 : kOob;
+      const int r = i * 32 + a_rin, rr = r < t.rows ? r : t.rows - 1;
+      a_off[i] = row_off(r, a.gather_indx ? (uint32_t)a.gather_indx[row0 + rr] : (uint32_t)(row0 + rr));
     }
-    if constexpr (AS) {
-      const int r = wave * 64 + lane;
-      const uint32_t src = a.gather_indx ? row_idx[NFR] : (uint32_t)(row0 + r);
-      if (x_mx && r < t.rows) as_off = src * (uint32_t)a.x_mx_stride_m;
-    }
+  }
+  auto rows_known = [&](auto newer) {   // (after `newer` further requests of the wave)
+    if (a.gather_indx) await_dwords<decltype(newer)::value>(row_idx);
+#pragma unroll
+    for (int i = 0; i < NFR; ++i) a_off[i] = row_off(i * 32 + a_rin, a.gather_indx ? row_idx[i] : (uint32_t)(row0 + i * 32 + a_rin));
   };
   // ---- weight DMA: instruction j copies LDS positions j*16 + lane/4, part slot lane%4
   // Codes in the block layout (TAMD_W_CDNA4_BLOCKS): a stage of this wave's strip is one 4 KB block that already has
@@ -1301,10 +1297,8 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
     if constexpr (PAIRED) {
       // Three activation stages; an even stage s moves the weights of s and s + 1 into registers and requests those of
       // s + 2 and s + 3 (one pair), the odd stage requests only activations.
-      issue_b_pair(0);
-      rows_known(std::integral_constant<int, CP_BPAIR>{});
       issue_a(0), issue_as(0);
-      issue_sc(0), issue_sc(1);
+      issue_b_pair(0), issue_sc(0), issue_sc(1);
       issue_a(1), issue_as(1);
       for (int it = 0; it < n_ka; it += 2) {
         // in flight at most: the activations of stage it + 1
@@ -1334,9 +1328,8 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
       // Stage s requests the activations of stage s + 1 and then the weights and scales of stage s + 2 (the weight
       // buffer of stage s is free as soon as its contents are in registers): in flight at the top of a stage are at
       // most the weights and scales the stage before requested (5 copies, or 8 with strided scales).
-      issue_b(0);
-      rows_known(std::integral_constant<int, CP_B>{});
-      issue_sc(0), issue_a(0), issue_as(0), issue_b(1), issue_sc(1);
+      issue_b(0), issue_sc(0);
+      issue_a(0), issue_as(0), issue_b(1), issue_sc(1);
       for (int it = 0; it < n_ka; ++it) {
         if (cdna4) wait_vmcnt<CP_B + 1>(); else wait_vmcnt<CP_B + NSC>();
         __syncthreads();
@@ -1352,10 +1345,15 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
     }
   } else {
   // (the scales of the whole tile are first read in stage 0: requested behind that stage's own copies, before any later one)
-  issue_b(0);
-  rows_known(std::integral_constant<int, CP_B>{});
-  issue_a(0);
-  if constexpr (SC_LDS) stage_scales();
+  if constexpr (FP8) {
+    if constexpr (SC_LDS) stage_scales();
+    issue_a(0), issue_b(0);
+  } else {
+    issue_b(0);
+    rows_known(std::integral_constant<int, CP_B>{});
+    issue_a(0);
+    if constexpr (SC_LDS) stage_scales();
+  }
   if constexpr (FP8) {
     issue_as(0);
     for (int it = 0; it < n_ka; ++it) {  // activation and weight stages coincide (128 K each)
@@ -1419,7 +1417,6 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
   }
   }
   wait_dma();
-  asm volatile("" ::"v"(warm));
 
   if constexpr (KS > 1) {
     // The groups' partial sums meet in LDS (the pipelines are dead: after the barrier every copy has landed and every
@@ -1549,7 +1546,7 @@ int launch_x16_act(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
   const int64_t fit = (int64_t)(2.5 * 1024 * 1024) / ((int64_t)BM * a.K * (is_fp8(XDT) ? 1 : 2));
   group_m = group_m > fit ? fit : group_m;
   group_m = group_m < 1 ? 1 : (group_m > 16 ? 16 : group_m);
-  if (counts_live_blocks(a)) group_m = -group_m;
+  if (!is_fp8(XDT) && counts_live_blocks(a)) group_m = -group_m;   // (fp8 rows: see locate_tile_live)
   if constexpr (!is_fp8(XDT) && BM <= 32) {
     // Fewer tiles than CUs: K groups, so that every SIMD of the CUs that do get a tile holds two to four waves
     // (at least two 128-K pairs per group; the groups' pipelines and the tile's scales have to fit one CU's LDS)
