@@ -1,0 +1,80 @@
+"""GPU: ragged products of few tiles, whose row blocks are smaller than the slices' sizes ask for (or, for fp8 rows, the streaming
+kernel's): around the lines of the rule, against float32 products of the same values; special block scales of fp8 rows, which give
+the same on both kernels that take them."""
+import pytest
+import torch
+
+from triton_amd.matmul import Epilogue, FnSpecs, PrecisionConfig, matmul
+from triton_amd.matmul_details.opt_flags import scoped_opt_flags_constraints
+from triton_amd.numerics_details.mxfp import downcast_to_mxfp, upcast_from_mxfp
+from triton_amd.tensor import make_ragged_tensor_metadata
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("rows,E,N", [(150, 8, 272), (40, 8, 1552), (20, 3, 304), (9, 12, 256), (2, 16, 1552), (1, 1, 16)])
+@pytest.mark.parametrize("kind", ["bf16", "f16", "fp8", "mxfp8", "mxfp4", "bf16 w"])
+@pytest.mark.parametrize("K", [512, 640, 4096, 4128])
+def test_few_tiles(rows, E, N, kind, K, device):
+    torch.manual_seed(rows)
+    sizes = torch.randint(max(0, rows - 3), rows + 4, (E,), dtype=torch.int32)
+    M = max(1, int(sizes.sum()))
+    sizes[0] += M - int(sizes.sum())
+    x, w = torch.randn(M, K, device=device), torch.randn(E, K, N, device=device) * 0.1
+    pc = {"out_dtype": torch.bfloat16}
+    if kind == "bf16 w":
+        w = w.bfloat16().transpose(1, 2).contiguous().transpose(1, 2)
+        wf = w.float()
+    else:
+        w, ws = downcast_to_mxfp(w, torch.uint8, axis=1)
+        wf = upcast_from_mxfp(w, ws, torch.float32, axis=1)
+        pc.update(b_mx_scale=ws, b_microblock_size=32)
+    if kind[:2] == "mx":
+        a, s = downcast_to_mxfp(x, torch.uint8 if kind == "mxfp4" else torch.float8_e4m3fn, axis=-1)
+        x = upcast_from_mxfp(a, s, torch.float32, axis=-1)
+        pc.update(a_mx_scale=s, a_microblock_size=32)
+    else:
+        a = x.to({"bf16": torch.bfloat16, "f16": torch.float16, "fp8": torch.float8_e4m3fn, "bf16 w": torch.bfloat16}[kind])
+        x = a.float()
+    md = make_ragged_tensor_metadata(sizes.to(device), M)
+    y = matmul(a, w, None, md, precision_config=PrecisionConfig(**pc)).float()
+    for e, (part, got) in enumerate(zip(x.split(sizes.tolist()), y.split(sizes.tolist()))):
+        ref = part @ wf[e]
+        # a 16-bit result (2^-8) of K float32 additions
+        assert bool(((got - ref).abs() <= 2.0 ** -8 * ref.abs() + K * 2.0 ** -23 * (part.abs() @ wf[e].abs()) + 1e-6).all()), e
+
+
+@pytest.mark.parametrize("byte", [0, 1, 238, 255])
+def test_special_block_scales(byte, device):
+    """A row's scale bytes at the ends of what bf16 holds of the values: the streaming kernel and the tiled one agree (NaN for 255)."""
+    torch.manual_seed(0)
+    K, N = 640, 256
+    a, s = downcast_to_mxfp(torch.randn(4, K, device=device), torch.float8_e4m3fn, axis=-1)
+    s[1, 3] = byte
+    s[2] = byte
+    w, ws = downcast_to_mxfp(torch.randn(1, K, N, device=device), torch.uint8, axis=1)
+    ws = ws.clone() if byte != 238 else (ws.int() - 40).clamp(min=1).to(torch.uint8)   # (keeps the products finite)
+    md = make_ragged_tensor_metadata(torch.tensor([4], dtype=torch.int32, device=device), 4)
+    out = []
+    for block_m in (16, 32):
+        with scoped_opt_flags_constraints({"block_m": block_m}):
+            pc = PrecisionConfig(a_mx_scale=s, a_microblock_size=32, b_mx_scale=ws.transpose(1, 2).contiguous().transpose(1, 2),
+                                 b_microblock_size=32, out_dtype=torch.float32)
+            out.append(matmul(a, w, None, md, precision_config=pc))
+    assert torch.equal(out[0].isnan(), out[1].isnan()) and bool(out[0][2].isnan().all()) == (byte == 255)
+    torch.testing.assert_close(out[0], out[1], rtol=1e-3, atol=1e-3, equal_nan=True)
+
+
+def test_microscaled_output_keeps_its_kernel(device):
+    torch.manual_seed(1)
+    K, N, M = 640, 256, 12
+    a, s = downcast_to_mxfp(torch.randn(M, K, device=device), torch.float8_e4m3fn, axis=-1)
+    w, ws = downcast_to_mxfp(torch.randn(2, K, N, device=device) * 0.1, torch.uint8, axis=1)
+    md = make_ragged_tensor_metadata(torch.tensor([5, 7], dtype=torch.int32, device=device), M)
+    ys = torch.zeros((M, N // 32), dtype=torch.uint8, device=device)
+    pc = PrecisionConfig(a_mx_scale=s, a_microblock_size=32, b_mx_scale=ws, b_microblock_size=32, c_mx_scale=ys, c_microblock_size=32)
+    y = matmul(a, w, None, md, precision_config=pc, epilogue=Epilogue(FnSpecs("QUANTIZE_MXFP8", None, (), ()), (), (), 6.0))
+    pc = PrecisionConfig(a_mx_scale=s, a_microblock_size=32, b_mx_scale=ws, b_microblock_size=32, out_dtype=torch.float32)
+    with scoped_opt_flags_constraints({"block_m": 32}):
+        want = downcast_to_mxfp(matmul(a, w, None, md, precision_config=pc), torch.float8_e4m3fn, axis=-1)
+    assert torch.equal(y.view(torch.uint8), want[0].view(torch.uint8)) and torch.equal(ys, want[1])

@@ -453,7 +453,9 @@ __global__ __launch_bounds__((NCW + NC + 2) * 64, 1) void mm_stream16_kernel(tam
         for (int j = 0; j < SS; ++j) {
           const int kg = kb + 4 * j + g;
           const bool live = kg < G && cb.rows > 0;
-          const float mult = (live && xs) ? bits_to_f32((uint32_t)xs[kg] << 23) : 1.0f;  // 2^(e - 127); 0xFF gives +inf
+          // 2^(e - 127) as the scaled MFMA of the tiled kernels reads it: 0 is 2^-127, 0xFF NaN
+          const uint32_t e = (live && xs) ? (uint32_t)xs[kg] : 127u;
+          const float mult = bits_to_f32(e == 0u ? 0x00400000u : (e == 255u ? 0x7FC00000u : e << 23));
 #pragma unroll
           for (int u = 0; u < 4; ++u) {
             uint2 v = make_uint2(0, 0);
