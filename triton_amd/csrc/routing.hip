@@ -546,7 +546,7 @@ __global__ __launch_bounds__(1024) void order_scan_kernel(const void *__restrict
                                                           int32_t *__restrict__ col_sorted, int32_t *__restrict__ row_sorted,
                                                           int32_t *__restrict__ gather, int32_t *__restrict__ offs,
                                                           int64_t offs_pitch, int32_t *__restrict__ sched,
-                                                          int64_t sched_pitch, int max_blocks, Gates gates) {
+                                                          int64_t sched_pitch, int max_blocks, Gates gates, int sub) {
   extern __shared__ int32_t sm[];
   int32_t *hist = sm;                          // [CH][E]  counts of this block's chunks, then their exclusive prefix
   int32_t *tot = hist + (int64_t)CH * E;       // [E]      entries per expert
@@ -556,7 +556,8 @@ __global__ __launch_bounds__(1024) void order_scan_kernel(const void *__restrict
   int32_t *tab = pbel + (int64_t)P * E;        // [6][E + 1]
   const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
   const int blk = blockIdx.x;
-  const bool orders = blk < nb;
+  const int nbo = (nb + sub - 1) / sub;        // blocks of CH chunks, `sub` rows of the table each
+  const bool orders = blk < nbo;
   // this wave's chunk of the index array: requested first, used after the table has been reduced
   const int i = (blk * CH + wave) * 64 + lane;
   const bool has = orders && wave < CH && i < n;
@@ -575,7 +576,7 @@ __global__ __launch_bounds__(1024) void order_scan_kernel(const void *__restrict
       const int per = (nb + P - 1) / P;
       const int b_hi = (part + 1) * per < nb ? (part + 1) * per : nb;
       int all, below;
-      sum_block_range(block_tot, E, e, part * per, b_hi, blk, all, below);
+      sum_block_range(block_tot, E, e, part * per, b_hi, blk * sub, all, below);
       psum[part * E + e] = all;
       pbel[part * E + e] = below;
     }
@@ -609,7 +610,7 @@ __global__ __launch_bounds__(1024) void order_scan_kernel(const void *__restrict
       }
     }
   }
-  ragged_scan_rows(tot, E, tab, blk == nb ? offs : nullptr, offs_pitch);
+  ragged_scan_rows(tot, E, tab, blk == nbo ? offs : nullptr, offs_pitch);
   __syncthreads();
   if (orders) {
     // 4. placement
@@ -630,16 +631,16 @@ __global__ __launch_bounds__(1024) void order_scan_kernel(const void *__restrict
   } else {
     // 4'. this workgroup's share of the block schedule
     const int64_t total = 5 * (int64_t)max_blocks;
-    const int64_t shares = (int64_t)gridDim.x - nb;
+    const int64_t shares = (int64_t)gridDim.x - nbo;
     const int64_t per = (total + shares - 1) / shares;
-    const int64_t first = per * (blk - nb);
+    const int64_t first = per * (blk - nbo);
     if (first < total) ragged_fill_schedule(tab, E, sched, sched_pitch, max_blocks, first, per < total - first ? per : total - first);
   }
 }
 
 // Second launch of the two: the grid, the LDS size and the limits of order_scan_kernel.
-inline bool order_scan_applicable(int64_t n, int E, int CH, int64_t nb) {
-  if (E > 1024 || nb < 1 || nb > kMaxTableBlocks || n > 0x7FFFFFFF - 64 * 1024) return false;
+inline bool order_scan_applicable(int64_t n, int E, int CH, int64_t nb, int64_t max_nb = kMaxTableBlocks) {
+  if (E > 1024 || nb < 1 || nb > max_nb || n > 0x7FFFFFFF - 64 * 1024) return false;
   int P = 1024 / E;
   P = P > 16 ? 16 : P;
   const int64_t ints = (int64_t)CH * E + 2 * (int64_t)E + 2 * (int64_t)P * E + 6 * ((int64_t)E + 1);
@@ -649,7 +650,7 @@ inline bool order_scan_applicable(int64_t n, int E, int CH, int64_t nb) {
 inline int launch_order_scan(const void *indx, int is16, int64_t n, int E, int CH, int nbits, int k, const int32_t *block_tot,
                              int64_t nb, int32_t *col_sum, int32_t *col_sorted, int32_t *row_sorted, int32_t *gather,
                              int32_t *offs, int64_t offs_pitch, int32_t *sched, int64_t sched_pitch, int max_blocks,
-                             Gates gates, hipStream_t st) {
+                             Gates gates, hipStream_t st, int sub = 1) {
   int P = 1024 / E;
   P = P > 16 ? 16 : P;
   P = P > nb ? (int)nb : P;
@@ -657,39 +658,41 @@ inline int launch_order_scan(const void *indx, int is16, int64_t n, int E, int C
   int64_t shares = (5 * (int64_t)max_blocks + 4095) / 4096;  // about four schedule entries per thread
   shares = shares < 1 ? 1 : (shares > 64 ? 64 : shares);
   if (int rc = raise_lds_limit_once((const void *)order_scan_kernel)) return rc;
-  order_scan_kernel<<<dim3((unsigned)(nb + shares)), 1024, (size_t)ints * 4, st>>>(
+  order_scan_kernel<<<dim3((unsigned)((nb + sub - 1) / sub + shares)), 1024, (size_t)ints * 4, st>>>(
       indx, is16, (int)n, E, CH, nbits, k, block_tot, (int)nb, P, col_sum, col_sorted, row_sorted, gather, offs, offs_pitch,
-      sched, sched_pitch, max_blocks, gates);
+      sched, sched_pitch, max_blocks, gates, sub);
   return launch_status();
 }
 
-// First launch of the two, from the logits: the experts of 1024 / L rows per workgroup (their picked columns also go to
-// LDS) and the histogram of that block of (1024 / L) * k / 64 whole chunks.
-template <int DT, int L, int EPL>
-__global__ __launch_bounds__(1024) void topk_hist_kernel(const void *__restrict__ x, int64_t x_stride, int n_rows, int E,
+// First launch of the two, from the logits: the experts of TH / L rows per workgroup (their picked columns also go to
+// LDS) and the histogram of that block of CH = (TH / L) * k / 64 whole chunks.  A row is a chain of some 400 instructions, so
+// the workgroups are as small as whole chunks allow (4096 rows of 128, top-4, both launches: 13.3 us with 1024
+// threads, 12.6 with 512; 1024 rows 12.4 and, with 256, 11.4).
+template <int DT, int L, int EPL, int TH>
+__global__ __launch_bounds__(TH) void topk_hist_kernel(const void *__restrict__ x, int64_t x_stride, int n_rows, int E,
                                                          int k, void *__restrict__ y_vals, int16_t *__restrict__ y_indx,
                                                          uint32_t *__restrict__ bits, int64_t bits_stride_row,
                                                          int64_t bits_stride_word, int nbits, int CH,
                                                          int32_t *__restrict__ block_tot) {
   extern __shared__ int32_t sm[];
-  constexpr int ROWS = 1024 / L;
+  constexpr int ROWS = TH / L;
   int32_t *lidx = sm;            // [CH * 64] picked columns of this block's rows
   int32_t *hist = sm + CH * 64;  // [CH][E]
   const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
   const int64_t row0 = (int64_t)blockIdx.x * ROWS;
-  for (int j = tid; j < CH * E; j += 1024) hist[j] = 0;  // (the barrier below covers them)
+  for (int j = tid; j < CH * E; j += TH) hist[j] = 0;  // (the barrier below covers them)
   topk_row<DT, L, EPL>(x, x_stride, n_rows, E, k, 1, 0, y_vals, y_indx, k, bits, bits_stride_row, bits_stride_word,
                        row0 + tid / L, lidx - row0 * k);
   __syncthreads();
-  if (wave < CH) {
-    const int j = wave * 64 + lane;  // entry of the block; its row exists or not
+  for (int c = wave; c < CH; c += TH / kWave) {
+    const int j = c * 64 + lane;  // entry of the block; its row exists or not
     const bool valid = row0 + j / k < n_rows;
     const int e = valid ? lidx[j] : -1;
     const uint64_t same = same_id_mask(e, valid, nbits);
-    if (valid && (same & lanemask_lt()) == 0) hist[wave * E + e] = __popcll(same);
+    if (valid && (same & lanemask_lt()) == 0) hist[c * E + e] = __popcll(same);
   }
   __syncthreads();
-  for (int e = tid; e < E; e += 1024) {
+  for (int e = tid; e < E; e += TH) {
     int run = 0;
     for (int c = 0; c < CH; ++c) run += hist[c * E + e];
     block_tot[(int64_t)blockIdx.x * E + e] = run;
@@ -698,11 +701,16 @@ __global__ __launch_bounds__(1024) void topk_hist_kernel(const void *__restrict_
 
 template <int DT>
 int launch_topk_hist(const void *x, int64_t xs, int n_rows, int E, int k, void *yv, int16_t *yi, uint32_t *bits, int64_t bsr,
-                     int64_t bsw, int nbits, int L, int CH, int32_t *block_tot, hipStream_t st) {
+                     int64_t bsw, int nbits, int L, int TH, int32_t *block_tot, hipStream_t st) {
+  const int CH = TH / L * k / 64;
   const size_t lds = ((size_t)CH * 64 + (size_t)CH * E) * 4;
-  const unsigned grid = (unsigned)((n_rows + 1024 / L - 1) / (1024 / L));
-#define TAMD_TH(LL, EE) \
-  topk_hist_kernel<DT, LL, EE><<<grid, 1024, lds, st>>>(x, xs, n_rows, E, k, yv, yi, bits, bsr, bsw, nbits, CH, block_tot)
+  const unsigned grid = (unsigned)((n_rows + TH / L - 1) / (TH / L));
+#define TAMD_TH(LL, EE)                                                                                                 \
+  do {                                                                                                                  \
+    auto kern = TH == 256 ? topk_hist_kernel<DT, LL, EE, 256>                                                           \
+                          : (TH == 512 ? topk_hist_kernel<DT, LL, EE, 512> : topk_hist_kernel<DT, LL, EE, 1024>);       \
+    kern<<<grid, TH, lds, st>>>(x, xs, n_rows, E, k, yv, yi, bits, bsr, bsw, nbits, CH, block_tot);                     \
+  } while (0)
   if (L == 8) TAMD_TH(8, 8);
   else if (L == 16) TAMD_TH(16, 8);
   else if (L == 32) TAMD_TH(32, 8);
@@ -1092,7 +1100,27 @@ extern "C" int tamd_routing_gates(const void *logits, int dtype, int64_t stride,
     int64_t P = 1024 / n_cols;
     P = P < 1 ? 1 : (P > NC ? NC : P);
     const int64_t ints = 2 * ((n + 3) / 4 * 4) + NC * n_cols + (int64_t)n_cols + P * n_cols + 6 * (int64_t)(n_cols + 1);
-    if (n_rows <= 2 * (1024 / L) && NC <= 64 && ints * 4 <= 156 * 1024) {
+    // two launches: top-k with the histogram of each workgroup's rows, then ordering and tables.  The rows of a workgroup
+    // (TH / L) must make whole chunks of 64 entries; the second launch orders 1024 / TH of the first one's blocks per workgroup.  It
+    // reduces the table with 16 loads per thread in flight, so TH grows where the table has more rows than one such batch
+    // (4096 rows of 128: 12.6 us with 512 threads, 13.8 with 256).  Beyond kMaxTableBlocks rows three small launches behind the
+    // top-k are faster up to 131072 entries (8192 rows of 256, top-8: 21.7 against 30), slower above (32768 of 64, top-6: 32 against 22).
+    int TH = 0;
+    const int CHO = 16 * k / L;
+    const int64_t batch = 16 * (1024 / n_cols > 16 ? 16 : (1024 / n_cols < 1 ? 1 : 1024 / n_cols));
+    if ((16 * k) % L == 0 && CHO >= 1 && CHO <= 16 && workspace)
+      for (int th = 256; th <= 1024 && !TH; th *= 2) {
+        const int64_t nb = ((int64_t)n_rows + th / L - 1) / (th / L);
+        const int64_t most = batch > kMaxTableBlocks && n <= 1024 * kMaxTableBlocks ? kMaxTableBlocks : batch;
+        if ((th / L * k) % 64 == 0 && (nb <= batch || th == 1024) &&
+            order_scan_applicable(n, n_cols, CHO, nb, th == 1024 && most < kMaxTableBlocks ? kMaxTableBlocks : most) &&
+            nb * n_cols <= tamd_bitmatrix_metadata_workspace(n, n_cols))
+          TH = th;
+      }
+    // one launch while a pass and a half of its threads hold the rows and the entries are few (128 rows of 128, top-8: 17.6 us in
+    // one launch, 11.5 in two; 256 rows of 16, top-8: 16.9 and 10.3; 96 rows of 128, top-4: 9.7 and 10.2)
+    const bool one = n_rows <= (TH ? 3 : 4) * (512 / L) && (!TH || NC <= 16);
+    if (one && NC <= 64 && ints * 4 <= 156 * 1024) {
       int nbits = 0;
       while ((1 << nbits) < n_cols) ++nbits;
       hipStream_t st = (hipStream_t)stream;
@@ -1105,28 +1133,24 @@ extern "C" int tamd_routing_gates(const void *logits, int dtype, int64_t stride,
       TAMD_RFD(TAMD_F16);
 #undef TAMD_RFD
     }
-    // two launches: top-k with the histogram of each workgroup's rows, then ordering and tables.  The rows of a
-    // workgroup (1024 / L) must make whole chunks of 64 entries.
-    const int CH = 16 * k / L;
-    const int64_t nb = ((int64_t)n_rows + 1024 / L - 1) / (1024 / L);
-    if ((16 * k) % L == 0 && CH >= 1 && CH <= 16 && workspace && order_scan_applicable(n, n_cols, CH, nb) &&
-        nb * n_cols <= tamd_bitmatrix_metadata_workspace(n, n_cols)) {
+    if (TH) {
+      const int64_t nb = ((int64_t)n_rows + TH / L - 1) / (TH / L);
       int nbits = 0;
       while ((1 << nbits) < n_cols) ++nbits;
       hipStream_t st = (hipStream_t)stream;
       int rc;
       if (dtype == TAMD_F32)
         rc = launch_topk_hist<TAMD_F32>(logits, stride, n_rows, n_cols, k, y_vals, y_indx, bits, bits_stride_row,
-                                        bits_stride_word, nbits, L, CH, workspace, st);
+                                        bits_stride_word, nbits, L, TH, workspace, st);
       else if (dtype == TAMD_BF16)
         rc = launch_topk_hist<TAMD_BF16>(logits, stride, n_rows, n_cols, k, y_vals, y_indx, bits, bits_stride_row,
-                                         bits_stride_word, nbits, L, CH, workspace, st);
+                                         bits_stride_word, nbits, L, TH, workspace, st);
       else
         rc = launch_topk_hist<TAMD_F16>(logits, stride, n_rows, n_cols, k, y_vals, y_indx, bits, bits_stride_row,
-                                        bits_stride_word, nbits, L, CH, workspace, st);
+                                        bits_stride_word, nbits, L, TH, workspace, st);
       if (rc != 0) return rc;
-      return launch_order_scan(y_indx, 1, n, n_cols, CH, nbits, k, workspace, nb, col_sum, col_sorted_indx, row_sorted_indx,
-                               gather_indx, offs, offs_pitch, schedule, sched_pitch, max_n_blocks, gates, st);
+      return launch_order_scan(y_indx, 1, n, n_cols, CHO, nbits, k, workspace, nb, col_sum, col_sorted_indx, row_sorted_indx,
+                               gather_indx, offs, offs_pitch, schedule, sched_pitch, max_n_blocks, gates, st, 1024 / TH);
     }
   }
   const int rc = tamd_topk_forward(logits, dtype, stride, n_rows, n_cols, k, 1, 0, y_vals, y_indx, k, bits, bits_stride_row,
