@@ -113,13 +113,17 @@ __global__ __launch_bounds__((NCW + NC + 2) * 64, 1) void mm_stream16_kernel(tam
   const uint32_t col_bytes = (uint32_t)(K / 2);
 
   // ---- this workgroup's range of units
-  const int n_blocks = a.block_schedule ? a.block_offs[a.n_experts] : dense_blocks;
-  const int64_t total = (int64_t)n_blocks * n_cg;
-  const int64_t first = (int64_t)blockIdx.x * total / gridDim.x;
-  const int64_t last = (int64_t)(blockIdx.x + 1) * total / gridDim.x;
-  if (first >= last) return;
-  const int total_stages = (int)(last - first);
-  const int blk0 = (int)(first / n_cg), cg0 = (int)(first - (int64_t)blk0 * n_cg);
+  // (The first copy waits for what is read here, so the schedule's first 64 entries come with its length, one per lane, and
+  // the arithmetic is 32 bits wide -- the launcher keeps the units below 2^31.  Layers of one
+  // token over 128 experts, 2880 -> 5760 -> 2880: 30.4 -> 30.0 us, of 35 tokens over 64, 1344 -> 1088 -> 1344: 29.2 -> 28.6.)
+  int sched_lane = -1;
+  if (a.block_schedule && lane < a.grid_m) sched_lane = a.block_schedule[lane];
+  const uint32_t n_blocks = (uint32_t)(a.block_schedule ? a.block_offs[a.n_experts] : dense_blocks);
+  const uint32_t units = n_blocks * (uint32_t)n_cg, wgs = gridDim.x, each = units / wgs, more = units - each * wgs;
+  const uint32_t first = blockIdx.x * each + (blockIdx.x < more ? blockIdx.x : more);
+  const int total_stages = (int)(each + (blockIdx.x < more ? 1u : 0u));
+  if (total_stages == 0) return;
+  const int blk0 = (int)(first / (uint32_t)n_cg), cg0 = (int)(first - (uint32_t)blk0 * (uint32_t)n_cg);
 
   struct Block {  // a row block of at most 16 rows
     int expert, z, row0, rows;
@@ -128,7 +132,7 @@ __global__ __launch_bounds__((NCW + NC + 2) * 64, 1) void mm_stream16_kernel(tam
     b.z = 0;
     int slice_rows, off_m;
     if (a.block_schedule) {
-      const int sched = a.block_schedule[blk];
+      const int sched = blk < kWave ? __builtin_amdgcn_readlane(sched_lane, blk) : a.block_schedule[blk];
       if (sched == -1) {  // cannot happen below block_offs[n_experts]; an empty block keeps the ring in step
         b.expert = 0, b.row0 = 0, b.rows = 0;
         return;
@@ -581,6 +585,7 @@ int launch_stream16_ss(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
   const int n_cg = (a.N + 15) / 16;
   const int64_t upper = (int64_t)grid_m * n_cg;
   if (upper <= 0) return 0;
+  if (upper > 0x7FFFFFFF) return TAMD_E_UNSUPPORTED;
   int cus = 0;
   if (int rc = cu_count(cus)) return rc;
   const int wgs = (int)(upper < cus ? upper : cus);
