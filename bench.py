@@ -498,7 +498,7 @@ def run_fc2(args, cfg, name):
     else:
         roof = dict(bound="mfma", achieved=round(tflops_kernel, 1), peak=PEAK_FP8_TFLOPS, unit="TFLOP/s",
                     frac=round(tflops_kernel / PEAK_FP8_TFLOPS, 4), traffic=traffic, traffic_source=traffic_source,
-                    kernel="mm_x8_mxfp4_kernel", kernel_ms=round(kernel_ms, 4), algorithmic_bytes=mm_bytes,
+                    kernel="mm_mx_kernel", kernel_ms=round(kernel_ms, 4), algorithmic_bytes=mm_bytes,
                     algorithmic_flops=flops, frac_of_mxfp4_peak=round(tflops_kernel / PEAK_MXFP4_TFLOPS, 4),
                     hbm_gbs=round(gbs_kernel, 1))
     combine_bytes = rows * N * 2 + T * N * 2
@@ -620,7 +620,7 @@ def run_fc1(args, cfg, name):
         roof = dict(bound="mfma", achieved=round(tflops_kernel, 1), peak=peak_mfma, unit="TFLOP/s",
                     frac=round(tflops_kernel / peak_mfma, 4), traffic=traffic, traffic_source=traffic_source)
     # row blocks of 16 (few rows per expert) run the weight-streaming kernel, everything else the tiled one
-    roof["kernel"] = "mm_stream16_kernel" if rows <= 16 * E else ("mm_x8_mxfp4_kernel" if mx8 else "mm_x16_mxfp4_kernel")
+    roof["kernel"] = "mm_stream16_kernel" if rows <= 16 * E else ("mm_mx_kernel" if mx8 else "mm_x16_mxfp4_kernel")
     if mx4:
         roof["kernel"] = "widen_e2m1_rows_kernel + " + roof["kernel"]
         roof["frac_of_fp8_mfma_peak"] = round(tflops_kernel / PEAK_FP8_TFLOPS, 4)
@@ -816,7 +816,7 @@ def run_mlp(args, cfg, name):
                     scale_layout=args.scale_layout, value_layout=args.value_layout)
     out["stages"] = last["stages"]
     out["roofline"] = {"bound": "hbm", "achieved": round(gbs, 1), "peak": PEAK_HBM_GBS, "unit": "GB/s",
-                       "frac": round(gbs / PEAK_HBM_GBS, 4), "traffic": None, "kernel": "mm_x8_mxfp4_kernel (FC1 + FC2)",
+                       "frac": round(gbs / PEAK_HBM_GBS, 4), "traffic": None, "kernel": "mm_mx_kernel (FC1 + FC2)",
                        "kernel_ms": round(last["mm_ms"], 4), "algorithmic_flops": last["mm_flops"],
                        "algorithmic_bytes": last["mm_bytes"], "tflops": round(tflops, 1),
                        "frac_of_fp8_mfma_peak": round(tflops / PEAK_FP8_TFLOPS, 4)}

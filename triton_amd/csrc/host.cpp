@@ -226,7 +226,8 @@ PyObject *py_matmul(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
     g.x_dtype = a4 ? TAMD_MXFP4 : type_code(a_type);
     need(g.x_dtype != TAMD_F32);
     const bool a8 = is_fp8_code(g.x_dtype);
-    if (a4)  // what the kernel for them reads as it is (_packed_rows_direct; anything else is widened by the general path)
+    if (a4)  // what the kernel for them reads as it is (_packed_rows_direct; rows of less than a stage, and what is widened, are
+             // the general path's)
       need(K >= 256 && a.stride(0) % 16 == 0 && (uintptr_t)a.data_ptr() % 16 == 0);
 
     // ---- precision options

@@ -1,4 +1,4 @@
-// Grouped (ragged-M) / dense matmul for gfx950: 16-bit or fp8 activations x MXFP4 weights.
+// Grouped (ragged-M) / dense matmul for gfx950: 16-bit activations x MXFP4 weights, and what every tiled kernel shares.
 //
 //   y[dst(r), :] = act(((x[src(r), :] . deq(w[e])) * sx * sw + bias[e, :] * beta[r]) * alpha) * gamma[r]
 //
@@ -14,14 +14,11 @@
 //   bf16 / f16 activations: the fp4 codes are expanded in registers with v_cvt_scalef32_pk_*_fp4
 //     (scale applied by the instruction) and feed v_mfma_f32_32x32x16, which sustains twice the rate
 //     of 16x16x32 on this part (measured 2.45 vs 1.25 PFLOP/s for bf16).
-//   fp8 activations: v_mfma_scale_f32_32x32x64_f8f6f4 consumes the fp8 bytes, the fp4 codes and the
-//     e8m0 scale bytes directly (no conversion instructions at all).
+//   (fp8 and packed activations: moe_matmul_mx.h.)
 //
 // K order inside a 128-K weight stage: lane half h = lane/32 holds K [64q + 32h, 64q + 32h + 32) of
-// its column for q = 0, 1 (two 128-bit LDS reads).  16-bit path: MFMA step s = 4q + u consumes
-// elements [8u, 8u+8) of load q in both halves, for A and B alike.  fp8 path: MFMA q consumes load q
-// whole; its A operand is, for lane half h, the 16 activations K 64q + 16h.. followed by the 16 at
-// K 64q + 32 + 16h.. (the operand layout of the instruction, established by one-hot probing).
+// its column for q = 0, 1 (two 128-bit LDS reads); MFMA step s = 4q + u consumes elements [8u, 8u+8) of load q in
+// both halves, for A and B alike.
 #pragma once
 #include <type_traits>
 
@@ -46,9 +43,7 @@ constexpr int NF = 2;              // 32-column fragments per wave
 constexpr int BLOCK_N = 4 * 32 * NF;
 
 template <int XDT>
-struct Mma {  // fp8 activations: operands are raw dwords, no expansion
-  typedef i32x8_t frag_t;
-};
+struct Mma;
 template <>
 struct Mma<TAMD_BF16> {
   typedef bf16x8_t frag_t;
@@ -186,7 +181,7 @@ TAMD_DEVICE bool locate_tile(const tamd_matmul_args &a, int grid_n, int64_t grid
 // first weights, see run_tile: 333 tokens over 32 experts, 2016 -> 2112, f16, layer 83.4 us -> 81.3).
 // Blocks that absorb remainders (EXTRA > 0) leave the absorbed ones out: at 128 rows per expert they are a third of the schedule,
 // and XCD ranges of equal numbers of its entries leave the XCDs with unequal work (32 experts, 2880 x 2880, 128 bf16 rows
-// each: 98 us, 76 so).  fp8 rows take the schedule: 13 tokens over 64 experts, 2528 -> 1024, layer 34.2 us against 34.7.  The ranges are in expert order; up to `group` blocks of an expert run next to each other on
+// each: 98 us, 76 so).  The ranges are in expert order; up to `group` blocks of an expert run next to each other on
 // a column tile.  (XCD ranges of equal estimated time with the longest tiles first take 2 us to find and read an expert's
 // weights once per block: 128 experts, 200 rows each, 2880 x 2880: 462 us against 414, fp8 rows 387 against 293 in plain order.
 // Where a launch is one to three rounds of tiles they win up to 7 % (32 experts of 160 bf16 rows, 2880 x 5760: 179 against 190),
@@ -268,19 +263,12 @@ TAMD_DEVICE void dma16(v4i_t rsrc, uint32_t lds_addr, uint32_t voff, uint32_t so
                  "s"(__builtin_amdgcn_readfirstlane(soff))
                : "memory", "m0");
 }
-// 1-, 2- and 4-byte global -> LDS copies: lane L's value lands (zero-extended) in the dword at
+// 2- and 4-byte global -> LDS copies: lane L's value lands (zero-extended) in the dword at
 // lds_addr + 4*L; out-of-range offsets deliver zero.  The five wait states before the load cover an
 // SGPR operand that a v_readfirstlane wrote just before the asm block (the compiler's hazard
 // recognizer does not look inside inline asm) as well as the write of M0.
 TAMD_DEVICE void dma2(v4i_t rsrc, uint32_t lds_addr, uint32_t voff, uint32_t soff) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_ushort %1, %2, %3 offen lds"
-               :
-               : "s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(voff), "s"(rsrc),
-                 "s"(__builtin_amdgcn_readfirstlane(soff))
-               : "memory", "m0");
-}
-TAMD_DEVICE void dma1(v4i_t rsrc, uint32_t lds_addr, uint32_t voff, uint32_t soff) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_ubyte %1, %2, %3 offen lds"
                :
                : "s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(voff), "s"(rsrc),
                  "s"(__builtin_amdgcn_readfirstlane(soff))
@@ -336,35 +324,27 @@ TAMD_DEVICE v4i_t make_rsrc(const void *base, uint32_t num_records) {
                __builtin_amdgcn_readfirstlane((int)((uint32_t)(p >> 32) & 0xFFFFu)), (int)num_records, 0x00020000};
 }
 
-constexpr int A_ROW_BYTES = 128;       // LDS bytes per activation row per stage (64 K of 16-bit, 128 K of fp8)
+constexpr int A_ROW_BYTES = 128;       // LDS bytes per activation row per stage (64 K of 16-bit values)
 constexpr int B_BYTES = 4 * 64 * 64;   // 4 waves x 64 columns x 64 bytes (128 K of fp4)
 // LDS of the K pipeline.  The usual layout: two activation stages, one weight stage (4 KB per wave), the e8m0 scales
-// of the whole tile staged once.  "Ring mode" (fp8 path without the whole-tile scale staging, i.e. pre-shuffled
-// scales, or strided scales that do not fit): the scales of a stage travel with its weights (1 KB per wave and
-// stage), which leaves room for two weight stages and -- for row blocks of at most 64 rows -- three activation
-// stages, so that two stages' copies are in flight instead of one.  The fp8 path needs that: it spends half the
-// matrix-core time per weight byte, and with few rows per expert the stream from HBM is all there is to wait for.
+// of the whole tile staged once.
 struct PipeShape {
-  int da, db;        // activation / weight (+ scale) stages
-  int as_bytes;      // block scales of MXFP8 activations: da stages x 4 planes x rows x 4 bytes
-  int scr_bytes;     // ring-mode scale ring: db stages x 4 waves x 1 KB
+  int da, db;        // activation / weight stages
   int bytes;
 };
-// "Deep mode" (16-bit path with the scales staged in LDS, row blocks of at most 64 rows): counted waits with three or
-// four activation stages and two weight stages.  With so few rows a stage's MFMAs take less time than a copy needs
+// "Deep mode" (scales staged in LDS, row blocks of at most 64 rows): counted waits with three or four activation
+// stages and two weight stages.  With so few rows a stage's MFMAs take less time than a copy needs
 // to arrive, and the K loop of the two-stage pipeline runs at the latency of the copies.
 // K groups (KS = 2 or 4, row blocks of at most 32 rows): KS groups of four waves share a tile, each taking a
 // contiguous part of K through a pipeline of its own; their partial sums meet in LDS.  A problem with fewer tiles than
 // the part has CUs is bound by what one wave per SIMD can issue (a copy instruction holds its wave for about a
 // hundred cycles); more waves per SIMD fill those gaps.
-constexpr bool deep_mode(bool fp8, int lds_rows) { return !fp8 && lds_rows <= 64; }
-constexpr PipeShape pipe_shape(bool fp8, bool ring, int lds_rows, bool deep = false, int ks = 1) {
+constexpr bool deep_mode(int lds_rows) { return lds_rows <= 64; }
+constexpr PipeShape pipe_shape(int lds_rows, bool deep = false, int ks = 1) {
   PipeShape p{};
-  p.da = deep ? (ks == 4 ? 3 : (lds_rows <= 32 ? 4 : 3)) : (ring && lds_rows <= 64 ? 3 : 2);
-  p.db = (ring || deep) && ks != 4 ? 2 : 1;
-  p.as_bytes = fp8 ? p.da * 4 * (lds_rows < 64 ? 64 : lds_rows) * 4 : 0;
-  p.scr_bytes = ring ? p.db * 4 * 1024 : 0;
-  p.bytes = p.da * lds_rows * 128 + p.db * B_BYTES + p.as_bytes + p.scr_bytes;
+  p.da = deep ? (ks == 4 ? 3 : (lds_rows <= 32 ? 4 : 3)) : 2;
+  p.db = deep && ks != 4 ? 2 : 1;
+  p.bytes = p.da * lds_rows * 128 + p.db * B_BYTES;
   return p;
 }
 
@@ -819,32 +799,29 @@ TAMD_DEVICE late_args_t &kernel_args_late() {
 }
 
 // One output tile with NFR (compile time) active 32-row fragments.
-// LDS: [A stages (2 to 4) | B: 4 wave-private regions, one or two stages | (fp8) activation block scales | scale ring or
-// the e8m0 scales of the whole tile]; with K groups (KS > 1) one such pipeline per group, the tile's scales behind them.
+// LDS: [A stages (2 to 4) | B: 4 wave-private regions, one or two stages | the e8m0 scales of the whole tile]; with K groups (KS > 1) one such pipeline per group, the tile's scales behind them.
 //
-// Both operands reach LDS by DMA.  Activations: 64 K per stage (128 K of fp8); wave w copies rows
+// Both operands reach LDS by DMA.  Activations: 64 K per stage; wave w copies rows
 // 8w..8w+7 of every 32-row fragment (8 lanes x 16 B per row); chunk c of row r sits at slot
 // c ^ ((r>>1)&7), which makes the 32-row MFMA operand reads bank-conflict free.  Weights: every
-// second stage (every stage of fp8) each wave copies 128 K of its own 64 columns into its private region: position
+// second stage each wave copies 128 K of its own 64 columns into its private region: position
 // p' = f*32 + c holds global column 2c + f of the wave's strip (so a lane ends up with a gate/linear column pair), the
 // four 16-byte parts rotated by ((p'>>2)&3) ^ 2f.  From column-strided weights that is 64 contiguous bytes of each
 // column; weights in the block layout (TAMD_W_CDNA4_BLOCKS) hold exactly this image, 4 KB per strip and 128 K, and
 // are copied as they lie.  The wave reads the region into registers at the start of the stage and immediately
 // requests the next 128 K into it, so weights need no barrier.
-// Loops: two stages and full waits (16-bit, row blocks above 64 rows or scales not in LDS); counted waits over a
-// deeper ring (deep mode, K groups: 16-bit; ring mode, paired: fp8), see pipe_shape.
+// Loops: two stages and full waits (row blocks above 64 rows or scales not in LDS); counted waits over a
+// deeper ring (deep mode, K groups), see pipe_shape.
 template <int XDT, int NFR, int LDS_ROWS, int ACT, bool SC_LDS, int KS = 1>
 TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds_wg) {
   typedef Mma<XDT> M;
   typedef typename M::frag_t frag_t;
-  constexpr bool FP8 = is_fp8(XDT);
-  constexpr int ESZ = FP8 ? 1 : 2;            // bytes per activation element
+  constexpr int ESZ = 2;                      // bytes per activation element
   constexpr int KA = A_ROW_BYTES / ESZ;       // K per activation stage
   constexpr int A_STAGE = LDS_ROWS * A_ROW_BYTES;
-  constexpr bool RING = FP8 && !SC_LDS;
-  constexpr bool DEEP = SC_LDS && deep_mode(FP8, LDS_ROWS);
+  constexpr bool DEEP = SC_LDS && deep_mode(LDS_ROWS);
   static_assert(KS == 1 || (DEEP && NFR == 1 && (KS == 2 || KS == 4)), "K groups: deep mode, one row fragment");
-  constexpr PipeShape PS = pipe_shape(FP8, RING, LDS_ROWS, DEEP, KS);
+  constexpr PipeShape PS = pipe_shape(LDS_ROWS, DEEP, KS);
   constexpr int DA = PS.da, DB = PS.db;
   auto a_slot = [](int it) { return DA == 2 ? (it & 1) : it % DA; };
   constexpr uint32_t kOob = 0x7FFFFFFFu;
@@ -874,11 +851,7 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
   const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds;
   const uint32_t lds_b = lds_base + DA * A_STAGE + wave * 4096;
   const uint8_t *bbuf = lds + DA * A_STAGE + wave * 4096;
-  // activation block scales (fp8 path): two stages of four planes (one per 32-K group of the stage) of one dword
-  // per row; a copy always writes 64 dwords (lanes past the tile's rows write zeros)
-  constexpr int AS_ROWS = LDS_ROWS < 64 ? 64 : LDS_ROWS;
-  constexpr int AS_BYTES = PS.as_bytes;
-  uint8_t *lds_sc = KS > 1 ? lds_wg + KS * PIPE_G : lds + DA * A_STAGE + DB * B_BYTES + AS_BYTES;
+  uint8_t *lds_sc = KS > 1 ? lds_wg + KS * PIPE_G : lds + DA * A_STAGE + DB * B_BYTES;
 
   // ---- scales of the whole tile, once.  Strided: 256 columns x G bytes, contiguous in memory.  CDNA4
   // pre-shuffle: the tile's 8 blocks of 32 columns are contiguous too (KSP*32 bytes each); byte
@@ -936,53 +909,10 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
   const int sc_lane_off[2] = {h * (cdna4 ? 64 : 1), (2 + h) * (cdna4 ? 64 : 1)};  // the (2q + h) part of a group's offset
   const int sc_clamp = cdna4 ? 0x7FFFFFFF : G - 1;
 
-  // ---- block scales of the activations (MXFP8): the 4 e8m0 bytes of a row's 128-K stage are copied per stage to
-  // LDS, one byte-sized copy per group (64 rows per instruction, waves 0 and 1; groups past K/32 are not read at
-  // all, so nothing beyond a row's own scales is touched)
-  const bool x_mx = FP8 && a.x_mx_scale != nullptr;
-  constexpr int AS_AT = DA * A_STAGE + DB * B_BYTES + PS.scr_bytes;
-  const uint32_t lds_as = lds_base + AS_AT;
-  const uint32_t *as_buf = (const uint32_t *)(lds + AS_AT);
-  // (bytes per copy and row: all four of a stage where rows and K allow aligned dwords, two, or one.  A copy of 64 rows
-  // touches up to 64 lines whatever its width; a layer of 2048 MXFP4 tokens, K 2880, 553 us byte by byte, 544 in pairs)
-  const uint64_t as_at = (uint64_t)(uintptr_t)a.x_mx_scale | (uint64_t)a.x_mx_stride_m | (uint64_t)a.x_mx_stride_z | (uint64_t)G;
-  const int as_w = (as_at & 3) == 0 ? 4 : ((as_at & 1) == 0 ? 2 : 1);
-  v4i_t ras = rx;
-  uint32_t as_off = kOob;
-  if (x_mx) {
-    const int64_t xr = a.x_rows > 0 ? a.x_rows : a.M;
-    ras = make_rsrc(a.x_mx_scale + (int64_t)t.z * a.x_mx_stride_z, (uint32_t)(xr * a.x_mx_stride_m));
-    const int r = wave * 64 + lane;
-    if (wave * 64 < LDS_ROWS && r < LDS_ROWS) {
-      const int rr = t.off_m + (r < t.rows ? r : t.rows - 1);
-      const uint32_t src = a.gather_indx ? (uint32_t)a.gather_indx[t.start_m + rr] : (uint32_t)(t.start_m + rr);
-      as_off = src * (uint32_t)a.x_mx_stride_m;
-    }
-  }
   // Copies per request, as the counted waits of the ring loops below see them (a wave's copies complete in the order
   // of their requests): the loops of the issue_* functions run to these numbers and the waits are written in them.
   constexpr int CP_A = NFR;        // issue_a: one copy per row fragment
-  constexpr int CP_AS = 4;         // issue_as: 4 / as_w, one per 32-K group of the stage at most (waves that hold rows only)
   constexpr int CP_B = 4;          // issue_b: four 1 KB pieces
-  constexpr int CP_BPAIR = 8;      // issue_b_pair: eight
-  constexpr int CP_SC_STRIDED = 4; // issue_sc: one per group with strided scales, one in all when pre-shuffled
-  auto issue_as = [&](int it) {
-    if (x_mx && wave * 64 < LDS_ROWS) {
-      const uint32_t at = lds_as + a_slot(it) * 4 * AS_ROWS * 4 + wave * 256;   // plane 0; planes are AS_ROWS dwords apart
-      if (as_w == 4) {
-        dma4(ras, at, it * 4 < G ? as_off : kOob, (uint32_t)(it * 4));
-      } else if (as_w == 2) {
-#pragma unroll
-        for (int p = 0; p < 2; ++p)
-          dma2(ras, at + p * AS_ROWS * 4, it * 4 + 2 * p < G ? as_off : kOob, (uint32_t)(it * 4 + 2 * p));
-      } else {
-#pragma unroll
-        for (int g4 = 0; g4 < CP_AS; ++g4)
-          dma1(ras, at + g4 * AS_ROWS * 4, it * 4 + g4 < G ? as_off : kOob, (uint32_t)(it * 4 + g4));
-      }
-    }
-  };
-
   // ---- activation DMA: one instruction per 32-row fragment, lane -> (row 8w + lane/8, slot lane%8)
   const int a_rin = wave * 8 + lane / 8;
   const int a_chunk = (lane % 8) ^ ((a_rin >> 1) & 7);
@@ -991,22 +921,12 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
   uint32_t a_off[NFR];
   const int row0 = t.start_m + t.off_m;
   auto row_off = [&](int r, uint32_t src) { return r < t.rows ? src * (uint32_t)(a.x_stride_m * ESZ) + a_chunk * 16 : kOob; };
-  // 16-bit rows: their indices are the first thing requested, and the first weights, which do not depend on them, are requested while
-  // they come.  (fp8 rows: the paired copies of their weights are twice as long and the tile starts later, 158 x 640 x 1080 7.6 us
-  // against 7.3.)
+  // The rows' indices are the first thing requested, and the first weights, which do not depend on them, while they come.
   uint32_t row_idx[NFR];
-  if constexpr (!FP8) {
-    const v4i_t rg = make_rsrc(a.gather_indx + row0, (uint32_t)__builtin_amdgcn_readfirstlane(t.rows) * 4u);
-    if (a.gather_indx) {
+  const v4i_t rg = make_rsrc(a.gather_indx + row0, (uint32_t)__builtin_amdgcn_readfirstlane(t.rows) * 4u);
+  if (a.gather_indx) {
 #pragma unroll
-      for (int i = 0; i < NFR; ++i) row_idx[i] = request_dword(rg, (uint32_t)(i * 32 + a_rin) * 4u);
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < NFR; ++i) {
-      const int r = i * 32 + a_rin, rr = r < t.rows ? r : t.rows - 1;
-      a_off[i] = row_off(r, a.gather_indx ? (uint32_t)a.gather_indx[row0 + rr] : (uint32_t)(row0 + rr));
-    }
+    for (int i = 0; i < NFR; ++i) row_idx[i] = request_dword(rg, (uint32_t)(i * 32 + a_rin) * 4u);
   }
   auto rows_known = [&](auto newer) {   // (after `newer` further requests of the wave)
     if (a.gather_indx) await_dwords<decltype(newer)::value>(row_idx);
@@ -1047,7 +967,7 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
   const int n_ka = (K + KA - 1) / KA;      // activation stages
   const int n_kb = (K + KB - 1) / KB;      // weight super-stages (two activation stages each)
   auto issue_a = [&](int it) {             // clamped: past the end the last stage is copied again
-    if constexpr (!RING && !DEEP) it = it < n_ka ? it : n_ka - 1;   // (ring / deep mode: chunks past K are not read at all)
+    if constexpr (!DEEP) it = it < n_ka ? it : n_ka - 1;   // (deep mode: chunks past K are not read at all)
     const int kb = k0 + it * KA;
     const uint32_t akill = kb + a_chunk * (16 / ESZ) < k_hi ? 0u : kOob;
     const uint32_t sb = lds_base + a_slot(it) * A_STAGE + wave * 8 * A_ROW_BYTES;
@@ -1056,7 +976,7 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
   };
   auto issue_b = [&](int sup) {
     const uint32_t region = DB == 2 ? (uint32_t)(sup & 1) * B_BYTES : 0u;
-    if constexpr (!RING && !DEEP) sup = sup < n_kb ? sup : n_kb - 1;
+    if constexpr (!DEEP) sup = sup < n_kb ? sup : n_kb - 1;
     const int kb = k0 + sup * KB;
     static_assert(CP_B == 4, "dma16_x4 makes four copies");
     if (wnat) {   // one 4 KB block, copied as it lies
@@ -1069,96 +989,17 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
       dma16(rw, lds_b + region + j * 1024, w_off[j] | bkill, (uint32_t)(sup0 + sup) << w_stage_shift);
     }
   };
-  // Paired form (ring mode, row blocks of up to 64 rows): the weights of stages 2p and 2p + 1 are 128 contiguous bytes
-  // of every column and are requested as such -- eight lanes per column, so that a column's piece is one 128-byte
-  // request where it lies inside a line instead of two of 64 bytes a stage apart.  With few rows per expert these
-  // requests are what keeps each CU's address unit and L1 busy.  Instruction j copies positions 8j + lane/8 (128 bytes
-  // each, wave-private 8 KB); slot lane%8 of position p holds the column's 16-byte part (lane%8) ^ ((p>>1)&7), which
-  // keeps the operand reads of 16 consecutive positions on distinct banks.
-  constexpr bool PAIRED = RING && DA == 3;
-  const uint32_t lds_b2 = lds_base + DA * A_STAGE + wave * 8192;
-  const uint8_t *bbuf2 = lds + DA * A_STAGE + wave * 8192;
-  uint32_t w2_off[PAIRED ? 8 : 1];
-  int w2_part[PAIRED ? 8 : 1];
-  if constexpr (PAIRED) {
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int pos = j * 8 + lane / 8;
-      const int col = t.n0 + wave * 64 + 2 * (pos % 32) + pos / 32;
-      w2_part[j] = (lane % 8) ^ ((pos >> 1) & 7);
-      w2_off[j] = (uint32_t)(col < N ? col : N - 1) * (uint32_t)a.w_stride_n + w2_part[j] * 16;
-    }
-  }
-  auto issue_b_pair = [&](int pair) {
-    if constexpr (PAIRED) {
-      const int kb = pair * 256;
-      static_assert(CP_BPAIR == 8, "two dma16_x4, or eight copies of 128 bytes per column");
-      if (wnat) {
-        // block layout: the pair's two stages are two 4 KB blocks, copied as they lie (first stage, then second)
-        dma16_x4(rw, lds_b2, w_off[0] | ((wave_live && kb < K) ? 0u : kOob), (uint32_t)(2 * pair) * 4096u);
-        dma16_x4(rw, lds_b2 + 4096, w_off[0] | ((wave_live && kb + KB < K) ? 0u : kOob), (uint32_t)(2 * pair + 1) * 4096u);
-        return;
-      }
-#pragma unroll
-      for (int j = 0; j < CP_BPAIR; ++j) {
-        const uint32_t bkill = (wave_live && kb + w2_part[j] * 32 < K) ? 0u : kOob;
-        dma16(rw, lds_b2 + j * 1024, w2_off[j] | bkill, kb >> 1);
-      }
-    }
-  };
-  // ring mode: the scales of weight stage `sup` for this wave's 64 columns, into the wave's 1 KB piece of the scale
-  // ring.  Pre-shuffled layout: one copy -- the wave's two blocks of 32 columns hold the 8 groups that contain the
-  // stage's 4 as 256 contiguous bytes each (lanes 0-15 / 16-31; the other lanes copy nothing).  Strided layout:
-  // one byte-sized copy per group, lane L fetching column L of the strip into dword [group][L]; slow (64 lines
-  // touched per copy) and only used when the scales of a tile do not fit LDS.
-  const uint32_t lds_scr = lds_base + DA * A_STAGE + DB * B_BYTES;
-  const uint8_t *scr_buf = lds + DA * A_STAGE + DB * B_BYTES;
-  uint32_t scr_voff = kOob;
-  v4i_t rsc = rw;
-  if constexpr (RING) {
-    rsc = make_rsrc(s_base, kOob);
-    if (cdna4) {
-      const int blk = (t.n0 + wave * 64) / 32 + lane / 16;
-      if (lane < 32 && blk * 32 < N && wave_live) scr_voff = (uint32_t)(blk * KSP * 32 + (lane % 16) * 16);
-    } else {
-      const int col = t.n0 + wave * 64 + lane;
-      if (col < N) scr_voff = (uint32_t)((int64_t)col * a.w_mx_stride_n);
-    }
-  }
-  auto issue_sc = [&](int sup) {
-    if constexpr (RING) {
-      const uint32_t dst = lds_scr + ((uint32_t)(sup & 1) * 4 + wave) * 1024;
-      if (cdna4) {
-        dma16(rsc, dst, sup * 4 < G ? scr_voff : kOob, (uint32_t)(256 * (sup >> 1)));
-      } else {
-#pragma unroll
-        for (int g4 = 0; g4 < CP_SC_STRIDED; ++g4) {
-          const int kg = sup * 4 + g4;
-          dma1(rsc, dst + g4 * 256, kg < G ? scr_voff : kOob, (uint32_t)((int64_t)kg * a.w_mx_stride_k));
-        }
-      }
-    }
-  };
-
-  // (two register sets: the ring loop for row blocks of up to 64 rows keeps the weights of two stages)
-  uint4 raw[2][NF][2];
-  float scf[NF][2];      // 16-bit path: 2^(e-127) as a float
-  uint32_t scw[2][NF];   // fp8 path: scale bytes of q = 0, 1 in bytes 0, 1
-  // registers (set `set`) <- this wave's weights and scales of super-stage `sup`
-  auto load_b = [&](int sup, auto set_c) {
-    constexpr int set = decltype(set_c)::value;
+  uint4 raw[NF][2];
+  float scf[NF][2];      // 2^(e-127) as a float
+  // registers <- this wave's weights and scales of super-stage `sup`
+  auto load_b = [&](int sup) {
 #pragma unroll
     for (int f = 0; f < NF; ++f)
 #pragma unroll
       for (int q = 0; q < 2; ++q) {
         const int pos = f * 32 + c32;
         const int rot = ((pos >> 2) & 3) ^ (f << 1);   // slot of part p of position pos: p ^ rot
-        if constexpr (PAIRED)
-          raw[set][f][q] = wnat ? *(const uint4 *)(bbuf2 + (sup & 1) * 4096 + pos * 64 + (((2 * q + h) ^ rot) * 16))
-                                : *(const uint4 *)(bbuf2 + pos * 128 + (((4 * (sup & 1) + 2 * q + h) ^ ((pos >> 1) & 7)) * 16));
-        else
-          raw[set][f][q] = *(const uint4 *)(bbuf + (DB == 2 ? (sup & 1) * B_BYTES : 0) + pos * 64 +
-                                            (((2 * q + h) ^ rot) * 16));
+        raw[f][q] = *(const uint4 *)(bbuf + (DB == 2 ? (sup & 1) * B_BYTES : 0) + pos * 64 + (((2 * q + h) ^ rot) * 16));
         // group kg = 4*sup + 2q + h of this lane's column.  Strided: byte kg, kept inside the column's G bytes
         // (groups past the end of K meet zero codes and zero activations; their scale only has to be some finite
         // value of this column).  Pre-shuffled: byte 256*(kg/8) + 64*(kg%4) + 2*((kg%8)/4); the padding up to a
@@ -1169,205 +1010,46 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
         int kg_off = sup_off + sc_lane_off[q];
         kg_off = kg_off < sc_clamp ? kg_off : sc_clamp;
         uint32_t sbyte;
-        if constexpr (RING) {
-          const uint8_t *piece = scr_buf + ((sup & 1) * 4 + wave) * 1024;
-          const int n = c32 * NF + f;  // column inside the wave's strip
-          sbyte = cdna4 ? piece[(n / 32) * 256 + 64 * (2 * q + h) + 4 * (n % 16) + 2 * (sup & 1) + (n % 32) / 16]
-                        : piece[((2 * q + h) * 64 + n) * 4];
-        } else if constexpr (SC_LDS) sbyte = lds_sc[sc_col_off[f] + kg_off];
+        if constexpr (SC_LDS) sbyte = lds_sc[sc_col_off[f] + kg_off];
         else if (cdna4) sbyte = s_base[sc_col_off[f] + kg_off];
         else sbyte = s_base[(int64_t)(col0 + f < N ? col0 + f : N - 1) * a.w_mx_stride_n + kg_off];
-        if constexpr (FP8) scw[set][f] = q == 0 ? sbyte : (scw[set][f] | (sbyte << 8));
-        else scf[f][q] = bits_to_f32(sbyte << 23);
+        scf[f][q] = bits_to_f32(sbyte << 23);
       }
   };
 
-  // fp8 path: A fragments of the two 64-K halves of a stage and the activations' scale operands
-  i32x8_t af8[FP8 ? 2 : 1][FP8 ? NFR : 1];
-  int sa8[FP8 ? NFR : 1];
-  auto fp8_read_frags = [&](const uint8_t *buf, int s, i32x8_t *af) {
-    const int swz = (c32 >> 1) & 7;
-#pragma unroll
-    for (int i = 0; i < NFR; ++i) {
-      const uint8_t *row = buf + (i * 32 + c32) * A_ROW_BYTES;
-      const uint4 lo = *(const uint4 *)(row + (((4 * s + h) ^ swz) * 16));
-      const uint4 hi = *(const uint4 *)(row + (((4 * s + 2 + h) ^ swz) * 16));
-      af[i] = i32x8_t{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
-    }
-  };
-  // first-half fragments and scale operands of stage `it`: issued together with the weight reads of the stage, so
-  // that their latency passes while the next stage's copies are requested
-  auto fp8_read0 = [&](int it) {
-    if constexpr (FP8) {
-      if (!wave_live) return;
-      const uint8_t *buf = lds + a_slot(it) * A_STAGE;
-      fp8_read_frags(buf, 0, af8[0]);
-      // A scale operand: lane half h supplies K block h of an MFMA; byte 0 is the group of s = 0, byte 2 of s = 1
-      const uint32_t *as = as_buf + a_slot(it) * 4 * AS_ROWS + c32;
-      if (!x_mx) {
-#pragma unroll
-        for (int i = 0; i < NFR; ++i) sa8[i] = 0x7F7F7F7F;
-      } else if (as_w == 4) {
-#pragma unroll
-        for (int i = 0; i < NFR; ++i) sa8[i] = (int)(as[i * 32] >> (8 * h));
-      } else if (as_w == 2) {
-#pragma unroll
-        for (int i = 0; i < NFR; ++i) sa8[i] = (int)(((as[i * 32] & 0xFFFFu) | (as[AS_ROWS + i * 32] << 16)) >> (8 * h));
-      } else {
-#pragma unroll
-        for (int i = 0; i < NFR; ++i) sa8[i] = (int)(as[h * AS_ROWS + i * 32] | (as[(2 + h) * AS_ROWS + i * 32] << 16));
-      }
-    }
-  };
-
-  auto compute = [&](int it, auto qc, auto set_c) {
+  auto compute = [&](int it, auto qc) {
     constexpr int q = decltype(qc)::value;
-    constexpr int set = decltype(set_c)::value;
     if (!wave_live) return;
     const uint8_t *buf = lds + a_slot(it) * A_STAGE;
-    if constexpr (FP8) {
-      // one stage = 128 K = two scaled MFMAs per (row fragment, column fragment); the fragments of the first half
-      // and the activations' scale operands are already in registers (fp8_read0)
-      constexpr int CBSZ = XDT == TAMD_FP8_E5M2 ? 1 : 0;
-      // (the fragments of the second half are requested one by one behind the last MFMAs that use those of the first:
-      // both halves of all fragments at once are 64 registers, which this kernel does not have)
-      const int swz = (c32 >> 1) & 7;
+    auto read_frags = [&](int s, frag_t *af) {
+      const int slot = (h * 4 + s) ^ ((c32 >> 1) & 7);
 #pragma unroll
-      for (int s = 0; s < 2; ++s) {
+      for (int i = 0; i < NFR; ++i) af[i] = *(const frag_t *)(buf + (i * 32 + c32) * A_ROW_BYTES + slot * 16);
+    };
+    frag_t af[2][NFR];
+    read_frags(0, af[0]);
 #pragma unroll
-        for (int f = 0; f < NF; ++f) {
-          const uint4 r = raw[set][f][s];
-          const i32x8_t bf = i32x8_t{(int)r.x, (int)r.y, (int)r.z, (int)r.w, 0, 0, 0, 0};
+    for (int s = 0; s < 4; ++s) {
+      if (s < 3) read_frags(s + 1, af[(s + 1) & 1]);
 #pragma unroll
-          for (int i = 0; i < NFR; ++i) {
-            if (s == 0) {
-              acc[i][f] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(af8[0][i], bf, acc[i][f], CBSZ, 4, 0, sa8[i], 0,
-                                                                        (int)scw[set][f]);
-              if (f == NF - 1) {
-                const uint8_t *row = buf + (i * 32 + c32) * A_ROW_BYTES;
-                const uint4 lo = *(const uint4 *)(row + (((4 + h) ^ swz) * 16));
-                const uint4 hi = *(const uint4 *)(row + (((6 + h) ^ swz) * 16));
-                af8[1][i] = i32x8_t{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
-              }
-            } else {
-              acc[i][f] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(af8[1][i], bf, acc[i][f], CBSZ, 4, 2, sa8[i], 1,
-                                                                        (int)scw[set][f]);
-            }
-          }
-        }
-      }
-    } else {
-      auto read_frags = [&](int s, frag_t *af) {
-        const int slot = (h * 4 + s) ^ ((c32 >> 1) & 7);
+      for (int f = 0; f < NF; ++f) {
+        const uint4 r = raw[f][q];
+        const uint32_t codes = s == 0 ? r.x : (s == 1 ? r.y : (s == 2 ? r.z : r.w));
+        const frag_t bf = M::expand(codes, scf[f][q]);
 #pragma unroll
-        for (int i = 0; i < NFR; ++i) af[i] = *(const frag_t *)(buf + (i * 32 + c32) * A_ROW_BYTES + slot * 16);
-      };
-      frag_t af[2][NFR];
-      read_frags(0, af[0]);
-#pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        if (s < 3) read_frags(s + 1, af[(s + 1) & 1]);
-#pragma unroll
-        for (int f = 0; f < NF; ++f) {
-          const uint4 r = raw[set][f][q];
-          const uint32_t codes = s == 0 ? r.x : (s == 1 ? r.y : (s == 2 ? r.z : r.w));
-          const frag_t bf = M::expand(codes, scf[f][q]);
-#pragma unroll
-          for (int i = 0; i < NFR; ++i) acc[i][f] = M::mma(af[s & 1][i], bf, acc[i][f]);
-        }
+        for (int i = 0; i < NFR; ++i) acc[i][f] = M::mma(af[s & 1][i], bf, acc[i][f]);
       }
     }
   };
 
-  typedef std::integral_constant<int, 0> Set0;
-  typedef std::integral_constant<int, 1> Set1;
-  if constexpr (RING) {
-    // Copies complete in the order of their requests, so a stage waits by count for what it needs and leaves the
-    // later requests in flight.
-    // copies of activation scales in a request of this wave, and the wait that leaves `base` other copies and them in flight
-    const int n_as = x_mx && wave * 64 < LDS_ROWS ? CP_AS / as_w : 0;
-    auto wait_with_as = [&](auto base_c) {
-      constexpr int base = decltype(base_c)::value;
-      if (n_as == 0) wait_vmcnt<base>();
-      else if (n_as == 1) wait_vmcnt<base + 1>();
-      else if (n_as == 2) wait_vmcnt<base + 2>();
-      else wait_vmcnt<base + CP_AS>();
-    };
-    constexpr int NSC = CP_SC_STRIDED;  // scale copies of a stage with strided scales (1 when pre-shuffled)
-    if constexpr (PAIRED) {
-      // Three activation stages; an even stage s moves the weights of s and s + 1 into registers and requests those of
-      // s + 2 and s + 3 (one pair), the odd stage requests only activations.
-      issue_a(0), issue_as(0);
-      issue_b_pair(0), issue_sc(0), issue_sc(1);
-      issue_a(1), issue_as(1);
-      for (int it = 0; it < n_ka; it += 2) {
-        // in flight at most: the activations of stage it + 1
-        wait_with_as(std::integral_constant<int, CP_A>{});
-        __syncthreads();
-        load_b(it, Set0{});
-        load_b(it + 1, Set1{});
-        fp8_read0(it);
-        issue_a(it + 2);
-        issue_as(it + 2);
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // weights are in registers: their buffer may be refilled
-        issue_b_pair((it >> 1) + 1);
-        issue_sc(it + 2), issue_sc(it + 3);
-        compute(it, Set0{}, Set0{});
-        if (it + 1 < n_ka) {
-          // in flight at most: everything the even stage requested
-          if (cdna4) wait_with_as(std::integral_constant<int, CP_A + CP_BPAIR + 2>{});
-          else wait_with_as(std::integral_constant<int, CP_A + CP_BPAIR + 2 * NSC>{});
-          __syncthreads();
-          fp8_read0(it + 1);
-          issue_a(it + 3);
-          issue_as(it + 3);
-          compute(it + 1, Set0{}, Set1{});
-        }
-      }
-    } else {
-      // Stage s requests the activations of stage s + 1 and then the weights and scales of stage s + 2 (the weight
-      // buffer of stage s is free as soon as its contents are in registers): in flight at the top of a stage are at
-      // most the weights and scales the stage before requested (5 copies, or 8 with strided scales).
-      issue_b(0), issue_sc(0);
-      issue_a(0), issue_as(0), issue_b(1), issue_sc(1);
-      for (int it = 0; it < n_ka; ++it) {
-        if (cdna4) wait_vmcnt<CP_B + 1>(); else wait_vmcnt<CP_B + NSC>();
-        __syncthreads();
-        load_b(it, Set0{});
-        fp8_read0(it);
-        issue_a(it + DA - 1);
-        issue_as(it + DA - 1);
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // weights are in registers: their buffer may be refilled
-        issue_b(it + 2);
-        issue_sc(it + 2);
-        compute(it, Set0{}, Set0{});
-      }
-    }
-  } else {
+  typedef std::integral_constant<int, 0> Even;
+  typedef std::integral_constant<int, 1> Odd;
   // (the scales of the whole tile are first read in stage 0: requested behind that stage's own copies, before any later one)
-  if constexpr (FP8) {
-    if constexpr (SC_LDS) stage_scales();
-    issue_a(0), issue_b(0);
-  } else {
-    issue_b(0);
-    rows_known(std::integral_constant<int, CP_B>{});
-    issue_a(0);
-    if constexpr (SC_LDS) stage_scales();
-  }
-  if constexpr (FP8) {
-    issue_as(0);
-    for (int it = 0; it < n_ka; ++it) {  // activation and weight stages coincide (128 K each)
-      wait_dma();
-      __syncthreads();
-      load_b(it, Set0{});
-      fp8_read0(it);
-      issue_a(it + 1);
-      issue_as(it + 1);
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // weights are in registers: the region may be refilled
-      issue_b(it + 1);
-      compute(it, Set0{}, Set0{});
-    }
-  } else if constexpr (DEEP) {
+  issue_b(0);
+  rows_known(std::integral_constant<int, CP_B>{});
+  issue_a(0);
+  if constexpr (SC_LDS) stage_scales();
+  if constexpr (DEEP) {
     // Stage s requests the activations of stage s + DA - 1, an even stage after them the weights of pair s/2 + DB
     // (a weight region is free once its pair's weights are in registers).  Copies complete in the order of their
     // requests: a stage waits until only the requests made after the ones it needs are outstanding
@@ -1384,37 +1066,36 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
     for (int it = 0; it < n_stage; it += 2) {
       wait_vmcnt<ring_outstanding(DA, DB, CP_A, CP_B, false)>();
       __syncthreads();
-      load_b(it >> 1, Set0{});
+      load_b(it >> 1);
       issue_a(it + DA - 1);
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // weights are in registers: the region may be refilled
       issue_b((it >> 1) + DB);
-      compute(it, Set0{}, Set0{});
+      compute(it, Even{});
       if (it + 1 < n_stage) {
         wait_vmcnt<ring_outstanding(DA, DB, CP_A, CP_B, true)>();
         __syncthreads();
         issue_a(it + DA);
-        compute(it + 1, Set1{}, Set0{});
+        compute(it + 1, Odd{});
       }
     }
   } else {
     for (int it = 0; it < n_ka; it += 2) {
       wait_dma();
       __syncthreads();
-      load_b(it >> 1, Set0{});
+      load_b(it >> 1);
       issue_a(it + 1);
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // weights are in registers: the region may be refilled
       issue_b((it >> 1) + 1);
-      compute(it, Set0{}, Set0{});
+      compute(it, Even{});
       if (it + 1 < n_ka) {
         // the weight copies just issued (4, after the activation stage it + 1) are not needed before the next
         // even stage and take the longest (weights stream from HBM, activations mostly hit L2): leave them in flight
         wait_vmcnt<CP_B>();
         __syncthreads();
         issue_a(it + 2);
-        compute(it + 1, Set1{}, Set0{});
+        compute(it + 1, Odd{});
       }
     }
-  }
   }
   wait_dma();
 
@@ -1452,9 +1133,9 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
     __syncthreads();   // the epilogue's tables take the same memory
   }
   // (the wave's own weight region is free by now: its table goes there)
-  uint8_t *tab = KS > 1 ? lds_wg + wave * 4096 : lds + DA * A_STAGE + wave * (PAIRED ? 8192 : 4096);
+  uint8_t *tab = KS > 1 ? lds_wg + wave * 4096 : lds + DA * A_STAGE + wave * 4096;
   static_assert(epilogue_table_bytes(NFR) <= 4096, "a wave's table fits its weight region");
-  tile_epilogue<NFR, ACT, FP8 ? TAMD_BF16 : XDT, FP8>(kernel_args_late(), t, acc, tab);
+  tile_epilogue<NFR, ACT, XDT, false>(kernel_args_late(), t, acc, tab);
 }
 
 // Row fragments a workgroup can hold: a 128-row block of 16-bit activations also takes a remainder of
@@ -1498,64 +1179,48 @@ __global__ __launch_bounds__(256 * KS, 1) void mm_x16_mxfp4_kgroups_kernel(tamd_
   tile_entry<XDT, BM, ACT, true, KS>(a, grid_n, grid_total, group_m, lds);
 }
 
-template <int XDT, int BM, int ACT, bool SC_LDS>
-__global__ __launch_bounds__(256, 2) void mm_x8_mxfp4_kernel(tamd_matmul_args a, int grid_n, int64_t grid_total,
-                                                                 int group_m) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-  tile_entry<XDT, BM, ACT, SC_LDS>(a, grid_n, grid_total, group_m, lds);
-}
-
 // Whether a problem takes locate_tile_live: it is ragged and the experts fit the lanes.
 inline bool counts_live_blocks(const tamd_matmul_args &a) { return a.block_schedule && a.n_experts <= kWave * kLivePerLane; }
 
 template <int XDT, int BM, int ACT>
 int launch_x16_act(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
   constexpr int LDS_ROWS = TileShape<XDT, BM>::LDS_ROWS;
-  constexpr bool DEEP = deep_mode(is_fp8(XDT), LDS_ROWS);   // (kernels with the scales in LDS)
-  constexpr int PIPE_BYTES = pipe_shape(is_fp8(XDT), false, LDS_ROWS, DEEP).bytes;
-  constexpr int RING_BYTES = pipe_shape(is_fp8(XDT), true, LDS_ROWS).bytes;
+  constexpr bool DEEP = deep_mode(LDS_ROWS);   // (kernels with the scales in LDS)
+  constexpr int PIPE_BYTES = pipe_shape(LDS_ROWS, DEEP).bytes;
   int grid_n = (a.N + BLOCK_N - 1) / BLOCK_N;
   int64_t total = (int64_t)grid_m * grid_n;
   if (total <= 0) return 0;
   int64_t launch = ((total + 7) / 8) * 8;
   if (launch > 0x7FFFFFFF) return TAMD_E_UNSUPPORTED;
-  // scales of a tile are staged in LDS when they are dense ([N][K/32]) or pre-shuffled and two workgroups still fit a CU;
-  // the fp8 path does not stage pre-shuffled scales: they travel with the weight stages (ring mode), as strided ones
-  // do when a tile's worth does not fit
+  // scales of a tile are staged in LDS when they are dense ([N][K/32]) or pre-shuffled and two workgroups still fit a CU
   const int64_t G = a.K / 32;
   const bool cdna4 = a.w_mx_layout == TAMD_SCALE_CDNA4;
   const int64_t sc_bytes = (BLOCK_N * (cdna4 ? (G + 7) / 8 * 8 : G) + 1023) / 1024 * 1024;  // whole 1 KB copies
   const bool dense_sc = cdna4 || (a.w_mx_stride_k == 1 && a.w_mx_stride_n == G && a.w_mx_stride_e % 4 == 0 &&
                                   aligned(a.w_mx_scale, 4) && (BLOCK_N * G) % 4 == 0);
   // (deep mode is worth a CU to itself: up to 156 KB; otherwise two workgroups have to fit)
-  const int sc_in_lds = dense_sc && PIPE_BYTES + sc_bytes <= (DEEP ? 156 : 80) * 1024 && !(is_fp8(XDT) && cdna4);
-  constexpr int PLAIN_BYTES = pipe_shape(is_fp8(XDT), false, LDS_ROWS).bytes;   // 16-bit path, scales read from memory
-  // (ring mode: the block scales of the activations are the pipeline's last region, left out when there are none)
-  constexpr int RING_AS_BYTES = pipe_shape(is_fp8(XDT), true, LDS_ROWS).as_bytes;
-  size_t lds_bytes = sc_in_lds ? PIPE_BYTES + sc_bytes
-                               : (is_fp8(XDT) ? RING_BYTES - (a.x_mx_scale ? 0 : RING_AS_BYTES) : PLAIN_BYTES);
-  void (*kern)(tamd_matmul_args, int, int64_t, int);
-  if constexpr (is_fp8(XDT))
-    kern = sc_in_lds ? mm_x8_mxfp4_kernel<XDT, BM, ACT, true> : mm_x8_mxfp4_kernel<XDT, BM, ACT, false>;
-  else
-    kern = sc_in_lds ? mm_x16_mxfp4_kernel<XDT, BM, ACT, true> : mm_x16_mxfp4_kernel<XDT, BM, ACT, false>;
+  const bool sc_in_lds = dense_sc && PIPE_BYTES + sc_bytes <= (DEEP ? 156 : 80) * 1024;
+  constexpr int PLAIN_BYTES = pipe_shape(LDS_ROWS).bytes;   // scales read from memory
+  const size_t lds_bytes = sc_in_lds ? PIPE_BYTES + sc_bytes : PLAIN_BYTES;
+  void (*kern)(tamd_matmul_args, int, int64_t, int) =
+      sc_in_lds ? mm_x16_mxfp4_kernel<XDT, BM, ACT, true> : mm_x16_mxfp4_kernel<XDT, BM, ACT, false>;
   // row blocks walked together: as many as one expert (or batch entry) has, while their activation
   // rows (BM x K each) fit comfortably in one XCD's 4 MB L2
   const int64_t rows_per_slice = a.block_schedule ? a.M / a.n_experts : a.M;
   int64_t group_m = rows_per_slice / BM;
-  const int64_t fit = (int64_t)(2.5 * 1024 * 1024) / ((int64_t)BM * a.K * (is_fp8(XDT) ? 1 : 2));
+  const int64_t fit = (int64_t)(2.5 * 1024 * 1024) / ((int64_t)BM * a.K * 2);
   group_m = group_m > fit ? fit : group_m;
   group_m = group_m < 1 ? 1 : (group_m > 16 ? 16 : group_m);
-  if (!is_fp8(XDT) && counts_live_blocks(a)) group_m = -group_m;   // (fp8 rows: see locate_tile_live)
-  if constexpr (!is_fp8(XDT) && BM <= 32) {
+  if (counts_live_blocks(a)) group_m = -group_m;
+  if constexpr (BM <= 32) {
     // Fewer tiles than CUs: K groups, so that every SIMD of the CUs that do get a tile holds two to four waves
     // (at least two 128-K pairs per group; the groups' pipelines and the tile's scales have to fit one CU's LDS)
     int cus = 0;
     if (int rc = cu_count(cus)) return rc;
     const int64_t pairs = (a.K + KB - 1) / KB;
     // (four groups where they fit beside the scales -- K up to 5632 --, else two)
-    constexpr size_t PIPE4 = 4 * (size_t)pipe_shape(false, false, LDS_ROWS, true, 4).bytes;
-    constexpr size_t PIPE2 = 2 * (size_t)pipe_shape(false, false, LDS_ROWS, true, 2).bytes;
+    constexpr size_t PIPE4 = 4 * (size_t)pipe_shape(LDS_ROWS, true, 4).bytes;
+    constexpr size_t PIPE2 = 2 * (size_t)pipe_shape(LDS_ROWS, true, 2).bytes;
     const bool four = total * 2 <= cus && pairs >= 8 && PIPE4 + sc_bytes <= 156 * 1024;
     const int ks = four ? 4 : (total <= cus && pairs >= 4 ? 2 : 1);
     const size_t pipe = four ? PIPE4 : PIPE2;
@@ -1614,7 +1279,5 @@ int dispatch_x16_act(const tamd_matmul_args &a, int block_m, int grid_m, hipStre
 }
 int tiled_mm_swiglu_bf16(const tamd_matmul_args &a, int block_m, int grid_m, hipStream_t st);
 int tiled_mm_swiglu_f16(const tamd_matmul_args &a, int block_m, int grid_m, hipStream_t st);
-int tiled_mm_swiglu_fp8e4m3(const tamd_matmul_args &a, int block_m, int grid_m, hipStream_t st);
-int tiled_mm_swiglu_fp8e5m2(const tamd_matmul_args &a, int block_m, int grid_m, hipStream_t st);
 
 }  // namespace tamd

@@ -83,12 +83,12 @@ def _data(t):
 
 def _packed_rows_direct(a_raw, flex, ragged, rows):
     """MXFP4 activations (packed e2m1 codes along K with one e8m0 byte per 32, matmul.py:131-136 of the reference) that
-    the kernel for them reads as they are: whole, aligned 16-byte chunks, K of at least a stage, no split of K (whose
-    ranges are cut in elements), no other type asked for."""
+    the kernel for them reads as they are: whole, aligned 16-byte chunks, no split of K (whose ranges are cut in elements),
+    no other type asked for."""
     split = _opt_flags._constraints().get("split_k") is not None or _opt_flags._opt_flags.get() is not None
     auto_split = not ragged and rows <= 256 and 2 * a_raw.shape[-1] >= 8192
     return (not split and not auto_split and flex.lhs_data.dtype is None and a_raw.is_cuda and a_raw.stride(-1) == 1
-            and a_raw.shape[-1] >= 128 and a_raw.data_ptr() % 16 == 0 and all(s % 16 == 0 for s in a_raw.stride()[:-1]))
+            and a_raw.data_ptr() % 16 == 0 and all(s % 16 == 0 for s in a_raw.stride()[:-1]))
 
 
 def _widen_mxfp4_activations(a_raw):
