@@ -1,6 +1,7 @@
 // Instantiates the tiled MXFP4 grouped matmul kernels (moe_matmul_impl.h) for fp16 activations with the plain epilogue
 // (the SwiGLU ones are compiled in moe_matmul_f16_swiglu.hip) and routes row blocks of 16 to the streaming kernel
 // (moe_matmul_stream.h), which is compiled in moe_matmul_stream_f16.hip.
+#include "moe_matmul_mx.h"
 #include "moe_matmul_stream.h"
 
 namespace tamd {

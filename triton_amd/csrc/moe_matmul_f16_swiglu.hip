@@ -1,5 +1,5 @@
 // Instantiates the tiled MXFP4 grouped matmul kernels (moe_matmul_impl.h) with the fused SwiGLU epilogue.
-#include "moe_matmul_impl.h"
+#include "moe_matmul_mx.h"
 
 namespace tamd {
 int tiled_mm_swiglu_f16(const tamd_matmul_args &a, int block_m, int grid_m, hipStream_t st) {

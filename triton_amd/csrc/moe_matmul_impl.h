@@ -326,29 +326,25 @@ TAMD_DEVICE v4i_t make_rsrc(const void *base, uint32_t num_records) {
 
 constexpr int A_ROW_BYTES = 128;       // LDS bytes per activation row per stage (64 K of 16-bit values)
 constexpr int B_BYTES = 4 * 64 * 64;   // 4 waves x 64 columns x 64 bytes (128 K of fp4)
-// LDS of the K pipeline.  The usual layout: two activation stages, one weight stage (4 KB per wave), the e8m0 scales
+// LDS of the K pipeline.  Row blocks of 128: two activation stages, one weight stage (4 KB per wave), the e8m0 scales
 // of the whole tile staged once.
+// K groups (KS = 2 or 4, row blocks of at most 32 rows): KS groups of four waves share a tile, each taking a contiguous part of
+// K through a pipeline of its own with counted waits, three or four activation stages and one or two weight stages; their
+// partial sums meet in LDS.  A problem with fewer tiles than the part has CUs is bound by what one wave per SIMD can issue (a
+// copy instruction holds its wave for about a hundred cycles); more waves per SIMD fill those gaps.
 struct PipeShape {
   int da, db;        // activation / weight stages
   int bytes;
 };
-// "Deep mode" (scales staged in LDS, row blocks of at most 64 rows): counted waits with three or four activation
-// stages and two weight stages.  With so few rows a stage's MFMAs take less time than a copy needs
-// to arrive, and the K loop of the two-stage pipeline runs at the latency of the copies.
-// K groups (KS = 2 or 4, row blocks of at most 32 rows): KS groups of four waves share a tile, each taking a
-// contiguous part of K through a pipeline of its own; their partial sums meet in LDS.  A problem with fewer tiles than
-// the part has CUs is bound by what one wave per SIMD can issue (a copy instruction holds its wave for about a
-// hundred cycles); more waves per SIMD fill those gaps.
-constexpr bool deep_mode(int lds_rows) { return lds_rows <= 64; }
-constexpr PipeShape pipe_shape(int lds_rows, bool deep = false, int ks = 1) {
+constexpr PipeShape pipe_shape(int lds_rows, int ks = 1) {
   PipeShape p{};
-  p.da = deep ? (ks == 4 ? 3 : (lds_rows <= 32 ? 4 : 3)) : 2;
-  p.db = deep && ks != 4 ? 2 : 1;
+  p.da = ks == 1 ? 2 : (ks == 4 ? 3 : 4);
+  p.db = ks == 2 ? 2 : 1;
   p.bytes = p.da * lds_rows * 128 + p.db * B_BYTES;
   return p;
 }
 
-// Copies that a stage of the counted-wait loop (deep mode) may leave in flight.  The requests are made in this order:
+// Copies that a stage of the counted-wait loop (K groups) may leave in flight.  The requests are made in this order:
 // stage j -- the stages before 0 are the loop's prologue -- asks for the activations of stage j + DA - 1 (NA copies)
 // and, if j is even, after them for the weights of pair j/2 + DB (NB copies).  A stage needs its own activations and,
 // if it is even, its pair's weights; copies complete in the order of their requests, so everything requested after
@@ -810,8 +806,7 @@ TAMD_DEVICE late_args_t &kernel_args_late() {
 // column; weights in the block layout (TAMD_W_CDNA4_BLOCKS) hold exactly this image, 4 KB per strip and 128 K, and
 // are copied as they lie.  The wave reads the region into registers at the start of the stage and immediately
 // requests the next 128 K into it, so weights need no barrier.
-// Loops: two stages and full waits (row blocks above 64 rows or scales not in LDS); counted waits over a
-// deeper ring (deep mode, K groups), see pipe_shape.
+// Loops: two stages and full waits; counted waits over a deeper ring (K groups), see pipe_shape.
 template <int XDT, int NFR, int LDS_ROWS, int ACT, bool SC_LDS, int KS = 1>
 TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds_wg) {
   typedef Mma<XDT> M;
@@ -819,9 +814,9 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
   constexpr int ESZ = 2;                      // bytes per activation element
   constexpr int KA = A_ROW_BYTES / ESZ;       // K per activation stage
   constexpr int A_STAGE = LDS_ROWS * A_ROW_BYTES;
-  constexpr bool DEEP = SC_LDS && deep_mode(LDS_ROWS);
-  static_assert(KS == 1 || (DEEP && NFR == 1 && (KS == 2 || KS == 4)), "K groups: deep mode, one row fragment");
-  constexpr PipeShape PS = pipe_shape(LDS_ROWS, DEEP, KS);
+  constexpr bool DEEP = KS > 1;               // counted waits
+  static_assert(KS == 1 || (SC_LDS && NFR == 1 && (KS == 2 || KS == 4)), "K groups: scales in LDS, one row fragment");
+  constexpr PipeShape PS = pipe_shape(LDS_ROWS, KS);
   constexpr int DA = PS.da, DB = PS.db;
   auto a_slot = [](int it) { return DA == 2 ? (it & 1) : it % DA; };
   constexpr uint32_t kOob = 0x7FFFFFFFu;
@@ -967,7 +962,7 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
   const int n_ka = (K + KA - 1) / KA;      // activation stages
   const int n_kb = (K + KB - 1) / KB;      // weight super-stages (two activation stages each)
   auto issue_a = [&](int it) {             // clamped: past the end the last stage is copied again
-    if constexpr (!DEEP) it = it < n_ka ? it : n_ka - 1;   // (deep mode: chunks past K are not read at all)
+    if constexpr (!DEEP) it = it < n_ka ? it : n_ka - 1;   // (K groups: chunks past K are not read at all)
     const int kb = k0 + it * KA;
     const uint32_t akill = kb + a_chunk * (16 / ESZ) < k_hi ? 0u : kOob;
     const uint32_t sb = lds_base + a_slot(it) * A_STAGE + wave * 8 * A_ROW_BYTES;
@@ -1062,7 +1057,7 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
       if (j + DA - 1 > 0) issue_a(j + DA - 1);
       if (j % 2 == 0 && j / 2 + DB > 0) issue_b(j / 2 + DB);
     }
-    const int n_stage = KS > 1 ? 2 * n_sup : n_ka;   // (K groups: the same trip count, and barriers, for every group)
+    const int n_stage = 2 * n_sup;   // (the same trip count, and barriers, for every group)
     for (int it = 0; it < n_stage; it += 2) {
       wait_vmcnt<ring_outstanding(DA, DB, CP_A, CP_B, false)>();
       __syncthreads();
@@ -1182,28 +1177,23 @@ __global__ __launch_bounds__(256 * KS, 1) void mm_x16_mxfp4_kgroups_kernel(tamd_
 // Whether a problem takes locate_tile_live: it is ragged and the experts fit the lanes.
 inline bool counts_live_blocks(const tamd_matmul_args &a) { return a.block_schedule && a.n_experts <= kWave * kLivePerLane; }
 
+// Blocks of up to 64 rows: moe_matmul_mx.h.
+template <int XDT, int BM, int ACT>
+int launch_mx(const tamd_matmul_args &a, int grid_m, hipStream_t st);
+
 template <int XDT, int BM, int ACT>
 int launch_x16_act(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
   constexpr int LDS_ROWS = TileShape<XDT, BM>::LDS_ROWS;
-  constexpr bool DEEP = deep_mode(LDS_ROWS);   // (kernels with the scales in LDS)
-  constexpr int PIPE_BYTES = pipe_shape(LDS_ROWS, DEEP).bytes;
   int grid_n = (a.N + BLOCK_N - 1) / BLOCK_N;
   int64_t total = (int64_t)grid_m * grid_n;
   if (total <= 0) return 0;
   int64_t launch = ((total + 7) / 8) * 8;
   if (launch > 0x7FFFFFFF) return TAMD_E_UNSUPPORTED;
-  // scales of a tile are staged in LDS when they are dense ([N][K/32]) or pre-shuffled and two workgroups still fit a CU
   const int64_t G = a.K / 32;
   const bool cdna4 = a.w_mx_layout == TAMD_SCALE_CDNA4;
   const int64_t sc_bytes = (BLOCK_N * (cdna4 ? (G + 7) / 8 * 8 : G) + 1023) / 1024 * 1024;  // whole 1 KB copies
   const bool dense_sc = cdna4 || (a.w_mx_stride_k == 1 && a.w_mx_stride_n == G && a.w_mx_stride_e % 4 == 0 &&
                                   aligned(a.w_mx_scale, 4) && (BLOCK_N * G) % 4 == 0);
-  // (deep mode is worth a CU to itself: up to 156 KB; otherwise two workgroups have to fit)
-  const bool sc_in_lds = dense_sc && PIPE_BYTES + sc_bytes <= (DEEP ? 156 : 80) * 1024;
-  constexpr int PLAIN_BYTES = pipe_shape(LDS_ROWS).bytes;   // scales read from memory
-  const size_t lds_bytes = sc_in_lds ? PIPE_BYTES + sc_bytes : PLAIN_BYTES;
-  void (*kern)(tamd_matmul_args, int, int64_t, int) =
-      sc_in_lds ? mm_x16_mxfp4_kernel<XDT, BM, ACT, true> : mm_x16_mxfp4_kernel<XDT, BM, ACT, false>;
   // row blocks walked together: as many as one expert (or batch entry) has, while their activation
   // rows (BM x K each) fit comfortably in one XCD's 4 MB L2
   const int64_t rows_per_slice = a.block_schedule ? a.M / a.n_experts : a.M;
@@ -1213,16 +1203,18 @@ int launch_x16_act(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
   group_m = group_m < 1 ? 1 : (group_m > 16 ? 16 : group_m);
   if (counts_live_blocks(a)) group_m = -group_m;
   if constexpr (BM <= 32) {
-    // Fewer tiles than CUs: K groups, so that every SIMD of the CUs that do get a tile holds two to four waves
-    // (at least two 128-K pairs per group; the groups' pipelines and the tile's scales have to fit one CU's LDS)
+    // Fewer tiles than CUs and K above 1344: K groups, so that every SIMD of the CUs that do get a tile holds two to four
+    // waves (the groups' pipelines and the tile's scales have to fit one CU's LDS).  Shorter K pays for the exchange of the
+    // partial sums more than it gains (over 700 layers with up to 256 tiles of 32 rows: without groups 0.89 of the time at K
+    // 600, 0.96 at 1200, 1.06 at 2100, 1.2 at 3600, 1.35 at 5000).
     int cus = 0;
     if (int rc = cu_count(cus)) return rc;
     const int64_t pairs = (a.K + KB - 1) / KB;
     // (four groups where they fit beside the scales -- K up to 5632 --, else two)
-    constexpr size_t PIPE4 = 4 * (size_t)pipe_shape(LDS_ROWS, true, 4).bytes;
-    constexpr size_t PIPE2 = 2 * (size_t)pipe_shape(LDS_ROWS, true, 2).bytes;
-    const bool four = total * 2 <= cus && pairs >= 8 && PIPE4 + sc_bytes <= 156 * 1024;
-    const int ks = four ? 4 : (total <= cus && pairs >= 4 ? 2 : 1);
+    constexpr size_t PIPE4 = 4 * (size_t)pipe_shape(LDS_ROWS, 4).bytes;
+    constexpr size_t PIPE2 = 2 * (size_t)pipe_shape(LDS_ROWS, 2).bytes;
+    const bool four = total * 2 <= cus && PIPE4 + sc_bytes <= 156 * 1024;
+    const int ks = pairs < 11 ? 1 : (four ? 4 : (total <= cus ? 2 : 1));
     const size_t pipe = four ? PIPE4 : PIPE2;
     if (ks > 1 && dense_sc && pipe + sc_bytes <= 156 * 1024) {
       void (*kk)(tamd_matmul_args, int, int64_t, int) =
@@ -1232,9 +1224,17 @@ int launch_x16_act(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
       return launch_status();
     }
   }
-  if (int rc = raise_lds_limit_once((const void *)kern)) return rc;
-  kern<<<dim3((unsigned)launch), 256, lds_bytes, st>>>(a, grid_n, total, (int)group_m);
-  return launch_status();
+  if constexpr (BM <= 64) {
+    return launch_mx<XDT, BM, ACT>(a, grid_m, st);
+  } else {
+    // scales of a tile are staged in LDS when they are dense ([N][K/32]) or pre-shuffled and two workgroups still fit a CU
+    constexpr int PIPE_BYTES = pipe_shape(LDS_ROWS).bytes;
+    const bool sc_in_lds = dense_sc && PIPE_BYTES + sc_bytes <= 80 * 1024;
+    auto kern = sc_in_lds ? mm_x16_mxfp4_kernel<XDT, BM, ACT, true> : mm_x16_mxfp4_kernel<XDT, BM, ACT, false>;
+    if (int rc = raise_lds_limit_once((const void *)kern)) return rc;
+    kern<<<dim3((unsigned)launch), 256, PIPE_BYTES + (sc_in_lds ? sc_bytes : 0), st>>>(a, grid_n, total, (int)group_m);
+    return launch_status();
+  }
 }
 
 // Row block size of a dense / batched problem (block_m == 0 on entry of a dispatcher): the largest block whose

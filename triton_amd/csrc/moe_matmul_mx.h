@@ -1,8 +1,9 @@
-// Grouped / dense matmul of fp8 or packed e2m1 activations x MXFP4 weights: v_mfma_scale_f32_32x32x64_f8f6f4 on the bytes or
-// codes of both operands and their e8m0 bytes, without any conversion.
+// Grouped / dense matmul of fp8, packed e2m1 or (blocks of up to 64 rows) 16-bit activations x MXFP4 weights.  fp8 and packed rows:
+// v_mfma_scale_f32_32x32x64_f8f6f4 on the bytes or codes of both operands and their e8m0 bytes, without any conversion.  16-bit
+// rows: codes expanded in registers, as in moe_matmul_impl.h.
 //
-// Tile, epilogue, tile location and LDS images are those of moe_matmul_impl.h.  A stage is 256 K (128 K for fp8 rows in blocks of
-// 128): one or two planes of 128 bytes per row against one or two 4 KB weight blocks per wave, four MFMA steps of 64 K (two).
+// Tile, epilogue, tile location and LDS images are those of moe_matmul_impl.h.  A stage is 256 K (128 K for 16-bit rows and for fp8
+// rows in blocks of 128): one or two planes of 128 bytes per row against one or two 4 KB weight blocks per wave, four MFMA steps of 64 K (two).
 // Step q takes, for lane half h, the 32 codes K 64 q + 32 h .. of a column (part 2 (q % 2) + h of weight block q / 2) and of a
 // packed row (chunk 2 q + h); of an fp8 row it takes the 16 values K 64 q + 16 h .. followed by the 16 at K 64 q + 32 + 16 h ..
 // (the operand layout of the instruction, established by one-hot probing).  The scale operand of lane half h is group 2 q + h's.
@@ -19,6 +20,9 @@
 // Before -> now, layers: packed rows, widening included, 2048 tokens, 128 experts (top-4) 531 -> 471 us, 2331 over 16 (top-8) 212 -> 177;
 // fp8 16384 over 32 1587 -> 1550, 13 over 64 (top-2) 34.3 -> 32.2, 509 over 128 647 -> 644; dense fp8, 3425 x 5600 x 2312
 // (strided scales) 104 -> 73, 2 x 3680 x 1336 19.4 -> 14.5, 158 x 640 x 1080 7.3 -> 6.6.
+// 16-bit rows in blocks of up to 64: a barrier per 128 K instead of 64, no scales in LDS, three workgroups per CU (blocks of 32: four) where
+// the kernel with deeper rings beside the tile's scales held one or two: 816 x 4960 x 2776 f16 62.3 -> 35.8 us, 2351 x 1664 x 6992
+// 62 -> 55; 256 tokens over 16 experts, 3776 -> 1280, layer 74.9 -> 66.8.
 #pragma once
 #include "moe_matmul_impl.h"
 
@@ -38,22 +42,34 @@ TAMD_DEVICE uint64_t load_scales(const uint8_t *base, uint32_t voff, int n) {
 
 template <int XDT, int BM>
 struct MxShape {
-  static constexpr bool FP4 = XDT == TAMD_MXFP4;
+  static constexpr bool FP4 = XDT == TAMD_MXFP4, X16 = XDT == TAMD_BF16 || XDT == TAMD_F16;
+  static constexpr int ESZ = X16 ? 2 : 1;                    // bytes per unit of the rows' strides
   static constexpr int MF = BM <= 32 ? 1 : BM / 32;
   static constexpr int ROWS = 32 * MF;
-  static constexpr int KA = FP4 || BM <= 64 ? 256 : 128;     // K per stage
-  static constexpr int PLANES = FP4 ? 1 : KA / 128;          // 128-byte pieces of a row per stage
+  static constexpr int KA = FP4 || (!X16 && BM <= 64) ? 256 : 128;     // K per stage
+  static constexpr int PLANE_K = FP4 ? 256 : (X16 ? 64 : 128);         // K of 128 bytes of a row
+  static constexpr int PLANES = KA / PLANE_K;                // 128-byte pieces of a row per stage
   static constexpr int BLOCKS = KA / KB;                     // weight blocks per wave and stage
   static constexpr int A_STAGE = PLANES * ROWS * A_ROW_BYTES;
   static constexpr int B_WAVE = BLOCKS * 4096;
   static constexpr int LDS = 2 * A_STAGE + 4 * B_WAVE;
-  static constexpr int WGS = BM >= 128 ? 2 : (FP4 ? (BM == 64 ? 3 : 4) : (BM == 64 ? 2 : 3));   // workgroups per CU
+  static constexpr int WGS = BM >= 128 ? 2 : (FP4 || X16 ? (BM == 64 ? 3 : 4) : (BM == 64 ? 2 : 3));   // workgroups per CU
+  static_assert(!X16 || BM <= 64, "larger blocks of 16-bit rows: run_tile");
 };
+
+template <int XDT>
+struct RowMma {   // scaled MFMA: raw dwords
+  typedef i32x8_t frag_t;
+};
+template <>
+struct RowMma<TAMD_BF16> : Mma<TAMD_BF16> {};
+template <>
+struct RowMma<TAMD_F16> : Mma<TAMD_F16> {};
 
 template <int XDT, int NFR, int BM, int ACT>
 TAMD_DEVICE void run_tile_mx(const tamd_matmul_args &a, const Tile &t, uint8_t *lds) {
   typedef MxShape<XDT, BM> S;
-  constexpr bool FP4 = S::FP4;
+  constexpr bool FP4 = S::FP4, X16 = S::X16;
   constexpr int KA = S::KA, PLANES = S::PLANES, BLOCKS = S::BLOCKS, STEPS = KA / 64, A_STAGE = S::A_STAGE, B_WAVE = S::B_WAVE;
   constexpr int FMT = XDT == TAMD_MXFP4 ? 4 : (XDT == TAMD_FP8_E5M2 ? 1 : 0);
   constexpr uint32_t kOob = 0x7FFFFFFFu;
@@ -61,7 +77,7 @@ TAMD_DEVICE void run_tile_mx(const tamd_matmul_args &a, const Tile &t, uint8_t *
   const int c32 = lane % 32, h = lane / 32;
   const int K = a.K, N = a.N, G = K / 32;
   const bool wave_live = t.n0 + wave * 64 < N;
-  const v4i_t rx = make_rsrc((const uint8_t *)a.x + (int64_t)t.z * a.x_stride_z, kOob);
+  const v4i_t rx = make_rsrc((const uint8_t *)a.x + (int64_t)t.z * a.x_stride_z * S::ESZ, kOob);
   const v4i_t rw = make_rsrc((const uint8_t *)a.w + (int64_t)t.expert * a.w_stride_e, kOob);
   const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds;
   const uint32_t lds_b = lds_base + 2 * A_STAGE + wave * B_WAVE;
@@ -72,14 +88,14 @@ TAMD_DEVICE void run_tile_mx(const tamd_matmul_args &a, const Tile &t, uint8_t *
   // ---- row indices: of the rows whose values the lane copies, and of the rows whose scales its MFMAs use
   const int a_rin = wave * 8 + lane / 8;
   const int a_chunk = (lane % 8) ^ ((a_rin >> 1) & 7);
-  uint32_t row_idx[2 * NFR];
+  uint32_t row_idx[X16 ? NFR : 2 * NFR];
   if (a.gather_indx) {
     const v4i_t rg = make_rsrc(a.gather_indx + t.start_m + t.off_m, (uint32_t)__builtin_amdgcn_readfirstlane(t.rows) * 4u);
 #pragma unroll
     for (int i = 0; i < NFR; ++i) {
       const int rs = i * 32 + c32;
       row_idx[i] = request_dword(rg, (uint32_t)(i * 32 + a_rin) * 4u);
-      row_idx[NFR + i] = request_dword(rg, (uint32_t)(rs < t.rows ? rs : t.rows - 1) * 4u);
+      if constexpr (!X16) row_idx[NFR + i] = request_dword(rg, (uint32_t)(rs < t.rows ? rs : t.rows - 1) * 4u);
     }
   }
 
@@ -174,14 +190,14 @@ TAMD_DEVICE void run_tile_mx(const tamd_matmul_args &a, const Tile &t, uint8_t *
 
   uint32_t a_off[NFR];
   auto issue_a = [&](int p) {   // (chunks past K are not read: zeros)
-    constexpr int PLANE_K = FP4 ? 256 : 128, CHUNK_K = PLANE_K / 8;
+    constexpr int PLANE_K = S::PLANE_K, CHUNK_K = PLANE_K / 8;
 #pragma unroll
     for (int u = 0; u < PLANES; ++u) {
       const int kb = p * KA + u * PLANE_K;
       const uint32_t kill = kb + a_chunk * CHUNK_K < K ? 0u : kOob;
       const uint32_t to = lds_base + (p & 1) * A_STAGE + u * S::ROWS * A_ROW_BYTES + wave * 8 * A_ROW_BYTES;
 #pragma unroll
-      for (int i = 0; i < NFR; ++i) dma16(rx, to + i * 32 * A_ROW_BYTES, a_off[i] | kill, FP4 ? kb >> 1 : kb);
+      for (int i = 0; i < NFR; ++i) dma16(rx, to + i * 32 * A_ROW_BYTES, a_off[i] | kill, FP4 ? kb >> 1 : kb * S::ESZ);
     }
   };
 
@@ -191,9 +207,9 @@ TAMD_DEVICE void run_tile_mx(const tamd_matmul_args &a, const Tile &t, uint8_t *
   for (int i = 0; i < NFR; ++i) {
     const int r = i * 32 + a_rin, rs = i * 32 + c32, row0 = t.start_m + t.off_m;
     const uint32_t src = a.gather_indx ? row_idx[i] : (uint32_t)(row0 + r);
-    const uint32_t srs = a.gather_indx ? row_idx[NFR + i] : (uint32_t)(row0 + (rs < t.rows ? rs : t.rows - 1));
+    const uint32_t srs = a.gather_indx ? row_idx[X16 ? i : NFR + i] : (uint32_t)(row0 + (rs < t.rows ? rs : t.rows - 1));
     // rows past the end of the slice are never stored: they are copied as zeros, which keeps the matrix cores' inputs quiet
-    a_off[i] = r < t.rows ? src * (uint32_t)a.x_stride_m + a_chunk * 16 : kOob;
+    a_off[i] = r < t.rows ? src * (uint32_t)(a.x_stride_m * S::ESZ) + a_chunk * 16 : kOob;
     as_off[i] = srs * (uint32_t)a.x_mx_stride_m;
   }
   issue_a(0);
@@ -212,19 +228,23 @@ TAMD_DEVICE void run_tile_mx(const tamd_matmul_args &a, const Tile &t, uint8_t *
         raw[q][f] = wnat || BLOCKS == 1 ? *(const uint4 *)(bbuf + (q >> 1) * 4096 + pos * 64 + (((2 * (q & 1) + h) ^ rot) * 16))
                                         : *(const uint4 *)(bbuf + pos * 128 + (((2 * q + h) ^ ((pos >> 1) & 7)) * 16));
       }
-    auto read_a = [&](int q, int i) {
-      const uint8_t *row = buf + (FP4 ? 0 : (q >> 1) * S::ROWS * A_ROW_BYTES) + (i * 32 + c32) * A_ROW_BYTES;
-      if constexpr (FP4) {
-        const uint4 v = *(const uint4 *)(row + (((2 * q + h) ^ swz) * 16));
+    // operand of step q (of 64 K), fragment i; of 16-bit rows of the u-th 16 K in it
+    auto read_a = [&](int q, int i, int u = 0) {
+      const uint8_t *row = buf + q * 64 / S::PLANE_K * S::ROWS * A_ROW_BYTES + (i * 32 + c32) * A_ROW_BYTES;
+      auto chunk = [&](int c) { return *(const uint4 *)(row + ((c ^ swz) * 16)); };
+      if constexpr (X16) {
+        return __builtin_bit_cast(typename RowMma<XDT>::frag_t, chunk(4 * h + u));
+      } else if constexpr (FP4) {
+        const uint4 v = chunk(2 * q + h);
         return i32x8_t{(int)v.x, (int)v.y, (int)v.z, (int)v.w, 0, 0, 0, 0};
       } else {
-        const uint4 lo = *(const uint4 *)(row + (((4 * (q & 1) + h) ^ swz) * 16)), hi = *(const uint4 *)(row + (((4 * (q & 1) + 2 + h) ^ swz) * 16));
+        const uint4 lo = chunk(4 * (q & 1) + h), hi = chunk(4 * (q & 1) + 2 + h);
         return i32x8_t{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
       }
     };
-    i32x8_t af[NFR];
+    typename RowMma<XDT>::frag_t af[X16 ? 2 : 1][NFR];
 #pragma unroll
-    for (int i = 0; i < NFR; ++i) af[i] = read_a(0, i);
+    for (int i = 0; i < NFR; ++i) af[0][i] = read_a(0, i);
     const int e = KA == 256 ? p : p >> 1;
     if (KA == 256 || (p & 1) == 0) {
       take_sc(e);
@@ -238,19 +258,38 @@ TAMD_DEVICE void run_tile_mx(const tamd_matmul_args &a, const Tile &t, uint8_t *
     if (KA == 256 || (p & 1) == 1) load_sc(e + 1);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the weights are in registers: their buffer may be refilled
     issue_b(p + 1);
-    if (wave_live) {
+    if (!wave_live) continue;
+    if constexpr (X16) {
+      // codes expanded in registers, the scale applied by the instruction
+      typedef Mma<XDT> M;
+#pragma unroll
+      for (int v = 0; v < 4 * STEPS; ++v) {
+        const int q = v / 4, u = v % 4;
+        if (v + 1 < 4 * STEPS) {
+#pragma unroll
+          for (int i = 0; i < NFR; ++i) af[(v + 1) & 1][i] = read_a((v + 1) / 4, i, (v + 1) % 4);
+        }
+#pragma unroll
+        for (int f = 0; f < NF; ++f) {
+          const uint32_t codes = u == 0 ? raw[q][f].x : (u == 1 ? raw[q][f].y : (u == 2 ? raw[q][f].z : raw[q][f].w));
+          const auto bf = M::expand(codes, bits_to_f32((sw[f] >> (8 * q) & 0xFFu) << 23));
+#pragma unroll
+          for (int i = 0; i < NFR; ++i) acc[i][f] = M::mma(af[v & 1][i], bf, acc[i][f]);
+        }
+      }
+    } else {
       // (the fragments of the next step are requested one by one behind the last MFMA that uses those of this one)
-#define TAMD_STEP(q)                                                                                                           \
-  if constexpr (q < STEPS) {                                                                                                   \
-    i32x8_t bf[NF];                                                                                                            \
-    _Pragma("unroll") for (int f = 0; f < NF; ++f)                                                                             \
-        bf[f] = i32x8_t{(int)raw[q < STEPS ? q : 0][f].x, (int)raw[q < STEPS ? q : 0][f].y, (int)raw[q < STEPS ? q : 0][f].z,  \
-                        (int)raw[q < STEPS ? q : 0][f].w, 0, 0, 0, 0};                                                         \
-    _Pragma("unroll") for (int i = 0; i < NFR; ++i) {                                                                          \
-      _Pragma("unroll") for (int f = 0; f < NF; ++f) acc[i][f] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(              \
-          af[i], bf[f], acc[i][f], FMT, 4, q, (int)sa[i], q, (int)sw[f]);                                                      \
-      if constexpr (q + 1 < STEPS) af[i] = read_a(q + 1, i);                                                                   \
-    }                                                                                                                          \
+#define TAMD_STEP(q)                                                                                                        \
+  if constexpr (q < STEPS) {                                                                                                \
+    constexpr int r = q < STEPS ? q : 0;                                                                                    \
+    i32x8_t bf[NF];                                                                                                         \
+    _Pragma("unroll") for (int f = 0; f < NF; ++f) bf[f] =                                                                  \
+        i32x8_t{(int)raw[r][f].x, (int)raw[r][f].y, (int)raw[r][f].z, (int)raw[r][f].w, 0, 0, 0, 0};                        \
+    _Pragma("unroll") for (int i = 0; i < NFR; ++i) {                                                                       \
+      _Pragma("unroll") for (int f = 0; f < NF; ++f) acc[i][f] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(           \
+          af[0][i], bf[f], acc[i][f], FMT, 4, q, (int)sa[i], q, (int)sw[f]);                                                \
+      if constexpr (q + 1 < STEPS) af[0][i] = read_a(q + 1, i);                                                             \
+    }                                                                                                                       \
   }
       TAMD_STEP(0) TAMD_STEP(1) TAMD_STEP(2) TAMD_STEP(3)
 #undef TAMD_STEP
@@ -258,7 +297,7 @@ TAMD_DEVICE void run_tile_mx(const tamd_matmul_args &a, const Tile &t, uint8_t *
   }
   wait_vmcnt<0>();
   // (the wave's own weight region is free by now: its table goes there)
-  tile_epilogue<NFR, ACT, TAMD_BF16, true>(kernel_args_late(), t, acc, lds + 2 * A_STAGE + wave * B_WAVE);
+  tile_epilogue<NFR, ACT, X16 ? XDT : TAMD_BF16, !X16>(kernel_args_late(), t, acc, lds + 2 * A_STAGE + wave * B_WAVE);
 }
 
 template <int XDT, int BM, int ACT>
@@ -288,7 +327,7 @@ int launch_mx(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
   if (launch > 0x7FFFFFFF) return TAMD_E_UNSUPPORTED;
   // row blocks walked together (see launch_x16_act)
   const int64_t rows_per_slice = a.block_schedule ? a.M / a.n_experts : a.M;
-  const int64_t fit = (int64_t)(2.5 * 1024 * 1024) / ((int64_t)BM * a.K / (XDT == TAMD_MXFP4 ? 2 : 1));
+  const int64_t fit = (int64_t)(2.5 * 1024 * 1024) / ((int64_t)BM * a.K * MxShape<XDT, BM>::ESZ / (XDT == TAMD_MXFP4 ? 2 : 1));
   int64_t group_m = rows_per_slice / BM;
   group_m = group_m > fit ? fit : group_m;
   group_m = group_m < 1 ? 1 : (group_m > 16 ? 16 : group_m);
@@ -306,7 +345,9 @@ int dispatch_mx_act(const tamd_matmul_args &a, int block_m, int grid_m, hipStrea
     case 16: return launch_mx<XDT, 16, ACT>(a, grid_m, st);
     case 32: return launch_mx<XDT, 32, ACT>(a, grid_m, st);
     case 64: return launch_mx<XDT, 64, ACT>(a, grid_m, st);
-    case 128: return launch_mx<XDT, 128, ACT>(a, grid_m, st);
+    case 128:
+      if constexpr (XDT != TAMD_BF16 && XDT != TAMD_F16) return launch_mx<XDT, 128, ACT>(a, grid_m, st);
+      [[fallthrough]];
     default: return TAMD_E_UNSUPPORTED;
   }
 }
