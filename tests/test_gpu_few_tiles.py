@@ -78,3 +78,31 @@ def test_microscaled_output_keeps_its_kernel(device):
     with scoped_opt_flags_constraints({"block_m": 32}):
         want = downcast_to_mxfp(matmul(a, w, None, md, precision_config=pc), torch.float8_e4m3fn, axis=-1)
     assert torch.equal(y.view(torch.uint8), want[0].view(torch.uint8)) and torch.equal(ys, want[1])
+
+
+@pytest.mark.parametrize("M,N", [(257, 448), (700, 272), (1500, 128), (161, 2560), (161, 2576), (2100, 1600), (33, 16)])
+@pytest.mark.parametrize("kind", ["bf16", "f16", "fp8", "mxfp4", "bf16 w", "fp8 w"])
+def test_dense(M, N, kind, device):
+    """Dense products around the lines between the streaming kernel's units, blocks of 32, 64 and 128 rows."""
+    torch.manual_seed(M)
+    K = 608
+    x, w = torch.randn(M, K, device=device), torch.randn(K, N, device=device) * 0.1
+    bias = torch.randn(N, device=device)
+    pc = {"out_dtype": torch.bfloat16}
+    if kind[-1] == "w":
+        w = w.to(torch.bfloat16 if kind == "bf16 w" else torch.float8_e4m3fn).t().contiguous().t()
+        wf = w.float()
+    else:
+        w, ws = downcast_to_mxfp(w, torch.uint8, axis=0)
+        wf = upcast_from_mxfp(w, ws, torch.float32, axis=0)
+        pc.update(b_mx_scale=ws, b_microblock_size=32)
+    if kind == "mxfp4":
+        a, s = downcast_to_mxfp(x, torch.uint8, axis=-1)
+        x = upcast_from_mxfp(a, s, torch.float32, axis=-1)
+        pc.update(a_mx_scale=s, a_microblock_size=32)
+    else:
+        a = x.to(torch.float16 if kind == "f16" else torch.float8_e4m3fn if kind[:3] == "fp8" else torch.bfloat16)
+        x = a.float()
+    y = matmul(a, w, bias, precision_config=PrecisionConfig(**pc)).float()
+    ref = x @ wf + bias
+    assert bool(((y - ref).abs() <= 2.0 ** -8 * ref.abs() + K * 2.0 ** -23 * (x.abs() @ wf.abs() + bias.abs()) + 1e-6).all())

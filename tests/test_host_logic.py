@@ -228,8 +228,8 @@ def test_native_host_path_is_tied_to_its_torch(monkeypatch):
         _native.load()
 
 
-def test_few_tiles_block_m_is_one_rule():
-    """The native host code and opt_flags choose the same block where tiles are few; more tiles never get a smaller block."""
+def test_tiles_block_m_is_one_rule():
+    """The native host code and opt_flags choose the same block from the tiles; more tiles never get a smaller block."""
     from triton_amd import _native
     _native.load()
     for m in (1, 7, 64, 300, 1000, 2048, 9000):
@@ -237,13 +237,13 @@ def test_few_tiles_block_m_is_one_rule():
             for expected in (None, 0, 9, 31, 33, 64, 65, 200):
                 for fp8 in (False, True):
                     base = OF.make_opt_flags(m, 1, 1, slices, True, expected, fp8_rows=fp8).block_m
-                    for k in (512, 640, 4096, 4128):
+                    for k in (512, 640, 1152, 1184, 4096, 4128):
                         for mx4, mx_out in ((True, False), (True, True), (False, False)):
                             last = 0
                             for n in (16, 256, 272, 1000, 4096, 11520):
-                                want = OF.few_tiles_block_m(base, m, n, k, slices, expected, mx4, fp8, mx_out)
+                                want = OF.tiles_block_m(base, m, n, k, slices, expected, mx4, fp8, mx_out)
                                 got = _native.choose_block_m(m, slices, True, -1 if expected is None else expected, fp8, n, k, mx4, mx_out)
-                                assert got == want and want <= base
+                                assert got == want and (want <= base or (base, want) == (16, 32))
                                 if n % 16 == 0:
                                     assert want >= last
                                     last = want

@@ -175,18 +175,19 @@ int choose_block_m(int64_t m, int64_t n_slices, bool ragged, int64_t expected, b
   if (ragged && fp8_rows && bm == 16) bm = 32;
   return bm;
 }
-// few_tiles_block_m of the same file; the same test compares the two.
-int few_tiles_block_m(int bm, int64_t m, int64_t n, int64_t k, int64_t n_slices, int64_t expected, bool mxfp4_weights, bool fp8_rows,
+// tiles_block_m of the same file; the same test compares the two.
+int tiles_block_m(int bm, int64_t m, int64_t n, int64_t k, int64_t n_slices, int64_t expected, bool mxfp4_weights, bool fp8_rows,
                       bool mx_out) {
   constexpr int64_t cus = 256;
   const int64_t mean = m / (n_slices > 1 ? n_slices : 1), rows = expected >= 0 ? expected : (mean > 1 ? mean : 1);
   const int64_t slices = n_slices < m ? n_slices : m, cols = (n + 255) / 256;
   auto tiles = [&](int64_t b) { return slices * ((rows + b - 1) / b) * cols; };
   const double cover = (double)rows + 2.0 * std::pow((double)rows, 0.5);
+  if (bm == 16 && mxfp4_weights && tiles(32) > cus * 3 / 4 && k <= 1152) return 32;
   if (bm == 128 && tiles(128) <= (mxfp4_weights ? cus : cus / 2)) bm = 64;
   if (bm == 64 && tiles(64) <= (mxfp4_weights ? cus * 3 / 4 : cus * 3 / 8)) bm = 32;
   if (bm == 32 && mxfp4_weights && !mx_out && n % 16 == 0 && k <= 4096 &&
-      (fp8_rows ? cover <= 16 && tiles(32) <= cus * 3 / 8 && k >= 640 : cover <= 32 && tiles(32) <= cus / 4))
+      (fp8_rows ? cover <= 16 && tiles(32) <= cus * 5 / 16 && k >= 640 : cover <= 32 && tiles(32) <= cus / 4))
     bm = 16;
   return bm;
 }
@@ -438,7 +439,7 @@ PyObject *py_matmul(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
       n_slices = tss.size(0);
       need(n_slices > 0 && n_slices <= n_mat && (!g.bias || tensor(bias_o).dim() == 2));
       const int64_t expected = ex.none() ? -1 : as_int(ex.p);
-      const int bm = few_tiles_block_m(choose_block_m(M, n_slices, true, expected, (a8 || a4) && w_fp4), M, N, K, n_slices, expected,
+      const int bm = tiles_block_m(choose_block_m(M, n_slices, true, expected, (a8 || a4) && w_fp4), M, N, K, n_slices, expected,
                                        w_fp4, a8, mx_out || a4);
       const int row = bm == 16 ? 0 : bm == 32 ? 1 : bm == 64 ? 2 : 3;
       g.slice_sizes = (const int32_t *)tss.data_ptr(), g.slice_offs = (const int32_t *)tso.data_ptr();
@@ -670,7 +671,7 @@ PyObject *py_choose_block_m(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
     need(nargs == 5 || nargs == 9);
     const int bm = choose_block_m(as_int(v[0]), as_int(v[1]), v[2] == Py_True, as_int(v[3]), v[4] == Py_True);
     if (nargs == 5) return PyLong_FromLong(bm);
-    return PyLong_FromLong(few_tiles_block_m(bm, as_int(v[0]), as_int(v[5]), as_int(v[6]), as_int(v[1]), as_int(v[3]), v[7] == Py_True,
+    return PyLong_FromLong(tiles_block_m(bm, as_int(v[0]), as_int(v[5]), as_int(v[6]), as_int(v[1]), as_int(v[3]), v[7] == Py_True,
                                              v[4] == Py_True, v[8] == Py_True));
   });
 }

@@ -85,25 +85,31 @@ def max_allowable_mn(max_mn: int, m: int, n: int, split_k: int) -> int:
 CUS = 256   # compute units of the part
 
 
-def few_tiles_block_m(block_m: int, m: int, n: int, k: int, n_slices: int, expected_slice_size: Optional[int],
-                      mxfp4_weights: bool, fp8_rows: bool, mx_out: bool) -> int:
-    """Row block of a ragged problem whose tiles (row blocks x 256 columns) leave CUs idle: a tile of half the rows takes
-    about half the time per K stage, so smaller blocks win until the CUs are taken, although they read a slice's
-    weights more often.  The lines are those that gave the shortest mean time over 700 layers of 1 to 4000 tokens, 8 to
-    128 experts, K 512 to 5760 (no product more than 5 % slower): MXFP4 weights with 16-bit rows 3.5 % in the mean,
-    fp8 rows 8 %, 16-bit weights 1 %; at 80 tiles of 128 rows (16 slices of 128 rows, 3776 x 1280) 83 us against 38.
-    Few rows per slice and few tiles: the weight-streaming kernel (blocks of 16, units of 16 columns) also for fp8 rows (14 to 60 %
-    up to 100 tiles; not with two blocks per slice, and not below K 640, where a unit is too short)."""
+def tiles_block_m(block_m: int, m: int, n: int, k: int, n_slices: int, expected_slice_size: Optional[int],
+                  mxfp4_weights: bool, fp8_rows: bool, mx_out: bool) -> int:
+    """Row block of a ragged problem, given the one that its slices' sizes ask for, from the number of its tiles (row blocks x
+    256 columns).
+
+    Tiles that leave CUs idle: a tile of half the rows takes about half the time per K stage, so smaller blocks win until
+    the CUs are taken, although they read a slice's weights more often; at 80 tiles of 128 rows (16 slices of 128 rows,
+    3776 x 1280) 83 us against 38.  Few rows per slice and few tiles: the weight-streaming kernel (blocks of 16, units of
+    16 columns), also for fp8 rows (10 to 40 % up to 80 tiles; not with two blocks per slice, and not below K 640, where
+    a unit is too short).  Few rows and many tiles of a short K (up to 1152, where a unit's barrier and start weigh
+    more than its copies): the tiled kernel instead of the streaming one (20 to 50 %).
+    The lines are those that gave the shortest mean time over 700 layers of 1 to 4000 tokens, 8 to 128 experts, K 512
+    to 5760."""
     rows = expected_slice_size if expected_slice_size is not None else max(1, m // max(1, n_slices))
     slices, cols = min(n_slices, m), -(-n // 256)
     tiles = lambda b: slices * -(-rows // b) * cols
     cover = rows + 2.0 * rows ** 0.5
+    if block_m == 16 and mxfp4_weights and tiles(32) > CUS * 3 // 4 and k <= 1152:
+        return 32
     if block_m == 128 and tiles(128) <= (CUS if mxfp4_weights else CUS // 2):
         block_m = 64
     if block_m == 64 and tiles(64) <= (CUS * 3 // 4 if mxfp4_weights else CUS * 3 // 8):
         block_m = 32
     if block_m == 32 and mxfp4_weights and not mx_out and n % 16 == 0 and k <= 4096:
-        if (cover <= 16 and tiles(32) <= CUS * 3 // 8 and k >= 640) if fp8_rows else (cover <= 32 and tiles(32) <= CUS // 4):
+        if (cover <= 16 and tiles(32) <= CUS * 5 // 16 and k >= 640) if fp8_rows else (cover <= 32 and tiles(32) <= CUS // 4):
             block_m = 16
     return block_m
 
