@@ -51,7 +51,8 @@ struct MxShape {
   static constexpr int PLANES = KA / PLANE_K;                // 128-byte pieces of a row per stage
   static constexpr int BLOCKS = KA / KB;                     // weight blocks per wave and stage
   static constexpr int A_STAGE = PLANES * ROWS * A_ROW_BYTES;
-  static constexpr int B_WAVE = BLOCKS * 4096;
+  static constexpr bool PAIRS = !FP4 && BM == 128;           // strided weights: 256 K at a time, every other stage
+  static constexpr int B_WAVE = (PAIRS ? 2 : BLOCKS) * 4096;
   static constexpr int LDS = 2 * A_STAGE + 4 * B_WAVE;
   static constexpr int WGS = BM >= 128 ? 2 : (FP4 || X16 ? (BM == 64 ? 3 : 4) : (BM == 64 ? 2 : 3));   // workgroups per CU
   static_assert(!X16 || BM <= 64, "larger blocks of 16-bit rows: run_tile");
@@ -100,10 +101,13 @@ TAMD_DEVICE void run_tile_mx(const tamd_matmul_args &a, const Tile &t, uint8_t *
   }
 
   // ---- weights: the stage's 4 KB blocks as they lie, or 64 contiguous bytes of every column per 128 K (128 of a pair of blocks:
-  // eight lanes per column, whole lines where the column's piece lies inside one)
+  // eight lanes per column, whole lines where the column's piece lies inside one).  Blocks of 128 rows, whose stage is 128 K,
+  // copy such a pair every other stage: half lines passed the caches twice (3168 fp8 tokens x 8 over 16 experts, 3008 -> 1568,
+  // layer 433 us -> 423; with the halves' shared scale loads below 446 -> 433).
   const bool wnat = a.w_layout == TAMD_W_CDNA4_BLOCKS;
   const uint32_t w_nat = (uint32_t)(((t.n0 >> 6) + wave) * ((K + KB - 1) / KB)) * 4096u + (uint32_t)lane * 16;
-  constexpr int W_LANES = 4 * BLOCKS;                 // lanes per column
+  constexpr int WIDE = S::PAIRS ? 2 : BLOCKS;         // blocks of K that strided weights are copied by
+  constexpr int W_LANES = 4 * WIDE;                   // lanes per column
   const int w_col = t.n0 + wave * 64 + 2 * (lane / W_LANES);
   auto issue_b = [&](int p) {
     const int kb = p * KA;
@@ -113,11 +117,12 @@ TAMD_DEVICE void run_tile_mx(const tamd_matmul_args &a, const Tile &t, uint8_t *
         dma16_x4(rw, lds_b + u * 4096, w_nat | ((wave_live && kb + u * KB < K) ? 0u : kOob), (uint32_t)(BLOCKS * p + u) * 4096u);
       return;
     }
+    if (S::PAIRS && (p & 1) != 0) return;   // (came with the stage before)
 #pragma unroll
-    for (int j = 0; j < 4 * BLOCKS; ++j) {
+    for (int j = 0; j < 4 * WIDE; ++j) {
       // instruction j copies positions (64 / W_LANES) j + lane / W_LANES; position 32 f + c holds column 2 c + f
       constexpr int PER = 64 / W_LANES;
-      const int part = BLOCKS == 2 ? (lane % 8) ^ ((4 * j + lane / 16) & 7) : (lane % 4) ^ ((lane / 16) & 3) ^ ((j >> 1) << 1);
+      const int part = WIDE == 2 ? (lane % 8) ^ ((4 * j + lane / 16) & 7) : (lane % 4) ^ ((lane / 16) & 3) ^ ((j >> 1) << 1);
       const int pos0 = PER * j, col = w_col + 2 * (pos0 % 32) + pos0 / 32;
       const uint32_t kill = (wave_live && kb + part * 32 < K) ? 0u : kOob;
       dma16(rw, lds_b + j * 1024, ((uint32_t)(col < N ? col : N - 1) * (uint32_t)a.w_stride_n + part * 16) | kill, kb >> 1);
@@ -136,8 +141,8 @@ TAMD_DEVICE void run_tile_mx(const tamd_matmul_args &a, const Tile &t, uint8_t *
     ws_off[0] = (uint32_t)((blk < last ? blk : last) * KSP * 32 + 64 * h + 4 * (col0 % 16));
     ws_off[1] = ws_off[0] + 128;
   } else {
-#pragma unroll
-    for (int f = 0; f < NF; ++f) ws_off[f] = (uint32_t)(col0 + f < N ? col0 + f : N - 1) * (uint32_t)a.w_mx_stride_n;
+    // a load touches a line per lane, so each half of the wave loads one of its lanes' two columns and the halves exchange them
+    ws_off[0] = ws_off[1] = (uint32_t)(col0 + h < N ? col0 + h : N - 1) * (uint32_t)a.w_mx_stride_n;
   }
   const int g_last = G > 8 ? G - 8 : 0;               // where the last eight bytes start
   uint64_t as_raw[NFR], ws_raw[NF];
@@ -152,8 +157,8 @@ TAMD_DEVICE void run_tile_mx(const tamd_matmul_args &a, const Tile &t, uint8_t *
       for (int i = 0; i < NFR; ++i) as_raw[i] = load_scales(xs_base + at, as_off[i], G);
     }
     const uint8_t *w = ws_base + (cdna4 ? 256 * e : at);
-#pragma unroll
-    for (int f = 0; f < NF; ++f) ws_raw[f] = load_scales(w, ws_off[f], cdna4 ? 8 : G);
+    ws_raw[0] = load_scales(w, ws_off[0], cdna4 ? 8 : G);
+    if (cdna4) ws_raw[1] = load_scales(w, ws_off[1], 8);
   };
   uint32_t sa[NFR], sw[NF];   // byte q: the scale of step q
   auto take_sc = [&](int e) {
@@ -170,8 +175,12 @@ TAMD_DEVICE void run_tile_mx(const tamd_matmul_args &a, const Tile &t, uint8_t *
 #pragma unroll
       for (int f = 0; f < NF; ++f) sw[f] = __builtin_amdgcn_perm((uint32_t)(ws_raw[1] >> (32 * f)), (uint32_t)(ws_raw[0] >> (32 * f)), s2);
     } else {
+      // (the lane's own column's: column 2 c32 + h)
+      const uint64_t x = ws_raw[0] >> shift;
+      const auto lo = __builtin_amdgcn_permlane32_swap((uint32_t)x, (uint32_t)x, false, false);
+      const auto hi = __builtin_amdgcn_permlane32_swap((uint32_t)(x >> 32), (uint32_t)(x >> 32), false, false);
 #pragma unroll
-      for (int f = 0; f < NF; ++f) sw[f] = pick(ws_raw[f]);
+      for (int f = 0; f < NF; ++f) sw[f] = __builtin_amdgcn_perm(hi[f], lo[f], sel);
     }
     // (made before the next ones are requested, which then come to the same registers)
 #pragma unroll
@@ -225,8 +234,9 @@ TAMD_DEVICE void run_tile_mx(const tamd_matmul_args &a, const Tile &t, uint8_t *
 #pragma unroll
       for (int f = 0; f < NF; ++f) {
         const int pos = f * 32 + c32, rot = ((pos >> 2) & 3) ^ (f << 1);
-        raw[q][f] = wnat || BLOCKS == 1 ? *(const uint4 *)(bbuf + (q >> 1) * 4096 + pos * 64 + (((2 * (q & 1) + h) ^ rot) * 16))
-                                        : *(const uint4 *)(bbuf + pos * 128 + (((2 * q + h) ^ ((pos >> 1) & 7)) * 16));
+        const int qp = S::PAIRS ? q + (p & 1) * STEPS : q;   // the step in its piece of a strided column
+        raw[q][f] = wnat || WIDE == 1 ? *(const uint4 *)(bbuf + (q >> 1) * 4096 + pos * 64 + (((2 * (q & 1) + h) ^ rot) * 16))
+                                      : *(const uint4 *)(bbuf + pos * 128 + (((2 * qp + h) ^ ((pos >> 1) & 7)) * 16));
       }
     // operand of step q (of 64 K), fragment i; of 16-bit rows of the u-th 16 K in it
     auto read_a = [&](int q, int i, int u = 0) {
