@@ -10,7 +10,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("T,E,k", [
-    (192, 16, 8), (193, 16, 8), (129, 16, 8), (96, 128, 4), (97, 128, 4), (129, 128, 8),      # one launch, then two
+    (160, 16, 8), (161, 16, 8), (192, 16, 6), (193, 16, 6), (256, 16, 2), (257, 16, 2), (129, 16, 8),   # one launch, then two
+    (80, 128, 8), (81, 128, 8), (96, 128, 6), (97, 128, 6), (128, 128, 4), (129, 128, 4), (128, 128, 1),
     (2047, 128, 4), (2049, 128, 4), (4096, 128, 4), (4097, 128, 4),                           # 256, 512, 1024 threads
     (255, 60, 6), (300, 100, 6), (1000, 200, 6), (700, 256, 8),                               # chunks that need larger workgroups
     (16385, 16, 8), (32768, 64, 6), (20000, 60, 8), (8192, 256, 8), (300, 200, 1), (130, 8, 1)])

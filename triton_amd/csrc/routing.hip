@@ -1117,9 +1117,12 @@ extern "C" int tamd_routing_gates(const void *logits, int dtype, int64_t stride,
             nb * n_cols <= tamd_bitmatrix_metadata_workspace(n, n_cols))
           TH = th;
       }
-    // one launch while a pass and a half of its threads hold the rows and the entries are few (128 rows of 128, top-8: 17.6 us in
-    // one launch, 11.5 in two; 256 rows of 16, top-8: 16.9 and 10.3; 96 rows of 128, top-4: 9.7 and 10.2)
-    const bool one = n_rows <= (TH ? 3 : 4) * (512 / L) && (!TH || NC <= 16);
+    // One launch while a pass and a half of its threads (two where few columns are picked) hold the rows and the entries are few.
+    // The lines lie where it takes up to 1.2 times as long as two on the GPU, since two take longer to launch than they
+    // run (128 rows of 128, top-8: 17.6 us in one launch, 11.5 in two; top-4 11.8 and 10.4, called on its own 11.8 and
+    // 13.4; 256 rows of 16, top-8: 16.9 and 10.3).
+    const int pass = 1024 / L;
+    const bool one = !TH ? n_rows <= 2 * pass : (2 * n_rows <= 3 * pass || (n_rows <= 2 * pass && k <= (L == 8 ? 2 : 4))) && n <= (L == 8 ? 1280 : 640);
     if (one && NC <= 64 && ints * 4 <= 156 * 1024) {
       int nbits = 0;
       while ((1 << nbits) < n_cols) ++nbits;
