@@ -51,9 +51,9 @@ struct MxShape {
   static constexpr int PLANES = KA / PLANE_K;                // 128-byte pieces of a row per stage
   static constexpr int BLOCKS = KA / KB;                     // weight blocks per wave and stage
   static constexpr int A_STAGE = PLANES * ROWS * A_ROW_BYTES;
-  static constexpr bool PAIRS = !FP4 && BM == 128;           // strided weights: 256 K at a time, every other stage
-  static constexpr int B_WAVE = (PAIRS ? 2 : BLOCKS) * 4096;
-  static constexpr int LDS = 2 * A_STAGE + 4 * B_WAVE;
+  static constexpr bool PAIRS = BLOCKS == 1;                 // strided weights: 256 K at a time, every other stage
+  static constexpr int b_wave(bool blocks) { return (PAIRS && !blocks ? 2 : BLOCKS) * 4096; }   // weight bytes of a wave
+  static constexpr int lds(bool blocks) { return 2 * A_STAGE + 4 * b_wave(blocks); }
   static constexpr int WGS = BM >= 128 ? 2 : (FP4 || X16 ? (BM == 64 ? 3 : 4) : (BM == 64 ? 2 : 3));   // workgroups per CU
   static_assert(!X16 || BM <= 64, "larger blocks of 16-bit rows: run_tile");
 };
@@ -71,7 +71,7 @@ template <int XDT, int NFR, int BM, int ACT>
 TAMD_DEVICE void run_tile_mx(const tamd_matmul_args &a, const Tile &t, uint8_t *lds) {
   typedef MxShape<XDT, BM> S;
   constexpr bool FP4 = S::FP4, X16 = S::X16;
-  constexpr int KA = S::KA, PLANES = S::PLANES, BLOCKS = S::BLOCKS, STEPS = KA / 64, A_STAGE = S::A_STAGE, B_WAVE = S::B_WAVE;
+  constexpr int KA = S::KA, PLANES = S::PLANES, BLOCKS = S::BLOCKS, STEPS = KA / 64, A_STAGE = S::A_STAGE;
   constexpr int FMT = XDT == TAMD_MXFP4 ? 4 : (XDT == TAMD_FP8_E5M2 ? 1 : 0);
   constexpr uint32_t kOob = 0x7FFFFFFFu;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
@@ -81,8 +81,10 @@ TAMD_DEVICE void run_tile_mx(const tamd_matmul_args &a, const Tile &t, uint8_t *
   const v4i_t rx = make_rsrc((const uint8_t *)a.x + (int64_t)t.z * a.x_stride_z * S::ESZ, kOob);
   const v4i_t rw = make_rsrc((const uint8_t *)a.w + (int64_t)t.expert * a.w_stride_e, kOob);
   const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds;
-  const uint32_t lds_b = lds_base + 2 * A_STAGE + wave * B_WAVE;
-  const uint8_t *bbuf = lds + 2 * A_STAGE + wave * B_WAVE;
+  const bool wnat = a.w_layout == TAMD_W_CDNA4_BLOCKS;
+  const int b_at = 2 * A_STAGE + wave * S::b_wave(wnat);   // the wave's weights
+  const uint32_t lds_b = lds_base + b_at;
+  const uint8_t *bbuf = lds + b_at;
   const int n_k = (K + KA - 1) / KA;
   const bool x_mx = FP4 || (XDT == TAMD_FP8_E4M3 && a.x_mx_scale != nullptr);
 
@@ -101,10 +103,10 @@ TAMD_DEVICE void run_tile_mx(const tamd_matmul_args &a, const Tile &t, uint8_t *
   }
 
   // ---- weights: the stage's 4 KB blocks as they lie, or 64 contiguous bytes of every column per 128 K (128 of a pair of blocks:
-  // eight lanes per column, whole lines where the column's piece lies inside one).  Blocks of 128 rows, whose stage is 128 K,
-  // copy such a pair every other stage: half lines passed the caches twice (3168 fp8 tokens x 8 over 16 experts, 3008 -> 1568,
-  // layer 433 us -> 423; with the halves' shared scale loads below 446 -> 433).
-  const bool wnat = a.w_layout == TAMD_W_CDNA4_BLOCKS;
+  // eight lanes per column, whole lines where the column's piece lies inside one).  Where a stage is 128 K such a pair is copied
+  // every other stage: half lines passed the caches twice (3168 fp8 tokens x 8 over 16 experts, 3008 -> 1568, layer 433 us
+  // -> 423, with the halves' shared scale loads below 446 -> 433; 333 f16 tokens x 4 over 32, 2016 -> 1056, 79.2 -> 75.2; 16-bit
+  // stages of 256 K, which hold whole lines too, run blocks of 16 and 32 rows at 0.97 to 1.05 of the speed).
   const uint32_t w_nat = (uint32_t)(((t.n0 >> 6) + wave) * ((K + KB - 1) / KB)) * 4096u + (uint32_t)lane * 16;
   constexpr int WIDE = S::PAIRS ? 2 : BLOCKS;         // blocks of K that strided weights are copied by
   constexpr int W_LANES = 4 * WIDE;                   // lanes per column
@@ -307,7 +309,7 @@ TAMD_DEVICE void run_tile_mx(const tamd_matmul_args &a, const Tile &t, uint8_t *
   }
   wait_vmcnt<0>();
   // (the wave's own weight region is free by now: its table goes there)
-  tile_epilogue<NFR, ACT, X16 ? XDT : TAMD_BF16, !X16>(kernel_args_late(), t, acc, lds + 2 * A_STAGE + wave * B_WAVE);
+  tile_epilogue<NFR, ACT, X16 ? XDT : TAMD_BF16, !X16>(kernel_args_late(), t, acc, lds + b_at);
 }
 
 template <int XDT, int BM, int ACT>
@@ -343,7 +345,7 @@ int launch_mx(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
   group_m = group_m < 1 ? 1 : (group_m > 16 ? 16 : group_m);
   auto kern = mm_mx_kernel<XDT, BM, ACT>;
   if (int rc = raise_lds_limit_once((const void *)kern)) return rc;
-  kern<<<dim3((unsigned)launch), 256, MxShape<XDT, BM>::LDS, st>>>(a, grid_n, total, (int)(counts_live_blocks(a) ? -group_m : group_m));
+  kern<<<dim3((unsigned)launch), 256, (MxShape<XDT, BM>::lds(a.w_layout == TAMD_W_CDNA4_BLOCKS)), st>>>(a, grid_n, total, (int)(counts_live_blocks(a) ? -group_m : group_m));
   return launch_status();
 }
 
