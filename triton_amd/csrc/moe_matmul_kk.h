@@ -87,13 +87,13 @@ TAMD_DEVICE void run_tile_kk(const tamd_matmul_args &a, const Tile &t, uint8_t *
   const int rin = lane / 8;
   const int chunk = (lane % 8) ^ ((wave8 & 1) * 4 + (rin >> 1));
   constexpr int NA0 = (NFR + 1) / 2, NA1 = NFR / 2, NB = 4;   // copies per wave and stage: group 0, group 1; columns
-  uint32_t a_off[NA0], b_off[NB], row_idx[NA0];
-  // (the row indices are on their way while the first stage's columns are requested: 17 bf16 tokens x 2 over 64 experts,
-  // 576 -> 736, layer 35.0 us -> 34.0; 98 f16 x 4 over 8, 1216 -> 544, 34.5 -> 33.7; nothing where a tile lasts long)
-  if (a.gather_indx) {
-    const v4i_t rg = make_rsrc(a.gather_indx + t.start_m + t.off_m, (uint32_t)__builtin_amdgcn_readfirstlane(t.rows) * 4u);
+  uint32_t a_off[NA0], b_off[NB];
 #pragma unroll
-    for (int u = 0; u < NA0; ++u) row_idx[u] = request_dword(rg, (uint32_t)((wave8 + 8 * u) * 8 + rin) * 4u);
+  for (int u = 0; u < NA0; ++u) {
+    const int r = (wave8 + 8 * u) * 8 + rin;
+    const int rr = t.off_m + (r < t.rows ? r : t.rows - 1);
+    const uint32_t src = a.gather_indx ? (uint32_t)a.gather_indx[t.start_m + rr] : (uint32_t)(t.start_m + rr);
+    a_off[u] = r < t.rows ? src * (uint32_t)(a.x_stride_m * ESZ) + chunk * 16 : kOob;
   }
 #pragma unroll
   for (int u = 0; u < NB; ++u) {
@@ -101,34 +101,17 @@ TAMD_DEVICE void run_tile_kk(const tamd_matmul_args &a, const Tile &t, uint8_t *
     const int col = t.n0 + (p & ~63) + 2 * (p % 32) + (p % 64) / 32;
     b_off[u] = col < N ? (uint32_t)col * (uint32_t)(a.w_stride_n * ESZ) + chunk * 16 : kOob;
   }
-  auto issue_a = [&](int it, int slot) {   // (chunks past K are not read: zeros)
+  auto issue = [&](int it, int slot) {   // (chunks past K are not read: zeros)
     const int kb = it * KS;
     const uint32_t kill = kb + chunk * EPC < K ? 0u : kOob;
     const uint32_t sa = lds_base + slot * STAGE + wave8 * 1024;
 #pragma unroll
     for (int u = 0; u < NA0; ++u)
       if (u < NA1 || grp == 0) dma16(rx, sa + u * 8192, a_off[u] | kill, kb * ESZ);
-  };
-  auto issue_b = [&](int it, int slot) {
-    const int kb = it * KS;
-    const uint32_t kill = kb + chunk * EPC < K ? 0u : kOob;
-    const uint32_t sb = lds_base + slot * STAGE + wave8 * 1024 + LDS_ROWS * 128;
+    const uint32_t sb = sa + LDS_ROWS * 128;
 #pragma unroll
     for (int u = 0; u < NB; ++u) dma16(rw, sb + u * 8192, b_off[u] | kill, kb * ESZ);
   };
-  auto issue = [&](int it, int slot) {
-    issue_a(it, slot);
-    issue_b(it, slot);
-  };
-  issue_b(0, 0);
-  if (a.gather_indx) await_dwords<NB>(row_idx);
-#pragma unroll
-  for (int u = 0; u < NA0; ++u) {
-    const int r = (wave8 + 8 * u) * 8 + rin;
-    const uint32_t src = a.gather_indx ? row_idx[u] : (uint32_t)(t.start_m + t.off_m + r);
-    a_off[u] = r < t.rows ? src * (uint32_t)(a.x_stride_m * ESZ) + chunk * 16 : kOob;
-  }
-  issue_a(0, 0);
 
   f32x16_t acc[NFR][NF];
 #pragma unroll
@@ -145,7 +128,7 @@ TAMD_DEVICE void run_tile_kk(const tamd_matmul_args &a, const Tile &t, uint8_t *
   const int a_lane = c32 * 128, b_lane = LDS_ROWS * 128 + (wave * 64 + c32) * 128;
   const int n_k = (K + KS - 1) / KS;
 #pragma unroll
-  for (int s = 1; s < RING - 1; ++s) issue(s, s);
+  for (int s = 0; s < RING - 1; ++s) issue(s, s);
   int rd = 0, wr = RING - 1;
   for (int it = 0; it < n_k; ++it) {
     // copies complete in the order of their requests: all but those of the newest RING - 2 stages have landed
@@ -302,12 +285,13 @@ TAMD_DEVICE void run_tile_narrow(const tamd_matmul_args &a, const Tile &t, uint8
   // chunk s ^ ((r >> 1) & 7)
   const int rin = lane / 8;
   const int chunk[2] = {(lane % 8) ^ (rin >> 1), (lane % 8) ^ (4 + (rin >> 1))};   // even, odd copies
-  uint32_t a_off[NA], b_off[NB], row_idx[NA];
-  // (row indices ahead, as in run_tile_kk)
-  if (a.gather_indx) {
-    const v4i_t rg = make_rsrc(a.gather_indx + t.start_m + t.off_m, (uint32_t)__builtin_amdgcn_readfirstlane(t.rows) * 4u);
+  uint32_t a_off[NA], b_off[NB];
 #pragma unroll
-    for (int u = 0; u < NA; ++u) row_idx[u] = request_dword(rg, (uint32_t)(u * 8 + rin) * 4u);
+  for (int u = 0; u < NA; ++u) {
+    const int r = u * 8 + rin;
+    const int rr = t.off_m + (r < t.rows ? r : t.rows - 1);
+    const uint32_t src = a.gather_indx ? (uint32_t)a.gather_indx[t.start_m + rr] : (uint32_t)(t.start_m + rr);
+    a_off[u] = r < t.rows ? src * (uint32_t)(a.x_stride_m * ESZ) + chunk[u & 1] * 16 : kOob;
   }
 #pragma unroll
   for (int u = 0; u < NB; ++u) {
@@ -315,31 +299,15 @@ TAMD_DEVICE void run_tile_narrow(const tamd_matmul_args &a, const Tile &t, uint8
     const int col = t.n0 + 2 * (p % 32) + p / 32;
     b_off[u] = col < N ? (uint32_t)col * (uint32_t)(a.w_stride_n * ESZ) + chunk[u & 1] * 16 : kOob;
   }
-  auto issue_a = [&](int it, int slot) {   // (chunks past K, and stages past the wave's own, are not read: zeros)
+  auto issue = [&](int it, int slot) {   // (chunks past K, and stages past the wave's own, are not read: zeros)
     const int kb = (first + it) * KS;
     const uint32_t kill[2] = {it < n_w && kb + chunk[0] * EPC < K ? 0u : kOob, it < n_w && kb + chunk[1] * EPC < K ? 0u : kOob};
+    const uint32_t sa = ring_base + slot * STAGE, sb = sa + S::A_LINES * 128;
 #pragma unroll
-    for (int u = 0; u < NA; ++u) dma16(rx, ring_base + slot * STAGE + u * 1024, a_off[u] | kill[u & 1], kb * ESZ);
-  };
-  auto issue_b = [&](int it, int slot) {
-    const int kb = (first + it) * KS;
-    const uint32_t kill[2] = {it < n_w && kb + chunk[0] * EPC < K ? 0u : kOob, it < n_w && kb + chunk[1] * EPC < K ? 0u : kOob};
+    for (int u = 0; u < NA; ++u) dma16(rx, sa + u * 1024, a_off[u] | kill[u & 1], kb * ESZ);
 #pragma unroll
-    for (int u = 0; u < NB; ++u) dma16(rw, ring_base + slot * STAGE + (S::A_LINES + u * 8) * 128, b_off[u] | kill[u & 1], kb * ESZ);
+    for (int u = 0; u < NB; ++u) dma16(rw, sb + u * 1024, b_off[u] | kill[u & 1], kb * ESZ);
   };
-  auto issue = [&](int it, int slot) {
-    issue_a(it, slot);
-    issue_b(it, slot);
-  };
-  issue_b(0, 0);
-  if (a.gather_indx) await_dwords<NB>(row_idx);
-#pragma unroll
-  for (int u = 0; u < NA; ++u) {
-    const int r = u * 8 + rin;
-    const uint32_t src = a.gather_indx ? row_idx[u] : (uint32_t)(t.start_m + t.off_m + r);
-    a_off[u] = r < t.rows ? src * (uint32_t)(a.x_stride_m * ESZ) + chunk[u & 1] * 16 : kOob;
-  }
-  issue_a(0, 0);
   f32x16_t acc[1][NF];
 #pragma unroll
   for (int f = 0; f < NF; ++f)
@@ -349,7 +317,7 @@ TAMD_DEVICE void run_tile_narrow(const tamd_matmul_args &a, const Tile &t, uint8
   const int a_line = c32 & (S::A_LINES - 1), a_swz = (a_line >> 1) & 7, b_swz = (c32 >> 1) & 7;
   const int a_lane = a_line * 128, b_lane = (S::A_LINES + c32) * 128;
 #pragma unroll
-  for (int s = 1; s < RING - 1; ++s) issue(s, s);
+  for (int s = 0; s < RING - 1; ++s) issue(s, s);
   int rd = 0, wr = RING - 1;
 #pragma unroll 1
   for (int it = 0; it < n_w; ++it) {
