@@ -249,6 +249,13 @@ TAMD_DEVICE bool locate_tile_live(const tamd_matmul_args &a, int grid_n, int gro
   return true;
 }
 
+// What a row of x is below: the rows that a gathered index can name.  An index outside of them (-1) names none: the row is read as
+// zeros, by the buffer descriptors where the address leaves their 2 GB, and by this limit where loads have no descriptor.
+TAMD_DEVICE uint32_t gather_limit(const tamd_matmul_args &a) {
+  const int64_t rows = a.x_rows > 0 ? a.x_rows : (int64_t)a.M;
+  return a.gather_indx && rows < 0x80000000ll ? (uint32_t)rows : 0x80000000u;
+}
+
 // 128-bit global -> LDS copy that bypasses registers (buffer_load ... lds).  The LDS destination of
 // lane L is lds_addr + 16*L; out-of-range offsets (>= num_records of the descriptor) deliver zeros.
 // Issued through inline asm so that the compiler does not serialise later LDS reads behind it; the

@@ -146,6 +146,9 @@ TAMD_DEVICE void run_tile_mx(const tamd_matmul_args &a, const Tile &t, uint8_t *
     // a load touches a line per lane, so each half of the wave loads one of its lanes' two columns and the halves exchange them
     ws_off[0] = ws_off[1] = (uint32_t)(col0 + h < N ? col0 + h : N - 1) * (uint32_t)a.w_mx_stride_n;
   }
+  // rows that a gathered index can name (ordinary loads have no descriptor that would end with them), and the offset of one it cannot
+  const uint32_t x_rows = gather_limit(a);
+  constexpr uint32_t kNoRow = 0xFFFFFFFFu;
   const int g_last = G > 8 ? G - 8 : 0;               // where the last eight bytes start
   uint64_t as_raw[NFR], ws_raw[NF];
 #pragma unroll
@@ -156,7 +159,7 @@ TAMD_DEVICE void run_tile_mx(const tamd_matmul_args &a, const Tile &t, uint8_t *
     const int at = 8 * e < g_last ? 8 * e : g_last;
     if (x_mx) {
 #pragma unroll
-      for (int i = 0; i < NFR; ++i) as_raw[i] = load_scales(xs_base + at, as_off[i], G);
+      for (int i = 0; i < NFR; ++i) as_raw[i] = load_scales(xs_base + at, as_off[i] == kNoRow ? 0u : as_off[i], G);
     }
     const uint8_t *w = ws_base + (cdna4 ? 256 * e : at);
     ws_raw[0] = load_scales(w, ws_off[0], cdna4 ? 8 : G);
@@ -171,7 +174,7 @@ TAMD_DEVICE void run_tile_mx(const tamd_matmul_args &a, const Tile &t, uint8_t *
       return __builtin_amdgcn_perm((uint32_t)(x >> 32), (uint32_t)x, sel);
     };
 #pragma unroll
-    for (int i = 0; i < NFR; ++i) sa[i] = x_mx ? pick(as_raw[i]) : 0x7F7F7F7Fu;
+    for (int i = 0; i < NFR; ++i) sa[i] = x_mx ? (as_off[i] == kNoRow ? 0u : pick(as_raw[i])) : 0x7F7F7F7Fu;
     if (cdna4) {
       const uint32_t s2 = 0x06020400u + (uint32_t)half * 0x01010101u;
 #pragma unroll
@@ -219,9 +222,10 @@ TAMD_DEVICE void run_tile_mx(const tamd_matmul_args &a, const Tile &t, uint8_t *
     const int r = i * 32 + a_rin, rs = i * 32 + c32, row0 = t.start_m + t.off_m;
     const uint32_t src = a.gather_indx ? row_idx[i] : (uint32_t)(row0 + r);
     const uint32_t srs = a.gather_indx ? row_idx[X16 ? i : NFR + i] : (uint32_t)(row0 + (rs < t.rows ? rs : t.rows - 1));
-    // rows past the end of the slice are never stored: they are copied as zeros, which keeps the matrix cores' inputs quiet
-    a_off[i] = r < t.rows ? src * (uint32_t)(a.x_stride_m * S::ESZ) + a_chunk * 16 : kOob;
-    as_off[i] = srs * (uint32_t)a.x_mx_stride_m;
+    // rows past the end of the slice are never stored: they are copied as zeros, which keeps the matrix cores' inputs quiet; so
+    // is the row of an index that names none (-1), whose scales are not read
+    a_off[i] = r < t.rows && src < x_rows ? src * (uint32_t)(a.x_stride_m * S::ESZ) + a_chunk * 16 : kOob;
+    as_off[i] = srs < x_rows ? srs * (uint32_t)a.x_mx_stride_m : kNoRow;
   }
   issue_a(0);
   load_sc(0);

@@ -450,13 +450,15 @@ __global__ __launch_bounds__((NCW + NC + 2) * 64, 1) void mm_stream16_kernel(tam
       int rc = c16 < cb.rows ? c16 : cb.rows - 1;
       rc = cb.row0 + (rc < 0 ? 0 : rc);
       const int64_t src = a.gather_indx ? (int64_t)a.gather_indx[rc] : (int64_t)rc;
+      // (an index that names no row, -1: zeros, as the tiled kernels read them past the end of a descriptor)
+      const bool have = cb.rows > 0 && (uint64_t)src < gather_limit(a);
       if constexpr (A8) {
         const uint8_t *xr = (const uint8_t *)a.x + (int64_t)cb.z * a.x_stride_z + src * a.x_stride_m;
         const uint8_t *xs = a.x_mx_scale ? a.x_mx_scale + (int64_t)cb.z * a.x_mx_stride_z + src * a.x_mx_stride_m : nullptr;
 #pragma unroll
         for (int j = 0; j < SS; ++j) {
           const int kg = kb + 4 * j + g;
-          const bool live = kg < G && cb.rows > 0;
+          const bool live = kg < G && have;
           // 2^(e - 127) as the scaled MFMA of the tiled kernels reads it: 0 is 2^-127, 0xFF NaN
           const uint32_t e = (live && xs) ? (uint32_t)xs[kg] : 127u;
           const float mult = bits_to_f32(e == 0u ? 0x00400000u : (e == 255u ? 0x7FC00000u : e << 23));
@@ -492,7 +494,7 @@ __global__ __launch_bounds__((NCW + NC + 2) * 64, 1) void mm_stream16_kernel(tam
 #pragma unroll
           for (int u = 0; u < 4; ++u) {
             uint4 v = make_uint4(0, 0, 0, 0);
-            if (kg < G && cb.rows > 0) v = *(const uint4 *)(xr + 32 * kg + 8 * u);
+            if (kg < G && have) v = *(const uint4 *)(xr + 32 * kg + 8 * u);
             areg[j * 4 + u] = __builtin_bit_cast(frag_t, v);
           }
         }
