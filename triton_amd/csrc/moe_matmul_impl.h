@@ -310,21 +310,6 @@ TAMD_DEVICE void wait_vmcnt() {
   asm volatile("" ::: "memory");
 }
 
-// A dword from memory into a register, requested through inline asm as well: the compiler would wait for an ordinary load with a
-// count that takes in the LDS copies requested after it, which it does not see.  `v` must not be touched before
-// await_dwords<N>, which waits until at most the N newest requests of the wave are outstanding.
-TAMD_DEVICE uint32_t request_dword(v4i_t rsrc, uint32_t voff) {
-  uint32_t v;
-  asm volatile("s_nop 4\n\tbuffer_load_dword %0, %1, %2, 0 offen" : "=v"(v) : "v"(voff), "s"(rsrc) : "memory");
-  return v;
-}
-template <int N, int COUNT>
-TAMD_DEVICE void await_dwords(uint32_t (&v)[COUNT]) {
-  asm volatile("s_waitcnt vmcnt(%1)" : "+v"(v[0]) : "n"(N) : "memory");
-#pragma unroll
-  for (int i = 1; i < COUNT; ++i) asm volatile("" : "+v"(v[i]));
-}
-
 TAMD_DEVICE v4i_t make_rsrc(const void *base, uint32_t num_records) {
   uint64_t p = (uint64_t)base;
   return v4i_t{__builtin_amdgcn_readfirstlane((int)(uint32_t)p),
@@ -923,17 +908,23 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
   uint32_t a_off[NFR];
   const int row0 = t.start_m + t.off_m;
   auto row_off = [&](int r, uint32_t src) { return r < t.rows ? src * (uint32_t)(a.x_stride_m * ESZ) + a_chunk * 16 : kOob; };
-  // The rows' indices are the first thing requested, and the first weights, which do not depend on them, while they come.
-  uint32_t row_idx[NFR];
+  // The rows' indices are the first thing requested, and the first weights, which do not depend on them, while they come.  They
+  // travel by LDS, each in front of the row pieces that the wave will copy there (an ordinary load would be waited for with a count
+  // that takes in the copies requested after it, which the compiler does not see).
   const v4i_t rg = make_rsrc(a.gather_indx + row0, (uint32_t)__builtin_amdgcn_readfirstlane(t.rows) * 4u);
+  const int idx_at = wave * 8 * A_ROW_BYTES;
   if (a.gather_indx) {
 #pragma unroll
-    for (int i = 0; i < NFR; ++i) row_idx[i] = request_dword(rg, (uint32_t)(i * 32 + a_rin) * 4u);
+    for (int i = 0; i < NFR; ++i) dma4(rg, lds_base + idx_at + i * 32 * A_ROW_BYTES, (uint32_t)(i * 32 + a_rin) * 4u, 0);
   }
   auto rows_known = [&](auto newer) {   // (after `newer` further requests of the wave)
-    if (a.gather_indx) await_dwords<decltype(newer)::value>(row_idx);
+    if (a.gather_indx) wait_vmcnt<decltype(newer)::value>();
 #pragma unroll
-    for (int i = 0; i < NFR; ++i) a_off[i] = row_off(i * 32 + a_rin, a.gather_indx ? row_idx[i] : (uint32_t)(row0 + i * 32 + a_rin));
+    for (int i = 0; i < NFR; ++i) {
+      const int at = idx_at + i * 32 * A_ROW_BYTES + lane * 4;
+      a_off[i] = row_off(i * 32 + a_rin, a.gather_indx ? *(const uint32_t *)(lds + at) : (uint32_t)(row0 + i * 32 + a_rin));
+    }
+    if (a.gather_indx) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // read before the rows are copied over them
   };
   // ---- weight DMA: instruction j copies LDS positions j*16 + lane/4, part slot lane%4
   // Codes in the block layout (TAMD_W_CDNA4_BLOCKS): a stage of this wave's strip is one 4 KB block that already has

@@ -88,17 +88,19 @@ TAMD_DEVICE void run_tile_mx(const tamd_matmul_args &a, const Tile &t, uint8_t *
   const int n_k = (K + KA - 1) / KA;
   const bool x_mx = FP4 || (XDT == TAMD_FP8_E4M3 && a.x_mx_scale != nullptr);
 
-  // ---- row indices: of the rows whose values the lane copies, and of the rows whose scales its MFMAs use
+  // ---- row indices: of the rows whose values the lane copies, and of the rows whose scales its MFMAs use; by LDS, each in front of
+  // the row pieces that the wave will copy there (see run_tile)
   const int a_rin = wave * 8 + lane / 8;
   const int a_chunk = (lane % 8) ^ ((a_rin >> 1) & 7);
-  uint32_t row_idx[X16 ? NFR : 2 * NFR];
+  const int idx_at = wave * 8 * A_ROW_BYTES;
   if (a.gather_indx) {
     const v4i_t rg = make_rsrc(a.gather_indx + t.start_m + t.off_m, (uint32_t)__builtin_amdgcn_readfirstlane(t.rows) * 4u);
 #pragma unroll
     for (int i = 0; i < NFR; ++i) {
       const int rs = i * 32 + c32;
-      row_idx[i] = request_dword(rg, (uint32_t)(i * 32 + a_rin) * 4u);
-      if constexpr (!X16) row_idx[NFR + i] = request_dword(rg, (uint32_t)(rs < t.rows ? rs : t.rows - 1) * 4u);
+      const uint32_t to = lds_base + idx_at + i * 32 * A_ROW_BYTES;
+      dma4(rg, to, (uint32_t)(i * 32 + a_rin) * 4u, 0);
+      if constexpr (!X16) dma4(rg, to + 4 * kWave, (uint32_t)(rs < t.rows ? rs : t.rows - 1) * 4u, 0);
     }
   }
 
@@ -216,17 +218,19 @@ TAMD_DEVICE void run_tile_mx(const tamd_matmul_args &a, const Tile &t, uint8_t *
   };
 
   issue_b(0);
-  if (a.gather_indx) await_dwords<4 * BLOCKS>(row_idx);
+  if (a.gather_indx) wait_vmcnt<4 * BLOCKS>();   // (the copies of the weights may be outstanding)
 #pragma unroll
   for (int i = 0; i < NFR; ++i) {
     const int r = i * 32 + a_rin, rs = i * 32 + c32, row0 = t.start_m + t.off_m;
-    const uint32_t src = a.gather_indx ? row_idx[i] : (uint32_t)(row0 + r);
-    const uint32_t srs = a.gather_indx ? row_idx[X16 ? i : NFR + i] : (uint32_t)(row0 + (rs < t.rows ? rs : t.rows - 1));
+    const uint32_t *idx = (const uint32_t *)(lds + idx_at + i * 32 * A_ROW_BYTES) + lane;
+    const uint32_t src = a.gather_indx ? idx[0] : (uint32_t)(row0 + r);
+    const uint32_t srs = a.gather_indx ? idx[X16 ? 0 : kWave] : (uint32_t)(row0 + (rs < t.rows ? rs : t.rows - 1));
     // rows past the end of the slice are never stored: they are copied as zeros, which keeps the matrix cores' inputs quiet; so
     // is the row of an index that names none (-1), whose scales are not read
     a_off[i] = r < t.rows && src < x_rows ? src * (uint32_t)(a.x_stride_m * S::ESZ) + a_chunk * 16 : kOob;
     as_off[i] = srs < x_rows ? srs * (uint32_t)a.x_mx_stride_m : kNoRow;
   }
+  if (a.gather_indx) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // read before the rows are copied over them
   issue_a(0);
   load_sc(0);
   const int swz = (c32 >> 1) & 7;
