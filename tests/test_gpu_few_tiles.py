@@ -1,6 +1,6 @@
 """GPU: ragged products of few tiles, whose row blocks are smaller than the slices' sizes ask for (or, for fp8 rows, the streaming
-kernel's): around the lines of the rule, against float32 products of the same values; special block scales of fp8 rows, which give
-the same on both kernels that take them."""
+kernel's): around the lines of the rule, against float32 products of the same values; block scales over their whole range, which only
+the scaled MFMA takes, whatever the number of tiles; the weight scales that the streaming kernel holds exactly."""
 import pytest
 import torch
 
@@ -46,7 +46,7 @@ def test_few_tiles(rows, E, N, kind, K, device):
 
 @pytest.mark.parametrize("byte", [0, 1, 238, 255])
 def test_special_block_scales(byte, device):
-    """A row's scale bytes at the ends of what bf16 holds of the values: the streaming kernel and the tiled one agree (NaN for 255)."""
+    """Scale bytes of a row: blocks of 16 and of 32 rows agree (NaN for 255)."""
     torch.manual_seed(0)
     K, N = 640, 256
     a, s = downcast_to_mxfp(torch.randn(4, K, device=device), torch.float8_e4m3fn, axis=-1)
@@ -63,6 +63,50 @@ def test_special_block_scales(byte, device):
             out.append(matmul(a, w, None, md, precision_config=pc))
     assert torch.equal(out[0].isnan(), out[1].isnan()) and bool(out[0][2].isnan().all()) == (byte == 255)
     torch.testing.assert_close(out[0], out[1], rtol=1e-3, atol=1e-3, equal_nan=True)
+
+
+def scaled_sums(x8, xs, codes, ws):
+    """The product in 64 bits: values and e8m0 bytes [M, K], [M, K/32] against [K, N], [K/32, N]."""
+    two = torch.tensor(2.0, dtype=torch.float64)
+    x = x8.double().cpu() * (two ** (xs.double().cpu() - 127)).repeat_interleave(32, dim=1)
+    return x @ (codes.double().cpu() * (two ** (ws.double().cpu() - 127)).repeat_interleave(32, dim=0))
+
+
+@pytest.mark.parametrize("ragged", [True, False])
+@pytest.mark.parametrize("byte,shift", [(2, 100), (119, 0), (247, -100), (254, -100)])
+def test_block_scales_of_the_whole_range(byte, shift, ragged, device):
+    """Few tiles of rows with block scales that bf16 does not hold the scaled values of: the sums are those of the whole range."""
+    torch.manual_seed(byte)
+    M, K, N = 4, 640, 256
+    a, s = downcast_to_mxfp(torch.randn(M, K, device=device), torch.float8_e4m3fn, axis=-1)
+    s = (s.int() - s.int().max(dim=1, keepdim=True).values + byte).clamp(0, 254).to(torch.uint8)
+    w, _ = downcast_to_mxfp(torch.randn(1, K, N, device=device), torch.uint8, axis=1)
+    ws = torch.randint(120 + shift, 128 + shift, (1, N, K // 32), dtype=torch.uint8, device=device).transpose(1, 2)
+    codes = upcast_from_mxfp(w, torch.full_like(ws, 127), torch.float32, axis=1)
+    pc = PrecisionConfig(a_mx_scale=s, a_microblock_size=32, b_mx_scale=ws if ragged else ws[0], b_microblock_size=32, out_dtype=torch.float32)
+    md = make_ragged_tensor_metadata(torch.tensor([M], dtype=torch.int32, device=device), M) if ragged else None
+    y = matmul(a, w if ragged else w[0], None, md, precision_config=pc).double().cpu()
+    ref = scaled_sums(a, s, codes[0], ws[0])
+    # (the scaled MFMA's sums are off by up to 6e-5 of the result; values that bf16 loses are at least 2^-9 of it)
+    assert float((y - ref).norm() / ref.norm()) <= 2.0 ** -13
+
+
+@pytest.mark.parametrize("byte", [0, 1, 127, 252])
+@pytest.mark.parametrize("block_m", [16, 32])
+def test_weight_scales_that_16_bit_operands_hold(byte, block_m, device):
+    """fp8 rows without block scales: weights of scale bytes up to 252 (6 * 2^125 is a bf16 number) are exact in the streaming kernel
+    (blocks of 16) as in the scaled MFMA; 0 stands for 2^-127."""
+    torch.manual_seed(byte)
+    M, K, N = 4, 640, 256
+    a = (torch.randn(M, K, device=device) * (2.0 ** -6 if byte > 200 else 8.0)).to(torch.float8_e4m3fn)
+    w, _ = downcast_to_mxfp(torch.randn(1, K, N, device=device), torch.uint8, axis=1)
+    ws = torch.full((1, N, K // 32), byte, dtype=torch.uint8, device=device).transpose(1, 2)
+    codes = upcast_from_mxfp(w, torch.full_like(ws, 127), torch.float32, axis=1)
+    md = make_ragged_tensor_metadata(torch.tensor([M], dtype=torch.int32, device=device), M)
+    with scoped_opt_flags_constraints({"block_m": block_m}):
+        y = matmul(a, w, None, md, precision_config=PrecisionConfig(b_mx_scale=ws, b_microblock_size=32, out_dtype=torch.float32))
+    ref = scaled_sums(a, torch.full((M, K // 32), 127, dtype=torch.uint8), codes[0], ws[0])
+    assert float((y.double().cpu() - ref).norm() / ref.norm()) <= 2.0 ** -13
 
 
 def test_microscaled_output_keeps_its_kernel(device):

@@ -1009,8 +1009,8 @@ def test_mxfp8_output_ragged_then_mxfp8_input(block_m, device):
 @pytest.mark.parametrize("mx", [False, True, "e5m2"])
 @pytest.mark.parametrize("act", [False, True])
 def test_decode_row_blocks_of_16_fp8_rows(K, mx, act, device):
-    """The streaming kernel with fp8 rows (e4m3 with a per-tensor flex scale or MXFP8 block scales; e5m2 with a flex scale), expanded to bf16
-    as a row block is loaded; gather, scatter with dropped rows, gate weights."""
+    """Row blocks of 16 fp8 rows: the streaming kernel (e4m3 or e5m2 with a per-tensor flex scale, expanded to bf16 as a row block is
+    loaded) and, with MXFP8 block scales, the scaled MFMA; gather, scatter with dropped rows, gate weights."""
     torch.manual_seed(K)
     E, N = 7, 608
     sizes = torch.tensor([3, 0, 1, 16, 5, 21, 2], dtype=torch.int32)

@@ -440,7 +440,7 @@ PyObject *py_matmul(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
       need(n_slices > 0 && n_slices <= n_mat && (!g.bias || tensor(bias_o).dim() == 2));
       const int64_t expected = ex.none() ? -1 : as_int(ex.p);
       const int bm = tiles_block_m(choose_block_m(M, n_slices, true, expected, (a8 || a4) && w_fp4), M, N, K, n_slices, expected,
-                                       w_fp4, a8, mx_out || a4);
+                                       w_fp4, a8, mx_out || a_mx);
       const int row = bm == 16 ? 0 : bm == 32 ? 1 : bm == 64 ? 2 : 3;
       g.slice_sizes = (const int32_t *)tss.data_ptr(), g.slice_offs = (const int32_t *)tso.data_ptr();
       g.block_offs = (const int32_t *)tbo.data_ptr() + row * tbo.stride(0);

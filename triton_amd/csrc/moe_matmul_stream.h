@@ -92,9 +92,8 @@ struct StreamShape {
 // NCW: compute waves (4 or 8) that split K between them.  The same kernel without its conversions and MFMAs runs the
 // decode shape in 144 instead of 159 us; eight waves halve each wave's part of a unit but were slower in all (171 us:
 // fourteen waves at the unit's barrier, eight partial sums to add), and the launcher uses four.
-// A8 (1: float8_e4m3fn, 2: float8_e5m2; 0: rows of XDT): the activations are stored as fp8 (optionally with e8m0 block
-// scales per 32 K) and are expanded to
-// XDT when a row block's slice is loaded into registers -- exact, so the K loop is the same as for 16-bit rows.
+// A8 (1: float8_e4m3fn, 2: float8_e5m2; 0: rows of XDT): the activations are stored as fp8 and are expanded to XDT when a row
+// block's slice is loaded into registers -- exact, so the K loop is the same as for 16-bit rows.
 // NC: copying waves (2 or 4).  A 1 KB copy holds the wave that issues it for about 110 cycles, so two copying waves
 // move at most 18 bytes per cycle and CU and, with the K of the decode shape (24 pieces of codes per unit), spend
 // most of a unit issuing; four take a quarter of a unit's pieces each (decode shape: 161 -> 158 us).
@@ -454,29 +453,25 @@ __global__ __launch_bounds__((NCW + NC + 2) * 64, 1) void mm_stream16_kernel(tam
       const bool have = cb.rows > 0 && (uint64_t)src < gather_limit(a);
       if constexpr (A8) {
         const uint8_t *xr = (const uint8_t *)a.x + (int64_t)cb.z * a.x_stride_z + src * a.x_stride_m;
-        const uint8_t *xs = a.x_mx_scale ? a.x_mx_scale + (int64_t)cb.z * a.x_mx_stride_z + src * a.x_mx_stride_m : nullptr;
 #pragma unroll
         for (int j = 0; j < SS; ++j) {
           const int kg = kb + 4 * j + g;
           const bool live = kg < G && have;
-          // 2^(e - 127) as the scaled MFMA of the tiled kernels reads it: 0 is 2^-127, 0xFF NaN
-          const uint32_t e = (live && xs) ? (uint32_t)xs[kg] : 127u;
-          const float mult = bits_to_f32(e == 0u ? 0x00400000u : (e == 255u ? 0x7FC00000u : e << 23));
 #pragma unroll
           for (int u = 0; u < 4; ++u) {
             uint2 v = make_uint2(0, 0);
             if (live) v = *(const uint2 *)(xr + 32 * kg + 8 * u);
             float f[8];
-            f[0] = fp8_byte<A8, 0>(v.x) * mult;
-            f[1] = fp8_byte<A8, 1>(v.x) * mult;
-            f[2] = fp8_byte<A8, 2>(v.x) * mult;
-            f[3] = fp8_byte<A8, 3>(v.x) * mult;
-            f[4] = fp8_byte<A8, 0>(v.y) * mult;
-            f[5] = fp8_byte<A8, 1>(v.y) * mult;
-            f[6] = fp8_byte<A8, 2>(v.y) * mult;
-            f[7] = fp8_byte<A8, 3>(v.y) * mult;
-            // packed by hand, two values per register: an fp8 value times a power of two has at most four significant
-            // bits, so the upper half of its float32 pattern is its bf16 pattern
+            f[0] = fp8_byte<A8, 0>(v.x);
+            f[1] = fp8_byte<A8, 1>(v.x);
+            f[2] = fp8_byte<A8, 2>(v.x);
+            f[3] = fp8_byte<A8, 3>(v.x);
+            f[4] = fp8_byte<A8, 0>(v.y);
+            f[5] = fp8_byte<A8, 1>(v.y);
+            f[6] = fp8_byte<A8, 2>(v.y);
+            f[7] = fp8_byte<A8, 3>(v.y);
+            // packed by hand, two values per register: an fp8 value has at most four significant bits, so the upper half of its
+            // float32 pattern is its bf16 pattern
             uint32_t w[4];
 #pragma unroll
             for (int p = 0; p < 4; ++p) {
@@ -554,13 +549,15 @@ __global__ __launch_bounds__((NCW + NC + 2) * 64, 1) void mm_stream16_kernel(tam
   }
 }
 
-// Whether the streaming kernel covers the problem: K contiguous and dense per column for codes and
+// Whether the streaming kernel covers the problem: rows without block scales (bf16 does not hold value times scale over the range that
+// the scaled MFMA takes: scales of 2^119 and above overflow, values below 2^-133 vanish), K contiguous and dense per column for codes and
 // scales, 16-byte aligned column groups, N a multiple of 16, K <= 4096, whole tensors addressable
 // with 32-bit offsets.
 inline bool stream16_applicable(const tamd_matmul_args &a) {
   const int64_t lim = 0x7FFFFF00;
   const int64_t G = a.K / 32;
   if (a.K > 4096 || a.K % 32 != 0) return false;
+  if (a.x_mx_scale) return false;
   const bool cdna4 = a.w_mx_layout == TAMD_SCALE_CDNA4;
   const bool wnat = a.w_layout == TAMD_W_CDNA4_BLOCKS;
   if (!wnat && (a.w_stride_k != 1 || a.w_stride_n != a.K / 2)) return false;

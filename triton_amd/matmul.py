@@ -355,7 +355,7 @@ def matmul(a, b, bias, a_ragged_metadata: Optional[RaggedTensorMetadata] = None,
                            fp8_rows=(a_packed or a.dtype in fp8_types) and b_fp4)
     if ragged and _opt_flags._opt_flags.get() is None and _opt_flags._constraints().get("block_m") is None:
         flags.block_m = _opt_flags.tiles_block_m(flags.block_m, M, N, K, n_slices, a_ragged_metadata.expected_slice_size,
-                                                     b_fp4, a.dtype in fp8_types, mx_out or a_packed)
+                                                     b_fp4, a.dtype in fp8_types, mx_out or a_mx_scale is not None)
     args = _lib.MatmulArgBag()
     args.x, args.x_dtype = a.data_ptr(), _lib.MXFP4 if a_packed else _lib.dtype_code(a.dtype)
     args.x_stride_m = a.stride(-2)

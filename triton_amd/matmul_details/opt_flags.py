@@ -93,8 +93,8 @@ def tiles_block_m(block_m: int, m: int, n: int, k: int, n_slices: int, expected_
     Tiles that leave CUs idle: a tile of half the rows takes about half the time per K stage, so smaller blocks win until
     the CUs are taken, although they read a slice's weights more often; at 80 tiles of 128 rows (16 slices of 128 rows,
     3776 x 1280) 83 us against 38.  Few rows per slice and few tiles: the weight-streaming kernel (blocks of 16, units of
-    16 columns), also for fp8 rows (10 to 40 % up to 80 tiles; not with two blocks per slice, and not below K 640, where
-    a unit is too short).  Few rows and many tiles of a short K (up to 1152, where a unit's barrier and start weigh
+    16 columns), also for fp8 rows without block scales (10 to 40 % up to 80 tiles; not with two blocks per slice, and not
+    below K 640, where a unit is too short).  Few rows and many tiles of a short K (up to 1152, where a unit's barrier and start weigh
     more than its copies): the tiled kernel instead of the streaming one (20 to 50 %).
     The lines are those that gave the shortest mean time over 700 layers of 1 to 4000 tokens, 8 to 128 experts, K 512
     to 5760."""
