@@ -109,6 +109,47 @@ def test_weight_scales_that_16_bit_operands_hold(byte, block_m, device):
     assert float((y.double().cpu() - ref).norm() / ref.norm()) <= 2.0 ** -13
 
 
+@pytest.mark.parametrize("form,block_m", [("dense", 16), ("padded codes", 32), ("padded scales", 32), ("odd start", 32)])
+def test_blocks_of_16_only_where_they_stream(form, block_m, device):
+    """Weights that the streaming kernel does not read run in blocks of 32 rows, one pass over them, with the same results."""
+    torch.manual_seed(3)
+    E, K, N = 3, 1280, 256
+    sizes = torch.tensor([20, 18, 22], dtype=torch.int32)
+    M = int(sizes.sum())
+    x = torch.randn(M, K, device=device).bfloat16()
+    w, ws = downcast_to_mxfp(torch.randn(E, K, N, device=device) * 0.1, torch.uint8, axis=1)
+    wf = upcast_from_mxfp(w, ws, torch.float32, axis=1)
+
+    def pitched(t, pitch, start=0):   # the same values, [E, N, pitch] in memory
+        room = torch.zeros(start + E * N * pitch, dtype=torch.uint8, device=device)
+        view = room[start:].view(E, N, pitch)[..., :t.shape[1]]
+        view.copy_(t.transpose(1, 2))
+        return view.transpose(1, 2)
+
+    if form == "padded codes":
+        w = pitched(w, K // 2 + 16)
+    elif form != "dense":
+        ws = pitched(ws, K // 32 + (8 if form == "padded scales" else 0), 4 if form == "odd start" else 0)
+    md = make_ragged_tensor_metadata(sizes.to(device), M)
+    asked = []
+
+    class Seen(type(md)):
+        def block_schedule(self, size):
+            asked.append(size)
+            return super().block_schedule(size)
+
+    seen = Seen(**{f: getattr(md, f) for f in md.__dataclass_fields__})
+    pc = PrecisionConfig(b_mx_scale=ws, b_microblock_size=32)
+    with scoped_opt_flags_constraints({"split_k": 1}):       # (a constraint: the general host path)
+        y = matmul(x, w, None, seen, precision_config=pc)
+    assert set(asked) == {block_m}
+    assert torch.equal(y, matmul(x, w, None, md, precision_config=pc))
+    for e, (rows, got) in enumerate(zip(x.float().split(sizes.tolist()), y.float().split(sizes.tolist()))):
+        ref = rows @ wf[e]
+        # a 16-bit result (2^-8) of K float32 additions
+        assert bool(((got - ref).abs() <= 2.0 ** -8 * ref.abs() + K * 2.0 ** -23 * (rows.abs() @ wf[e].abs()) + 1e-6).all()), e
+
+
 def test_microscaled_output_keeps_its_kernel(device):
     torch.manual_seed(1)
     K, N, M = 640, 256, 12

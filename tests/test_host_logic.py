@@ -247,3 +247,36 @@ def test_tiles_block_m_is_one_rule():
                                 if n % 16 == 0:
                                     assert want >= last
                                     last = want
+
+
+def test_blocks_of_16_only_where_they_stream():
+    """MXFP4 weights: the streaming kernel's conditions on the arguments, and no row block of 16 where one of them fails."""
+    import ctypes
+    from triton_amd import _lib, _native
+    E, K, N, G = 3, 1280, 512, 40
+    plain = dict(x=1 << 20, w=2 << 20, w_mx_scale=3 << 20, x_dtype=_lib.BF16, w_dtype=_lib.MXFP4, M=60, K=K, N=N, n_experts=E,
+                 w_stride_e=K // 2 * N, w_stride_k=1, w_stride_n=K // 2, w_mx_stride_e=G * N, w_mx_stride_k=1, w_mx_stride_n=G,
+                 block_offs=4 << 20, block_schedule=5 << 20)
+
+    def streams(**changed):
+        bag = _lib.MatmulArgBag()
+        for name, value in {**plain, **changed}.items():
+            setattr(bag, name, value)
+        packed = bag.pack()
+        return _native.blocks_of_16_stream(ctypes.addressof(packed))
+
+    assert streams() is True
+    assert streams(n_experts=1, w_stride_e=7, w_mx_stride_e=7) is True       # (the pitch of one matrix is never used)
+    for changed in (dict(w_stride_n=K // 2 + 16), dict(w_mx_stride_n=G + 8), dict(w=(2 << 20) + 8), dict(w_mx_scale=(3 << 20) + 4),
+                    dict(w_stride_e=K // 2 * N + 8), dict(w_mx_stride_e=G * N + 4), dict(w_stride_e=1 << 30), dict(N=N - 8),
+                    dict(K=4128, w_stride_n=2064, w_mx_stride_n=129), dict(x_mx_scale=6 << 20), dict(y_mx_scale=6 << 20),
+                    dict(x_dtype=_lib.MXFP4, x_mx_scale=6 << 20), dict(w_dtype=_lib.BF16)):
+        assert streams(**changed) is False, changed
+    assert streams(w_layout=_lib.W_CDNA4_BLOCKS, w_stride_n=0, w_mx_layout=_lib.SCALE_CDNA4, w_mx_stride_n=0, w_mx_stride_k=0) is True
+    for base in (16, 32, 64, 128):
+        for fp8 in (False, True):
+            for m, slices in ((2, 1), (60, 3), (2000, 128)):
+                for n in (16, 512, 5760):
+                    assert OF.tiles_block_m(base, m, n, 1280, slices, None, True, fp8, True) >= 32
+                    assert _native.choose_block_m(m, slices, True, -1, fp8, n, 1280, True, True) >= 32
+    assert OF.tiles_block_m(32, 60, 512, 1280, 3, None, True, False, False) == 16

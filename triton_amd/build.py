@@ -109,14 +109,14 @@ def build(force=True, verbose=False):
     srcs = [s for s in SOURCES if os.path.exists(os.path.join(CSRC, s))]
     objs = [os.path.join(objdir, os.path.splitext(s)[0] + ".o") for s in srcs]
     deps = [os.path.join(CSRC, "common.h"), os.path.join(CSRC, "moe_matmul_impl.h"), os.path.join(CSRC, "moe_matmul_stream.h"), os.path.join(CSRC, "moe_matmul_dense.h"),
-            os.path.join(CSRC, "moe_matmul_kk.h"), os.path.join(CSRC, "moe_matmul_mx.h"),
+            os.path.join(CSRC, "moe_matmul_kk.h"), os.path.join(CSRC, "moe_matmul_mx.h"), os.path.join(CSRC, "tile_rules.h"),
             os.path.join(HERE, "..", "include", "triton_amd.h")]
     todo = []
     for s, o in zip(srcs, objs):
         newest = max(os.path.getmtime(p) for p in [os.path.join(CSRC, s), *deps])
         if force or not os.path.exists(o) or os.path.getmtime(o) < newest:
             todo.append((s, o))
-    host_src = [os.path.join(CSRC, "host.cpp"), os.path.join(HERE, "..", "include", "triton_amd.h")]
+    host_src = [os.path.join(CSRC, "host.cpp"), os.path.join(CSRC, "tile_rules.h"), os.path.join(HERE, "..", "include", "triton_amd.h")]
     host = force or not os.path.exists(HOST) or os.path.getmtime(HOST) < max(map(os.path.getmtime, host_src))
     with ThreadPoolExecutor(max_workers=min(8, max(1, len(todo)))) as ex:
         jobs = [ex.submit(_compile, s, o) for s, o in todo] + ([ex.submit(_build_host)] if host else [])

@@ -8,6 +8,7 @@
 #include <unordered_set>
 
 #include "../../include/triton_amd.h"
+#include "tile_rules.h"
 
 #define TAMD_DEVICE __device__ __forceinline__
 
@@ -135,8 +136,6 @@ inline int dtype_size(int dt) {
     default: return 0;
   }
 }
-
-inline bool aligned(const void *p, size_t a) { return (reinterpret_cast<uintptr_t>(p) % a) == 0; }
 
 // One-time set-up per kernel and device, kept out of the per-call path: raising a kernel's dynamic LDS limit (an
 // attribute of the function in the device's loaded code object) and the device's CU count.  The only process-wide

@@ -22,6 +22,7 @@
 #include <cstring>
 
 #include "../../include/triton_amd.h"
+#include "tile_rules.h"
 
 namespace {
 
@@ -177,16 +178,16 @@ int choose_block_m(int64_t m, int64_t n_slices, bool ragged, int64_t expected, b
 }
 // tiles_block_m of the same file; the same test compares the two.
 int tiles_block_m(int bm, int64_t m, int64_t n, int64_t k, int64_t n_slices, int64_t expected, bool mxfp4_weights, bool fp8_rows,
-                      bool mx_out) {
+                  bool not_streamed) {
   constexpr int64_t cus = 256;
   const int64_t mean = m / (n_slices > 1 ? n_slices : 1), rows = expected >= 0 ? expected : (mean > 1 ? mean : 1);
   const int64_t slices = n_slices < m ? n_slices : m, cols = (n + 255) / 256;
   auto tiles = [&](int64_t b) { return slices * ((rows + b - 1) / b) * cols; };
   const double cover = (double)rows + 2.0 * std::pow((double)rows, 0.5);
-  if (bm == 16 && mxfp4_weights && tiles(32) > cus * 3 / 4 && k <= 1152) return 32;
+  if (bm == 16 && mxfp4_weights && (not_streamed || (tiles(32) > cus * 3 / 4 && k <= 1152))) return 32;
   if (bm == 128 && tiles(128) <= (mxfp4_weights ? cus : cus / 2)) bm = 64;
   if (bm == 64 && tiles(64) <= (mxfp4_weights ? cus * 3 / 4 : cus * 3 / 8)) bm = 32;
-  if (bm == 32 && mxfp4_weights && !mx_out && n % 16 == 0 && k <= 4096 &&
+  if (bm == 32 && mxfp4_weights && !not_streamed &&
       (fp8_rows ? cover <= 16 && tiles(32) <= cus * 5 / 16 && k >= 640 : cover <= 32 && tiles(32) <= cus / 4))
     bm = 16;
   return bm;
@@ -437,10 +438,12 @@ PyObject *py_matmul(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
            tbs.scalar_type() == at::kInt && tbo.dim() == 2 && tbs.dim() == 2 && tbo.size(0) == 5 && tbs.size(0) == 5 &&
            (tbo.stride(1) == 1 || tbo.size(1) == 1) && (tbs.stride(1) == 1 || tbs.size(1) == 1));
       n_slices = tss.size(0);
-      need(n_slices > 0 && n_slices <= n_mat && (!g.bias || tensor(bias_o).dim() == 2));
+      need(n_slices > 0 && n_slices <= n_mat && N <= 0x7FFFFFFF && K <= 0x7FFFFFFF && (!g.bias || tensor(bias_o).dim() == 2));
       const int64_t expected = ex.none() ? -1 : as_int(ex.p);
+      g.N = (int)N, g.K = (int)K, g.n_experts = (int)n_slices;
+      g.block_offs = (const int32_t *)tbo.data_ptr(), g.block_schedule = (const int32_t *)tbs.data_ptr();
       const int bm = tiles_block_m(choose_block_m(M, n_slices, true, expected, (a8 || a4) && w_fp4), M, N, K, n_slices, expected,
-                                       w_fp4, a8, mx_out || a_mx);
+                                   w_fp4, a8, mx_out || !tamd::blocks_of_16_stream(g));
       const int row = bm == 16 ? 0 : bm == 32 ? 1 : bm == 64 ? 2 : 3;
       g.slice_sizes = (const int32_t *)tss.data_ptr(), g.slice_offs = (const int32_t *)tso.data_ptr();
       g.block_offs = (const int32_t *)tbo.data_ptr() + row * tbo.stride(0);
@@ -676,6 +679,16 @@ PyObject *py_choose_block_m(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
   });
 }
 
+// (address of a tamd_matmul_args): whether its row blocks of 16 would take the streaming kernel.
+PyObject *py_blocks_of_16_stream(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
+  return covered([&]() -> PyObject * {
+    need(nargs == 1);
+    tamd_matmul_args a;
+    std::memcpy(&a, (const void *)(intptr_t)as_int(v[0]), sizeof a);
+    return PyBool_FromLong(tamd::blocks_of_16_stream(a));
+  });
+}
+
 // (addresses of the C ABI functions by name, Tensor, CDNA4MXValueLayout, CDNA4MXScaleLayout, FP4, constraints ContextVar,
 //  flags ContextVar)
 PyObject *py_init(PyObject *, PyObject *args) {
@@ -717,6 +730,7 @@ PyMethodDef methods[] = {{"init", py_init, METH_VARARGS, nullptr},
                          {"downcast", TAMD_FAST(py_downcast)},
                          {"upcast", TAMD_FAST(py_upcast)},
                          {"choose_block_m", TAMD_FAST(py_choose_block_m)},
+                         {"blocks_of_16_stream", TAMD_FAST(py_blocks_of_16_stream)},
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

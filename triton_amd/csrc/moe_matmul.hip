@@ -27,7 +27,7 @@ extern "C" int tamd_matmul_sized(const tamd_matmul_args *args, size_t args_size,
   memcpy(&a, args, args_size);
   if (a.y_rows == 0 && !a.scatter_indx) a.y_rows = a.M;
   if (a.M < 0 || a.N < 0 || a.K < 0 || a.n_experts < 1) return TAMD_E_INVALID;
-  if (a.n_experts == 1) a.w_stride_e = a.w_mx_stride_e = a.bias_stride_e = 0;  // never used; keeps the alignment checks honest
+  drop_unused_pitches(a);
   if (a.M == 0 || a.N == 0) return 0;
   // K == 0 would be a bias-only problem; no kernel is built for it, and the K loops assume at least one stage
   if (a.K == 0) return TAMD_E_UNSUPPORTED;

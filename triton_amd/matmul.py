@@ -353,9 +353,6 @@ def matmul(a, b, bias, a_ragged_metadata: Optional[RaggedTensorMetadata] = None,
     flags = make_opt_flags(M, N, K, n_slices, ragged,
                            a_ragged_metadata.expected_slice_size if ragged else None,
                            fp8_rows=(a_packed or a.dtype in fp8_types) and b_fp4)
-    if ragged and _opt_flags._opt_flags.get() is None and _opt_flags._constraints().get("block_m") is None:
-        flags.block_m = _opt_flags.tiles_block_m(flags.block_m, M, N, K, n_slices, a_ragged_metadata.expected_slice_size,
-                                                     b_fp4, a.dtype in fp8_types, mx_out or a_mx_scale is not None)
     args = _lib.MatmulArgBag()
     args.x, args.x_dtype = a.data_ptr(), _lib.MXFP4 if a_packed else _lib.dtype_code(a.dtype)
     args.x_stride_m = a.stride(-2)
@@ -448,6 +445,12 @@ def matmul(a, b, bias, a_ragged_metadata: Optional[RaggedTensorMetadata] = None,
     if ragged:
         md = a_ragged_metadata
         args.slice_sizes, args.slice_offs = md.slice_sizes.data_ptr(), md.slice_offs.data_ptr()
+        if _opt_flags._opt_flags.get() is None and _opt_flags._constraints().get("block_m") is None:
+            args.block_offs, args.block_schedule = md.block_offs_data.data_ptr(), md.block_schedule_data.data_ptr()
+            packed = args.pack()   # (the ranges of a split K are no dense columns)
+            streams = flags.split_k == 1 and _native.blocks_of_16_stream(ctypes.addressof(packed))
+            flags.block_m = _opt_flags.tiles_block_m(flags.block_m, M, N, K, n_slices, md.expected_slice_size, b_fp4,
+                                                     a.dtype in fp8_types, not streams)
         args.block_offs = md.block_offs(flags.block_m).data_ptr()
         args.block_schedule = md.block_schedule(flags.block_m).data_ptr()
         args.block_m = flags.block_m

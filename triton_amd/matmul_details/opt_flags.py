@@ -86,7 +86,7 @@ CUS = 256   # compute units of the part
 
 
 def tiles_block_m(block_m: int, m: int, n: int, k: int, n_slices: int, expected_slice_size: Optional[int],
-                  mxfp4_weights: bool, fp8_rows: bool, mx_out: bool) -> int:
+                  mxfp4_weights: bool, fp8_rows: bool, not_streamed: bool) -> int:
     """Row block of a ragged problem, given the one that its slices' sizes ask for, from the number of its tiles (row blocks x
     256 columns).
 
@@ -96,19 +96,22 @@ def tiles_block_m(block_m: int, m: int, n: int, k: int, n_slices: int, expected_
     16 columns), also for fp8 rows without block scales (10 to 40 % up to 80 tiles; not with two blocks per slice, and not
     below K 640, where a unit is too short).  Few rows and many tiles of a short K (up to 1152, where a unit's barrier and start weigh
     more than its copies): the tiled kernel instead of the streaming one (20 to 50 %).
+    `not_streamed`: blocks of 16 would not run in the streaming kernel (weights or scales with a padded pitch, an unaligned
+    base or 2 GB of them, a long K, odd columns, microscaled rows or output); a block of 16 is then a whole 32-row
+    fragment of the tiled kernel, and never the choice for MXFP4 weights.
     The lines are those that gave the shortest mean time over 700 layers of 1 to 4000 tokens, 8 to 128 experts, K 512
     to 5760."""
     rows = expected_slice_size if expected_slice_size is not None else max(1, m // max(1, n_slices))
     slices, cols = min(n_slices, m), -(-n // 256)
     tiles = lambda b: slices * -(-rows // b) * cols
     cover = rows + 2.0 * rows ** 0.5
-    if block_m == 16 and mxfp4_weights and tiles(32) > CUS * 3 // 4 and k <= 1152:
+    if block_m == 16 and mxfp4_weights and (not_streamed or (tiles(32) > CUS * 3 // 4 and k <= 1152)):
         return 32
     if block_m == 128 and tiles(128) <= (CUS if mxfp4_weights else CUS // 2):
         block_m = 64
     if block_m == 64 and tiles(64) <= (CUS * 3 // 4 if mxfp4_weights else CUS * 3 // 8):
         block_m = 32
-    if block_m == 32 and mxfp4_weights and not mx_out and n % 16 == 0 and k <= 4096:
+    if block_m == 32 and mxfp4_weights and not not_streamed:
         if (cover <= 16 and tiles(32) <= CUS * 5 // 16 and k >= 640) if fp8_rows else (cover <= 32 and tiles(32) <= CUS // 4):
             block_m = 16
     return block_m
