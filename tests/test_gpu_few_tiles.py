@@ -166,7 +166,7 @@ def test_microscaled_output_keeps_its_kernel(device):
 
 
 @pytest.mark.parametrize("M,N", [(257, 448), (700, 272), (1500, 128), (161, 2560), (161, 2576), (2100, 1600), (33, 16)])
-@pytest.mark.parametrize("kind", ["bf16", "f16", "fp8", "mxfp4", "bf16 w", "fp8 w"])
+@pytest.mark.parametrize("kind", ["bf16", "f16", "fp8", "mxfp4", "bf16 w", "fp8 w", "bf16 along N w"])
 def test_dense(M, N, kind, device):
     """Dense products around the lines between the streaming kernel's units, blocks of 32, 64 and 128 rows."""
     torch.manual_seed(M)
@@ -175,7 +175,8 @@ def test_dense(M, N, kind, device):
     bias = torch.randn(N, device=device)
     pc = {"out_dtype": torch.bfloat16}
     if kind[-1] == "w":
-        w = w.to(torch.bfloat16 if kind == "bf16 w" else torch.float8_e4m3fn).t().contiguous().t()
+        w = w.to(torch.float8_e4m3fn if kind == "fp8 w" else torch.bfloat16)
+        w = w if "along N" in kind else w.t().contiguous().t()
         wf = w.float()
     else:
         w, ws = downcast_to_mxfp(w, torch.uint8, axis=0)

@@ -280,3 +280,24 @@ def test_blocks_of_16_only_where_they_stream():
                     assert OF.tiles_block_m(base, m, n, 1280, slices, None, True, fp8, True) >= 32
                     assert _native.choose_block_m(m, slices, True, -1, fp8, n, 1280, True, True) >= 32
     assert OF.tiles_block_m(32, 60, 512, 1280, 3, None, True, False, False) == 16
+
+
+def dense_block_m(M, N, K, x, w, along_n=False, cus=256, batch=1):
+    import ctypes
+    from triton_amd import _lib, _native
+    bag = _lib.MatmulArgBag()
+    bag.M, bag.N, bag.K, bag.n_experts, bag.x_dtype, bag.w_dtype = M, N, K, batch, getattr(_lib, x), getattr(_lib, w)
+    bag.w_stride_k, bag.w_stride_n = (N, 1) if along_n else (1, K)
+    packed = bag.pack()
+    return _native.dense_block_m(ctypes.addressof(packed), cus)
+
+
+@pytest.mark.parametrize("M,N,K,block_m", [
+    (2048, 4096, 2048, 128), (4096, 4096, 2048, 128), (3943, 7464, 6144, 128), (12572, 1024, 6688, 128),   # whole rounds of 128
+    (256, 4096, 2048, 32), (64, 512, 576, 32), (5749, 512, 2432, 64), (603, 4864, 1344, 64), (5056, 280, 672, 64),
+])
+def test_dense_blocks_of_weights_along_n(M, N, K, block_m):
+    """16-bit weights contiguous along N: the kernel for them holds one tile per CU, and a tile of few rows takes almost as long as one
+    of many, so rounds count and rows hardly do (sizes timed with every block)."""
+    assert dense_block_m(M, N, K, "BF16", "BF16", along_n=True) == block_m
+    assert dense_block_m(M, N, K, "F16", "F16", along_n=True) == block_m

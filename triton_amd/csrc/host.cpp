@@ -689,6 +689,16 @@ PyObject *py_blocks_of_16_stream(PyObject *, PyObject *const *v, Py_ssize_t narg
   });
 }
 
+// (address of a tamd_matmul_args, compute units): the row block of a dense product.
+PyObject *py_dense_block_m(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
+  return covered([&]() -> PyObject * {
+    need(nargs == 2);
+    tamd_matmul_args a;
+    std::memcpy(&a, (const void *)(intptr_t)as_int(v[0]), sizeof a);
+    return PyLong_FromLong(tamd::dense_block_m(a, (int)as_int(v[1])));
+  });
+}
+
 // (addresses of the C ABI functions by name, Tensor, CDNA4MXValueLayout, CDNA4MXScaleLayout, FP4, constraints ContextVar,
 //  flags ContextVar)
 PyObject *py_init(PyObject *, PyObject *args) {
@@ -731,6 +741,7 @@ PyMethodDef methods[] = {{"init", py_init, METH_VARARGS, nullptr},
                          {"upcast", TAMD_FAST(py_upcast)},
                          {"choose_block_m", TAMD_FAST(py_choose_block_m)},
                          {"blocks_of_16_stream", TAMD_FAST(py_blocks_of_16_stream)},
+                         {"dense_block_m", TAMD_FAST(py_dense_block_m)},
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

@@ -6,7 +6,9 @@
 // per K row); a lane gathers the 8 K values of its column with 2-byte LDS reads.  The MFMA wants K-contiguous operands
 // on both sides, so one of the two has to be transposed somewhere; doing it on the LDS read costs no extra pass.
 //
-// One workgroup per CU (three 32 KB weight stages); not a tuned kernel.
+// One workgroup per CU (three 32 KB weight stages); not a tuned kernel.  What bounds it: the 2-byte LDS reads of the weights, which a
+// tile of 32 rows has as many of as one of 128 (4224 K values: 57 us against 75), so the row block of a dense product is one that
+// saves rounds over the CUs before it saves rows (dense_block_m).
 #pragma once
 #include "moe_matmul_impl.h"
 
@@ -328,8 +330,8 @@ int dispatch_w16(const tamd_matmul_args &a, int block_m, int grid_m, hipStream_t
   if (skinny16_applicable(a)) return launch_skinny16<XDT>(a, st);
   if (a.w_stride_k == 1)
     return XDT == TAMD_BF16 ? dispatch_mm_kk_bf16(a, block_m, grid_m, st) : dispatch_mm_kk_f16(a, block_m, grid_m, st);
-  dense_grid(a, block_m, grid_m);
   if (a.w_stride_n != 1) return TAMD_E_UNSUPPORTED;
+  dense_grid(a, block_m, grid_m);
   if (a.K % 8 != 0 || a.N % 8 != 0) return TAMD_E_UNSUPPORTED;  // whole 16-byte chunks along K and N
   if (!aligned(a.w, 16) || (a.w_stride_k * 2) % 16 != 0 || (a.w_stride_e * 2) % 16 != 0) return TAMD_E_ALIGNMENT;
   if (!aligned(a.x, 16) || (a.x_stride_m * 2) % 16 != 0 || (a.x_stride_z * 2) % 16 != 0) return TAMD_E_ALIGNMENT;

@@ -1235,37 +1235,18 @@ int launch_x16_act(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
   }
 }
 
-// Row block size of a dense / batched problem (block_m == 0 on entry of a dispatcher): the block whose tiles take the fewest
-// rounds over the CUs, weighted with what a tile of it takes.  MXFP4 weights: one and a half tiles per CU (fp8
-// and packed rows one and a quarter) run at the speed of one, a tile of 64 or 32 rows takes 0.45 or 0.35 of one of 128; kernels for operands of one type hold a tile per CU, 0.6 and 0.45.
-// (Fitted to 800 products of 1 to 4096 rows timed with every block, against the largest block that gave every CU a tile: one type 9 %
-// faster in the mean -- 2000 rows of K 2000 and N 1600 two rounds of 64 rows instead of one of 128 on half the CUs, up to 1.7 times --,
-// MXFP4 2.5 %, none slower by more than 5 %.)
-inline int dense_block_m(const tamd_matmul_args &a, bool one_type) {
-  int cus = 0;
-  if (cu_count(cus) != 0) cus = 256;
-  const bool x16 = a.x_dtype == TAMD_BF16 || a.x_dtype == TAMD_F16;
-  const int64_t cols = (int64_t)((a.N + BLOCK_N - 1) / BLOCK_N) * a.n_experts, slots = one_type ? cus : (x16 ? cus * 3 / 2 : cus * 5 / 4);
-  const int extra = x16 ? 32 : 0;   // remainder that a block of 128 absorbs
-  const int bm[3] = {128, 64, 32}, weight[3] = {100, one_type ? 60 : 45, one_type ? 45 : 35};
-  int best = 0;
-  int64_t least = 0;
-  for (int i = 0; i < 3; ++i) {
-    const int64_t m = i == 0 && a.M > 128 ? a.M - extra : a.M;
-    const int64_t cost = ((m + bm[i] - 1) / bm[i] * cols + slots - 1) / slots * weight[i];
-    if (best == 0 || cost < least) best = bm[i], least = cost;
-  }
-  return best;
-}
 // Whether a dense / batched problem has enough 32-row tiles for the tiled kernels: more than `tiles`.  Fewer
 // run as 16-row blocks through the streaming kernel, whose units of 16 columns reach every CU.  (800 products: with 16-bit rows
 // 4 to 60 % faster up to 63 tiles, 18 to 50 % slower from 84 on; with fp8 rows the line is at 24 to 48.)
 inline bool dense_prefers_tiles(const tamd_matmul_args &a, int tiles) {
   return (int64_t)((a.M + 31) / 32) * a.n_experts * ((a.N + BLOCK_N - 1) / BLOCK_N) > tiles;
 }
-inline void dense_grid(const tamd_matmul_args &a, int &block_m, int &grid_m, bool one_type = false) {
+// Row blocks of a dense / batched problem (block_m == 0 on entry of a dispatcher).
+inline void dense_grid(const tamd_matmul_args &a, int &block_m, int &grid_m) {
   if (block_m != 0) return;
-  block_m = dense_block_m(a, one_type);
+  int cus = 0;
+  if (cu_count(cus) != 0) cus = 256;
+  block_m = dense_block_m(a, cus);
   grid_m = ((a.M + block_m - 1) / block_m) * a.n_experts;
 }
 

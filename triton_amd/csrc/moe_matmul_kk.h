@@ -425,7 +425,7 @@ int launch_kk(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
 template <int XDT>
 int dispatch_kk(const tamd_matmul_args &a, int block_m, int grid_m, hipStream_t st) {
   constexpr int ESZ = KK<XDT>::ESZ;
-  dense_grid(a, block_m, grid_m, true);
+  dense_grid(a, block_m, grid_m);
   if (a.w_stride_k != 1 || a.K % (16 / ESZ) != 0) return TAMD_E_UNSUPPORTED;
   if (!aligned(a.w, 16) || (a.w_stride_n * ESZ) % 16 != 0 || (a.w_stride_e * ESZ) % 16 != 0) return TAMD_E_ALIGNMENT;
   if (!aligned(a.x, 16) || (a.x_stride_m * ESZ) % 16 != 0 || (a.x_stride_z * ESZ) % 16 != 0) return TAMD_E_ALIGNMENT;

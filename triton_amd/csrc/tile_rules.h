@@ -45,4 +45,29 @@ inline bool blocks_of_16_stream(tamd_matmul_args a) {
   return a.w_dtype == TAMD_MXFP4 && stream16_applicable(a);
 }
 
+// Row block size of a dense / batched problem: the block whose tiles take the fewest rounds over the CUs, weighted with what a
+// tile of it takes.  MXFP4 weights: one and a half tiles per CU (fp8 and packed rows one and a quarter) run at the speed of one, a tile of 64 or 32
+// rows takes 0.45 or 0.35 of one of 128.  Kernels for operands of one type hold one tile per CU: 0.6 and 0.45 where the weights are
+// contiguous along K, 0.8 and 0.76 where they are contiguous along N (the LDS reads of the weights do not follow the rows).
+// (Fitted to products timed with every block.  800 of 1 to 4096 rows, against the largest block that gave every CU a tile: one type along K 9 %
+// faster in the mean -- 2000 rows of K 2000 and N 1600 two rounds of 64 rows instead of one of 128 on half the CUs, up to 1.7 times --,
+// MXFP4 2.5 %, none slower by more than 5 %.  150 of 16 to 16384 rows along N: 0.7 % slower than the best block of each
+// in the mean, 12 % with the MXFP4 figures; 3943 x 6144 x 7464 815 us in blocks of 64, 471 in blocks of 128, 5749 x 2432 x 512 68 in
+// blocks of 32, 39 in blocks of 64.)
+inline int dense_block_m(const tamd_matmul_args &a, int cus) {
+  const bool x16 = a.x_dtype == TAMD_BF16 || a.x_dtype == TAMD_F16, mxfp4 = a.w_dtype == TAMD_MXFP4;
+  const bool along_n = !mxfp4 && a.w_stride_k != 1;
+  const int64_t cols = (int64_t)((a.N + 255) / 256) * a.n_experts, slots = !mxfp4 ? cus : (x16 ? cus * 3 / 2 : cus * 5 / 4);
+  const int extra = x16 && !along_n ? 32 : 0;   // remainder that a block of 128 absorbs
+  const int bm[3] = {128, 64, 32}, weight[3] = {100, mxfp4 ? 45 : (along_n ? 80 : 60), mxfp4 ? 35 : (along_n ? 76 : 45)};
+  int best = 0;
+  int64_t least = 0;
+  for (int i = 0; i < 3; ++i) {
+    const int64_t m = i == 0 && a.M > 128 ? a.M - extra : a.M;
+    const int64_t cost = ((m + bm[i] - 1) / bm[i] * cols + slots - 1) / slots * weight[i];
+    if (best == 0 || cost < least) best = bm[i], least = cost;
+  }
+  return best;
+}
+
 }  // namespace tamd
