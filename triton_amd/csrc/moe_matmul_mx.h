@@ -138,7 +138,8 @@ TAMD_DEVICE void run_tile_mx(const tamd_matmul_args &a, const Tile &t, uint8_t *
   const bool cdna4 = a.w_mx_layout == TAMD_SCALE_CDNA4;
   const uint8_t *xs_base = a.x_mx_scale + (int64_t)t.z * a.x_mx_stride_z;
   const uint8_t *ws_base = a.w_mx_scale + (int64_t)t.expert * a.w_mx_stride_e;
-  uint32_t as_off[NFR], ws_off[NF];
+  constexpr uint32_t kSel = 0x06040200u;             // byte selectors: every second scale, from the lane half's first on
+  uint32_t as_off[NFR], as_sel[NFR], ws_off[NF];
   const int col0 = t.n0 + wave * 64 + c32 * NF, half = (c32 >> 3) & 1;
   if (cdna4) {   // ws_off[0]: groups h and 2 + h of both columns lie 128 bytes apart
     const int KSP = (G + 7) / 8 * 8, last = (N - 1) / 32, blk = col0 / 32;
@@ -148,9 +149,6 @@ TAMD_DEVICE void run_tile_mx(const tamd_matmul_args &a, const Tile &t, uint8_t *
     // a load touches a line per lane, so each half of the wave loads one of its lanes' two columns and the halves exchange them
     ws_off[0] = ws_off[1] = (uint32_t)(col0 + h < N ? col0 + h : N - 1) * (uint32_t)a.w_mx_stride_n;
   }
-  // rows that a gathered index can name (ordinary loads have no descriptor that would end with them), and the offset of one it cannot
-  const uint32_t x_rows = gather_limit(a);
-  constexpr uint32_t kNoRow = 0xFFFFFFFFu;
   const int g_last = G > 8 ? G - 8 : 0;               // where the last eight bytes start
   uint64_t as_raw[NFR], ws_raw[NF];
 #pragma unroll
@@ -161,7 +159,7 @@ TAMD_DEVICE void run_tile_mx(const tamd_matmul_args &a, const Tile &t, uint8_t *
     const int at = 8 * e < g_last ? 8 * e : g_last;
     if (x_mx) {
 #pragma unroll
-      for (int i = 0; i < NFR; ++i) as_raw[i] = load_scales(xs_base + at, as_off[i] == kNoRow ? 0u : as_off[i], G);
+      for (int i = 0; i < NFR; ++i) as_raw[i] = load_scales(xs_base + at, as_off[i], G);
     }
     const uint8_t *w = ws_base + (cdna4 ? 256 * e : at);
     ws_raw[0] = load_scales(w, ws_off[0], cdna4 ? 8 : G);
@@ -170,13 +168,12 @@ TAMD_DEVICE void run_tile_mx(const tamd_matmul_args &a, const Tile &t, uint8_t *
   uint32_t sa[NFR], sw[NF];   // byte q: the scale of step q
   auto take_sc = [&](int e) {
     const int shift = 8 * (8 * e > g_last ? 8 * e - g_last : 0);
-    const uint32_t sel = 0x06040200u + (uint32_t)h * 0x01010101u;
-    auto pick = [&](uint64_t v) {
+    auto pick = [&](uint64_t v, uint32_t sel) {
       const uint64_t x = v >> shift;
       return __builtin_amdgcn_perm((uint32_t)(x >> 32), (uint32_t)x, sel);
     };
 #pragma unroll
-    for (int i = 0; i < NFR; ++i) sa[i] = x_mx ? (as_off[i] == kNoRow ? 0u : pick(as_raw[i])) : 0x7F7F7F7Fu;
+    for (int i = 0; i < NFR; ++i) sa[i] = x_mx ? pick(as_raw[i], as_sel[i]) : 0x7F7F7F7Fu;
     if (cdna4) {
       const uint32_t s2 = 0x06020400u + (uint32_t)half * 0x01010101u;
 #pragma unroll
@@ -187,7 +184,7 @@ TAMD_DEVICE void run_tile_mx(const tamd_matmul_args &a, const Tile &t, uint8_t *
       const auto lo = __builtin_amdgcn_permlane32_swap((uint32_t)x, (uint32_t)x, false, false);
       const auto hi = __builtin_amdgcn_permlane32_swap((uint32_t)(x >> 32), (uint32_t)(x >> 32), false, false);
 #pragma unroll
-      for (int f = 0; f < NF; ++f) sw[f] = __builtin_amdgcn_perm(hi[f], lo[f], sel);
+      for (int f = 0; f < NF; ++f) sw[f] = __builtin_amdgcn_perm(hi[f], lo[f], kSel + (uint32_t)h * 0x01010101u);
     }
     // (made before the next ones are requested, which then come to the same registers)
 #pragma unroll
@@ -217,6 +214,7 @@ TAMD_DEVICE void run_tile_mx(const tamd_matmul_args &a, const Tile &t, uint8_t *
     }
   };
 
+  const uint32_t x_rows = gather_limit(a);
   issue_b(0);
   if (a.gather_indx) wait_vmcnt<4 * BLOCKS>();   // (the copies of the weights may be outstanding)
 #pragma unroll
@@ -226,9 +224,11 @@ TAMD_DEVICE void run_tile_mx(const tamd_matmul_args &a, const Tile &t, uint8_t *
     const uint32_t src = a.gather_indx ? idx[0] : (uint32_t)(row0 + r);
     const uint32_t srs = a.gather_indx ? idx[X16 ? 0 : kWave] : (uint32_t)(row0 + (rs < t.rows ? rs : t.rows - 1));
     // rows past the end of the slice are never stored: they are copied as zeros, which keeps the matrix cores' inputs quiet; so
-    // is the row of an index that names none (-1), whose scales are not read
+    // is the row of an index that names none (-1), for which the first row's scales are read (ordinary loads have no descriptor that
+    // would end with them) and zero bytes taken (selector 12)
     a_off[i] = r < t.rows && src < x_rows ? src * (uint32_t)(a.x_stride_m * S::ESZ) + a_chunk * 16 : kOob;
-    as_off[i] = srs < x_rows ? srs * (uint32_t)a.x_mx_stride_m : kNoRow;
+    as_off[i] = srs < x_rows ? srs * (uint32_t)a.x_mx_stride_m : 0u;
+    as_sel[i] = srs < x_rows ? kSel + (uint32_t)h * 0x01010101u : 0x0C0C0C0Cu;
   }
   if (a.gather_indx) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // read before the rows are copied over them
   issue_a(0);

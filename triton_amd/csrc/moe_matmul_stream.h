@@ -442,15 +442,17 @@ __global__ __launch_bounds__((NCW + NC + 2) * 64, 1) void mm_stream16_kernel(tam
     const bool cdna4 = a.w_mx_layout == TAMD_SCALE_CDNA4;
     const int kb = 4 * SS * wave;  // first e8m0 group of this wave's K slice
     frag_t areg[SS * 4];           // this wave's K slice of the block's rows, row c16
+    const uint32_t x_rows = gather_limit(a);
     int c_blk = blk0 - 1, c_cg = cg0;
     auto load_block = [&](int blk) {
       Block cb;
       get_block(blk, cb);
       int rc = c16 < cb.rows ? c16 : cb.rows - 1;
       rc = cb.row0 + (rc < 0 ? 0 : rc);
-      const int64_t src = a.gather_indx ? (int64_t)a.gather_indx[rc] : (int64_t)rc;
+      const uint32_t idx = (uint32_t)(a.gather_indx ? a.gather_indx[rc] : rc);
       // (an index that names no row, -1: zeros, as the tiled kernels read them past the end of a descriptor)
-      const bool have = cb.rows > 0 && (uint64_t)src < gather_limit(a);
+      const bool have = cb.rows > 0 && idx < x_rows;
+      const int64_t src = (int64_t)idx;
       if constexpr (A8) {
         const uint8_t *xr = (const uint8_t *)a.x + (int64_t)cb.z * a.x_stride_z + src * a.x_stride_m;
 #pragma unroll
