@@ -70,7 +70,7 @@ extern "C" int tamd_matmul_sized(const tamd_matmul_args *args, size_t args_size,
         (int64_t)a.N * (cdna4_sc ? (int64_t)(a.K / 32 + 7) : a.w_mx_stride_n) >= (int64_t)0x7FFFFF00)
       return TAMD_E_UNSUPPORTED;
     if (a.x_mx_scale) {
-      // block scales of the activations: MXFP8 (e4m3 values) and MXFP4 through the scaled MFMA only
+      // block scales of the activations: fp8 values and MXFP4 through the scaled MFMA only
       if (!x8 && !x4) return TAMD_E_UNSUPPORTED;
       if (a.x_mx_stride_m < a.K / 32 || x_rows * a.x_mx_stride_m >= (int64_t)0x7FFFFF00) return TAMD_E_UNSUPPORTED;
     }

@@ -86,7 +86,7 @@ TAMD_DEVICE void run_tile_mx(const tamd_matmul_args &a, const Tile &t, uint8_t *
   const uint32_t lds_b = lds_base + b_at;
   const uint8_t *bbuf = lds + b_at;
   const int n_k = (K + KA - 1) / KA;
-  const bool x_mx = FP4 || (XDT == TAMD_FP8_E4M3 && a.x_mx_scale != nullptr);
+  const bool x_mx = FP4 || (!X16 && a.x_mx_scale != nullptr);
 
   // ---- row indices: of the rows whose values the lane copies, and of the rows whose scales its MFMAs use; by LDS, each in front of
   // the row pieces that the wave will copy there (see run_tile)
