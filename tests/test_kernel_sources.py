@@ -43,3 +43,16 @@ def test_requests_deliver_to_lds(path):
         text = f.read()
     assert loads_to_registers(text) == []
     assert not re.search(r"\basm\s*\((?!\s*\))", re.sub(r"//[^\n]*", "", text)), "asm that is not volatile"
+
+
+def test_barriers_wait_for_lds():
+    """Every barrier is sync_threads(), whose wait for the wave's LDS accesses the compiler cannot take out."""
+    bare = re.compile(r"\b__syncthreads\s*\(|\bs_barrier\b|__builtin_amdgcn_s_barrier")
+    for path in sorted(glob.glob(os.path.join(CSRC, "*.h")) + glob.glob(os.path.join(CSRC, "*.hip"))):
+        with open(path) as f:
+            text = re.sub(r"//[^\n]*", "", f.read())
+        if os.path.basename(path) == "common.h":
+            at = re.search(r"void sync_threads\(\) \{\s*asm volatile\(\"s_waitcnt lgkmcnt\(0\)\" ::: \"memory\"\);\s*__syncthreads\(\);\s*\}", text)
+            assert at
+            text = text[:at.start()] + text[at.end():]
+        assert not bare.findall(text), path

@@ -16,6 +16,14 @@ namespace tamd {
 
 constexpr int kWave = 64;
 
+// Barrier of the workgroup, behind every LDS access of the wave.  __syncthreads() alone does not promise it with this compiler: its wait is a soft
+// one, taken out of the head of a loop when nothing is outstanding on the way in, and not put back for what the loop's own end
+// leaves outstanding (the partial sums of a unit in moe_matmul_stream.h were read before they were written).
+TAMD_DEVICE void sync_threads() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __syncthreads();
+}
+
 TAMD_DEVICE float bits_to_f32(uint32_t u) { return __builtin_bit_cast(float, u); }
 TAMD_DEVICE uint32_t f32_to_bits(float f) { return __builtin_bit_cast(uint32_t, f); }
 

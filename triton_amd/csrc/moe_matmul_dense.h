@@ -117,13 +117,13 @@ TAMD_DEVICE void run_tile_w16(const tamd_matmul_args &a, const Tile &t, uint8_t 
   int rd = 0;  // ring slot of the stage being consumed (stage it lives in slot it % 3)
   for (int it = 0; it < n_k; ++it) {
     wait_vmcnt<NFR + 8>();  // copies complete in order: all but the NFR + 8 of stage it + 1 have landed
-    __syncthreads();        // stage `it` is visible; everyone is done with the slot stage it + 2 goes to
+    sync_threads();        // stage `it` is visible; everyone is done with the slot stage it + 2 goes to
     issue(it + 2, rd == 0 ? 2 : rd - 1);
     compute(rd);
     rd = rd == 2 ? 0 : rd + 1;
   }
   wait_dma();
-  __syncthreads();  // every wave is done with the stages: the epilogue's tables go there
+  sync_threads();  // every wave is done with the stages: the epilogue's tables go there
   tile_epilogue<NFR, ACT, XDT, false>(a, t, acc, lds + wave * 4096);
 }
 
@@ -261,7 +261,7 @@ __global__ __launch_bounds__(256) void mm_skinny16_kernel(tamd_matmul_args a) {
   for (int j = 0; j < 4; ++j)
 #pragma unroll
     for (int i = 0; i < 4; ++i) red[(wave * 16 + g * 4 + i) * SKINNY_PITCH + j * 16 + c] = acc[j][i];
-  __syncthreads();
+  sync_threads();
   // thread -> row tid / 16, four columns
   const int r = tid / 16, cq = (tid % 16) * 4;
   if (row0 + r >= M) return;

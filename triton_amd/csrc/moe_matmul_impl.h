@@ -1058,7 +1058,7 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
     const int n_stage = 2 * n_sup;   // (the same trip count, and barriers, for every group)
     for (int it = 0; it < n_stage; it += 2) {
       wait_vmcnt<ring_outstanding(DA, DB, CP_A, CP_B, false)>();
-      __syncthreads();
+      sync_threads();
       load_b(it >> 1);
       issue_a(it + DA - 1);
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // weights are in registers: the region may be refilled
@@ -1066,7 +1066,7 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
       compute(it, Even{});
       if (it + 1 < n_stage) {
         wait_vmcnt<ring_outstanding(DA, DB, CP_A, CP_B, true)>();
-        __syncthreads();
+        sync_threads();
         issue_a(it + DA);
         compute(it + 1, Odd{});
       }
@@ -1074,7 +1074,7 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
   } else {
     for (int it = 0; it < n_ka; it += 2) {
       wait_dma();
-      __syncthreads();
+      sync_threads();
       load_b(it >> 1);
       issue_a(it + 1);
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // weights are in registers: the region may be refilled
@@ -1084,7 +1084,7 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
         // the weight copies just issued (4, after the activation stage it + 1) are not needed before the next
         // even stage and take the longest (weights stream from HBM, activations mostly hit L2): leave them in flight
         wait_vmcnt<CP_B>();
-        __syncthreads();
+        sync_threads();
         issue_a(it + 2);
         compute(it + 1, Odd{});
       }
@@ -1099,7 +1099,7 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
     // (16 bytes per lane and access: a plane is [4 waves][NF x 4 quads][64 lanes] of four accumulators)
     f32x4_t *red = (f32x4_t *)lds_wg;
     constexpr int PLANE = 4 * NF * 4 * kWave;
-    __syncthreads();
+    sync_threads();
     if (grp > 0) {
 #pragma unroll
       for (int f = 0; f < NF; ++f)
@@ -1108,7 +1108,7 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
           red[(grp - 1) * PLANE + ((wave * NF + f) * 4 + j) * kWave + lane] =
               f32x4_t{acc[0][f][4 * j], acc[0][f][4 * j + 1], acc[0][f][4 * j + 2], acc[0][f][4 * j + 3]};
     }
-    __syncthreads();
+    sync_threads();
     if (grp > 0) return;
 #pragma unroll
     for (int g = 1; g < KS; ++g)
@@ -1123,7 +1123,7 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
     // (added here: left for the epilogue, which has several forms, the planes would not fit the registers until then)
 #pragma unroll
     for (int f = 0; f < NF; ++f) asm volatile("" : "+v"(acc[0][f]));
-    __syncthreads();   // the epilogue's tables take the same memory
+    sync_threads();   // the epilogue's tables take the same memory
   }
   // (the wave's own weight region is free by now: its table goes there)
   uint8_t *tab = KS > 1 ? lds_wg + wave * 4096 : lds + DA * A_STAGE + wave * 4096;

@@ -133,7 +133,7 @@ TAMD_DEVICE void run_tile_kk(const tamd_matmul_args &a, const Tile &t, uint8_t *
   for (int it = 0; it < n_k; ++it) {
     // copies complete in the order of their requests: all but those of the newest RING - 2 stages have landed
     if (grp == 0) wait_vmcnt<(RING - 2) * (NA0 + NB)>(); else wait_vmcnt<(RING - 2) * (NA1 + NB)>();
-    __syncthreads();   // stage `it` is visible; every wave is done with the slot that is refilled now
+    sync_threads();   // stage `it` is visible; every wave is done with the slot that is refilled now
     const uint8_t *buf = lds + rd * STAGE;
     uint4 av[NFR][2], bv[NF][2];
     if (live) {
@@ -170,7 +170,7 @@ TAMD_DEVICE void run_tile_kk(const tamd_matmul_args &a, const Tile &t, uint8_t *
     wr = wr + 1 == RING ? 0 : wr + 1;
   }
   wait_dma();
-  __syncthreads();
+  sync_threads();
 
   // ---- the groups' partial sums: group 0 finishes the row fragments [0, N0), group 1 the rest.  Plane (fragment,
   // strip) of the exchange is [NF x 4][64 lanes] of four accumulators; a wave reads only what its partner left for it.
@@ -203,7 +203,7 @@ TAMD_DEVICE void run_tile_kk(const tamd_matmul_args &a, const Tile &t, uint8_t *
 #pragma unroll
     for (int i = 0; i < N0; ++i) put(i);
   }
-  __syncthreads();
+  sync_threads();
   if (grp == 0) {
     f32x16_t mine[N0][NF];
 #pragma unroll
@@ -345,7 +345,7 @@ TAMD_DEVICE void run_tile_narrow(const tamd_matmul_args &a, const Tile &t, uint8
     wr = wr + 1 == RING ? 0 : wr + 1;
   }
   wait_dma();
-  __syncthreads();   // every ring is dead
+  sync_threads();   // every ring is dead
   f32x4_t *ex = (f32x4_t *)lds;
   constexpr int PLANE = NF * 4 * kWave;
   if (wave > 0) {
@@ -356,7 +356,7 @@ TAMD_DEVICE void run_tile_narrow(const tamd_matmul_args &a, const Tile &t, uint8
         ex[wave * PLANE + (f * 4 + j) * kWave + lane] =
             f32x4_t{acc[0][f][4 * j], acc[0][f][4 * j + 1], acc[0][f][4 * j + 2], acc[0][f][4 * j + 3]};
   }
-  __syncthreads();
+  sync_threads();
   if (wave > 0) return;
 #pragma unroll
   for (int w = 1; w < 4; ++w)

@@ -236,7 +236,7 @@ TAMD_DEVICE void run_tile_mx(const tamd_matmul_args &a, const Tile &t, uint8_t *
   const int swz = (c32 >> 1) & 7;
   for (int p = 0; p < n_k; ++p) {
     wait_vmcnt<0>();   // (everything requested so far belongs to this stage)
-    __syncthreads();   // stage p is visible; every wave is done with the buffer that stage p + 1 goes to
+    sync_threads();   // stage p is visible; every wave is done with the buffer that stage p + 1 goes to
     const uint8_t *buf = lds + (p & 1) * A_STAGE;
     uint4 raw[STEPS][NF];
 #pragma unroll

@@ -225,7 +225,7 @@ __global__ __launch_bounds__((NCW + NC + 2) * 64, 1) void mm_stream16_kernel(tam
       int slot = 0;
 #pragma unroll 1
       for (int s = 0; s < total_stages; ++s) {
-        __syncthreads();  // the partial sums of stage s - 1 and the bias of stage s are visible
+        sync_threads();  // the partial sums of stage s - 1 and the bias of stage s are visible
         if (s > 0) finish_fast((s - 1) & 1);
         if (c_blk < blk0 || c_cg == n_cg) {
           if (c_cg == n_cg) c_cg = 0;
@@ -246,7 +246,7 @@ __global__ __launch_bounds__((NCW + NC + 2) * 64, 1) void mm_stream16_kernel(tam
         ++c_cg;
         slot = slot + 1 == S::RING ? 0 : slot + 1;
       }
-      __syncthreads();
+      sync_threads();
       finish_fast((total_stages - 1) & 1);
       return;
     }
@@ -304,7 +304,7 @@ __global__ __launch_bounds__((NCW + NC + 2) * 64, 1) void mm_stream16_kernel(tam
     int slot = 0;
 #pragma unroll 1
     for (int s = 0; s < total_stages; ++s) {
-      __syncthreads();  // the partial sums of stage s - 1 and the bias of stage s are visible
+      sync_threads();  // the partial sums of stage s - 1 and the bias of stage s are visible
       if (s > 0) finish((s - 1) & 1);
       if (c_blk < blk0 || c_cg == n_cg) {
         if (c_cg == n_cg) c_cg = 0;
@@ -318,7 +318,7 @@ __global__ __launch_bounds__((NCW + NC + 2) * 64, 1) void mm_stream16_kernel(tam
       ++c_cg;
       slot = slot + 1 == S::RING ? 0 : slot + 1;
     }
-    __syncthreads();
+    sync_threads();
     finish((total_stages - 1) & 1);
     if (a.y_actual_scale) {
       // wave maximum, then one atomic per wave; positive floats order like their bit patterns
@@ -430,11 +430,11 @@ __global__ __launch_bounds__((NCW + NC + 2) * 64, 1) void mm_stream16_kernel(tam
       if (half == 0) wait_vmcnt<(S::RING - 2) * (NP + S::NSC)>();
       else if (half == 1) wait_vmcnt<(S::RING - 2) * (NP + 1)>();
       else wait_vmcnt<(S::RING - 2) * NP>();
-      __syncthreads();  // publishes stage s; every wave is done with stage s - 1, whose slot is refilled now
+      sync_threads();  // publishes stage s; every wave is done with stage s - 1, whose slot is refilled now
       issue(i_slot);
       i_slot = i_slot + 1 == S::RING ? 0 : i_slot + 1;
     }
-    __syncthreads();
+    sync_threads();
     wait_vmcnt<0>();  // the empty copies issued past the end still write (zeros) to LDS
   } else {
     // =========================================================================== compute waves
@@ -518,7 +518,7 @@ __global__ __launch_bounds__((NCW + NC + 2) * 64, 1) void mm_stream16_kernel(tam
     int slot = 0;
 #pragma unroll 1
     for (int s = 0; s < total_stages; ++s) {
-      __syncthreads();
+      sync_threads();
       if (c_blk < blk0 || c_cg == n_cg) {
         if (c_cg == n_cg) c_cg = 0;
         load_block(++c_blk);
@@ -547,7 +547,7 @@ __global__ __launch_bounds__((NCW + NC + 2) * 64, 1) void mm_stream16_kernel(tam
       *(f32x4_t *)(red + (s & 1) * (NCW * 256) + wave * 256 + lane * 4) = (acc0 + acc1) + (acc2 + acc3);
       slot = slot + 1 == S::RING ? 0 : slot + 1;
     }
-    __syncthreads();
+    sync_threads();
   }
 }
 

@@ -387,7 +387,7 @@ __global__ __launch_bounds__(256) void downcast_cols_tile_kernel(
       s_sc[cl * GT + gl] = (uint8_t)sbyte;
     }
   }
-  __syncthreads();
+  sync_threads();
   const int64_t n_g = G - gc * GT < GT ? G - gc * GT : GT;
   const int64_t n_c = nr - br * CW < CW ? nr - br * CW : CW;
   uint8_t *vbase = vals + b * vsb + br * CW * vsr + gc * GT * 16;
@@ -591,7 +591,7 @@ __global__ __launch_bounds__(256) void upcast_cols_tile_kernel(
       s_sc[c * GT + part] = sbase[(int64_t)c * csr + part];
     }
   }
-  __syncthreads();
+  sync_threads();
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
   const int cs = lane % 32;
   const int64_t col0 = br * CW + cs * NV;

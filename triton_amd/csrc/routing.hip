@@ -244,7 +244,7 @@ __global__ __launch_bounds__(1024) void hist_kernel(const void *__restrict__ ind
   extern __shared__ int32_t hist[];  // [CH][E]
   const int blk = blockIdx.x;
   for (int i = threadIdx.x; i < CH * E; i += 1024) hist[i] = 0;
-  __syncthreads();
+  sync_threads();
   const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
   for (int c = wave; c < CH; c += 16) {  // CH <= 16: one chunk per wave, so a workgroup waits for memory once
     int64_t i = ((int64_t)blk * CH + c) * 64 + lane;
@@ -253,7 +253,7 @@ __global__ __launch_bounds__(1024) void hist_kernel(const void *__restrict__ ind
     uint64_t same = same_id_mask(e, valid, nbits);
     if (valid && (same & lanemask_lt()) == 0) hist[c * E + e] = __popcll(same);
   }
-  __syncthreads();
+  sync_threads();
   for (int e = threadIdx.x; e < E; e += 1024) {
     int run = 0;
     for (int c = 0; c < CH; ++c) {
@@ -269,9 +269,9 @@ __global__ __launch_bounds__(1024) void hist_kernel(const void *__restrict__ ind
 TAMD_DEVICE int block_excl_scan_1024(int v, int &total, int *lds /* >= 17 ints */) {
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
   const int inc = wave_incl_scan(v);
-  __syncthreads();
+  sync_threads();
   if (lane == kWave - 1) lds[wave] = inc;
-  __syncthreads();
+  sync_threads();
   if (threadIdx.x == 0) {
     int run = 0;
     for (int w = 0; w < 16; ++w) {
@@ -281,7 +281,7 @@ TAMD_DEVICE int block_excl_scan_1024(int v, int &total, int *lds /* >= 17 ints *
     }
     lds[16] = run;
   }
-  __syncthreads();
+  sync_threads();
   total = lds[16];
   return inc - v + lds[wave];
 }
@@ -464,7 +464,7 @@ __global__ __launch_bounds__(1024) void ragged_kernel(const int32_t *__restrict_
                                                       int32_t *__restrict__ sched, int64_t sched_pitch, int max_blocks) {
   extern __shared__ int32_t tab[];  // [6][S + 1]
   ragged_scan_rows(sizes, S, tab, blockIdx.x == 0 ? offs : nullptr, offs_pitch);
-  __syncthreads();
+  sync_threads();
   const int64_t total = 5 * (int64_t)max_blocks;
   const int64_t per = (total + gridDim.x - 1) / gridDim.x;
   const int64_t first = per * blockIdx.x;
@@ -498,11 +498,11 @@ __global__ __launch_bounds__(1024) void scan_ragged_kernel(int E, int n_blocks, 
     const int ex = block_excl_scan_1024(run, total, scr);
     if (lead && e < E) col_offs[e] = carry + ex;
     carry += total;
-    __syncthreads();
+    sync_threads();
   }
   if (lead && threadIdx.x == 0) *n_valid = carry;
   ragged_scan_rows(csum, E, tab, lead ? offs : nullptr, offs_pitch);
-  __syncthreads();
+  sync_threads();
   const int64_t total_e = 5 * (int64_t)max_blocks;
   const int64_t per = (total_e + gridDim.x - 1) / gridDim.x;
   const int64_t first = per * blockIdx.x;
@@ -583,7 +583,7 @@ __global__ __launch_bounds__(1024) void order_scan_kernel(const void *__restrict
   }
   asm volatile("" : "+v"(ev), "+v"(gate));
   ev = has ? ev : -1;
-  __syncthreads();
+  sync_threads();
   // 2. totals per expert; counts of this wave's chunk
   for (int e = tid; e < E; e += 1024) {
     int all = 0, below = 0;
@@ -598,7 +598,7 @@ __global__ __launch_bounds__(1024) void order_scan_kernel(const void *__restrict
   const bool valid = ev >= 0 && ev < E;
   const uint64_t same = same_id_mask(ev, valid, nbits);
   if (valid && (same & lanemask_lt()) == 0) hist[wave * E + ev] = __popcll(same);
-  __syncthreads();
+  sync_threads();
   // 3. exclusive prefix over this block's chunks; the ragged tables (row 0: exclusive prefix over the experts)
   if (orders) {
     for (int e = tid; e < E; e += 1024) {
@@ -611,7 +611,7 @@ __global__ __launch_bounds__(1024) void order_scan_kernel(const void *__restrict
     }
   }
   ragged_scan_rows(tot, E, tab, blk == nbo ? offs : nullptr, offs_pitch);
-  __syncthreads();
+  sync_threads();
   if (orders) {
     // 4. placement
     const int nv = tab[E];
@@ -683,7 +683,7 @@ __global__ __launch_bounds__(TH) void topk_hist_kernel(const void *__restrict__ 
   for (int j = tid; j < CH * E; j += TH) hist[j] = 0;  // (the barrier below covers them)
   topk_row<DT, L, EPL>(x, x_stride, n_rows, E, k, 1, 0, y_vals, y_indx, k, bits, bits_stride_row, bits_stride_word,
                        row0 + tid / L, lidx - row0 * k);
-  __syncthreads();
+  sync_threads();
   for (int c = wave; c < CH; c += TH / kWave) {
     const int j = c * 64 + lane;  // entry of the block; its row exists or not
     const bool valid = row0 + j / k < n_rows;
@@ -691,7 +691,7 @@ __global__ __launch_bounds__(TH) void topk_hist_kernel(const void *__restrict__ 
     const uint64_t same = same_id_mask(e, valid, nbits);
     if (valid && (same & lanemask_lt()) == 0) hist[c * E + e] = __popcll(same);
   }
-  __syncthreads();
+  sync_threads();
   for (int e = tid; e < E; e += TH) {
     int run = 0;
     for (int c = 0; c < CH; ++c) run += hist[c * E + e];
@@ -739,7 +739,7 @@ TAMD_DEVICE void meta_fused_body(int32_t *sm, bool zeroed, const int32_t *lidx, 
   const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
   if (!zeroed) {
     for (int i = tid; i < NC * E; i += 1024) hist[i] = 0;
-    __syncthreads();
+    sync_threads();
   }
   // 1. per-chunk histogram.  A wave takes its chunks eight at a time so that eight index loads are in
   // flight together (one workgroup has nothing else to hide their latency with).
@@ -768,7 +768,7 @@ TAMD_DEVICE void meta_fused_body(int32_t *sm, bool zeroed, const int32_t *lidx, 
       if (valid && (same & lanemask_lt()) == 0) hist[c * E + e] = __popcll(same);
     }
   }
-  __syncthreads();
+  sync_threads();
   // 2. exclusive prefix over chunks for every expert: a few chunks in one go, else P chunk ranges per expert in two passes
   const int per = (NC + P - 1) / P;
   if (NC <= 8) {
@@ -789,7 +789,7 @@ TAMD_DEVICE void meta_fused_body(int32_t *sm, bool zeroed, const int32_t *lidx, 
     for (int c = part * per; c < NC && c < (part + 1) * per; ++c) run += hist[c * E + e];
     psum[part * E + e] = run;
   }
-  __syncthreads();
+  sync_threads();
   for (int t = tid; t < P * E; t += 1024) {
     const int part = t / E, e = t - part * E;
     int run = 0;
@@ -805,10 +805,10 @@ TAMD_DEVICE void meta_fused_body(int32_t *sm, bool zeroed, const int32_t *lidx, 
     }
   }
   }
-  __syncthreads();
+  sync_threads();
   // 3. ragged tables of the histogram; the first one is the exclusive prefix over experts that places the entries
   ragged_scan_rows(csum, E, tab, offs, offs_pitch);
-  __syncthreads();
+  sync_threads();
   const int32_t *coff = tab;
   const int nv = tab[E];
   // 4. placement
@@ -894,7 +894,7 @@ __global__ __launch_bounds__(1024) void routing_fused_kernel(const void *__restr
   for (int row0 = (int)(threadIdx.x / kWave) * (kWave / L), wave0 = row0; row0 < n_rows; row0 += ROWS)
     topk_row<DT, L, EPL>(x, x_stride, n_rows, E, k, 1, 0, y_vals, y_indx, k, bits, bits_stride_row, bits_stride_word,
                          (int64_t)(row0 - wave0) + threadIdx.x / L, lidx, lgate);
-  __syncthreads();
+  sync_threads();
   meta_fused_body(meta, true, lidx, lgate, nullptr, 0, n, E, k, nbits, NC, P, col_sum, col_sorted, row_sorted, gather, offs,
                   offs_pitch, sched, sched_pitch, max_blocks, gates);
 }
