@@ -319,7 +319,7 @@ TAMD_DEVICE v4i_t make_rsrc(const void *base, uint32_t num_records) {
 constexpr int A_ROW_BYTES = 128;       // LDS bytes per activation row per stage (64 K of 16-bit values)
 constexpr int B_BYTES = 4 * 64 * 64;   // 4 waves x 64 columns x 64 bytes (128 K of fp4)
 // LDS of the K pipeline.  Row blocks of 128: two activation stages, one weight stage (4 KB per wave), the e8m0 scales
-// of the whole tile staged once.
+// of the whole tile staged once.  Row blocks of at most 32 (KS = 1): the counted waits and stages of one of two K groups.
 // K groups (KS = 2 or 4, row blocks of at most 32 rows): KS groups of four waves share a tile, each taking a contiguous part of
 // K through a pipeline of its own with counted waits, three or four activation stages and one or two weight stages; their
 // partial sums meet in LDS.  A problem with fewer tiles than the part has CUs is bound by what one wave per SIMD can issue (a
@@ -330,8 +330,9 @@ struct PipeShape {
 };
 constexpr PipeShape pipe_shape(int lds_rows, int ks = 1) {
   PipeShape p{};
-  p.da = ks == 1 ? 2 : (ks == 4 ? 3 : 4);
-  p.db = ks == 2 ? 2 : 1;
+  const bool deep = ks == 2 || (ks == 1 && lds_rows <= 32);
+  p.da = deep ? 4 : (ks == 4 ? 3 : 2);
+  p.db = deep ? 2 : 1;
   p.bytes = p.da * lds_rows * 128 + p.db * B_BYTES;
   return p;
 }
@@ -806,8 +807,8 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
   constexpr int ESZ = 2;                      // bytes per activation element
   constexpr int KA = A_ROW_BYTES / ESZ;       // K per activation stage
   constexpr int A_STAGE = LDS_ROWS * A_ROW_BYTES;
-  constexpr bool DEEP = KS > 1;               // counted waits
-  static_assert(KS == 1 || (SC_LDS && NFR == 1 && (KS == 2 || KS == 4)), "K groups: scales in LDS, one row fragment");
+  constexpr bool DEEP = KS > 1 || LDS_ROWS <= 32;   // counted waits
+  static_assert(!DEEP || (SC_LDS && NFR == 1 && (KS == 1 || KS == 2 || KS == 4)), "counted waits: scales in LDS, one row fragment");
   constexpr PipeShape PS = pipe_shape(LDS_ROWS, KS);
   constexpr int DA = PS.da, DB = PS.db;
   auto a_slot = [](int it) { return DA == 2 ? (it & 1) : it % DA; };
@@ -1219,6 +1220,21 @@ int launch_x16_act(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
           ks == 4 ? mm_x16_mxfp4_kgroups_kernel<XDT, BM, ACT, 4> : mm_x16_mxfp4_kgroups_kernel<XDT, BM, ACT, 2>;
       if (int rc = raise_lds_limit_once((const void *)kk)) return rc;
       kk<<<dim3((unsigned)launch), 256 * ks, pipe + sc_bytes, st>>>(a, grid_n, total, (int)group_m);
+      return launch_status();
+    }
+  }
+  if constexpr (BM <= 32) {
+    // Weights of slices of one row block whose columns do not start on 64 bytes: pieces of 64 bytes of a column, two and more stages
+    // ahead, instead of launch_mx's pieces of 128.  The other way round where columns are aligned, where slices share their weights'
+    // lines between row blocks, with pre-shuffled scales, and for short K (953 rows of 64 slices, 2496 x 3552: 77 us against 104, pitch padded to 64 bytes 81
+    // against 77; 161 x 4 of 60, 3776 x 5488: 182 against 242; 1159 of 60, 5024 x 1616: 78 against 91; 157 x 2 of 16, 992 x 1392 11.5
+    // against 10.7).
+    constexpr int PIPE_BYTES = pipe_shape(LDS_ROWS).bytes;
+    if (a.block_schedule && rows_per_slice <= LDS_ROWS && a.w_layout != TAMD_W_CDNA4_BLOCKS && a.w_stride_n % 64 != 0 && a.K > 1024 &&
+        !cdna4 && dense_sc && PIPE_BYTES + sc_bytes <= 156 * 1024) {
+      auto kern = mm_x16_mxfp4_kernel<XDT, BM, ACT, true>;
+      if (int rc = raise_lds_limit_once((const void *)kern)) return rc;
+      kern<<<dim3((unsigned)launch), 256, PIPE_BYTES + sc_bytes, st>>>(a, grid_n, total, (int)group_m);
       return launch_status();
     }
   }
