@@ -353,7 +353,14 @@ int launch_mx(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
   group_m = group_m < 1 ? 1 : (group_m > 16 ? 16 : group_m);
   auto kern = mm_mx_kernel<XDT, BM, ACT>;
   if (int rc = raise_lds_limit_once((const void *)kern)) return rc;
-  kern<<<dim3((unsigned)launch), 256, (MxShape<XDT, BM>::lds(a.w_layout == TAMD_W_CDNA4_BLOCKS)), st>>>(a, grid_n, total, (int)(counts_live_blocks(a) ? -group_m : group_m));
+  const bool blocks = a.w_layout == TAMD_W_CDNA4_BLOCKS;
+  size_t lds_bytes = MxShape<XDT, BM>::lds(blocks);
+  // Columns that do not start on 64 bytes: a line that two pieces of a column share is read for each, a stage or two apart, and with
+  // three workgroups per CU an XCD's L2 has lost it by then (3 x 32 CUs x 256 columns, requested and requested next).  Two per CU from K
+  // 1920 on, ragged: 120 x 4 packed rows of 60 slices, 2368 x 3584 80 -> 71 us, 512 x 2 of 128, 3744 x 2176 193 -> 168, fp8 184 -> 172;
+  // 320 of 64, 1760 x 2352 40.5 -> 42.2, 64 x 4 of 128, 704 x 1536 18.8 -> 20.
+  if (BM <= 32 && a.block_schedule && !blocks && a.w_stride_n % 64 != 0 && a.K >= 1920 && lds_bytes < 56 * 1024) lds_bytes = 56 * 1024;
+  kern<<<dim3((unsigned)launch), 256, lds_bytes, st>>>(a, grid_n, total, (int)(counts_live_blocks(a) ? -group_m : group_m));
   return launch_status();
 }
 
