@@ -282,12 +282,13 @@ def test_blocks_of_16_only_where_they_stream():
     assert OF.tiles_block_m(32, 60, 512, 1280, 3, None, True, False, False) == 16
 
 
-def dense_block_m(M, N, K, x, w, along_n=False, cus=256, batch=1):
+def dense_block_m(M, N, K, x, w, along_n=False, cus=256, batch=1, blocks=False):
     import ctypes
     from triton_amd import _lib, _native
     bag = _lib.MatmulArgBag()
     bag.M, bag.N, bag.K, bag.n_experts, bag.x_dtype, bag.w_dtype = M, N, K, batch, getattr(_lib, x), getattr(_lib, w)
     bag.w_stride_k, bag.w_stride_n = (N, 1) if along_n else (1, K)
+    bag.w_layout = _lib.W_CDNA4_BLOCKS if blocks else _lib.W_STRIDED
     packed = bag.pack()
     return _native.dense_block_m(ctypes.addressof(packed), cus)
 
@@ -301,3 +302,20 @@ def test_dense_blocks_of_weights_along_n(M, N, K, block_m):
     of many, so rounds count and rows hardly do (sizes timed with every block)."""
     assert dense_block_m(M, N, K, "BF16", "BF16", along_n=True) == block_m
     assert dense_block_m(M, N, K, "F16", "F16", along_n=True) == block_m
+
+
+@pytest.mark.parametrize("M,N,K,rows,block_m", [
+    (16384, 2880, 2880, "BF16", 128), (14716, 8144, 2080, "BF16", 128), (4096, 8192, 8192, "BF16", 64), (9960, 2784, 5984, "BF16", 64),
+    (8192, 5760, 2880, "FP8_E4M3", 128), (16384, 1024, 8192, "FP8_E4M3", 128), (1486, 3064, 5376, "FP8_E4M3", 64),
+    (4122, 3152, 7808, "MXFP4", 128), (9652, 1320, 2144, "MXFP4", 128), (256, 4096, 2048, "BF16", 32), (64, 512, 576, "MXFP4", 32),
+])
+def test_dense_blocks_of_mxfp4_weights(M, N, K, rows, block_m):
+    """Products of many rounds in blocks of 128, except 16-bit rows whose scales such a block does not have in LDS (sizes timed with every
+    block)."""
+    assert dense_block_m(M, N, K, rows, "MXFP4") == block_m
+    assert dense_block_m(M, N, K, rows, "MXFP4", blocks=True) == block_m
+
+
+def test_dense_blocks_of_few_rounds_in_the_block_layout():
+    assert dense_block_m(3337, 4768, 608, "BF16", "MXFP4", blocks=True) == 64
+    assert dense_block_m(3337, 4768, 608, "BF16", "MXFP4") == 128

@@ -46,20 +46,33 @@ inline bool blocks_of_16_stream(tamd_matmul_args a) {
 }
 
 // Row block size of a dense / batched problem: the block whose tiles take the fewest rounds over the CUs, weighted with what a
-// tile of it takes.  MXFP4 weights: one and a half tiles per CU (fp8 and packed rows one and a quarter) run at the speed of one, a tile of 64 or 32
-// rows takes 0.45 or 0.35 of one of 128.  Kernels for operands of one type hold one tile per CU: 0.6 and 0.45 where the weights are
-// contiguous along K, 0.8 and 0.76 where they are contiguous along N (the LDS reads of the weights do not follow the rows).
-// (Fitted to products timed with every block.  800 of 1 to 4096 rows, against the largest block that gave every CU a tile: one type along K 9 %
-// faster in the mean -- 2000 rows of K 2000 and N 1600 two rounds of 64 rows instead of one of 128 on half the CUs, up to 1.7 times --,
-// MXFP4 2.5 %, none slower by more than 5 %.  150 of 16 to 16384 rows along N: 0.7 % slower than the best block of each
-// in the mean, 12 % with the MXFP4 figures; 3943 x 6144 x 7464 815 us in blocks of 64, 471 in blocks of 128, 5749 x 2432 x 512 68 in
-// blocks of 32, 39 in blocks of 64.)
+// tile of it takes, of one of 128 rows: `weight` (in percent) for 64 and 32 rows, `slots` tiles at the speed of one round.
+// Fitted to products timed with every block (mean and worst time against the best block of each):
+//   16-bit rows x MXFP4, 130 of 64 to 16384 rows: one and a half tiles per CU, 0.45 and 0.35; from K 3072 down, where a block of 128 has its scales in
+//     LDS, one per CU, 0.58 and 0.4 for strided weights and from four rounds on.  1.009, 1.14; with the first figures for all 1.019,
+//     1.23 (14716 x 2080 x 8144 481 us in blocks of 64, 413 of 128; block layout, 16384 x 2880 x 2880 232 and 217, 3337 x 608 x 4768 24 and
+//     31), with the largest block that gives every CU a tile 1.041, 1.47;
+//   fp8 x MXFP4, the same: one and three quarters, 0.68 and 0.4.  1.009, 1.18 (the figures of 16-bit rows 1.039, 1.24: 8192 x 2880 x
+//     5760 131 us in blocks of 64, 118 of 128; the largest block 1.011, 1.19);
+//   packed rows, the same: one, 0.58 and 0.4.  1.014, 1.15 (1.037, 1.27: 4122 x 7808 x 3152 119 us, 90; 1.028, 1.24);
+//   one type along K, 800 of 1 to 4096 rows: one, 0.6 and 0.45, 9 % faster in the mean than the largest block (2000 rows of K 2000 and N 1600
+//     two rounds of 64 rows instead of one of 128 on half the CUs, up to 1.7 times);
+//   one type along N, 150 of 16 to 16384 rows: one, 0.8 and 0.76 (the LDS reads of the weights do not follow the rows).  1.007; 3943 x 6144 x 7464
+//     815 us in blocks of 64, 471 of 128, 5749 x 2432 x 512 68 of 32, 39 of 64.
 inline int dense_block_m(const tamd_matmul_args &a, int cus) {
   const bool x16 = a.x_dtype == TAMD_BF16 || a.x_dtype == TAMD_F16, mxfp4 = a.w_dtype == TAMD_MXFP4;
   const bool along_n = !mxfp4 && a.w_stride_k != 1;
-  const int64_t cols = (int64_t)((a.N + 255) / 256) * a.n_experts, slots = !mxfp4 ? cus : (x16 ? cus * 3 / 2 : cus * 5 / 4);
+  const int64_t cols = (int64_t)((a.N + 255) / 256) * a.n_experts;
+  int slots = cus, w64 = 58, w32 = 40;
+  if (!mxfp4) {
+    w64 = along_n ? 80 : 60, w32 = along_n ? 76 : 45;
+  } else if (x16 && (a.K > 3072 || (a.w_layout == TAMD_W_CDNA4_BLOCKS && (a.M + 127) / 128 * cols < 4 * (int64_t)cus))) {
+    slots = cus * 3 / 2, w64 = 45, w32 = 35;
+  } else if (!x16 && a.x_dtype != TAMD_MXFP4) {
+    slots = cus * 7 / 4, w64 = 68, w32 = 40;
+  }
   const int extra = x16 && !along_n ? 32 : 0;   // remainder that a block of 128 absorbs
-  const int bm[3] = {128, 64, 32}, weight[3] = {100, mxfp4 ? 45 : (along_n ? 80 : 60), mxfp4 ? 35 : (along_n ? 76 : 45)};
+  const int bm[3] = {128, 64, 32}, weight[3] = {100, w64, w32};
   int best = 0;
   int64_t least = 0;
   for (int i = 0; i < 3; ++i) {
