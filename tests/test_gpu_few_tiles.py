@@ -46,14 +46,15 @@ def test_few_tiles(rows, E, N, kind, K, device):
 
 @pytest.mark.parametrize("byte", [0, 1, 238, 255])
 def test_special_block_scales(byte, device):
-    """Scale bytes of a row: blocks of 16 and of 32 rows agree (NaN for 255)."""
+    """Scale bytes of a row: blocks of 16 and of 32 rows agree (NaN for 255; 0 stands for 2^-127, against weights that make sums of it)."""
     torch.manual_seed(0)
     K, N = 640, 256
     a, s = downcast_to_mxfp(torch.randn(4, K, device=device), torch.float8_e4m3fn, axis=-1)
     s[1, 3] = byte
     s[2] = byte
     w, ws = downcast_to_mxfp(torch.randn(1, K, N, device=device), torch.uint8, axis=1)
-    ws = ws.clone() if byte != 238 else (ws.int() - 40).clamp(min=1).to(torch.uint8)   # (keeps the products finite)
+    codes = upcast_from_mxfp(w, torch.full_like(ws, 127), torch.float32, axis=1)
+    ws = (ws.int() - 40).clamp(min=1).to(torch.uint8) if byte == 238 else torch.full_like(ws, 230) if byte < 2 else ws.clone()   # (finite products)
     md = make_ragged_tensor_metadata(torch.tensor([4], dtype=torch.int32, device=device), 4)
     out = []
     for block_m in (16, 32):
@@ -63,6 +64,10 @@ def test_special_block_scales(byte, device):
             out.append(matmul(a, w, None, md, precision_config=pc))
     assert torch.equal(out[0].isnan(), out[1].isnan()) and bool(out[0][2].isnan().all()) == (byte == 255)
     torch.testing.assert_close(out[0], out[1], rtol=1e-3, atol=1e-3, equal_nan=True)
+    if byte < 2:   # (2^-13: see below; twice or half the scale, or none, is far off)
+        ref = scaled_sums(a, s, codes[0], ws[0])
+        for y in out:
+            assert float((y[2].double().cpu() - ref[2]).norm() / ref[2].norm()) <= 2.0 ** -13
 
 
 def scaled_sums(x8, xs, codes, ws):
