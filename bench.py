@@ -287,9 +287,9 @@ def run_dense(args, cfg, name):
     out["matmul_kernel_tflops"] = round(flops / (kernel_ms * 1e-3) / 1e12, 2)
     out["roofline"] = {"bound": "hbm", "achieved": round(gbs, 1), "peak": PEAK_HBM_GBS, "unit": "GB/s",
                        "frac": round(gbs / PEAK_HBM_GBS, 4), "traffic": None,
-                       # 161-256 rows: 32-row tiles shared by four K groups; fewer rows or a forced block of 16: streaming kernel
-                       "kernel": "mm_x16_mxfp4_kgroups_kernel" if 160 < M <= 256 and args.block_m in (0, None, 32)
-                       else ("mm_stream16_kernel" if args.block_m in (0, None, 16) else "mm_x16_mxfp4_kernel"),
+                       # up to 80 tiles of 32 rows, or a forced block of 16: streaming kernel; 32-row tiles are shared by K groups
+                       "kernel": {16: "mm_stream16_kernel", 32: "mm_x16_mxfp4_kgroups_kernel", 64: "mm_mx_kernel",
+                                  128: "mm_x16_mxfp4_kernel"}[args.block_m or (16 if -(-M // 32) * -(-N // 256) <= 80 else 32)],
                        "kernel_ms": round(kernel_ms, 4), "algorithmic_bytes": alg_bytes, "algorithmic_flops": flops,
                        "event_pair_ms": round(event_ms, 4),
                        "note": "kernel_ms: 16 calls replayed as one HIP graph, per call (event pairs around single calls "
@@ -382,6 +382,25 @@ def run_quant(args, cfg, name):
                            "kind": "port", "sample": f"oracle (numpy) on one expert's first 256 columns, {cpu_s:.2f} s"}
     out["parity"] = parity
     return out
+
+
+def product_kernel(args, rows, M, N, K, E):
+    """Name of the kernel that a ragged product of M `rows` ("bf16", "fp8", "mx8", "mx4") x MXFP4 weights takes here."""
+    from triton_amd.matmul_details.opt_flags import make_opt_flags, tiles_block_m
+    from triton_amd.tensor import RaggedTensorMetadata
+    streams = rows in ("bf16", "fp8") and K <= 4096 and N % 16 == 0    # (weights and scales are dense and aligned)
+    block_m = args.block_m or tiles_block_m(make_opt_flags(M, N, K, E, True, fp8_rows=rows != "bf16").block_m, M, N, K, E, None, True,
+                                            rows in ("fp8", "mx8"), not streams)
+    if block_m == 16 and streams:
+        return "mm_stream16_kernel"
+    if rows != "bf16" or block_m == 64:
+        return "mm_mx_kernel"
+    if block_m == 128:
+        return "mm_x16_mxfp4_kernel"
+    if K > 1344 and RaggedTensorMetadata.n_blocks(E, M, block_m) * -(-N // 256) <= 256:
+        return "mm_x16_mxfp4_kgroups_kernel"
+    strided = args.value_layout == "strided" and args.scale_layout == "strided"
+    return "mm_x16_mxfp4_kernel" if strided and K // 2 % 64 and K > 1024 and M // E <= 32 else "mm_mx_kernel"
 
 
 def algorithmic_bytes(col_sum, T, k, K, N, act, x_row_bytes=None):
@@ -493,12 +512,12 @@ def run_fc2(args, cfg, name):
     if rows <= 16 * E:  # decode size: weight streaming, bound by HBM
         roof = dict(bound="hbm", achieved=round(gbs_kernel, 1), peak=PEAK_HBM_GBS, unit="GB/s",
                     frac=round(gbs_kernel / PEAK_HBM_GBS, 4), traffic=traffic, traffic_source=traffic_source,
-                    kernel="mm_stream16_kernel", kernel_ms=round(kernel_ms, 4), algorithmic_bytes=mm_bytes,
+                    kernel=product_kernel(args, "fp8", rows, N, K, E), kernel_ms=round(kernel_ms, 4), algorithmic_bytes=mm_bytes,
                     algorithmic_flops=flops)
     else:
         roof = dict(bound="mfma", achieved=round(tflops_kernel, 1), peak=PEAK_FP8_TFLOPS, unit="TFLOP/s",
                     frac=round(tflops_kernel / PEAK_FP8_TFLOPS, 4), traffic=traffic, traffic_source=traffic_source,
-                    kernel="mm_mx_kernel", kernel_ms=round(kernel_ms, 4), algorithmic_bytes=mm_bytes,
+                    kernel=product_kernel(args, "fp8", rows, N, K, E), kernel_ms=round(kernel_ms, 4), algorithmic_bytes=mm_bytes,
                     algorithmic_flops=flops, frac_of_mxfp4_peak=round(tflops_kernel / PEAK_MXFP4_TFLOPS, 4),
                     hbm_gbs=round(gbs_kernel, 1))
     combine_bytes = rows * N * 2 + T * N * 2
@@ -564,7 +583,7 @@ def run_fc1(args, cfg, name):
     constraints = {"block_m": args.block_m} if args.block_m else {}
     wq = weights_for_matmul(vals, args.value_layout)
 
-    mx4 = bool(cfg.get("mx4"))   # MXFP4 activations: packed e2m1 codes, widened (exactly) to fp8 inside matmul
+    mx4 = bool(cfg.get("mx4"))   # MXFP4 activations: packed e2m1 codes, multiplied as they are
     mx8 = bool(cfg.get("mx8")) or mx4
     x_store = torch.uint8 if mx4 else torch.float8_e4m3fn
     if mx8:
@@ -608,8 +627,7 @@ def run_fc1(args, cfg, name):
     tflops_step = flops / (ms_per_step * 1e-3) / 1e12
     tflops_kernel = flops / (kernel_ms * 1e-3) / 1e12
     gbs_kernel = abytes / (kernel_ms * 1e-3) / 1e9
-    # the operands' own peak decides which roofline binds (MXFP4 x MXFP4: 10.1 PFLOP/s, so the bytes bind); the
-    # kernel multiplies widened fp8 values either way
+    # the operands' own peak decides which roofline binds (MXFP4 x MXFP4: 10.1 PFLOP/s, so the bytes bind)
     peak_mfma = PEAK_MXFP4_TFLOPS if mx4 else PEAK_FP8_TFLOPS if mx8 else PEAK_BF16_TFLOPS
     hbm_bound = (abytes / (PEAK_HBM_GBS * 1e9)) > (flops / (peak_mfma * 1e12))
     traffic, traffic_source = measured_traffic(name)
@@ -619,18 +637,16 @@ def run_fc1(args, cfg, name):
     else:
         roof = dict(bound="mfma", achieved=round(tflops_kernel, 1), peak=peak_mfma, unit="TFLOP/s",
                     frac=round(tflops_kernel / peak_mfma, 4), traffic=traffic, traffic_source=traffic_source)
-    # row blocks of 16 (few rows per expert) run the weight-streaming kernel, everything else the tiled one
-    roof["kernel"] = "mm_stream16_kernel" if rows <= 16 * E else ("mm_mx_kernel" if mx8 else "mm_x16_mxfp4_kernel")
+    roof["kernel"] = product_kernel(args, "mx4" if mx4 else "mx8" if mx8 else "bf16", rows, N, K, E)
     if mx4:
-        roof["kernel"] = "widen_e2m1_rows_kernel + " + roof["kernel"]
         roof["frac_of_fp8_mfma_peak"] = round(tflops_kernel / PEAK_FP8_TFLOPS, 4)
     roof["kernel_ms"] = round(kernel_ms, 4)
     roof["algorithmic_bytes"] = abytes
     roof["algorithmic_flops"] = flops
     roof["frac_of_mxfp4_peak"] = round(tflops_kernel / PEAK_MXFP4_TFLOPS, 4)
     roof["hbm_gbs"] = round(gbs_kernel, 1)
-    if rows > 16 * E:
-        # the tiled kernel computes whole 32-row MFMA fragments: rows of the ragged experts rounded up to 32 are what
+    if roof["kernel"] != "mm_stream16_kernel":
+        # the tiled kernels compute whole 32-row MFMA fragments: rows of the ragged experts rounded up to 32 are what
         # the matrix cores actually run (the share that is padding is the price of the ragged row counts)
         issued_rows = int(((col_sum + 31) // 32 * 32).sum())
         roof["mfma_rows_issued"] = issued_rows
