@@ -1226,8 +1226,8 @@ int launch_x16_act(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
   if constexpr (BM <= 32) {
     // Weights of slices of one row block whose columns do not start on 64 bytes: pieces of 64 bytes of a column, two and more stages
     // ahead, instead of launch_mx's pieces of 128.  The other way round where columns are aligned, where slices share their weights'
-    // lines between row blocks, with pre-shuffled scales, and for short K (953 rows of 64 slices, 2496 x 3552: 77 us against 104, pitch padded to 64 bytes 81
-    // against 77; 161 x 4 of 60, 3776 x 5488: 182 against 242; 1159 of 60, 5024 x 1616: 78 against 91; 157 x 2 of 16, 992 x 1392 11.5
+    // lines between row blocks, with pre-shuffled scales, and for short K (953 rows of 64 slices,
+    // 2496 x 3552: 77 us against 104; 539 x 2 of 60, 1024 x 5488, aligned: 48 against 38; 161 x 4 of 60, 3776 x 5488: 182 against 242; 1159 of 60, 5024 x 1616: 78 against 91; 157 x 2 of 16, 992 x 1392 11.5
     // against 10.7).
     constexpr int PIPE_BYTES = pipe_shape(LDS_ROWS).bytes;
     if (a.block_schedule && rows_per_slice <= LDS_ROWS && a.w_layout != TAMD_W_CDNA4_BLOCKS && a.w_stride_n % 64 != 0 && a.K > 1024 &&

@@ -18,10 +18,10 @@
 // changed nothing).  Packed rows, against being widened to fp8 in front of the kernel: half the MFMA cycles, row copies and LDS reads,
 // no pass over the rows.
 // Before -> now, layers: packed rows, widening included, 2048 tokens, 128 experts (top-4) 531 -> 471 us, 2331 over 16 (top-8) 212 -> 177;
-// fp8 16384 over 32 1587 -> 1550, 13 over 64 (top-2) 34.3 -> 32.2, 509 over 128 647 -> 644; dense fp8, 3425 x 5600 x 2312
+// fp8 16384 over 32 1587 -> 1550, 13 over 64 (top-2) 34.3 -> 32.2, 509 over 128 the same; dense fp8, 3425 x 5600 x 2312
 // (strided scales) 104 -> 73, 2 x 3680 x 1336 19.4 -> 14.5, 158 x 640 x 1080 7.3 -> 6.6.
-// 16-bit rows in blocks of up to 64: a barrier per 128 K instead of 64, no scales in LDS, three workgroups per CU (blocks of 32: four) where
-// the kernel with deeper rings beside the tile's scales held one or two: 816 x 4960 x 2776 f16 62.3 -> 35.8 us, 2351 x 1664 x 6992
+// 16-bit rows in blocks of up to 64: a barrier per 128 K instead of 64, no scales in LDS, three workgroups per CU (blocks of 32: four; with strided
+// weights, which take twice the LDS, two and three) where the kernel with deeper rings beside the tile's scales held one or two: 816 x 4960 x 2776 f16 62.3 -> 35.8 us, 2351 x 1664 x 6992
 // 62 -> 55; 256 tokens over 16 experts, 3776 -> 1280, layer 74.9 -> 66.8.
 #pragma once
 #include "moe_matmul_impl.h"
@@ -54,7 +54,7 @@ struct MxShape {
   static constexpr bool PAIRS = BLOCKS == 1;                 // strided weights: 256 K at a time, every other stage
   static constexpr int b_wave(bool blocks) { return (PAIRS && !blocks ? 2 : BLOCKS) * 4096; }   // weight bytes of a wave
   static constexpr int lds(bool blocks) { return 2 * A_STAGE + 4 * b_wave(blocks); }
-  static constexpr int WGS = BM >= 128 ? 2 : (FP4 || X16 ? (BM == 64 ? 3 : 4) : (BM == 64 ? 2 : 3));   // workgroups per CU
+  static constexpr int WGS = BM >= 128 ? 2 : (FP4 || X16 ? (BM == 64 ? 3 : 4) : (BM == 64 ? 2 : 3));   // workgroups per CU (block layout)
   static_assert(!X16 || BM <= 64, "larger blocks of 16-bit rows: run_tile");
 };
 
@@ -325,6 +325,7 @@ __global__ __launch_bounds__(256, (MxShape<XDT, BM>::WGS)) void mm_mx_kernel(tam
                                                                            int group_m) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   typedef MxShape<XDT, BM> S;
+  static_assert(S::WGS * S::lds(true) <= 160 * 1024, "the workgroups that the registers are limited for fit a CU's LDS");
   Tile t;
   if (group_m < 0) {
     if (!locate_tile_live<BM, 0>(a, grid_n, -group_m, t)) return;

@@ -666,7 +666,7 @@ inline int launch_order_scan(const void *indx, int is16, int64_t n, int E, int C
 
 // First launch of the two, from the logits: the experts of TH / L rows per workgroup (their picked columns also go to
 // LDS) and the histogram of that block of CH = (TH / L) * k / 64 whole chunks.  A row is a chain of some 400 instructions, so
-// the workgroups are as small as whole chunks allow (4096 rows of 128, top-4, both launches: 13.3 us with 1024
+// the workgroups are as small as whole chunks allow (4096 rows of 128, top-4, both launches in a graph -- a call waits for the host --: 13.3 us with 1024
 // threads, 12.6 with 512; 1024 rows 12.4 and, with 256, 11.4).
 template <int DT, int L, int EPL, int TH>
 __global__ __launch_bounds__(TH) void topk_hist_kernel(const void *__restrict__ x, int64_t x_stride, int n_rows, int E,
