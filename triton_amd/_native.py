@@ -50,6 +50,7 @@ def _on_first_call(name):
     return call
 
 
-_FUNCTIONS = ("matmul", "routing", "view", "reduce", "downcast", "upcast", "choose_block_m", "blocks_of_16_stream", "dense_block_m")
+_FUNCTIONS = ("matmul", "routing", "view", "reduce", "downcast", "upcast", "choose_block_m", "blocks_of_16_stream", "dense_block_m",
+              "ring_rows")
 for _n in _FUNCTIONS:
     globals()[_n] = _on_first_call(_n)

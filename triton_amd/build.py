@@ -16,6 +16,7 @@ SOURCES = ["api.cpp", "mxfp.hip", "routing.hip", "elementwise.hip", "moe_matmul.
            "moe_matmul_fp8.hip", "moe_matmul_bf16_swiglu.hip", "moe_matmul_f16_swiglu.hip", "moe_matmul_fp8_swiglu.hip",
            "moe_matmul_fp8e5m2.hip", "moe_matmul_fp8e5m2_swiglu.hip", "moe_matmul_stream_fp8e5m2.hip",
            "moe_matmul_stream_bf16.hip", "moe_matmul_stream_f16.hip", "moe_matmul_stream_fp8.hip",
+           "moe_matmul_ring_bf16.hip", "moe_matmul_ring_f16.hip", "moe_matmul_ring_fp8.hip", "moe_matmul_ring_fp4.hip",
            "moe_matmul_fp4.hip", "moe_matmul_fp4_swiglu.hip",
            "moe_matmul_w16_bf16.hip", "moe_matmul_w16_f16.hip",
            "moe_matmul_kk_bf16.hip", "moe_matmul_kk_f16.hip", "moe_matmul_kk_fp8.hip"]
@@ -109,7 +110,7 @@ def build(force=True, verbose=False):
     srcs = [s for s in SOURCES if os.path.exists(os.path.join(CSRC, s))]
     objs = [os.path.join(objdir, os.path.splitext(s)[0] + ".o") for s in srcs]
     deps = [os.path.join(CSRC, "common.h"), os.path.join(CSRC, "moe_matmul_impl.h"), os.path.join(CSRC, "moe_matmul_stream.h"), os.path.join(CSRC, "moe_matmul_dense.h"),
-            os.path.join(CSRC, "moe_matmul_kk.h"), os.path.join(CSRC, "moe_matmul_mx.h"), os.path.join(CSRC, "tile_rules.h"),
+            os.path.join(CSRC, "moe_matmul_kk.h"), os.path.join(CSRC, "moe_matmul_mx.h"), os.path.join(CSRC, "moe_matmul_ring.h"), os.path.join(CSRC, "tile_rules.h"),
             os.path.join(HERE, "..", "include", "triton_amd.h")]
     todo = []
     for s, o in zip(srcs, objs):

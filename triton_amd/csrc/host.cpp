@@ -699,6 +699,16 @@ PyObject *py_dense_block_m(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
   });
 }
 
+// (address of a tamd_matmul_args, compute units): the row block of the persistent kernel for few rows per slice, or 0.
+PyObject *py_ring_rows(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
+  return covered([&]() -> PyObject * {
+    need(nargs == 2);
+    tamd_matmul_args a;
+    std::memcpy(&a, (const void *)(intptr_t)as_int(v[0]), sizeof a);
+    return PyLong_FromLong(tamd::ring_rows(a, (int)as_int(v[1])));
+  });
+}
+
 // (addresses of the C ABI functions by name, Tensor, CDNA4MXValueLayout, CDNA4MXScaleLayout, FP4, constraints ContextVar,
 //  flags ContextVar)
 PyObject *py_init(PyObject *, PyObject *args) {
@@ -742,6 +752,7 @@ PyMethodDef methods[] = {{"init", py_init, METH_VARARGS, nullptr},
                          {"choose_block_m", TAMD_FAST(py_choose_block_m)},
                          {"blocks_of_16_stream", TAMD_FAST(py_blocks_of_16_stream)},
                          {"dense_block_m", TAMD_FAST(py_dense_block_m)},
+                         {"ring_rows", TAMD_FAST(py_ring_rows)},
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

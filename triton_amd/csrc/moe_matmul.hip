@@ -16,6 +16,10 @@ int dispatch_mm_w16_bf16(const tamd_matmul_args &a, int block_m, int grid_m, hip
 int dispatch_mm_w16_f16(const tamd_matmul_args &a, int block_m, int grid_m, hipStream_t st);
 int dispatch_mm_kk_fp8e4m3(const tamd_matmul_args &a, int block_m, int grid_m, hipStream_t st);
 int dispatch_mm_kk_fp8e5m2(const tamd_matmul_args &a, int block_m, int grid_m, hipStream_t st);
+int ring_mm_bf16(const tamd_matmul_args &a, int rows, hipStream_t st);
+int ring_mm_f16(const tamd_matmul_args &a, int rows, hipStream_t st);
+int ring_mm_fp8e4m3(const tamd_matmul_args &a, int rows, hipStream_t st);
+int ring_mm_fp4(const tamd_matmul_args &a, int rows, hipStream_t st);
 }  // namespace tamd
 
 using namespace tamd;
@@ -83,6 +87,13 @@ extern "C" int tamd_matmul_sized(const tamd_matmul_args *args, size_t args_size,
       // 0: the dispatcher chooses (it knows which kernels apply)
       block_m = a.force_variant;
       grid_m = block_m ? ((a.M + block_m - 1) / block_m) * a.n_experts : 0;
+    }
+    int cus = 0;
+    if (int rc = cu_count(cus)) return rc;
+    if (const int rows = ring_rows(a, cus)) {
+      if (x4) return ring_mm_fp4(a, rows, st);
+      if (x8) return ring_mm_fp8e4m3(a, rows, st);
+      return a.x_dtype == TAMD_BF16 ? ring_mm_bf16(a, rows, st) : ring_mm_f16(a, rows, st);
     }
     if (x4) return dispatch_mm_fp4(a, block_m, grid_m, st);
     if (a.x_dtype == TAMD_BF16) return dispatch_mm_bf16(a, block_m, grid_m, st);

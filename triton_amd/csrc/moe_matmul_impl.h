@@ -251,7 +251,8 @@ TAMD_DEVICE bool locate_tile_live(const tamd_matmul_args &a, int grid_n, int gro
 
 // What a row of x is below: the rows that a gathered index can name.  An index outside of them (-1) names none: the row is read as
 // zeros, by the buffer descriptors where the address leaves their 2 GB, and by this limit where loads have no descriptor.
-TAMD_DEVICE uint32_t gather_limit(const tamd_matmul_args &a) {
+template <typename Args>
+TAMD_DEVICE uint32_t gather_limit(const Args &a) {
   const int64_t rows = a.x_rows > 0 ? a.x_rows : (int64_t)a.M;
   return a.gather_indx && rows < 0x80000000ll ? (uint32_t)rows : 0x80000000u;
 }
@@ -297,6 +298,18 @@ TAMD_DEVICE void dma16_x4(v4i_t rsrc, uint32_t lds_addr, uint32_t voff, uint32_t
       "buffer_load_dwordx4 %1, %2, %3 offen offset:1024 lds\n\t"
       "buffer_load_dwordx4 %1, %2, %3 offen offset:2048 lds\n\t"
       "buffer_load_dwordx4 %1, %2, %3 offen offset:3072 lds"
+      :
+      : "s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(voff), "s"(rsrc), "s"(__builtin_amdgcn_readfirstlane(soff))
+      : "memory", "m0");
+}
+// The same for data that is read once (non-temporal).
+TAMD_DEVICE void dma16_x4_nt(v4i_t rsrc, uint32_t lds_addr, uint32_t voff, uint32_t soff) {
+  asm volatile(
+      "s_mov_b32 m0, %0\n\ts_nop 4\n\t"
+      "buffer_load_dwordx4 %1, %2, %3 offen nt lds\n\t"
+      "buffer_load_dwordx4 %1, %2, %3 offen offset:1024 nt lds\n\t"
+      "buffer_load_dwordx4 %1, %2, %3 offen offset:2048 nt lds\n\t"
+      "buffer_load_dwordx4 %1, %2, %3 offen offset:3072 nt lds"
       :
       : "s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(voff), "s"(rsrc), "s"(__builtin_amdgcn_readfirstlane(soff))
       : "memory", "m0");
@@ -389,8 +402,12 @@ TAMD_DEVICE void store_actual_scale(float *actual, uint32_t amax, float out_max,
 // scratch memory).
 // pairs: a lane's two outputs lie whole on one aligned word, which is stored at once (only read by the forms of one width;
 // the others are entered with such outputs).
+// ready: the operands whose table is written already, or null.  pace: called after every four rows of a lane.
 // Args: tamd_matmul_args, or the same structure read in place from the kernel-argument segment (see kernel_args_late).
 // tab: LDS that belongs to the wave alone, epilogue_table_bytes(NFR).
+struct NoPace {
+  TAMD_DEVICE void operator()() const {}
+};
 constexpr int epilogue_table_bytes(int nfr) { return nfr * 32 * 16; }
 // Maximum over a lane's aligned group of 32 / NO lanes: inside 16 lanes by moves in the register file (mirrored lanes
 // serve once the blocks of four and eight hold one value), across them through the LDS crossbar.
@@ -405,9 +422,71 @@ TAMD_DEVICE float group_max_lanes(float m) {
   return m;
 }
 
+// What the epilogue of a tile reads from memory, as it lies there: a lane's rows of the table (64 u + lane), its columns' bias, the
+// per-tensor scales.  Nothing is computed from the values where they are loaded, so that they may be requested long before.
+template <int NFR>
+struct EpilogueOperands {
+  static constexpr int PER_LANE = (NFR + 1) / 2;
+  int dst[PER_LANE];
+  float beta[PER_LANE], gamma[PER_LANE];
+  uint32_t bias[NF];
+  float x_scale, w_scale;
+};
+TAMD_DEVICE uint32_t load_any_bits(const void *p, int dt, int64_t i) {
+  return dt == TAMD_F32 ? ((const uint32_t *)p)[i] : (uint32_t)((const uint16_t *)p)[i];
+}
+TAMD_DEVICE float bits_of_type(uint32_t v, int dt) {
+  return dt == TAMD_F32 ? bits_to_f32(v) : (dt == TAMD_BF16 ? bf16_bits_to_f32(v) : f16_bits_to_f32(v));
+}
+template <int NFR, bool ROWSC, typename Args>
+TAMD_DEVICE void epilogue_operands(const Args &a, const Tile &t, EpilogueOperands<NFR> &o) {
+  const int wave = (threadIdx.x / kWave) & 3, lane = threadIdx.x % kWave;
+#pragma unroll
+  for (int u = 0; u < EpilogueOperands<NFR>::PER_LANE; ++u) {
+    const int r = u * kWave + lane;
+    const int erow = t.start_m + t.off_m + (r < t.rows ? r : t.rows - 1);  // expert-sorted row
+    o.dst[u] = a.scatter_indx ? a.scatter_indx[erow] : erow;
+    o.beta[u] = o.gamma[u] = 1.0f;
+    if constexpr (ROWSC) {
+      if (a.betas) o.beta[u] = a.betas[erow];
+      if (a.gammas) o.gamma[u] = a.gammas[erow];
+    }
+  }
+  const int col0 = t.n0 + wave * 64 + lane % 32 * NF, last = a.N - 1;
+#pragma unroll
+  for (int f = 0; f < NF; ++f)
+    o.bias[f] = a.bias ? load_any_bits(a.bias, a.bias_dtype, (int64_t)t.expert * a.bias_stride_e + (col0 + f < last ? col0 + f : last)) : 0u;
+  o.x_scale = a.x_scale ? *a.x_scale : 1.0f;
+  o.w_scale = a.w_scale ? *a.w_scale : 1.0f;
+}
+
+// The wave's row table: [rows] destinations (byte offsets into y, out of range for a row that is not stored), [rows] betas, [rows] gammas,
+// [rows] destinations of the scales (MXO).
+template <int NFR, int OSZ, bool ROWSC, bool MXO, typename Args>
+TAMD_DEVICE void epilogue_table(const Args &a, const Tile &t, const int *dsts, const float *betas, const float *gammas, uint8_t *tab) {
+  constexpr uint32_t kDrop = 0x80000000u;
+  const int lane = threadIdx.x % kWave;
+  uint32_t *tab_dst = (uint32_t *)tab;
+  float *tab_beta = (float *)tab + NFR * 32, *tab_gamma = (float *)tab + NFR * 64;
+#pragma unroll
+  for (int u = 0; u < (NFR + 1) / 2; ++u) {
+    const int r = u * kWave + lane, dst = dsts[u];
+    if (NFR % 2 == 0 || r < NFR * 32) {
+      const bool keep = r < t.rows && dst >= 0;
+      tab_dst[r] = keep ? (uint32_t)dst * (uint32_t)(a.y_stride_m * OSZ) : kDrop;
+      if constexpr (MXO) tab_dst[NFR * 96 + r] = keep ? (uint32_t)dst * (uint32_t)a.y_mx_stride_m : kDrop;
+      if constexpr (ROWSC) {
+        tab_beta[r] = betas[u];
+        tab_gamma[r] = gammas[u];
+      }
+    }
+  }
+}
+
 constexpr int kAny16 = 0x100, kAny8 = 0x101;
-template <int NFR, int ACT, int YDT, bool ROWSC, bool FLEX, bool MXO = false, typename Args = tamd_matmul_args>
-TAMD_DEVICE void tile_epilogue_t(const Args &a, const Tile &t, f32x16_t (&acc)[NFR][NF], uint8_t *tab, bool pairs = true) {
+template <int NFR, int ACT, int YDT, bool ROWSC, bool FLEX, bool MXO, typename Args, typename Pace>
+TAMD_DEVICE void tile_epilogue_t(const Args &a, const Tile &t, f32x16_t (&acc)[NFR][NF], uint8_t *tab, const EpilogueOperands<NFR> *ready,
+                                 Pace &pace, bool pairs = true) {
   const int wave = (threadIdx.x / kWave) & 3, lane = threadIdx.x % kWave;
   const int c32 = lane % 32, h = lane / 32;
   const int N = a.N;
@@ -420,39 +499,20 @@ TAMD_DEVICE void tile_epilogue_t(const Args &a, const Tile &t, f32x16_t (&acc)[N
   const int out_col0 = ACT == TAMD_ACT_SWIGLU ? col0 / 2 : col0;
   constexpr int osz = YDT == TAMD_F32 ? 4 : (is_fp8(YDT) || YDT == kAny8 ? 1 : 2);   // bytes per output
   if (t.n0 + wave * 64 >= N) return;
-  // ---- the wave's row table: [rows] destinations, [rows] betas, [rows] gammas, [rows] destinations of the scales (MXO)
   uint32_t *tab_dst = (uint32_t *)tab;
   float *tab_beta = (float *)tab + NFR * 32, *tab_gamma = (float *)tab + NFR * 64;
-#pragma unroll
-  for (int u = 0; u < (NFR + 1) / 2; ++u) {
-    const int r = u * kWave + lane;
-    if (NFR % 2 == 0 || r < NFR * 32) {
-      const int erow = t.start_m + t.off_m + (r < t.rows ? r : t.rows - 1);  // expert-sorted row
-      const int dst = a.scatter_indx ? a.scatter_indx[erow] : erow;
-      float beta = 1.0f, gamma = 1.0f;
-      if constexpr (ROWSC) {
-        if (a.betas) beta = a.betas[erow];
-        if (a.gammas) gamma = a.gammas[erow];
-      }
-      const bool keep = r < t.rows && dst >= 0;
-      tab_dst[r] = keep ? (uint32_t)dst * (uint32_t)(a.y_stride_m * osz) : kDrop;
-      if constexpr (MXO) tab_dst[NFR * 96 + r] = keep ? (uint32_t)dst * (uint32_t)a.y_mx_stride_m : kDrop;
-      if constexpr (ROWSC) {
-        tab_beta[r] = beta;
-        tab_gamma[r] = gamma;
-      }
-    }
+  EpilogueOperands<NFR> ops;
+  if (ready) {
+    ops = *ready;
+  } else {
+    epilogue_operands<NFR, ROWSC, Args>(a, t, ops);
+    epilogue_table<NFR, osz, ROWSC, MXO, Args>(a, t, ops.dst, ops.beta, ops.gamma, tab);
   }
-  float flex = 1.0f;
-  if (a.x_scale) flex *= *a.x_scale;
-  if (a.w_scale) flex *= *a.w_scale;
-  flex *= a.out_alpha;
+  const float flex = ops.x_scale * ops.w_scale * a.out_alpha;
   // without per-row factors bias * beta * out_alpha is one value per column
   float bias_a[NF];
 #pragma unroll
-  for (int f = 0; f < NF; ++f)
-    bias_a[f] = ((a.bias && col0 + f < N) ? load_any_f32(a.bias, a.bias_dtype, (int64_t)t.expert * a.bias_stride_e + col0 + f)
-                                          : 0.f) * a.out_alpha;
+  for (int f = 0; f < NF; ++f) bias_a[f] = (a.bias && col0 + f < N ? bits_of_type(ops.bias[f], a.bias_dtype) : 0.f) * a.out_alpha;
   const bool has_limit = a.act_has_limit != 0;
   // flexpoint output: scale by 1 / expected, optionally clamp, and track max|result| for the actual scale
   const float inv_expected = (FLEX && a.y_expected_scale) ? 1.0f / *a.y_expected_scale : 1.0f;
@@ -623,6 +683,7 @@ TAMD_DEVICE void tile_epilogue_t(const Args &a, const Tile &t, f32x16_t (&acc)[N
           for (int e = 0; e < 12; ++e) acc[i][f][e] = acc[i][f][e + 4];
       }
       __builtin_amdgcn_sched_barrier(0);
+      pace();
     }
   }
   if constexpr (FLEX) {
@@ -633,8 +694,8 @@ TAMD_DEVICE void tile_epilogue_t(const Args &a, const Tile &t, f32x16_t (&acc)[N
 // The general epilogue: any output type, alignment and size, every feature read at run time, stores through 64-bit
 // addresses.  A row fragment's accumulators are taken four at a time in a rolled loop and move up by four after each
 // step, so that the loop indexes registers with constants.
-template <int NFR, int ACT, typename Args>
-TAMD_DEVICE void tile_epilogue_general(const Args &a, const Tile &t, f32x16_t (&acc)[NFR][NF], uint8_t *tab) {
+template <int NFR, int ACT, typename Args, typename Pace>
+TAMD_DEVICE void tile_epilogue_general(const Args &a, const Tile &t, f32x16_t (&acc)[NFR][NF], uint8_t *tab, Pace &pace) {
   const int wave = (threadIdx.x / kWave) & 3, lane = threadIdx.x % kWave;
   const int c32 = lane % 32, h = lane / 32;
   const int N = a.N;
@@ -723,6 +784,7 @@ TAMD_DEVICE void tile_epilogue_general(const Args &a, const Tile &t, f32x16_t (&
     for (int f = 0; f < NF; ++f)
 #pragma unroll
       for (int j = 0; j < 12; ++j) acc[i][f][j] = acc[i][f][j + 4];
+    pace();
   }
   if (a.y_actual_scale) store_actual_scale(a.y_actual_scale, amax, out_max, lane);
 }
@@ -755,23 +817,24 @@ TAMD_DEVICE bool epilogue_is_regular(const Args &a) {
 // bf16 116 us against 88; bf16 rows, 5760 columns of float32 145 against 128, of e4m3 with a flexpoint scale 161 against 126.
 template <int NFR, int ACT, int FAST_YDT, bool FP8_ROWS, typename Args>
 TAMD_DEVICE void tile_epilogue(const Args &a, const Tile &t, f32x16_t (&acc)[NFR][NF], uint8_t *tab) {
+  const NoPace pace;
   const bool flexo = a.y_expected_scale != nullptr || a.y_actual_scale != nullptr;
   const bool spans = epilogue_spans_32_bits(a), pairs = epilogue_stores_pairs<ACT>(a);
   if (spans && pairs && a.y_mx_scale) {  // always e4m3 values and no flexpoint output (checked by the entry point)
-    tile_epilogue_t<NFR, ACT, TAMD_FP8_E4M3, true, false, true, Args>(a, t, acc, tab);
+    tile_epilogue_t<NFR, ACT, TAMD_FP8_E4M3, true, false, true, Args>(a, t, acc, tab, nullptr, pace);
   } else if (!spans || a.y_mx_scale) {
-    tile_epilogue_general<NFR, ACT, Args>(a, t, acc, tab);
+    tile_epilogue_general<NFR, ACT, Args>(a, t, acc, tab, pace);
   } else if (FP8_ROWS && pairs && a.y_dtype == TAMD_FP8_E4M3) {
-    if constexpr (FP8_ROWS) tile_epilogue_t<NFR, ACT, TAMD_FP8_E4M3, true, true, false, Args>(a, t, acc, tab);
+    if constexpr (FP8_ROWS) tile_epilogue_t<NFR, ACT, TAMD_FP8_E4M3, true, true, false, Args>(a, t, acc, tab, nullptr, pace);
   } else if (pairs && a.y_dtype == FAST_YDT && !flexo) {
-    if (a.betas || a.gammas) tile_epilogue_t<NFR, ACT, FAST_YDT, true, false, false, Args>(a, t, acc, tab);
-    else tile_epilogue_t<NFR, ACT, FAST_YDT, false, false, false, Args>(a, t, acc, tab);
+    if (a.betas || a.gammas) tile_epilogue_t<NFR, ACT, FAST_YDT, true, false, false, Args>(a, t, acc, tab, nullptr, pace);
+    else tile_epilogue_t<NFR, ACT, FAST_YDT, false, false, false, Args>(a, t, acc, tab, nullptr, pace);
   } else if (a.y_dtype == TAMD_F32) {
-    tile_epilogue_t<NFR, ACT, TAMD_F32, true, true, false, Args>(a, t, acc, tab, pairs);
+    tile_epilogue_t<NFR, ACT, TAMD_F32, true, true, false, Args>(a, t, acc, tab, nullptr, pace, pairs);
   } else if (is_fp8(a.y_dtype)) {
-    tile_epilogue_t<NFR, ACT, kAny8, true, true, false, Args>(a, t, acc, tab, pairs);
+    tile_epilogue_t<NFR, ACT, kAny8, true, true, false, Args>(a, t, acc, tab, nullptr, pace, pairs);
   } else {
-    tile_epilogue_t<NFR, ACT, kAny16, true, true, false, Args>(a, t, acc, tab, pairs);
+    tile_epilogue_t<NFR, ACT, kAny16, true, true, false, Args>(a, t, acc, tab, nullptr, pace, pairs);
   }
 }
 

@@ -1,6 +1,7 @@
 // Which kernel and which row block a product takes: rules on the arguments alone, shared by the kernels' launchers and the host path
 // (no HIP here).
 #pragma once
+#include <math.h>
 #include <stddef.h>
 #include <stdint.h>
 
@@ -43,6 +44,62 @@ inline bool stream16_applicable(const tamd_matmul_args &a) {
 inline bool blocks_of_16_stream(tamd_matmul_args a) {
   drop_unused_pitches(a);
   return a.w_dtype == TAMD_MXFP4 && stream16_applicable(a);
+}
+
+inline int64_t output_size(int dtype) { return dtype == TAMD_F32 ? 4 : (dtype == TAMD_FP8_E4M3 || dtype == TAMD_FP8_E5M2 ? 1 : 2); }
+
+// What the persistent kernel of few rows per slice (moe_matmul_ring.h) covers: ragged problems with weights in 4 KB blocks, pre-shuffled scales, outputs of
+// the usual type in pairs of columns that 32-bit offsets reach.
+inline bool ring_applicable(const tamd_matmul_args &a) {
+  if (!a.block_schedule || a.w_layout != TAMD_W_CDNA4_BLOCKS || a.w_mx_layout != TAMD_SCALE_CDNA4) return false;
+  if (a.n_experts > 256 || (a.N + 63) / 64 > 0x8000 || ((int64_t)a.M + a.n_experts) * ((a.N + 63) / 64) > 0x7FFFFFF0) return false;
+  const bool x16 = a.x_dtype == TAMD_BF16 || a.x_dtype == TAMD_F16, sw = a.activation == TAMD_ACT_SWIGLU;
+  if (!x16 && a.x_dtype != TAMD_FP8_E4M3 && a.x_dtype != TAMD_MXFP4) return false;
+  const int64_t lim = 0x7FFFFF00, size = output_size(a.y_dtype);
+  if (a.y_rows <= 0 || a.y_stride_m < 0 || a.y_rows * a.y_stride_m * size >= lim) return false;
+  if (a.y_mx_scale && a.y_rows * a.y_mx_stride_m >= lim) return false;
+  if (!sw && (((a.N | (int)a.y_stride_m) & 1) != 0 || !aligned(a.y, 2 * (size_t)size))) return false;
+  const bool flex = a.y_expected_scale || a.y_actual_scale;
+  if (x16) return !a.y_mx_scale && !flex && a.y_dtype == a.x_dtype;
+  return a.y_dtype == TAMD_FP8_E4M3 || (a.y_dtype == TAMD_BF16 && !flex);
+}
+
+// Rows of the persistent kernel's blocks, 0 where another kernel is the faster (or the only one).  The block is the smallest that covers a slice's mean size and
+// two standard deviations, up to 96; the lines between the kernels are in tiles per CU, one row block for every slice that has rows (on the
+// average of random choices).  Up to one, a tile is alone on its CU and wins by its depth; just above, the second round is nearly empty, where smaller tiles, three
+// and four to a CU, lose less; from two on the rounds fill.  Below K 1024 the loop over K is too short to hide the tile before, unless there is none.
+// 16-bit rows of up to 16 per slice are the streaming kernel's, except where its parts of K (multiples of 1024) fit badly; their larger
+// blocks are bound by the conversion of the codes, as in the other kernels.
+// From 38 000 products (layers of 1 to 16384 tokens, 8 to 128 slices, K and N 512 to 5760, random choices), time with this rule where it chooses this kernel
+// over the time without: 16-bit rows 0.905, fp8 0.907, MXFP8 0.95, packed 0.914; more than 10 % slower in 1 to 2 % of them.
+inline int ring_rows(const tamd_matmul_args &a, int cus) {
+  if (!ring_applicable(a)) return 0;
+  const double mean = (double)a.M / a.n_experts, cover = mean + 2.0 * sqrt(mean);
+  const double live = -expm1(a.M * log1p(-1.0 / a.n_experts)) * a.n_experts;
+  const double tiles = live * ((a.N + 255) / 256) / cus;
+  if (mean > 96.0 || (a.K < 1024 && tiles > 1.0)) return 0;
+  const bool alone = tiles <= 1.0;
+  if (a.x_dtype == TAMD_BF16 || a.x_dtype == TAMD_F16) {
+    if (cover <= 16.0 && a.K <= 4096) {
+      const bool padded = a.K > 1024 && (a.K + 1023) / 1024 * 1024 >= 1.3 * a.K;
+      return (alone && tiles > (mean < 3.0 ? 0.75 : 0.5)) || (padded && tiles > 2.0) ? 32 : 0;
+    }
+    if (cover <= 32.0) return (alone && tiles > 0.3) || tiles > (cover <= 16.0 ? 2.2 : 8.0) ? 32 : 0;
+    if (mean < 50.0) return alone && tiles > 0.75 ? 64 : 0;
+    return mean <= 80.0 && tiles > 1.1 && tiles < 8.0 ? 64 : 0;
+  }
+  const bool packed = a.x_dtype == TAMD_MXFP4, scaled = !packed && a.x_mx_scale;
+  if (cover <= 32.0) {
+    if (scaled) return alone || tiles > 2.0 ? 32 : 0;
+    if (packed) return alone || tiles > 1.4 ? 32 : 0;
+    if (tiles > 6.0 && mean >= 12.0) return 64;   // (a slice in two blocks costs more than the larger ones: 509 tokens, 128 slices, 588 us, 601)
+    return (alone && tiles > (mean < 10.0 ? 0.27 : 0.1)) || tiles > 2.0 ? 32 : 0;
+  }
+  if (cover <= 64.0) return tiles > 2.0 || (alone && !scaled && tiles > (packed ? 0.0 : 0.6)) ? 64 : 0;
+  // (of blocks of 96 rows what the products of a layer write is built)
+  const bool swiglu = a.activation == TAMD_ACT_SWIGLU;
+  if (a.y_dtype == TAMD_FP8_E4M3 && (!swiglu || (packed && a.y_mx_scale))) return 0;
+  return tiles > (packed ? 1.4 : 2.0) ? 96 : 0;
 }
 
 // Row block size of a dense / batched problem: the block whose tiles take the fewest rounds over the CUs, weighted with what a
