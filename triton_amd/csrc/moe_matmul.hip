@@ -88,12 +88,14 @@ extern "C" int tamd_matmul_sized(const tamd_matmul_args *args, size_t args_size,
       block_m = a.force_variant;
       grid_m = block_m ? ((a.M + block_m - 1) / block_m) * a.n_experts : 0;
     }
-    int cus = 0;
-    if (int rc = cu_count(cus)) return rc;
-    if (const int rows = ring_rows(a, cus)) {
-      if (x4) return ring_mm_fp4(a, rows, st);
-      if (x8) return ring_mm_fp8e4m3(a, rows, st);
-      return a.x_dtype == TAMD_BF16 ? ring_mm_bf16(a, rows, st) : ring_mm_f16(a, rows, st);
+    if (ring_applicable(a)) {
+      int cus = 0;
+      if (int rc = cu_count(cus)) return rc;
+      if (const int rows = ring_rows(a, cus)) {
+        if (x4) return ring_mm_fp4(a, rows, st);
+        if (x8) return ring_mm_fp8e4m3(a, rows, st);
+        return a.x_dtype == TAMD_BF16 ? ring_mm_bf16(a, rows, st) : ring_mm_f16(a, rows, st);
+      }
     }
     if (x4) return dispatch_mm_fp4(a, block_m, grid_m, st);
     if (a.x_dtype == TAMD_BF16) return dispatch_mm_bf16(a, block_m, grid_m, st);

@@ -271,6 +271,14 @@ TAMD_DEVICE void dma16(v4i_t rsrc, uint32_t lds_addr, uint32_t voff, uint32_t so
                  "s"(__builtin_amdgcn_readfirstlane(soff))
                : "memory", "m0");
 }
+// The same for data that is read once (non-temporal).
+TAMD_DEVICE void dma16_nt(v4i_t rsrc, uint32_t lds_addr, uint32_t voff, uint32_t soff) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds"
+               :
+               : "s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(voff), "s"(rsrc),
+                 "s"(__builtin_amdgcn_readfirstlane(soff))
+               : "memory", "m0");
+}
 // 2- and 4-byte global -> LDS copies: lane L's value lands (zero-extended) in the dword at
 // lds_addr + 4*L; out-of-range offsets deliver zero.  The five wait states before the load cover an
 // SGPR operand that a v_readfirstlane wrote just before the asm block (the compiler's hazard

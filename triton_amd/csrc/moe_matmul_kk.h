@@ -65,7 +65,7 @@ struct KKShape {
   static_assert(LDS <= 160 * 1024, "one workgroup per CU");
 };
 
-template <int XDT, int NFR, int BM, int ACT>
+template <int XDT, int NFR, int BM, int ACT, bool ONCE>
 TAMD_DEVICE void run_tile_kk(const tamd_matmul_args &a, const Tile &t, uint8_t *lds) {
   typedef KK<XDT> O;
   typedef typename O::frag_t frag_t;
@@ -110,7 +110,10 @@ TAMD_DEVICE void run_tile_kk(const tamd_matmul_args &a, const Tile &t, uint8_t *
       if (u < NA1 || grp == 0) dma16(rx, sa + u * 8192, a_off[u] | kill, kb * ESZ);
     const uint32_t sb = sa + LDS_ROWS * 128;
 #pragma unroll
-    for (int u = 0; u < NB; ++u) dma16(rw, sb + u * 8192, b_off[u] | kill, kb * ESZ);
+    for (int u = 0; u < NB; ++u) {
+      if constexpr (ONCE) dma16_nt(rw, sb + u * 8192, b_off[u] | kill, kb * ESZ);
+      else dma16(rw, sb + u * 8192, b_off[u] | kill, kb * ESZ);
+    }
   };
 
   f32x16_t acc[NFR][NF];
@@ -232,7 +235,8 @@ TAMD_DEVICE void run_tile_kk(const tamd_matmul_args &a, const Tile &t, uint8_t *
   }
 }
 
-template <int XDT, int BM, int ACT>
+// ONCE: weights are copied non-temporally (a slice of more than one row block reads them again).
+template <int XDT, int BM, int ACT, bool ONCE>
 __global__ __launch_bounds__(512, 1) void mm_kk_kernel(tamd_matmul_args a, int grid_n, int64_t grid_total, int group_m) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   typedef TileShape<XDT, BM> S;
@@ -241,9 +245,9 @@ __global__ __launch_bounds__(512, 1) void mm_kk_kernel(tamd_matmul_args a, int g
     if (!locate_tile_live<BM, S::EXTRA>(a, grid_n, -group_m, t)) return;
   } else if (!locate_tile<BM, S::EXTRA>(a, grid_n, grid_total, group_m, t)) return;
   const int nfr = (t.rows + 31) / 32;
-#define TAMD_CASE(n)                                                      \
-  case n:                                                                 \
-    if constexpr (n <= S::MF) run_tile_kk<XDT, n, BM, ACT>(a, t, lds);    \
+#define TAMD_CASE(n)                                                         \
+  case n:                                                                    \
+    if constexpr (n <= S::MF) run_tile_kk<XDT, n, BM, ACT, ONCE>(a, t, lds); \
     break;
   switch (nfr) { TAMD_CASE(1) TAMD_CASE(2) TAMD_CASE(3) TAMD_CASE(4) TAMD_CASE(5) }
 #undef TAMD_CASE
@@ -411,7 +415,16 @@ int launch_kk(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
       return launch_status();
     }
   }
-  auto kern = mm_kk_kernel<XDT, BM, ACT>;
+  // 16-bit weights of slices that hardly ever need two row blocks are copied non-temporally where their columns are whole lines and a call
+  // reads more of them (320 MB) than the 256 MB behind the L2s keep for the next one: 300 tokens x 4 of 32 slices, 2880 -> 2880, layer 342 -> 310 us,
+  // over 80 products 0.92 of the time.  Below that 1.0 to 1.5, with lines that two stages share 1.08 (0.95 to 1.3), and 1021 tokens x 4
+  // of 32, where a slice in eight has two blocks, 397 -> 410.
+  auto kern = mm_kk_kernel<XDT, BM, ACT, false>;
+  if constexpr (!KK<XDT>::FP8) {
+    const bool lines = aligned(a.w, 128) && (a.w_stride_n * 2) % 128 == 0 && (a.w_stride_e * 2) % 128 == 0;
+    if (lines && 4 * rows_per_slice <= 3 * BM && live_slices(a) * a.N * ((double)a.K * 2) >= 320.0 * (1 << 20))
+      kern = mm_kk_kernel<XDT, BM, ACT, true>;
+  }
   if (int rc = raise_lds_limit_once((const void *)kern)) return rc;
   // (one workgroup per CU: an XCD holds 32 tiles, and an expert's blocks share a column tile only side by side; 32 experts
   // of 250 bf16 rows, 2880 x 2880: 181 us in fours, 199 one after the other, 217 in schedule order)

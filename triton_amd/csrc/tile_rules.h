@@ -46,6 +46,11 @@ inline bool blocks_of_16_stream(tamd_matmul_args a) {
   return a.w_dtype == TAMD_MXFP4 && stream16_applicable(a);
 }
 
+// Slices of a ragged problem that have rows, if they are spread at random; all of a batch.
+inline double live_slices(const tamd_matmul_args &a) {
+  return a.block_schedule ? -expm1(a.M * log1p(-1.0 / a.n_experts)) * a.n_experts : a.n_experts;
+}
+
 inline int64_t output_size(int dtype) { return dtype == TAMD_F32 ? 4 : (dtype == TAMD_FP8_E4M3 || dtype == TAMD_FP8_E5M2 ? 1 : 2); }
 
 // What the persistent kernel of few rows per slice (moe_matmul_ring.h) covers: ragged problems with weights in 4 KB blocks, pre-shuffled scales, outputs of
@@ -75,8 +80,7 @@ inline bool ring_applicable(const tamd_matmul_args &a) {
 inline int ring_rows(const tamd_matmul_args &a, int cus) {
   if (!ring_applicable(a)) return 0;
   const double mean = (double)a.M / a.n_experts, cover = mean + 2.0 * sqrt(mean);
-  const double live = -expm1(a.M * log1p(-1.0 / a.n_experts)) * a.n_experts;
-  const double tiles = live * ((a.N + 255) / 256) / cus;
+  const double tiles = live_slices(a) * ((a.N + 255) / 256) / cus;
   if (mean > 96.0 || (a.K < 1024 && tiles > 1.0)) return 0;
   const bool alone = tiles <= 1.0;
   if (a.x_dtype == TAMD_BF16 || a.x_dtype == TAMD_F16) {
