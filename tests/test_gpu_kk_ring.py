@@ -1,0 +1,75 @@
+"""GPU: the persistent kernel for unquantised 16-bit weights at the sizes where it can go wrong: K of its fewest stages and off them, columns off strips,
+tiles and lines, empty slices, slices of one row, of whole blocks, one more, and many, rows that are not there, against float32 products."""
+import ctypes
+
+import pytest
+import torch
+
+from triton_amd import _lib, _native
+from triton_amd.matmul import FnSpecs, FusedActivation, PrecisionConfig, matmul
+from triton_amd.swiglu import swiglu_fn
+from triton_amd.tensor import make_ragged_tensor_metadata
+
+SWIGLU = FusedActivation(FnSpecs("swiglu", swiglu_fn, ("alpha", "limit"), reduction_n=2), (1.702, 7.0))
+
+
+def ring_rows(m, n, k, e, swiglu=False, **changed):
+    bag = _lib.MatmulArgBag()
+    bag.x_dtype = bag.w_dtype = bag.y_dtype = _lib.BF16
+    bag.M, bag.N, bag.K, bag.n_experts, bag.block_schedule = m, n, k, e, 1 << 20
+    bag.activation = _lib.ACT_SWIGLU if swiglu else _lib.ACT_NONE
+    bag.y, bag.y_rows, bag.y_stride_m = 1 << 20, m, n // 2 if swiglu else n
+    for name, value in changed.items():
+        setattr(bag, name, value)
+    packed = bag.pack()
+    return _native.ring_rows(ctypes.addressof(packed), 256)
+
+
+def test_where_it_is_taken():
+    assert ring_rows(1200, 5760, 2880, 32) == 64 and ring_rows(4084, 5760, 2880, 32, True) == 160
+    assert ring_rows(4, 3904, 1760, 8) == 0
+    for changed in (dict(block_schedule=None), dict(n_experts=257), dict(y_dtype=_lib.F32), dict(y_rows=0), dict(y_rows=1 << 20), dict(K=248),
+                    dict(y_expected_scale=1 << 20), dict(N=5759), dict(y=(1 << 20) + 2), dict(y_stride_m=5761), dict(x_dtype=_lib.F16)):
+        assert ring_rows(4084, 5760, 2880, 32, **changed) == 0, changed
+
+
+# (slice sizes, K, columns)
+SIZES = [([1, 0, 31, 32, 33, 64, 65, 0, 129, 3], 256, 6200), ([2] * 70 + [0] * 30, 1096, 648), ([160, 161, 0, 320, 321, 95, 97, 700], 776, 3176),
+         ([1500, 0, 40], 520, 4100), ([5000], 264, 1032)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("sizes,K,N", SIZES)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("swiglu", [False, True])
+@pytest.mark.parametrize("gathered", [False, True])
+def test_edges(sizes, K, N, dtype, swiglu, gathered, device):
+    E, M, T = len(sizes), sum(sizes), 50
+    assert ring_rows(M, N, K, E, swiglu)
+    torch.manual_seed(K)
+    gather, scatter = torch.randint(0, T, (M,), dtype=torch.int32), torch.randperm(M, dtype=torch.int32)
+    gather[M // 2], scatter[M // 3] = -1, -1
+    x = torch.randn(T if gathered else M, K, device=device).to(dtype)
+    w = (torch.randn(E, N, K, device=device) * 0.1).to(dtype).transpose(1, 2)
+    bias, gammas = torch.randn(E, N, device=device), torch.rand(M, device=device)
+    md = make_ragged_tensor_metadata(torch.tensor(sizes, dtype=torch.int32, device=device), M)
+    kw = dict(gather_indx=gather.to(device)) if gathered else dict(scatter_indx=scatter.to(device), gammas=gammas)
+    got = matmul(x, w, bias, md, precision_config=PrecisionConfig(), fused_activation=SWIGLU if swiglu else None, **kw)
+    rows = torch.where((gather >= 0)[:, None].to(device), x.float()[gather.clamp(min=0).long().to(device)], 0.0) if gathered else x.float()
+    full = torch.empty(M, N // 2 if swiglu else N, device=device)
+    slack = torch.empty_like(full)
+    at = 0
+    for e, n in enumerate(sizes):
+        r = slice(at, at + n)
+        at += n
+        v, mag = rows[r] @ w[e].float() + bias[e], K * 2.0 ** -23 * (rows[r].abs() @ w[e].float().abs())
+        if swiglu:
+            g, l = v[:, 0::2].clamp(max=7.0), v[:, 1::2].clamp(-7.0, 7.0)
+            s = g * torch.sigmoid(1.702 * g)
+            v, mag = s * (l + 1), 1.2 * mag[:, 0::2] * (l.abs() + 1) + s.abs() * mag[:, 1::2]   # (|d swish| <= 1.1)
+        full[r], slack[r] = v, mag
+    if not gathered:
+        there = scatter >= 0
+        full, slack, got = full[there.to(device)] * gammas[there.to(device), None], slack[there.to(device)], got[scatter[there].long().to(device)]
+    # a 16-bit result (2^-8) of K float32 additions, and the hardware's exponential and reciprocal (2^-20)
+    assert bool(((got.float() - full).abs() <= 2.0 ** -8 * full.abs() + slack + 1e-5).all())

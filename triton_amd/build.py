@@ -19,7 +19,8 @@ SOURCES = ["api.cpp", "mxfp.hip", "routing.hip", "elementwise.hip", "moe_matmul.
            "moe_matmul_ring_bf16.hip", "moe_matmul_ring_f16.hip", "moe_matmul_ring_fp8.hip", "moe_matmul_ring_fp4.hip",
            "moe_matmul_fp4.hip", "moe_matmul_fp4_swiglu.hip",
            "moe_matmul_w16_bf16.hip", "moe_matmul_w16_f16.hip",
-           "moe_matmul_kk_bf16.hip", "moe_matmul_kk_f16.hip", "moe_matmul_kk_fp8.hip"]
+           "moe_matmul_kk_bf16.hip", "moe_matmul_kk_f16.hip", "moe_matmul_kk_fp8.hip",
+           "moe_matmul_kkring_bf16.hip", "moe_matmul_kkring_f16.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 # packed fp32 math is switched off on purpose (device code only); the unroll limit is raised because the tile
 # epilogues index their accumulators with loops that must unroll completely (up to 80 element rows per lane):
@@ -110,7 +111,7 @@ def build(force=True, verbose=False):
     srcs = [s for s in SOURCES if os.path.exists(os.path.join(CSRC, s))]
     objs = [os.path.join(objdir, os.path.splitext(s)[0] + ".o") for s in srcs]
     deps = [os.path.join(CSRC, "common.h"), os.path.join(CSRC, "moe_matmul_impl.h"), os.path.join(CSRC, "moe_matmul_stream.h"), os.path.join(CSRC, "moe_matmul_dense.h"),
-            os.path.join(CSRC, "moe_matmul_kk.h"), os.path.join(CSRC, "moe_matmul_mx.h"), os.path.join(CSRC, "moe_matmul_ring.h"), os.path.join(CSRC, "tile_rules.h"),
+            os.path.join(CSRC, "moe_matmul_kk.h"), os.path.join(CSRC, "moe_matmul_mx.h"), os.path.join(CSRC, "moe_matmul_ring.h"), os.path.join(CSRC, "moe_matmul_kkring.h"), os.path.join(CSRC, "tile_rules.h"),
             os.path.join(HERE, "..", "include", "triton_amd.h")]
     todo = []
     for s, o in zip(srcs, objs):

@@ -705,7 +705,7 @@ PyObject *py_ring_rows(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
     need(nargs == 2);
     tamd_matmul_args a;
     std::memcpy(&a, (const void *)(intptr_t)as_int(v[0]), sizeof a);
-    return PyLong_FromLong(tamd::ring_rows(a, (int)as_int(v[1])));
+    return PyLong_FromLong(a.w_dtype == TAMD_MXFP4 ? tamd::ring_rows(a, (int)as_int(v[1])) : tamd::kk_ring_rows(a, (int)as_int(v[1])));
   });
 }
 

@@ -88,7 +88,7 @@ extern "C" int tamd_matmul_sized(const tamd_matmul_args *args, size_t args_size,
       block_m = a.force_variant;
       grid_m = block_m ? ((a.M + block_m - 1) / block_m) * a.n_experts : 0;
     }
-    if (ring_applicable(a)) {
+    if (known_block(block_m) && ring_applicable(a)) {
       int cus = 0;
       if (int rc = cu_count(cus)) return rc;
       if (const int rows = ring_rows(a, cus)) {

@@ -433,6 +433,9 @@ int launch_kk(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
   return launch_status();
 }
 
+int kk_ring_mm_bf16(const tamd_matmul_args &a, int rows, hipStream_t st);
+int kk_ring_mm_f16(const tamd_matmul_args &a, int rows, hipStream_t st);
+
 // Both operands contiguous along K, 16-byte aligned rows and columns, whole 16-byte chunks along K, and offsets inside
 // an operand below 2 GB: anything else is refused (TAMD_E_UNSUPPORTED / _ALIGNMENT).
 template <int XDT>
@@ -444,6 +447,13 @@ int dispatch_kk(const tamd_matmul_args &a, int block_m, int grid_m, hipStream_t 
   if (!aligned(a.x, 16) || (a.x_stride_m * ESZ) % 16 != 0 || (a.x_stride_z * ESZ) % 16 != 0) return TAMD_E_ALIGNMENT;
   const int64_t x_rows = a.x_rows > 0 ? a.x_rows : a.M, lim = 0x7FFFFF00;
   if (x_rows * a.x_stride_m * ESZ >= lim || (int64_t)a.N * a.w_stride_n * ESZ >= lim) return TAMD_E_UNSUPPORTED;
+  if constexpr (!KK<XDT>::FP8) {
+    if (known_block(block_m) && kk_ring_applicable(a)) {
+      int cus = 0;
+      if (int rc = cu_count(cus)) return rc;
+      if (const int rows = kk_ring_rows(a, cus)) return XDT == TAMD_BF16 ? kk_ring_mm_bf16(a, rows, st) : kk_ring_mm_f16(a, rows, st);
+    }
+  }
   const bool sw = a.activation == TAMD_ACT_SWIGLU;
   switch (block_m) {
     case 16: return sw ? launch_kk<XDT, 16, TAMD_ACT_SWIGLU>(a, grid_m, st) : launch_kk<XDT, 16, TAMD_ACT_NONE>(a, grid_m, st);

@@ -51,6 +51,9 @@ inline double live_slices(const tamd_matmul_args &a) {
   return a.block_schedule ? -expm1(a.M * log1p(-1.0 / a.n_experts)) * a.n_experts : a.n_experts;
 }
 
+// The row blocks that a ragged schedule may have.
+inline bool known_block(int block_m) { return block_m == 16 || block_m == 32 || block_m == 64 || block_m == 128; }
+
 inline int64_t output_size(int dtype) { return dtype == TAMD_F32 ? 4 : (dtype == TAMD_FP8_E4M3 || dtype == TAMD_FP8_E5M2 ? 1 : 2); }
 
 // What the persistent kernel of few rows per slice (moe_matmul_ring.h) covers: ragged problems with weights in 4 KB blocks, pre-shuffled scales, outputs of
@@ -104,6 +107,28 @@ inline int ring_rows(const tamd_matmul_args &a, int cus) {
   const bool swiglu = a.activation == TAMD_ACT_SWIGLU;
   if (a.y_dtype == TAMD_FP8_E4M3 && (!swiglu || (packed && a.y_mx_scale))) return 0;
   return tiles > (packed ? 1.4 : 2.0) ? 96 : 0;
+}
+
+// What the persistent kernel for unquantised 16-bit weights (moe_matmul_kkring.h) covers, of the products that the tiled kernel of two operands along K
+// takes: ragged problems of four stages of K and more, outputs of the rows' type in pairs of columns that 32-bit offsets reach.
+inline bool kk_ring_applicable(const tamd_matmul_args &a) {
+  if (!a.block_schedule || a.K < 256 || a.n_experts > 256) return false;
+  if ((a.x_dtype != TAMD_BF16 && a.x_dtype != TAMD_F16) || a.w_dtype != a.x_dtype || a.y_dtype != a.x_dtype) return false;
+  if (a.y_mx_scale || a.y_expected_scale || a.y_actual_scale) return false;
+  if ((a.N + 63) / 64 > 0x8000 || ((int64_t)a.M + a.n_experts) * ((a.N + 63) / 64) > 0x7FFFFFF0) return false;
+  if (a.y_rows <= 0 || a.y_stride_m < 0 || a.y_rows * a.y_stride_m * 2 >= (int64_t)0x7FFFFF00) return false;
+  return a.activation == TAMD_ACT_SWIGLU || (((a.N | (int)a.y_stride_m) & 1) == 0 && aligned(a.y, 4));
+}
+
+// Rows of its blocks, 0 where the tiled kernels are the faster: with fewer than a third as many tiles of 256 columns as CUs one workgroup's stages are all
+// latency (four rows for 8 slices, 1760 x 3904: 13.4 us, 16 with this one).  486 products of 1 to 16384 tokens, 8 to 128 slices, K and N 512 to 5760: 0.876 of the
+// time in the mean (0.866 with the best choice for each), none above 1.05; with the line at 0.25 0.874, three above 1.1; at 0.5 0.888.  Blocks of 64 up to 56 rows per slice
+// lose up to 1.21, where slices come in two.
+inline int kk_ring_rows(const tamd_matmul_args &a, int cus) {
+  if (!kk_ring_applicable(a)) return 0;
+  const double mean = (double)a.M / a.n_experts, tiles = live_slices(a) * ((a.N + 255) / 256) / cus;
+  if (3.0 * tiles * (mean > 160.0 ? mean / 160.0 : 1.0) < 1.0) return 0;
+  return mean <= 48.0 ? 64 : 160;
 }
 
 // Row block size of a dense / batched problem: the block whose tiles take the fewest rounds over the CUs, weighted with what a
