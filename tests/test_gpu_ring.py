@@ -1,6 +1,6 @@
-"""GPU: the persistent kernel of few rows per slice (weights in 4 KB blocks, pre-shuffled scales) at the sizes where it can go wrong: K below a stage, below the
+"""GPU: the persistent kernel of few rows per slice (weights in 4 KB blocks and pre-shuffled scales, or both strided) at the sizes where it can go wrong: K below a stage, below the
 ring and off both, columns off strips and tiles, empty slices and slices of several blocks, with gathered and scattered rows that are not
-there, every kind of row and of output.  Rows of 8 and 4 bits give the bits of the tiled kernels, which strided weights take; 16-bit
+there, every kind of row and of output.  Rows of 8 and 4 bits give the bits of the tiled kernels, which strided weights with pre-shuffled scales take; 16-bit
 rows are held against float32 products."""
 import ctypes
 
@@ -60,6 +60,57 @@ SIZES = [(9, 10, 96, 2832), (4, 12, 352, 1872), (14, 16, 736, 1296), (20, 16, 14
          (40, 16, 608, 2608), (30, 60, 1248, 2320), (72, 32, 1056, 4368)]
 
 
+def test_where_strided_weights_take_it():
+    """Where a call leaves CUs without a tile, and 16-bit rows in blocks of 64 over several rounds; not with one side in the other layout."""
+    both = dict(w_layout=_lib.W_STRIDED, w_mx_layout=_lib.SCALE_STRIDED)
+    assert ring_rows(60, 1696, 1440, 16, "mxfp4", **both) == 32 and ring_rows(500, 2048, 2880, 16, "mxfp4", **both) == 64
+    assert ring_rows(100, 2560, 2880, 16, "fp8", **both) == 32 and ring_rows(1332, 5760, 2880, 32, "bf16", **both) == 64
+    for M, N, K, E, kind in ((512, 5760, 2880, 128, "fp8"), (100, 2560, 2880, 16, "bf16"), (2048, 5760, 2880, 16, "bf16"), (8, 512, 2880, 16, "mxfp8")):
+        assert ring_rows(M, N, K, E, kind, **both) == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,rows,E,K,N", [("mxfp4", 9, 10, 96, 2832), ("mxfp4", 4, 12, 352, 1872), ("mxfp4", 30, 8, 1440, 1394), ("mxfp8", 9, 10, 96, 2832),
+                                             ("mxfp8", 9, 20, 736, 1298), ("fp8", 9, 20, 1056, 1298), ("fp8", 4, 12, 2144, 2832), ("bf16", 15, 20, 544, 1296),
+                                             ("f16", 30, 20, 1312, 2328), ("bf16", 40, 60, 1056, 2322)])
+@pytest.mark.parametrize("byte", [0, 1])
+def test_strided_edges(kind, rows, E, K, N, byte, device):
+    """The bits that the same kernel gives with blocks and pre-shuffled scales, weights and scales at addresses off 64 bytes and (byte) off four."""
+    sizes = torch.randint(max(0, rows - 9), rows + 10, (E,), generator=torch.Generator().manual_seed(K), dtype=torch.int32)
+    sizes[1] = 0
+    M = int(sizes.sum())
+    strided = dict(w_layout=_lib.W_STRIDED, w_mx_layout=_lib.SCALE_STRIDED)
+    assert ring_rows(M, N, K, E, kind, **strided)
+    torch.manual_seed(K + N)
+    w, ws = downcast_to_mxfp((torch.randn(E, N, K, device=device) * torch.exp(2 * torch.randn(E, N, 1, device=device))).bfloat16(), torch.uint8, axis=-1)
+    room = torch.full((16 + w.numel(),), 0x55, dtype=torch.uint8, device=device)
+    w_at = room[16:].view(w.shape).copy_(w)
+    ends = torch.full((byte + ws.numel() + 64,), 255, dtype=torch.uint8, device=device)   # (NaN scales around the tensor)
+    ws_at = ends[byte:byte + ws.numel()].view(ws.shape).copy_(ws)
+    x, opts = torch.randn(50, K, device=device), {}
+    if kind[:2] == "mx":
+        x, s = downcast_to_mxfp(x, torch.uint8 if kind == "mxfp4" else torch.float8_e4m3fn, axis=-1)
+        opts.update(a_mx_scale=s, a_microblock_size=32)
+    else:
+        x = x.to(TYPES[kind])
+    gather = torch.randint(-1, 50, (M,), dtype=torch.int32, device=device)
+    bias, md = torch.randn(E, N, device=device), make_ragged_tensor_metadata(sizes.to(device), M)
+
+    def run(weights, scales):
+        return matmul(x, weights, bias, md, gather_indx=gather, precision_config=PrecisionConfig(
+            b_mx_scale=scales, b_microblock_size=32, out_dtype=torch.float16 if kind == "f16" else torch.bfloat16, **opts))
+
+    got = run(w_at.transpose(1, 2), ws_at.transpose(1, 2))
+    if ring_rows(M, N, K, E, kind) or kind[:2] == "mx":
+        assert torch.equal(got, run(*blocks(w.transpose(1, 2), ws.transpose(1, 2))))
+        return
+    # (blocks take a kernel with sums in another order: float32 sums, a rounding to 16 bits on either side)
+    want = run(*blocks(w.transpose(1, 2), ws.transpose(1, 2))).float()
+    wf = upcast_from_mxfp(w, ws, torch.float32, axis=-1).transpose(1, 2)
+    mag = torch.cat([x.float().abs()[gather[a:b].clamp(min=0).long()] @ wf[e].abs() for e, (a, b) in enumerate(zip(*(lambda c: (c - sizes.long(), c))(sizes.long().cumsum(0))))])
+    assert bool(((got.float() - want).abs() <= 2.0 ** -7 * want.abs() + K * 2.0 ** -22 * mag + 1e-6).all())
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("rows,E,K,N", SIZES)
 @pytest.mark.parametrize("kind", ["bf16", "f16", "fp8", "mxfp8", "mxfp4"])
@@ -106,7 +157,7 @@ def test_edges(rows, E, K, N, kind, out, device):
 
     got, got_scales, there = run(wb, wsb)
     if kind not in ("bf16", "f16"):
-        ref, ref_scales, _ = run(w, ws)
+        ref, ref_scales, _ = run(w, wsb)
         assert torch.equal(got.view(torch.uint8), ref.view(torch.uint8))
         assert got_scales is None or torch.equal(got_scales, ref_scales)
         return

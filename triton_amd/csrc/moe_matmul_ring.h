@@ -1,4 +1,4 @@
-// Grouped (ragged) matmul of up to about 96 rows per slice x MXFP4 weights in 4 KB blocks with pre-shuffled scales: a persistent kernel whose copies never stop at
+// Grouped (ragged) matmul of up to about 96 rows per slice x MXFP4 weights in 4 KB blocks with pre-shuffled scales, or both strided: a persistent kernel whose copies never stop at
 // the end of a tile.
 //
 // With few rows per slice HBM is the bound, and one tile per workgroup (moe_matmul_mx.h) reaches 5.3 TB/s of the 7 that copies alone read: a tile
@@ -13,6 +13,11 @@
 //   * the weights of a slice with one row block are read once: non-temporal copies (632 -> 563 us on the first of the layers below);
 //   * tiles of fewer than four strips where that fills the one or two rounds over the workgroups.
 // Barriers of the whole workgroup, one per stage, publish a stage and free the one before.
+//
+// Strided weights (blocks of up to 64 rows): pieces of 64 bytes per column and 128 K, sixteen bytes of scales per column and 256 K.  They read 3 to 4.7 TB/s, by
+// whether a piece crosses a line, as in moe_matmul_mx.h; what is won is the narrower tiles of small calls and, for 16-bit rows, multiplying waves that do not
+// copy.  (Scales a dword at a time asked for twice as many lines as the weights, 5 to 15 % slower.)  Layers, tiled kernel -> now, us: 100 packed tokens x 4 of 16 slices, 2880
+// -> 1440, 62.3 -> 57.8; 60 fp8 x 4 of 16, 1760 -> 1440, 38.1 -> 33.6; 80 bf16 x 4 of 16, 2048 -> 1024, 43.5 -> 35.9; 512 bf16 x 4 of 60, 2880 -> 2880, 284 -> 266.
 //
 // Time of a layer (routing, both products, sum) before -> now: 509 fp8 tokens, 128 slices, 5760 -> 2880, 638 -> 548 us (the copies alone 499; the stores of the results
 // cost the rest: scattered lines between the reads, 45 us for 29 MB, 10 if they stay in the caches); 2880 -> 2880, 128 slices: 512 tokens fp8 346 -> 297, MXFP8
@@ -40,7 +45,10 @@ struct RingShape {
   static constexpr int KA = FP4 ? 256 : 128;                 // K per stage
   static constexpr int PLANES = KA / PLANE_K, BLOCKS = KA / KB;
   static constexpr int AHEAD = X16 ? 1 : 0;                  // stages past its own whose operands a wave reads
-  static constexpr int A_STAGE = PLANES * ROWS * A_ROW_BYTES, B_STAGE = 4 * BLOCKS * 4096, SC_STAGE = 2048;
+  static constexpr int A_STAGE = PLANES * ROWS * A_ROW_BYTES, B_STAGE = 4 * BLOCKS * 4096;
+  // Strided column scales: sixteen bytes of every column from the dword on that holds the first of 256 K (a stage of 128 K: every other one).
+  static constexpr bool STRIDED = MF <= 2;                   // (blocks of 96 rows have neither the LDS nor the registers)
+  static constexpr int SC_STAGE = STRIDED ? 4096 : 2048;
   // Block scales of the rows (XMX): the dwords that cover a row's bytes of the stage, whatever their alignment, for whole waves of rows.
   static constexpr int XS_WORDS = XMX ? KA / 128 + 1 : 0, XS_WAVES = (MF + 1) / 2, XS_STAGE = XS_WORDS * XS_WAVES * kWave * 4;
   static constexpr int STAGE = A_STAGE + B_STAGE + SC_STAGE + XS_STAGE;
@@ -51,7 +59,7 @@ struct RingShape {
   static constexpr int RING = FIT > 5 + AHEAD ? 5 + AHEAD : FIT;
   static constexpr int LDS = RING * STAGE + FIXED;
   static constexpr int COPIES = 4 * BLOCKS + PLANES * MF;   // of a copying wave and stage, without scales
-  static_assert(RING >= 2 + AHEAD && (RING - 2) * (COPIES + (XS_WORDS > 1 ? XS_WORDS : 1)) < 64, "ring does not fit the vmcnt counter");
+  static_assert(RING >= 2 + AHEAD && (RING - 2) * (COPIES + 1 + XS_WORDS) < 64, "ring does not fit the vmcnt counter");
 };
 
 // The tiles of a workgroup: every step-th of its XCD's range, so that the workgroups of an XCD are at about the same slices.
@@ -177,6 +185,11 @@ TAMD_DEVICE void ring_copy(const Args &a, const RingWork &work, uint8_t *lds) {
   const v4i_t rx = make_rsrc(a.x, kOob);
   const uint8_t *w_base = nullptr, *s_base = nullptr;
   uint32_t a_off[MF], w_off = kOob, s_off = kOob, xs_off = kOob;
+  // Strided weights: instruction j copies positions 16 j + lane / 4 of a strip, 16-byte part `part` (j > 1: part ^ 2) of 64 bytes, so that
+  // they lie in LDS as blocks do; position 32 f + c holds column 2 c + f.
+  const bool strided = S::STRIDED && a.w_layout != TAMD_W_CDNA4_BLOCKS;
+  const int part = (lane % 4) ^ ((lane / 16) & 3);
+  uint32_t c_off[4], s_end = kOob;
   // the row scales as aligned dwords, up to the one that holds the last row's last byte
   const uint32_t xs_mis = XMX ? (uint32_t)(uintptr_t)a.x_mx_scale & 3u : 0u;
   const v4i_t rxs = make_rsrc(a.x_mx_scale - xs_mis,
@@ -191,20 +204,42 @@ TAMD_DEVICE void ring_copy(const Args &a, const RingWork &work, uint8_t *lds) {
       }
       w_base = (const uint8_t *)a.w + (int64_t)t.expert * a.w_stride_e;
       s_base = a.w_mx_scale + (int64_t)t.expert * a.w_mx_stride_e;
-      w_off = w < strips ? (uint32_t)(((t.n0 >> 6) + w) * n_kb) * 4096u + (uint32_t)lane * 16u : kOob;
-      const int blk = (t.n0 >> 5) + 4 * w + lane / 16;
-      s_off = blk * 32 < N && (4 * w + lane / 16) / 2 < strips ? (uint32_t)(blk * KSP * 32 + (lane % 16) * 16) : kOob;
+      if (strided) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int col = t.n0 + w * 64 + 2 * (lane / 4 + 16 * j % 32) + 16 * j / 32;
+          c_off[j] = w < strips ? (uint32_t)(col < N ? col : N - 1) * (uint32_t)a.w_stride_n + (uint32_t)(part ^ (j >> 1) << 1) * 16u : kOob;
+        }
+        // (scales as aligned dwords, up to the one that holds the last column's last byte)
+        const uint32_t mis = (uint32_t)(uintptr_t)s_base & 3u, col = (uint32_t)(t.n0 + w * 64 + lane);
+        s_base -= mis;
+        s_end = (mis + (uint32_t)((N - 1) * a.w_mx_stride_n + K / 32) + 3u) & ~3u;
+        s_off = w < strips && (int)col < N ? (mis + col * (uint32_t)a.w_mx_stride_n) & ~3u : kOob;
+      } else {
+        w_off = w < strips ? (uint32_t)(((t.n0 >> 6) + w) * n_kb) * 4096u + (uint32_t)lane * 16u : kOob;
+        const int blk = (t.n0 >> 5) + 4 * w + lane / 16;
+        s_off = blk * 32 < N && (4 * w + lane / 16) / 2 < strips ? (uint32_t)(blk * KSP * 32 + (lane % 16) * 16) : kOob;
+      }
     }
-    const v4i_t rw = make_rsrc(w_base, kOob), rs = make_rsrc(s_base, kOob);
+    const v4i_t rw = make_rsrc(w_base, kOob), rs = make_rsrc(s_base, strided ? (uint32_t)__builtin_amdgcn_readfirstlane((int)s_end) : kOob);
     const uint32_t sb = lds_base + slot * S::STAGE;
 #pragma unroll
     for (int u = 0; u < S::BLOCKS; ++u) {
-      const uint32_t to = sb + S::A_STAGE + (w * S::BLOCKS + u) * 4096, from = w_off | (p * KA + u * KB < K ? 0u : kOob);
+      const uint32_t to = sb + S::A_STAGE + (w * S::BLOCKS + u) * 4096;
+      if (strided) {
+        const int kb = p * KA + u * KB;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) dma16(rw, to + j * 1024, c_off[j] | (kb + (part ^ (j >> 1) << 1) * 32 < K ? 0u : kOob), kb >> 1);
+        continue;
+      }
+      const uint32_t from = w_off | (p * KA + u * KB < K ? 0u : kOob);
       const uint32_t so = (uint32_t)(S::BLOCKS * p + u) * 4096u;
       if (once) dma16_x4_nt(rw, to, from, so);
       else dma16_x4(rw, to, from, so);
     }
-    if (w < 2) dma16(rs, sb + S::A_STAGE + S::B_STAGE + w * 1024, s_off, (uint32_t)(p * KA / 256) * 256u);
+    if (strided) {
+      if (KA == 256 || (p & 1) == 0) dma16(rs, sb + S::A_STAGE + S::B_STAGE + w * 1024, s_off + (uint32_t)(p * (KA / 32)), 0);
+    } else if (w < 2) dma16(rs, sb + S::A_STAGE + S::B_STAGE + w * 1024, s_off, (uint32_t)(p * KA / 256) * 256u);
     if (fresh) {
       if (a.gather_indx && (i_tile == 0 || n_k < RING)) wait_vmcnt<4 * S::BLOCKS>();
       auto index = [&](int at) { return *(const uint32_t *)(lds + idx_at + (i_tile & 1) * 256 + at * 4); };
@@ -238,7 +273,11 @@ TAMD_DEVICE void ring_copy(const Args &a, const RingWork &work, uint8_t *lds) {
   };
   auto wait = [&](auto newer) {
     constexpr int n = decltype(newer)::value;
-    if (w < 2) wait_vmcnt<n * (S::COPIES + 1)>();
+    // (strided and 128 K: with the column scales of every other stage one or two more may be outstanding than are waited for)
+    constexpr int SC = KA == 256 ? 1 : 0;
+    if (strided && row_scales) wait_vmcnt<n * (S::COPIES + SC + S::XS_WORDS)>();
+    else if (strided) wait_vmcnt<n * (S::COPIES + SC)>();
+    else if (w < 2) wait_vmcnt<n * (S::COPIES + 1)>();
     else if (row_scales) wait_vmcnt<n * (S::COPIES + S::XS_WORDS)>();
     else wait_vmcnt<n * S::COPIES>();
   };
@@ -304,13 +343,26 @@ TAMD_DEVICE void ring_products(const Args &a, const Tile &t, uint8_t *lds, uint8
   if constexpr (NFR >= 3 && !XMX) asm volatile("" : "+v"(lane));   // (nothing made of it is kept over the tiles: registers)
   const int c32 = lane % 32, h = lane / 32;
   const int K = a.K, G = K / 32, n_k = (K + KA - 1) / KA;
-  const uint32_t sc_sel = 0x06020400u + (uint32_t)((c32 >> 3) & 1) * 0x01010101u;
+  const bool strided = S::STRIDED && a.w_layout != TAMD_W_CDNA4_BLOCKS;
+  // Column scales of 256 K: bytes h, 2 + h, ... of eight (strided: of the sixteen that start with their dword).
+  uint32_t sc_sel[NF];
+#pragma unroll
+  for (int f = 0; f < NF; ++f) {
+    if (strided) {
+      const uint32_t at = (uint32_t)(uintptr_t)(a.w_mx_scale + (int64_t)t.expert * a.w_mx_stride_e) +
+                          (uint32_t)(t.n0 + strip * 64 + 2 * c32 + f) * (uint32_t)a.w_mx_stride_n;
+      sc_sel[f] = 0x0C0C0200u + ((at & 3u) + h) * 0x0101u;
+    } else {
+      sc_sel[f] = 0x06020400u + (uint32_t)((c32 >> 3) & 1) * 0x01010101u;
+    }
+  }
   // Offsets into a stage: a lane's first chunk of a row and of a column, the others an exclusive or away (a stage starts on 128 bytes),
   // so that one address register serves all of them.
   static_assert(S::STAGE % 128 == 0 && S::A_STAGE % 128 == 0, "chunks are picked by the low seven address bits");
   const uint32_t a_lane = (uint32_t)(c32 * A_ROW_BYTES + (((X16 ? 4 * h : h) ^ ((c32 >> 1) & 7)) * 16));
   const uint32_t b_lane = (uint32_t)(S::A_STAGE + strip * S::BLOCKS * 4096 + c32 * 64 + ((h ^ ((c32 >> 2) & 3)) * 16));
-  const uint32_t sc_lane = (uint32_t)(S::A_STAGE + S::B_STAGE + (2 * strip + c32 / 16) * 256 + 64 * h + 8 * (c32 % 8));
+  const uint32_t sc_lane = S::A_STAGE + S::B_STAGE + (uint32_t)(strided ? strip * 1024 + 32 * c32 : (2 * strip + c32 / 16) * 256 + 64 * h + 8 * (c32 % 8));
+  const uint32_t sc_lane1 = sc_lane + (strided ? 16 : 128);
   epilogue_table<NFR, OUT == kRing16 ? 2 : 1, true, OUT == kRingMx>(kernel_args_late(), t, ops.dst, ops.beta, ops.gamma, tab);
   u32x2_t *tab_bias = (u32x2_t *)(tab + epilogue_table_bytes(MF)) + strip * 32 + c32;
   *tab_bias = u32x2_t{ops.bias[0], ops.bias[1]};
@@ -326,11 +378,28 @@ TAMD_DEVICE void ring_products(const Args &a, const Tile &t, uint8_t *lds, uint8
   auto read_b = [&](uint32_t buf, int q, int f) {
     return *(const uint4 *)(lds + ((buf + b_lane) ^ (uint32_t)(((q & 1) ^ f) * 32)) + f * 2048 + (q >> 1) * 4096);
   };
+  // groups past K, whose place the next row's or column's scales take: zero bytes
+  auto within = [&](int left, int n) {   // (of n groups, `left` of them before K ends)
+    if (left >= n) return 0xFFFFFFFFu;
+    const int steps = (left + 1 - h) / 2;
+    return steps > 0 ? 0xFFFFFFFFu >> (32 - 8 * steps) : 0u;
+  };
   // the column scales of a stage's steps, a byte each
-  auto take_w = [&](const uint2 &s0, const uint2 &s1, int p, uint32_t (&sw)[NF]) {
-    sw[0] = __builtin_amdgcn_perm(s1.x, s0.x, sc_sel);
-    sw[1] = __builtin_amdgcn_perm(s1.y, s0.y, sc_sel);
-    if (KA == 128 && (p & 1) != 0) sw[0] >>= 16, sw[1] >>= 16;
+  auto take_w = [&](const uint2 &s0, const uint2 &s1, int p, uint32_t buf, uint32_t (&sw)[NF]) {
+    if (S::STRIDED && KA == 128 && (p & 1) != 0) {   // the second half of the 256 K
+      sw[0] >>= 16, sw[1] >>= 16;
+    } else if (strided) {   // s0, s1: the first eight bytes of either column
+      const uint32_t third[NF] = {*(const uint32_t *)(lds + buf + sc_lane + 8), *(const uint32_t *)(lds + buf + sc_lane1 + 8)};
+      const uint2 of[NF] = {s0, s1};
+      const uint32_t keep = within(G - p * (KA / 32), 8);
+#pragma unroll
+      for (int f = 0; f < NF; ++f)
+        sw[f] = __builtin_amdgcn_perm(__builtin_amdgcn_perm(third[f], of[f].y, sc_sel[f]), __builtin_amdgcn_perm(of[f].y, of[f].x, sc_sel[f]), 0x05040100u) & keep;
+    } else {
+      sw[0] = __builtin_amdgcn_perm(s1.x, s0.x, sc_sel[0]);
+      sw[1] = __builtin_amdgcn_perm(s1.y, s0.y, sc_sel[1]);
+      if (!S::STRIDED && KA == 128 && (p & 1) != 0) sw[0] >>= 16, sw[1] >>= 16;   // (read again: registers)
+    }
   };
   // operand of step q (of 64 K), fragment i; of 16-bit rows of the u-th 16 K in it
   auto read_a = [&](uint32_t buf, int q, int i, int u = 0) {
@@ -358,7 +427,7 @@ TAMD_DEVICE void ring_products(const Args &a, const Tile &t, uint8_t *lds, uint8
     for (int q = 0; q < STEPS; ++q)
 #pragma unroll
       for (int f = 0; f < NF; ++f) raw[q][f] = read_b(buf, q, f);
-    take_w(*(const uint2 *)(lds + buf + sc_lane), *(const uint2 *)(lds + buf + sc_lane + 128), 0, sw);
+    take_w(*(const uint2 *)(lds + buf + sc_lane), *(const uint2 *)(lds + buf + sc_lane1), 0, buf, sw);
 #pragma unroll
     for (int i = 0; i < NFR; ++i) af[0][i] = read_a(buf, 0, i);
 #pragma unroll 1
@@ -378,7 +447,7 @@ TAMD_DEVICE void ring_products(const Args &a, const Tile &t, uint8_t *lds, uint8
 #pragma unroll
           for (int f = 0; f < NF; ++f) raw_next[q][f] = read_b(ahead, q, f);
         }
-        if (v == 2) s0 = *(const uint2 *)(lds + ahead + sc_lane), s1 = *(const uint2 *)(lds + ahead + sc_lane + 128);
+        if (v == 2) s0 = *(const uint2 *)(lds + ahead + sc_lane), s1 = *(const uint2 *)(lds + ahead + sc_lane1);
 #pragma unroll
         for (int f = 0; f < NF; ++f) {
           const uint32_t codes = u == 0 ? raw[q][f].x : (u == 1 ? raw[q][f].y : (u == 2 ? raw[q][f].z : raw[q][f].w));
@@ -391,7 +460,7 @@ TAMD_DEVICE void ring_products(const Args &a, const Tile &t, uint8_t *lds, uint8
       for (int q = 0; q < STEPS; ++q)
 #pragma unroll
         for (int f = 0; f < NF; ++f) raw[q][f] = raw_next[q][f];
-      take_w(s0, s1, p + 1, sw);
+      take_w(s0, s1, p + 1, ahead, sw);
       buf = ahead;
     }
   } else {
@@ -400,20 +469,15 @@ TAMD_DEVICE void ring_products(const Args &a, const Tile &t, uint8_t *lds, uint8
     for (int i = 0; i < NFR; ++i) sa[i] = 0x7F7F7F7Fu;
     auto row_scales = [&](int p, uint32_t buf) {
       if constexpr (XMX) {
-        // bytes h, 2 + h, ... of the stage's groups; zero bytes for groups past K, whose place the next row's scales take
-        const int left = G - p * (KA / 32);
-        uint32_t within = 0xFFFFFFFFu;
-        if (left < KA / 32) {
-          const int steps = (left + 1 - h) / 2;
-          within = steps > 0 ? 0xFFFFFFFFu >> (32 - 8 * steps) : 0u;
-        }
+        // bytes h, 2 + h, ... of the stage's groups
+        const uint32_t keep = within(G - p * (KA / 32), KA / 32);
         const uint32_t *words = (const uint32_t *)(lds + buf + S::A_STAGE + S::B_STAGE + S::SC_STAGE) + c32;
 #pragma unroll
         for (int i = 0; i < NFR; ++i) {
           auto word = [&](int j) { return words[j * S::XS_WAVES * kWave + i * 32]; };
           sa[i] = __builtin_amdgcn_perm(word(1), word(0), xs_sel[i]);
           if constexpr (KA == 256) sa[i] = __builtin_amdgcn_perm(__builtin_amdgcn_perm(word(2), word(1), xs_sel[i]), sa[i], 0x05040100u);
-          sa[i] &= within;
+          sa[i] &= keep;
         }
       }
     };
@@ -433,12 +497,12 @@ TAMD_DEVICE void ring_products(const Args &a, const Tile &t, uint8_t *lds, uint8
       typename RowMma<XDT>::frag_t af[NFR];
 #pragma unroll
       for (int i = 0; i < NFR; ++i) af[i] = read_a(buf, 0, i);
-      const uint2 s0 = *(const uint2 *)(lds + buf + sc_lane), s1 = *(const uint2 *)(lds + buf + sc_lane + 128);
+      const uint2 s0 = *(const uint2 *)(lds + buf + sc_lane), s1 = *(const uint2 *)(lds + buf + sc_lane1);
       if constexpr (NB > 1) {
 #pragma unroll
         for (int f = 0; f < NF; ++f) raw[NB - 1][f] = read_b(buf, 1, f);
       }
-      take_w(s0, s1, p, sw);
+      take_w(s0, s1, p, buf, sw);
       if constexpr (XMX && !(FP4 && NFR >= 3)) row_scales(p, buf);
       // (the operands of the next step are requested one by one behind the last MFMA that uses those of this one)
 #define TAMD_STEP(q)                                                                                                        \

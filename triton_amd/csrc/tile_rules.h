@@ -56,10 +56,10 @@ inline bool known_block(int block_m) { return block_m == 16 || block_m == 32 || 
 
 inline int64_t output_size(int dtype) { return dtype == TAMD_F32 ? 4 : (dtype == TAMD_FP8_E4M3 || dtype == TAMD_FP8_E5M2 ? 1 : 2); }
 
-// What the persistent kernel of few rows per slice (moe_matmul_ring.h) covers: ragged problems with weights in 4 KB blocks, pre-shuffled scales, outputs of
-// the usual type in pairs of columns that 32-bit offsets reach.
+// What the persistent kernel of few rows per slice (moe_matmul_ring.h) covers: ragged problems with weights in 4 KB blocks and pre-shuffled scales or both strided
+// along K, outputs of the usual type in pairs of columns that 32-bit offsets reach.
 inline bool ring_applicable(const tamd_matmul_args &a) {
-  if (!a.block_schedule || a.w_layout != TAMD_W_CDNA4_BLOCKS || a.w_mx_layout != TAMD_SCALE_CDNA4) return false;
+  if (!a.block_schedule || (a.w_layout == TAMD_W_CDNA4_BLOCKS) != (a.w_mx_layout == TAMD_SCALE_CDNA4)) return false;
   if (a.n_experts > 256 || (a.N + 63) / 64 > 0x8000 || ((int64_t)a.M + a.n_experts) * ((a.N + 63) / 64) > 0x7FFFFFF0) return false;
   const bool x16 = a.x_dtype == TAMD_BF16 || a.x_dtype == TAMD_F16, sw = a.activation == TAMD_ACT_SWIGLU;
   if (!x16 && a.x_dtype != TAMD_FP8_E4M3 && a.x_dtype != TAMD_MXFP4) return false;
@@ -70,6 +70,20 @@ inline bool ring_applicable(const tamd_matmul_args &a) {
   const bool flex = a.y_expected_scale || a.y_actual_scale;
   if (x16) return !a.y_mx_scale && !flex && a.y_dtype == a.x_dtype;
   return a.y_dtype == TAMD_FP8_E4M3 || (a.y_dtype == TAMD_BF16 && !flex);
+}
+
+// Strided weights come in pieces of 64 bytes, at 3 to 4.7 TB/s in either kernel, and the copies no longer run ahead of anything over several rounds
+// (1.0 to 1.05 there): it is the faster where most CUs have no tile or one and narrower tiles share them out, and for the larger blocks of 16-bit
+// rows.  4000 products, time over the tiled kernel's, where it is taken: packed rows 0.83, MXFP8 0.89, fp8 0.89, 16-bit rows 0.93; one in ten above 1.04.
+inline int ring_rows_strided(const tamd_matmul_args &a, double cover, double tiles) {
+  if (a.x_dtype == TAMD_BF16 || a.x_dtype == TAMD_F16) {
+    if (cover <= 16.0 || cover > 64.0) return 0;
+    if (cover <= 32.0) return tiles > 0.3 && tiles <= 1.0 ? 32 : 0;
+    return (tiles > 0.5 && tiles <= 1.0) || tiles > 2.0 ? 64 : 0;
+  }
+  const bool packed = a.x_dtype == TAMD_MXFP4;
+  if (cover > (packed ? 64.0 : 32.0) || tiles > 0.75 || tiles <= (packed ? 0.0 : a.x_mx_scale ? 0.15 : 0.3)) return 0;
+  return cover <= 32.0 ? 32 : 64;
 }
 
 // Rows of the persistent kernel's blocks, 0 where another kernel is the faster (or the only one).  The block is the smallest that covers a slice's mean size and
@@ -84,6 +98,7 @@ inline int ring_rows(const tamd_matmul_args &a, int cus) {
   if (!ring_applicable(a)) return 0;
   const double mean = (double)a.M / a.n_experts, cover = mean + 2.0 * sqrt(mean);
   const double tiles = live_slices(a) * ((a.N + 255) / 256) / cus;
+  if (a.w_layout != TAMD_W_CDNA4_BLOCKS) return ring_rows_strided(a, cover, tiles);
   if (mean > 96.0 || (a.K < 1024 && tiles > 1.0)) return 0;
   const bool alone = tiles <= 1.0;
   if (a.x_dtype == TAMD_BF16 || a.x_dtype == TAMD_F16) {
