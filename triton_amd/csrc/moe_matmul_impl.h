@@ -341,20 +341,20 @@ constexpr int A_ROW_BYTES = 128;       // LDS bytes per activation row per stage
 constexpr int B_BYTES = 4 * 64 * 64;   // 4 waves x 64 columns x 64 bytes (128 K of fp4)
 // LDS of the K pipeline.  Row blocks of 128: two activation stages, one weight stage (4 KB per wave), the e8m0 scales
 // of the whole tile staged once.  Row blocks of at most 32 (KS = 1): the counted waits and stages of one of two K groups.
-// K groups (KS = 2 or 4, row blocks of at most 32 rows): KS groups of four waves share a tile, each taking a contiguous part of
-// K through a pipeline of its own with counted waits, three or four activation stages and one or two weight stages; their
+// K groups (KS = 2 on tiles of four strips, 8 on tiles of two; row blocks of at most 32 rows): KS groups of a wave per strip share a tile, each taking a contiguous part of
+// K through a pipeline of its own with counted waits, four activation stages and two weight stages (two and one); their
 // partial sums meet in LDS.  A problem with fewer tiles than the part has CUs is bound by what one wave per SIMD can issue (a
 // copy instruction holds its wave for about a hundred cycles); more waves per SIMD fill those gaps.
 struct PipeShape {
   int da, db;        // activation / weight stages
   int bytes;
 };
-constexpr PipeShape pipe_shape(int lds_rows, int ks = 1) {
+constexpr PipeShape pipe_shape(int lds_rows, int ks = 1, int strips = 4) {
   PipeShape p{};
   const bool deep = ks == 2 || (ks == 1 && lds_rows <= 32);
-  p.da = deep ? 4 : (ks == 4 ? 3 : 2);
+  p.da = deep ? 4 : 2;
   p.db = deep ? 2 : 1;
-  p.bytes = p.da * lds_rows * 128 + p.db * B_BYTES;
+  p.bytes = p.da * lds_rows * 128 + p.db * strips * (B_BYTES / 4);
   return p;
 }
 
@@ -378,7 +378,7 @@ constexpr int ring_outstanding(int DA, int DB, int NA, int NB, bool odd) {
 }
 static_assert(ring_outstanding(4, 2, 1, 4, false) == 6 && ring_outstanding(4, 2, 1, 4, true) == 10, "ring bookkeeping");
 static_assert(ring_outstanding(3, 2, 2, 4, false) == 6 && ring_outstanding(3, 2, 2, 4, true) == 6, "ring bookkeeping");
-static_assert(ring_outstanding(3, 1, 1, 4, false) == 1 && ring_outstanding(3, 1, 1, 4, true) == 5, "ring bookkeeping");
+static_assert(ring_outstanding(2, 1, 2, 4, false) == 0 && ring_outstanding(2, 1, 2, 4, true) == 4, "ring bookkeeping");
 
 // Flexpoint actual scale: the wave's max|result| by one atomic; positive floats order like their bit patterns.
 TAMD_DEVICE void store_actual_scale(float *actual, uint32_t amax, float out_max, int lane) {
@@ -871,7 +871,7 @@ TAMD_DEVICE late_args_t &kernel_args_late() {
 // are copied as they lie.  The wave reads the region into registers at the start of the stage and immediately
 // requests the next 128 K into it, so weights need no barrier.
 // Loops: two stages and full waits; counted waits over a deeper ring (K groups), see pipe_shape.
-template <int XDT, int NFR, int LDS_ROWS, int ACT, bool SC_LDS, int KS = 1>
+template <int XDT, int NFR, int LDS_ROWS, int ACT, bool SC_LDS, int KS = 1, int NS = 4>
 TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds_wg) {
   typedef Mma<XDT> M;
   typedef typename M::frag_t frag_t;
@@ -879,15 +879,17 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
   constexpr int KA = A_ROW_BYTES / ESZ;       // K per activation stage
   constexpr int A_STAGE = LDS_ROWS * A_ROW_BYTES;
   constexpr bool DEEP = KS > 1 || LDS_ROWS <= 32;   // counted waits
-  static_assert(!DEEP || (SC_LDS && NFR == 1 && (KS == 1 || KS == 2 || KS == 4)), "counted waits: scales in LDS, one row fragment");
-  constexpr PipeShape PS = pipe_shape(LDS_ROWS, KS);
+  static_assert(!DEEP || (SC_LDS && NFR == 1 && (KS == 1 || KS == 2 || KS == 8)), "counted waits: scales in LDS, one row fragment");
+  static_assert(NS == 4 || (NS == 2 && KS > 1), "a tile is four strips of 64 columns, with K groups two or four");
+  constexpr PipeShape PS = pipe_shape(LDS_ROWS, KS, NS);
   constexpr int DA = PS.da, DB = PS.db;
+  constexpr int COLS = 64 * NS, WB_STAGE = NS * 4096;
   auto a_slot = [](int it) { return DA == 2 ? (it & 1) : it % DA; };
   constexpr uint32_t kOob = 0x7FFFFFFFu;
   const int tid = threadIdx.x;
-  // K group of the wave (0 unless KS > 1) and its place among the group's four waves
-  const int grp = KS > 1 ? __builtin_amdgcn_readfirstlane(tid / 256) : 0;
-  const int wave = KS > 1 ? __builtin_amdgcn_readfirstlane((tid / kWave) & 3) : tid / kWave, lane = tid % kWave;
+  // K group of the wave (0 unless KS > 1) and its place among the group's NS waves, one per strip
+  const int grp = KS > 1 ? __builtin_amdgcn_readfirstlane(tid / (kWave * NS)) : 0;
+  const int wave = KS > 1 ? __builtin_amdgcn_readfirstlane((tid / kWave) & (NS - 1)) : tid / kWave, lane = tid % kWave;
   const int c32 = lane % 32, h = lane / 32;
   const int K = a.K, N = a.N, G = K / 32;
   // a wave whose 64 columns lie beyond N (last column tile) copies its share of the activations and keeps the
@@ -910,33 +912,33 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
   const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds;
   const uint32_t lds_b = lds_base + DA * A_STAGE + wave * 4096;
   const uint8_t *bbuf = lds + DA * A_STAGE + wave * 4096;
-  uint8_t *lds_sc = KS > 1 ? lds_wg + KS * PIPE_G : lds + DA * A_STAGE + DB * B_BYTES;
+  uint8_t *lds_sc = KS > 1 ? lds_wg + KS * PIPE_G : lds + DA * A_STAGE + DB * WB_STAGE;
 
   // ---- scales of the whole tile, once.  Strided: 256 columns x G bytes, contiguous in memory.  CDNA4
   // pre-shuffle: the tile's 8 blocks of 32 columns are contiguous too (KSP*32 bytes each); byte
   // 256*(k/8) + 64*(k%4) + 4*(n%16) + 2*((k%8)/4) + (n%32)/16 of a block is the scale of (group k, column n).
   const bool cdna4 = a.w_mx_layout == TAMD_SCALE_CDNA4;
   const int KSP = (G + 7) / 8 * 8;
-  const int tile_cols = N - t.n0 < BLOCK_N ? N - t.n0 : BLOCK_N;
+  const int tile_cols = N - t.n0 < COLS ? N - t.n0 : COLS;
   const int64_t sc_tile_off = cdna4 ? (int64_t)(t.n0 / 32) * KSP * 32 : (int64_t)t.n0 * G;
   auto stage_scales = [&]() {
   if constexpr (SC_LDS) {
     const uint8_t *sc_src = s_base + sc_tile_off;
-    const int sc_tile_bytes = BLOCK_N * (cdna4 ? KSP : G);
+    const int sc_tile_bytes = COLS * (cdna4 ? KSP : G);
     const int sc_avail = cdna4 ? ((N + 31) / 32 * 32 - t.n0) * KSP : (N - t.n0) * G;  // bytes up to the expert's end
     if (cdna4 || ((((uintptr_t)sc_src) & 15) == 0 && (N * G) % 16 == 0)) {
       // by DMA, 1 KB per instruction: in flight together with the first activation / weight stages and
       // awaited with them at the first barrier of the K loop
       const v4i_t rs = make_rsrc(sc_src, (uint32_t)sc_avail);
       const uint32_t lds_sc_addr = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds_sc;
-      for (int i = wave + 4 * grp; i * 1024 < sc_tile_bytes; i += 4 * KS)
+      for (int i = wave + NS * grp; i * 1024 < sc_tile_bytes; i += NS * KS)
         dma16(rs, lds_sc_addr + i * 1024, i * 1024 + lane * 16, 0);
     } else {
       const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)sc_src, 0, (uint32_t)(tile_cols * G),
                                                                         0x00020000);
-      const int n_dw = (BLOCK_N * G + 3) / 4;
+      const int n_dw = (COLS * G + 3) / 4;
       const int avail = tile_cols * G;
-      for (int i = tid; i < n_dw; i += 256 * KS) {
+      for (int i = tid; i < n_dw; i += kWave * NS * KS) {
         uint32_t v;
         if (i * 4 + 4 <= avail || i * 4 >= avail) {
           v = __builtin_amdgcn_raw_buffer_load_b32(rs, i * 4, 0, 0);  // whole, or wholly outside (zeros)
@@ -970,15 +972,17 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
 
   // Copies per request, as the counted waits of the ring loops below see them (a wave's copies complete in the order
   // of their requests): the loops of the issue_* functions run to these numbers and the waits are written in them.
-  constexpr int CP_A = NFR;        // issue_a: one copy per row fragment
+  constexpr int PIECES = 4 / NS;   // (of eight rows of a fragment, NS pieces apart)
+  constexpr int CP_A = NFR * PIECES;   // issue_a: one copy per row fragment and piece
   constexpr int CP_B = 4;          // issue_b: four 1 KB pieces
   // ---- activation DMA: one instruction per 32-row fragment, lane -> (row 8w + lane/8, slot lane%8)
   const int a_rin = wave * 8 + lane / 8;
   const int a_chunk = (lane % 8) ^ ((a_rin >> 1) & 7);
   // Rows past the end of the slice are never stored: they are copied as zeros (out-of-range offset), which keeps the matrix
   // cores' inputs quiet for the padding of a ragged tile.
-  uint32_t a_off[NFR];
+  uint32_t a_off[CP_A];
   const int row0 = t.start_m + t.off_m;
+  auto piece = [](int i) { return i / PIECES * 32 + i % PIECES * (8 * NS); };   // first row of copy i, of wave 0
   auto row_off = [&](int r, uint32_t src) { return r < t.rows ? src * (uint32_t)(a.x_stride_m * ESZ) + a_chunk * 16 : kOob; };
   // The rows' indices are the first thing requested, and the first weights, which do not depend on them, while they come.  They
   // travel by LDS, each in front of the row pieces that the wave will copy there (an ordinary load would be waited for with a count
@@ -987,14 +991,14 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
   const int idx_at = wave * 8 * A_ROW_BYTES;
   if (a.gather_indx) {
 #pragma unroll
-    for (int i = 0; i < NFR; ++i) dma4(rg, lds_base + idx_at + i * 32 * A_ROW_BYTES, (uint32_t)(i * 32 + a_rin) * 4u, 0);
+    for (int i = 0; i < CP_A; ++i) dma4(rg, lds_base + idx_at + piece(i) * A_ROW_BYTES, (uint32_t)(piece(i) + a_rin) * 4u, 0);
   }
   auto rows_known = [&](auto newer) {   // (after `newer` further requests of the wave)
     if (a.gather_indx) wait_vmcnt<decltype(newer)::value>();
 #pragma unroll
-    for (int i = 0; i < NFR; ++i) {
-      const int at = idx_at + i * 32 * A_ROW_BYTES + lane * 4;
-      a_off[i] = row_off(i * 32 + a_rin, a.gather_indx ? *(const uint32_t *)(lds + at) : (uint32_t)(row0 + i * 32 + a_rin));
+    for (int i = 0; i < CP_A; ++i) {
+      const int at = idx_at + piece(i) * A_ROW_BYTES + lane * 4;
+      a_off[i] = row_off(piece(i) + a_rin, a.gather_indx ? *(const uint32_t *)(lds + at) : (uint32_t)(row0 + piece(i) + a_rin));
     }
     if (a.gather_indx) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // read before the rows are copied over them
   };
@@ -1037,10 +1041,10 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
     const uint32_t akill = kb + a_chunk * (16 / ESZ) < k_hi ? 0u : kOob;
     const uint32_t sb = lds_base + a_slot(it) * A_STAGE + wave * 8 * A_ROW_BYTES;
 #pragma unroll
-    for (int i = 0; i < CP_A; ++i) dma16(rx, sb + i * 32 * A_ROW_BYTES, a_off[i] | akill, kb * ESZ);
+    for (int i = 0; i < CP_A; ++i) dma16(rx, sb + piece(i) * A_ROW_BYTES, a_off[i] | akill, kb * ESZ);
   };
   auto issue_b = [&](int sup) {
-    const uint32_t region = DB == 2 ? (uint32_t)(sup & 1) * B_BYTES : 0u;
+    const uint32_t region = DB == 2 ? (uint32_t)(sup & 1) * WB_STAGE : 0u;
     if constexpr (!DEEP) sup = sup < n_kb ? sup : n_kb - 1;
     const int kb = k0 + sup * KB;
     static_assert(CP_B == 4, "dma16_x4 makes four copies");
@@ -1064,7 +1068,7 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
       for (int q = 0; q < 2; ++q) {
         const int pos = f * 32 + c32;
         const int rot = ((pos >> 2) & 3) ^ (f << 1);   // slot of part p of position pos: p ^ rot
-        raw[f][q] = *(const uint4 *)(bbuf + (DB == 2 ? (sup & 1) * B_BYTES : 0) + pos * 64 + (((2 * q + h) ^ rot) * 16));
+        raw[f][q] = *(const uint4 *)(bbuf + (DB == 2 ? (sup & 1) * WB_STAGE : 0) + pos * 64 + (((2 * q + h) ^ rot) * 16));
         // group kg = 4*sup + 2q + h of this lane's column.  Strided: byte kg, kept inside the column's G bytes
         // (groups past the end of K meet zero codes and zero activations; their scale only has to be some finite
         // value of this column).  Pre-shuffled: byte 256*(kg/8) + 64*(kg%4) + 2*((kg%8)/4); the padding up to a
@@ -1168,9 +1172,9 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
     // The groups' partial sums meet in LDS (the pipelines are dead: after the barrier every copy has landed and every
     // operand has been read): group g > 0 leaves its accumulators in plane g - 1 and ends; group 0 adds the planes in
     // the order of the groups and finishes the tile alone (a barrier waits only for the waves that are still alive).
-    // (16 bytes per lane and access: a plane is [4 waves][NF x 4 quads][64 lanes] of four accumulators)
+    // (16 bytes per lane and access: a plane is [NS waves][NF x 4 quads][64 lanes] of four accumulators)
     f32x4_t *red = (f32x4_t *)lds_wg;
-    constexpr int PLANE = 4 * NF * 4 * kWave;
+    constexpr int PLANE = NS * NF * 4 * kWave;
     sync_threads();
     if (grp > 0) {
 #pragma unroll
@@ -1213,17 +1217,18 @@ struct TileShape {
 };
 
 // BM: block size of the ragged schedule the kernel consumes (16..128).
-template <int XDT, int BM, int ACT, bool SC_LDS, int KS = 1>
+template <int XDT, int BM, int ACT, bool SC_LDS, int KS = 1, int NS = 4>
 TAMD_DEVICE void tile_entry(const tamd_matmul_args &a, int grid_n, int64_t grid_total, int group_m, uint8_t *lds) {
   typedef TileShape<XDT, BM> S;
   Tile t;
   if (group_m < 0) {  // from the slices' sizes; up to -group_m blocks of an expert together
     if (!locate_tile_live<BM, S::EXTRA>(a, grid_n, -group_m, t)) return;
   } else if (!locate_tile<BM, S::EXTRA>(a, grid_n, grid_total, group_m, t)) return;
+  t.n0 = t.n0 / BLOCK_N * (64 * NS);
   const int nfr = (t.rows + 31) / 32;  // active row fragments (workgroup uniform)
 #define TAMD_CASE(n)                                                                     \
   case n:                                                                                \
-    if constexpr (n <= S::MF) run_tile<XDT, n, S::LDS_ROWS, ACT, SC_LDS, KS>(a, t, lds); \
+    if constexpr (n <= S::MF) run_tile<XDT, n, S::LDS_ROWS, ACT, SC_LDS, KS, NS>(a, t, lds); \
     break;
   switch (nfr) { TAMD_CASE(1) TAMD_CASE(2) TAMD_CASE(3) TAMD_CASE(4) TAMD_CASE(5) }
 #undef TAMD_CASE
@@ -1236,12 +1241,12 @@ __global__ __launch_bounds__(256, 2) void mm_x16_mxfp4_kernel(tamd_matmul_args a
   tile_entry<XDT, BM, ACT, SC_LDS>(a, grid_n, grid_total, group_m, lds);
 }
 
-// K groups: KS x 4 waves per tile of at most 32 rows, scales of the tile in LDS (see pipe_shape).
-template <int XDT, int BM, int ACT, int KS>
-__global__ __launch_bounds__(256 * KS, 1) void mm_x16_mxfp4_kgroups_kernel(tamd_matmul_args a, int grid_n, int64_t grid_total,
+// K groups: KS x NS waves per tile of at most 32 rows and NS strips, scales of the tile in LDS (see pipe_shape).
+template <int XDT, int BM, int ACT, int KS, int NS>
+__global__ __launch_bounds__(kWave * NS * KS, 1) void mm_x16_mxfp4_kgroups_kernel(tamd_matmul_args a, int grid_n, int64_t grid_total,
                                                                             int group_m) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-  tile_entry<XDT, BM, ACT, true, KS>(a, grid_n, grid_total, group_m, lds);
+  tile_entry<XDT, BM, ACT, true, KS, NS>(a, grid_n, grid_total, group_m, lds);
 }
 
 // Whether a problem takes locate_tile_live: it is ragged and the experts fit the lanes.
@@ -1273,24 +1278,31 @@ int launch_x16_act(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
   group_m = group_m < 1 ? 1 : (group_m > 16 ? 16 : group_m);
   if (counts_live_blocks(a)) group_m = -group_m;
   if constexpr (BM <= 32) {
-    // Fewer tiles than CUs and K above 1344: K groups, so that every SIMD of the CUs that do get a tile holds two to four
-    // waves (the groups' pipelines and the tile's scales have to fit one CU's LDS).  Shorter K pays for the exchange of the
-    // partial sums more than it gains (over 700 layers with up to 256 tiles of 32 rows: without groups 0.89 of the time at K
-    // 600, 0.96 at 1200, 1.06 at 2100, 1.2 at 3600, 1.35 at 5000).
+    // Fewer tiles than CUs: K groups, so that every SIMD of the CUs that do get a tile holds two to four waves (the groups' pipelines and the tile's scales
+    // have to fit one CU's LDS).
+    // Up to half as many tiles as CUs: tiles of 128 columns on twice as many CUs, eight groups, K of 928 to 7168.  A wave then has half the stages to wait for;
+    // against four groups on 256 columns 300 products take 0.57 to 0.95 of the time (256 x 2048 x 4096, block layout, 13.4 -> 11.5 us; 208 x 2656 x 2848 19.9 -> 14.3; 46 rows of 3
+    // slices, 6496 x 352, 32.5 -> 19.0).  Shorter K pays for the exchange of the partial sums more than it gains (K 800 1.0 to 1.1 of launch_mx's time, 500 1.25).
+    // Four groups and two such tiles per CU for up to 256 tiles: 0.95 to 1.1, not taken.
+    // Else two groups on 256 columns from K 1312 on (over 700 layers with up to 256 tiles of 32 rows: without groups 0.96 of the time at K
+    // 1200, 1.06 at 2100, 1.2 at 3600, 1.35 at 5000).
     int cus = 0;
     if (int rc = cu_count(cus)) return rc;
     const int64_t pairs = (a.K + KB - 1) / KB;
-    // (four groups where they fit beside the scales -- K up to 5632 --, else two)
-    constexpr size_t PIPE4 = 4 * (size_t)pipe_shape(LDS_ROWS, 4).bytes;
-    constexpr size_t PIPE2 = 2 * (size_t)pipe_shape(LDS_ROWS, 2).bytes;
-    const bool four = total * 2 <= cus && PIPE4 + sc_bytes <= 156 * 1024;
-    const int ks = pairs < 11 ? 1 : (four ? 4 : (total <= cus ? 2 : 1));
-    const size_t pipe = four ? PIPE4 : PIPE2;
-    if (ks > 1 && dense_sc && pipe + sc_bytes <= 156 * 1024) {
-      void (*kk)(tamd_matmul_args, int, int64_t, int) =
-          ks == 4 ? mm_x16_mxfp4_kgroups_kernel<XDT, BM, ACT, 4> : mm_x16_mxfp4_kgroups_kernel<XDT, BM, ACT, 2>;
+    constexpr size_t PIPE8 = 8 * (size_t)pipe_shape(LDS_ROWS, 8, 2).bytes, PIPE2 = 2 * (size_t)pipe_shape(LDS_ROWS, 2).bytes;
+    const int64_t sc_half = (sc_bytes / 2 + 1023) / 1024 * 1024;
+    if (dense_sc && pairs >= 8 && total * 2 <= cus && PIPE8 + sc_half <= 156 * 1024) {
+      auto kk = mm_x16_mxfp4_kgroups_kernel<XDT, BM, ACT, 8, 2>;
       if (int rc = raise_lds_limit_once((const void *)kk)) return rc;
-      kk<<<dim3((unsigned)launch), 256 * ks, pipe + sc_bytes, st>>>(a, grid_n, total, (int)group_m);
+      const int grid128 = (a.N + 127) / 128;
+      const int64_t tiles = (int64_t)grid_m * grid128;
+      kk<<<dim3((unsigned)((tiles + 7) / 8 * 8)), 1024, PIPE8 + sc_half, st>>>(a, grid128, tiles, (int)group_m);
+      return launch_status();
+    }
+    if (dense_sc && pairs >= 11 && total <= cus && PIPE2 + sc_bytes <= 156 * 1024) {
+      auto kk = mm_x16_mxfp4_kgroups_kernel<XDT, BM, ACT, 2, 4>;
+      if (int rc = raise_lds_limit_once((const void *)kk)) return rc;
+      kk<<<dim3((unsigned)launch), 512, PIPE2 + sc_bytes, st>>>(a, grid_n, total, (int)group_m);
       return launch_status();
     }
   }
