@@ -858,6 +858,40 @@ TAMD_DEVICE late_args_t &kernel_args_late() {
   return *p;
 }
 
+// The K groups' partial sums of one row fragment meet in LDS: group g > 0 leaves its accumulators in plane g - 1 and ends (false); group 0 adds the planes in
+// the order of the groups and finishes the tile alone (a barrier waits only for the waves that are still alive).
+// (16 bytes per lane and access: a plane is [NS waves][NF x 4 quads][64 lanes] of four accumulators)
+template <int KS, int NS>
+TAMD_DEVICE bool k_groups_add(f32x16_t (&acc)[NF], uint8_t *lds, int grp, int wave) {
+  const int lane = threadIdx.x % kWave;
+  f32x4_t *red = (f32x4_t *)lds;
+  constexpr int PLANE = NS * NF * 4 * kWave;
+  if (grp > 0) {
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        red[(grp - 1) * PLANE + ((wave * NF + f) * 4 + j) * kWave + lane] = f32x4_t{acc[f][4 * j], acc[f][4 * j + 1], acc[f][4 * j + 2], acc[f][4 * j + 3]};
+  }
+  sync_threads();
+  if (grp > 0) return false;
+#pragma unroll
+  for (int g = 1; g < KS; ++g)
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const f32x4_t v = red[(g - 1) * PLANE + ((wave * NF + f) * 4 + j) * kWave + lane];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[f][4 * j + e] += v[e];
+      }
+  // (added here: left for the epilogue, which has several forms, the planes would not fit the registers until then)
+#pragma unroll
+  for (int f = 0; f < NF; ++f) asm volatile("" : "+v"(acc[f]));
+  sync_threads();   // the epilogue's tables take the same memory
+  return true;
+}
+
 // One output tile with NFR (compile time) active 32-row fragments.
 // LDS: [A stages (2 to 4) | B: 4 wave-private regions, one or two stages | the e8m0 scales of the whole tile]; with K groups (KS > 1) one such pipeline per group, the tile's scales behind them.
 //
@@ -1169,37 +1203,8 @@ TAMD_DEVICE void run_tile(const tamd_matmul_args &a, const Tile &t, uint8_t *lds
   wait_dma();
 
   if constexpr (KS > 1) {
-    // The groups' partial sums meet in LDS (the pipelines are dead: after the barrier every copy has landed and every
-    // operand has been read): group g > 0 leaves its accumulators in plane g - 1 and ends; group 0 adds the planes in
-    // the order of the groups and finishes the tile alone (a barrier waits only for the waves that are still alive).
-    // (16 bytes per lane and access: a plane is [NS waves][NF x 4 quads][64 lanes] of four accumulators)
-    f32x4_t *red = (f32x4_t *)lds_wg;
-    constexpr int PLANE = NS * NF * 4 * kWave;
-    sync_threads();
-    if (grp > 0) {
-#pragma unroll
-      for (int f = 0; f < NF; ++f)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          red[(grp - 1) * PLANE + ((wave * NF + f) * 4 + j) * kWave + lane] =
-              f32x4_t{acc[0][f][4 * j], acc[0][f][4 * j + 1], acc[0][f][4 * j + 2], acc[0][f][4 * j + 3]};
-    }
-    sync_threads();
-    if (grp > 0) return;
-#pragma unroll
-    for (int g = 1; g < KS; ++g)
-#pragma unroll
-      for (int f = 0; f < NF; ++f)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const f32x4_t v = red[(g - 1) * PLANE + ((wave * NF + f) * 4 + j) * kWave + lane];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) acc[0][f][4 * j + e] += v[e];
-        }
-    // (added here: left for the epilogue, which has several forms, the planes would not fit the registers until then)
-#pragma unroll
-    for (int f = 0; f < NF; ++f) asm volatile("" : "+v"(acc[0][f]));
-    sync_threads();   // the epilogue's tables take the same memory
+    sync_threads();   // (the pipelines are dead: every copy has landed and every operand has been read)
+    if (!k_groups_add<KS, NS>(acc[0], lds_wg, grp, wave)) return;
   }
   // (the wave's own weight region is free by now: its table goes there)
   uint8_t *tab = KS > 1 ? lds_wg + wave * 4096 : lds + DA * A_STAGE + wave * 4096;

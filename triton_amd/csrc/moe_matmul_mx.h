@@ -67,16 +67,20 @@ struct RowMma<TAMD_BF16> : Mma<TAMD_BF16> {};
 template <>
 struct RowMma<TAMD_F16> : Mma<TAMD_F16> {};
 
-template <int XDT, int NFR, int BM, int ACT>
-TAMD_DEVICE void run_tile_mx(const tamd_matmul_args &a, const Tile &t, uint8_t *lds) {
+// KS > 1: K groups of NS waves share a tile of NS strips (blocks of up to 32 rows), as in moe_matmul_impl.h.
+template <int XDT, int NFR, int BM, int ACT, int KS = 1, int NS = 4>
+TAMD_DEVICE void run_tile_mx(const tamd_matmul_args &a, const Tile &t, uint8_t *lds_wg) {
   typedef MxShape<XDT, BM> S;
   constexpr bool FP4 = S::FP4, X16 = S::X16;
   constexpr int KA = S::KA, PLANES = S::PLANES, BLOCKS = S::BLOCKS, STEPS = KA / 64, A_STAGE = S::A_STAGE;
   constexpr int FMT = XDT == TAMD_MXFP4 ? 4 : (XDT == TAMD_FP8_E5M2 ? 1 : 0);
   constexpr uint32_t kOob = 0x7FFFFFFFu;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
+  const int wave_wg = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), wave = KS > 1 ? wave_wg % NS : wave_wg, grp = KS > 1 ? wave_wg / NS : 0;
+  static_assert(KS == 1 ? NS == 4 : NFR == 1 && !X16 && !S::PAIRS, "K groups: one row fragment, stages of 256 K");
+  const int lane = threadIdx.x % kWave;
   const int c32 = lane % 32, h = lane / 32;
   const int K = a.K, N = a.N, G = K / 32;
+  uint8_t *lds = lds_wg + grp * (2 * A_STAGE + NS * S::b_wave(true));
   const bool wave_live = t.n0 + wave * 64 < N;
   const v4i_t rx = make_rsrc((const uint8_t *)a.x + (int64_t)t.z * a.x_stride_z * S::ESZ, kOob);
   const v4i_t rw = make_rsrc((const uint8_t *)a.w + (int64_t)t.expert * a.w_stride_e, kOob);
@@ -86,6 +90,7 @@ TAMD_DEVICE void run_tile_mx(const tamd_matmul_args &a, const Tile &t, uint8_t *
   const uint32_t lds_b = lds_base + b_at;
   const uint8_t *bbuf = lds + b_at;
   const int n_k = (K + KA - 1) / KA;
+  const int n_p = (n_k + KS - 1) / KS, p0 = grp * n_p;   // the group's stages (past K: nothing is copied or multiplied)
   const bool x_mx = FP4 || (!X16 && a.x_mx_scale != nullptr);
 
   // ---- row indices: of the rows whose values the lane copies, and of the rows whose scales its MFMAs use; by LDS, each in front of
@@ -93,14 +98,18 @@ TAMD_DEVICE void run_tile_mx(const tamd_matmul_args &a, const Tile &t, uint8_t *
   const int a_rin = wave * 8 + lane / 8;
   const int a_chunk = (lane % 8) ^ ((a_rin >> 1) & 7);
   const int idx_at = wave * 8 * A_ROW_BYTES;
+  constexpr int PIECES = 4 / NS, CP_A = NFR * PIECES;   // copies of rows: eight of a fragment each, a wave's NS pieces apart
+  auto piece = [](int i) { return i / PIECES * 32 + i % PIECES * (8 * NS); };   // first row of copy i, of wave 0
   if (a.gather_indx) {
     const v4i_t rg = make_rsrc(a.gather_indx + t.start_m + t.off_m, (uint32_t)__builtin_amdgcn_readfirstlane(t.rows) * 4u);
 #pragma unroll
-    for (int i = 0; i < NFR; ++i) {
-      const int rs = i * 32 + c32;
-      const uint32_t to = lds_base + idx_at + i * 32 * A_ROW_BYTES;
-      dma4(rg, to, (uint32_t)(i * 32 + a_rin) * 4u, 0);
-      if constexpr (!X16) dma4(rg, to + 4 * kWave, (uint32_t)(rs < t.rows ? rs : t.rows - 1) * 4u, 0);
+    for (int i = 0; i < CP_A; ++i) dma4(rg, lds_base + idx_at + piece(i) * A_ROW_BYTES, (uint32_t)(piece(i) + a_rin) * 4u, 0);
+    if constexpr (!X16) {
+#pragma unroll
+      for (int i = 0; i < NFR; ++i) {
+        const int rs = i * 32 + c32;
+        dma4(rg, lds_base + idx_at + i * 32 * A_ROW_BYTES + 4 * kWave, (uint32_t)(rs < t.rows ? rs : t.rows - 1) * 4u, 0);
+      }
     }
   }
 
@@ -201,43 +210,48 @@ TAMD_DEVICE void run_tile_mx(const tamd_matmul_args &a, const Tile &t, uint8_t *
 #pragma unroll
       for (int j = 0; j < 16; ++j) acc[i][f][j] = 0.f;
 
-  uint32_t a_off[NFR];
+  uint32_t a_off[CP_A];
   auto issue_a = [&](int p) {   // (chunks past K are not read: zeros)
     constexpr int PLANE_K = S::PLANE_K, CHUNK_K = PLANE_K / 8;
 #pragma unroll
     for (int u = 0; u < PLANES; ++u) {
       const int kb = p * KA + u * PLANE_K;
       const uint32_t kill = kb + a_chunk * CHUNK_K < K ? 0u : kOob;
-      const uint32_t to = lds_base + (p & 1) * A_STAGE + u * S::ROWS * A_ROW_BYTES + wave * 8 * A_ROW_BYTES;
+      const uint32_t to = lds_base + ((p - p0) & 1) * A_STAGE + u * S::ROWS * A_ROW_BYTES + wave * 8 * A_ROW_BYTES;
 #pragma unroll
-      for (int i = 0; i < NFR; ++i) dma16(rx, to + i * 32 * A_ROW_BYTES, a_off[i] | kill, FP4 ? kb >> 1 : kb * S::ESZ);
+      for (int i = 0; i < CP_A; ++i) dma16(rx, to + piece(i) * A_ROW_BYTES, a_off[i] | kill, FP4 ? kb >> 1 : kb * S::ESZ);
     }
   };
 
   const uint32_t x_rows = gather_limit(a);
-  issue_b(0);
+  issue_b(p0);
   if (a.gather_indx) wait_vmcnt<4 * BLOCKS>();   // (the copies of the weights may be outstanding)
+  const int row0 = t.start_m + t.off_m;
+#pragma unroll
+  for (int i = 0; i < CP_A; ++i) {
+    const int r = piece(i) + a_rin;
+    const uint32_t src = a.gather_indx ? ((const uint32_t *)(lds + idx_at + piece(i) * A_ROW_BYTES))[lane] : (uint32_t)(row0 + r);
+    a_off[i] = r < t.rows && src < x_rows ? src * (uint32_t)(a.x_stride_m * S::ESZ) + a_chunk * 16 : kOob;
+  }
 #pragma unroll
   for (int i = 0; i < NFR; ++i) {
-    const int r = i * 32 + a_rin, rs = i * 32 + c32, row0 = t.start_m + t.off_m;
+    const int rs = i * 32 + c32;
     const uint32_t *idx = (const uint32_t *)(lds + idx_at + i * 32 * A_ROW_BYTES) + lane;
-    const uint32_t src = a.gather_indx ? idx[0] : (uint32_t)(row0 + r);
     const uint32_t srs = a.gather_indx ? idx[X16 ? 0 : kWave] : (uint32_t)(row0 + (rs < t.rows ? rs : t.rows - 1));
     // rows past the end of the slice are never stored: they are copied as zeros, which keeps the matrix cores' inputs quiet; so
     // is the row of an index that names none (-1), for which the first row's scales are read (ordinary loads have no descriptor that
     // would end with them) and zero bytes taken (selector 12)
-    a_off[i] = r < t.rows && src < x_rows ? src * (uint32_t)(a.x_stride_m * S::ESZ) + a_chunk * 16 : kOob;
     as_off[i] = srs < x_rows ? srs * (uint32_t)a.x_mx_stride_m : 0u;
     as_sel[i] = srs < x_rows ? kSel + (uint32_t)h * 0x01010101u : 0x0C0C0C0Cu;
   }
   if (a.gather_indx) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // read before the rows are copied over them
-  issue_a(0);
-  load_sc(0);
+  issue_a(p0);
+  load_sc(KA == 256 ? p0 : 0);
   const int swz = (c32 >> 1) & 7;
-  for (int p = 0; p < n_k; ++p) {
+  for (int p = p0; p < p0 + n_p; ++p) {
     wait_vmcnt<0>();   // (everything requested so far belongs to this stage)
     sync_threads();   // stage p is visible; every wave is done with the buffer that stage p + 1 goes to
-    const uint8_t *buf = lds + (p & 1) * A_STAGE;
+    const uint8_t *buf = lds + ((p - p0) & 1) * A_STAGE;
     uint4 raw[STEPS][NF];
 #pragma unroll
     for (int q = 0; q < STEPS; ++q)
@@ -278,7 +292,7 @@ TAMD_DEVICE void run_tile_mx(const tamd_matmul_args &a, const Tile &t, uint8_t *
     if (KA == 256 || (p & 1) == 1) load_sc(e + 1);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the weights are in registers: their buffer may be refilled
     issue_b(p + 1);
-    if (!wave_live) continue;
+    if (!wave_live || (KS > 1 && p >= n_k)) continue;
     if constexpr (X16) {
       // codes expanded in registers, the scale applied by the instruction
       typedef Mma<XDT> M;
@@ -316,6 +330,10 @@ TAMD_DEVICE void run_tile_mx(const tamd_matmul_args &a, const Tile &t, uint8_t *
     }
   }
   wait_vmcnt<0>();
+  if constexpr (KS > 1) {
+    sync_threads();   // (every copy has landed, every operand has been read)
+    if (!k_groups_add<KS, NS>(acc[0], lds_wg, grp, wave)) return;
+  }
   // (the wave's own weight region is free by now: its table goes there)
   tile_epilogue<NFR, ACT, X16 ? XDT : TAMD_BF16, !X16>(kernel_args_late(), t, acc, lds + b_at);
 }
@@ -339,6 +357,25 @@ __global__ __launch_bounds__(256, (MxShape<XDT, BM>::WGS)) void mm_mx_kernel(tam
 #undef TAMD_CASE
 }
 
+// Few tiles: four K groups of two waves on tiles of 128 columns.  A tile's stages wait for a trip to memory each, which only the tile's own waves could fill, and half of the
+// CUs and more have none: four times as many waves on twice as many CUs, a quarter of the stages each.  Tiled kernel -> this one, us: dense fp8, 256 x 2048 x 4096 10.1 -> 8.2, 208 x 2656 x
+// 2848, strided, 17.1 -> 11.1, 60 x 6144 x 3000 24.5 -> 14.0; layers: one packed token x 4 of 128 slices, 2880 -> 2880, 50.0 -> 38.4, one MXFP8 token x 4 of 32 44.6 -> 37.0, 100 fp8
+// tokens x 2 of 8, 5760 -> 768, 45.2 -> 36.2.
+// (mx_groups in tile_rules.h says which problems.)
+constexpr int kMxGroups = 4, kMxStrips = 2;
+template <int XDT, int BM>
+constexpr int kMxGroupsLds = kMxGroups * (2 * MxShape<XDT, BM>::A_STAGE + kMxStrips * MxShape<XDT, BM>::b_wave(true));
+template <int XDT, int BM, int ACT>
+__global__ __launch_bounds__(kWave * kMxGroups * kMxStrips, 1) void mm_mx_kgroups_kernel(tamd_matmul_args a, int grid_n, int64_t grid_total, int group_m) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  Tile t;
+  if (group_m < 0) {
+    if (!locate_tile_live<BM, 0>(a, grid_n, -group_m, t)) return;
+  } else if (!locate_tile<BM, 0>(a, grid_n, grid_total, group_m, t)) return;
+  t.n0 = t.n0 / BLOCK_N * (64 * kMxStrips);
+  run_tile_mx<XDT, 1, BM, ACT, kMxGroups, kMxStrips>(a, t, lds);
+}
+
 template <int XDT, int BM, int ACT>
 int launch_mx(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
   const int grid_n = (a.N + BLOCK_N - 1) / BLOCK_N;
@@ -352,6 +389,18 @@ int launch_mx(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
   int64_t group_m = rows_per_slice / BM;
   group_m = group_m > fit ? fit : group_m;
   group_m = group_m < 1 ? 1 : (group_m > 16 ? 16 : group_m);
+  if constexpr (BM <= 32 && !MxShape<XDT, BM>::X16) {
+    int cus = 0;
+    if (int rc = cu_count(cus)) return rc;
+    if (mx_groups(a, cus, BM)) {
+      auto kk = mm_mx_kgroups_kernel<XDT, BM, ACT>;
+      if (int rc = raise_lds_limit_once((const void *)kk)) return rc;
+      const int grid128 = (a.N + 127) / 128;
+      const int64_t tiles = (int64_t)grid_m * grid128;
+      kk<<<dim3((unsigned)((tiles + 7) / 8 * 8)), kWave * kMxGroups * kMxStrips, kMxGroupsLds<XDT, BM>, st>>>(a, grid128, tiles, (int)(counts_live_blocks(a) ? -group_m : group_m));
+      return launch_status();
+    }
+  }
   auto kern = mm_mx_kernel<XDT, BM, ACT>;
   if (int rc = raise_lds_limit_once((const void *)kern)) return rc;
   const bool blocks = a.w_layout == TAMD_W_CDNA4_BLOCKS;

@@ -56,6 +56,15 @@ inline bool known_block(int block_m) { return block_m == 16 || block_m == 32 || 
 
 inline int64_t output_size(int dtype) { return dtype == TAMD_F32 ? 4 : (dtype == TAMD_FP8_E4M3 || dtype == TAMD_FP8_E5M2 ? 1 : 2); }
 
+// Products of 8- and 4-bit rows x MXFP4 weights, row blocks of up to 32, that K groups share (moe_matmul_mx.h): up to half as many tiles of 256 columns as CUs, four
+// stages of 256 K and more.  1500 products, dense: K 769 to 1024 0.95 of the tiled kernel's time, 1025 to 1280 (two stages for some groups) 1.0, to 2048 0.83, to
+// 4096 0.74, to 8192 0.58; three stages 1.05.
+inline bool mx_groups(const tamd_matmul_args &a, int cus, int block_m) {
+  if (a.K <= 768 || block_m > 32) return false;
+  const double blocks = a.block_schedule ? live_slices(a) * ceil((double)a.M / a.n_experts / block_m) : (double)a.n_experts * ((a.M + block_m - 1) / block_m);
+  return 2.0 * blocks * ((a.N + 255) / 256) <= cus;
+}
+
 // What the persistent kernel of few rows per slice (moe_matmul_ring.h) covers: ragged problems with weights in 4 KB blocks and pre-shuffled scales or both strided
 // along K, outputs of the usual type in pairs of columns that 32-bit offsets reach.
 inline bool ring_applicable(const tamd_matmul_args &a) {
@@ -98,6 +107,9 @@ inline int ring_rows(const tamd_matmul_args &a, int cus) {
   if (!ring_applicable(a)) return 0;
   const double mean = (double)a.M / a.n_experts, cover = mean + 2.0 * sqrt(mean);
   const double tiles = live_slices(a) * ((a.N + 255) / 256) / cus;
+  // (K groups, mx_groups, against this kernel: MXFP8 0.65 to 0.9, fp8 0.6 to 0.95, packed rows 0.75 to 1.0; with more tiles 1.0 to 1.5)
+  const bool x8 = a.x_dtype == TAMD_FP8_E4M3;
+  if ((x8 || a.x_dtype == TAMD_MXFP4) && a.block_m <= 32 && a.K > 1280 && cover <= 32.0 && tiles <= (x8 && a.K > 2048 ? 0.375 : 0.25)) return 0;
   if (a.w_layout != TAMD_W_CDNA4_BLOCKS) return ring_rows_strided(a, cover, tiles);
   if (mean > 96.0 || (a.K < 1024 && tiles > 1.0)) return 0;
   const bool alone = tiles <= 1.0;
