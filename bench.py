@@ -11,9 +11,11 @@ product, routing, decode, fp8 down projection + combine, quantise, dequantise), 
 achieved rate, roofline fraction and parity flags.
 """
 import argparse
+import ctypes
 import gc
 import hashlib
 import json
+import math
 import os
 import re
 import sys
@@ -388,16 +390,34 @@ def product_kernel(args, rows, M, N, K, E):
     """Name of the kernel that a ragged product of M `rows` ("bf16", "fp8", "mx8", "mx4") x MXFP4 weights takes here."""
     from triton_amd.matmul_details.opt_flags import make_opt_flags, tiles_block_m
     from triton_amd.tensor import RaggedTensorMetadata
+    from triton_amd import _lib, _native
     streams = rows in ("bf16", "fp8") and K <= 4096 and N % 16 == 0    # (weights and scales are dense and aligned)
     block_m = args.block_m or tiles_block_m(make_opt_flags(M, N, K, E, True, fp8_rows=rows != "bf16").block_m, M, N, K, E, None, True,
                                             rows in ("fp8", "mx8"), not streams)
+    bag = _lib.MatmulArgBag()          # (the rule of the persistent kernel, for a plain product with 16-bit outputs)
+    bag.x_dtype = {"bf16": _lib.BF16, "mx4": _lib.MXFP4}.get(rows, _lib.FP8_E4M3)
+    bag.y_dtype, bag.w_dtype, bag.M, bag.N, bag.K, bag.n_experts, bag.block_m = _lib.BF16, _lib.MXFP4, M, N, K, E, block_m
+    bag.block_schedule, bag.y, bag.y_rows, bag.y_stride_m = 1 << 20, 1 << 20, M, N
+    if args.value_layout != "strided":
+        bag.w_layout = _lib.W_CDNA4_BLOCKS
+    if args.scale_layout != "strided":
+        bag.w_mx_layout = _lib.SCALE_CDNA4
+    if rows in ("mx8", "mx4"):
+        bag.x_mx_scale = 1 << 20
+    packed = bag.pack()
+    if _native.ring_rows(ctypes.addressof(packed), 256):
+        return "mm_ring_kernel"
     if block_m == 16 and streams:
         return "mm_stream16_kernel"
+    tiles = E * -(-N // 256) * -math.expm1(M * math.log1p(-1.0 / E)) if E > 1 else -(-N // 256)   # (slices that have rows)
+    if rows != "bf16" and block_m <= 32 and K > 768 and 2 * tiles * -(-M // (E * block_m)) <= 256:
+        return "mm_mx_kgroups_kernel"
     if rows != "bf16" or block_m == 64:
         return "mm_mx_kernel"
     if block_m == 128:
         return "mm_x16_mxfp4_kernel"
-    if K > 1344 and RaggedTensorMetadata.n_blocks(E, M, block_m) * -(-N // 256) <= 256:
+    tiles = RaggedTensorMetadata.n_blocks(E, M, block_m) * -(-N // 256)
+    if (896 < K <= 7168 and tiles <= 128) or (K > 1280 and tiles <= 256):
         return "mm_x16_mxfp4_kgroups_kernel"
     strided = args.value_layout == "strided" and args.scale_layout == "strided"
     return "mm_x16_mxfp4_kernel" if strided and K // 2 % 64 and K > 1024 and M // E <= 32 else "mm_mx_kernel"
@@ -832,7 +852,7 @@ def run_mlp(args, cfg, name):
                     scale_layout=args.scale_layout, value_layout=args.value_layout)
     out["stages"] = last["stages"]
     out["roofline"] = {"bound": "hbm", "achieved": round(gbs, 1), "peak": PEAK_HBM_GBS, "unit": "GB/s",
-                       "frac": round(gbs / PEAK_HBM_GBS, 4), "traffic": None, "kernel": "mm_mx_kernel (FC1 + FC2)",
+                       "frac": round(gbs / PEAK_HBM_GBS, 4), "traffic": None, "kernel": "mm_ring_kernel, mm_mx_kernel (FC1 + FC2)",
                        "kernel_ms": round(last["mm_ms"], 4), "algorithmic_flops": last["mm_flops"],
                        "algorithmic_bytes": last["mm_bytes"], "tflops": round(tflops, 1),
                        "frac_of_fp8_mfma_peak": round(tflops / PEAK_FP8_TFLOPS, 4)}
