@@ -60,6 +60,17 @@ SIZES = [(9, 10, 96, 2832), (4, 12, 352, 1872), (14, 16, 736, 1296), (20, 16, 14
          (40, 16, 608, 2608), (30, 60, 1248, 2320), (72, 32, 1056, 4368)]
 
 
+@pytest.mark.parametrize("layout", [dict(), dict(w_layout=_lib.W_STRIDED, w_mx_layout=_lib.SCALE_STRIDED, w_stride_k=1, w_stride_n=1440, w_mx_stride_k=1,
+                                                 w_mx_stride_n=90)])
+def test_fp8_rows_that_stream_stay_there(layout):
+    """Row blocks of 16 that the streaming kernel covers are summed exactly by it; other blocks, longer K and rows with block scales are not its."""
+    ptr = dict(w=1 << 20, w_mx_scale=1 << 20, block_offs=1 << 20, w_stride_e=2560 * 1440, w_mx_stride_e=2560 * 90, **layout)
+    for m in (40, 100):
+        assert ring_rows(m, 2560, 2880, 16, "fp8", block_m=16, **ptr) == 0
+        assert ring_rows(m, 2560, 2880, 16, "fp8", block_m=32, **ptr) == 32
+    assert ring_rows(100, 2560, 2880, 16, "mxfp8", block_m=16, **ptr) == 32
+
+
 def test_where_strided_weights_take_it():
     """Where a call leaves CUs without a tile, and 16-bit rows in blocks of 64 over several rounds; not with one side in the other layout."""
     both = dict(w_layout=_lib.W_STRIDED, w_mx_layout=_lib.SCALE_STRIDED)

@@ -109,6 +109,8 @@ inline int ring_rows(const tamd_matmul_args &a, int cus) {
   const double tiles = live_slices(a) * ((a.N + 255) / 256) / cus;
   // (K groups, mx_groups, against this kernel: MXFP8 0.65 to 0.9, fp8 0.6 to 0.95, packed rows 0.75 to 1.0; with more tiles 1.0 to 1.5)
   const bool x8 = a.x_dtype == TAMD_FP8_E4M3;
+  // (fp8 rows whose row blocks stream stay there: widened to bf16 their sums are 5e-9 off 64-bit ones, 4e-6 with the MFMA that takes them as they are)
+  if (x8 && a.block_m == 16 && stream16_applicable(a)) return 0;
   if ((x8 || a.x_dtype == TAMD_MXFP4) && a.block_m <= 32 && a.K > 1280 && cover <= 32.0 && tiles <= (x8 && a.K > 2048 ? 0.375 : 0.25)) return 0;
   if (a.w_layout != TAMD_W_CDNA4_BLOCKS) return ring_rows_strided(a, cover, tiles);
   if (mean > 96.0 || (a.K < 1024 && tiles > 1.0)) return 0;
