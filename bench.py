@@ -289,9 +289,9 @@ def run_dense(args, cfg, name):
     out["matmul_kernel_tflops"] = round(flops / (kernel_ms * 1e-3) / 1e12, 2)
     out["roofline"] = {"bound": "hbm", "achieved": round(gbs, 1), "peak": PEAK_HBM_GBS, "unit": "GB/s",
                        "frac": round(gbs / PEAK_HBM_GBS, 4), "traffic": None,
-                       # up to 80 tiles of 32 rows, or a forced block of 16: streaming kernel; 32-row tiles are shared by K groups
+                       # up to 72 tiles of 32 rows, or a forced block of 16: streaming kernel; 32-row tiles are shared by K groups
                        "kernel": {16: "mm_stream16_kernel", 32: "mm_x16_mxfp4_kgroups_kernel", 64: "mm_mx_kernel",
-                                  128: "mm_x16_mxfp4_kernel"}[args.block_m or (16 if -(-M // 32) * -(-N // 256) <= 80 else 32)],
+                                  128: "mm_x16_mxfp4_kernel"}[args.block_m or (16 if -(-M // 32) * -(-N // 256) <= 72 else 32)],
                        "kernel_ms": round(kernel_ms, 4), "algorithmic_bytes": alg_bytes, "algorithmic_flops": flops,
                        "event_pair_ms": round(event_ms, 4),
                        "note": "kernel_ms: 16 calls replayed as one HIP graph, per call (event pairs around single calls "

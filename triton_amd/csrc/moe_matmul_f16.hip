@@ -6,7 +6,7 @@
 
 namespace tamd {
 int dispatch_mm_f16(const tamd_matmul_args &a, int block_m, int grid_m, hipStream_t st) {
-  if (block_m == 0 && stream16_applicable(a) && !dense_prefers_tiles(a, 80)) {
+  if (block_m == 0 && stream16_applicable(a) && !dense_prefers_tiles(a, a.K > 2048 ? 48 : 72)) {
     // dense with few tiles: row blocks of 16 through the streaming kernel (every CU busy, weights re-read from L2)
     block_m = 16;
     grid_m = ((a.M + 15) / 16) * a.n_experts;

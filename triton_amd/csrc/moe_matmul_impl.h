@@ -1340,8 +1340,9 @@ int launch_x16_act(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
 }
 
 // Whether a dense / batched problem has enough 32-row tiles for the tiled kernels: more than `tiles`.  Fewer
-// run as 16-row blocks through the streaming kernel, whose units of 16 columns reach every CU.  (800 products: with 16-bit rows
-// 4 to 60 % faster up to 63 tiles, 18 to 50 % slower from 84 on; with fp8 rows the line is at 24 to 48.)
+// run as 16-row blocks through the streaming kernel, whose units of 16 columns reach every CU.  (900 products, time in tiles that K groups share over
+// the streaming kernel's: 16-bit rows, K up to 2048, 33 to 48 tiles 1.1 to 1.25, 65 to 72 0.94 to 1.04, 73 to 80 0.75 to 0.95; longer K, 17 to 32 1.06 to 1.28, 49 to 64 0.93 to 1.06, 65 to 80 0.7 to
+// 0.9.  fp8 rows would be faster in tiles from 24 on, 0.7 to 0.95, but their products are exact in the streaming kernel: 5e-9 off 64-bit sums, 4e-6 in tiles.)
 inline bool dense_prefers_tiles(const tamd_matmul_args &a, int tiles) {
   return (int64_t)((a.M + 31) / 32) * a.n_experts * ((a.N + BLOCK_N - 1) / BLOCK_N) > tiles;
 }
