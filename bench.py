@@ -397,7 +397,7 @@ def product_kernel(args, rows, M, N, K, E):
     bag = _lib.MatmulArgBag()          # (the rule of the persistent kernel, for a plain product with 16-bit outputs)
     bag.x_dtype = {"bf16": _lib.BF16, "mx4": _lib.MXFP4}.get(rows, _lib.FP8_E4M3)
     bag.y_dtype, bag.w_dtype, bag.M, bag.N, bag.K, bag.n_experts, bag.block_m = _lib.BF16, _lib.MXFP4, M, N, K, E, block_m
-    bag.block_schedule, bag.y, bag.y_rows, bag.y_stride_m = 1 << 20, 1 << 20, M, N
+    bag.block_schedule, bag.y, bag.y_rows, bag.y_stride_m, bag.force_variant = 1 << 20, 1 << 20, M, N, args.block_m or 0
     if args.value_layout != "strided":
         bag.w_layout = _lib.W_CDNA4_BLOCKS
     if args.scale_layout != "strided":

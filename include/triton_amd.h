@@ -266,7 +266,8 @@ typedef struct tamd_matmul_args {
   int activation; /* TAMD_ACT_* */
   float act_alpha, act_limit;
   int act_has_limit;
-  /* tuning overrides (0 = heuristic) */
+  /* tuning overrides (0 = heuristic).  Dense / batched: the row block.  Ragged: any other value keeps the product to the kernels
+   * that take the schedule's row blocks as they are (the persistent ones cut the slices into blocks of their own) */
   int force_variant;
   /* rows of x addressable through gather_indx (0 = M); x_rows * x_stride_m must stay below 2^30 elements */
   int64_t x_rows;

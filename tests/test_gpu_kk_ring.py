@@ -29,7 +29,7 @@ def test_where_it_is_taken():
     assert ring_rows(1200, 5760, 2880, 32) == 64 and ring_rows(4084, 5760, 2880, 32, True) == 160
     assert ring_rows(4, 3904, 1760, 8) == 0
     for changed in (dict(block_schedule=None), dict(n_experts=257), dict(y_dtype=_lib.F32), dict(y_rows=0), dict(y_rows=1 << 20), dict(K=248),
-                    dict(y_expected_scale=1 << 20), dict(N=5759), dict(y=(1 << 20) + 2), dict(y_stride_m=5761), dict(x_dtype=_lib.F16)):
+                    dict(y_expected_scale=1 << 20), dict(N=5759), dict(y=(1 << 20) + 2), dict(y_stride_m=5761), dict(x_dtype=_lib.F16), dict(force_variant=64)):
         assert ring_rows(4084, 5760, 2880, 32, **changed) == 0, changed
 
 

@@ -3,12 +3,14 @@ ring and off both, columns off strips and tiles, empty slices and slices of seve
 there, every kind of row and of output.  Rows of 8 and 4 bits give the bits of the tiled kernels, which strided weights with pre-shuffled scales take; 16-bit
 rows are held against float32 products."""
 import ctypes
+import sys
 
 import pytest
 import torch
 
 from triton_amd import _lib, _native
 from triton_amd.matmul import Epilogue, FlexCtx, FnSpecs, FusedActivation, InFlexData, OutFlexData, PrecisionConfig, matmul
+from triton_amd.matmul_details.opt_flags import scoped_opt_flags_constraints
 from triton_amd.numerics_details.mxfp import downcast_to_mxfp, upcast_from_mxfp
 from triton_amd.swiglu import swiglu_fn
 from triton_amd.tensor import FP4, convert_layout, make_ragged_tensor_metadata, wrap_torch_tensor
@@ -46,7 +48,7 @@ def test_where_it_is_taken():
         assert ring_rows(M, N, K, E, kind) == 0
     for changed in (dict(w_layout=_lib.W_STRIDED), dict(w_mx_layout=_lib.SCALE_STRIDED), dict(block_schedule=None), dict(n_experts=257),
                     dict(x_dtype=_lib.FP8_E5M2), dict(y_dtype=_lib.F32), dict(y_dtype=_lib.F16), dict(y_rows=0), dict(y_rows=1 << 20),
-                    dict(y_expected_scale=1 << 20), dict(N=5759), dict(y=(1 << 20) + 2), dict(y_stride_m=5761)):
+                    dict(y_expected_scale=1 << 20), dict(N=5759), dict(y=(1 << 20) + 2), dict(y_stride_m=5761), dict(force_variant=32)):
         assert ring_rows(512, 5760, 2880, 128, "fp8", **changed) == 0, changed
 
 
@@ -188,3 +190,40 @@ def test_edges(rows, E, K, N, kind, out, device):
     full, slack = full[there.to(device)], slack[there.to(device)]
     # a 16-bit result (2^-8) of K float32 additions, and the hardware's exponential and reciprocal (2^-20)
     assert bool(((got.float() - full).abs() <= 2.0 ** -8 * full.abs() + slack + 1e-5).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("constraint", [{"block_m": 16}, {"block_m": 32}, {"block_m": 64}, {"block_m": 128}, {"is_persistent": False}])
+@pytest.mark.parametrize("kind", ["mxfp4", "bf16 weights"])
+def test_not_where_blocks_are_asked_for(kind, constraint, monkeypatch, device):
+    """A product whose caller asks for a row block, or for no persistent kernel, runs in blocks of its schedule, with the same result."""
+    torch.manual_seed(5)
+    E, M, K, N = 40, 400, 1056, 2560
+    md = make_ragged_tensor_metadata(torch.full((E,), M // E, dtype=torch.int32, device=device), M)
+    x, w = torch.randn(M, K, device=device), (torch.randn(E, N, K, device=device) * 0.1).bfloat16()
+    opts = {}
+    if kind == "mxfp4":
+        w, ws = downcast_to_mxfp(w, torch.uint8, axis=-1)
+        x, s = downcast_to_mxfp(x, torch.uint8, axis=-1)
+        w, ws = blocks(w.transpose(1, 2), ws.transpose(1, 2))
+        opts = dict(a_mx_scale=s, a_microblock_size=32, b_mx_scale=ws, b_microblock_size=32, out_dtype=torch.bfloat16)
+    else:
+        x, w = x.bfloat16(), w.transpose(1, 2)
+    seen = []
+    module = sys.modules["triton_amd.matmul"]
+    launch = module._launch
+    monkeypatch.setattr(module, "_launch", lambda args, dev: seen.append(args) or launch(args, dev))
+    y = []
+    for c in ({"num_warps": 4}, constraint):   # (the first asks for nothing, through the general host path)
+        with scoped_opt_flags_constraints(c):
+            y.append(matmul(x, w, None, md, precision_config=PrecisionConfig(**opts)))
+    free, asked = seen
+    assert _native.ring_rows(ctypes.addressof(free), 256)
+    assert not _native.ring_rows(ctypes.addressof(asked), 256)
+    assert asked.block_m == constraint.get("block_m", asked.block_m)
+    if kind == "mxfp4":
+        assert torch.equal(y[0], y[1])
+    else:
+        # a 16-bit result (2^-8) of K float32 additions on either side
+        mag = torch.cat([x[10 * e:10 * e + 10].float().abs() @ w[e].float().abs() for e in range(E)])
+        assert bool(((y[0].float() - y[1].float()).abs() <= 2.0 ** -8 * y[0].float().abs() + K * 2.0 ** -22 * mag).all())

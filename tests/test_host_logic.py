@@ -102,6 +102,12 @@ def test_opt_flags_constraints_scope_and_errors():
     with OF.scoped_opt_flags_constraints({"is_persistent": True}):
         with pytest.raises(OF.InapplicableConstraint):
             OF.make_opt_flags(100, 64, 64, 1, False)
+    assert not OF.blocks_asked_for()
+    for asked, c in ((True, {"block_m": 64}), (True, {"is_persistent": False}), (False, {"block_m": None, "is_persistent": None}), (False, {"split_k": 1})):
+        with OF.scoped_opt_flags_constraints(c):
+            assert OF.blocks_asked_for() == asked
+    with OF.scoped_opt_flags(OF.OptFlags(block_m=64)):
+        assert OF.blocks_asked_for()
     OF.update_opt_flags_constraints({"block_m": 16})
     assert OF.make_opt_flags(16384, 5760, 2880, 128, True).block_m == 16
     OF.reset_opt_flags_constraints()

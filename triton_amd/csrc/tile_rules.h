@@ -68,7 +68,8 @@ inline bool mx_groups(const tamd_matmul_args &a, int cus, int block_m) {
 // What the persistent kernel of few rows per slice (moe_matmul_ring.h) covers: ragged problems with weights in 4 KB blocks and pre-shuffled scales or both strided
 // along K, outputs of the usual type in pairs of columns that 32-bit offsets reach.
 inline bool ring_applicable(const tamd_matmul_args &a) {
-  if (!a.block_schedule || (a.w_layout == TAMD_W_CDNA4_BLOCKS) != (a.w_mx_layout == TAMD_SCALE_CDNA4)) return false;
+  if (!a.block_schedule || a.force_variant) return false;
+  if ((a.w_layout == TAMD_W_CDNA4_BLOCKS) != (a.w_mx_layout == TAMD_SCALE_CDNA4)) return false;
   if (a.n_experts > 256 || (a.N + 63) / 64 > 0x8000 || ((int64_t)a.M + a.n_experts) * ((a.N + 63) / 64) > 0x7FFFFFF0) return false;
   const bool x16 = a.x_dtype == TAMD_BF16 || a.x_dtype == TAMD_F16, sw = a.activation == TAMD_ACT_SWIGLU;
   if (!x16 && a.x_dtype != TAMD_FP8_E4M3 && a.x_dtype != TAMD_MXFP4) return false;
@@ -141,7 +142,7 @@ inline int ring_rows(const tamd_matmul_args &a, int cus) {
 // What the persistent kernel for unquantised 16-bit weights (moe_matmul_kkring.h) covers, of the products that the tiled kernel of two operands along K
 // takes: ragged problems of four stages of K and more, outputs of the rows' type in pairs of columns that 32-bit offsets reach.
 inline bool kk_ring_applicable(const tamd_matmul_args &a) {
-  if (!a.block_schedule || a.K < 256 || a.n_experts > 256) return false;
+  if (!a.block_schedule || a.force_variant || a.K < 256 || a.n_experts > 256) return false;
   if ((a.x_dtype != TAMD_BF16 && a.x_dtype != TAMD_F16) || a.w_dtype != a.x_dtype || a.y_dtype != a.x_dtype) return false;
   if (a.y_mx_scale || a.y_expected_scale || a.y_actual_scale) return false;
   if ((a.N + 63) / 64 > 0x8000 || ((int64_t)a.M + a.n_experts) * ((a.N + 63) / 64) > 0x7FFFFFF0) return false;

@@ -454,6 +454,7 @@ def matmul(a, b, bias, a_ragged_metadata: Optional[RaggedTensorMetadata] = None,
         args.block_offs = md.block_offs(flags.block_m).data_ptr()
         args.block_schedule = md.block_schedule(flags.block_m).data_ptr()
         args.block_m = flags.block_m
+        args.force_variant = flags.block_m if _opt_flags.blocks_asked_for() else 0
         args.grid_m = RaggedTensorMetadata.n_blocks(md.n_slices, M, flags.block_m)
         # the kernels read up to grid_m entries of the schedule: metadata made for fewer rows than the matmul has is a
         # caller's mistake that must not become a read past the table

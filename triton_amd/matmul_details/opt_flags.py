@@ -77,6 +77,13 @@ CONSTRAINTS_SUPPORTED = frozenset({"block_m", "block_n", "block_k", "split_k", "
                                    "idle_sms", "max_allowable_mn", "num_warps", "disable_mx4_block_swap"})
 
 
+def blocks_asked_for() -> bool:
+    """Whether a ragged product has to run in the row blocks of its schedule: forced flags, a constraint on `block_m`, or one that
+    rules persistent kernels out (those cut the slices into blocks of their own, whatever block the schedule has)."""
+    c = _constraints()
+    return _opt_flags.get() is not None or c.get("block_m") is not None or c.get("is_persistent") not in (None, True)
+
+
 def max_allowable_mn(max_mn: int, m: int, n: int, split_k: int) -> int:
     """split_k only while the output is small (matmul_details/opt_flags.py:37-43)."""
     return 1 if m * n >= max_mn else split_k
@@ -128,8 +135,10 @@ def make_opt_flags(m: int, n: int, k: int, n_slices: int, ragged: bool,
 
     Constraints are validated as the reference validates them (opt_flags.py:71-73, 46-50): an unknown key is
     an AssertionError; a known key has to hold for the flags that come out, and since the tile's width, depth
-    and wave count are fixed in the kernels (256 columns, 128 K, 4 waves, no persistent kernel, no epilogue
-    sub-tiling, no idle CUs) any other value for them raises InapplicableConstraint instead of being dropped."""
+    and wave count are fixed in the kernels (256 columns, 128 K, 4 waves, no epilogue sub-tiling, no idle CUs) any
+    other value for them raises InapplicableConstraint instead of being dropped.  So does is_persistent = True: only
+    some ragged products have a persistent kernel, and which of them take it is the library's choice; a block_m or
+    is_persistent = False keeps a product off it (`blocks_asked_for`)."""
     forced = _opt_flags.get()
     if forced is not None:
         return forced
@@ -137,7 +146,7 @@ def make_opt_flags(m: int, n: int, k: int, n_slices: int, ragged: bool,
     unsupported = set(c) - CONSTRAINTS_SUPPORTED
     assert not unsupported, f"Given unsupported constraint: {unsupported}"
     if c.get("is_persistent"):
-        raise InapplicableConstraint("there is no persistent kernel on gfx950")
+        raise InapplicableConstraint("a persistent kernel cannot be asked for: some ragged products take one, by the library's choice")
     fixed = OptFlags(block_m=0)
     for key, have in (("block_n", fixed.block_n), ("block_k", fixed.block_k), ("num_warps", fixed.num_warps),
                       ("epilogue_subtile", 1), ("idle_sms", 0)):
