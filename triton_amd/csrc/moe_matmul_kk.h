@@ -416,9 +416,10 @@ int launch_kk(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
     }
   }
   // 16-bit weights of slices that hardly ever need two row blocks are copied non-temporally where their columns are whole lines and a call
-  // reads more of them (320 MB) than the 256 MB behind the L2s keep for the next one: 300 tokens x 4 of 32 slices, 2880 -> 2880, layer 342 -> 310 us,
-  // over 80 products 0.92 of the time.  Below that 1.0 to 1.5, with lines that two stages share 1.08 (0.95 to 1.3), and 1021 tokens x 4
-  // of 32, where a slice in eight has two blocks, 397 -> 410.
+  // reads more of them (320 MB) than the 256 MB behind the L2s keep for the next one.  Of what the persistent kernel leaves here, us, ordinary
+  // copies -> these: float32 outputs, K 2880, 1200 rows of 32 slices, N 5760 203 -> 192, N 2880 118 -> 108, 64 rows, N 5760 180 -> 161 (6.6 TB/s);
+  // 300 slices, K and N 1024, 300 rows 76 -> 66, 3000 rows 119 -> 108; dense, 8192 x 28672, 16 rows 115 -> 110, 64 rows 131 -> 130 (8192 x 24576
+  // 110 -> 111).  Below 320 MB 1.0 to 1.5 of the time, with lines that two stages share 1.08 (0.95 to 1.3).
   auto kern = mm_kk_kernel<XDT, BM, ACT, false>;
   if constexpr (!KK<XDT>::FP8) {
     const bool lines = aligned(a.w, 128) && (a.w_stride_n * 2) % 128 == 0 && (a.w_stride_e * 2) % 128 == 0;
