@@ -288,10 +288,15 @@ TAMD_DEVICE void run_tile_mx(const tamd_matmul_args &a, const Tile &t, uint8_t *
 #pragma unroll
       for (int f = 0; f < NF; ++f) sw[f] >>= 16;
     }
-    issue_a(p + 1);
-    if (KA == 256 || (p & 1) == 1) load_sc(e + 1);
+    // (the stage after a group's last is the next group's: copied for nothing, and waited for behind the loop, dense fp8 256 x 2048 x 4096 took
+    // 8.6 us instead of 8.1; without groups it lies past K, where nothing is read)
+    const bool more = KS == 1 || p + 1 < p0 + n_p;
+    if (more) {
+      issue_a(p + 1);
+      if (KA == 256 || (p & 1) == 1) load_sc(e + 1);
+    }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the weights are in registers: their buffer may be refilled
-    issue_b(p + 1);
+    if (more) issue_b(p + 1);
     if (!wave_live || (KS > 1 && p >= n_k)) continue;
     if constexpr (X16) {
       // codes expanded in registers, the scale applied by the instruction
@@ -357,10 +362,11 @@ __global__ __launch_bounds__(256, (MxShape<XDT, BM>::WGS)) void mm_mx_kernel(tam
 #undef TAMD_CASE
 }
 
-// Few tiles: four K groups of two waves on tiles of 128 columns.  A tile's stages wait for a trip to memory each, which only the tile's own waves could fill, and half of the
-// CUs and more have none: four times as many waves on twice as many CUs, a quarter of the stages each.  Tiled kernel -> this one, us: dense fp8, 256 x 2048 x 4096 10.1 -> 8.2, 208 x 2656 x
-// 2848, strided, 17.1 -> 11.1, 60 x 6144 x 3000 24.5 -> 14.0; layers: one packed token x 4 of 128 slices, 2880 -> 2880, 50.0 -> 38.4, one MXFP8 token x 4 of 32 44.6 -> 37.0, 100 fp8
-// tokens x 2 of 8, 5760 -> 768, 45.2 -> 36.2.
+// Few tiles: four K groups of two waves on tiles of 128 columns.  A tile's stages wait for a trip to memory each, which only the tile's own
+// waves could fill, and half of the CUs and more have none: four times as many waves on twice as many CUs, a quarter of the stages each.
+// Tiled kernel -> this one, us: dense fp8, 256 x 2048 x 4096 10.1 -> 8.1, 208 x 2656 x 2848, strided, 17.1 -> 10.9, 60 x 6144 x 3000
+// 24.5 -> 13.7; layers: one packed token x 4 of 128 slices, 2880 -> 2880, 50.0 -> 38.0, one MXFP8 token x 4 of 32 44.6 -> 35.9, 100 fp8 tokens x 2
+// of 8, 5760 -> 768, 45.2 -> 35.3.
 // (mx_groups in tile_rules.h says which problems.)
 constexpr int kMxGroups = 4, kMxStrips = 2;
 template <int XDT, int BM>
