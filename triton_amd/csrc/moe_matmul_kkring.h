@@ -12,7 +12,7 @@
 //     (300 tokens x 4 of 32 slices, 2880 -> 2 x 2880: 188 -> 170 us; of columns off the lines 137 -> 150 and 28 -> 34, so not there);
 //   * tiles of fewer strips where that fills the rounds over the workgroups (1021 tokens x 4 of 32: 228 -> 216); blocks of one slice are of one size.
 // Blocks of 160 rows, the most that three stages have LDS for (128: 1021 tokens 225, 2000 tokens 357 where 160 take 311; 96: 266 and 393); of 64 where slices
-// are smaller, whose copies of rows that are not there cost 2 to 4 % (300 tokens: 170 -> 165; 32 rows, ring of four: 208).
+// are smaller, whose copies of rows that are not there cost 2 to 4 % (300 tokens: 170 -> 165; blocks of 32 with a ring of four: 208).
 //
 // Products of 32 slices, 2880 -> 2 x 2880 with SwiGLU, tiled kernel -> now, us: 300 tokens x 4 176 -> 166 (6.4 TB/s), 600 197 -> 189, 1021 246 -> 216, 2000 389 -> 311;
 // 2880 -> 2880, 300 tokens 98 -> 88, 1021 130 -> 116; 4000 tokens x 4 of 16 slices 350 -> 262 (1.01 PFLOP/s).
@@ -31,14 +31,14 @@ struct KKRingShape {
   typedef typename KK<XDT>::frag_t frag_t;
   static constexpr int MF = MF_, ROWS = 32 * MF, KS = KK<XDT>::KS;
   static constexpr int N0 = (MF + 1) / 2;                                    // row fragments of a wave, at most
-  static constexpr int STAGE = (ROWS + BLOCK_N) * 128, RING = MF == 1 ? 4 : 3;
+  static constexpr int STAGE = (ROWS + BLOCK_N) * 128, RING = 3;
   static constexpr int COPIES = 8 + MF;                                      // of a copying wave and stage
   static constexpr int CONSUMERS = 8, THREADS = (CONSUMERS + kKKRingCopiers) * kWave;
   static constexpr int TABLE = N0 * 32 * 12;                                 // destinations, betas, gammas of half of the rows
   static constexpr int TABLE_AT = RING * STAGE, INDEX_AT = TABLE_AT + 2 * TABLE, TILE_AT = INDEX_AT + kKKRingCopiers * 256;
   static constexpr int LDS = TILE_AT + 4 * 32 + 16;
-  static constexpr int MIN_K = RING * KS;                                    // a tile's row indices are requested a tile ahead
   static_assert(LDS <= 160 * 1024 && (RING - 1) * COPIES < 64, "one workgroup per CU, copies that vmcnt can count");
+  static_assert(RING * KS <= 256, "a tile has RING stages and more (kk_ring_applicable): its row indices are requested a tile ahead");
 };
 
 // A tile: up to four strips of 64 columns from t.n0 on.
@@ -233,15 +233,11 @@ TAMD_DEVICE void kk_ring_copy(const Args &a, int group, bool nt, uint8_t *lds) {
     advance();
   }
   // the last RING - 1 stages, with nothing left to request
-  if constexpr (RING > 3) {
-    wait_vmcnt<2 * S::COPIES>();
-    sync_threads();
-  }
+  static_assert(RING == 3, "stages written out below");
   wait_vmcnt<S::COPIES>();
   sync_threads();
   wait_vmcnt<0>();
   sync_threads();
-  static_assert(RING == 3 || RING == 4, "stages written out above");
 }
 
 // A multiplying wave's part of a tile, NFR row fragments of one strip: the K loop and the epilogue.
