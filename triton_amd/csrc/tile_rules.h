@@ -51,6 +51,9 @@ inline double live_slices(const tamd_matmul_args &a) {
   return a.block_schedule ? -expm1(a.M * log1p(-1.0 / a.n_experts)) * a.n_experts : a.n_experts;
 }
 
+// The most of them that its rows can fall on.
+inline int most_live_slices(const tamd_matmul_args &a) { return a.M < a.n_experts ? a.M : a.n_experts; }
+
 // The row blocks that a ragged schedule may have.
 inline bool known_block(int block_m) { return block_m == 16 || block_m == 32 || block_m == 64 || block_m == 128; }
 
@@ -79,6 +82,8 @@ inline bool ring_applicable(const tamd_matmul_args &a) {
   if (!sw && (((a.N | (int)a.y_stride_m) & 1) != 0 || !aligned(a.y, 2 * (size_t)size))) return false;
   const bool flex = a.y_expected_scale || a.y_actual_scale;
   if (x16) return !a.y_mx_scale && !flex && a.y_dtype == a.x_dtype;
+  // (fp8 rows whose row blocks stream stay there: widened to bf16 their sums are 5e-9 off 64-bit ones, 4e-6 with the MFMA that takes them as they are)
+  if (a.x_dtype == TAMD_FP8_E4M3 && a.block_m == 16 && stream16_applicable(a)) return false;
   return a.y_dtype == TAMD_FP8_E4M3 || (a.y_dtype == TAMD_BF16 && !flex);
 }
 
@@ -106,17 +111,18 @@ inline int ring_rows_strided(const tamd_matmul_args &a, double cover, double til
 // over the time without: 16-bit rows 0.905, fp8 0.907, MXFP8 0.95, packed 0.914; more than 10 % slower in 1 to 2 % of them.
 inline int ring_rows(const tamd_matmul_args &a, int cus) {
   if (!ring_applicable(a)) return 0;
+  const bool x16 = a.x_dtype == TAMD_BF16 || a.x_dtype == TAMD_F16;
+  // (16-bit rows: no line lies below 0.3 tiles per CU; a few rows have fewer whichever slices they fall on)
+  if (x16 && 10.0 * most_live_slices(a) * ((a.N + 255) / 256) <= 3.0 * cus) return 0;
   const double mean = (double)a.M / a.n_experts, cover = mean + 2.0 * sqrt(mean);
   const double tiles = live_slices(a) * ((a.N + 255) / 256) / cus;
   // (K groups, mx_groups, against this kernel: MXFP8 0.65 to 0.9, fp8 0.6 to 0.95, packed rows 0.75 to 1.0; with more tiles 1.0 to 1.5)
   const bool x8 = a.x_dtype == TAMD_FP8_E4M3;
-  // (fp8 rows whose row blocks stream stay there: widened to bf16 their sums are 5e-9 off 64-bit ones, 4e-6 with the MFMA that takes them as they are)
-  if (x8 && a.block_m == 16 && stream16_applicable(a)) return 0;
   if ((x8 || a.x_dtype == TAMD_MXFP4) && a.block_m <= 32 && a.K > 1280 && cover <= 32.0 && tiles <= (x8 && a.K > 2048 ? 0.375 : 0.25)) return 0;
   if (a.w_layout != TAMD_W_CDNA4_BLOCKS) return ring_rows_strided(a, cover, tiles);
   if (mean > 96.0 || (a.K < 1024 && tiles > 1.0)) return 0;
   const bool alone = tiles <= 1.0;
-  if (a.x_dtype == TAMD_BF16 || a.x_dtype == TAMD_F16) {
+  if (x16) {
     if (cover <= 16.0 && a.K <= 4096) {
       const bool padded = a.K > 1024 && (a.K + 1023) / 1024 * 1024 >= 1.3 * a.K;
       return (alone && tiles > (mean < 3.0 ? 0.75 : 0.5)) || (padded && tiles > 2.0) ? 32 : 0;
@@ -156,6 +162,7 @@ inline bool kk_ring_applicable(const tamd_matmul_args &a) {
 // lose up to 1.21, where slices come in two.
 inline int kk_ring_rows(const tamd_matmul_args &a, int cus) {
   if (!kk_ring_applicable(a)) return 0;
+  if (a.M <= a.n_experts && 3 * (int64_t)most_live_slices(a) * ((a.N + 255) / 256) < cus) return 0;   // (the line below, whichever slices the rows fall on)
   const double mean = (double)a.M / a.n_experts, tiles = live_slices(a) * ((a.N + 255) / 256) / cus;
   if (3.0 * tiles * (mean > 160.0 ? mean / 160.0 : 1.0) < 1.0) return 0;
   return mean <= 48.0 ? 64 : 160;
