@@ -83,8 +83,8 @@ def test_where_strided_weights_take_it():
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("kind,rows,E,K,N", [("mxfp4", 9, 10, 96, 2832), ("mxfp4", 4, 12, 352, 1872), ("mxfp4", 30, 8, 1440, 1394), ("mxfp8", 9, 10, 96, 2832),
-                                             ("mxfp8", 9, 20, 736, 1298), ("fp8", 9, 20, 1056, 1298), ("fp8", 4, 12, 2144, 2832), ("bf16", 15, 20, 544, 1296),
+@pytest.mark.parametrize("kind,rows,E,K,N", [("mxfp4", 9, 10, 96, 2832), ("mxfp4", 4, 12, 544, 1872), ("mxfp4", 30, 8, 1440, 1394), ("mxfp8", 9, 10, 96, 2832),
+                                             ("mxfp8", 9, 20, 800, 1298), ("fp8", 9, 20, 1056, 1298), ("fp8", 4, 12, 2144, 2832), ("bf16", 15, 20, 800, 1296),
                                              ("f16", 30, 20, 1312, 2328), ("bf16", 40, 60, 1056, 2322)])
 @pytest.mark.parametrize("byte", [0, 1])
 def test_strided_edges(kind, rows, E, K, N, byte, device):
@@ -93,7 +93,7 @@ def test_strided_edges(kind, rows, E, K, N, byte, device):
     sizes[1] = 0
     M = int(sizes.sum())
     strided = dict(w_layout=_lib.W_STRIDED, w_mx_layout=_lib.SCALE_STRIDED)
-    assert ring_rows(M, N, K, E, kind, **strided)
+    assert ring_rows(M, N, K, E, kind, block_m=32, **strided)
     torch.manual_seed(K + N)
     w, ws = downcast_to_mxfp((torch.randn(E, N, K, device=device) * torch.exp(2 * torch.randn(E, N, 1, device=device))).bfloat16(), torch.uint8, axis=-1)
     room = torch.full((16 + w.numel(),), 0x55, dtype=torch.uint8, device=device)
@@ -133,7 +133,7 @@ def test_edges(rows, E, K, N, kind, out, device):
     sizes = torch.randint(max(0, rows - 9), rows + 10, (E,), generator=torch.Generator().manual_seed(rows), dtype=torch.int32)
     sizes[1], sizes[E // 2] = 0, 3 * rows
     M, T = int(sizes.sum()), 50
-    used = ring_rows(M, N, K, E, kind, to, swiglu)
+    used = ring_rows(M, N, K, E, kind, to, swiglu, block_m=32)
     if not used:
         pytest.skip("another kernel's")
     torch.manual_seed(K)
@@ -227,3 +227,60 @@ def test_not_where_blocks_are_asked_for(kind, constraint, monkeypatch, device):
         # a 16-bit result (2^-8) of K float32 additions on either side
         mag = torch.cat([x[10 * e:10 * e + 10].float().abs() @ w[e].float().abs() for e in range(E)])
         assert bool(((y[0].float() - y[1].float()).abs() <= 2.0 ** -8 * y[0].float().abs() + K * 2.0 ** -22 * mag).all())
+
+
+def test_where_stages_are_too_few():
+    """A tile alone on its CU with a K of few stages is the tiled kernel's, unless the blocks are those that stream; so are 16-bit rows of one stage in several rounds."""
+    strided = dict(w_layout=_lib.W_STRIDED, w_mx_layout=_lib.SCALE_STRIDED)
+    for K, rows in ((768, 0), (800, 32)):
+        assert ring_rows(400, 1296, K, 20, "bf16", block_m=32) == rows and ring_rows(400, 1296, K, 20, "f16", block_m=32, **strided) == rows
+        assert ring_rows(180, 1298, K, 20, "mxfp8", block_m=32) == rows and ring_rows(180, 1298, K, 20, "mxfp8", block_m=32, **strided) == rows
+    assert ring_rows(300, 768, 64, 60, "bf16", block_m=16) == 32
+    for K, rows in ((256, 32), (288, 0), (512, 0), (544, 32)):
+        assert ring_rows(40, 1872, K, 12, "mxfp4", block_m=32, **strided) == rows and ring_rows(40, 1872, K, 12, "mxfp4", block_m=32) == 32
+    assert ring_rows(500, 2608, 512, 12, "mxfp4", block_m=64) == 0 and ring_rows(500, 2608, 544, 12, "mxfp4", block_m=64) == 64
+    assert ring_rows(2400, 2322, 128, 60, "bf16", block_m=64, **strided) == 0 and ring_rows(2400, 2322, 160, 60, "bf16", block_m=64, **strided) == 64
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,rows,E,K,N,layout", [
+    ("bf16", 40, 60, 160, 2322, "strided"), ("f16", 40, 60, 256, 2322, "strided"), ("bf16", 40, 60, 384, 2322, "strided"), ("f16", 15, 20, 800, 1296, "strided"),
+    ("mxfp8", 9, 10, 96, 2832, "strided"), ("mxfp8", 9, 20, 800, 1298, "strided"), ("mxfp4", 9, 10, 256, 2832, "strided"), ("mxfp4", 4, 12, 544, 1872, "strided"),
+    ("fp8", 20, 20, 224, 1298, "strided"), ("bf16", 5, 60, 64, 768, "blocks"), ("f16", 9, 60, 96, 768, "blocks"), ("bf16", 9, 60, 352, 752, "blocks"),
+    ("mxfp8", 9, 20, 800, 1298, "blocks"), ("mxfp4", 9, 20, 288, 1298, "blocks"), ("fp8", 20, 20, 288, 1298, "blocks")])
+def test_few_stages(kind, rows, E, K, N, layout, monkeypatch, device):
+    """Fewer stages than the ring holds, one tile to a workgroup and several: as the tiled kernel has it, which blocks of 32 rows that a caller asks for take."""
+    sizes = torch.randint(max(0, rows - 4), rows + 5, (E,), generator=torch.Generator().manual_seed(K), dtype=torch.int32)
+    sizes[1] = 0
+    M = int(sizes.sum())
+    torch.manual_seed(K + N)
+    # (columns of other scales; float16 results stay below 65504: 140 000 columns of up to e^4.5 times sums of 800 products of normal values, 28 x 5)
+    w, ws = downcast_to_mxfp((torch.randn(E, N, K, device=device) * torch.exp(torch.randn(E, N, 1, device=device))).bfloat16(), torch.uint8, axis=-1)
+    wf = upcast_from_mxfp(w, ws, torch.float32, axis=-1).transpose(1, 2)
+    w, ws = w.transpose(1, 2), ws.transpose(1, 2)
+    if layout == "blocks":
+        w, ws = blocks(w, ws)
+    x, opts = torch.randn(50, K, device=device), {}
+    if kind[:2] == "mx":
+        x, s = downcast_to_mxfp(x, torch.uint8 if kind == "mxfp4" else torch.float8_e4m3fn, axis=-1)
+        opts.update(a_mx_scale=s, a_microblock_size=32)
+    else:
+        x = x.to(TYPES[kind])
+    gather = torch.randint(-1, 50, (M,), dtype=torch.int32, device=device)
+    bias, md = torch.randn(E, N, device=device), make_ragged_tensor_metadata(sizes.to(device), M)
+    took, y = [], []
+    module = sys.modules["triton_amd.matmul"]
+    launch = module._launch
+    monkeypatch.setattr(module, "_launch", lambda args, dev: took.append(_native.ring_rows(ctypes.addressof(args), 256)) or launch(args, dev))
+    for c in ({"num_warps": 4}, {"block_m": 32}):   # (the first asks for nothing, through the general host path)
+        with scoped_opt_flags_constraints(c):
+            y.append(matmul(x, w, bias, md, gather_indx=gather, precision_config=PrecisionConfig(
+                b_mx_scale=ws, b_microblock_size=32, out_dtype=torch.float16 if kind == "f16" else torch.bfloat16, **opts)))
+    assert took[0] and not took[1]
+    if kind not in ("bf16", "f16"):
+        assert torch.equal(y[0], y[1])
+        return
+    at = [0, *sizes.cumsum(0).tolist()]
+    mag = torch.cat([x.float().abs()[gather[at[e]:at[e + 1]].clamp(min=0).long()] @ wf[e].abs() for e in range(E)])
+    # (float32 sums in another order, a rounding to 16 bits on either side)
+    assert bool(((y[0].float() - y[1].float()).abs() <= 2.0 ** -7 * y[1].float().abs() + K * 2.0 ** -22 * mag + 1e-6).all())

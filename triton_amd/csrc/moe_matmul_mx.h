@@ -364,9 +364,9 @@ __global__ __launch_bounds__(256, (MxShape<XDT, BM>::WGS)) void mm_mx_kernel(tam
 
 // Few tiles: four K groups of two waves on tiles of 128 columns.  A tile's stages wait for a trip to memory each, which only the tile's own
 // waves could fill, and half of the CUs and more have none: four times as many waves on twice as many CUs, a quarter of the stages each.
-// Tiled kernel -> this one, us: dense fp8, 256 x 2048 x 4096 10.1 -> 8.1, 208 x 2656 x 2848, strided, 17.1 -> 10.9, 60 x 6144 x 3000
-// 24.5 -> 13.7; layers: one packed token x 4 of 128 slices, 2880 -> 2880, 50.0 -> 38.0, one MXFP8 token x 4 of 32 44.6 -> 35.9, 100 fp8 tokens x 2
-// of 8, 5760 -> 768, 45.2 -> 35.3.
+// Tiled kernel -> this one, us: dense fp8, 256 x 2048 x 4096 10.1 -> 8.1, 208 x 2656 x 2848, strided, 17.4 -> 10.9, 60 x 6144 x 3000
+// 24.9 -> 13.8; layers: one packed token x 4 of 128 slices, 2880 -> 2880, 45.4 -> 38.6, one MXFP8 token x 4 of 32 44.8 -> 35.7, 100 fp8 tokens x 2
+// of 8, 5760 -> 768, 45.9 -> 36.5.
 // (mx_groups in tile_rules.h says which problems.)
 constexpr int kMxGroups = 4, kMxStrips = 2;
 template <int XDT, int BM>

@@ -90,15 +90,29 @@ inline bool ring_applicable(const tamd_matmul_args &a) {
 // Strided weights come in pieces of 64 bytes, at 3 to 4.7 TB/s in either kernel, and the copies no longer run ahead of anything over several rounds
 // (1.0 to 1.05 there): it is the faster where most CUs have no tile or one and narrower tiles share them out, and for the larger blocks of 16-bit
 // rows.  4000 products, time over the tiled kernel's, where it is taken: packed rows 0.83, MXFP8 0.89, fp8 0.89, 16-bit rows 0.93; one in ten above 1.04.
+// (16-bit rows in blocks of 64 with 0.85 to 1.0 tiles per CU, slices spread as a router's: K 800 to 1200 1.00, to 1800 0.94, to 2880 0.89; with 1.0 to 1.15 1.06, 1.00, 0.94.)
 inline int ring_rows_strided(const tamd_matmul_args &a, double cover, double tiles) {
   if (a.x_dtype == TAMD_BF16 || a.x_dtype == TAMD_F16) {
     if (cover <= 16.0 || cover > 64.0) return 0;
     if (cover <= 32.0) return tiles > 0.3 && tiles <= 1.0 ? 32 : 0;
-    return (tiles > 0.5 && tiles <= 1.0) || tiles > 2.0 ? 64 : 0;
+    return (tiles > 0.5 && tiles <= 1.0) || (tiles > 2.0 && a.K > 128) ? 64 : 0;   // (K 32 to 96 1.05 of the tiled kernel's time, to 256 0.92)
   }
   const bool packed = a.x_dtype == TAMD_MXFP4;
   if (cover > (packed ? 64.0 : 32.0) || tiles > 0.75 || tiles <= (packed ? 0.0 : a.x_mx_scale ? 0.15 : 0.3)) return 0;
   return cover <= 32.0 ? 32 : 64;
+}
+
+// A tile alone on its CU wins by copies that run ahead, which takes stages: with fewer, the start of a workgroup of twelve waves and its table
+// cost more than they give, against tiles (not against streaming, the blocks of 16, which is slower still there).  Rows of 8 and 4 bits
+// win again where one stage or two are all of K.  4700 products of K 32 to 1500, time over the tiled kernel's:
+//   16-bit rows         strided K to 512 1.08, to 640 1.04, to 768 1.00, to 1500 0.96; 4 KB blocks to 512 1.15, to 640 1.07, to 768 1.05, to 1500 0.98
+//   MXFP8               strided K to 256 0.87, to 768 1.08; 4 KB blocks to 256 0.95, to 768 1.04
+//   fp8 and packed rows strided K to 256 0.89, to 512 1.04 (64 rows 1.09), to 768 1.01; 4 KB blocks to 512 0.99 (64 rows 1.06)
+inline bool ring_stages_too_few(const tamd_matmul_args &a, double cover) {
+  if (a.block_m <= 16) return false;
+  if (a.x_dtype == TAMD_BF16 || a.x_dtype == TAMD_F16) return a.K <= 768;
+  const bool scaled = a.x_dtype == TAMD_FP8_E4M3 && a.x_mx_scale;
+  return a.K > 256 && a.K <= (scaled ? 768 : 512) && (scaled || a.w_layout != TAMD_W_CDNA4_BLOCKS || cover > 32.0);
 }
 
 // Rows of the persistent kernel's blocks, 0 where another kernel is the faster (or the only one).  The block is the smallest that covers a slice's mean size and
@@ -119,6 +133,7 @@ inline int ring_rows(const tamd_matmul_args &a, int cus) {
   // (K groups, mx_groups, against this kernel: MXFP8 0.65 to 0.9, fp8 0.6 to 0.95, packed rows 0.75 to 1.0; with more tiles 1.0 to 1.5)
   const bool x8 = a.x_dtype == TAMD_FP8_E4M3;
   if ((x8 || a.x_dtype == TAMD_MXFP4) && a.block_m <= 32 && a.K > 1280 && cover <= 32.0 && tiles <= (x8 && a.K > 2048 ? 0.375 : 0.25)) return 0;
+  if (tiles <= 1.0 && ring_stages_too_few(a, cover)) return 0;
   if (a.w_layout != TAMD_W_CDNA4_BLOCKS) return ring_rows_strided(a, cover, tiles);
   if (mean > 96.0 || (a.K < 1024 && tiles > 1.0)) return 0;
   const bool alone = tiles <= 1.0;
@@ -135,7 +150,10 @@ inline int ring_rows(const tamd_matmul_args &a, int cus) {
   if (cover <= 32.0) {
     if (scaled) return alone || tiles > 2.0 ? 32 : 0;
     if (packed) return alone || tiles > 1.4 ? 32 : 0;
-    if (tiles > 6.0 && mean >= 12.0) return 64;   // (a slice in two blocks costs more than the larger ones: 509 tokens, 128 slices, 588 us, 601)
+    // (A slice in two blocks of 32 costs more than a block of 64, and a router picks some experts more often than others.  476 products with
+    // slices spread as a router's, 0.45 in the logarithm, time over that with blocks of 32: above 6 tiles per CU mean 12 to 16 0.989, to 23 0.964,
+    // below 12 0.999; up to 6 tiles 0.99 to 1.00 for any mean.  With even slices 1.00 to 1.01 throughout.)
+    if (tiles > 6.0 && mean >= 12.0) return 64;
     return (alone && tiles > (mean < 10.0 ? 0.27 : 0.1)) || tiles > 2.0 ? 32 : 0;
   }
   if (cover <= 64.0) return tiles > 2.0 || (alone && !scaled && tiles > (packed ? 0.0 : 0.6)) ? 64 : 0;
