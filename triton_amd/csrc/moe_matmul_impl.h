@@ -341,10 +341,10 @@ constexpr int A_ROW_BYTES = 128;       // LDS bytes per activation row per stage
 constexpr int B_BYTES = 4 * 64 * 64;   // 4 waves x 64 columns x 64 bytes (128 K of fp4)
 // LDS of the K pipeline.  Row blocks of 128: two activation stages, one weight stage (4 KB per wave), the e8m0 scales
 // of the whole tile staged once.  Row blocks of at most 32 (KS = 1): the counted waits and stages of one of two K groups.
-// K groups (KS = 2 on tiles of four strips, 8 on tiles of two; row blocks of at most 32 rows): KS groups of a wave per strip share a tile, each taking a contiguous part of
-// K through a pipeline of its own with counted waits, four activation stages and two weight stages (two and one); their
-// partial sums meet in LDS.  A problem with fewer tiles than the part has CUs is bound by what one wave per SIMD can issue (a
-// copy instruction holds its wave for about a hundred cycles); more waves per SIMD fill those gaps.
+// K groups (KS = 2 on tiles of four strips, 8 on tiles of two; row blocks of at most 32 rows): KS groups of a wave per strip share a tile,
+// each taking a contiguous part of K through a pipeline of its own with counted waits, four activation stages and two weight stages (two
+// and one); their partial sums meet in LDS.  A problem with fewer tiles than the part has CUs is bound by what one wave per SIMD can issue
+// (a copy instruction holds its wave for about a hundred cycles); more waves per SIMD fill those gaps.
 struct PipeShape {
   int da, db;        // activation / weight stages
   int bytes;
@@ -858,8 +858,8 @@ TAMD_DEVICE late_args_t &kernel_args_late() {
   return *p;
 }
 
-// The K groups' partial sums of one row fragment meet in LDS: group g > 0 leaves its accumulators in plane g - 1 and ends (false); group 0 adds the planes in
-// the order of the groups and finishes the tile alone (a barrier waits only for the waves that are still alive).
+// The K groups' partial sums of one row fragment meet in LDS: group g > 0 leaves its accumulators in plane g - 1 and ends (false); group 0
+// adds the planes in the order of the groups and finishes the tile alone (a barrier waits only for the waves that are still alive).
 // (16 bytes per lane and access: a plane is [NS waves][NF x 4 quads][64 lanes] of four accumulators)
 template <int KS, int NS>
 TAMD_DEVICE bool k_groups_add(f32x16_t (&acc)[NF], uint8_t *lds, int grp, int wave) {
@@ -893,7 +893,8 @@ TAMD_DEVICE bool k_groups_add(f32x16_t (&acc)[NF], uint8_t *lds, int grp, int wa
 }
 
 // One output tile with NFR (compile time) active 32-row fragments.
-// LDS: [A stages (2 to 4) | B: 4 wave-private regions, one or two stages | the e8m0 scales of the whole tile]; with K groups (KS > 1) one such pipeline per group, the tile's scales behind them.
+// LDS: [A stages (2 to 4) | B: 4 wave-private regions, one or two stages | the e8m0 scales of the whole tile]; with K groups (KS > 1) one
+// such pipeline per group, the tile's scales behind them.
 //
 // Both operands reach LDS by DMA.  Activations: 64 K per stage; wave w copies rows
 // 8w..8w+7 of every 32-row fragment (8 lanes x 16 B per row); chunk c of row r sits at slot
@@ -1283,11 +1284,12 @@ int launch_x16_act(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
   group_m = group_m < 1 ? 1 : (group_m > 16 ? 16 : group_m);
   if (counts_live_blocks(a)) group_m = -group_m;
   if constexpr (BM <= 32) {
-    // Fewer tiles than CUs: K groups, so that every SIMD of the CUs that do get a tile holds two to four waves (the groups' pipelines and the tile's scales
-    // have to fit one CU's LDS).
-    // Up to half as many tiles as CUs: tiles of 128 columns on twice as many CUs, eight groups, K of 928 to 7168.  A wave then has half the stages to wait for;
-    // against four groups on 256 columns 300 products take 0.57 to 0.95 of the time (256 x 2048 x 4096, block layout, 13.4 -> 11.5 us; 208 x 2656 x 2848 19.9 -> 14.3; 46 rows of 3
-    // slices, 6496 x 352, 32.5 -> 19.0).  Shorter K pays for the exchange of the partial sums more than it gains (K 800 1.0 to 1.1 of launch_mx's time, 500 1.25).
+    // Fewer tiles than CUs: K groups, so that every SIMD of the CUs that do get a tile holds two to four waves (the groups' pipelines and
+    // the tile's scales have to fit one CU's LDS).
+    // Up to half as many tiles as CUs: tiles of 128 columns on twice as many CUs, eight groups, K of 928 to 7168.  A wave then has half the
+    // stages to wait for; against four groups on 256 columns 300 products take 0.57 to 0.95 of the time (256 x 2048 x 4096, block layout,
+    // 13.4 -> 11.5 us; 208 x 2656 x 2848 19.9 -> 14.3; 46 rows of 3 slices, 6496 x 352, 32.5 -> 19.0).  Shorter K pays for the exchange of
+    // the partial sums more than it gains (K 800 1.0 to 1.1 of launch_mx's time, 500 1.25).
     // Four groups and two such tiles per CU for up to 256 tiles: 0.95 to 1.1, not taken.
     // Else two groups on 256 columns from K 1312 on (over 700 layers with up to 256 tiles of 32 rows: without groups 0.96 of the time at K
     // 1200, 1.06 at 2100, 1.2 at 3600, 1.35 at 5000).
@@ -1312,11 +1314,11 @@ int launch_x16_act(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
     }
   }
   if constexpr (BM <= 32) {
-    // Weights of slices of one row block whose columns do not start on 64 bytes: pieces of 64 bytes of a column, two and more stages
-    // ahead, instead of launch_mx's pieces of 128.  The other way round where columns are aligned, where slices share their weights'
-    // lines between row blocks, with pre-shuffled scales, and for short K (953 rows of 64 slices,
-    // 2496 x 3552: 77 us against 104; 539 x 2 of 60, 1024 x 5488, aligned: 48 against 38; 161 x 4 of 60, 3776 x 5488: 182 against 242; 1159 of 60, 5024 x 1616: 78 against 91; 157 x 2 of 16, 992 x 1392 11.5
-    // against 10.7).
+    // Weights of slices of one row block whose columns do not start on 64 bytes: pieces of 64 bytes of a column, two and more stages ahead,
+    // instead of launch_mx's pieces of 128.  The other way round where columns are aligned, where slices share their weights' lines between
+    // row blocks, with pre-shuffled scales, and for short K (953 rows of 64 slices, 2496 x 3552: 77 us against 104; 539 x 2 of 60, 1024 x
+    // 5488, aligned: 48 against 38; 161 x 4 of 60, 3776 x 5488: 182 against 242; 1159 of 60, 5024 x 1616: 78 against 91; 157 x 2 of 16, 992
+    // x 1392 11.5 against 10.7).
     constexpr int PIPE_BYTES = pipe_shape(LDS_ROWS).bytes;
     if (a.block_schedule && rows_per_slice <= LDS_ROWS && a.w_layout != TAMD_W_CDNA4_BLOCKS && a.w_stride_n % 64 != 0 && a.K > 1024 &&
         !cdna4 && dense_sc && PIPE_BYTES + sc_bytes <= 156 * 1024) {
@@ -1339,10 +1341,11 @@ int launch_x16_act(const tamd_matmul_args &a, int grid_m, hipStream_t st) {
   }
 }
 
-// Whether a dense / batched problem has enough 32-row tiles for the tiled kernels: more than `tiles`.  Fewer
-// run as 16-row blocks through the streaming kernel, whose units of 16 columns reach every CU.  (900 products, time in tiles that K groups share over
-// the streaming kernel's: 16-bit rows, K up to 2048, 33 to 48 tiles 1.1 to 1.25, 65 to 72 0.94 to 1.04, 73 to 80 0.75 to 0.95; longer K, 17 to 32 1.06 to 1.28, 49 to 64 0.93 to 1.06, 65 to 80 0.7 to
-// 0.9.  fp8 rows would be faster in tiles from 24 on, 0.7 to 0.95, but their products are exact in the streaming kernel: 5e-9 off 64-bit sums, 4e-6 in tiles.)
+// Whether a dense / batched problem has enough 32-row tiles for the tiled kernels: more than `tiles`.  Fewer run as 16-row blocks through
+// the streaming kernel, whose units of 16 columns reach every CU.  (900 products, time in tiles that K groups share over the streaming
+// kernel's: 16-bit rows, K up to 2048, 33 to 48 tiles 1.1 to 1.25, 65 to 72 0.94 to 1.04, 73 to 80 0.75 to 0.95; longer K, 17 to 32 1.06 to
+// 1.28, 49 to 64 0.93 to 1.06, 65 to 80 0.7 to 0.9.  fp8 rows would be faster in tiles from 24 on, 0.7 to 0.95, but their products are
+// exact in the streaming kernel: 5e-9 off 64-bit sums, 4e-6 in tiles.)
 inline bool dense_prefers_tiles(const tamd_matmul_args &a, int tiles) {
   return (int64_t)((a.M + 31) / 32) * a.n_experts * ((a.N + BLOCK_N - 1) / BLOCK_N) > tiles;
 }

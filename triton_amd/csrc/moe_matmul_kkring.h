@@ -1,21 +1,23 @@
-// Grouped (ragged) matmul of 16-bit activations x unquantised weights of their type, both contiguous along K: a persistent kernel whose copies never stop at
-// the end of a tile.
+// Grouped (ragged) matmul of 16-bit activations x unquantised weights of their type, both contiguous along K: a persistent kernel whose
+// copies never stop at the end of a tile.
 //
-// Bound by HBM up to some 150 rows per slice, then by the matrix units.  One tile per workgroup (moe_matmul_kk.h) starts with an empty pipeline, exchanges
-// partial sums and ends with an epilogue beside which it copies nothing, and its waves wait for their own copies between the products (one holds its
-// wave for a hundred cycles): 4.3 TB/s of the 6.4 to 7 that copies alone read, matrix cores busy 29 % of the cycles.  Here a workgroup owns a CU and walks over tiles:
-//   * four waves copy and do nothing else, through a ring of three stages (64 K of a tile's rows and columns, 128-byte lines of both) that runs on into the
-//     next tile; they find the tiles and leave them for the others in LDS;
+// Bound by HBM up to some 150 rows per slice, then by the matrix units.  One tile per workgroup (moe_matmul_kk.h) starts with an empty
+// pipeline, exchanges partial sums and ends with an epilogue beside which it copies nothing, and its waves wait for their own copies
+// between the products (one holds its wave for a hundred cycles): 4.3 TB/s of the 6.4 to 7 that copies alone read, matrix cores busy 29 %
+// of the cycles.  Here a workgroup owns a CU and walks over tiles:
+//   * four waves copy and do nothing else, through a ring of three stages (64 K of a tile's rows and columns, 128-byte lines of both) that
+//     runs on into the next tile; they find the tiles and leave them for the others in LDS;
 //   * eight waves multiply, two halves of the row fragments times four strips of 64 columns, and finish the tile from registers; the two or three
 //     stages ahead cover the copies for most of that time;
 //   * weights of slices with one row block are copied non-temporally where their columns are whole lines and the call reads more than the caches keep
 //     (300 tokens x 4 of 32 slices, 2880 -> 2 x 2880: 188 -> 170 us; of columns off the lines 137 -> 150 and 28 -> 34, so not there);
 //   * tiles of fewer strips where that fills the rounds over the workgroups (1021 tokens x 4 of 32: 228 -> 216); blocks of one slice are of one size.
-// Blocks of 160 rows, the most that three stages have LDS for (128: 1021 tokens 225, 2000 tokens 357 where 160 take 311; 96: 266 and 393); of 64 where slices
-// are smaller, whose copies of rows that are not there cost 2 to 4 % (300 tokens: 170 -> 165; blocks of 32 with a ring of four: 208).
+// Blocks of 160 rows, the most that three stages have LDS for (128: 1021 tokens 225, 2000 tokens 357 where 160 take 311; 96: 266 and 393);
+// of 64 where slices are smaller, whose copies of rows that are not there cost 2 to 4 % (300 tokens: 170 -> 165; blocks of 32 with a ring
+// of four: 208).
 //
-// Products of 32 slices, 2880 -> 2 x 2880 with SwiGLU, tiled kernel -> now, us: 300 tokens x 4 176 -> 166 (6.4 TB/s), 600 197 -> 189, 1021 246 -> 216, 2000 389 -> 311;
-// 2880 -> 2880, 300 tokens 98 -> 88, 1021 130 -> 116; 4000 tokens x 4 of 16 slices 350 -> 262 (1.01 PFLOP/s).
+// Products of 32 slices, 2880 -> 2 x 2880 with SwiGLU, tiled kernel -> now, us: 300 tokens x 4 176 -> 166 (6.4 TB/s), 600 197 -> 189, 1021
+// 246 -> 216, 2000 389 -> 311; 2880 -> 2880, 300 tokens 98 -> 88, 1021 130 -> 116; 4000 tokens x 4 of 16 slices 350 -> 262 (1.01 PFLOP/s).
 #pragma once
 #include <algorithm>
 
@@ -127,9 +129,9 @@ struct KKRingWork {
   }
 };
 
-// Copying waves: strip w's columns, rows 8 w .. of every row fragment.  Stage s goes to slot s % RING and is requested RING - 1 stages ahead; copies
-// complete in the order of their requests, so a stage has landed once only those of the stages after it are outstanding (the indices of the next tile's rows,
-// requested behind a tile's first stage, only make that wait a little longer).
+// Copying waves: strip w's columns, rows 8 w .. of every row fragment.  Stage s goes to slot s % RING and is requested RING - 1 stages
+// ahead; copies complete in the order of their requests, so a stage has landed once only those of the stages after it are outstanding (the
+// indices of the next tile's rows, requested behind a tile's first stage, only make that wait a little longer).
 template <int XDT, int MF, typename Args>
 TAMD_DEVICE void kk_ring_copy(const Args &a, int group, bool nt, uint8_t *lds) {
   typedef KKRingShape<XDT, MF> S;

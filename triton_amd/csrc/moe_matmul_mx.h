@@ -20,9 +20,9 @@
 // Before -> now, layers: packed rows, widening included, 2048 tokens, 128 experts (top-4) 531 -> 471 us, 2331 over 16 (top-8) 212 -> 177;
 // fp8 16384 over 32 1587 -> 1550, 13 over 64 (top-2) 34.3 -> 32.2, 509 over 128 the same; dense fp8, 3425 x 5600 x 2312
 // (strided scales) 104 -> 73, 2 x 3680 x 1336 19.4 -> 14.5, 158 x 640 x 1080 7.3 -> 6.6.
-// 16-bit rows in blocks of up to 64: a barrier per 128 K instead of 64, no scales in LDS, three workgroups per CU (blocks of 32: four; with strided
-// weights, which take twice the LDS, two and three) where the kernel with deeper rings beside the tile's scales held one or two: 816 x 4960 x 2776 f16 62.3 -> 35.8 us, 2351 x 1664 x 6992
-// 62 -> 55; 256 tokens over 16 experts, 3776 -> 1280, layer 74.9 -> 66.8.
+// 16-bit rows in blocks of up to 64: a barrier per 128 K instead of 64, no scales in LDS, three workgroups per CU (blocks of 32: four; with
+// strided weights, which take twice the LDS, two and three) where the kernel with deeper rings beside the tile's scales held one or two:
+// 816 x 4960 x 2776 f16 62.3 -> 35.8 us, 2351 x 1664 x 6992 62 -> 55; 256 tokens over 16 experts, 3776 -> 1280, layer 74.9 -> 66.8.
 #pragma once
 #include "moe_matmul_impl.h"
 

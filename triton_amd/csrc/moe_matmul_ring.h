@@ -1,5 +1,5 @@
-// Grouped (ragged) matmul of up to about 96 rows per slice x MXFP4 weights in 4 KB blocks with pre-shuffled scales, or both strided: a persistent kernel whose copies never stop at
-// the end of a tile.
+// Grouped (ragged) matmul of up to about 96 rows per slice x MXFP4 weights in 4 KB blocks with pre-shuffled scales, or both strided: a
+// persistent kernel whose copies never stop at the end of a tile.
 //
 // With few rows per slice HBM is the bound, and one tile per workgroup (moe_matmul_mx.h) reaches 5.3 TB/s of the 7 that copies alone read: a tile
 // starts with an empty pipeline and ends with an epilogue beside which it copies nothing, 8 of its 46 us, and three such workgroups per CU fill only
@@ -7,22 +7,23 @@
 //   * four waves copy and do nothing else, through a ring of three to six stages that runs on into the next tile; a stage is its tile's rows,
 //     weights and the block scales of both, so that no other wave waits for memory inside the K loop (an ordinary load there is served behind the
 //     CU's outstanding copies: row scales loaded by the multiplying waves took 3 000 cycles, with one piece of 256 K in advance every stage waited);
-//   * two sets of four waves (one per strip of 64 columns, all rows of the tile) take the tiles in turn: while one multiplies, the other finishes the tile before,
-//     one barrier of the stages for every four rows, and requests what its next tile's epilogue needs.  (Eight waves on every tile, epilogue
-//     at its end: 560 us where this takes 545, and 474 where this takes 440, see below.)
+//   * two sets of four waves (one per strip of 64 columns, all rows of the tile) take the tiles in turn: while one multiplies, the other
+//     finishes the tile before, one barrier of the stages for every four rows, and requests what its next tile's epilogue needs.  (Eight
+//     waves on every tile, epilogue at its end: 560 us where this takes 545, and 474 where this takes 440, see below.)
 //   * the weights of a slice with one row block are read once: non-temporal copies (632 -> 563 us on the first of the layers below);
 //   * tiles of fewer than four strips where that fills the one or two rounds over the workgroups.
 // Barriers of the whole workgroup, one per stage, publish a stage and free the one before.
 //
-// Strided weights (blocks of up to 64 rows): pieces of 64 bytes per column and 128 K, sixteen bytes of scales per column and 256 K.  They read 3 to 4.7 TB/s, by
-// whether a piece crosses a line, as in moe_matmul_mx.h; what is won is the narrower tiles of small calls and, for 16-bit rows, multiplying waves that do not
-// copy.  (Scales a dword at a time asked for twice as many lines as the weights, 5 to 15 % slower.)  Layers, tiled kernel -> now, us: 100 packed tokens x 4 of 16 slices, 2880
-// -> 1440, 62.3 -> 57.8; 60 fp8 x 4 of 16, 1760 -> 1440, 38.1 -> 33.6; 80 bf16 x 4 of 16, 2048 -> 1024, 43.5 -> 35.9; 512 bf16 x 4 of 60, 2880 -> 2880, 284 -> 266.
+// Strided weights (blocks of up to 64 rows): pieces of 64 bytes per column and 128 K, sixteen bytes of scales per column and 256 K.  They
+// read 3 to 4.7 TB/s, by whether a piece crosses a line, as in moe_matmul_mx.h; what is won is the narrower tiles of small calls and, for
+// 16-bit rows, multiplying waves that do not copy.  (Scales a dword at a time asked for twice as many lines as the weights, 5 to 15 %
+// slower.)  Layers, tiled kernel -> now, us: 100 packed tokens x 4 of 16 slices, 2880 -> 1440, 62.3 -> 57.8; 60 fp8 x 4 of 16, 1760 ->
+// 1440, 38.1 -> 33.6; 80 bf16 x 4 of 16, 2048 -> 1024, 43.5 -> 35.9; 512 bf16 x 4 of 60, 2880 -> 2880, 284 -> 266.
 //
-// Time of a layer (routing, both products, sum) before -> now: 509 fp8 tokens, 128 slices, 5760 -> 2880, 638 -> 548 us (the copies alone 499; the stores of the results
-// cost the rest: scattered lines between the reads, 45 us for 29 MB, 10 if they stay in the caches); 2880 -> 2880, 128 slices: 512 tokens fp8 346 -> 297, MXFP8
-// 355 -> 316, packed 365 -> 312, 1024 fp8 377 -> 339, packed 398 -> 353, 2048 packed 467 -> 436, fp8 446 -> 427.  (ring_rows in tile_rules.h says
-// which problems.)
+// Time of a layer (routing, both products, sum) before -> now: 509 fp8 tokens, 128 slices, 5760 -> 2880, 638 -> 548 us (the copies alone
+// 499; the stores of the results cost the rest: scattered lines between the reads, 45 us for 29 MB, 10 if they stay in the caches); 2880 ->
+// 2880, 128 slices: 512 tokens fp8 346 -> 297, MXFP8 355 -> 316, packed 365 -> 312, 1024 fp8 377 -> 339, packed 398 -> 353, 2048 packed 467
+// -> 436, fp8 446 -> 427.  (ring_rows in tile_rules.h says which problems.)
 #pragma once
 #include <algorithm>
 
@@ -33,8 +34,8 @@ namespace tamd {
 constexpr int kRingSlices = 256;   // slices that the table of the work holds
 constexpr int kRingProducers = 4;
 
-// Weights of up to four strips, columns' scales: eight blocks of 32 columns x 256 bytes (256 K, also where a stage is 128 K).  A deeper ring changes nothing: copies
-// alone reach their rate with two stages in flight, and 5 stages were 1 % faster than 7.
+// Weights of up to four strips, columns' scales: eight blocks of 32 columns x 256 bytes (256 K, also where a stage is 128 K).  A deeper
+// ring changes nothing: copies alone reach their rate with two stages in flight, and 5 stages were 1 % faster than 7.
 
 template <int XDT, int MF_, bool XMX = false>
 struct RingShape {

@@ -59,17 +59,17 @@ inline bool known_block(int block_m) { return block_m == 16 || block_m == 32 || 
 
 inline int64_t output_size(int dtype) { return dtype == TAMD_F32 ? 4 : (dtype == TAMD_FP8_E4M3 || dtype == TAMD_FP8_E5M2 ? 1 : 2); }
 
-// Products of 8- and 4-bit rows x MXFP4 weights, row blocks of up to 32, that K groups share (moe_matmul_mx.h): up to half as many tiles of 256 columns as CUs, four
-// stages of 256 K and more.  1500 products, dense: K 769 to 1024 0.95 of the tiled kernel's time, 1025 to 1280 (two stages for some groups) 1.0, to 2048 0.83, to
-// 4096 0.74, to 8192 0.58; three stages 1.05.
+// Products of 8- and 4-bit rows x MXFP4 weights, row blocks of up to 32, that K groups share (moe_matmul_mx.h): up to half as many tiles of
+// 256 columns as CUs, four stages of 256 K and more.  1500 products, dense: K 769 to 1024 0.95 of the tiled kernel's time, 1025 to 1280
+// (two stages for some groups) 1.0, to 2048 0.83, to 4096 0.74, to 8192 0.58; three stages 1.05.
 inline bool mx_groups(const tamd_matmul_args &a, int cus, int block_m) {
   if (a.K <= 768 || block_m > 32) return false;
   const double blocks = a.block_schedule ? live_slices(a) * ceil((double)a.M / a.n_experts / block_m) : (double)a.n_experts * ((a.M + block_m - 1) / block_m);
   return 2.0 * blocks * ((a.N + 255) / 256) <= cus;
 }
 
-// What the persistent kernel of few rows per slice (moe_matmul_ring.h) covers: ragged problems with weights in 4 KB blocks and pre-shuffled scales or both strided
-// along K, outputs of the usual type in pairs of columns that 32-bit offsets reach.
+// What the persistent kernel of few rows per slice (moe_matmul_ring.h) covers: ragged problems with weights in 4 KB blocks and pre-shuffled
+// scales or both strided along K, outputs of the usual type in pairs of columns that 32-bit offsets reach.
 inline bool ring_applicable(const tamd_matmul_args &a) {
   if (!a.block_schedule || a.force_variant) return false;
   if ((a.w_layout == TAMD_W_CDNA4_BLOCKS) != (a.w_mx_layout == TAMD_SCALE_CDNA4)) return false;
@@ -82,15 +82,18 @@ inline bool ring_applicable(const tamd_matmul_args &a) {
   if (!sw && (((a.N | (int)a.y_stride_m) & 1) != 0 || !aligned(a.y, 2 * (size_t)size))) return false;
   const bool flex = a.y_expected_scale || a.y_actual_scale;
   if (x16) return !a.y_mx_scale && !flex && a.y_dtype == a.x_dtype;
-  // (fp8 rows whose row blocks stream stay there: widened to bf16 their sums are 5e-9 off 64-bit ones, 4e-6 with the MFMA that takes them as they are)
+  // (fp8 rows whose row blocks stream stay there: widened to bf16 their sums are 5e-9 off 64-bit ones, 4e-6 with the MFMA that takes them
+  // as they are)
   if (a.x_dtype == TAMD_FP8_E4M3 && a.block_m == 16 && stream16_applicable(a)) return false;
   return a.y_dtype == TAMD_FP8_E4M3 || (a.y_dtype == TAMD_BF16 && !flex);
 }
 
-// Strided weights come in pieces of 64 bytes, at 3 to 4.7 TB/s in either kernel, and the copies no longer run ahead of anything over several rounds
-// (1.0 to 1.05 there): it is the faster where most CUs have no tile or one and narrower tiles share them out, and for the larger blocks of 16-bit
-// rows.  4000 products, time over the tiled kernel's, where it is taken: packed rows 0.83, MXFP8 0.89, fp8 0.89, 16-bit rows 0.93; one in ten above 1.04.
-// (16-bit rows in blocks of 64 with 0.85 to 1.0 tiles per CU, slices spread as a router's: K 800 to 1200 1.00, to 1800 0.94, to 2880 0.89; with 1.0 to 1.15 1.06, 1.00, 0.94.)
+// Strided weights come in pieces of 64 bytes, at 3 to 4.7 TB/s in either kernel, and the copies no longer run ahead of anything over
+// several rounds (1.0 to 1.05 there): it is the faster where most CUs have no tile or one and narrower tiles share them out, and for the
+// larger blocks of 16-bit rows.  4000 products, time over the tiled kernel's, where it is taken: packed rows 0.83, MXFP8 0.89, fp8 0.89,
+// 16-bit rows 0.93; one in ten above 1.04.
+// (16-bit rows in blocks of 64 with 0.85 to 1.0 tiles per CU, slices spread as a router's: K 800 to 1200 1.00, to 1800 0.94, to 2880 0.89;
+// with 1.0 to 1.15 1.06, 1.00, 0.94.)
 inline int ring_rows_strided(const tamd_matmul_args &a, double cover, double tiles) {
   if (a.x_dtype == TAMD_BF16 || a.x_dtype == TAMD_F16) {
     if (cover <= 16.0 || cover > 64.0) return 0;
@@ -105,7 +108,7 @@ inline int ring_rows_strided(const tamd_matmul_args &a, double cover, double til
 // A tile alone on its CU wins by copies that run ahead, which takes stages: with fewer, the start of a workgroup of twelve waves and its table
 // cost more than they give, against tiles (not against streaming, the blocks of 16, which is slower still there).  Rows of 8 and 4 bits
 // win again where one stage or two are all of K.  4700 products of K 32 to 1500, time over the tiled kernel's:
-//   16-bit rows         strided K to 512 1.08, to 640 1.04, to 768 1.00, to 1500 0.96; 4 KB blocks to 512 1.15, to 640 1.07, to 768 1.05, to 1500 0.98
+//   16-bit rows         strided K to 512 1.08, to 640 1.04, to 768 1.00, to 1500 0.96; in 4 KB blocks 1.15, 1.07, 1.05, 0.98
 //   MXFP8               strided K to 256 0.87, to 768 1.08; 4 KB blocks to 256 0.95, to 768 1.04
 //   fp8 and packed rows strided K to 256 0.89, to 512 1.04 (64 rows 1.09), to 768 1.01; 4 KB blocks to 512 0.99 (64 rows 1.06)
 inline bool ring_stages_too_few(const tamd_matmul_args &a, double cover) {
@@ -115,14 +118,16 @@ inline bool ring_stages_too_few(const tamd_matmul_args &a, double cover) {
   return a.K > 256 && a.K <= (scaled ? 768 : 512) && (scaled || a.w_layout != TAMD_W_CDNA4_BLOCKS || cover > 32.0);
 }
 
-// Rows of the persistent kernel's blocks, 0 where another kernel is the faster (or the only one).  The block is the smallest that covers a slice's mean size and
-// two standard deviations, up to 96; the lines between the kernels are in tiles per CU, one row block for every slice that has rows (on the
-// average of random choices).  Up to one, a tile is alone on its CU and wins by its depth; just above, the second round is nearly empty, where smaller tiles, three
-// and four to a CU, lose less; from two on the rounds fill.  Below K 1024 the loop over K is too short to hide the tile before, unless there is none.
+// Rows of the persistent kernel's blocks, 0 where another kernel is the faster (or the only one).  The block is the smallest that covers a
+// slice's mean size and two standard deviations, up to 96; the lines between the kernels are in tiles per CU, one row block for every slice
+// that has rows (on the average of random choices).  Up to one, a tile is alone on its CU and wins by its depth; just above, the second
+// round is nearly empty, where smaller tiles, three and four to a CU, lose less; from two on the rounds fill.  Below K 1024 the loop over K
+// is too short to hide the tile before, unless there is none.
 // 16-bit rows of up to 16 per slice are the streaming kernel's, except where its parts of K (multiples of 1024) fit badly; their larger
 // blocks are bound by the conversion of the codes, as in the other kernels.
-// From 38 000 products (layers of 1 to 16384 tokens, 8 to 128 slices, K and N 512 to 5760, random choices), time with this rule where it chooses this kernel
-// over the time without: 16-bit rows 0.905, fp8 0.907, MXFP8 0.95, packed 0.914; more than 10 % slower in 1 to 2 % of them.
+// From 38 000 products (layers of 1 to 16384 tokens, 8 to 128 slices, K and N 512 to 5760, random choices), time with this rule where it
+// chooses this kernel over the time without: 16-bit rows 0.905, fp8 0.907, MXFP8 0.95, packed 0.914; more than 10 % slower in 1 to 2 % of
+// them.
 inline int ring_rows(const tamd_matmul_args &a, int cus) {
   if (!ring_applicable(a)) return 0;
   const bool x16 = a.x_dtype == TAMD_BF16 || a.x_dtype == TAMD_F16;
@@ -163,8 +168,9 @@ inline int ring_rows(const tamd_matmul_args &a, int cus) {
   return tiles > (packed ? 1.4 : 2.0) ? 96 : 0;
 }
 
-// What the persistent kernel for unquantised 16-bit weights (moe_matmul_kkring.h) covers, of the products that the tiled kernel of two operands along K
-// takes: ragged problems of four stages of K and more, outputs of the rows' type in pairs of columns that 32-bit offsets reach.
+// What the persistent kernel for unquantised 16-bit weights (moe_matmul_kkring.h) covers, of the products that the tiled kernel of two
+// operands along K takes: ragged problems of four stages of K and more, outputs of the rows' type in pairs of columns that 32-bit offsets
+// reach.
 inline bool kk_ring_applicable(const tamd_matmul_args &a) {
   if (!a.block_schedule || a.force_variant || a.K < 256 || a.n_experts > 256) return false;
   if ((a.x_dtype != TAMD_BF16 && a.x_dtype != TAMD_F16) || a.w_dtype != a.x_dtype || a.y_dtype != a.x_dtype) return false;
@@ -174,13 +180,14 @@ inline bool kk_ring_applicable(const tamd_matmul_args &a) {
   return a.activation == TAMD_ACT_SWIGLU || (((a.N | (int)a.y_stride_m) & 1) == 0 && aligned(a.y, 4));
 }
 
-// Rows of its blocks, 0 where the tiled kernels are the faster: with fewer than a third as many tiles of 256 columns as CUs one workgroup's stages are all
-// latency (four rows for 8 slices, 1760 x 3904: 13.4 us, 16 with this one).  486 products of 1 to 16384 tokens, 8 to 128 slices, K and N 512 to 5760: 0.876 of the
-// time in the mean (0.866 with the best choice for each), none above 1.05; with the line at 0.25 0.874, three above 1.1; at 0.5 0.888.  Blocks of 64 up to 56 rows per slice
-// lose up to 1.21, where slices come in two.
+// Rows of its blocks, 0 where the tiled kernels are the faster: with fewer than a third as many tiles of 256 columns as CUs one workgroup's
+// stages are all latency (four rows for 8 slices, 1760 x 3904: 13.4 us, 16 with this one).  486 products of 1 to 16384 tokens, 8 to 128
+// slices, K and N 512 to 5760: 0.876 of the time in the mean (0.866 with the best choice for each), none above 1.05; with the line at 0.25
+// 0.874, three above 1.1; at 0.5 0.888.  Blocks of 64 up to 56 rows per slice lose up to 1.21, where slices come in two.
 inline int kk_ring_rows(const tamd_matmul_args &a, int cus) {
   if (!kk_ring_applicable(a)) return 0;
-  if (a.M <= a.n_experts && 3 * (int64_t)most_live_slices(a) * ((a.N + 255) / 256) < cus) return 0;   // (the line below, whichever slices the rows fall on)
+  // (the line below, whichever slices the rows fall on)
+  if (a.M <= a.n_experts && 3 * (int64_t)most_live_slices(a) * ((a.N + 255) / 256) < cus) return 0;
   const double mean = (double)a.M / a.n_experts, tiles = live_slices(a) * ((a.N + 255) / 256) / cus;
   if (3.0 * tiles * (mean > 160.0 ? mean / 160.0 : 1.0) < 1.0) return 0;
   return mean <= 48.0 ? 64 : 160;
@@ -189,8 +196,8 @@ inline int kk_ring_rows(const tamd_matmul_args &a, int cus) {
 // Row block size of a dense / batched problem: the block whose tiles take the fewest rounds over the CUs, weighted with what a
 // tile of it takes, of one of 128 rows: `weight` (in percent) for 64 and 32 rows, `slots` tiles at the speed of one round.
 // Fitted to products timed with every block (mean and worst time against the best block of each):
-//   16-bit rows x MXFP4, 130 of 64 to 16384 rows: one and a half tiles per CU, 0.45 and 0.35; from K 3072 down, where a block of 128 has its scales in
-//     LDS, one per CU, 0.58 and 0.4 for strided weights and from four rounds on.  1.009, 1.14; with the first figures for all 1.019,
+//   16-bit rows x MXFP4, 130 of 64 to 16384 rows: one and a half tiles per CU, 0.45 and 0.35; from K 3072 down, where a block of 128 has
+//     its scales in LDS, one per CU, 0.58 and 0.4 for strided weights and from four rounds on.  1.009, 1.14; with the first figures for all 1.019,
 //     1.23 (14716 x 2080 x 8144 481 us in blocks of 64, 413 of 128; block layout, 16384 x 2880 x 2880 232 and 217, 3337 x 608 x 4768 24 and
 //     31), with the largest block that gives every CU a tile 1.041, 1.47;
 //   fp8 x MXFP4, the same: one and three quarters, 0.68 and 0.4.  1.009, 1.18 (the figures of 16-bit rows 1.039, 1.24: 8192 x 2880 x
