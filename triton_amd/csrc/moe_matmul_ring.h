@@ -9,21 +9,25 @@
 //     CU's outstanding copies: row scales loaded by the multiplying waves took 3 000 cycles, with one piece of 256 K in advance every stage waited);
 //   * two sets of four waves (one per strip of 64 columns, all rows of the tile) take the tiles in turn: while one multiplies, the other
 //     finishes the tile before, one barrier of the stages for every four rows, and requests what its next tile's epilogue needs.  (Eight
-//     waves on every tile, epilogue at its end: 560 us where this takes 545, and 474 where this takes 440, see below.)
-//   * the weights of a slice with one row block are read once: non-temporal copies (632 -> 563 us on the first of the layers below);
+//     waves on every tile, epilogue at its end: 3 and 8 % slower on the 509 fp8 and the 2048 packed tokens below.)
+//   * the weights of a slice with one row block are read once: non-temporal copies (0.89 of the time on the first of the layers below);
 //   * tiles of fewer than four strips where that fills the one or two rounds over the workgroups.
 // Barriers of the whole workgroup, one per stage, publish a stage and free the one before.
 //
 // Strided weights (blocks of up to 64 rows): pieces of 64 bytes per column and 128 K, sixteen bytes of scales per column and 256 K.  They
 // read 3 to 4.7 TB/s, by whether a piece crosses a line, as in moe_matmul_mx.h; what is won is the narrower tiles of small calls and, for
 // 16-bit rows, multiplying waves that do not copy.  (Scales a dword at a time asked for twice as many lines as the weights, 5 to 15 %
-// slower.)  Layers, tiled kernel -> now, us: 100 packed tokens x 4 of 16 slices, 2880 -> 1440, 62.3 -> 57.8; 60 fp8 x 4 of 16, 1760 ->
-// 1440, 38.1 -> 33.6; 80 bf16 x 4 of 16, 2048 -> 1024, 43.5 -> 35.9; 512 bf16 x 4 of 60, 2880 -> 2880, 284 -> 266.
+// slower.)  Layers, tiled kernel -> now, us: 100 packed tokens x 4 of 16 slices, 2880 -> 1440, 52.8 -> 48.1; 60 fp8 x 4 of 16, 1760 ->
+// 1440, 38.1 -> 34.6; 80 bf16 x 4 of 16, 2048 -> 1024, 44.1 -> 37.4; 512 bf16 x 4 of 60, 2880 -> 2880, 284 -> 271.
 //
-// Time of a layer (routing, both products, sum) before -> now: 509 fp8 tokens, 128 slices, 5760 -> 2880, 638 -> 548 us (the copies alone
-// 499; the stores of the results cost the rest: scattered lines between the reads, 45 us for 29 MB, 10 if they stay in the caches); 2880 ->
-// 2880, 128 slices: 512 tokens fp8 346 -> 297, MXFP8 355 -> 316, packed 365 -> 312, 1024 fp8 377 -> 339, packed 398 -> 353, 2048 packed 467
-// -> 436, fp8 446 -> 427.  (ring_rows in tile_rules.h says which problems.)
+// Time of a layer (routing, both products, sum), tiled kernels -> now, us: 509 fp8 tokens x 4 of 128 slices, 5760 -> 2880, 643 -> 583;
+// 2880 -> 2880, 128 slices: 512 tokens fp8 353 -> 325, MXFP8 363 -> 346, packed 372 -> 343, 1024 fp8 388 -> 374, packed 409 -> 381, 2048
+// packed 471 -> 437, fp8 453 -> 434.  (ring_rows in tile_rules.h says which problems.)
+//
+// What is left of the 509, the 2048 packed and the 2048 fp8 tokens' time without one part of the work: without the products 1.00, 0.99,
+// 0.99; without the copies of the rows 0.98, 0.95, 0.89; without the stores 0.92, 0.87, 0.88.  The copies are the bound, and what the
+// stores take from them: scattered lines between the reads.  Weights are read once (2.27 GB fetched for 2.26 of weights, 1.26 for 1.13),
+// matrix cores are busy 16 to 12 % of the cycles.
 #pragma once
 #include <algorithm>
 
@@ -106,7 +110,7 @@ TAMD_DEVICE void ring_work(const Args &a, int group, int32_t *tab, RingWork &w) 
   const uint32_t blocks = (uint32_t)__builtin_amdgcn_readfirstlane(tab[3 * kRingSlices]), wgs = gridDim.x;
   w.strips = (uint32_t)(a.N + 63) / 64;
   w.gn = (w.strips + 3) / 4;
-  if (blocks > 0) {   // narrower tiles where they fill one or two rounds (later on they only repeat the rows' copies: 545 -> 551 us)
+  if (blocks > 0) {   // narrower tiles where they fill one or two rounds (later on they only repeat the rows' copies: 1 % slower)
     const uint32_t rounds = (blocks * w.gn + wgs - 1) / wgs, fill = rounds * wgs / blocks;
     if (rounds <= 2) w.gn = fill < w.strips ? fill : w.strips;
   }
