@@ -59,7 +59,7 @@ def blocks(w, ws):
 # (rows per slice, slices, K, columns): blocks of 32 alone on their CUs (K of one stage and less, of fewer stages than the ring, off the
 # stages), in several rounds; of 64; of 96
 SIZES = [(9, 10, 96, 2832), (4, 12, 352, 1872), (14, 16, 736, 1296), (20, 16, 1440, 1392), (5, 128, 1056, 1184), (11, 64, 2144, 2320),
-         (40, 16, 608, 2608), (30, 60, 1248, 2320), (72, 32, 1056, 4368)]
+         (40, 16, 608, 2608), (30, 60, 1248, 2320), (72, 32, 1056, 4368), (14, 16, 800, 1296), (4, 12, 992, 1872)]
 
 
 @pytest.mark.parametrize("layout", [dict(), dict(w_layout=_lib.W_STRIDED, w_mx_layout=_lib.SCALE_STRIDED, w_stride_k=1, w_stride_n=1440, w_mx_stride_k=1,
