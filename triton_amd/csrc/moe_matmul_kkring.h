@@ -7,11 +7,15 @@
 // of the cycles.  Here a workgroup owns a CU and walks over tiles:
 //   * four waves copy and do nothing else, through a ring of three stages (64 K of a tile's rows and columns, 128-byte lines of both) that
 //     runs on into the next tile; they find the tiles and leave them for the others in LDS;
-//   * eight waves multiply, two halves of the row fragments times four strips of 64 columns, and finish the tile from registers; the two or three
+//   * eight waves multiply, two halves of the row fragments times four strips of 64 columns, and finish the tile from registers; the two
 //     stages ahead cover the copies for most of that time;
-//   * weights of slices with one row block are copied non-temporally where their columns are whole lines and the call reads more than the caches keep
-//     (300 tokens x 4 of 32 slices, 2880 -> 2 x 2880: 188 -> 170 us; of columns off the lines 137 -> 150 and 28 -> 34, so not there);
-//   * tiles of fewer strips where that fills the rounds over the workgroups (1021 tokens x 4 of 32: 228 -> 216); blocks of one slice are of one size.
+//   * weights of slices with one row block are copied non-temporally where their columns are whole lines and the call reads more than the
+//     caches keep (300 tokens x 4 of 32 slices, 2880 -> 2 x 2880: 188 -> 170 us; of columns off the lines 137 -> 150 and 28 -> 34, so not there);
+//   * tiles of fewer strips where that fills the rounds over the workgroups (1021 tokens x 4 of 32: 228 -> 216); blocks of one slice are of one
+//     size.
+// A sum is one float32 accumulator for all of K, the tiled kernel's two (of either half of every stage): a wave of blocks of 160 rows has
+// the registers for one.  Results of K 2880 against 64-bit sums (2-norm): bf16 1.662372e-3 from both, which is what rounding the exact sums gives;
+// f16 2.077690e-4, 2.077689e-4 from the tiled kernel, 2.077687e-4 from rounding alone.
 // Blocks of 160 rows, the most that three stages have LDS for (128: 1021 tokens 225, 2000 tokens 357 where 160 take 311; 96: 266 and 393);
 // of 64 where slices are smaller, whose copies of rows that are not there cost 2 to 4 % (300 tokens: 170 -> 165; blocks of 32 with a ring
 // of four: 208).

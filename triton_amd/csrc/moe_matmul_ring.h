@@ -1,12 +1,13 @@
 // Grouped (ragged) matmul of up to about 96 rows per slice x MXFP4 weights in 4 KB blocks with pre-shuffled scales, or both strided: a
 // persistent kernel whose copies never stop at the end of a tile.
 //
-// With few rows per slice HBM is the bound, and one tile per workgroup (moe_matmul_mx.h) reaches 5.3 TB/s of the 7 that copies alone read: a tile
-// starts with an empty pipeline and ends with an epilogue beside which it copies nothing, 8 of its 46 us, and three such workgroups per CU fill only
-// part of one another's gaps.  Here one workgroup owns a CU and walks over its tiles:
+// With few rows per slice HBM is the bound, and one tile per workgroup (moe_matmul_mx.h) reaches 5.3 TB/s of the 7 that copies alone read:
+// a tile starts with an empty pipeline and ends with an epilogue beside which it copies nothing, 8 of its 46 us, and three such workgroups
+// per CU fill only part of one another's gaps.  Here one workgroup owns a CU and walks over its tiles:
 //   * four waves copy and do nothing else, through a ring of three to six stages that runs on into the next tile; a stage is its tile's rows,
-//     weights and the block scales of both, so that no other wave waits for memory inside the K loop (an ordinary load there is served behind the
-//     CU's outstanding copies: row scales loaded by the multiplying waves took 3 000 cycles, with one piece of 256 K in advance every stage waited);
+//     weights and the block scales of both, so that no other wave waits for memory inside the K loop (an ordinary load there is served
+//     behind the CU's outstanding copies: row scales loaded by the multiplying waves took 3 000 cycles, with one piece of 256 K in advance
+//     every stage waited);
 //   * two sets of four waves (one per strip of 64 columns, all rows of the tile) take the tiles in turn: while one multiplies, the other
 //     finishes the tile before, one barrier of the stages for every four rows, and requests what its next tile's epilogue needs.  (Eight
 //     waves on every tile, epilogue at its end: 3 and 8 % slower on the 509 fp8 and the 2048 packed tokens below.)
@@ -158,10 +159,10 @@ TAMD_DEVICE void ring_tile(const RingWork &w, int i, Tile &t, int &strips, bool 
   t.rows = left > BM ? BM : left;
 }
 
-// Copying waves: strip w's weights, rows 8 w .. of every row fragment, the column scales (waves 0 and 1, four blocks of 32 columns each) or the row
-// scales (waves 2 and, past 64 rows, 3).  Stage s goes to slot s % RING and is requested RING - 1 stages ahead; copies complete in the order of their
-// requests, so a stage has landed once only those of the stages after it are outstanding (the indices of the next tile's rows, requested
-// in front of a tile's first stage, only make that wait a little longer).
+// Copying waves: strip w's weights, rows 8 w .. of every row fragment, the column scales (waves 0 and 1, four blocks of 32 columns each) or
+// the row scales (waves 2 and, past 64 rows, 3).  Stage s goes to slot s % RING and is requested RING - 1 stages ahead; copies complete in
+// the order of their requests, so a stage has landed once only those of the stages after it are outstanding (the indices of the next tile's
+// rows, requested in front of a tile's first stage, only make that wait a little longer).
 template <int XDT, int MF, bool XMX, typename Args>
 TAMD_DEVICE void ring_copy(const Args &a, const RingWork &work, uint8_t *lds) {
   typedef RingShape<XDT, MF, XMX> S;
@@ -198,7 +199,8 @@ TAMD_DEVICE void ring_copy(const Args &a, const RingWork &work, uint8_t *lds) {
   // the row scales as aligned dwords, up to the one that holds the last row's last byte
   const uint32_t xs_mis = XMX ? (uint32_t)(uintptr_t)a.x_mx_scale & 3u : 0u;
   const v4i_t rxs = make_rsrc(a.x_mx_scale - xs_mis,
-                              (uint32_t)__builtin_amdgcn_readfirstlane((int)((xs_mis + (uint32_t)(((a.x_rows > 0 ? a.x_rows : (int64_t)a.M) - 1) * a.x_mx_stride_m + K / 32) + 3u) & ~3u)));
+                              (uint32_t)__builtin_amdgcn_readfirstlane(
+                                  (int)((xs_mis + (uint32_t)(((a.x_rows > 0 ? a.x_rows : (int64_t)a.M) - 1) * a.x_mx_stride_m + K / 32) + 3u) & ~3u)));
   auto issue = [&](int slot) {
     const bool fresh = p == 0;
     if (fresh) {
