@@ -16,140 +16,251 @@ static __device__ __align__(256) int32_t scratch[kStaticWorkspaceInts];
 // ---------------------------------------------------------------------------
 // top-k
 // ---------------------------------------------------------------------------
-// Sort key of a logit: order-preserving map of the float32 bits in the high
-// part, (0xFFFF - column) in the low 16 bits so that the lower column wins ties
-// (topk_details/_topk_forward.py:15-30).  -0.0 is keyed as +0.0 so that both
-// zeros tie, as they do under the reference's stable argsort of -x.
-TAMD_DEVICE uint64_t logit_key(float x, int col) {
-  uint32_t u = f32_to_bits(x);
-  if (u == 0x80000000u) u = 0u;
-  u ^= (u >> 31) ? 0xFFFFFFFFu : 0x80000000u;
-  return ((uint64_t)u << 16) | (uint64_t)(0xFFFFu - (uint32_t)col);
+// Order-preserving map of a logit's bits.  -0.0 counts as +0.0, so that both zeros tie, as they do under the reference's
+// stable argsort of -x (topk_details/_topk_forward.py:15-30; the sum with +0.0 takes the sign).
+TAMD_DEVICE uint32_t ordered_bits(float x) {
+  const uint32_t u = f32_to_bits(x + 0.0f);
+  return u ^ ((uint32_t)((int32_t)u >> 31) | 0x80000000u);
 }
+// Its inverse (a -0.0 logit comes back as +0.0).
+TAMD_DEVICE float logit_of(uint32_t u) { return bits_to_f32(u ^ (~(uint32_t)((int32_t)u >> 31) | 0x80000000u)); }
 
-// Inverse of the value part of logit_key (a -0.0 logit comes back as +0.0).
-TAMD_DEVICE float logit_of_key(uint64_t key) {
-  uint32_t u = (uint32_t)(key >> 16);
-  u ^= (u >> 31) ? 0x80000000u : 0xFFFFFFFFu;
-  return bits_to_f32(u);
-}
+// Sort key of a logit and its column, all different: the higher logit first, the lower column among equals
+// (_topk_forward.py:15-30).  A 16-bit logit and its column are one 32-bit integer, a float32 and its column two.  (As one double
+// between 1 and 2 the latter would need one instruction to find the larger of two keys, but v_max_f64 takes a quarter of the lanes
+// at a time; a 64-bit integer comparison likewise.)
+template <int DT>
+struct SortKey {
+  uint32_t v;  // logit in the high half, 0xFFFF - column in the low half
+  TAMD_DEVICE static SortKey of(float x, int col) {
+    const uint32_t u = (DT == TAMD_F16 ? f32_to_f16_bits(x + 0.0f) : f32_to_bf16_bits(x + 0.0f)) << 16;  // exact: x was loaded from such bits
+    return {((u ^ ((uint32_t)((int32_t)u >> 31) | 0x80000000u)) & 0xFFFF0000u) | (0xFFFFu - (uint32_t)col)};
+  }
+  TAMD_DEVICE static SortKey none(int col) { return {0xFFFFu - (uint32_t)col}; }
+  TAMD_DEVICE uint32_t column_field() const { return v & 0xFFFFu; }
+  TAMD_DEVICE bool same(SortKey o) const { return v == o.v; }
+  TAMD_DEVICE float logit() const {
+    const uint32_t u = f32_to_bits(logit_of(v & 0xFFFF0000u)) >> 16;
+    return DT == TAMD_F16 ? f16_bits_to_f32(u) : bf16_bits_to_f32(u);
+  }
+  TAMD_DEVICE static void order(SortKey &a, SortKey &b) {
+    const uint32_t x = a.v, y = b.v;
+    a.v = x > y ? x : y;
+    b.v = x > y ? y : x;
+  }
+  TAMD_DEVICE static SortKey pick(bool first, SortKey a, SortKey b) { return {first ? a.v : b.v}; }
+  template <int L>
+  TAMD_DEVICE static SortKey group_largest(SortKey q);
+};
+template <>
+struct SortKey<TAMD_F32> {
+  uint32_t u, c;  // logit, 0xFFFF - column
+  TAMD_DEVICE static SortKey of(float x, int col) { return {ordered_bits(x), 0xFFFFu - (uint32_t)col}; }
+  TAMD_DEVICE static SortKey none(int col) { return {0u, 0xFFFFu - (uint32_t)col}; }
+  TAMD_DEVICE uint32_t column_field() const { return c; }
+  TAMD_DEVICE bool same(SortKey o) const { return c == o.c; }
+  TAMD_DEVICE float logit() const { return logit_of(u); }
+  TAMD_DEVICE static void order(SortKey &a, SortKey &b) {
+    const SortKey x = a, y = b;
+    const bool less = x.u < y.u;  // (equal ones stay as they are: the lower column is in front)
+    a = {x.u > y.u ? x.u : y.u, less ? y.c : x.c};
+    b = {x.u > y.u ? y.u : x.u, less ? x.c : y.c};
+  }
+  TAMD_DEVICE static SortKey pick(bool first, SortKey a, SortKey b) { return {first ? a.u : b.u, first ? a.c : b.c}; }
+  template <int L>
+  TAMD_DEVICE static SortKey group_largest(SortKey q);
+};
 
-// Step O (1, 2, 4, ...) of a butterfly reduction over groups of lanes: the value of a lane of the other aligned block
-// of O lanes.  All lanes of a block of O hold the same value by then, so for O = 4 and 8 the partner may be the
-// mirrored lane, which, like the swaps inside a quad, the data-parallel move does in the register file; from 16 up it
-// is the lane at XOR distance O, through the LDS crossbar.
+// Reductions over aligned groups of L lanes; every lane gets the result.  Step O (1, 2, 4, ...) of the butterfly combines a lane with
+// one of the other aligned block of O lanes.  All lanes of a block of O hold the same value by then, so for O = 4 and 8 the
+// partner may be the mirrored lane, which, like the swaps inside a quad, the data-parallel move does in the register
+// file; for 16 and 32 rows of lanes change places, and the two registers that hold the halves then are combined.
 template <int O>
-TAMD_DEVICE uint32_t butterfly_partner(uint32_t v) {
-  if constexpr (O == 1) return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, true);        // quad_perm [1,0,3,2]
-  else if constexpr (O == 2) return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xF, 0xF, true);   // quad_perm [2,3,0,1]
-  else if constexpr (O == 4) return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xF, 0xF, true);  // row_half_mirror
-  else if constexpr (O == 8) return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xF, 0xF, true);  // row_mirror
-  else return (uint32_t)__shfl_xor((int)v, O);
+TAMD_DEVICE void butterfly(uint32_t v, uint32_t &a, uint32_t &b) {
+  a = v;
+  if constexpr (O == 1) b = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, true);        // quad_perm [1,0,3,2]
+  else if constexpr (O == 2) b = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xF, 0xF, true);   // quad_perm [2,3,0,1]
+  else if constexpr (O == 4) b = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xF, 0xF, true);  // row_half_mirror
+  else if constexpr (O == 8) b = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xF, 0xF, true);  // row_mirror
+  else if constexpr (O == 16) { const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false); a = r[0]; b = r[1]; }
+  else { const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false); a = r[0]; b = r[1]; }
 }
-
-template <int L, int O = 1>
-TAMD_DEVICE uint64_t group_max_u64(uint64_t v) {
-  if constexpr (O < L) {
-    const uint32_t lo = butterfly_partner<O>((uint32_t)v);
-    const uint32_t hi = butterfly_partner<O>((uint32_t)(v >> 32));
-    const uint64_t w = ((uint64_t)hi << 32) | lo;
-    return group_max_u64<L, O * 2>(w > v ? w : v);
-  } else {
+template <int L, int O = 1, typename OP>
+TAMD_DEVICE uint32_t group_reduce(uint32_t v, OP op) {
+  if constexpr (O >= L) {
     return v;
+  } else {
+    uint32_t a, b;
+    butterfly<O>(v, a, b);
+    return group_reduce<L, O * 2>(op(a, b), op);
   }
 }
-
-template <int L, int O = 1>
+template <int L>
+TAMD_DEVICE uint32_t group_max_u32(uint32_t v) {
+  return group_reduce<L>(v, [](uint32_t a, uint32_t b) { return a > b ? a : b; });
+}
+template <int L>
+TAMD_DEVICE uint32_t group_min_u32(uint32_t v) {
+  return group_reduce<L>(v, [](uint32_t a, uint32_t b) { return a < b ? a : b; });
+}
+template <int DT>
+template <int L>
+TAMD_DEVICE SortKey<DT> SortKey<DT>::group_largest(SortKey q) { return {group_max_u32<L>(q.v)}; }
+template <int L>
+TAMD_DEVICE SortKey<TAMD_F32> SortKey<TAMD_F32>::group_largest(SortKey q) {
+  const uint32_t m = group_max_u32<L>(q.u);
+  return {m, group_max_u32<L>(q.u == m ? q.c : 0u)};
+}
+template <int L>
 TAMD_DEVICE float group_sum_f32(float v) {
-  if constexpr (O < L) return group_sum_f32<L, O * 2>(v + bits_to_f32(butterfly_partner<O>(f32_to_bits(v))));
-  else return v;
+  return bits_to_f32(group_reduce<L>(f32_to_bits(v), [](uint32_t a, uint32_t b) { return f32_to_bits(bits_to_f32(a) + bits_to_f32(b)); }));
+}
+template <int L>
+TAMD_DEVICE float group_max_f32(float v) {
+  return bits_to_f32(group_reduce<L>(f32_to_bits(v), [](uint32_t a, uint32_t b) { return f32_to_bits(__builtin_fmaxf(bits_to_f32(a), bits_to_f32(b))); }));
 }
 
-template <int L, int O = 1>
-TAMD_DEVICE float group_max_f32(float v) {
-  if constexpr (O < L) return group_max_f32<L, O * 2>(__builtin_fmaxf(v, bits_to_f32(butterfly_partner<O>(f32_to_bits(v)))));
-  else return v;
+// The logits of a row, EPL of its L lanes' columns `sub + j * L` each, requested together: every lane loads (columns past the
+// end re-read the last one), and `take` pins the values before they are selected: a load that the compiler may move under
+// the per-lane condition is awaited before the next one is issued, EPL round trips to memory instead of one.
+template <int DT, int L, int EPL>
+struct RowLogits {
+  float x[EPL];
+  TAMD_DEVICE void request(const void *p, int64_t off, int n_cols, int sub) {
+#pragma unroll
+    for (int j = 0; j < EPL; ++j) {
+      const int c = sub + j * L;
+      x[j] = load_as_f32<DT>(p, off + (c < n_cols ? c : n_cols - 1));
+    }
+  }
+  TAMD_DEVICE void take(SortKey<DT> *keys, int n_cols, int sub) {
+#pragma unroll
+    for (int j = 0; j < EPL; ++j) asm volatile("" : "+v"(x[j]));
+#pragma unroll
+    for (int j = 0; j < EPL; ++j)
+      keys[j] = SortKey<DT>::pick(sub + j * L < n_cols, SortKey<DT>::of(x[j], sub + j * L), SortKey<DT>::none(sub + j * L));
+  }
+};
+
+// What a lane of a row's group knows of the k picked columns: the column and the key of the pick that its own place in the
+// group stands for, the largest key, and the picked columns among 32 * sub .. 32 * sub + 31 as bits.
+template <int DT>
+struct Picks {
+  SortKey<DT> key, top;
+  uint32_t word;
+  TAMD_DEVICE int col() const { return (int)(0xFFFFu - key.column_field()); }
+};
+
+// Every lane sorts its own keys; then k rounds of: the largest of the lanes' first keys, taken out of its lane's list.  What it costs is
+// the number of instructions, about six cycles each to a wave that has its SIMD to itself: one row of 128 float32
+// logits and four picks 2200 cycles, 3200 when every round compared all keys as 64-bit integers.  (Two 32-bit searches of all
+// keys per round 2100 and, with eight picks of 16-bit logits, 64 rows of 256 9.2 us instead of 8.4; as doubles 2100.)
+template <int L, int EPL, int DT>
+TAMD_DEVICE Picks<DT> pick_columns(SortKey<DT> *q, int k, int sub) {
+  // neighbours in turn: equal logits never pass each other, so one comparison of 32 bits decides (28 exchanges for 8 keys, where
+  // the 19 of a shorter network would have to compare the columns too)
+#pragma unroll
+  for (int round = 0; round < EPL; ++round)
+#pragma unroll
+    for (int j = round & 1; j + 1 < EPL; j += 2) SortKey<DT>::order(q[j], q[j + 1]);
+  Picks<DT> r{q[0], q[0], 0u};
+#pragma clang loop unroll(disable)
+  for (int pass = 0; pass < k; ++pass) {
+    const SortKey<DT> m = SortKey<DT>::template group_largest<L>(q[0]);
+    const bool mine = q[0].same(m);
+#pragma unroll
+    for (int j = 0; j < 3; ++j) q[j] = SortKey<DT>::pick(mine, q[j + 1], q[j]);
+    if (EPL > 4 && k > 4) {  // (of four picks no lane gives more than its first four)
+#pragma unroll
+      for (int j = 3; j < EPL - 1; ++j) q[j] = SortKey<DT>::pick(mine, q[j + 1], q[j]);
+    }
+    if (mine && (EPL == 4 || k > 4)) q[EPL - 1] = SortKey<DT>::none(0xFFFF);  // the list's end
+    r.top = SortKey<DT>::pick(pass == 0, m, r.top);
+    r.key = SortKey<DT>::pick(sub == pass, m, r.key);
+    const uint32_t f = m.column_field();
+    r.word |= f >> 5 == 0x7FFu - (uint32_t)sub ? 0x80000000u >> (f & 31u) : 0u;
+  }
+  return r;
+}
+
+// The softmax over the picked logits, of this lane's slot (lanes past the last slot: 0).
+template <int L, int DT>
+TAMD_DEVICE float pick_softmax(const Picks<DT> &r, bool slot) {
+  const float e = slot ? expf(r.key.logit() - r.top.logit()) : 0.f;
+  return e / group_sum_f32<L>(e);
+}
+
+// Bits of a gate weight as stored.
+template <int DT>
+TAMD_DEVICE uint32_t stored_bits(float v) {
+  return DT == TAMD_F32 ? f32_to_bits(v) : DT == TAMD_BF16 ? f32_to_bf16_bits(v) : f32_to_f16_bits(v);
 }
 
 // L lanes cooperate on one row; EPL > 0 keeps ceil(n_cols/L) <= EPL keys in registers.  `row` is the row of this
-// thread's group of L lanes (any row >= n_rows: a group that only takes part in the shuffles); lds_indx, when given,
-// also receives the picked columns ([row][k] ints) for a kernel that goes on to use them, and lds_gate the bits of the
-// stored values.
+// thread's group of L lanes (any row >= n_rows: a group that only takes part in the shuffles).
 template <int DT, int L, int EPL>
 TAMD_DEVICE void topk_row(const void *__restrict__ x, int64_t x_stride, int n_rows, int n_cols, int k,
                           int apply_softmax, int use_provided, void *__restrict__ y_vals,
                           int16_t *__restrict__ y_indx, int64_t y_stride, uint32_t *__restrict__ bits,
-                          int64_t bits_stride_row, int64_t bits_stride_word, int64_t row, int32_t *lds_indx,
-                          uint32_t *lds_gate = nullptr) {
+                          int64_t bits_stride_row, int64_t bits_stride_word, int64_t row) {
   const int sub = threadIdx.x % L;
   const bool live = row < n_rows;
   const int64_t rrow = live ? row : 0;
   const int64_t xoff = rrow * x_stride;
   int my_idx = 0;
-  uint64_t mine = 0ull;  // key of the column this lane's slot picked
-  if (use_provided) {
-    if (sub < k) my_idx = y_indx[rrow * y_stride + sub];
-  } else {
-    uint64_t keys[EPL > 0 ? EPL : 1];
-    if constexpr (EPL > 0) {
-      // every lane loads (columns past the end re-read the last one) and the values are pinned before they are
-      // selected: a load that the compiler may move under the per-lane condition is awaited before the next one is
-      // issued, eight round trips to memory instead of one
-      float xv[EPL];
-#pragma unroll
-      for (int j = 0; j < EPL; ++j) {
-        const int c = sub + j * L;
-        xv[j] = load_as_f32<DT>(x, xoff + (c < n_cols ? c : n_cols - 1));
-      }
-#pragma unroll
-      for (int j = 0; j < EPL; ++j) asm volatile("" : "+v"(xv[j]));
-#pragma unroll
-      for (int j = 0; j < EPL; ++j) {
-        const int c = sub + j * L;
-        keys[j] = c < n_cols ? logit_key(xv[j], c) : 0ull;
-      }
-    }
-    uint64_t prev = ~0ull;
-    for (int pass = 0; pass < k; ++pass) {
-      uint64_t best = 0ull;
-      if constexpr (EPL > 0) {
-#pragma unroll
-        for (int j = 0; j < EPL; ++j) {
-          uint64_t q = keys[j];
-          best = (q < prev && q > best) ? q : best;
-        }
-      } else {
-        for (int c = sub; c < n_cols; c += L) {
-          uint64_t q = logit_key(load_as_f32<DT>(x, xoff + c), c);
-          best = (q < prev && q > best) ? q : best;
-        }
-      }
-      best = group_max_u64<L>(best);
-      if (sub == pass) mine = best;
-      prev = best;
-    }
-    my_idx = (int)(0xFFFFu - (uint32_t)(mine & 0xFFFFull));
-  }
+  uint32_t words = 0u;  // (EPL > 0)
+  float v = 0.f, top = 0.f;
   const bool slot = sub < k;
-  float v;
-  if (apply_softmax && !use_provided) {
-    v = slot ? logit_of_key(mine) : 0.f;  // a zero's sign is lost in the key and makes no difference to the softmax
+  if (use_provided) {
+    if (slot) my_idx = y_indx[rrow * y_stride + sub];
+  } else if constexpr (EPL > 0) {
+    RowLogits<DT, L, EPL> logits;
+    SortKey<DT> keys[EPL];
+    logits.request(x, xoff, n_cols, sub);
+    logits.take(keys, n_cols, sub);
+    const Picks<DT> r = pick_columns<L, EPL, DT>(keys, k, sub);
+    my_idx = r.col();
+    words = r.word;
+    v = r.key.logit();  // a zero's sign is lost in the key and makes no difference to the softmax
+    top = r.top.logit();
   } else {
-    v = slot ? load_as_f32<DT>(x, xoff + my_idx) : 0.f;
+    // bits and column of the last pick: what comes after it in the order has lower bits, or the same and a higher column
+    uint32_t prev = 0u, prev_c = 0u;
+    for (int pass = 0; pass < k; ++pass) {
+      uint32_t m = 0u, mc = 0xFFFFu;
+      for (int c = sub; c < n_cols; c += L) {
+        const uint32_t q = ordered_bits(load_as_f32<DT>(x, xoff + c));
+        const bool left = pass == 0 || q < prev || (q == prev && (uint32_t)c > prev_c);
+        if (left && (mc == 0xFFFFu || q > m)) {
+          m = q;
+          mc = (uint32_t)c;
+        }
+      }
+      const uint32_t best = group_max_u32<L>(mc == 0xFFFFu ? 0u : m);
+      prev_c = group_min_u32<L>(m == best ? mc : 0xFFFFu);
+      prev = best;
+      if (pass == 0) top = logit_of(best);
+      if (sub == pass) {
+        v = logit_of(best);
+        my_idx = (int)prev_c;
+      }
+    }
   }
+  if (!apply_softmax || use_provided) v = slot ? load_as_f32<DT>(x, xoff + my_idx) : 0.f;
   if (apply_softmax) {
-    float mx = group_max_f32<L>(slot ? v : -__builtin_inff());
-    float e = slot ? expf(v - mx) : 0.f;
-    float s = group_sum_f32<L>(e);
-    v = e / s;
+    const float mx = use_provided ? group_max_f32<L>(slot ? v : -__builtin_inff()) : top;
+    const float e = slot ? expf(v - mx) : 0.f;
+    v = e / group_sum_f32<L>(e);
   }
   if (live && slot) {
     store_from_f32<DT>(y_vals, rrow * y_stride + sub, v);
     if (!use_provided) y_indx[rrow * y_stride + sub] = (int16_t)my_idx;
-    if (lds_indx) lds_indx[rrow * k + sub] = my_idx;
-    if (lds_gate) lds_gate[rrow * k + sub] = DT == TAMD_F32 ? f32_to_bits(v) : DT == TAMD_BF16 ? f32_to_bf16_bits(v) : f32_to_f16_bits(v);
   }
   const int n_words = (n_cols + 31) / 32;
+  if (EPL > 0 && !use_provided) {
+    if (live && sub < n_words) bits[rrow * bits_stride_row + (int64_t)sub * bits_stride_word] = words;
+    return;
+  }
   const int base_lane = (threadIdx.x % kWave) - sub;
   for (int w0 = 0; w0 < n_words; w0 += L) {
     int w = w0 + sub;
@@ -170,7 +281,7 @@ __global__ __launch_bounds__(256) void topk_kernel(const void *__restrict__ x, i
                                                    int64_t bits_stride_row, int64_t bits_stride_word) {
   constexpr int ROWS_PER_BLOCK = 256 / L;
   topk_row<DT, L, EPL>(x, x_stride, n_rows, n_cols, k, apply_softmax, use_provided, y_vals, y_indx, y_stride, bits,
-                       bits_stride_row, bits_stride_word, (int64_t)blockIdx.x * ROWS_PER_BLOCK + threadIdx.x / L, nullptr);
+                       bits_stride_row, bits_stride_word, (int64_t)blockIdx.x * ROWS_PER_BLOCK + threadIdx.x / L);
 }
 
 template <int DT>
@@ -181,8 +292,10 @@ int launch_topk(const void *x, int64_t xs, int n_rows, int n_cols, int k, int sm
 #define TAMD_TOPK(LL, EE)                                                                                    \
   topk_kernel<DT, LL, EE><<<dim3((unsigned)((n_rows + (256 / LL) - 1) / (256 / LL))), 256, 0, st>>>(          \
       x, xs, n_rows, n_cols, k, sm, prov, yv, yi, ys, bits, bsr, bsw)
-  if (need <= 8) TAMD_TOPK(8, 8);
-  else if (need <= 16) TAMD_TOPK(16, 8);
+  if (need <= 8) {
+    if (n_cols <= 32) TAMD_TOPK(8, 4);
+    else TAMD_TOPK(8, 8);
+  } else if (need <= 16) TAMD_TOPK(16, 8);
   else if (need <= 32) TAMD_TOPK(32, 8);
   else if (n_cols <= 512) TAMD_TOPK(64, 8);
   else TAMD_TOPK(64, 0);
@@ -513,8 +626,7 @@ __global__ __launch_bounds__(1024) void scan_ragged_kernel(int E, int n_blocks, 
 // ---------------------------------------------------------------------------
 // metadata in two launches (up to kMaxTableBlocks blocks of chunks)
 // ---------------------------------------------------------------------------
-// The first launch leaves one histogram per block of CH chunks (hist_kernel, or topk_hist_kernel straight from the
-// logits).  In the second, every workgroup reduces that small table by itself -- the experts' totals, their prefix and,
+// The first launch leaves one histogram per block of CH chunks (hist_kernel).  In the second, every workgroup reduces that small table by itself -- the experts' totals, their prefix and,
 // for the workgroup that orders block `blk`, the counts of the blocks before it -- instead of waiting for a scan kernel
 // in between: workgroups 0..nb-1 recount their own chunks and place their entries, the remaining ones build the ragged
 // tables and fill the block schedule.
@@ -546,7 +658,7 @@ __global__ __launch_bounds__(1024) void order_scan_kernel(const void *__restrict
                                                           int32_t *__restrict__ col_sorted, int32_t *__restrict__ row_sorted,
                                                           int32_t *__restrict__ gather, int32_t *__restrict__ offs,
                                                           int64_t offs_pitch, int32_t *__restrict__ sched,
-                                                          int64_t sched_pitch, int max_blocks, Gates gates, int sub) {
+                                                          int64_t sched_pitch, int max_blocks, Gates gates) {
   extern __shared__ int32_t sm[];
   int32_t *hist = sm;                          // [CH][E]  counts of this block's chunks, then their exclusive prefix
   int32_t *tot = hist + (int64_t)CH * E;       // [E]      entries per expert
@@ -556,8 +668,7 @@ __global__ __launch_bounds__(1024) void order_scan_kernel(const void *__restrict
   int32_t *tab = pbel + (int64_t)P * E;        // [6][E + 1]
   const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
   const int blk = blockIdx.x;
-  const int nbo = (nb + sub - 1) / sub;        // blocks of CH chunks, `sub` rows of the table each
-  const bool orders = blk < nbo;
+  const bool orders = blk < nb;
   // this wave's chunk of the index array: requested first, used after the table has been reduced
   const int i = (blk * CH + wave) * 64 + lane;
   const bool has = orders && wave < CH && i < n;
@@ -576,7 +687,7 @@ __global__ __launch_bounds__(1024) void order_scan_kernel(const void *__restrict
       const int per = (nb + P - 1) / P;
       const int b_hi = (part + 1) * per < nb ? (part + 1) * per : nb;
       int all, below;
-      sum_block_range(block_tot, E, e, part * per, b_hi, blk * sub, all, below);
+      sum_block_range(block_tot, E, e, part * per, b_hi, blk, all, below);
       psum[part * E + e] = all;
       pbel[part * E + e] = below;
     }
@@ -610,7 +721,7 @@ __global__ __launch_bounds__(1024) void order_scan_kernel(const void *__restrict
       }
     }
   }
-  ragged_scan_rows(tot, E, tab, blk == nbo ? offs : nullptr, offs_pitch);
+  ragged_scan_rows(tot, E, tab, blk == nb ? offs : nullptr, offs_pitch);
   sync_threads();
   if (orders) {
     // 4. placement
@@ -631,16 +742,16 @@ __global__ __launch_bounds__(1024) void order_scan_kernel(const void *__restrict
   } else {
     // 4'. this workgroup's share of the block schedule
     const int64_t total = 5 * (int64_t)max_blocks;
-    const int64_t shares = (int64_t)gridDim.x - nbo;
+    const int64_t shares = (int64_t)gridDim.x - nb;
     const int64_t per = (total + shares - 1) / shares;
-    const int64_t first = per * (blk - nbo);
+    const int64_t first = per * (blk - nb);
     if (first < total) ragged_fill_schedule(tab, E, sched, sched_pitch, max_blocks, first, per < total - first ? per : total - first);
   }
 }
 
 // Second launch of the two: the grid, the LDS size and the limits of order_scan_kernel.
-inline bool order_scan_applicable(int64_t n, int E, int CH, int64_t nb, int64_t max_nb = kMaxTableBlocks) {
-  if (E > 1024 || nb < 1 || nb > max_nb || n > 0x7FFFFFFF - 64 * 1024) return false;
+inline bool order_scan_applicable(int64_t n, int E, int CH, int64_t nb) {
+  if (E > 1024 || nb < 1 || nb > kMaxTableBlocks || n > 0x7FFFFFFF - 64 * 1024) return false;
   int P = 1024 / E;
   P = P > 16 ? 16 : P;
   const int64_t ints = (int64_t)CH * E + 2 * (int64_t)E + 2 * (int64_t)P * E + 6 * ((int64_t)E + 1);
@@ -650,7 +761,7 @@ inline bool order_scan_applicable(int64_t n, int E, int CH, int64_t nb, int64_t 
 inline int launch_order_scan(const void *indx, int is16, int64_t n, int E, int CH, int nbits, int k, const int32_t *block_tot,
                              int64_t nb, int32_t *col_sum, int32_t *col_sorted, int32_t *row_sorted, int32_t *gather,
                              int32_t *offs, int64_t offs_pitch, int32_t *sched, int64_t sched_pitch, int max_blocks,
-                             Gates gates, hipStream_t st, int sub = 1) {
+                             Gates gates, hipStream_t st) {
   int P = 1024 / E;
   P = P > 16 ? 16 : P;
   P = P > nb ? (int)nb : P;
@@ -658,64 +769,231 @@ inline int launch_order_scan(const void *indx, int is16, int64_t n, int E, int C
   int64_t shares = (5 * (int64_t)max_blocks + 4095) / 4096;  // about four schedule entries per thread
   shares = shares < 1 ? 1 : (shares > 64 ? 64 : shares);
   if (int rc = raise_lds_limit_once((const void *)order_scan_kernel)) return rc;
-  order_scan_kernel<<<dim3((unsigned)((nb + sub - 1) / sub + shares)), 1024, (size_t)ints * 4, st>>>(
+  order_scan_kernel<<<dim3((unsigned)(nb + shares)), 1024, (size_t)ints * 4, st>>>(
       indx, is16, (int)n, E, CH, nbits, k, block_tot, (int)nb, P, col_sum, col_sorted, row_sorted, gather, offs, offs_pitch,
-      sched, sched_pitch, max_blocks, gates, sub);
+      sched, sched_pitch, max_blocks, gates);
   return launch_status();
 }
 
-// First launch of the two, from the logits: the experts of TH / L rows per workgroup (their picked columns also go to
-// LDS) and the histogram of that block of CH = (TH / L) * k / 64 whole chunks.  A row is a chain of some 400 instructions, so
-// the workgroups are as small as whole chunks allow (4096 rows of 128, top-4, both launches in a graph -- a call waits for the host --: 13.3 us with 1024
-// threads, 12.6 with 512; 1024 rows 12.4 and, with 256, 11.4).
+// ---------------------------------------------------------------------------
+// routing from the logits in two launches
+// ---------------------------------------------------------------------------
+// A row picks an expert at most once.  So a block of up to 255 rows counts its entries per expert in a byte, and the place of
+// an entry among those of its expert is the number of earlier rows that picked it: bits of a mask with one bit per row
+// and expert, set in LDS in any order, and counted.  No ballots per chunk, no prefix sums over chunks.
+constexpr int kMaxRowsPerBlock = 255;
+
+// i / k for i * k < 2^19, k <= 64: i * reciprocal_of(k) >> 19 (the reciprocal is too large by at most k / 2^19).
+inline uint32_t reciprocal_of(int k) { return (1u << 19) / (uint32_t)k + 1u; }
+TAMD_DEVICE int over_k(int i, uint32_t inv) { return (int)((uint32_t)i * inv >> 19); }
+
+// Rows of `members` [E][W]: the rows before row r that picked expert e.
+TAMD_DEVICE int rows_before(const uint32_t *members, int W, int e, int r) {
+  const int rw = r >> 5;
+  int n = 0;
+  for (int w = 0; w < W; ++w) {
+    const uint32_t m = members[e * W + w];
+    n += __popc(w < rw ? m : (w == rw ? m & ((1u << (r & 31)) - 1u) : 0u));
+  }
+  return n;
+}
+
+// First launch: the experts of RB rows per workgroup, TH / L at a time, and the bytes of their counts: row `blockIdx.x` of
+// the table, `pitch` bytes.  The workgroups are as small as a short table allows, since a row is a chain of
+// instructions that the waves of a SIMD share.  (Both launches in a graph, with 32-bit tables and a histogram per 64 entries before:
+// 4096 rows of 128, top-4: 12.0 -> 8.5 us; 333 of 32: 9.0 -> 6.8; 9350 of 256, bf16, top-8: 22.8 -> 16.2, four launches
+// before; 32768 of 256, top-8: 52 -> 36.)
 template <int DT, int L, int EPL, int TH>
 __global__ __launch_bounds__(TH) void topk_hist_kernel(const void *__restrict__ x, int64_t x_stride, int n_rows, int E,
                                                          int k, void *__restrict__ y_vals, int16_t *__restrict__ y_indx,
                                                          uint32_t *__restrict__ bits, int64_t bits_stride_row,
-                                                         int64_t bits_stride_word, int nbits, int CH,
-                                                         int32_t *__restrict__ block_tot) {
-  extern __shared__ int32_t sm[];
+                                                         int64_t bits_stride_word, int RB, int pitch,
+                                                         uint32_t *__restrict__ table) {
+  __shared__ int32_t hist[512];
   constexpr int ROWS = TH / L;
-  int32_t *lidx = sm;            // [CH * 64] picked columns of this block's rows
-  int32_t *hist = sm + CH * 64;  // [CH][E]
-  const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
-  const int64_t row0 = (int64_t)blockIdx.x * ROWS;
-  for (int j = tid; j < CH * E; j += TH) hist[j] = 0;  // (the barrier below covers them)
-  topk_row<DT, L, EPL>(x, x_stride, n_rows, E, k, 1, 0, y_vals, y_indx, k, bits, bits_stride_row, bits_stride_word,
-                       row0 + tid / L, lidx - row0 * k);
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / kWave), sub = tid % L, n_words = (E + 31) / 32;
+  const int64_t end = (int64_t)(blockIdx.x + 1) * RB < n_rows ? (int64_t)(blockIdx.x + 1) * RB : n_rows;
+  int64_t row = (int64_t)blockIdx.x * RB + tid / L;
+  RowLogits<DT, L, EPL> logits;
+  logits.request(x, (row < end ? row : end - 1) * x_stride, E, sub);
+  for (int j = tid; j < pitch; j += TH) hist[j] = 0;
   sync_threads();
-  for (int c = wave; c < CH; c += TH / kWave) {
-    const int j = c * 64 + lane;  // entry of the block; its row exists or not
-    const bool valid = row0 + j / k < n_rows;
-    const int e = valid ? lidx[j] : -1;
-    const uint64_t same = same_id_mask(e, valid, nbits);
-    if (valid && (same & lanemask_lt()) == 0) hist[c * E + e] = __popcll(same);
+  // (a wave without a row of its own stays out)
+  for (int64_t row0 = (int64_t)blockIdx.x * RB + wave * (kWave / L); row0 < end; row0 += ROWS, row += ROWS) {
+    SortKey<DT> keys[EPL];
+    logits.take(keys, E, sub);
+    if (row0 + ROWS < end) logits.request(x, (row + ROWS < end ? row + ROWS : end - 1) * x_stride, E, sub);
+    const Picks<DT> r = pick_columns<L, EPL, DT>(keys, k, sub);
+    const bool slot = sub < k;
+    if (row < end && slot) atomicAdd(&hist[r.col()], 1);
+    const float v = pick_softmax<L, DT>(r, slot);
+    if (row < end) {
+      if (slot) {
+        store_from_f32<DT>(y_vals, row * k + sub, v);
+        y_indx[row * k + sub] = (int16_t)r.col();
+      }
+      if (sub < n_words) bits[row * bits_stride_row + (int64_t)sub * bits_stride_word] = r.word;
+    }
   }
   sync_threads();
-  for (int e = tid; e < E; e += TH) {
-    int run = 0;
-    for (int c = 0; c < CH; ++c) run += hist[c * E + e];
-    block_tot[(int64_t)blockIdx.x * E + e] = run;
+  for (int j = tid; j < pitch / 4; j += TH)
+    table[(int64_t)blockIdx.x * (pitch / 4) + j] =
+        (uint32_t)hist[4 * j] | (uint32_t)hist[4 * j + 1] << 8 | (uint32_t)hist[4 * j + 2] << 16 | (uint32_t)hist[4 * j + 3] << 24;
+}
+
+// Second launch: every workgroup sums the bytes of the table by itself (all blocks, and those before its own rows: two
+// experts to a register, sixteen bits each, so up to 65535 rows).  The first `nbo` place the entries of `sub` blocks
+// each; the others build the ragged tables and fill the block schedule, about an entry per thread (a search of the
+// table's row is a chain of LDS reads, and four of them in a row were the longest path of the launch).
+__global__ __launch_bounds__(1024) void order_rows_kernel(const int16_t *__restrict__ indx, int n, int E, int k, uint32_t inv_k,
+                                                          const uint32_t *__restrict__ table, int lg_cols, int nb, int RB,
+                                                          int sub, int nbo, int W, int32_t *__restrict__ col_sum,
+                                                          int32_t *__restrict__ col_sorted, int32_t *__restrict__ row_sorted,
+                                                          int32_t *__restrict__ gather, int32_t *__restrict__ offs,
+                                                          int64_t offs_pitch, int32_t *__restrict__ sched,
+                                                          int64_t sched_pitch, int max_blocks, Gates gates) {
+  extern __shared__ int32_t sm[];
+  const int cols = 1 << lg_cols;                       // dwords of a table row
+  uint32_t *sums = (uint32_t *)sm;                     // [4][cols]  experts 4c, 4c + 2 | 4c + 1, 4c + 3: all blocks, then the earlier ones
+  uint32_t *members = sums + 4 * cols;                 // [E][W]
+  int32_t *place = (int32_t *)members + E * W;         // [waves][E] first entry of each expert (a copy per wave) or [6][E + 1]
+  const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave, blk = blockIdx.x;
+  const bool orders = blk < nbo;
+  const int first = blk * sub * RB * k;                // this workgroup's entries
+  const int count = orders ? (sub * RB * k < n - first ? sub * RB * k : n - first) : 0;
+  // entries and table are requested together; LDS is cleared meanwhile
+  const int i0 = tid < count ? tid : 0;
+  int ev = indx[first < n ? first + i0 : 0];
+  uint32_t gate = load_gate(gates, first < n ? first + i0 : 0);
+  const int c = tid & (cols - 1), r0 = tid >> lg_cols, step = 1024 >> lg_cols;
+  uint32_t t[8];
+#pragma unroll
+  for (int u = 0; u < 8; ++u) t[u] = table[(int64_t)(r0 + u * step < nb ? r0 + u * step : nb - 1) * cols + c];
+  for (int j = tid; j < 4 * cols + E * W; j += 1024) sm[j] = 0;
+  sync_threads();
+  uint32_t all0 = 0, all1 = 0, bel0 = 0, bel1 = 0;
+  for (int b0 = r0;;) {
+#pragma unroll
+    for (int u = 0; u < 8; ++u) asm volatile("" : "+v"(t[u]));
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int b = b0 + u * step;
+      const uint32_t even = b < nb ? t[u] & 0x00FF00FFu : 0u, odd = b < nb ? t[u] >> 8 & 0x00FF00FFu : 0u;
+      all0 += even;
+      all1 += odd;
+      bel0 += b < blk * sub ? even : 0u;
+      bel1 += b < blk * sub ? odd : 0u;
+    }
+    b0 += 8 * step;
+    if (b0 - r0 >= nb) break;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) t[u] = table[(int64_t)(b0 + u * step < nb ? b0 + u * step : nb - 1) * cols + c];
   }
+  if (r0 < nb) {
+    atomicAdd(&sums[c], all0);
+    atomicAdd(&sums[cols + c], all1);
+    if (orders) {
+      atomicAdd(&sums[2 * cols + c], bel0);
+      atomicAdd(&sums[3 * cols + c], bel1);
+    }
+  }
+  for (int i = tid; i < count; i += 1024) {
+    const int e = i == tid ? ev : indx[first + i], r = over_k(i, inv_k);
+    atomicOr(&members[e * W + (r >> 5)], 1u << (r & 31));
+  }
+  sync_threads();
+  const auto total_of = [&](const uint32_t *part, int e) { return (int)(part[(e & 1) * cols + (e >> 2)] >> ((e & 2) * 8) & 0xFFFFu); };
+  if (orders) {
+    // a wave with entries scans the totals into a copy of its own: no barrier in between
+    if (wave * kWave < count) {
+      int32_t *mine = place + wave * E;
+      int carry = 0;
+      for (int s0 = 0; s0 < E; s0 += kWave) {
+        const int s = s0 + lane, v = s < E ? total_of(sums, s) : 0, inc = wave_incl_scan(v);
+        if (s < E) mine[s] = carry + inc - v;
+        if (s < E && blk == 0 && wave == 0) col_sum[s] = v;
+        carry += __builtin_amdgcn_readlane(inc, kWave - 1);
+      }
+      for (int i = tid; i < count; i += 1024) {
+        const int e = i == tid ? ev : indx[first + i], r = over_k(i, inv_k);
+        const int pos = mine[e] + total_of(sums + 2 * cols, e) + rows_before(members, W, e, r);
+        row_sorted[first + i] = pos;
+        col_sorted[pos] = first + i;
+        if (gather) gather[pos] = blk * sub * RB + r;
+        store_gate(gates, pos, i == tid ? gate : load_gate(gates, first + i));
+      }
+    }
+  } else {
+    int32_t *sizes = (int32_t *)members, *tab = place;  // (E * W >= E)
+    for (int e = tid; e < E; e += 1024) sizes[e] = total_of(sums, e);
+    sync_threads();
+    ragged_scan_rows(sizes, E, tab, blk == nbo ? offs : nullptr, offs_pitch);
+    sync_threads();
+    const int64_t total = 5 * (int64_t)max_blocks;
+    const int64_t shares = (int64_t)gridDim.x - nbo;
+    const int64_t per = (total + shares - 1) / shares;
+    const int64_t begin = per * (blk - nbo);
+    if (begin < total) ragged_fill_schedule(tab, E, sched, sched_pitch, max_blocks, begin, per < total - begin ? per : total - begin);
+  }
+}
+
+// How the two launches cut n_rows rows.
+struct RowPlan {
+  int TH, RB, pitch, lg_cols, nb, sub, nbo, W;
+  size_t lds;
+};
+
+// Fills the plan, or returns false where the table or the counts do not fit.  The workgroups of the first launch are the smallest whose table
+// is read with four loads per thread (16 KB); a longer input makes the blocks larger, up to 255 rows.
+inline bool make_row_plan(int64_t n_rows, int E, int k, int L, int64_t workspace_ints, RowPlan &p) {
+  if (n_rows < 1 || n_rows > 65535 || E > 512) return false;
+  p.pitch = 16;
+  while (p.pitch < E) p.pitch *= 2;
+  p.lg_cols = __builtin_ctz(p.pitch / 4);
+  p.TH = 256;
+  while (p.TH < 1024 && (n_rows + p.TH / L - 1) / (p.TH / L) * p.pitch > 16384) p.TH *= 2;
+  p.RB = p.TH / L;
+  while (2 * p.RB <= kMaxRowsPerBlock && (n_rows + p.RB - 1) / p.RB * p.pitch > 65536) p.RB *= 2;
+  p.nb = (int)((n_rows + p.RB - 1) / p.RB);
+  if ((int64_t)p.nb * (p.pitch / 4) > workspace_ints) return false;
+  p.sub = 1;
+  while (p.RB * p.sub * 2 * k <= 1024 && p.RB * p.sub * 2 <= 128 && p.sub < p.nb) p.sub *= 2;
+  p.nbo = (p.nb + p.sub - 1) / p.sub;
+  p.W = (p.RB * p.sub + 31) / 32;
+  if ((int64_t)p.RB * p.sub * k * k >= 1 << 19) return false;  // over_k
+  const int64_t waves = p.RB * p.sub * k >= 1024 ? 16 : (p.RB * p.sub * k + kWave - 1) / kWave;
+  const int64_t copies = waves * E > 6 * (E + 1) ? waves * E : 6 * (E + 1);
+  p.lds = (size_t)(p.pitch + (int64_t)E * p.W + copies) * 4;
+  return p.lds <= 150 * 1024;
 }
 
 template <int DT>
 int launch_topk_hist(const void *x, int64_t xs, int n_rows, int E, int k, void *yv, int16_t *yi, uint32_t *bits, int64_t bsr,
-                     int64_t bsw, int nbits, int L, int TH, int32_t *block_tot, hipStream_t st) {
-  const int CH = TH / L * k / 64;
-  const size_t lds = ((size_t)CH * 64 + (size_t)CH * E) * 4;
-  const unsigned grid = (unsigned)((n_rows + TH / L - 1) / (TH / L));
+                     int64_t bsw, int L, const RowPlan &p, uint32_t *table, hipStream_t st) {
 #define TAMD_TH(LL, EE)                                                                                                 \
   do {                                                                                                                  \
-    auto kern = TH == 256 ? topk_hist_kernel<DT, LL, EE, 256>                                                           \
-                          : (TH == 512 ? topk_hist_kernel<DT, LL, EE, 512> : topk_hist_kernel<DT, LL, EE, 1024>);       \
-    kern<<<grid, TH, lds, st>>>(x, xs, n_rows, E, k, yv, yi, bits, bsr, bsw, nbits, CH, block_tot);                     \
+    auto kern = p.TH == 256 ? topk_hist_kernel<DT, LL, EE, 256>                                                         \
+                            : (p.TH == 512 ? topk_hist_kernel<DT, LL, EE, 512> : topk_hist_kernel<DT, LL, EE, 1024>);   \
+    kern<<<(unsigned)p.nb, p.TH, 0, st>>>(x, xs, n_rows, E, k, yv, yi, bits, bsr, bsw, p.RB, p.pitch, table);           \
   } while (0)
-  if (L == 8) TAMD_TH(8, 8);
+  if (L == 8 && E <= 32) TAMD_TH(8, 4);
+  else if (L == 8) TAMD_TH(8, 8);
   else if (L == 16) TAMD_TH(16, 8);
   else if (L == 32) TAMD_TH(32, 8);
   else TAMD_TH(64, 8);
 #undef TAMD_TH
+  return launch_status();
+}
+
+inline int launch_order_rows(const int16_t *indx, int64_t n, int E, int k, const RowPlan &p, const uint32_t *table, int32_t *col_sum,
+                             int32_t *col_sorted, int32_t *row_sorted, int32_t *gather, int32_t *offs, int64_t offs_pitch,
+                             int32_t *sched, int64_t sched_pitch, int max_blocks, Gates gates, hipStream_t st) {
+  int64_t shares = (5 * (int64_t)max_blocks + 1023) / 1024;
+  shares = shares < 1 ? 1 : (shares > 64 ? 64 : shares);
+  if (int rc = raise_lds_limit_once((const void *)order_rows_kernel)) return rc;
+  order_rows_kernel<<<(unsigned)(p.nbo + shares), 1024, p.lds, st>>>(indx, (int)n, E, k, reciprocal_of(k), table, p.lg_cols, p.nb, p.RB,
+                                                                    p.sub, p.nbo, p.W, col_sum, col_sorted, row_sorted, gather, offs,
+                                                                    offs_pitch, sched, sched_pitch, max_blocks, gates);
   return launch_status();
 }
 
@@ -725,22 +1003,20 @@ int launch_topk_hist(const void *x, int64_t xs, int n_rows, int E, int k, void *
 // For index arrays small enough that the per-chunk histogram fits LDS (n/64 * E ints): histogram,
 // the three prefix sums, the ordering and the ragged tables without leaving the workgroup --
 // one launch instead of four, which is what the cost of routing is made of at these sizes.
-// lidx: the index array in LDS (a kernel that has just computed it), or null to read `indx` from memory.
-// lgate: the gate weights' bits in LDS beside it, or null likewise.
-TAMD_DEVICE void meta_fused_body(int32_t *sm, bool zeroed, const int32_t *lidx, const uint32_t *lgate, const void *__restrict__ indx, int is16,
-                                 int n, int E, int k, int nbits, int NC, int P, int32_t *__restrict__ col_sum,
-                                 int32_t *__restrict__ col_sorted, int32_t *__restrict__ row_sorted,
-                                 int32_t *__restrict__ gather, int32_t *__restrict__ offs, int64_t offs_pitch,
-                                 int32_t *__restrict__ sched, int64_t sched_pitch, int max_blocks, Gates gates) {
+__global__ __launch_bounds__(1024) void meta_fused_kernel(const void *__restrict__ indx, int is16, int n, int E, int k,
+                                                          int nbits, int NC, int P, int32_t *__restrict__ col_sum,
+                                                          int32_t *__restrict__ col_sorted, int32_t *__restrict__ row_sorted,
+                                                          int32_t *__restrict__ gather, int32_t *__restrict__ offs,
+                                                          int64_t offs_pitch, int32_t *__restrict__ sched,
+                                                          int64_t sched_pitch, int max_blocks, Gates gates) {
+  extern __shared__ int32_t sm[];
   int32_t *hist = sm;                         // [NC][E]  counts, then exclusive prefix over chunks
   int32_t *csum = hist + (int64_t)NC * E;     // [E]
   int32_t *psum = csum + E;                   // [P][E]   partial sums of chunk ranges
   int32_t *tab = psum + (int64_t)P * E;       // [6][E + 1]
   const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
-  if (!zeroed) {
-    for (int i = tid; i < NC * E; i += 1024) hist[i] = 0;
-    sync_threads();
-  }
+  for (int i = tid; i < NC * E; i += 1024) hist[i] = 0;
+  sync_threads();
   // 1. per-chunk histogram.  A wave takes its chunks eight at a time so that eight index loads are in
   // flight together (one workgroup has nothing else to hide their latency with).
   for (int c0 = wave; c0 < NC && n > 0; c0 += 16 * 8) {
@@ -749,7 +1025,7 @@ TAMD_DEVICE void meta_fused_body(int32_t *sm, bool zeroed, const int32_t *lidx, 
     for (int u = 0; u < 8; ++u) {  // unconditional loads (entries past the end re-read entry 0), so all eight are in flight
       const int i = (c0 + 16 * u) * 64 + lane;
       const bool ok = c0 + 16 * u < NC && i < n;
-      ev[u] = lidx ? lidx[ok ? i : 0] : load_indx(indx, is16, ok ? i : 0);
+      ev[u] = load_indx(indx, is16, ok ? i : 0);
     }
 #pragma unroll
     for (int u = 0; u < 8; ++u) asm volatile("" : "+v"(ev[u]));  // pinned: the loads stay outside the selection below
@@ -818,7 +1094,7 @@ TAMD_DEVICE void meta_fused_body(int32_t *sm, bool zeroed, const int32_t *lidx, 
     for (int u = 0; u < 8; ++u) {  // unconditional loads (entries past the end re-read entry 0), so all eight are in flight
       const int i = (c0 + 16 * u) * 64 + lane;
       const bool ok = c0 + 16 * u < NC && i < n;
-      ev[u] = lidx ? lidx[ok ? i : 0] : load_indx(indx, is16, ok ? i : 0);
+      ev[u] = load_indx(indx, is16, ok ? i : 0);
     }
 #pragma unroll
     for (int u = 0; u < 8; ++u) asm volatile("" : "+v"(ev[u]));  // pinned: the loads stay outside the selection below
@@ -840,7 +1116,7 @@ TAMD_DEVICE void meta_fused_body(int32_t *sm, bool zeroed, const int32_t *lidx, 
         row_sorted[i] = pos;
         col_sorted[pos] = i;
         if (gather) gather[pos] = i / k;
-        store_gate(gates, pos, lgate ? lgate[i] : load_gate(gates, i));
+        store_gate(gates, pos, load_gate(gates, i));
       } else if (i < n) {
         row_sorted[i] = -1;
       }
@@ -854,68 +1130,118 @@ TAMD_DEVICE void meta_fused_body(int32_t *sm, bool zeroed, const int32_t *lidx, 
   ragged_fill_schedule(tab, E, sched, sched_pitch, max_blocks, 0, 5 * (int64_t)max_blocks);
 }
 
-__global__ __launch_bounds__(1024) void meta_fused_kernel(const void *__restrict__ indx, int is16, int n, int E, int k,
-                                                          int nbits, int NC, int P, int32_t *__restrict__ col_sum,
-                                                          int32_t *__restrict__ col_sorted, int32_t *__restrict__ row_sorted,
-                                                          int32_t *__restrict__ gather, int32_t *__restrict__ offs,
-                                                          int64_t offs_pitch, int32_t *__restrict__ sched,
-                                                          int64_t sched_pitch, int max_blocks, Gates gates) {
-  extern __shared__ int32_t sm[];
-  meta_fused_body(sm, false, nullptr, nullptr, indx, is16, n, E, k, nbits, NC, P, col_sum, col_sorted, row_sorted, gather, offs,
-                  offs_pitch, sched, sched_pitch, max_blocks, gates);
-}
-
 // ---------------------------------------------------------------------------
 // top-k and all routing metadata in one workgroup (decode sizes)
 // ---------------------------------------------------------------------------
-// With a few dozen tokens the two launches of routing cost more than their work.  Here the 1024 threads first pick
-// the experts of 1024 / L rows at a time (the picked columns also go to LDS), then run the metadata phases of
-// meta_fused_kernel on the index array in LDS.
+// With a few dozen tokens two launches of routing cost more than their work.  Here 1024 threads pick the experts of as many
+// rows as they hold and set the rows' bits per expert (`members`, as above); six waves sum and scan those bits into the
+// ragged tables, each the row of one block size, and write their entries of the block schedule from the scan's registers;
+// then every entry is placed by the lane that picked it.  What such a workgroup is made of is the length of its chains, not its work:
+// with a histogram per 64 entries, prefix sums over them and a search per schedule entry one row of 128 logits took 14 500
+// cycles (6.4 us; 64 rows 9.5), now @@.
 template <int DT, int L, int EPL>
 __global__ __launch_bounds__(1024) void routing_fused_kernel(const void *__restrict__ x, int64_t x_stride, int n_rows,
-                                                             int E, int k, void *__restrict__ y_vals,
+                                                             int E, int k, int W, void *__restrict__ y_vals,
                                                              int16_t *__restrict__ y_indx, uint32_t *__restrict__ bits,
-                                                             int64_t bits_stride_row, int64_t bits_stride_word, int nbits,
-                                                             int NC, int P, int32_t *__restrict__ col_sum,
+                                                             int64_t bits_stride_row, int64_t bits_stride_word,
+                                                             int32_t *__restrict__ col_sum,
                                                              int32_t *__restrict__ col_sorted,
                                                              int32_t *__restrict__ row_sorted, int32_t *__restrict__ gather,
                                                              int32_t *__restrict__ offs, int64_t offs_pitch,
                                                              int32_t *__restrict__ sched, int64_t sched_pitch,
                                                              int max_blocks, Gates gates) {
   extern __shared__ int32_t sm[];
-  const int n = n_rows * k, n4 = (n + 3) / 4 * 4;
-  int32_t *lidx = sm;                        // [n] picked columns
-  uint32_t *lgate = (uint32_t *)sm + n4;     // [n] gate weights
-  int32_t *meta = sm + 2 * n4;
-  constexpr int ROWS = 1024 / L;
-  for (int i = threadIdx.x; i < NC * E; i += 1024) meta[i] = 0;  // the histograms (the barrier below covers them)
-  // (a wave without a row of its own stays out: the passes of a row are a chain of instructions, and four waves of a SIMD
-  // working on nothing made the one that had a row wait: 1 row of 128 logits 7.9 us, now 6.6)
-  for (int row0 = (int)(threadIdx.x / kWave) * (kWave / L), wave0 = row0; row0 < n_rows; row0 += ROWS)
-    topk_row<DT, L, EPL>(x, x_stride, n_rows, E, k, 1, 0, y_vals, y_indx, k, bits, bits_stride_row, bits_stride_word,
-                         (int64_t)(row0 - wave0) + threadIdx.x / L, lidx, lgate);
+  constexpr int PER = L * EPL > kWave ? L * EPL / kWave : 1;  // neighbouring experts to a lane of the scans
+  uint32_t *members = (uint32_t *)sm;              // [E][W]
+  int32_t *place = sm + E * W;                     // [E]  first entry of each expert
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / kWave), lane = tid % kWave, sub = tid % L;
+  const int row = tid / L;
+  const bool busy = wave * (kWave / L) < n_rows;   // (a wave without a row stays out of the way of those that have one)
+  const bool slot = sub < k && row < n_rows;
+  RowLogits<DT, L, EPL> logits;
+  if (busy) logits.request(x, (int64_t)(row < n_rows ? row : n_rows - 1) * x_stride, E, sub);
+  for (int i = tid; i < E * W; i += 1024) members[i] = 0;
   sync_threads();
-  meta_fused_body(meta, true, lidx, lgate, nullptr, 0, n, E, k, nbits, NC, P, col_sum, col_sorted, row_sorted, gather, offs,
-                  offs_pitch, sched, sched_pitch, max_blocks, gates);
+  Picks<DT> r{};
+  if (busy) {
+    SortKey<DT> keys[EPL];
+    logits.take(keys, E, sub);
+    r = pick_columns<L, EPL, DT>(keys, k, sub);
+    if (slot) atomicOr(&members[r.col() * W + (row >> 5)], 1u << (row & 31));
+  }
+  sync_threads();
+  const int t = wave - 10;  // the last six waves: row t of the tables
+  if (t >= 0) {
+    const int sh = t == 0 ? 0 : t + 3;
+    int32_t *orow = offs + (int64_t)t * offs_pitch, *srow = sched + (int64_t)(t - 1) * sched_pitch;
+    int size[PER], v[PER], sum = 0;
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+      const int s = lane * PER + u;
+      size[u] = 0;
+      for (int w = 0; w < W; ++w) size[u] += __popc(members[(s < E ? s : 0) * W + w]);
+      size[u] = s < E ? size[u] : 0;
+      v[u] = (size[u] + ((1 << sh) - 1)) >> sh;
+      sum += v[u];
+    }
+    const int inc = wave_incl_scan(sum), total = __builtin_amdgcn_readlane(inc, kWave - 1);
+    int ex = inc - sum;
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+      const int s = lane * PER + u;
+      if (s < E) {
+        if (t == 0) {
+          place[s] = ex;
+          col_sum[s] = size[u];
+        }
+        orow[s] = ex;
+        if (t > 0)
+          for (int q = 0; q < v[u] && ex + q < max_blocks; ++q) srow[ex + q] = (q << 16) + s;
+      }
+      ex += v[u];
+    }
+    if (lane == 0) orow[E] = total;
+    if (t > 0)
+      for (int j = total + lane; j < max_blocks; j += kWave) srow[j] = -1;
+  }
+  uint32_t gate = 0;
+  int rank = 0;
+  if (busy) {
+    const float p = pick_softmax<L, DT>(r, sub < k);
+    gate = stored_bits<DT>(p);
+    if (slot) {
+      rank = rows_before(members, W, r.col(), row);
+      store_from_f32<DT>(y_vals, (int64_t)row * k + sub, p);
+      y_indx[(int64_t)row * k + sub] = (int16_t)r.col();
+    }
+    if (row < n_rows && sub < (E + 31) / 32) bits[row * bits_stride_row + (int64_t)sub * bits_stride_word] = r.word;
+  }
+  sync_threads();
+  if (busy && slot) {
+    const int i = row * k + sub, pos = place[r.col()] + rank;
+    row_sorted[i] = pos;
+    col_sorted[pos] = i;
+    if (gather) gather[pos] = row;
+    store_gate(gates, pos, gate);
+  }
 }
 
 template <int DT>
-int launch_routing_fused(const void *x, int64_t xs, int n_rows, int E, int k, void *yv, int16_t *yi, uint32_t *bits,
-                         int64_t bsr, int64_t bsw, int nbits, int NC, int P, size_t lds, int32_t *col_sum,
+int launch_routing_fused(const void *x, int64_t xs, int n_rows, int E, int k, int L, void *yv, int16_t *yi, uint32_t *bits,
+                         int64_t bsr, int64_t bsw, int W, size_t lds, int32_t *col_sum,
                          int32_t *col_sorted, int32_t *row_sorted, int32_t *gather, int32_t *offs, int64_t offs_pitch,
                          int32_t *sched, int64_t sched_pitch, int max_blocks, Gates gates, hipStream_t st) {
-  int need = (E + 7) / 8;
-  if (need < k) need = k;
 #define TAMD_RF(LL, EE)                                                                                              \
   do {                                                                                                               \
     auto kern = routing_fused_kernel<DT, LL, EE>;                                                                    \
     if (int rc = raise_lds_limit_once((const void *)kern)) return rc;                                                \
-    kern<<<1, 1024, lds, st>>>(x, xs, n_rows, E, k, yv, yi, bits, bsr, bsw, nbits, NC, P, col_sum, col_sorted,        \
+    kern<<<1, 1024, lds, st>>>(x, xs, n_rows, E, k, W, yv, yi, bits, bsr, bsw, col_sum, col_sorted, \
                                row_sorted, gather, offs, offs_pitch, sched, sched_pitch, max_blocks, gates);         \
   } while (0)
-  if (need <= 8) TAMD_RF(8, 8);
-  else if (need <= 16) TAMD_RF(16, 8);
-  else if (need <= 32) TAMD_RF(32, 8);
+  if (L == 8 && E <= 32) TAMD_RF(8, 4);
+  else if (L == 8) TAMD_RF(8, 8);
+  else if (L == 16) TAMD_RF(16, 8);
+  else if (L == 32) TAMD_RF(32, 8);
   else TAMD_RF(64, 8);
 #undef TAMD_RF
   return launch_status();
@@ -1086,8 +1412,6 @@ extern "C" int tamd_routing_gates(const void *logits, int dtype, int64_t stride,
                                   void *sorted_vals, int32_t *offs, int64_t offs_pitch, int32_t *schedule,
                                   int64_t sched_pitch, int max_n_blocks, int32_t *workspace, void *stream) {
   const Gates gates{y_vals, sorted_vals, sorted_vals ? dtype_size(dtype) : 0};
-  // a few rows (at most two passes of the workgroup's 1024 threads over them), at most 512 columns, and the
-  // metadata workspace of one workgroup fits LDS: one launch for everything
   if (n_rows > 0 && n_cols > 0 && n_cols <= 512 && k >= 1 && k <= 64 && k <= n_cols && logits && y_vals && y_indx && bits &&
       (dtype == TAMD_F32 || dtype == TAMD_BF16 || dtype == TAMD_F16) && col_sum && offs && col_sorted_indx &&
       row_sorted_indx && max_n_blocks >= 0 && offs_pitch >= n_cols + 1 && sched_pitch >= max_n_blocks &&
@@ -1096,64 +1420,34 @@ extern "C" int tamd_routing_gates(const void *logits, int dtype, int64_t stride,
     if (need < k) need = k;
     const int L = need <= 8 ? 8 : (need <= 16 ? 16 : (need <= 32 ? 32 : 64));
     const int64_t n = (int64_t)n_rows * k;
-    const int64_t NC = (n + 63) / 64;
-    int64_t P = 1024 / n_cols;
-    P = P < 1 ? 1 : (P > NC ? NC : P);
-    const int64_t ints = 2 * ((n + 3) / 4 * 4) + NC * n_cols + (int64_t)n_cols + P * n_cols + 6 * (int64_t)(n_cols + 1);
-    // two launches: top-k with the histogram of each workgroup's rows, then ordering and tables.  The rows of a workgroup
-    // (TH / L) must make whole chunks of 64 entries; the second launch orders 1024 / TH of the first one's blocks per workgroup.  It
-    // reduces the table with 16 loads per thread in flight, so TH grows where the table has more rows than one such batch
-    // (4096 rows of 128: 12.6 us with 512 threads, 13.8 with 256).  Beyond kMaxTableBlocks rows three small launches behind the
-    // top-k are faster up to 131072 entries (8192 rows of 256, top-8: 21.7 against 30), slower above (32768 of 64, top-6: 32 against 22).
-    int TH = 0;
-    const int CHO = 16 * k / L;
-    const int64_t batch = 16 * (1024 / n_cols > 16 ? 16 : (1024 / n_cols < 1 ? 1 : 1024 / n_cols));
-    if ((16 * k) % L == 0 && CHO >= 1 && CHO <= 16 && workspace)
-      for (int th = 256; th <= 1024 && !TH; th *= 2) {
-        const int64_t nb = ((int64_t)n_rows + th / L - 1) / (th / L);
-        const int64_t most = batch > kMaxTableBlocks && n <= 1024 * kMaxTableBlocks ? kMaxTableBlocks : batch;
-        if ((th / L * k) % 64 == 0 && (nb <= batch || th == 1024) &&
-            order_scan_applicable(n, n_cols, CHO, nb, th == 1024 && most < kMaxTableBlocks ? kMaxTableBlocks : most) &&
-            nb * n_cols <= tamd_bitmatrix_metadata_workspace(n, n_cols))
-          TH = th;
-      }
-    // One launch while a pass and a half of its threads (two where few columns are picked) hold the rows and the entries are few.
-    // The lines lie where it takes up to 1.2 times as long as two on the GPU, since two take longer to launch than they
-    // run (128 rows of 128, top-8: 17.6 us in one launch, 11.5 in two; top-4 11.8 and 10.4, called on its own 11.8 and
-    // 13.4; 256 rows of 16, top-8: 16.9 and 10.3).
-    const int pass = 1024 / L;
-    const bool one = !TH ? n_rows <= 2 * pass : (2 * n_rows <= 3 * pass || (n_rows <= 2 * pass && k <= (L == 8 ? 2 : 4))) && n <= (L == 8 ? 1280 : 640);
-    if (one && NC <= 64 && ints * 4 <= 156 * 1024) {
-      int nbits = 0;
-      while ((1 << nbits) < n_cols) ++nbits;
-      hipStream_t st = (hipStream_t)stream;
+    hipStream_t st = (hipStream_t)stream;
+    // One launch where 1024 threads hold the rows: also at the line it is the faster (64 rows of 128: 5.9 us against 7.5 in
+    // two launches, which take 2.8 us longer to launch; 128 of 32: 4.7 and 6.5).
+    if (n_rows <= 1024 / L) {
+      const int W = (n_rows + 31) / 32;
+      const size_t lds = (size_t)n_cols * (W + 1) * 4;
 #define TAMD_RFD(DT)                                                                                                  \
-  return launch_routing_fused<DT>(logits, stride, n_rows, n_cols, k, y_vals, y_indx, bits, bits_stride_row,            \
-                                  bits_stride_word, nbits, (int)NC, (int)P, (size_t)ints * 4, col_sum, col_sorted_indx,  \
-                                  row_sorted_indx, gather_indx, offs, offs_pitch, schedule, sched_pitch, max_n_blocks, gates, st)
+  return launch_routing_fused<DT>(logits, stride, n_rows, n_cols, k, L, y_vals, y_indx, bits, bits_stride_row,         \
+                                  bits_stride_word, W, lds, col_sum, col_sorted_indx, row_sorted_indx, gather_indx,    \
+                                  offs, offs_pitch, schedule, sched_pitch, max_n_blocks, gates, st)
       if (dtype == TAMD_F32) TAMD_RFD(TAMD_F32);
       if (dtype == TAMD_BF16) TAMD_RFD(TAMD_BF16);
       TAMD_RFD(TAMD_F16);
 #undef TAMD_RFD
     }
-    if (TH) {
-      const int64_t nb = ((int64_t)n_rows + TH / L - 1) / (TH / L);
-      int nbits = 0;
-      while ((1 << nbits) < n_cols) ++nbits;
-      hipStream_t st = (hipStream_t)stream;
+    RowPlan plan;
+    if (workspace && make_row_plan(n_rows, n_cols, k, L, tamd_bitmatrix_metadata_workspace(n, n_cols), plan)) {
+      uint32_t *table = (uint32_t *)workspace;
       int rc;
       if (dtype == TAMD_F32)
-        rc = launch_topk_hist<TAMD_F32>(logits, stride, n_rows, n_cols, k, y_vals, y_indx, bits, bits_stride_row,
-                                        bits_stride_word, nbits, L, TH, workspace, st);
+        rc = launch_topk_hist<TAMD_F32>(logits, stride, n_rows, n_cols, k, y_vals, y_indx, bits, bits_stride_row, bits_stride_word, L, plan, table, st);
       else if (dtype == TAMD_BF16)
-        rc = launch_topk_hist<TAMD_BF16>(logits, stride, n_rows, n_cols, k, y_vals, y_indx, bits, bits_stride_row,
-                                         bits_stride_word, nbits, L, TH, workspace, st);
+        rc = launch_topk_hist<TAMD_BF16>(logits, stride, n_rows, n_cols, k, y_vals, y_indx, bits, bits_stride_row, bits_stride_word, L, plan, table, st);
       else
-        rc = launch_topk_hist<TAMD_F16>(logits, stride, n_rows, n_cols, k, y_vals, y_indx, bits, bits_stride_row,
-                                        bits_stride_word, nbits, L, TH, workspace, st);
+        rc = launch_topk_hist<TAMD_F16>(logits, stride, n_rows, n_cols, k, y_vals, y_indx, bits, bits_stride_row, bits_stride_word, L, plan, table, st);
       if (rc != 0) return rc;
-      return launch_order_scan(y_indx, 1, n, n_cols, CHO, nbits, k, workspace, nb, col_sum, col_sorted_indx, row_sorted_indx,
-                               gather_indx, offs, offs_pitch, schedule, sched_pitch, max_n_blocks, gates, st, 1024 / TH);
+      return launch_order_rows(y_indx, n, n_cols, k, plan, table, col_sum, col_sorted_indx, row_sorted_indx, gather_indx, offs,
+                               offs_pitch, schedule, sched_pitch, max_n_blocks, gates, st);
     }
   }
   const int rc = tamd_topk_forward(logits, dtype, stride, n_rows, n_cols, k, 1, 0, y_vals, y_indx, k, bits, bits_stride_row,
