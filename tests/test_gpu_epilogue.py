@@ -6,7 +6,7 @@ import torch
 from oracle import matmul_ref as MR
 from oracle.mxfp_ref import downcast_to_mxfp_ref
 from triton_amd import _lib
-from triton_amd.matmul import (FlexCtx, FnSpecs, FusedActivation, InFlexData, OutFlexData, PrecisionConfig, matmul)
+from triton_amd.matmul import (Epilogue, FlexCtx, FnSpecs, FusedActivation, InFlexData, OutFlexData, PrecisionConfig, matmul)
 from triton_amd.matmul_details.opt_flags import scoped_opt_flags_constraints
 from triton_amd.numerics_details.mxfp import downcast_to_mxfp
 from triton_amd.swiglu import swiglu_fn
@@ -89,3 +89,91 @@ def test_output_types(M, N, pad, swiglu, flex, known, out_dtype, dtype, device, 
     named = torch.zeros(M, dtype=torch.bool)
     named[scatter[kept].long()] = True
     assert (bytes_[~named] == 0x35).all() and (bytes_[:, n_out * out_dtype.itemsize:] == 0x35).all()
+
+
+def _bytes_of(x):
+    return x.contiguous().view(torch.uint8)
+
+
+@pytest.mark.parametrize("block_m,M", [(32, 33), (128, 127)])
+@pytest.mark.parametrize("N,first,pad", [(64, 0, 0), (192, 0, 0), (200, 0, 4), (200, 4, 4), (200, 2, 0), (200, 0, 3), (196, 0, 0), (328, 0, 0)])
+@pytest.mark.parametrize("swiglu", [False, True])
+@pytest.mark.parametrize("saturate,factors", [(True, False), (False, False), (True, True), (None, True)])
+def test_fp8_output_bytes(block_m, M, N, first, pad, swiglu, saturate, factors, device):
+    """float8_e4m3fn outputs in whole quads of lanes on whole words and in others, infinite, NaN and overflowing ones among them: the bytes
+    that a cast of the float32 output of the same product gives."""
+    g = torch.Generator().manual_seed(3)
+    K, n_out = 128, N // 2 if swiglu else N
+    x = (torch.randn(M, K, generator=g) * 2).to(torch.float8_e4m3fn).to(device)
+    rv, rs = downcast_to_mxfp_ref(torch.randn(K, N, generator=g), torch.uint8, 0)
+    v, s = (t.to(device).t().contiguous().t() for t in (rv, rs))
+    bias = torch.randn(N, generator=g)
+    bias[6], bias[9], bias[14], bias[21] = float("inf"), -float("inf"), float("nan"), 3.0e4
+    kw = dict(gammas=(torch.rand(M, generator=g) + 0.5).to(device), betas=(torch.rand(M, generator=g) + 0.5).to(device)) if factors else {}
+    act = FusedActivation(FnSpecs("swiglu", swiglu_fn, ("alpha", "limit"), reduction_n=2), (1.702, 7.0 if factors else None)) if swiglu else None
+    expected, actual = torch.full((1,), 0.25, device=device), torch.zeros(1, device=device)
+
+    def run(dtype, **out):
+        fc = FlexCtx(lhs_data=InFlexData(x.dtype, torch.full((1,), 0.5, device=device)), **out)
+        flat = torch.zeros(first + M * (n_out + pad) + 16, dtype=dtype, device=device)
+        y = flat[first:first + M * (n_out + pad)].view(M, n_out + pad)[:, :n_out]
+        with scoped_opt_flags_constraints({"block_m": block_m}):
+            matmul(x, v, bias.to(device), c=y, fused_activation=act, precision_config=PrecisionConfig(
+                b_mx_scale=s, b_microblock_size=32, flex_ctx=fc, out_dtype=dtype, flexpoint_saturate_inf=bool(saturate)), **kw)
+        rest = torch.ones_like(flat, dtype=torch.bool)
+        rest[first:first + M * (n_out + pad)].view(M, n_out + pad)[:, :n_out] = False
+        assert (_bytes_of(flat[rest]) == 0).all()
+        return y
+    ref = run(torch.float32)
+    if saturate is None:
+        got = run(torch.float8_e4m3fn)
+    else:
+        got = run(torch.float8_e4m3fn, out_data=OutFlexData(torch.float8_e4m3fn, expected, actual if saturate else None))
+        if saturate:
+            assert float(actual) == float("inf") or torch.isclose(actual, ref.abs().amax() / 448.0 + 1e-30, rtol=1e-6).all()
+        ref = ref * 4.0
+        if saturate:
+            ref = torch.where(ref.isnan(), -448.0, ref.clamp(-448.0, 448.0))   # (a NaN takes the lower bound)
+    want = ref.to(torch.float8_e4m3fn)
+    over = ref.abs() >= 464.0   # rounds beyond the largest value
+    finite = ~(over | ref.isnan())
+    assert torch.equal(_bytes_of(got)[finite], _bytes_of(want)[finite])
+    assert (_bytes_of(got)[~finite] & 0x7F == 0x7F).all()
+    assert torch.equal(_bytes_of(got)[over] >> 7, (ref[over] < 0).to(torch.uint8))
+
+
+@pytest.mark.parametrize("block_m,M", [(32, 5), (128, 127)])
+@pytest.mark.parametrize("N", [64, 192, 256, 448])
+@pytest.mark.parametrize("swiglu", [False, True])
+def test_mxfp8_output_specials(block_m, M, N, swiglu, device):
+    """MXFP8 outputs whose groups hold zeros only, tiny and infinite values and NaNs: a NaN does not count for its group's scale and
+    stays one, an infinity makes the scale 255 and the other values zero."""
+    g = torch.Generator().manual_seed(4)
+    K, n_out = 128, N // 2 if swiglu else N
+    x = torch.randn(M, K, generator=g)
+    x[0] = 0.0
+    x[1] = 2.0 ** -6 * torch.sign(x[1])
+    x = x.to(torch.float8_e4m3fn).to(device)
+    xs = torch.full((M, K // 32), 127, dtype=torch.uint8)
+    xs[2], xs[3] = 7, 240
+    rv, rs = downcast_to_mxfp_ref(torch.randn(K, N, generator=g), torch.uint8, 0)
+    v, s = (t.to(device).t().contiguous().t() for t in (rv, rs))
+    bias = torch.zeros(N)
+    if n_out >= 96:
+        bias[70], bias[130 if swiglu else 40] = float("nan"), float("inf")
+    act = FusedActivation(FnSpecs("swiglu", swiglu_fn, ("alpha", "limit"), reduction_n=2), (1.702, None)) if swiglu else None
+    ys = torch.empty((M, n_out // 32), dtype=torch.uint8, device=device)
+    kw = dict(b_mx_scale=s, b_microblock_size=32, a_mx_scale=xs.to(device), a_microblock_size=32)
+    with scoped_opt_flags_constraints({"block_m": block_m}):
+        ref = matmul(x, v, bias.to(device), fused_activation=act, precision_config=PrecisionConfig(out_dtype=torch.float32, **kw)).cpu()
+        got = matmul(x, v, bias.to(device), fused_activation=act, precision_config=PrecisionConfig(c_mx_scale=ys, **kw),
+                     epilogue=Epilogue(FnSpecs("QUANTIZE_MXFP8", None, (), ()), (), (), 6.0)).cpu()
+    groups = ref.view(M, n_out // 32, 32)
+    top = groups.abs().nan_to_num(nan=0.0, posinf=float("inf")).amax(-1)
+    exponent = torch.ceil(torch.log2(top.double() / 448.0)).clamp(-126, 127)
+    byte = torch.where(top.isinf(), 255.0, torch.where(top == 0, 0.0, exponent + 127.0)).to(torch.int64)
+    assert torch.equal(ys.cpu().long(), byte)
+    scale = torch.where((byte == 0) | (byte == 255), 0.0, torch.exp2(127.0 - byte.double())).float()
+    want = (groups * scale[..., None]).view(M, n_out).to(torch.float8_e4m3fn)
+    nan = want.isnan()
+    assert torch.equal(got.isnan(), nan) and torch.equal(_bytes_of(got)[~nan], _bytes_of(want)[~nan])

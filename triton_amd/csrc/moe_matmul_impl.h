@@ -416,17 +416,25 @@ TAMD_DEVICE void store_actual_scale(float *actual, uint32_t amax, float out_max,
 struct NoPace {
   TAMD_DEVICE void operator()() const {}
 };
+// Two float32 in range (or NaN) -> e4m3fn bytes in the low or high half of `into`.
+template <bool HIGH>
+TAMD_DEVICE uint32_t e4m3_pair_bits(float lo, float hi, uint32_t into) {
+  return (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(lo, hi, (int)into, HIGH);
+}
 constexpr int epilogue_table_bytes(int nfr) { return nfr * 32 * 16; }
-// Maximum over a lane's aligned group of 32 / NO lanes: inside 16 lanes by moves in the register file (mirrored lanes
-// serve once the blocks of four and eight hold one value), across them through the LDS crossbar.
+// Maximum over a lane's aligned group of 32 / NO lanes, by moves in the register file (mirrored lanes serve once the blocks of four and
+// eight hold one value; for 32 the rows of 16 lanes change places).
 template <int NO>
-TAMD_DEVICE float group_max_lanes(float m) {
-  auto with = [&](uint32_t other) { m = __builtin_fmaxf(m, bits_to_f32(other)); };
-  with((uint32_t)__builtin_amdgcn_update_dpp(0, (int)f32_to_bits(m), 0xB1, 0xF, 0xF, true));    // quad_perm [1,0,3,2]
-  with((uint32_t)__builtin_amdgcn_update_dpp(0, (int)f32_to_bits(m), 0x4E, 0xF, 0xF, true));    // quad_perm [2,3,0,1]
-  with((uint32_t)__builtin_amdgcn_update_dpp(0, (int)f32_to_bits(m), 0x141, 0xF, 0xF, true));   // row_half_mirror
-  with((uint32_t)__builtin_amdgcn_update_dpp(0, (int)f32_to_bits(m), 0x140, 0xF, 0xF, true));   // row_mirror
-  if constexpr (NO == 1) with((uint32_t)__shfl_xor((int)f32_to_bits(m), 16));
+TAMD_DEVICE uint32_t group_max_lanes(uint32_t m) {
+  auto with = [&](uint32_t other) { m = other > m ? other : m; };
+  with((uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0xB1, 0xF, 0xF, true));    // quad_perm [1,0,3,2]
+  with((uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0x4E, 0xF, 0xF, true));    // quad_perm [2,3,0,1]
+  with((uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0x141, 0xF, 0xF, true));   // row_half_mirror
+  with((uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0x140, 0xF, 0xF, true));   // row_mirror
+  if constexpr (NO == 1) {
+    const auto r = __builtin_amdgcn_permlane16_swap(m, m, false, false);
+    m = r[0] > r[1] ? r[0] : r[1];
+  }
   return m;
 }
 
@@ -491,15 +499,42 @@ TAMD_DEVICE void epilogue_table(const Args &a, const Tile &t, const int *dsts, c
   }
 }
 
+// Four rows of a quad of lanes change places with its columns: lane q ends with what the four lanes hold of row q, in the order of the
+// lanes.  A register holds a byte of each row (one column per lane), or 16 bits of two rows each (two columns).
+TAMD_DEVICE uint32_t quad_xor1(uint32_t v) { return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, true); }
+TAMD_DEVICE uint32_t quad_xor2(uint32_t v) { return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xF, 0xF, true); }
+// (The selectors by arithmetic on a constant that the compiler does not see through: as selections between two constants it keeps both
+// in vector registers over the tiles of a persistent kernel.)
+TAMD_DEVICE uint32_t flip_where(uint32_t base, int bit_mask, uint32_t diff) {
+  asm("" : "+s"(diff));
+  return base ^ ((uint32_t)bit_mask & diff);
+}
+TAMD_DEVICE uint32_t quad_rows(uint32_t rows0123, int lane) {
+  const uint32_t x = __builtin_amdgcn_perm(quad_xor1(rows0123), rows0123, flip_where(0x06020400u, __builtin_amdgcn_sbfe(lane, 0, 1), 0x05050505u));
+  return __builtin_amdgcn_perm(quad_xor2(x), x, flip_where(0x05040100u, __builtin_amdgcn_sbfe(lane, 1, 1), 0x06060606u));
+}
+TAMD_DEVICE u32x2_t quad_rows(uint32_t rows01, uint32_t rows23, int lane) {
+  const uint32_t sel = flip_where(0x05040100u, __builtin_amdgcn_sbfe(lane, 0, 1), 0x06060606u);
+  const uint32_t a = __builtin_amdgcn_perm(quad_xor1(rows01), rows01, sel), b = __builtin_amdgcn_perm(quad_xor1(rows23), rows23, sel);
+  const bool up = (lane & 2) != 0;
+  const uint32_t r = quad_xor2(up ? a : b);
+  return up ? u32x2_t{r, b} : u32x2_t{a, r};
+}
+
 constexpr int kAny16 = 0x100, kAny8 = 0x101;
 template <int NFR, int ACT, int YDT, bool ROWSC, bool FLEX, bool MXO, typename Args, typename Pace>
 TAMD_DEVICE void tile_epilogue_t(const Args &a, const Tile &t, f32x16_t (&acc)[NFR][NF], uint8_t *tab, const EpilogueOperands<NFR> *ready,
                                  Pace &pace, bool pairs = true) {
-  const int wave = (threadIdx.x / kWave) & 3, lane = threadIdx.x % kWave;
+  constexpr bool BYTES = is_fp8(YDT);
+  const int wave = (threadIdx.x / kWave) & 3;
+  int lane = threadIdx.x % kWave;
+  float log2e = 1.4426950408889634f, inf = __builtin_inff();
+  uint32_t kDrop = 0x80000000u;                             // an offset that no descriptor here covers
+  // (nothing made of these is kept in registers over the tiles of a persistent kernel)
+  if constexpr (BYTES) asm volatile("" : "+v"(lane), "+s"(log2e), "+s"(inf), "+s"(kDrop));
   const int c32 = lane % 32, h = lane / 32;
   const int N = a.N;
   const int col0 = t.n0 + wave * 64 + c32 * NF;
-  constexpr uint32_t kDrop = 0x80000000u;                   // an offset that no descriptor here covers
   constexpr bool ANY = YDT == kAny16 || YDT == kAny8 || YDT == TAMD_F32;   // one width
   const int ydt = ANY ? a.y_dtype : YDT;
   constexpr int NO = ACT == TAMD_ACT_SWIGLU ? NF / 2 : NF;  // outputs per lane per row
@@ -540,15 +575,26 @@ TAMD_DEVICE void tile_epilogue_t(const Args &a, const Tile &t, f32x16_t (&acc)[N
                                                                      0x7FFFFFFF, 0x00020000);
   const uint32_t col_off = (uint32_t)out_col0 * (uint32_t)osz, col_kill = out_col0 < n_out ? 0u : kDrop;
   const uint32_t col_kill1 = out_col0 + 1 < n_out ? 0u : kDrop;   // (the second output of a pair that N cuts)
+  // Bytes: whole quads of lanes inside the output, whole words: one store of four or eight bytes per lane and four rows.  (Of 16 bits the
+  // stores are not what a tile waits for: 8 and 16 bytes per lane took 1 to 3 % longer for the exchange between the lanes.)
+  const bool quads = BYTES && n_out % (4 * NO) == 0 &&
+                     (((uint32_t)(uintptr_t)a.y | (uint32_t)a.y_stride_m | (uint32_t)a.y_stride_z) & 3u) == 0;
+  const bool factors = ROWSC && (a.betas || a.gammas);
+  const float act_scale = ACT == TAMD_ACT_SWIGLU ? -a.act_alpha * log2e : 0.f, limit = ACT == TAMD_ACT_SWIGLU ? a.act_limit : 0.f;
+  const float limit_lo = __builtin_fminf(-limit, limit);
   const __amdgpu_buffer_rsrc_t rsc = __builtin_amdgcn_make_buffer_rsrc(
       MXO ? a.y_mx_scale + (int64_t)t.z * a.y_mx_stride_z : nullptr, 0, MXO ? 0x7FFFFFFF : 0, 0x00020000);
   // the scales of four rows go out together: in a group's lanes, lane jj takes row jj's
   const uint32_t sc_off = ((c32 & (32 / NO - 1)) < 4 && (out_col0 & ~31) < n_out) ? (uint32_t)(out_col0 / 32) : kDrop;
   // four rows of the table at a time, read one step ahead; the scheduling barrier keeps the compiler from reading the
   // whole table up front (registers)
-  uint4 next_dst = *(const uint4 *)(tab_dst + h * 4);
+  // (of bytes a lane stores one row in four: only that row's destination is read)
+  constexpr bool DST_AHEAD = !BYTES;
+  uint4 next_dst = DST_AHEAD ? *(const uint4 *)(tab_dst + h * 4) : uint4{0u, 0u, 0u, 0u};
+  // (the factors of a SwiGLU tile, which a layer has none of, are read where they are used: registers)
+  constexpr bool FACTORS_AHEAD = ROWSC && (!BYTES || ACT != TAMD_ACT_SWIGLU);
   f32x4_t next_beta = f32x4_t{1.f, 1.f, 1.f, 1.f}, next_gamma = next_beta;
-  if constexpr (ROWSC) {
+  if constexpr (FACTORS_AHEAD) {
     next_beta = *(const f32x4_t *)(tab_beta + h * 4);
     next_gamma = *(const f32x4_t *)(tab_gamma + h * 4);
   }
@@ -560,8 +606,8 @@ TAMD_DEVICE void tile_epilogue_t(const Args &a, const Tile &t, f32x16_t (&acc)[N
       const f32x4_t beta4 = next_beta, gamma4 = next_gamma;
       if (ANY || i * 4 + jq + 1 < NFR * 4) {   // (one row past the last: still the table)
         const int r1 = (i * 4 + jq + 1) * 8 + h * 4;
-        next_dst = *(const uint4 *)(tab_dst + r1);
-        if constexpr (ROWSC) {
+        if constexpr (DST_AHEAD) next_dst = *(const uint4 *)(tab_dst + r1);
+        if constexpr (FACTORS_AHEAD) {
           next_beta = *(const f32x4_t *)(tab_beta + r1);
           next_gamma = *(const f32x4_t *)(tab_gamma + r1);
         }
@@ -582,65 +628,164 @@ TAMD_DEVICE void tile_epilogue_t(const Args &a, const Tile &t, f32x16_t (&acc)[N
           for (int p = 0; p < NO; ++p) o[p] *= gamma4[jj];
         }
       };
+      const int r0 = (i * 4 + jq) * 8 + h * 4;
+      const uint32_t own = DST_AHEAD ? 0u : tab_dst[r0 + (lane & 3)];
       float out4[4][NO];
-      if constexpr (MXO) {
-        // MXFP8 output: a group is 32 consecutive output columns of a row = the outputs of one half wave (of
-        // half of it when a lane holds two columns).  max |o| over the group, scale = 2^ceil(log2(max / 448)),
-        // o / scale clamped to +-448; the cast below rounds to nearest even (as tamd_downcast_mxfp does).  Four rows at a
-        // time, so that their maxima overlap (67218 rows x 736 -> 544 outputs: 213 us row by row with shuffles through
-        // LDS and two divisions each, 165 now).
-        float m4[4];
+      if constexpr (!BYTES) {
 #pragma unroll
         for (int jj = 0; jj < 4; ++jj) {
-          result(jj, out4[jj]);
-          m4[jj] = 0.f;
+          float (&o)[NO] = out4[jj];
+          result(jj, o);
+          if constexpr (!ANY) {
+            const int off = (int)((dst4[jj] + col_off) | col_kill);
+            if constexpr (NO == 2) __builtin_amdgcn_raw_buffer_store_b32(narrow2(o[0], o[NO - 1]), ry, off, 0, 0);
+            else __builtin_amdgcn_raw_buffer_store_b16((uint16_t)narrow(o[0]), ry, off, 0, 0);
+          }
+        }
+      } else {
+        // Four rows at once, and what is the same for the launch decided by a branch for all of them (the empty asm keeps it one): the
+        // epilogue of a tile of 128 x 256 with SwiGLU is a third of a short tile's time, bound by its instructions -- 270 per four rows
+        // with MXFP8 output when everything was selected per value, each row's scale made by every lane and every byte stored by
+        // itself, 130 now.  1028 MXFP8 tokens x 6 of 32 slices, 1248 -> 2688: 60.2 -> 51.4 us (the epilogue 12.4 -> 8.4 of a tile's 30);
+        // 5670 x 4 of 64, 2144 -> 1472, strided, 135 -> 123; fp8, 16384 x 4 of 32, 2880 -> 5760: 961 -> 942.
+        float v[4][NF];
+        if (ROWSC && factors) {
+          const f32x4_t beta = FACTORS_AHEAD ? beta4 : *(const f32x4_t *)(tab_beta + r0);
 #pragma unroll
-          for (int p = 0; p < NO; ++p) m4[jj] = __builtin_fmaxf(m4[jj], out_col0 + p < n_out ? __builtin_fabsf(out4[jj][p]) : 0.f);
+          for (int jj = 0; jj < 4; ++jj)
+#pragma unroll
+            for (int f = 0; f < NF; ++f) v[jj][f] = __builtin_fmaf(acc[i][f][jq * 4 + jj], flex, bias_a[f] * beta[jj]);
+        } else {
+#pragma unroll
+          for (int jj = 0; jj < 4; ++jj)
+#pragma unroll
+            for (int f = 0; f < NF; ++f) v[jj][f] = __builtin_fmaf(acc[i][f][jq * 4 + jj], flex, bias_a[f]);
+        }
+        if constexpr (ACT == TAMD_ACT_SWIGLU) {   // swiglu_fast, a step for four rows at a time
+          if (has_limit) {
+            asm volatile("");
+#pragma unroll
+            for (int jj = 0; jj < 4; ++jj) {
+              v[jj][0] = __builtin_fminf(v[jj][0], limit);
+              v[jj][1] = __builtin_amdgcn_fmed3f(v[jj][1], limit_lo, limit);   // (a NaN gives the lower bound, as the maximum does)
+            }
+          }
+#pragma unroll
+          for (int jj = 0; jj < 4; ++jj) {
+            const float e = __builtin_amdgcn_exp2f(act_scale * v[jj][0]);
+            const float g = v[jj][0] * __builtin_amdgcn_rcpf(1.0f + e);
+            out4[jj][0] = __builtin_fmaf(g, v[jj][1], g);
+          }
+        } else {
+#pragma unroll
+          for (int jj = 0; jj < 4; ++jj)
+#pragma unroll
+            for (int p = 0; p < NO; ++p) out4[jj][p] = v[jj][p];
+        }
+        if (ROWSC && factors) {
+          asm volatile("");
+          const f32x4_t gamma = FACTORS_AHEAD ? gamma4 : *(const f32x4_t *)(tab_gamma + r0);
+#pragma unroll
+          for (int jj = 0; jj < 4; ++jj)
+#pragma unroll
+            for (int p = 0; p < NO; ++p) out4[jj][p] *= gamma[jj];
+        }
+      }
+      if constexpr (MXO) {
+        // MXFP8 output: a group is 32 consecutive output columns of a row = the outputs of one half wave (of
+        // half of it when a lane holds two columns).  max |o| over the group, scale = 2^ceil(log2(max / 448)), o / scale
+        // (within +-448 by the choice of the scale); the cast below rounds to nearest even (as tamd_downcast_mxfp does).  The maxima
+        // of non-negative numbers are those of their bits (a NaN counts as 0); lane jj of every quad makes row jj's scale and
+        // hands it to the others.
+        const float cap = out_col0 < n_out ? inf : 0.f, cap1 = out_col0 + 1 < n_out ? inf : 0.f;
+        uint32_t m4[4];
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj) {
+          m4[jj] = f32_to_bits(__builtin_amdgcn_fmed3f(__builtin_fabsf(out4[jj][0]), 0.f, cap));
+          if constexpr (NO == 2) {
+            const uint32_t m1 = f32_to_bits(__builtin_amdgcn_fmed3f(__builtin_fabsf(out4[jj][NO - 1]), 0.f, cap1));
+            m4[jj] = m1 > m4[jj] ? m1 : m4[jj];
+          }
         }
 #pragma unroll
         for (int jj = 0; jj < 4; ++jj) m4[jj] = group_max_lanes<NO>(m4[jj]);
-        uint32_t my_scale = 0;
+        const uint32_t mine = (c32 & 2) ? ((c32 & 1) ? m4[3] : m4[2]) : ((c32 & 1) ? m4[1] : m4[0]);
+        const uint32_t se = ceil_scale_byte<TAMD_FP8_E4M3>(bits_to_f32(mine));
+        const uint32_t qs = se == 0u || se == 255u ? 0u : (254u - se) << 23;   // 1 / 2^(se - 127)
+        const float qs4[4] = {bits_to_f32((uint32_t)__builtin_amdgcn_update_dpp(0, (int)qs, 0x00, 0xF, 0xF, true)),
+                              bits_to_f32((uint32_t)__builtin_amdgcn_update_dpp(0, (int)qs, 0x55, 0xF, 0xF, true)),
+                              bits_to_f32((uint32_t)__builtin_amdgcn_update_dpp(0, (int)qs, 0xAA, 0xF, 0xF, true)),
+                              bits_to_f32((uint32_t)__builtin_amdgcn_update_dpp(0, (int)qs, 0xFF, 0xF, 0xF, true))};
 #pragma unroll
-        for (int jj = 0; jj < 4; ++jj) {
-          const uint32_t se = ceil_scale_byte<TAMD_FP8_E4M3>(m4[jj]);
-          const float qs = bits_to_f32(se == 0u || se == 255u ? 0u : (254u - se) << 23);   // 1 / 2^(se - 127)
+        for (int jj = 0; jj < 4; ++jj)
 #pragma unroll
-          for (int p = 0; p < NO; ++p) {
-            const float q = out4[jj][p] * qs;
-            out4[jj][p] = q != q ? q : __builtin_fminf(__builtin_fmaxf(q, -448.0f), 448.0f);
-          }
-          my_scale = (c32 & 3) == jj ? se : my_scale;
-        }
+          for (int p = 0; p < NO; ++p) out4[jj][p] *= qs4[jj];
         const uint32_t sdst = tab_dst[NFR * 96 + (i * 4 + jq) * 8 + h * 4 + (c32 & 3)];
-        __builtin_amdgcn_raw_buffer_store_b8((uint8_t)my_scale, rsc, (int)(((sdst | sc_off) & kDrop) ? kDrop : sdst + sc_off), 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b8((uint8_t)se, rsc, (int)(((sdst | sc_off) & kDrop) | (sdst + sc_off)), 0, 0);
       }
+      if constexpr (FLEX) {
+        if (ANY || track_max) {
+          const uint4 d = DST_AHEAD ? uint4{dst4[0], dst4[1], dst4[2], dst4[3]} : *(const uint4 *)(tab_dst + r0);
+          const uint32_t rows[4] = {d.x, d.y, d.z, d.w};
 #pragma unroll
-      for (int jj = 0; jj < 4; ++jj) {
-        float (&o)[NO] = out4[jj];
-        if constexpr (!MXO) result(jj, o);
-        const uint32_t dst = dst4[jj];
-        if constexpr (FLEX) {
-          // (selections, no branches: a branch per element breaks the fragment into hundreds of blocks)
+          for (int jj = 0; jj < 4; ++jj)
 #pragma unroll
-          for (int p = 0; p < NO; ++p) {
-            const uint32_t amask = (dst | (ANY && p == 1 ? col_kill1 : col_kill)) & kDrop ? 0u : track_mask;
-            const uint32_t b = f32_to_bits(o[p]) & amask;
-            amax = b > amax ? b : amax;
-            o[p] *= inv_expected;
-            const float oc = __builtin_fminf(__builtin_fmaxf(o[p], -out_max), out_max);
-            o[p] = clamp_out ? oc : o[p];
+            for (int p = 0; p < NO; ++p) {
+              const uint32_t amask = (rows[jj] | (ANY && p == 1 ? col_kill1 : col_kill)) & kDrop ? 0u : track_mask;
+              const uint32_t b = f32_to_bits(out4[jj][p]) & amask;
+              amax = b > amax ? b : amax;
+            }
+        }
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj)
+#pragma unroll
+          for (int p = 0; p < NO; ++p) out4[jj][p] *= inv_expected;
+        if (clamp_out) {
+          asm volatile("");
+#pragma unroll
+          for (int jj = 0; jj < 4; ++jj)
+#pragma unroll
+            for (int p = 0; p < NO; ++p) out4[jj][p] = __builtin_amdgcn_fmed3f(out4[jj][p], -out_max, out_max);
+        }
+      }
+      if constexpr (BYTES) {
+        // the bytes of a column's four rows (of two columns' rows two by two)
+        uint32_t w[NO];
+        bool in_range = clamp_out;   // then the conversion alone
+        if constexpr (MXO) {         // unless one is a NaN, whose sign it would lose
+          bool nan = false;
+#pragma unroll
+          for (int jj = 0; jj < 4; ++jj) nan |= __builtin_isunordered(out4[jj][0], out4[jj][NO - 1]);
+          in_range = __ballot(nan) == 0;
+        }
+        if (in_range) {
+          if constexpr (NO == 1) w[0] = e4m3_pair_bits<true>(out4[2][0], out4[3][0], e4m3_pair_bits<false>(out4[0][0], out4[1][0], 0u));
+          else {
+            w[0] = e4m3_pair_bits<true>(out4[1][0], out4[1][NO - 1], e4m3_pair_bits<false>(out4[0][0], out4[0][NO - 1], 0u));
+            w[NO - 1] = e4m3_pair_bits<true>(out4[3][0], out4[3][NO - 1], e4m3_pair_bits<false>(out4[2][0], out4[2][NO - 1], 0u));
+          }
+        } else {
+          asm volatile("");
+          if constexpr (NO == 1) w[0] = narrow(out4[0][0]) | narrow(out4[1][0]) << 8 | narrow(out4[2][0]) << 16 | narrow(out4[3][0]) << 24;
+          else {
+            w[0] = narrow(out4[0][0]) | narrow(out4[0][NO - 1]) << 8 | narrow(out4[1][0]) << 16 | narrow(out4[1][NO - 1]) << 24;
+            w[NO - 1] = narrow(out4[2][0]) | narrow(out4[2][NO - 1]) << 8 | narrow(out4[3][0]) << 16 | narrow(out4[3][NO - 1]) << 24;
           }
         }
-        const int off = (int)((dst + col_off) | col_kill);
-        if constexpr (ANY) {
-          // stored below, four rows at a time
-        } else if constexpr (osz == 2) {
-          if constexpr (NO == 2) __builtin_amdgcn_raw_buffer_store_b32(narrow2(o[0], o[NO - 1]), ry, off, 0, 0);
-          else __builtin_amdgcn_raw_buffer_store_b16((uint16_t)narrow(o[0]), ry, off, 0, 0);
+        if (quads) {
+          const int off = (int)((own + col_off - (uint32_t)((lane & 3) * NO)) | col_kill);
+          if constexpr (NO == 1) __builtin_amdgcn_raw_buffer_store_b32(quad_rows(w[0], lane), ry, off, 0, 0);
+          else __builtin_amdgcn_raw_buffer_store_b64(quad_rows(w[0], w[NO - 1], lane), ry, off, 0, 0);
         } else {
-          if constexpr (NO == 2)
-            __builtin_amdgcn_raw_buffer_store_b16((uint16_t)(narrow(o[0]) | (narrow(o[NO - 1]) << 8)), ry, off, 0, 0);
-          else __builtin_amdgcn_raw_buffer_store_b8((uint8_t)narrow(o[0]), ry, off, 0, 0);
+          asm volatile("");
+          const uint4 d = *(const uint4 *)(tab_dst + r0);
+          const uint32_t rows[4] = {d.x, d.y, d.z, d.w};
+#pragma unroll
+          for (int jj = 0; jj < 4; ++jj) {
+            const int off = (int)((rows[jj] + col_off) | col_kill);
+            if constexpr (NO == 1) __builtin_amdgcn_raw_buffer_store_b8((uint8_t)(w[0] >> 8 * jj), ry, off, 0, 0);
+            else __builtin_amdgcn_raw_buffer_store_b16((uint16_t)(w[(jj >> 1) * (NO - 1)] >> 16 * (jj & 1)), ry, off, 0, 0);
+          }
         }
       }
       if constexpr (ANY) {
