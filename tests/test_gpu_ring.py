@@ -52,14 +52,25 @@ def test_where_it_is_taken():
         assert ring_rows(512, 5760, 2880, 128, "fp8", **changed) == 0, changed
 
 
+def test_where_blocks_of_96_come_before_tiles():
+    """SwiGLU products with about a hundred to a thousand rows per slice, by their rounds over the CUs; not without SwiGLU, few tiles or 16-bit rows."""
+    for m, n, k, e, kind, out in ((6168, 2688, 1248, 32, "mxfp8", "mx"), (6432, 1152, 2048, 60, "fp8", "fp8"), (14760, 2240, 5312, 16, "mxfp4", "16")):
+        assert ring_rows(m, n, k, e, kind, out, True) == 96
+        assert ring_rows(m, n, k, e, kind) == 0
+        assert ring_rows(m, n, k, e, kind, out, True, w_layout=_lib.W_STRIDED, w_mx_layout=_lib.SCALE_STRIDED) == 0
+        assert ring_rows(m, n, k, e, kind, out, True, force_variant=128) == 0
+    assert ring_rows(65536, 5760, 2880, 32, "fp8", "fp8", True) == 0 and ring_rows(2000, 1024, 2880, 16, "mxfp8", "mx", True) == 0
+    assert ring_rows(6168, 2688, 1248, 32, "bf16", "16", True) == 0 and ring_rows(6168, 2688, 640, 32, "mxfp8", "mx", True) == 0
+
+
 def blocks(w, ws):
     return convert_layout(wrap_torch_tensor(w, dtype=FP4), CDNA4MXValueLayout()), convert_layout(wrap_torch_tensor(ws), CDNA4MXScaleLayout())
 
 
 # (rows per slice, slices, K, columns): blocks of 32 alone on their CUs (K of one stage and less, of fewer stages than the ring, off the
-# stages), in several rounds; of 64; of 96
+# stages), in several rounds; of 64; of 96, also several of them to a slice
 SIZES = [(9, 10, 96, 2832), (4, 12, 352, 1872), (14, 16, 736, 1296), (20, 16, 1440, 1392), (5, 128, 1056, 1184), (11, 64, 2144, 2320),
-         (40, 16, 608, 2608), (30, 60, 1248, 2320), (72, 32, 1056, 4368), (14, 16, 800, 1296), (4, 12, 992, 1872)]
+         (40, 16, 608, 2608), (30, 60, 1248, 2320), (72, 32, 1056, 4368), (14, 16, 800, 1296), (4, 12, 992, 1872), (190, 30, 1056, 2384), (420, 8, 1312, 4368)]
 
 
 @pytest.mark.parametrize("layout", [dict(), dict(w_layout=_lib.W_STRIDED, w_mx_layout=_lib.SCALE_STRIDED, w_stride_k=1, w_stride_n=1440, w_mx_stride_k=1,

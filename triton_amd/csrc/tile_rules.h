@@ -118,6 +118,22 @@ inline bool ring_stages_too_few(const tamd_matmul_args &a, double cover) {
   return a.K > 256 && a.K <= (scaled ? 768 : 512) && (scaled || a.w_layout != TAMD_W_CDNA4_BLOCKS || cover > 32.0);
 }
 
+// SwiGLU products of 8- and 4-bit rows with more than 64 rows per slice: the persistent kernel's blocks of 96 against tiles of 128, by what each
+// is estimated to take (us): a start, and rounds over the CUs (two tiles of 128 to a CU) whose last is paid for in part.  The epilogue of
+// such a tile is a third of its time, which the persistent kernel hides behind the next tile's products; without SwiGLU, and from
+// about a thousand rows per slice on, tiles are the faster.  Fitted to 2300 products (8 to 128 slices of 24 to 2000 rows, K 512 to 5760); where
+// the rule takes this kernel, time over the tiles': fp8 0.957, MXFP8 0.931, packed rows 0.921, 20 of 550 above 1.05.
+inline bool ring_96_before_tiles(const tamd_matmul_args &a, int cus, double mean) {
+  if (a.activation != TAMD_ACT_SWIGLU || a.K < 800 || mean < 60.0 || mean > 1024.0) return false;
+  const bool packed = a.x_dtype == TAMD_MXFP4, scaled = !packed && a.x_mx_scale;
+  const double cols = live_slices(a) * ((a.N + 255) / 256) / cus, k = a.K / 1000.0;
+  const double r = cols * fmax(1.0, mean / 96.0 + 0.5), m = cols * 0.5 * fmax(1.0, mean / 128.0 + 0.5);
+  if (m < 0.75) return false;
+  const double ring = 5.0 + (packed ? 3.2 + 3.5 * k : scaled ? 4.2 + 4.8 * k : 3.2 + 4.4 * k) * (r + 0.6 * (ceil(r) - r) + 0.1);
+  const double tiles = 5.0 + (packed ? 5.9 + 11.1 * k : scaled ? 9.7 + 13.9 * k : 7.9 + 11.6 * k) * (m + 0.05 * (ceil(m) - m) + 0.07);
+  return ring < (scaled ? 1.0 : 0.97) * tiles;
+}
+
 // Rows of the persistent kernel's blocks, 0 where another kernel is the faster (or the only one).  The block is the smallest that covers a
 // slice's mean size and two standard deviations, up to 96; the lines between the kernels are in tiles per CU, one row block for every slice
 // that has rows (on the average of random choices).  Up to one, a tile is alone on its CU and wins by its depth; just above, the second
@@ -140,6 +156,10 @@ inline int ring_rows(const tamd_matmul_args &a, int cus) {
   if ((x8 || a.x_dtype == TAMD_MXFP4) && a.block_m <= 32 && a.K > 1280 && cover <= 32.0 && tiles <= (x8 && a.K > 2048 ? 0.375 : 0.25)) return 0;
   if (tiles <= 1.0 && ring_stages_too_few(a, cover)) return 0;
   if (a.w_layout != TAMD_W_CDNA4_BLOCKS) return ring_rows_strided(a, cover, tiles);
+  const bool packed = a.x_dtype == TAMD_MXFP4, scaled = !packed && a.x_mx_scale;
+  // (of blocks of 96 rows what the products of a layer write is built)
+  const bool rows_96 = !x16 && cover > 64.0 && (a.y_dtype != TAMD_FP8_E4M3 || (a.activation == TAMD_ACT_SWIGLU && !(packed && a.y_mx_scale)));
+  if (rows_96 && ring_96_before_tiles(a, cus, mean)) return 96;
   if (mean > 96.0 || (a.K < 1024 && tiles > 1.0)) return 0;
   const bool alone = tiles <= 1.0;
   if (x16) {
@@ -151,7 +171,6 @@ inline int ring_rows(const tamd_matmul_args &a, int cus) {
     if (mean < 50.0) return alone && tiles > 0.75 ? 64 : 0;
     return mean <= 80.0 && tiles > 1.1 && tiles < 8.0 ? 64 : 0;
   }
-  const bool packed = a.x_dtype == TAMD_MXFP4, scaled = !packed && a.x_mx_scale;
   if (cover <= 32.0) {
     if (scaled) return alone || tiles > 2.0 ? 32 : 0;
     if (packed) return alone || tiles > 1.4 ? 32 : 0;
@@ -162,10 +181,7 @@ inline int ring_rows(const tamd_matmul_args &a, int cus) {
     return (alone && tiles > (mean < 10.0 ? 0.27 : 0.1)) || tiles > 2.0 ? 32 : 0;
   }
   if (cover <= 64.0) return tiles > 2.0 || (alone && !scaled && tiles > (packed ? 0.0 : 0.6)) ? 64 : 0;
-  // (of blocks of 96 rows what the products of a layer write is built)
-  const bool swiglu = a.activation == TAMD_ACT_SWIGLU;
-  if (a.y_dtype == TAMD_FP8_E4M3 && (!swiglu || (packed && a.y_mx_scale))) return 0;
-  return tiles > (packed ? 1.4 : 2.0) ? 96 : 0;
+  return rows_96 && tiles > (packed ? 1.4 : 2.0) ? 96 : 0;
 }
 
 // What the persistent kernel for unquantised 16-bit weights (moe_matmul_kkring.h) covers, of the products that the tiled kernel of two
