@@ -68,6 +68,36 @@ def test_upcast_matches_oracle(shape, axis, dtype, device):
     assert torch.equal(torch.nan_to_num(a), torch.nan_to_num(b))
 
 
+@pytest.mark.parametrize("shape", [(8, 288, 1032), (8, 544, 1024), (2, 1056, 2056), (1, 2048, 3208), (5, 32, 4104), (3, 800, 1544)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("pitch", [0, 8])
+def test_tiles_of_eight_groups(shape, dtype, pitch, device):
+    """A strided quantised axis in tiles (more than 96 and 40 of them on 256 CUs), cut in groups and columns, rows that start on a line of 128
+    bytes and rows that do not, also in a wider tensor; back through plain and non-temporal stores."""
+    b, K, N = shape
+    g = torch.Generator().manual_seed(K + N)
+    # (six deviations of either: 6 * exp(9) = 48600, which float16 holds; infinities are not quantised)
+    x = (torch.randn((b, K, N), generator=g) * torch.exp(1.5 * torch.randn((b, K // 32, N), generator=g)).repeat_interleave(32, 1)).to(dtype)
+    assert x.isfinite().all()
+    wide = torch.zeros((b, K, N + pitch), dtype=dtype, device=device)
+    wide[..., :N] = x.to(device)
+    v, s = downcast_to_mxfp(wide[..., :N], torch.uint8, axis=1)
+    rv, rs = downcast_to_mxfp_ref(x, torch.uint8, 1)
+    assert torch.equal(v.cpu(), rv) and torch.equal(s.cpu(), rs)
+    back = upcast_from_mxfp(v, s, dtype, axis=1)
+    assert torch.equal(back.cpu(), upcast_from_mxfp_ref(rv, rs, dtype, 1))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_tiles_of_more_groups(dtype, device):
+    """1040 tiles of 32 groups or 1560 of 16, the last of each matrix one group deep: from four rounds of 256 CUs on they replace those of 8."""
+    x = torch.randn((520, 1056, 64), generator=torch.Generator().manual_seed(3)).to(dtype)
+    v, s = downcast_to_mxfp(x.to(device), torch.uint8, axis=1)
+    rv, rs = downcast_to_mxfp_ref(x, torch.uint8, 1)
+    assert torch.equal(v.cpu(), rv) and torch.equal(s.cpu(), rs)
+    assert torch.equal(upcast_from_mxfp(v, s, dtype, axis=1).cpu(), upcast_from_mxfp_ref(rv, rs, dtype, 1))
+
+
 def test_all_e2m1_values_roundtrip(device):
     """Every e2m1 value times 2^p, p in [-8, 8), survives quantise -> dequantise (tests/test_mxfp.py:171-205)."""
     grid = torch.tensor([0, 0.5, 1, 1.5, 2, 3, 4, 6])

@@ -1,7 +1,7 @@
 // MXFP4 / MXFP8 quantise / dequantise for gfx950.  Bandwidth kernels: 128-bit global
 // accesses, one 32-element group handled by 4 lanes (quantised axis contiguous)
 // or by one lane per column set (quantised axis strided, i.e. the weight layout: tiles
-// of 16 or 32 groups x 128 or 256 columns that pass through LDS).
+// of 8, 16 or 32 groups x 128 or 256 columns that pass through LDS).
 //
 // Arithmetic follows numerics_details/mxfp.py:212-363 and :384-449 of the
 // reference: scale = 2^ceil(log2(max/6)) taken from the float32 bit pattern,
@@ -302,24 +302,20 @@ __global__ __launch_bounds__(256) void downcast_cols_kernel(
 // downcast, source contiguous along r, 16-byte aligned: a workgroup quantises a tile of GT groups x 32*NV
 // columns.  A load instruction of a wave reads 512 contiguous bytes of two source rows (a thread keeps the 32
 // rows of its NV columns in registers, as above); the codes pass through LDS so that they leave as GT x 16
-// contiguous bytes per column.  The source is read once: its loads are non-temporal.
+// contiguous bytes per column.  ONCE: the source's loads are non-temporal, since each is read once (a line too).
 // ---------------------------------------------------------------------------
-// groups per tile: 64 KiB of codes in LDS either way
-template <int DT>
-constexpr int kTileGroups = DT == TAMD_F32 ? 32 : 16;
 template <int DT>
 constexpr int kTileCols = 32 * (DT == TAMD_F32 ? 4 : 8);
-template <int DT>
-constexpr size_t kTileLds = (size_t)kTileCols<DT> * kTileGroups<DT> * 17;
+template <int DT, int GT>
+constexpr size_t kTileLds = (size_t)kTileCols<DT> * GT * 17;
 
-template <int DT>
+template <int DT, int GT, bool ONCE>
 __global__ __launch_bounds__(256) void downcast_cols_tile_kernel(
     const void *__restrict__ src, int64_t nb, int64_t G, int64_t nr, int64_t ssb, int64_t ssl,
     uint8_t *__restrict__ vals, int64_t vsb, int64_t vsr, uint8_t *__restrict__ scales, int64_t csb,
     int64_t csr, int mode) {
   constexpr int ES = DT == TAMD_F32 ? 4 : 2;
   constexpr int NV = 16 / ES;
-  constexpr int GT = kTileGroups<DT>;
   constexpr int CW = kTileCols<DT>;
   // s_codes[column][slot]: slot = group ^ (column / NV) % 8 keeps both the writes (two groups, 32 column sets
   // per wave) and the reads (GT groups of 256 / GT columns per workgroup) spread over the banks
@@ -344,7 +340,7 @@ __global__ __launch_bounds__(256) void downcast_cols_tile_kernel(
     const char *base = (const char *)src + (b * ssb + g * 32 * ssl + col0) * ES;
     uint4 raw[32];
 #pragma unroll
-    for (int l = 0; l < 32; ++l) raw[l] = load_once(base + (int64_t)l * ssl * ES);
+    for (int l = 0; l < 32; ++l) raw[l] = ONCE ? load_once(base + (int64_t)l * ssl * ES) : load16((const uint8_t *)base + (int64_t)l * ssl * ES);
     auto elem = [&](int l, int c) -> float {
       const uint4 &q = raw[l];
       uint32_t w[4] = {q.x, q.y, q.z, q.w};
@@ -547,27 +543,31 @@ TAMD_DEVICE void upcast_rows2_regs(const uint32_t *w, const float *mult, uint4 &
     r1 = make_uint4(hi[0], hi[1], hi[2], hi[3]);
   }
 }
-template <int DT, int BS>
+template <int DT, int BS, bool ONCE = true>
 TAMD_DEVICE void upcast_rows2(const uint32_t *w, const float *mult, char *p, int64_t pitch) {
   uint4 r0, r1;
   upcast_rows2_regs<DT, BS>(w, mult, r0, r1);
-  store_once(p, r0);
-  store_once(p + pitch, r1);
+  if (ONCE) {
+    store_once(p, r0);
+    store_once(p + pitch, r1);
+  } else {
+    store16((uint8_t *)p, r0);
+    store16((uint8_t *)p + pitch, r1);
+  }
 }
 
 // ---------------------------------------------------------------------------
 // upcast, destination contiguous along r, 16-byte aligned: the mirror image of downcast_cols_tile_kernel.  The
 // codes and scales of a tile of GT groups x 32*NV columns come in as GT x 16 contiguous bytes per column, pass
-// through LDS, and a store instruction of a wave writes 512 contiguous bytes of two destination rows.
+// through LDS, and a store instruction of a wave writes 512 contiguous bytes of two destination rows (ONCE: past the caches).
 // ---------------------------------------------------------------------------
-template <int DT>
+template <int DT, int GT, bool ONCE>
 __global__ __launch_bounds__(256) void upcast_cols_tile_kernel(
     const uint8_t *__restrict__ vals, int64_t vsb, int64_t vsr, const uint8_t *__restrict__ scales,
     int64_t csb, int64_t csr, void *__restrict__ dst, int64_t nb, int64_t G, int64_t nr, int64_t dsb,
     int64_t dsl) {
   constexpr int ES = DT == TAMD_F32 ? 4 : 2;
   constexpr int NV = 16 / ES;
-  constexpr int GT = kTileGroups<DT>;
   constexpr int CW = kTileCols<DT>;
   extern __shared__ uint4 s_tile[];
   uint4 *s_codes = s_tile;
@@ -622,10 +622,10 @@ __global__ __launch_bounds__(256) void upcast_cols_tile_kernel(
         uint32_t w[NV];
 #pragma unroll
         for (int c = 0; c < NV; ++c) w[c] = j == 0 ? code[c].x : (j == 1 ? code[c].y : (j == 2 ? code[c].z : code[c].w));
-        upcast_rows2<DT, 0>(w, mult, base + (int64_t)(8 * j + 0) * dsl * ES, dsl * ES);
-        upcast_rows2<DT, 1>(w, mult, base + (int64_t)(8 * j + 2) * dsl * ES, dsl * ES);
-        upcast_rows2<DT, 2>(w, mult, base + (int64_t)(8 * j + 4) * dsl * ES, dsl * ES);
-        upcast_rows2<DT, 3>(w, mult, base + (int64_t)(8 * j + 6) * dsl * ES, dsl * ES);
+        upcast_rows2<DT, 0, ONCE>(w, mult, base + (int64_t)(8 * j + 0) * dsl * ES, dsl * ES);
+        upcast_rows2<DT, 1, ONCE>(w, mult, base + (int64_t)(8 * j + 2) * dsl * ES, dsl * ES);
+        upcast_rows2<DT, 2, ONCE>(w, mult, base + (int64_t)(8 * j + 4) * dsl * ES, dsl * ES);
+        upcast_rows2<DT, 3, ONCE>(w, mult, base + (int64_t)(8 * j + 6) * dsl * ES, dsl * ES);
       }
       continue;
     }
@@ -648,20 +648,20 @@ __global__ __launch_bounds__(256) void upcast_cols_tile_kernel(
   }
 }
 
-// Up to how many tiles a tensor whose quantised axis is strided goes to the kernels of one column per thread instead of the tile
-// kernels.  A tile is 131072 elements to a workgroup whose passes follow one another, so that one round of tiles takes the
-// same time for few of them as for one per CU: 13 to 23 us to quantise, 8 to 12 to dequantise; the column kernels have 64 times
-// the workgroups and take about 4 us and 1 us per million elements.  Measured over 97 shapes [1 .. 8, 512 .. 2880, 512 .. 5760] of
-// 5 to 300 tiles on 256 CUs, the lines with the least time lost to the wrong kernel (us, by tiles / by columns):
-//   quantising    float32  152 tiles 17.4 / 15.2, 168: 22.1 / 19.3, 192: 22.7 / 19.9, 195: 16.1 / 17.5, 216: 26.0 / 26.8
-//                 16-bit    96 tiles 16.3 / 13.5, 105: 17.3 / 15.5, 114: 17.0 / 15.5, 120: 17.8 / 18.2, 126: 17.2 / 19.1
-//   dequantising  float32   44 tiles 10.8 / 10.0,  48: 11.6 / 10.3,  52: 12.3 / 12.1,  56: 10.7 / 12.4,  64: 11.9 / 12.4
-//                 16-bit    26 tiles  8.2 /  6.8,  32:  8.8 /  8.1,  35:  8.9 /  8.1,  39:  8.9 / 10.0,  48:  9.1 / 11.7
-// Fewer CUs hold a round of fewer tiles: the lines are shares of their number, given for 256.
-template <int DT>
-constexpr int64_t kColumnsUpToDown = DT == TAMD_F32 ? 192 : 116;
-template <int DT>
-constexpr int64_t kColumnsUpToUp = DT == TAMD_F32 ? 52 : 36;
+// Up to how many tiles of 8 groups a tensor whose quantised axis is strided goes to the kernels of one column per thread instead of the tile
+// kernels, given for 256 CUs.  Tiles of 32 groups (float32) and 16 left most of a last round empty on all but the largest tensors: 160
+// of [1 .. 8, 512 .. 2880, 512 .. 5760], time with tiles of 8 over the time before: quantising float32 0.927, bf16 0.911, dequantising to
+// float32 0.87, to bf16 0.855; from four rounds of the larger tiles on those are as fast or faster (quantising 8 x 2880 x 5760 float32:
+// 109.5 us in tiles of 32, 109.8 of 8), if rows start on lines.  With the merged halves below, float32 and back to bf16: 8 x 2304 x 3032
+// 55.9 + 43.2 -> 48.9 + 24.1 us, 8 x 2432 x 1432 39.9 + 23.3 -> 24.5 + 14.7; 150 others 0.88 and 0.79.  Just above the lines columns and
+// tiles take about as long: quantising 7.5 us and 7.8 at 130 tiles (float32), 8.6 and 8.7 at 105 (bf16), dequantising 4.9 and 5.7 at 33,
+// 5.3 and 5.6 at 45.
+constexpr int64_t kColumnsUpToDown = 96, kColumnsUpToUp = 40;
+// Rows that do not start on a line of 128 bytes: a line that two tiles share is read, or written in part, by both.  Non-temporal loads fetch
+// it from memory for each (plain loads 0.86 to 0.98 of the time); non-temporal stores send it out in halves, where the second-level
+// cache would have merged them: from 160 tiles on plain ones take 0.70 to 0.87 of the time, below 1.0 to 1.08.  With rows on lines
+// plain loads and stores take 1.04 to 1.2.
+constexpr int64_t kMergedFromUp = 160;
 
 // Groups from which a thread of the row kernels takes two: below, the grid would no longer give every SIMD a few waves.
 constexpr int64_t kRowsUnrolled = 64 * 2048;
@@ -688,16 +688,20 @@ int launch_downcast(const void *src, int64_t nb, int64_t L, int64_t nr, int64_t 
   if constexpr (QK != QK_E2M1) return TAMD_E_UNSUPPORTED;  // fp8 values: quantised axis contiguous only
   constexpr int NV = 16 / ES;
   bool vec = nr % NV == 0 && aligned(src, 16) && (ssb * ES) % 16 == 0 && (ssl * ES) % 16 == 0;
-  constexpr int CW = kTileCols<DT>, GT = kTileGroups<DT>;
-  const int64_t tiles = ((nr + CW - 1) / CW) * ((G + GT - 1) / GT) * nb;
+  constexpr int CW = kTileCols<DT>;
+  constexpr int WIDE = DT == TAMD_F32 ? 32 : 16;   // 64 KiB of codes
+  const int64_t cols = (nr + CW - 1) / CW * nb, tiles = cols * ((G + 7) / 8);
   int cus = 0;
   if (int rc = cu_count(cus)) return rc;
-  if (vec && tiles * 256 > kColumnsUpToDown<DT> * cus) {
-    const int64_t blocks = tiles;
+  if (vec && tiles * 256 > kColumnsUpToDown * cus) {
+    const bool lines = aligned(src, 128) && (ssb * ES) % 128 == 0 && (ssl * ES) % 128 == 0;
+    const bool wide = lines && cols * ((G + WIDE - 1) / WIDE) >= 4 * (int64_t)cus;   // (there longer runs weigh more than the tail of the last round)
+    const int64_t blocks = wide ? cols * ((G + WIDE - 1) / WIDE) : tiles;
     if (blocks > 0x7FFFFFFF) return TAMD_E_UNSUPPORTED;
-    if (int rc = raise_lds_limit_once((const void *)downcast_cols_tile_kernel<DT>)) return rc;
-    downcast_cols_tile_kernel<DT><<<dim3((unsigned)blocks), 256, kTileLds<DT>, st>>>(src, nb, G, nr, ssb, ssl, vals, vsb, vsr,
-                                                                         scales, csb, csr, mode);
+    auto kern = wide ? downcast_cols_tile_kernel<DT, WIDE, true> : (lines ? downcast_cols_tile_kernel<DT, 8, true> : downcast_cols_tile_kernel<DT, 8, false>);
+    if (int rc = raise_lds_limit_once((const void *)kern)) return rc;
+    kern<<<dim3((unsigned)blocks), 256, wide ? kTileLds<DT, WIDE> : kTileLds<DT, 8>, st>>>(src, nb, G, nr, ssb, ssl, vals, vsb, vsr, scales, csb, csr,
+                                                                               mode);
   } else {
     int64_t blocks = ((nr + 31) / 32) * ((G + 7) / 8) * nb;
     if (blocks > 0x7FFFFFFF) return TAMD_E_UNSUPPORTED;
@@ -727,16 +731,19 @@ int launch_upcast(const uint8_t *vals, int64_t vsb, int64_t vsr, const uint8_t *
   if constexpr (QK != QK_E2M1) return TAMD_E_UNSUPPORTED;  // fp8 values: quantised axis contiguous only
   constexpr int NV = 16 / ES;
   bool vec = nr % NV == 0 && aligned(dst, 16) && (dsb * ES) % 16 == 0 && (dsl * ES) % 16 == 0;
-  constexpr int CW = kTileCols<DT>, GT = kTileGroups<DT>;
-  const int64_t tiles = ((nr + CW - 1) / CW) * ((G + GT - 1) / GT) * nb;
+  constexpr int CW = kTileCols<DT>;
+  const int64_t cols = (nr + CW - 1) / CW * nb, tiles = cols * ((G + 7) / 8);
   int cus = 0;
   if (int rc = cu_count(cus)) return rc;
-  if (vec && tiles * 256 > kColumnsUpToUp<DT> * cus) {
-    const int64_t blocks = tiles;
+  if (vec && tiles * 256 > kColumnsUpToUp * cus) {
+    const bool lines = aligned(dst, 128) && (dsb * ES) % 128 == 0 && (dsl * ES) % 128 == 0;
+    const bool wide = lines && cols * ((G + 15) / 16) >= 4 * (int64_t)cus;   // (as when quantising)
+    const int64_t blocks = wide ? cols * ((G + 15) / 16) : tiles;
     if (blocks > 0x7FFFFFFF) return TAMD_E_UNSUPPORTED;
-    if (int rc = raise_lds_limit_once((const void *)upcast_cols_tile_kernel<DT>)) return rc;
-    upcast_cols_tile_kernel<DT><<<dim3((unsigned)blocks), 256, kTileLds<DT>, st>>>(vals, vsb, vsr, scales, csb, csr, dst, nb, G,
-                                                                       nr, dsb, dsl);
+    auto kern = wide ? upcast_cols_tile_kernel<DT, 16, true>
+                     : (lines || tiles * 256 <= kMergedFromUp * cus ? upcast_cols_tile_kernel<DT, 8, true> : upcast_cols_tile_kernel<DT, 8, false>);
+    if (int rc = raise_lds_limit_once((const void *)kern)) return rc;
+    kern<<<dim3((unsigned)blocks), 256, wide ? kTileLds<DT, 16> : kTileLds<DT, 8>, st>>>(vals, vsb, vsr, scales, csb, csr, dst, nb, G, nr, dsb, dsl);
   } else {
     int64_t blocks = ((nr + 31) / 32) * ((G + 7) / 8) * nb;
     if (blocks > 0x7FFFFFFF) return TAMD_E_UNSUPPORTED;
