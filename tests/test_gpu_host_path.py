@@ -1,5 +1,7 @@
 """GPU: what the routing kernels leave in expert-sorted order, on every launch form of the routing, against the oracle; what the
 host code of the entry points hands out and keeps."""
+import sys
+
 import pytest
 import torch
 
@@ -30,6 +32,40 @@ def test_expert_sorted_gate_weights(T, E, k, dtype, device):
     assert torch.equal(r.scatter_indx.cpu(), ref["scatter_indx"])
     gates = r.expert_sorted_gate_weights
     assert gates.dtype == dtype and torch.equal(gates.cpu(), r.vals.cpu().flatten()[ref["scatter_indx"].long()])
+
+
+@pytest.mark.parametrize("T,E,k", [(1, 1, 1), (3, 64, 2), (16, 500, 4), (700, 33, 3), (9000, 128, 4)])
+def test_routing_tables_of_one_call(T, E, k, device):
+    """Each table against the oracle, whichever is asked for first, by the call that lays a shape out and by the next one, and
+    after so many other shapes that the layouts were dropped."""
+    module = sys.modules["triton_amd.routing"]
+    torch.manual_seed(T)
+    logits = torch.randn(T, E)
+    ref = RR.routing_ref(logits, k)
+    dev = logits.to(device)
+    module._layouts.clear()
+    for i in range(3):
+        if i == 2:
+            module._layouts.update({(j, 0, 0, 0): {} for j in range(600)})   # (600 entries of no shape: the next new shape drops all)
+            routing(torch.randn(T + 1, E, device=device), k)
+            assert len(module._layouts) == 1
+        r = routing(dev, k)
+        if i == 1:
+            assert torch.equal(r.gather_indx.cpu(), ref["gather_indx"])
+        md = r.ragged_metadata
+        assert torch.equal(r.scatter_indx.cpu(), ref["scatter_indx"]) and torch.equal(r.gather_indx.cpu(), ref["gather_indx"])
+        assert torch.equal(r.col_sum.cpu(), ref["col_sum"]) and md.slice_sizes is r.col_sum
+        inverse = torch.empty_like(ref["scatter_indx"])
+        inverse[ref["scatter_indx"].long()] = torch.arange(T * k, dtype=inverse.dtype)
+        assert torch.equal(r.row_sorted_indx.cpu(), inverse)
+        sizes = ref["col_sum"].long()
+        assert torch.equal(md.slice_offs.cpu().long(), torch.cat([torch.zeros(1, dtype=torch.long), sizes.cumsum(0)]))
+        for b in md.block_sizes():
+            blocks = (sizes + b - 1) // b
+            assert torch.equal(md.block_offs(b).cpu().long(), torch.cat([torch.zeros(1, dtype=torch.long), blocks.cumsum(0)]))
+            want = [(j << 16) | e for e in range(E) for j in range(int(blocks[e]))]
+            got = md.block_schedule(b).cpu().tolist()
+            assert got[:len(want)] == want and all(v == -1 for v in got[len(want):])
 
 
 @pytest.mark.parametrize("inference", [False, True])

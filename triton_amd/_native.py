@@ -1,7 +1,7 @@
 """Loader of the native host path (csrc/host.cpp, built into `_host.so`).
 
-`matmul`, `routing`, `view`, `reduce`, `downcast` and `upcast` are the extension's functions once it is loaded, which the
-first call does.  Each answers None for a call it does not cover; the caller then runs its general path."""
+`matmul`, `routing`, `view`, `int_views`, `reduce`, `downcast` and `upcast` are the extension's functions once it is loaded,
+which the first call does.  Each answers None for a call it does not cover; the caller then runs its general path."""
 import ctypes
 import os
 
@@ -50,7 +50,7 @@ def _on_first_call(name):
     return call
 
 
-_FUNCTIONS = ("matmul", "routing", "view", "reduce", "downcast", "upcast", "choose_block_m", "blocks_of_16_stream", "dense_block_m",
-              "ring_rows")
+_FUNCTIONS = ("matmul", "routing", "view", "int_views", "reduce", "downcast", "upcast", "choose_block_m", "blocks_of_16_stream",
+              "dense_block_m", "ring_rows")
 for _n in _FUNCTIONS:
     globals()[_n] = _on_first_call(_n)

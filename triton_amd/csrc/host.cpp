@@ -45,7 +45,7 @@ struct Names {
       *b_mx_tensor_scale, *acc_scale, *a_mx_scale, *a_microblock_size, *b_mx_scale, *b_microblock_size, *flex_ctx, *lhs_data,
       *rhs_data, *out_data, *acc_data, *scale, *expected_scale, *actual_scale, *checksum_scale, *out_dtype,
       *flexpoint_saturate_inf, *specs, *name, *fn_arg_names, *fn_args, *reduction_n, *slice_sizes, *slice_offs,
-      *block_offs_data, *block_schedule_data, *expected_slice_size;
+      *block_offs_data, *block_schedule_data, *expected_slice_size, *native;
 } nm;
 
 // ------------------------------------------------------------------ small helpers
@@ -505,19 +505,28 @@ PyObject *py_matmul(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
 }
 
 // ------------------------------------------------------------------ routing
-// (logits, k, layout): `layout` is the tuple of routing._arena_layout (sizes and byte offsets of one call's arena).  The
-// arena, an error code, or None.
+// (logits, k, layouts): `layouts` is routing._layouts, (rows, experts, k, type code) -> layout of one call's arena; its part
+// "native" holds the numbers that follow as 64-bit integers (arena's length, sizes of the tables, byte offset of every part).
+// (arena, layout), an error code, or None.  (Checks and the look-up in Python took 0.9 us of the 5 of a call of one launch.)
 PyObject *py_routing(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
   return covered([&]() -> PyObject * {
-    need(nargs == 3 && PyTuple_Check(v[2]) && PyTuple_GET_SIZE(v[2]) == 16);
+    need(nargs == 3 && PyDict_Check(v[2]));
     int dev = -1;
     const at::Tensor &x = gpu_tensor(v[0], dev);
-    int64_t o[16];
-    for (int i = 0; i < 16; ++i) o[i] = as_int(PyTuple_GET_ITEM(v[2], i));
+    need(x.dim() == 2 && x.stride(1) == 1);
     const int code = type_code(x.scalar_type());
+    const int64_t T = x.size(0), E = x.size(1), k = as_int(v[1]);
+    Ref key(Py_BuildValue("LLLi", (long long)T, (long long)E, (long long)k, code));
+    if (!key.p) return nullptr;
+    PyObject *lay = PyDict_GetItem(v[2], key.p);
+    need(lay != nullptr && PyDict_Check(lay));
+    const Ref held(Py_NewRef(lay));   // (the launch lets other threads run)
+    PyObject *numbers = PyDict_GetItem(lay, nm.native);
+    int64_t o[16];
+    need(numbers && PyBytes_Check(numbers) && PyBytes_GET_SIZE(numbers) == sizeof o);
+    std::memcpy(o, PyBytes_AS_STRING(numbers), sizeof o);
     at::Tensor arena = new_empty({o[0]}, at::kInt, dev);
     uint8_t *b = (uint8_t *)arena.data_ptr();
-    const int64_t T = x.size(0), E = x.size(1), k = as_int(v[1]);
     void *st = stream_of(dev);
     auto p = [&](int i) { return (int32_t *)(b + o[i]); };
     const int rc = without_gil([&] {
@@ -525,7 +534,31 @@ PyObject *py_routing(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
                          o[4], p(8), p(9), p(10), p(11), p(12), p(13), o[2], p(14), o[3], (int)o[1], p(15), st);
     });
     if (rc != 0) return PyLong_FromLong(rc);
-    return THPVariable_Wrap(arena);
+    Ref t(THPVariable_Wrap(arena));
+    return t.p ? PyTuple_Pack(2, t.p, lay) : nullptr;
+  });
+}
+
+// (base, numbers): int32 tensors over parts of `base`'s storage, a tuple; five 64-bit integers each: element offset, size0,
+// stride0, size1 (-1: one dimension), stride1.
+PyObject *py_int_views(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
+  return covered([&]() -> PyObject * {
+    need(nargs == 2 && PyBytes_Check(v[1]));
+    const at::Tensor &t = tensor(v[0]);
+    constexpr size_t kEach = 5 * sizeof(int64_t);
+    const Py_ssize_t n = PyBytes_GET_SIZE(v[1]) / (Py_ssize_t)kEach;
+    Ref all(PyTuple_New(n));
+    if (!all.p) return nullptr;
+    for (Py_ssize_t i = 0; i < n; ++i) {
+      int64_t o[5];
+      std::memcpy(o, PyBytes_AS_STRING(v[1]) + i * kEach, kEach);
+      const int64_t sizes[2] = {o[1], o[3]}, strides[2] = {o[2], o[4]};
+      const size_t nd = o[3] < 0 ? 1 : 2;
+      PyObject *w = THPVariable_Wrap(alias(t, at::kInt, o[0], at::IntArrayRef(sizes, nd), at::IntArrayRef(strides, nd)));
+      if (!w) return nullptr;
+      PyTuple_SET_ITEM(all.p, i, w);
+    }
+    return Py_NewRef(all.p);
   });
 }
 
@@ -736,7 +769,7 @@ PyObject *py_init(PyObject *, PyObject *args) {
       TAMD_NAME(acc_data), TAMD_NAME(scale), TAMD_NAME(expected_scale), TAMD_NAME(actual_scale), TAMD_NAME(checksum_scale),
       TAMD_NAME(out_dtype), TAMD_NAME(flexpoint_saturate_inf), TAMD_NAME(specs), TAMD_NAME(name), TAMD_NAME(fn_arg_names),
       TAMD_NAME(fn_args), TAMD_NAME(reduction_n), TAMD_NAME(slice_sizes), TAMD_NAME(slice_offs), TAMD_NAME(block_offs_data),
-      TAMD_NAME(block_schedule_data), TAMD_NAME(expected_slice_size);
+      TAMD_NAME(block_schedule_data), TAMD_NAME(expected_slice_size), TAMD_NAME(native);
 #undef TAMD_NAME
   Py_RETURN_NONE;
 }
@@ -746,6 +779,7 @@ PyMethodDef methods[] = {{"init", py_init, METH_VARARGS, nullptr},
                          {"matmul", TAMD_FAST(py_matmul)},
                          {"routing", TAMD_FAST(py_routing)},
                          {"view", TAMD_FAST(py_view)},
+                         {"int_views", TAMD_FAST(py_int_views)},
                          {"reduce", TAMD_FAST(py_reduce)},
                          {"downcast", TAMD_FAST(py_downcast)},
                          {"upcast", TAMD_FAST(py_upcast)},

@@ -4,9 +4,9 @@ metadata; gather = col_sorted // k, scatter = col_sorted).
 
 One foreign call (`tamd_routing`: one launch at decode sizes, two up to 65535 rows, else four) writes into
 one int32 arena that holds every output and the kernels' workspace; its layout is computed once per shape and the
-tensors of the result are views of that arena, built when they are first asked for: at these sizes the host time of
-this function is what a step waits for."""
-import functools
+tensors of the result are views of that arena, built when they are first asked for (the index arrays and ragged tables
+together, in one call): at these sizes the host time of this function is what a step waits for."""
+import struct
 
 import torch
 
@@ -28,12 +28,16 @@ class RoutingResult:
     def __init__(self, arena, lay, bits=None, indx=None, vals=None):
         self._arena, self._lay, self._bits, self._indx, self._vals, self._cache = arena, lay, bits, indx, vals, {}
 
+    def _tables(self):
+        """The index arrays and the ragged tables, all with one call (seven calls of their own took twice as long)."""
+        c = self._cache
+        c["col_sum"], c["offs"], c["block_offs"], c["sched"], c["gather"], c["col_sorted"], c["row_sorted"] = \
+            _native.int_views(self._arena, self._lay["tables"])
+        return c
+
     def _view(self, name):
         v = self._cache.get(name)
-        if v is None:
-            off, n = self._lay[name]
-            v = self._cache[name] = _native.view(self._arena, torch.int32, off, n, 1, -1, 0)
-        return v
+        return self._tables()[name] if v is None else v
 
     def _view2(self, name, dtype, n0, stride0, n1, stride1=1, skip=0):
         """A two-dimensional view of part `name` of the arena in another type (sizes, strides and `skip` in its elements)."""
@@ -71,14 +75,11 @@ class RoutingResult:
     def ragged_metadata(self):
         md = self._cache.get("ragged")
         if md is None:
-            E, width, po, ps = self._lay["dims"]
+            c = self._cache if "row_sorted" in self._cache else self._tables()   # (the last one that _tables() writes)
             # (an instance made field by field: the checks of its constructor hold by construction)
-            md = self._cache["ragged"] = RaggedTensorMetadata.__new__(RaggedTensorMetadata)
-            md.__dict__.update(slice_sizes=self.col_sum,
-                               slice_offs=_native.view(self._arena, torch.int32, self._lay["offs"][0], E + 1, 1, -1, 0),
-                               block_offs_data=self._view2("offs", torch.int32, 5, po, E + 1, skip=po),
-                               block_schedule_data=self._view2("sched", torch.int32, 5, ps, width),
-                               expected_slice_size=None, slice_sizes_divisibility=None)
+            md = c["ragged"] = RaggedTensorMetadata.__new__(RaggedTensorMetadata)
+            md.__dict__.update(slice_sizes=c["col_sum"], slice_offs=c["offs"], block_offs_data=c["block_offs"],
+                               block_schedule_data=c["sched"], expected_slice_size=None, slice_sizes_divisibility=None)
         return md
 
     @property
@@ -116,7 +117,18 @@ class RoutingResult:
         return self._vals is None or (not self._vals.is_inference() and self._vals._version == 0)
 
 
-@functools.lru_cache(maxsize=512)
+def _int_tables(lay):
+    """What `RoutingResult._tables` views: offset, size and stride of each axis (size -1: there is none)."""
+    E, width, po, ps = lay["dims"]
+    at = lambda name: lay[name][0]
+    line = lambda name: (at(name), lay[name][1], 1, -1, 0)
+    return struct.pack("35q", *line("col_sum"), at("offs"), E + 1, 1, -1, 0, at("offs") + po, 5, po, E + 1, 1, at("sched"), 5, ps, width, 1,
+                       *line("gather"), *line("col_sorted"), *line("row_sorted"))
+
+
+_layouts = {}  # (T, E, k, type code) -> _arena_layout: the native call looks them up
+
+
 def _arena_layout(T: int, E: int, k: int, vals_dtype: torch.dtype):
     """Where every output of `tamd_routing` (and its workspace) sits in the int32 arena of one call: name -> (offset,
     length) in ints, each part 16-byte aligned.  Depends on the shapes only, so it is built once per shape."""
@@ -136,25 +148,39 @@ def _arena_layout(T: int, E: int, k: int, vals_dtype: torch.dtype):
         off += -(-size // 4) * 4
     # what the native call needs, in the order that csrc/host.cpp reads: the arena's length, the sizes of the tables, the
     # byte offset of every part
-    lay["native"] = (off, width, po, ps, pad_t, *(4 * lay[name][0] for name in (
+    lay["native"] = struct.pack("16q", off, width, po, ps, pad_t, *(4 * lay[name][0] for name in (
         "vals", "indx", "bits", "col_sum", "col_sorted", "row_sorted", "gather", "gates", "offs", "sched", "ws")))
+    lay["tables"] = _int_tables(lay)
     return lay
 
 
 def routing(logits: torch.Tensor, n_expts_act: int, y_indx=None) -> RoutingResult:
-    if y_indx is not None or logits.stride(1) != 1:
-        return _routing_two_calls(logits, n_expts_act, y_indx)
+    if y_indx is None:
+        done = _native.routing(logits, n_expts_act, _layouts)
+        if done is None:
+            done = _routing_first_call(logits, n_expts_act)
+        if type(done) is tuple:
+            return RoutingResult(*done)
+        if type(done) is int:
+            _lib.check(done, "routing")
+    return _routing_two_calls(logits, n_expts_act, y_indx)
+
+
+def _routing_first_call(logits, k):
+    """The first call of a shape: checks, the arena's layout, then what `_native.routing` answers; None for strided logits."""
+    if logits.stride(1) != 1:
+        return None
     _lib.require_gpu(logits, "logits")
     assert logits.ndim == 2 and logits.shape[1] < 32768
     T, E = logits.shape
-    k = n_expts_act
-    _lib.dtype_code(logits.dtype)  # (refuses other types before the layout divides by their size)
+    code = _lib.dtype_code(logits.dtype)  # (refuses other types before the layout divides by their size)
     lay = _arena_layout(T, E, k, logits.dtype)
-    arena = _native.routing(logits, k, lay["native"])
-    if type(arena) is int:
-        _lib.check(arena, "routing")
-    assert arena is not None, "k must be an int and logits of a floating type"
-    return RoutingResult(arena, lay)
+    if len(_layouts) >= 512:
+        _layouts.clear()
+    _layouts[T, E, k, code] = lay
+    done = _native.routing(logits, k, _layouts)
+    assert done is not None, "k must be an int and logits of a floating type"
+    return done
 
 
 def _routing_two_calls(logits, n_expts_act, y_indx):
@@ -174,6 +200,7 @@ def _routing_two_calls(logits, n_expts_act, y_indx):
                        ("ws", n_ws)):
         lay[name] = (off, size)
         off += -(-size // 4) * 4
+    lay["tables"] = _int_tables(lay)
     arena = torch.empty(off, dtype=torch.int32, device=dev)
     base = arena.data_ptr()
     p = lambda name: base + 4 * lay[name][0]
