@@ -506,7 +506,7 @@ TAMD_DEVICE uint32_t quad_xor2(uint32_t v) { return (uint32_t)__builtin_amdgcn_u
 // (The selectors by arithmetic on a constant that the compiler does not see through: as selections between two constants it keeps both
 // in vector registers over the tiles of a persistent kernel.)
 TAMD_DEVICE uint32_t flip_where(uint32_t base, int bit_mask, uint32_t diff) {
-  asm("" : "+s"(diff));
+  asm volatile("" : "+s"(diff));
   return base ^ ((uint32_t)bit_mask & diff);
 }
 TAMD_DEVICE uint32_t quad_rows(uint32_t rows0123, int lane) {
