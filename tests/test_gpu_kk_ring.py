@@ -28,6 +28,8 @@ def ring_rows(m, n, k, e, swiglu=False, **changed):
 def test_where_it_is_taken():
     assert ring_rows(1200, 5760, 2880, 32) == 64 and ring_rows(4084, 5760, 2880, 32, True) == 160
     assert ring_rows(4, 3904, 1760, 8) == 0
+    assert all(ring_rows(sum(sizes), N, K, len(sizes)) == 64 for sizes, K, N in FEW)
+    assert ring_rows(816, 1024, 5376, 8) == 0 and ring_rows(31, 2560, 5376, 8) == 0
     for changed in (dict(block_schedule=None), dict(n_experts=257), dict(y_dtype=_lib.F32), dict(y_rows=0), dict(y_rows=1 << 20), dict(K=248),
                     dict(y_expected_scale=1 << 20), dict(N=5759), dict(y=(1 << 20) + 2), dict(y_stride_m=5761), dict(x_dtype=_lib.F16), dict(force_variant=64)):
         assert ring_rows(4084, 5760, 2880, 32, **changed) == 0, changed
@@ -36,10 +38,13 @@ def test_where_it_is_taken():
 # (slice sizes, K, columns)
 SIZES = [([1, 0, 31, 32, 33, 64, 65, 0, 129, 3], 256, 6200), ([2] * 70 + [0] * 30, 1096, 648), ([160, 161, 0, 320, 321, 95, 97, 700], 776, 3176),
          ([1500, 0, 40], 520, 4100), ([5000], 264, 1032)]
+# fewer than a tile of 256 columns for every third CU, and just above: blocks of 64
+FEW = [([100, 64, 65, 128, 129, 0, 200, 130], 1032, 1288), ([700, 0, 65, 127], 520, 2056), ([33, 40, 1, 64, 70, 10, 66, 0], 264, 1800),
+       ([10, 0, 16, 3, 33, 1, 2, 3] * 2, 776, 1096), ([100] * 10 + [128, 129], 776, 1800)]
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("sizes,K,N", SIZES)
+@pytest.mark.parametrize("sizes,K,N", SIZES + FEW)
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("swiglu", [False, True])
 @pytest.mark.parametrize("gathered", [False, True])

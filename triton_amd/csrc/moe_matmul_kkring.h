@@ -15,7 +15,8 @@
 //     size.
 // A sum is one float32 accumulator for all of K, the tiled kernel's two (of either half of every stage): a wave of blocks of 160 rows has
 // the registers for one.  Results of K 2880 against 64-bit sums (2-norm): bf16 1.662372e-3 from both, which is what rounding the exact sums gives;
-// f16 2.077690e-4, 2.077689e-4 from the tiled kernel, 2.077687e-4 from rounding alone.
+// f16 2.077690e-4, 2.077689e-4 from the tiled kernel, 2.077687e-4 from rounding alone; of K 5376 bf16 1.6563609e-3 all three, f16 2.0717160e-4,
+// 2.0717133e-4 and 2.0717109e-4.
 // Blocks of 160 rows, the most that three stages have LDS for (128: 1021 tokens 225, 2000 tokens 357 where 160 take 311; 96: 266 and 393);
 // of 64 where slices are smaller, whose copies of rows that are not there cost 2 to 4 % (300 tokens: 170 -> 165; blocks of 32 with a ring
 // of four: 208).

@@ -196,17 +196,23 @@ inline bool kk_ring_applicable(const tamd_matmul_args &a) {
   return a.activation == TAMD_ACT_SWIGLU || (((a.N | (int)a.y_stride_m) & 1) == 0 && aligned(a.y, 4));
 }
 
-// Rows of its blocks, 0 where the tiled kernels are the faster: with fewer than a third as many tiles of 256 columns as CUs one workgroup's
-// stages are all latency (four rows for 8 slices, 1760 x 3904: 13.4 us, 16 with this one).  486 products of 1 to 16384 tokens, 8 to 128
-// slices, K and N 512 to 5760: 0.876 of the time in the mean (0.866 with the best choice for each), none above 1.05; with the line at 0.25
-// 0.874, three above 1.1; at 0.5 0.888.  Blocks of 64 up to 56 rows per slice lose up to 1.21, where slices come in two.
+// Rows of its blocks, 0 where the tiled kernels are the faster.  The lines are in thirds of a tile of 256 columns per CU, row blocks of 160 counted:
+// where there are few, one workgroup's stages are all latency (four rows for 8 slices, 1760 x 3904: 13.4 us, 16 with this one).
+// From one third on, 486 products of 1 to 16384 tokens, 8 to 128 slices, K and N 512 to 5760: 0.876 of the time in the mean (0.866 with the
+// best choice for each), none above 1.05.  Blocks of 64 up to 56 rows per slice lose up to 1.21, where slices come in two.
+// Below it blocks of 64 give four narrow strips and their row blocks a CU each, where the tiled kernel leaves most CUs without a tile: the more rows per
+// slice, the earlier.  Of 10600 products below the line (8 to 60 slices, bf16) the 3000 that the lines take: 0.84 of the time in the mean,
+// 14 above 1.05 (1.10 at most); 102 rows for each of 8 slices, 5376 x 1984: 66.8 -> 50 us.  Under four rows per slice up to 1.9, half a line further
+// down 0.93 to 1.25 with 2.1 at worst.  Just above it blocks of 64 up to 128 rows per slice take 0.84 to 0.9 of what those of 160 do, from 1.3
+// thirds on up to 1.5.
 inline int kk_ring_rows(const tamd_matmul_args &a, int cus) {
   if (!kk_ring_applicable(a)) return 0;
   // (the line below, whichever slices the rows fall on)
   if (a.M <= a.n_experts && 3 * (int64_t)most_live_slices(a) * ((a.N + 255) / 256) < cus) return 0;
   const double mean = (double)a.M / a.n_experts, tiles = live_slices(a) * ((a.N + 255) / 256) / cus;
-  if (3.0 * tiles * (mean > 160.0 ? mean / 160.0 : 1.0) < 1.0) return 0;
-  return mean <= 48.0 ? 64 : 160;
+  const double thirds = 3.0 * tiles * (mean > 160.0 ? mean / 160.0 : 1.0);
+  if (thirds < 1.0) return mean >= 4.0 && thirds >= (mean < 32.0 ? 0.9 : mean < 48.0 ? 0.6 : mean < 128.0 ? 0.5 : 0.4) ? 64 : 0;
+  return mean <= 48.0 || (mean < 128.0 && thirds < 1.15) ? 64 : 160;
 }
 
 // Row block size of a dense / batched problem: the block whose tiles take the fewest rounds over the CUs, weighted with what a
