@@ -200,11 +200,11 @@ inline bool kk_ring_applicable(const tamd_matmul_args &a) {
 // where there are few, one workgroup's stages are all latency (four rows for 8 slices, 1760 x 3904: 13.4 us, 16 with this one).
 // From one third on, 486 products of 1 to 16384 tokens, 8 to 128 slices, K and N 512 to 5760: 0.876 of the time in the mean (0.866 with the
 // best choice for each), none above 1.05.  Blocks of 64 up to 56 rows per slice lose up to 1.21, where slices come in two.
-// Below it blocks of 64 give four narrow strips and their row blocks a CU each, where the tiled kernel leaves most CUs without a tile: the more rows per
-// slice, the earlier.  Of 10600 products below the line (8 to 60 slices, bf16) the 3000 that the lines take: 0.84 of the time in the mean,
-// 14 above 1.05 (1.10 at most); 102 rows for each of 8 slices, 5376 x 1984: 66.8 -> 50 us.  Under four rows per slice up to 1.9, half a line further
-// down 0.93 to 1.25 with 2.1 at worst.  Just above it blocks of 64 up to 128 rows per slice take 0.84 to 0.9 of what those of 160 do, from 1.3
-// thirds on up to 1.5.
+// Below it tiles of one to three strips of 64 columns and blocks of 64 rows reach every CU, where the tiled kernel leaves most of them without
+// a tile: the more rows per slice, the earlier.  Of 10600 products below the line (8 to 60 slices, bf16) the 3000 that the lines take:
+// 0.84 of the time in the mean, 14 above 1.05 (1.10 at most); layer of 102 rows for each of 8 slices, f16, 5376 -> 992, 112 -> 93 us.  Under four
+// rows per slice up to 1.9; half a line further down 0.93 to 1.25, 2.1 at worst.  Just above the line blocks of 64 for up to 128
+// rows per slice take 0.84 to 0.9 of what those of 160 do; from 1.3 thirds on up to 1.5.
 inline int kk_ring_rows(const tamd_matmul_args &a, int cus) {
   if (!kk_ring_applicable(a)) return 0;
   // (the line below, whichever slices the rows fall on)
