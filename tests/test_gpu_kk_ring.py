@@ -7,6 +7,7 @@ import torch
 
 from triton_amd import _lib, _native
 from triton_amd.matmul import FnSpecs, FusedActivation, PrecisionConfig, matmul
+from triton_amd.matmul_details.opt_flags import scoped_opt_flags_constraints
 from triton_amd.swiglu import swiglu_fn
 from triton_amd.tensor import make_ragged_tensor_metadata
 
@@ -78,3 +79,29 @@ def test_edges(sizes, K, N, dtype, swiglu, gathered, device):
         full, slack, got = full[there.to(device)] * gammas[there.to(device), None], slack[there.to(device)], got[scatter[there].long().to(device)]
     # a 16-bit result (2^-8) of K float32 additions, and the hardware's exponential and reciprocal (2^-20)
     assert bool(((got.float() - full).abs() <= 2.0 ** -8 * full.abs() + slack + 1e-5).all())
+
+
+# (slice sizes, K, columns, row block that the tiled kernels take it in) below the line
+SUMMED = [([55, 64, 33, 70, 41, 60, 0, 66], 576, 2152, 64), ([200, 170, 190, 230], 640, 1800, 64), ([9, 14, 0, 11, 12, 16, 8, 20], 3784, 2560, 32),
+          ([34, 20, 41, 0, 70, 36, 31, 25] * 2, 2768, 904, 32), ([60, 52, 71, 66, 40, 64, 63, 61], 2544, 1856, 64), ([85, 80, 64, 96, 0, 101, 120, 77], 712, 1288, 64)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("sizes,K,N,block_m", SUMMED)
+def test_sums_below_the_line(sizes, K, N, block_m, device):
+    """As many float32 sums to a result as in the tiled kernels: their bits up to ten stages and where they take narrow tiles, elsewhere no more
+    results that are not the rounded 64-bit sum."""
+    E, M = len(sizes), sum(sizes)
+    assert ring_rows(M, N, K, E) == 64
+    g = torch.Generator().manual_seed(K)
+    x, w = torch.randn(M, K, generator=g).half().to(device), (torch.randn(E, N, K, generator=g) * 0.05).half().to(device).transpose(1, 2)
+    md = make_ragged_tensor_metadata(torch.tensor(sizes, dtype=torch.int32, device=device), M)
+    got = matmul(x, w, None, md, precision_config=PrecisionConfig())
+    with scoped_opt_flags_constraints({"block_m": block_m}):
+        tiled = matmul(x, w, None, md, precision_config=PrecisionConfig())
+    if K <= 640 or block_m < 64:
+        assert torch.equal(got, tiled)
+        return
+    ends = torch.tensor(sizes).cumsum(0).tolist()
+    rounded = torch.cat([x[b - n:b].double() @ w[e].double() for e, (n, b) in enumerate(zip(sizes, ends))]).half()
+    assert int((got != rounded).sum()) <= int((tiled != rounded).sum())

@@ -13,10 +13,15 @@
 //     caches keep (300 tokens x 4 of 32 slices, 2880 -> 2 x 2880: 188 -> 170 us; of columns off the lines 137 -> 150 and 28 -> 34, so not there);
 //   * tiles of fewer strips where that fills the rounds over the workgroups (1021 tokens x 4 of 32: 228 -> 216); blocks of one slice are of one
 //     size.
-// A sum is one float32 accumulator for all of K, the tiled kernel's two (of either half of every stage): a wave of blocks of 160 rows has
+// Sums.  In blocks of 160 rows one float32 accumulator for all of K, where the tiled kernel has two (of either half of every stage): a wave has
 // the registers for one.  Results of K 2880 against 64-bit sums (2-norm): bf16 1.662372e-3 from both, which is what rounding the exact sums gives;
 // f16 2.077690e-4, 2.077689e-4 from the tiled kernel, 2.077687e-4 from rounding alone; of K 5376 bf16 1.6563609e-3 all three, f16 2.0717160e-4,
-// 2.0717133e-4 and 2.0717109e-4.
+// 2.0717133e-4 and 2.0717109e-4.  Blocks of 64 have the registers for two sets: products below the line of kk_ring_rows are summed as the tiled
+// kernels do, up to ten stages in the same two sums to the bit, beyond in four, one for each quarter of K, which are those of the narrow
+// tiles to the bit.  Results that are not the 64-bit sum rounded, f16, tiled kernels / one sum / now: 8 slices of 55 rows, 576 -> 2152, of
+// 951184 743 / 761 / 743; 8 of 12, 3784 -> 2560, of 238080 347 / 446 / 347 (narrow tiles); 8 of 60, 2544 -> 1856, of 885312 1406 / 1451 / 1195.  Of 100 products
+// of 3 to 200 rows per slice, K 256 to 5600, 9 of 19 below the line had more than the tiled kernels with one sum, none now.  The second set costs up to 3 %
+// of a short tile.
 // Blocks of 160 rows, the most that three stages have LDS for (128: 1021 tokens 225, 2000 tokens 357 where 160 take 311; 96: 266 and 393);
 // of 64 where slices are smaller, whose copies of rows that are not there cost 2 to 4 % (300 tokens: 170 -> 165; blocks of 32 with a ring
 // of four: 208).
@@ -27,6 +32,7 @@
 // the address units 80 % (63): 1.12 GB are fetched for 1.06 of weights.
 #pragma once
 #include <algorithm>
+#include <type_traits>
 
 #include "moe_matmul_kk.h"
 
@@ -40,6 +46,7 @@ struct KKRingShape {
   typedef typename KK<XDT>::frag_t frag_t;
   static constexpr int MF = MF_, ROWS = 32 * MF, KS = KK<XDT>::KS;
   static constexpr int N0 = (MF + 1) / 2;                                    // row fragments of a wave, at most
+  static constexpr bool TWO = N0 == 1;                                       // registers for two sums
   static constexpr int STAGE = (ROWS + BLOCK_N) * 128, RING = 3;
   static constexpr int COPIES = 8 + MF;                                      // of a copying wave and stage
   static constexpr int CONSUMERS = 8, THREADS = (CONSUMERS + kKKRingCopiers) * kWave;
@@ -249,9 +256,9 @@ TAMD_DEVICE void kk_ring_copy(const Args &a, int group, bool nt, uint8_t *lds) {
   sync_threads();
 }
 
-// A multiplying wave's part of a tile, NFR row fragments of one strip: the K loop and the epilogue.
+// A multiplying wave's part of a tile, NFR row fragments of one strip: the K loop, into `sums` float32 sums (kk_ring_sums), and the epilogue.
 template <int XDT, int MF, int NFR, int ACT, typename Args>
-TAMD_DEVICE void kk_ring_products(const Args &a, const Tile &t, int half, int first_row, uint8_t *lds, int &slot) {
+TAMD_DEVICE void kk_ring_products(const Args &a, const Tile &t, int half, int first_row, int sums, uint8_t *lds, int &slot) {
   typedef KKRingShape<XDT, MF> S;
   const int strip = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave) & 3, lane = threadIdx.x % kWave;
   const int c32 = lane % 32, h = lane / 32, n_k = (a.K + S::KS - 1) / S::KS;
@@ -267,8 +274,22 @@ TAMD_DEVICE void kk_ring_products(const Args &a, const Tile &t, int half, int fi
     for (int f = 0; f < NF; ++f)
 #pragma unroll
       for (int j = 0; j < 16; ++j) acc[i][f][j] = 0.f;
-#pragma unroll 1
-  for (int p = 0; p < n_k; ++p) {
+  f32x16_t other[S::TWO ? NFR : 1][NF];   // of the upper halves of the stages, or of the parts that are through
+  if constexpr (S::TWO) {
+#pragma unroll
+    for (int i = 0; i < NFR; ++i)
+#pragma unroll
+      for (int f = 0; f < NF; ++f) other[i][f] = acc[i][f];
+  }
+  auto add = [&](f32x16_t (&to)[NFR][NF], const f32x16_t (&from)[NFR][NF]) {
+#pragma unroll
+    for (int i = 0; i < NFR; ++i)
+#pragma unroll
+      for (int f = 0; f < NF; ++f)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) to[i][f][j] += from[i][f][j];
+  };
+  auto stage = [&](auto halves) {
     sync_threads();
     const uint32_t buf = (uint32_t)slot * S::STAGE;
     slot = slot + 1 == S::RING ? 0 : slot + 1;
@@ -288,7 +309,37 @@ TAMD_DEVICE void kk_ring_products(const Args &a, const Tile &t, int half, int fi
 #pragma unroll
       for (int i = 0; i < NFR; ++i)
 #pragma unroll
-        for (int f = 0; f < NF; ++f) acc[i][f] = S::M::mma(af[v & 1][i], bf[v & 1][f], acc[i][f]);
+        for (int f = 0; f < NF; ++f) {
+          f32x16_t &to = halves.value && v >= 2 ? other[S::TWO ? i : 0][f] : acc[i][f];
+          to = S::M::mma(af[v & 1][i], bf[v & 1][f], to);
+        }
+    }
+  };
+  if (S::TWO && sums == 2) {
+    if constexpr (S::TWO) {
+#pragma unroll 1
+      for (int p = 0; p < n_k; ++p) stage(std::true_type{});
+      add(acc, other);
+    }
+  } else {
+    const int n_part = (n_k + sums - 1) / sums;
+    int left = n_part;
+#pragma unroll 1
+    for (int p = 0; p < n_k; ++p) {
+      stage(std::false_type{});
+      if constexpr (S::TWO) {
+        if (--left == 0 && p + 1 < n_k) {
+          left = n_part;
+          add(other, acc);
+#pragma unroll
+          for (int i = 0; i < NFR; ++i)
+#pragma unroll
+            for (int f = 0; f < NF; ++f) acc[i][f] = f32x16_t{};
+        }
+      }
+    }
+    if constexpr (S::TWO) {
+      if (sums > 1) add(acc, other);
     }
   }
   // The waves of a half write the same table; all of them have passed a barrier since the last tile's was read.
@@ -302,7 +353,7 @@ TAMD_DEVICE void kk_ring_products(const Args &a, const Tile &t, int half, int fi
 
 // Multiplying waves: two halves of the tile's row fragments, four strips.
 template <int XDT, int MF, int ACT, typename Args>
-TAMD_DEVICE void kk_ring_compute(const Args &a, uint8_t *lds) {
+TAMD_DEVICE void kk_ring_compute(const Args &a, int sums, uint8_t *lds) {
   typedef KKRingShape<XDT, MF> S;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), strip = wave & 3, half = wave >> 2;
   const int n_k = (a.K + S::KS - 1) / S::KS;
@@ -326,21 +377,21 @@ TAMD_DEVICE void kk_ring_compute(const Args &a, uint8_t *lds) {
       for (int p = 0; p < n_k; ++p) sync_threads();
       slot = (slot + n_k) % S::RING;
     } else if (S::N0 == 1 || mine == 1) {
-      kk_ring_products<XDT, MF, 1, ACT>(a, t, half, first_row, lds, slot);
+      kk_ring_products<XDT, MF, 1, ACT>(a, t, half, first_row, sums, lds, slot);
     } else if (S::N0 == 2 || mine == 2) {
-      kk_ring_products<XDT, MF, (S::N0 < 2 ? S::N0 : 2), ACT>(a, t, half, first_row, lds, slot);
+      kk_ring_products<XDT, MF, (S::N0 < 2 ? S::N0 : 2), ACT>(a, t, half, first_row, sums, lds, slot);
     } else {
-      kk_ring_products<XDT, MF, S::N0, ACT>(a, t, half, first_row, lds, slot);
+      kk_ring_products<XDT, MF, S::N0, ACT>(a, t, half, first_row, sums, lds, slot);
     }
   }
 }
 
 template <int XDT, int MF, int ACT>
-__global__ __launch_bounds__((KKRingShape<XDT, MF>::THREADS), 1) void mm_kk_ring_kernel(tamd_matmul_args, int group, int nt) {
+__global__ __launch_bounds__((KKRingShape<XDT, MF>::THREADS), 1) void mm_kk_ring_kernel(tamd_matmul_args, int group, int nt, int sums) {
   extern __shared__ __attribute__((aligned(128))) uint8_t lds_ring[];
   // (the arguments are read where they are used, see kernel_args_late)
   if (threadIdx.x >= KKRingShape<XDT, MF>::CONSUMERS * kWave) kk_ring_copy<XDT, MF>(kernel_args_late(), group, nt != 0, lds_ring);
-  else kk_ring_compute<XDT, MF, ACT>(kernel_args_late(), lds_ring);
+  else kk_ring_compute<XDT, MF, ACT>(kernel_args_late(), sums, lds_ring);
 }
 
 template <int XDT, int MF, int ACT>
@@ -356,7 +407,7 @@ int launch_kk_ring(const tamd_matmul_args &a, hipStream_t st) {
   if (int rc = raise_lds_limit_once((const void *)kern)) return rc;
   const bool lines = aligned(a.w, 128) && (a.w_stride_n * 2) % 128 == 0 && (a.w_stride_e * 2) % 128 == 0;
   const bool nt = lines && live_slices(a) * a.N * ((double)a.K * 2) >= 320.0 * (1 << 20);
-  kern<<<dim3((unsigned)wgs), S::THREADS, S::LDS, st>>>(a, (int)group, (int)nt);
+  kern<<<dim3((unsigned)wgs), S::THREADS, S::LDS, st>>>(a, (int)group, (int)nt, S::TWO ? kk_ring_sums(a, cus) : 1);
   return launch_status();
 }
 

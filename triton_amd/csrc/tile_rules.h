@@ -205,15 +205,23 @@ inline bool kk_ring_applicable(const tamd_matmul_args &a) {
 // 0.84 of the time in the mean, 14 above 1.05 (1.10 at most); layer of 102 rows for each of 8 slices, f16, 5376 -> 992, 112 -> 93 us.  Under four
 // rows per slice up to 1.9; half a line further down 0.93 to 1.25, 2.1 at worst.  Just above the line blocks of 64 for up to 128
 // rows per slice take 0.84 to 0.9 of what those of 160 do; from 1.3 thirds on up to 1.5.
+inline double kk_ring_thirds(const tamd_matmul_args &a, int cus) {
+  const double mean = (double)a.M / a.n_experts, tiles = live_slices(a) * ((a.N + 255) / 256) / cus;
+  return 3.0 * tiles * (mean > 160.0 ? mean / 160.0 : 1.0);
+}
 inline int kk_ring_rows(const tamd_matmul_args &a, int cus) {
   if (!kk_ring_applicable(a)) return 0;
   // (the line below, whichever slices the rows fall on)
   if (a.M <= a.n_experts && 3 * (int64_t)most_live_slices(a) * ((a.N + 255) / 256) < cus) return 0;
-  const double mean = (double)a.M / a.n_experts, tiles = live_slices(a) * ((a.N + 255) / 256) / cus;
-  const double thirds = 3.0 * tiles * (mean > 160.0 ? mean / 160.0 : 1.0);
+  const double mean = (double)a.M / a.n_experts, thirds = kk_ring_thirds(a, cus);
   if (thirds < 1.0) return mean >= 4.0 && thirds >= (mean < 32.0 ? 0.9 : mean < 48.0 ? 0.6 : mean < 128.0 ? 0.5 : 0.4) ? 64 : 0;
   return mean <= 48.0 || (mean < 128.0 && thirds < 1.15) ? 64 : 160;
 }
+
+// Float32 sums that a result of a block of 64 rows is made of: below the line no fewer than in the tiled kernels, which products take there otherwise.
+// Two, of the halves of every stage, are those of their wide tiles to the bit; four, of the quarters of K, those of the narrow tiles, which only
+// products of more than ten stages take.  Above the line one, as in blocks of 160.
+inline int kk_ring_sums(const tamd_matmul_args &a, int cus) { return kk_ring_thirds(a, cus) >= 1.0 ? 1 : a.K <= 640 ? 2 : 4; }
 
 // Row block size of a dense / batched problem: the block whose tiles take the fewest rounds over the CUs, weighted with what a
 // tile of it takes, of one of 128 rows: `weight` (in percent) for 64 and 32 rows, `slots` tiles at the speed of one round.
