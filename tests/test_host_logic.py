@@ -325,3 +325,42 @@ def test_dense_blocks_of_mxfp4_weights(M, N, K, rows, block_m):
 def test_dense_blocks_of_few_rounds_in_the_block_layout():
     assert dense_block_m(3337, 4768, 608, "BF16", "MXFP4", blocks=True) == 64
     assert dense_block_m(3337, 4768, 608, "BF16", "MXFP4") == 128
+
+
+def _fake_native(monkeypatch, before_look_up):
+    """`routing` without a GPU: the look-up of the native call, and what another thread does just before it."""
+    import importlib
+
+    from triton_amd import _lib, _native
+    module = importlib.import_module("triton_amd.routing")
+
+    def native(logits, k, layouts):
+        before_look_up(module)
+        lay = layouts.get((*logits.shape, k, _lib.dtype_code(logits.dtype)))
+        return None if lay is None else (torch.empty(lay["ws"][0] + 1), lay)
+    monkeypatch.setattr(_native, "routing", native)
+    monkeypatch.setattr(_lib, "require_gpu", lambda t, name: None)
+    module._layouts.clear()
+    return module
+
+
+def test_routing_while_another_thread_drops_the_layouts(monkeypatch):
+    module = _fake_native(monkeypatch, lambda m: m._layouts.clear())
+    r = module.routing(torch.zeros(3, 8), 2)
+    assert r._lay["shape"] == (3, 2) and r._lay["dims"][0] == 8
+    module._layouts.clear()
+
+
+def test_routing_keeps_what_is_still_asked_for(monkeypatch):
+    """Of very many shapes, one that every other call has is laid out once, however often old ones are dropped; no more than 1024 are held."""
+    module = _fake_native(monkeypatch, lambda m: None)
+    module._dropped.clear()
+    made, lay_out = [], module._arena_layout
+    monkeypatch.setattr(module, "_arena_layout", lambda *shape: made.append(shape) or lay_out(*shape))
+    for T in range(2, 1800):
+        module.routing(torch.zeros(1, 8), 2)
+        module.routing(torch.zeros(T, 8), 2)
+        assert len(module._layouts) + len(module._dropped) <= 1024
+    assert sum(shape[0] == 1 for shape in made) == 1
+    module._layouts.clear()
+    module._dropped.clear()

@@ -7,6 +7,7 @@ one int32 arena that holds every output and the kernels' workspace; its layout i
 tensors of the result are views of that arena, built when they are first asked for (the index arrays and ragged tables
 together, in one call): at these sizes the host time of this function is what a step waits for."""
 import struct
+import threading
 
 import torch
 
@@ -126,7 +127,10 @@ def _int_tables(lay):
                        *line("gather"), *line("col_sorted"), *line("row_sorted"))
 
 
-_layouts = {}  # (T, E, k, type code) -> _arena_layout: the native call looks them up
+# (T, E, k, type code) -> _arena_layout: the native call looks the first up; the second holds up to 512 that the first dropped, of
+# which those that are still asked for come back
+_layouts, _dropped = {}, {}
+_publishing = threading.Lock()
 
 
 def _arena_layout(T: int, E: int, k: int, vals_dtype: torch.dtype):
@@ -167,19 +171,25 @@ def routing(logits: torch.Tensor, n_expts_act: int, y_indx=None) -> RoutingResul
 
 
 def _routing_first_call(logits, k):
-    """The first call of a shape: checks, the arena's layout, then what `_native.routing` answers; None for strided logits."""
+    """A call of a shape that is not among `_layouts`: checks, the arena's layout, then what `_native.routing` answers; None for
+    strided logits."""
     if logits.stride(1) != 1:
         return None
     _lib.require_gpu(logits, "logits")
     assert logits.ndim == 2 and logits.shape[1] < 32768
     T, E = logits.shape
     code = _lib.dtype_code(logits.dtype)  # (refuses other types before the layout divides by their size)
-    lay = _arena_layout(T, E, k, logits.dtype)
-    if len(_layouts) >= 512:
-        _layouts.clear()
-    _layouts[T, E, k, code] = lay
-    done = _native.routing(logits, k, _layouts)
+    key = T, E, k, code
+    lay = _dropped.get(key) or _arena_layout(T, E, k, logits.dtype)
+    done = _native.routing(logits, k, {key: lay})   # (handed over: another thread may clear what is published)
     assert done is not None, "k must be an int and logits of a floating type"
+    if type(done) is tuple:
+        with _publishing:
+            if len(_layouts) >= 512:
+                _dropped.clear()
+                _dropped.update(list(_layouts.items())[-512:])
+                _layouts.clear()
+            _layouts[key] = lay
     return done
 
 
