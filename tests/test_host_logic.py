@@ -364,3 +364,21 @@ def test_routing_keeps_what_is_still_asked_for(monkeypatch):
     assert sum(shape[0] == 1 for shape in made) == 1
     module._layouts.clear()
     module._dropped.clear()
+
+
+def test_tables_asked_for_under_inference_mode_are_ordinary():
+    """One call makes all tables: what the mode was when the first was asked for must not decide what may be done with the others."""
+    import struct
+
+    from triton_amd import _native
+    base = torch.arange(64, dtype=torch.int32)
+    numbers = struct.pack("10q", 0, 4, 1, -1, 0, 16, 2, 8, 5, 1)
+    with torch.inference_mode():
+        line, table = _native.int_views(base, numbers)
+    line.add_(1)
+    assert line.tolist() == [1, 2, 3, 4] and base[:4].tolist() == [1, 2, 3, 4] and table.tolist() == [list(range(16, 21)), list(range(24, 29))]
+    with torch.inference_mode():
+        of_inference = torch.arange(64, dtype=torch.int32)
+    line, table = _native.int_views(of_inference, numbers)
+    table.mul_(2)
+    assert not line.is_inference() and table[0].tolist() == [32, 34, 36, 38, 40] and not torch.is_inference_mode_enabled()

@@ -13,6 +13,7 @@
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <c10/core/InferenceMode.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/DynamicTypes.h>
 #include <torch/csrc/Dtype.h>
@@ -547,6 +548,8 @@ PyObject *py_int_views(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
     const at::Tensor &t = tensor(v[0]);
     constexpr size_t kEach = 5 * sizeof(int64_t);
     const Py_ssize_t n = PyBytes_GET_SIZE(v[1]) / (Py_ssize_t)kEach;
+    // (ordinary tensors also under inference mode: who asks for one of them there may write to another, or save it for a backward pass, later)
+    const c10::InferenceMode ordinary(false);
     Ref all(PyTuple_New(n));
     if (!all.p) return nullptr;
     for (Py_ssize_t i = 0; i < n; ++i) {
