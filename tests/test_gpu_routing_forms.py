@@ -4,6 +4,7 @@ import pytest
 import torch
 
 from oracle import routing_ref as RR
+from triton_amd import _lib
 from triton_amd.routing import routing
 
 pytestmark = pytest.mark.gpu
@@ -36,3 +37,23 @@ def test_forms(T, E, k, dtype, device):
         assert int(md.block_offs(b)[E]) == int(n.sum())
         want = torch.cat([torch.arange(int(c)) * 65536 + e for e, c in enumerate(n)])
         assert torch.equal(md.block_schedule(b)[: len(want)].cpu().long(), want.long())
+
+
+@pytest.mark.parametrize("T,E,k", [(64, 128, 4), (65, 128, 4), (128, 128, 8), (256, 16, 8), (200, 40, 5), (64, 256, 32), (32, 512, 64)])
+def test_without_a_workspace(T, E, k, device):
+    """The C entry up to twice the rows that 1024 threads hold: what it writes with a workspace."""
+    logits = torch.randn(T, E, generator=torch.Generator().manual_seed(T + E)).to(device)
+    r = routing(logits, k)
+    (_, width, po, ps), (n_words, pad_t) = r._lay["dims"], r._lay["bits_shape"]
+    i32 = lambda *shape: torch.full(shape, -7, dtype=torch.int32, device=device)
+    vals, indx, bits = torch.empty(T, k, device=device), torch.empty(T, k, dtype=torch.int16, device=device), i32(n_words, pad_t)
+    col_sum, col_sorted, row_sorted, gather, offs, sched = i32(E), i32(T * k), i32(T * k), i32(T * k), i32(6, po), i32(5, ps)
+    ptr = _lib.ptr
+    rc = _lib.lib().tamd_routing(ptr(logits), _lib.F32, E, T, E, k, ptr(vals), ptr(indx), ptr(bits), 1, pad_t, ptr(col_sum), ptr(col_sorted),
+                                 ptr(row_sorted), ptr(gather), ptr(offs), po, ptr(sched), ps, width, None, _lib.stream_ptr(device))
+    assert rc == 0
+    md = r.ragged_metadata
+    assert torch.equal(indx, r.indx) and torch.equal(vals, r.vals) and torch.equal(bits[:, :T], r._mask_words.t()[:, :T])
+    assert torch.equal(col_sum, r.col_sum) and torch.equal(col_sorted, r.scatter_indx) and torch.equal(row_sorted, r.row_sorted_indx)
+    assert torch.equal(gather, r.gather_indx) and torch.equal(offs[0, :E + 1], md.slice_offs) and torch.equal(offs[1:, :E + 1], md.block_offs_data)
+    assert torch.equal(sched[:, :width], md.block_schedule_data)

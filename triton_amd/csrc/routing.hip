@@ -1328,6 +1328,28 @@ bool ragged_between(void *p) {
 }
 }  // namespace
 
+// One workgroup does it all, without a workspace, where the per-chunk histogram fits its LDS; false where it does not.  (Beyond about 4096
+// entries one CU is slower than three launches.)
+static bool metadata_by_one_workgroup(const void *indx, int indx_is_int16, int64_t n_indx, int n_cols, int k, int32_t *col_sum,
+                                      int32_t *col_sorted_indx, int32_t *row_sorted_indx, int32_t *gather_indx, int32_t *offs,
+                                      int64_t offs_pitch, int32_t *schedule, int64_t sched_pitch, int max_n_blocks, Gates gates,
+                                      hipStream_t st, int &rc) {
+  const int64_t NC = (n_indx + 63) / 64 > 0 ? (n_indx + 63) / 64 : 1;
+  int64_t P = 1024 / n_cols;
+  P = P < 1 ? 1 : (P > NC ? NC : P);
+  const int64_t ints = NC * n_cols + (int64_t)n_cols + P * n_cols + 6 * (int64_t)(n_cols + 1);
+  if (NC > 64 || ints * 4 > 156 * 1024) return false;
+  int nbits = 0;
+  while ((1 << nbits) < n_cols) ++nbits;
+  rc = raise_lds_limit_once((const void *)meta_fused_kernel);
+  if (rc != 0) return true;
+  meta_fused_kernel<<<1, 1024, (size_t)ints * 4, st>>>(indx, indx_is_int16, (int)n_indx, n_cols, k, nbits, (int)NC, (int)P, col_sum,
+                                                       col_sorted_indx, row_sorted_indx, gather_indx, offs, offs_pitch, schedule,
+                                                       sched_pitch, max_n_blocks, gates);
+  rc = launch_status();
+  return true;
+}
+
 static int routing_metadata_impl(const void *indx, int indx_is_int16, int64_t n_indx, int n_cols, int k,
                                  int32_t *col_sum, int32_t *col_sorted_indx, int32_t *row_sorted_indx,
                                  int32_t *gather_indx, int32_t *offs, int64_t offs_pitch, int32_t *schedule,
@@ -1336,22 +1358,10 @@ static int routing_metadata_impl(const void *indx, int indx_is_int16, int64_t n_
   if (max_n_blocks < 0 || offs_pitch < n_cols + 1 || sched_pitch < max_n_blocks) return TAMD_E_INVALID;
   if (!col_sum || !workspace || !offs || (max_n_blocks > 0 && !schedule)) return TAMD_E_INVALID;
   if (n_indx > 0 && (!indx || !col_sorted_indx || !row_sorted_indx)) return TAMD_E_INVALID;
-  {
-    // one workgroup does it all when the per-chunk histogram fits its LDS
-    const int64_t NC = (n_indx + 63) / 64 > 0 ? (n_indx + 63) / 64 : 1;
-    int64_t P = 1024 / n_cols;
-    P = P < 1 ? 1 : (P > NC ? NC : P);
-    const int64_t ints = NC * n_cols + (int64_t)n_cols + P * n_cols + 6 * (int64_t)(n_cols + 1);
-    if (NC <= 64 && ints * 4 <= 156 * 1024) {  // beyond ~4096 entries one CU is slower than three launches
-      int nbits = 0;
-      while ((1 << nbits) < n_cols) ++nbits;
-      if (int rc = raise_lds_limit_once((const void *)meta_fused_kernel)) return rc;
-      meta_fused_kernel<<<1, 1024, (size_t)ints * 4, (hipStream_t)stream>>>(
-          indx, indx_is_int16, (int)n_indx, n_cols, k, nbits, (int)NC, (int)P, col_sum, col_sorted_indx, row_sorted_indx,
-          gather_indx, offs, offs_pitch, schedule, sched_pitch, max_n_blocks, gates);
-      return launch_status();
-    }
-  }
+  int one_rc = 0;
+  if (metadata_by_one_workgroup(indx, indx_is_int16, n_indx, n_cols, k, col_sum, col_sorted_indx, row_sorted_indx, gather_indx, offs,
+                                offs_pitch, schedule, sched_pitch, max_n_blocks, gates, (hipStream_t)stream, one_rc))
+    return one_rc;
   {
     // two launches while the table of block histograms is small enough for every workgroup to reduce by itself
     const MetaPlan p = make_meta_plan(n_indx, n_cols);
@@ -1434,6 +1444,13 @@ extern "C" int tamd_routing_gates(const void *logits, int dtype, int64_t stride,
       if (dtype == TAMD_BF16) TAMD_RFD(TAMD_BF16);
       TAMD_RFD(TAMD_F16);
 #undef TAMD_RFD
+    }
+    // Up to twice as many rows a caller may leave the workspace out.
+    if (!workspace && n_rows <= 2 * (1024 / L)) {
+      int rc = tamd_topk_forward(logits, dtype, stride, n_rows, n_cols, k, 1, 0, y_vals, y_indx, k, bits, bits_stride_row, bits_stride_word, stream);
+      if (rc != 0) return rc;
+      return metadata_by_one_workgroup(y_indx, 1, n, n_cols, k, col_sum, col_sorted_indx, row_sorted_indx, gather_indx, offs, offs_pitch,
+                                       schedule, sched_pitch, max_n_blocks, gates, st, rc) ? rc : TAMD_E_INVALID;
     }
     RowPlan plan;
     if (workspace && make_row_plan(n_rows, n_cols, k, L, tamd_bitmatrix_metadata_workspace(n, n_cols), plan)) {
