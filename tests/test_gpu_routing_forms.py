@@ -57,3 +57,19 @@ def test_without_a_workspace(T, E, k, device):
     assert torch.equal(col_sum, r.col_sum) and torch.equal(col_sorted, r.scatter_indx) and torch.equal(row_sorted, r.row_sorted_indx)
     assert torch.equal(gather, r.gather_indx) and torch.equal(offs[0, :E + 1], md.slice_offs) and torch.equal(offs[1:, :E + 1], md.block_offs_data)
     assert torch.equal(sched[:, :width], md.block_schedule_data)
+
+
+@pytest.mark.parametrize("E", [31, 33, 127, 384, 512])
+@pytest.mark.parametrize("k", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_few_picks(E, k, dtype, device):
+    """A lane sorts only as many of its keys as it can give: rows whose picks all come from one lane, equal ones among them."""
+    T, L = 700, 8 if E <= 64 else 16 if E <= 128 else 64
+    g = torch.Generator().manual_seed(E + k)
+    logits = torch.randn(T, E, generator=g)
+    lane = torch.randint(0, L, (T, 1), generator=g)
+    own = torch.arange(E)[None, :] % L == lane
+    logits = torch.where(own, 4 + torch.randint(0, 3, (T, E), generator=g).float(), logits).to(dtype)
+    r, ref = routing(logits.to(device), k), RR.routing_ref(logits, k)
+    assert torch.equal(r.indx.cpu().int(), ref["indx"].int()) and torch.equal(r.col_sum.cpu(), ref["col_sum"])
+    assert torch.equal(r.scatter_indx.cpu(), ref["scatter_indx"])
