@@ -382,3 +382,13 @@ def test_tables_asked_for_under_inference_mode_are_ordinary():
     line, table = _native.int_views(of_inference, numbers)
     table.mul_(2)
     assert not line.is_inference() and table[0].tolist() == [32, 34, 36, 38, 40] and not torch.is_inference_mode_enabled()
+
+
+def test_where_two_launches_route():
+    """Not where their workgroups pass over many rows and leave the chip idle, nor where these are more than one round and a row gives few entries."""
+    from triton_amd._native import routing_block_rows as rows
+    assert rows(4096, 128, 4) == 32 and rows(3000, 512, 8) == 32 and rows(32768, 256, 1) == 128 and rows(65535, 8, 1) and rows(40000, 40, 1)
+    assert rows(65536, 8, 1) == 0 and rows(1000, 513, 1) == 0 and rows(0, 8, 1) == 0
+    assert all(rows(T, E, k) == 0 for T, E in ((5000, 257), (10000, 384), (65535, 512)) for k in (1, 4, 16))
+    assert all(rows(T, E, k) == 0 for T, E in ((32769, 128), (32769, 256), (65535, 200)) for k in (1, 2, 3))
+    assert all(rows(T, E, k) for T, E in ((32769, 128), (32769, 256), (65535, 200)) for k in (4, 8)) and rows(65535, 60, 40)

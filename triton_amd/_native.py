@@ -51,6 +51,6 @@ def _on_first_call(name):
 
 
 _FUNCTIONS = ("matmul", "routing", "view", "int_views", "reduce", "downcast", "upcast", "choose_block_m", "blocks_of_16_stream",
-              "dense_block_m", "ring_rows")
+              "dense_block_m", "ring_rows", "routing_block_rows")
 for _n in _FUNCTIONS:
     globals()[_n] = _on_first_call(_n)

@@ -745,6 +745,17 @@ PyObject *py_ring_rows(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
   });
 }
 
+// (rows, experts, picks per row): rows to a workgroup of the routing's two launches, 0 where others take them.
+PyObject *py_routing_block_rows(PyObject *, PyObject *const *v, Py_ssize_t nargs) {
+  return covered([&]() -> PyObject * {
+    need(nargs == 3);
+    const int64_t T = as_int(v[0]), E = as_int(v[1]), k = as_int(v[2]);
+    need(E >= 1 && k >= 1 && k <= 64 && k <= E && E <= 1 << 20);
+    tamd::RowPlan p;
+    return PyLong_FromLong(tamd::make_row_plan(T, (int)E, (int)k, tamd::lanes_per_row((int)E, (int)k), INT64_MAX, p) ? p.RB : 0);
+  });
+}
+
 // (addresses of the C ABI functions by name, Tensor, CDNA4MXValueLayout, CDNA4MXScaleLayout, FP4, constraints ContextVar,
 //  flags ContextVar)
 PyObject *py_init(PyObject *, PyObject *args) {
@@ -783,6 +794,7 @@ PyMethodDef methods[] = {{"init", py_init, METH_VARARGS, nullptr},
                          {"routing", TAMD_FAST(py_routing)},
                          {"view", TAMD_FAST(py_view)},
                          {"int_views", TAMD_FAST(py_int_views)},
+                         {"routing_block_rows", TAMD_FAST(py_routing_block_rows)},
                          {"reduce", TAMD_FAST(py_reduce)},
                          {"downcast", TAMD_FAST(py_downcast)},
                          {"upcast", TAMD_FAST(py_upcast)},

@@ -792,10 +792,9 @@ inline int launch_order_scan(const void *indx, int is16, int64_t n, int E, int C
 // ---------------------------------------------------------------------------
 // routing from the logits in two launches
 // ---------------------------------------------------------------------------
-// A row picks an expert at most once.  So a block of up to 255 rows counts its entries per expert in a byte, and the place of
+// A row picks an expert at most once.  So a block of rows (kMaxRowsPerBlock) counts its entries per expert in a byte, and the place of
 // an entry among those of its expert is the number of earlier rows that picked it: bits of a mask with one bit per row
 // and expert, set in LDS in any order, and counted.  No ballots per chunk, no prefix sums over chunks.
-constexpr int kMaxRowsPerBlock = 255;
 
 // i / k for i * k < 2^19, k <= 64: i * reciprocal_of(k) >> 19 (the reciprocal is too large by at most k / 2^19).
 inline uint32_t reciprocal_of(int k) { return (1u << 19) / (uint32_t)k + 1u; }
@@ -949,36 +948,6 @@ __global__ __launch_bounds__(1024) void order_rows_kernel(const int16_t *__restr
     const int64_t begin = per * (blk - nbo);
     if (begin < total) ragged_fill_schedule(tab, E, sched, sched_pitch, max_blocks, begin, per < total - begin ? per : total - begin);
   }
-}
-
-// How the two launches cut n_rows rows.
-struct RowPlan {
-  int TH, RB, pitch, lg_cols, nb, sub, nbo, W;
-  size_t lds;
-};
-
-// Fills the plan, or returns false where the table or the counts do not fit.  The workgroups of the first launch are the smallest whose table
-// is read with four loads per thread (16 KB); a longer input makes the blocks larger, up to 255 rows.
-inline bool make_row_plan(int64_t n_rows, int E, int k, int L, int64_t workspace_ints, RowPlan &p) {
-  if (n_rows < 1 || n_rows > 65535 || E > 512) return false;
-  p.pitch = 16;
-  while (p.pitch < E) p.pitch *= 2;
-  p.lg_cols = __builtin_ctz(p.pitch / 4);
-  p.TH = 256;
-  while (p.TH < 1024 && (n_rows + p.TH / L - 1) / (p.TH / L) * p.pitch > 16384) p.TH *= 2;
-  p.RB = p.TH / L;
-  while (2 * p.RB <= kMaxRowsPerBlock && (n_rows + p.RB - 1) / p.RB * p.pitch > 65536) p.RB *= 2;
-  p.nb = (int)((n_rows + p.RB - 1) / p.RB);
-  if ((int64_t)p.nb * (p.pitch / 4) > workspace_ints) return false;
-  p.sub = 1;
-  while (p.RB * p.sub * 2 * k <= 1024 && p.RB * p.sub * 2 <= 128 && p.sub < p.nb) p.sub *= 2;
-  p.nbo = (p.nb + p.sub - 1) / p.sub;
-  p.W = (p.RB * p.sub + 31) / 32;
-  if ((int64_t)p.RB * p.sub * k * k >= 1 << 19) return false;  // over_k
-  const int64_t waves = p.RB * p.sub * k >= 1024 ? 16 : (p.RB * p.sub * k + kWave - 1) / kWave;
-  const int64_t copies = waves * E > 6 * (E + 1) ? waves * E : 6 * (E + 1);
-  p.lds = (size_t)(p.pitch + (int64_t)E * p.W + copies) * 4;
-  return p.lds <= 150 * 1024;
 }
 
 template <int DT>
@@ -1440,9 +1409,7 @@ extern "C" int tamd_routing_gates(const void *logits, int dtype, int64_t stride,
       (dtype == TAMD_F32 || dtype == TAMD_BF16 || dtype == TAMD_F16) && col_sum && offs && col_sorted_indx &&
       row_sorted_indx && max_n_blocks >= 0 && offs_pitch >= n_cols + 1 && sched_pitch >= max_n_blocks &&
       (max_n_blocks == 0 || schedule)) {
-    int need = (n_cols + 7) / 8;
-    if (need < k) need = k;
-    const int L = need <= 8 ? 8 : (need <= 16 ? 16 : (need <= 32 ? 32 : 64));
+    const int L = lanes_per_row(n_cols, k);
     const int64_t n = (int64_t)n_rows * k;
     hipStream_t st = (hipStream_t)stream;
     // One launch where 1024 threads hold the rows: also at the line it is the faster (64 rows of 128: 5.9 us against 7.5 in

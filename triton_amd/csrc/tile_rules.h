@@ -1,4 +1,4 @@
-// Which kernel and which row block a product takes: rules on the arguments alone, shared by the kernels' launchers and the host path
+// Which kernel and which row block a product or a routing takes: rules on the arguments alone, shared by the kernels' launchers and the host path
 // (no HIP here).
 #pragma once
 #include <math.h>
@@ -259,6 +259,53 @@ inline int dense_block_m(const tamd_matmul_args &a, int cus) {
     if (best == 0 || cost < least) best = bm[i], least = cost;
   }
   return best;
+}
+
+// ---------------------------------------------------------------------------
+// routing
+// ---------------------------------------------------------------------------
+// Lanes that share a row of up to 512 logits, eight of them or fewer each, a lane for every pick.
+inline int lanes_per_row(int n_cols, int k) {
+  const int need = (n_cols + 7) / 8 > k ? (n_cols + 7) / 8 : k;
+  return need <= 8 ? 8 : (need <= 16 ? 16 : (need <= 32 ? 32 : 64));
+}
+
+// How the two launches of the routing (routing.hip) cut n_rows rows: blocks of RB rows, TH threads each.
+struct RowPlan {
+  int TH, RB, pitch, lg_cols, nb, sub, nbo, W;
+  size_t lds;
+};
+constexpr int kMaxRowsPerBlock = 128;   // (a byte would count 255; RB is a power of two)
+
+// Fills the plan, or returns false where the table or the counts do not fit or the older launches are the faster: more than 65535 rows (the sums of
+// the table's bytes have 16 bits), more than 512 experts, and the two lines below.  The workgroups of the first launch are the smallest whose
+// table is read with four loads per thread (16 KB); a longer input makes the blocks larger, so that a workgroup passes over its rows several times.
+// There the chip idles: above 256 experts, 16 rows to a pass, from four passes on (79 workgroups for 10000 rows; k 1 1.32 to 1.41 of the other
+// launches' time, k 8 1.57 to 1.68, 24000 rows 1.02 to 1.06 and 0.90 to 0.93, two passes 0.44 to 1.06); below, where the workgroups no longer are one
+// round over 256 CUs (from 32769 rows) and a row gives fewer than four entries to place (200 experts, 33000 rows, k 1 1.35, k 2
+// 1.38, k 4 1.07, k 8 1.02; 65000 1.27, 1.25, 0.91, 0.82; 128 experts 1.14, 1.15, 0.82, 0.76 and 1.09, 1.13, 0.72, 0.63).
+inline bool make_row_plan(int64_t n_rows, int E, int k, int L, int64_t workspace_ints, RowPlan &p) {
+  if (n_rows < 1 || n_rows > 65535 || E > 512) return false;
+  p.pitch = 16;
+  while (p.pitch < E) p.pitch *= 2;
+  p.lg_cols = __builtin_ctz(p.pitch / 4);
+  p.TH = 256;
+  while (p.TH < 1024 && (n_rows + p.TH / L - 1) / (p.TH / L) * p.pitch > 16384) p.TH *= 2;
+  p.RB = p.TH / L;
+  while (2 * p.RB <= kMaxRowsPerBlock && (n_rows + p.RB - 1) / p.RB * p.pitch > 65536) p.RB *= 2;
+  p.nb = (int)((n_rows + p.RB - 1) / p.RB);
+  const int passes = p.RB / (p.TH / L);
+  if (E > 256 ? passes >= 4 : passes > 1 && p.nb > 256 && k < 4) return false;
+  if ((int64_t)p.nb * (p.pitch / 4) > workspace_ints) return false;
+  p.sub = 1;
+  while (p.RB * p.sub * 2 * k <= 1024 && p.RB * p.sub * 2 <= 128 && p.sub < p.nb) p.sub *= 2;
+  p.nbo = (p.nb + p.sub - 1) / p.sub;
+  p.W = (p.RB * p.sub + 31) / 32;
+  if ((int64_t)p.RB * p.sub * k * k >= 1 << 19) return false;  // over_k
+  const int64_t waves = p.RB * p.sub * k >= 1024 ? 16 : (p.RB * p.sub * k + 64 - 1) / 64;
+  const int64_t copies = waves * E > 6 * (E + 1) ? waves * E : 6 * (E + 1);
+  p.lds = (size_t)(p.pitch + (int64_t)E * p.W + copies) * 4;
+  return p.lds <= 150 * 1024;
 }
 
 }  // namespace tamd
