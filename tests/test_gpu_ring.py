@@ -63,6 +63,15 @@ def test_where_blocks_of_96_come_before_tiles():
     assert ring_rows(6168, 2688, 1248, 32, "bf16", "16", True) == 0 and ring_rows(6168, 2688, 640, 32, "mxfp8", "mx", True) == 0
 
 
+def test_where_one_round_of_tiles_is_full():
+    """Products timed at 1.05 to 1.29 of the tiles' time: a tile of 128 for every slice, two to a CU, is one round."""
+    for m, n, k, e, kind, out in ((10631, 832, 2400, 128, "mxfp8", "16"), (7960, 640, 3040, 128, "fp8", "fp8"), (10356, 896, 2720, 128, "mxfp8", "mx"),
+                                  (1547, 6976, 2784, 16, "mxfp4", "16"), (10747, 1024, 1184, 128, "fp8", "fp8"), (1504, 8000, 1984, 16, "mxfp8", "16"),
+                                  (4619, 1984, 2304, 60, "mxfp8", "mx"), (1966, 3904, 2240, 32, "mxfp8", "16")):
+        assert ring_rows(m, n, k, e, kind, out, True) == 0
+        assert ring_rows(m, n * 2, k, e, kind, out, True) == 96   # (two rounds)
+
+
 def blocks(w, ws):
     return convert_layout(wrap_torch_tensor(w, dtype=FP4), CDNA4MXValueLayout()), convert_layout(wrap_torch_tensor(ws), CDNA4MXScaleLayout())
 

@@ -121,14 +121,18 @@ inline bool ring_stages_too_few(const tamd_matmul_args &a, double cover) {
 // SwiGLU products of 8- and 4-bit rows with more than 64 rows per slice: the persistent kernel's blocks of 96 against tiles of 128, by what each
 // is estimated to take (us): a start, and rounds over the CUs (two tiles of 128 to a CU) whose last is paid for in part.  The epilogue of
 // such a tile is a third of its time, which the persistent kernel hides behind the next tile's products; without SwiGLU, and from
-// about a thousand rows per slice on, tiles are the faster.  Fitted to 2300 products (8 to 128 slices of 24 to 2000 rows, K 512 to 5760); where
-// the rule takes this kernel, time over the tiles': fp8 0.957, MXFP8 0.931, packed rows 0.921, 20 of 550 above 1.05.
-inline bool ring_96_before_tiles(const tamd_matmul_args &a, int cus, double mean) {
+// about a thousand rows per slice on, tiles are the faster.  Fitted to 2300 products (8 to 128 slices of 24 to 2000 rows, K 512 to 5760, slices as
+// uneven as a router's).  900 others, a third each with even slices, 0.2 and 0.45 in the logarithm: 0.857 of the tiles' time in the mean, 38
+// above 1.05, 1.23 at worst.  25 of those have even slices: with 97 to 126 and 200 to 226 rows one tile takes what two blocks of 96 share,
+// or two what three, 1.02 in the mean and up to 1.23 (0.86 to 0.93 if slices are uneven).  Where that one round of tiles is nearly full
+// as well, 18 products took 0.75 to 1.29, 0.98 in the mean: left to the tiles.
+inline bool ring_96_before_tiles(const tamd_matmul_args &a, int cus, double mean, double cover) {
   if (a.activation != TAMD_ACT_SWIGLU || a.K < 800 || mean < 60.0 || mean > 1024.0) return false;
   const bool packed = a.x_dtype == TAMD_MXFP4, scaled = !packed && a.x_mx_scale;
   const double cols = live_slices(a) * ((a.N + 255) / 256) / cus, k = a.K / 1000.0;
   const double r = cols * fmax(1.0, mean / 96.0 + 0.5), m = cols * 0.5 * fmax(1.0, mean / 128.0 + 0.5);
   if (m < 0.75) return false;
+  if (cover <= 128.0 && cols > 1.4 && cols <= 2.0) return false;   // one round of tiles of 128, nearly full
   const double ring = 5.0 + (packed ? 3.2 + 3.5 * k : scaled ? 4.2 + 4.8 * k : 3.2 + 4.4 * k) * (r + 0.6 * (ceil(r) - r) + 0.1);
   const double tiles = 5.0 + (packed ? 5.9 + 11.1 * k : scaled ? 9.7 + 13.9 * k : 7.9 + 11.6 * k) * (m + 0.05 * (ceil(m) - m) + 0.07);
   return ring < (scaled ? 1.0 : 0.97) * tiles;
@@ -159,7 +163,7 @@ inline int ring_rows(const tamd_matmul_args &a, int cus) {
   const bool packed = a.x_dtype == TAMD_MXFP4, scaled = !packed && a.x_mx_scale;
   // (of blocks of 96 rows what the products of a layer write is built)
   const bool rows_96 = !x16 && cover > 64.0 && (a.y_dtype != TAMD_FP8_E4M3 || (a.activation == TAMD_ACT_SWIGLU && !(packed && a.y_mx_scale)));
-  if (rows_96 && ring_96_before_tiles(a, cus, mean)) return 96;
+  if (rows_96 && ring_96_before_tiles(a, cus, mean, cover)) return 96;
   if (mean > 96.0 || (a.K < 1024 && tiles > 1.0)) return 0;
   const bool alone = tiles <= 1.0;
   if (x16) {
