@@ -36,6 +36,14 @@ def test_where_it_is_taken():
         assert ring_rows(4084, 5760, 2880, 32, **changed) == 0, changed
 
 
+def test_where_blocks_of_64_are_the_slower():
+    """Products timed at 1.05 to 1.3 of the kernels that take them now."""
+    for m, n, k, e in ((412, 2328, 256, 8), (489, 1840, 384, 8), (987, 584, 392, 16), (802, 528, 336, 16)):
+        assert ring_rows(m, n, k, e) == 0 and ring_rows(m, n, k + 408, e) == 64
+    for m, n, k, e in ((992, 3048, 5608, 8), (1918, 760, 5304, 32), (548, 3064, 5712, 8), (1968, 720, 4856, 32)):
+        assert ring_rows(m, n, k, e) == 160 and ring_rows(m, n, k - 3000, e) == 64
+
+
 # (slice sizes, K, columns)
 SIZES = [([1, 0, 31, 32, 33, 64, 65, 0, 129, 3], 256, 6200), ([2] * 70 + [0] * 30, 1096, 648), ([160, 161, 0, 320, 321, 95, 97, 700], 776, 3176),
          ([1500, 0, 40], 520, 4100), ([5000], 264, 1032)]

@@ -205,10 +205,12 @@ inline bool kk_ring_applicable(const tamd_matmul_args &a) {
 // From one third on, 486 products of 1 to 16384 tokens, 8 to 128 slices, K and N 512 to 5760: 0.876 of the time in the mean (0.866 with the
 // best choice for each), none above 1.05.  Blocks of 64 up to 56 rows per slice lose up to 1.21, where slices come in two.
 // Below it tiles of one to three strips of 64 columns and blocks of 64 rows reach every CU, where the tiled kernel leaves most of them without
-// a tile: the more rows per slice, the earlier.  Of 10600 products below the line (8 to 60 slices, bf16) the 3000 that the lines take:
-// 0.84 of the time in the mean, 14 above 1.05 (1.10 at most); layer of 102 rows for each of 8 slices, f16, 5376 -> 992, 112 -> 93 us.  Under four
-// rows per slice up to 1.9; half a line further down 0.93 to 1.25, 2.1 at worst.  Just above the line blocks of 64 for up to 128
-// rows per slice take 0.84 to 0.9 of what those of 160 do; from 1.3 thirds on up to 1.5.
+// a tile: the more rows per slice, the earlier.  675 products below the line (8 to 60 slices, bf16 and f16, even slices, 0.2 and 0.45 in the
+// logarithm): 0.84 of the time in the mean; up to K 640 0.87 to 1.05, beyond 0.75 to 0.99.  Above 1.05 are 24, 1.10 at worst but for one
+// of five rows per slice (1.25), 21 of them of K up to 832; of 48 to 64 rows and K up to 400 were 16 of 40, 1.03 in the mean: not taken.  Layer
+// of 102 rows for each of 8 slices, f16, 5376 -> 992, 112 -> 93 us.  Under four rows per slice up to 1.9; half a line further down 0.93 to
+// 1.25, 2.1 at worst.  Just above the line blocks of 64 for up to 128 rows per slice take 0.88 of what those of 160 do in the mean of 125
+// products, 1.054 at worst, with K above 4096 up to 1.3; from 1.3 thirds on up to 1.5.
 inline double kk_ring_thirds(const tamd_matmul_args &a, int cus) {
   const double mean = (double)a.M / a.n_experts, tiles = live_slices(a) * ((a.N + 255) / 256) / cus;
   return 3.0 * tiles * (mean > 160.0 ? mean / 160.0 : 1.0);
@@ -218,8 +220,11 @@ inline int kk_ring_rows(const tamd_matmul_args &a, int cus) {
   // (the line below, whichever slices the rows fall on)
   if (a.M <= a.n_experts && 3 * (int64_t)most_live_slices(a) * ((a.N + 255) / 256) < cus) return 0;
   const double mean = (double)a.M / a.n_experts, thirds = kk_ring_thirds(a, cus);
-  if (thirds < 1.0) return mean >= 4.0 && thirds >= (mean < 32.0 ? 0.9 : mean < 48.0 ? 0.6 : mean < 128.0 ? 0.5 : 0.4) ? 64 : 0;
-  return mean <= 48.0 || (mean < 128.0 && thirds < 1.15) ? 64 : 160;
+  if (thirds < 1.0) {
+    if (a.K <= 400 && mean >= 48.0 && mean < 64.0) return 0;
+    return mean >= 4.0 && thirds >= (mean < 32.0 ? 0.9 : mean < 48.0 ? 0.6 : mean < 128.0 ? 0.5 : 0.4) ? 64 : 0;
+  }
+  return mean <= 48.0 || (mean < 128.0 && thirds < 1.15 && a.K <= 4096) ? 64 : 160;
 }
 
 // Float32 sums that a result of a block of 64 rows is made of: below the line no fewer than in the tiled kernels, which products take there otherwise.
