@@ -88,6 +88,19 @@ def test_tiles_of_eight_groups(shape, dtype, pitch, device):
     assert torch.equal(back.cpu(), upcast_from_mxfp_ref(rv, rs, dtype, 1))
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("N", [2056, 2048])
+def test_tiles_with_scales_of_all_kinds(dtype, N, device):
+    """More than 320 tiles, rows on lines and off them, whose groups have scales that the fast path does not take: zero, very small, NaN."""
+    g = torch.Generator().manual_seed(N)
+    v = torch.randint(0, 256, (8, 528, N), dtype=torch.uint8, generator=g)
+    s = torch.randint(100, 140, (8, 33, N), dtype=torch.uint8, generator=g)
+    s[:, 3], s[:, 5, ::7], s[:, 6, 100:300], s[:, 9, 5] = 0, 1, 255, 113
+    strided = lambda t: t.transpose(1, 2).contiguous().to(device).transpose(1, 2)
+    got, want = upcast_from_mxfp(strided(v), strided(s), dtype, axis=1).cpu(), upcast_from_mxfp_ref(v, s, dtype, 1)
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(), want.nan_to_num())
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_tiles_of_more_groups(dtype, device):
     """1040 tiles of 32 groups or 1560 of 16, the last of each matrix one group deep: from four rounds of 256 CUs on they replace those of 8."""

@@ -56,3 +56,11 @@ def test_barriers_wait_for_lds():
             assert at
             text = text[:at.start()] + text[at.end():]
         assert not bare.findall(text), path
+
+
+def test_stores_of_a_kernel_are_all_of_its_variant():
+    """A kernel whose stores are non-temporal or not by a parameter makes all of them by it, also where scales are outside the fast range."""
+    with open(os.path.join(CSRC, "mxfp.hip")) as f:
+        kernels = re.findall(r"template <int DT, int GT, bool ONCE>\n__global__.*?\n}\n", re.sub(r"//[^\n]*", "", f.read()), re.S)
+    assert len(kernels) == 2
+    assert all(not re.search(r"\b(?:store_once|store16)\s*\((?:p\b|base\b)", k) for k in kernels)

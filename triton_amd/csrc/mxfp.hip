@@ -543,17 +543,17 @@ TAMD_DEVICE void upcast_rows2_regs(const uint32_t *w, const float *mult, uint4 &
     r1 = make_uint4(hi[0], hi[1], hi[2], hi[3]);
   }
 }
+template <bool ONCE>
+TAMD_DEVICE void store_row(char *p, const uint4 &v) {
+  if (ONCE) store_once(p, v);
+  else store16((uint8_t *)p, v);
+}
 template <int DT, int BS, bool ONCE = true>
 TAMD_DEVICE void upcast_rows2(const uint32_t *w, const float *mult, char *p, int64_t pitch) {
   uint4 r0, r1;
   upcast_rows2_regs<DT, BS>(w, mult, r0, r1);
-  if (ONCE) {
-    store_once(p, r0);
-    store_once(p + pitch, r1);
-  } else {
-    store16((uint8_t *)p, r0);
-    store16((uint8_t *)p + pitch, r1);
-  }
+  store_row<ONCE>(p, r0);
+  store_row<ONCE>(p + pitch, r1);
 }
 
 // ---------------------------------------------------------------------------
@@ -639,10 +639,10 @@ __global__ __launch_bounds__(256) void upcast_cols_tile_kernel(
       }
       char *p = base + (int64_t)l * dsl * ES;
       if constexpr (DT == TAMD_F32) {
-        store_once(p, make_uint4(f32_to_bits(o[0]), f32_to_bits(o[1]), f32_to_bits(o[2]), f32_to_bits(o[3])));
+        store_row<ONCE>(p, make_uint4(f32_to_bits(o[0]), f32_to_bits(o[1]), f32_to_bits(o[2]), f32_to_bits(o[3])));
       } else {
-        store_once(p, make_uint4(pack2<DT>(o[0], o[1]), pack2<DT>(o[2], o[3]), pack2<DT>(o[4], o[5]),
-                                 pack2<DT>(o[6], o[7])));
+        store_row<ONCE>(p, make_uint4(pack2<DT>(o[0], o[1]), pack2<DT>(o[2], o[3]), pack2<DT>(o[4], o[5]),
+                                      pack2<DT>(o[6], o[7])));
       }
     }
   }
