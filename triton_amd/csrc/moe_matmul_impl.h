@@ -521,11 +521,22 @@ TAMD_DEVICE u32x2_t quad_rows(uint32_t rows01, uint32_t rows23, int lane) {
   return up ? u32x2_t{r, b} : u32x2_t{a, r};
 }
 
+// Whole quads of lanes, of NO columns each, inside the output, and whole words.
+template <int NO, typename Args>
+TAMD_DEVICE bool epilogue_stores_quads(const Args &a, int n_out) {
+  return n_out % (4 * NO) == 0 && (((uint32_t)(uintptr_t)a.y | (uint32_t)a.y_stride_m | (uint32_t)a.y_stride_z) & 3u) == 0;
+}
+
 constexpr int kAny16 = 0x100, kAny8 = 0x101;
+// float8_e4m3fn: bounded by flexpoint, without factors, in whole quads (`quads` below), which a layer's rows are: four rows at once without a
+// branch; everything else row by row.  Deciding by branches in one form for all took 1.02 to 1.07 of the time of row by row where a CU has one
+// tile (700 products of 5 to 12 us; the 4-row form was 1.025 with SwiGLU, as it is now 0.98): blocks of four rows whose latencies no
+// other wave hides.  16384 fp8 tokens x 4 of 32, layer 1551 -> 1531 us.
+constexpr int kQuads8 = 0x102, kRows8 = 0x103;
 template <int NFR, int ACT, int YDT, bool ROWSC, bool FLEX, bool MXO, typename Args, typename Pace>
 TAMD_DEVICE void tile_epilogue_t(const Args &a, const Tile &t, f32x16_t (&acc)[NFR][NF], uint8_t *tab, const EpilogueOperands<NFR> *ready,
                                  Pace &pace, bool pairs = true) {
-  constexpr bool BYTES = is_fp8(YDT);
+  constexpr bool BYTES = is_fp8(YDT) || YDT == kQuads8;
   const int wave = (threadIdx.x / kWave) & 3;
   int lane = threadIdx.x % kWave;
   float log2e = 1.4426950408889634f, inf = __builtin_inff();
@@ -536,11 +547,11 @@ TAMD_DEVICE void tile_epilogue_t(const Args &a, const Tile &t, f32x16_t (&acc)[N
   const int N = a.N;
   const int col0 = t.n0 + wave * 64 + c32 * NF;
   constexpr bool ANY = YDT == kAny16 || YDT == kAny8 || YDT == TAMD_F32;   // one width
-  const int ydt = ANY ? a.y_dtype : YDT;
+  const int ydt = ANY ? a.y_dtype : (YDT == kQuads8 || YDT == kRows8 ? TAMD_FP8_E4M3 : YDT);
   constexpr int NO = ACT == TAMD_ACT_SWIGLU ? NF / 2 : NF;  // outputs per lane per row
   const int n_out = ACT == TAMD_ACT_SWIGLU ? N / 2 : N;
   const int out_col0 = ACT == TAMD_ACT_SWIGLU ? col0 / 2 : col0;
-  constexpr int osz = YDT == TAMD_F32 ? 4 : (is_fp8(YDT) || YDT == kAny8 ? 1 : 2);   // bytes per output
+  constexpr int osz = YDT == TAMD_F32 ? 4 : (BYTES || YDT == kRows8 || YDT == kAny8 ? 1 : 2);   // bytes per output
   if (t.n0 + wave * 64 >= N) return;
   uint32_t *tab_dst = (uint32_t *)tab;
   float *tab_beta = (float *)tab + NFR * 32, *tab_gamma = (float *)tab + NFR * 64;
@@ -559,7 +570,7 @@ TAMD_DEVICE void tile_epilogue_t(const Args &a, const Tile &t, f32x16_t (&acc)[N
   const bool has_limit = a.act_has_limit != 0;
   // flexpoint output: scale by 1 / expected, optionally clamp, and track max|result| for the actual scale
   const float inv_expected = (FLEX && a.y_expected_scale) ? 1.0f / *a.y_expected_scale : 1.0f;
-  const bool clamp_out = FLEX && a.y_expected_scale != nullptr && a.y_saturate_inf != 0;
+  const bool clamp_out = YDT == kQuads8 || (FLEX && a.y_expected_scale != nullptr && a.y_saturate_inf != 0);
   const float out_max = max_finite_of(ydt);
   const bool track_max = FLEX && a.y_actual_scale != nullptr;
   const uint32_t track_mask = track_max ? 0x7FFFFFFFu : 0u;
@@ -577,8 +588,7 @@ TAMD_DEVICE void tile_epilogue_t(const Args &a, const Tile &t, f32x16_t (&acc)[N
   const uint32_t col_kill1 = out_col0 + 1 < n_out ? 0u : kDrop;   // (the second output of a pair that N cuts)
   // Bytes: whole quads of lanes inside the output, whole words: one store of four or eight bytes per lane and four rows.  (Of 16 bits the
   // stores are not what a tile waits for: 8 and 16 bytes per lane took 1 to 3 % longer for the exchange between the lanes.)
-  const bool quads = BYTES && n_out % (4 * NO) == 0 &&
-                     (((uint32_t)(uintptr_t)a.y | (uint32_t)a.y_stride_m | (uint32_t)a.y_stride_z) & 3u) == 0;
+  const bool quads = YDT == kQuads8 || (BYTES && epilogue_stores_quads<NO>(a, n_out));
   const bool factors = ROWSC && (a.betas || a.gammas);
   const float act_scale = ACT == TAMD_ACT_SWIGLU ? -a.act_alpha * log2e : 0.f, limit = ACT == TAMD_ACT_SWIGLU ? a.act_limit : 0.f;
   const float limit_lo = __builtin_fminf(-limit, limit);
@@ -636,7 +646,20 @@ TAMD_DEVICE void tile_epilogue_t(const Args &a, const Tile &t, f32x16_t (&acc)[N
         for (int jj = 0; jj < 4; ++jj) {
           float (&o)[NO] = out4[jj];
           result(jj, o);
-          if constexpr (!ANY) {
+          if constexpr (YDT == kRows8) {
+            // (selections, no branches: a branch per element breaks the fragment into hundreds of blocks)
+#pragma unroll
+            for (int p = 0; p < NO; ++p) {
+              const uint32_t b = f32_to_bits(o[p]) & ((dst4[jj] | col_kill) & kDrop ? 0u : track_mask);
+              amax = b > amax ? b : amax;
+              o[p] *= inv_expected;
+              const float oc = __builtin_fminf(__builtin_fmaxf(o[p], -out_max), out_max);
+              o[p] = clamp_out ? oc : o[p];
+            }
+            const int off = (int)((dst4[jj] + col_off) | col_kill);
+            if constexpr (NO == 2) __builtin_amdgcn_raw_buffer_store_b16((uint16_t)(narrow(o[0]) | (narrow(o[NO - 1]) << 8)), ry, off, 0, 0);
+            else __builtin_amdgcn_raw_buffer_store_b8((uint8_t)narrow(o[0]), ry, off, 0, 0);
+          } else if constexpr (!ANY) {
             const int off = (int)((dst4[jj] + col_off) | col_kill);
             if constexpr (NO == 2) __builtin_amdgcn_raw_buffer_store_b32(narrow2(o[0], o[NO - 1]), ry, off, 0, 0);
             else __builtin_amdgcn_raw_buffer_store_b16((uint16_t)narrow(o[0]), ry, off, 0, 0);
@@ -723,7 +746,7 @@ TAMD_DEVICE void tile_epilogue_t(const Args &a, const Tile &t, f32x16_t (&acc)[N
         const uint32_t sdst = tab_dst[NFR * 96 + (i * 4 + jq) * 8 + h * 4 + (c32 & 3)];
         __builtin_amdgcn_raw_buffer_store_b8((uint8_t)se, rsc, (int)(((sdst | sc_off) & kDrop) | (sdst + sc_off)), 0, 0);
       }
-      if constexpr (FLEX) {
+      if constexpr (FLEX && YDT != kRows8) {
         if (ANY || track_max) {
           const uint4 d = DST_AHEAD ? uint4{dst4[0], dst4[1], dst4[2], dst4[3]} : *(const uint4 *)(tab_dst + r0);
           const uint32_t rows[4] = {d.x, d.y, d.z, d.w};
@@ -741,7 +764,7 @@ TAMD_DEVICE void tile_epilogue_t(const Args &a, const Tile &t, f32x16_t (&acc)[N
 #pragma unroll
           for (int p = 0; p < NO; ++p) out4[jj][p] *= inv_expected;
         if (clamp_out) {
-          asm volatile("");
+          if constexpr (YDT != kQuads8) asm volatile("");
 #pragma unroll
           for (int jj = 0; jj < 4; ++jj)
 #pragma unroll
@@ -978,7 +1001,12 @@ TAMD_DEVICE void tile_epilogue(const Args &a, const Tile &t, f32x16_t (&acc)[NFR
   } else if (!spans || a.y_mx_scale) {
     tile_epilogue_general<NFR, ACT, Args>(a, t, acc, tab, pace);
   } else if (FP8_ROWS && pairs && a.y_dtype == TAMD_FP8_E4M3) {
-    if constexpr (FP8_ROWS) tile_epilogue_t<NFR, ACT, TAMD_FP8_E4M3, true, true, false, Args>(a, t, acc, tab, nullptr, pace);
+    if constexpr (FP8_ROWS) {
+      constexpr int NO = ACT == TAMD_ACT_SWIGLU ? NF / 2 : NF;
+      if (a.y_expected_scale && a.y_saturate_inf && !a.betas && !a.gammas && epilogue_stores_quads<NO>(a, ACT == TAMD_ACT_SWIGLU ? a.N / 2 : a.N))
+        tile_epilogue_t<NFR, ACT, kQuads8, false, true, false, Args>(a, t, acc, tab, nullptr, pace);
+      else tile_epilogue_t<NFR, ACT, kRows8, true, true, false, Args>(a, t, acc, tab, nullptr, pace);
+    }
   } else if (pairs && a.y_dtype == FAST_YDT && !flexo) {
     if (a.betas || a.gammas) tile_epilogue_t<NFR, ACT, FAST_YDT, true, false, false, Args>(a, t, acc, tab, nullptr, pace);
     else tile_epilogue_t<NFR, ACT, FAST_YDT, false, false, false, Args>(a, t, acc, tab, nullptr, pace);
