@@ -331,7 +331,7 @@ def run_routing(args, cfg, name):
     out = base_line(args, "moe_routing_tokens_per_s", round(T / (wall * 1e-3), 1), "tokens/s", wall, "f32 logits -> int32",
                     f"{name}: routing (top-{k} of {E} + softmax, histogram, gather / scatter indices, ragged tables), T={T}")
     out["roofline"] = {"bound": "hbm", "achieved": round(gbs, 1), "peak": PEAK_HBM_GBS, "unit": "GB/s",
-                       "frac": round(gbs / PEAK_HBM_GBS, 4), "traffic": None, "kernel": "topk_hist_kernel + order_scan_kernel",
+                       "frac": round(gbs / PEAK_HBM_GBS, 4), "traffic": None, "kernel": "topk_hist_kernel + order_rows_kernel",
                        "kernel_ms": round(kernel_ms, 4), "algorithmic_bytes": alg_bytes,
                        "event_pair_ms": round(event_ms, 4),
                        "note": "2.4 MB in two launches: bound by launch latency, not by HBM; kernel_ms: 16 calls replayed as "

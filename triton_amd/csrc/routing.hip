@@ -814,7 +814,7 @@ TAMD_DEVICE int rows_before(const uint32_t *members, int W, int e, int r) {
 // First launch: the experts of RB rows per workgroup, TH / L at a time, and the bytes of their counts: row `blockIdx.x` of
 // the table, `pitch` bytes.  The workgroups are as small as a short table allows, since a row is a chain of
 // instructions that the waves of a SIMD share.  (Both launches in a graph, with 32-bit tables and a histogram per 64 entries before:
-// 4096 rows of 128, top-4: 12.0 -> 8.5 us; 333 of 32: 9.0 -> 6.8; 9350 of 256, bf16, top-8: 22.8 -> 16.2, four launches
+// 4096 rows of 128, top-4: 12.0 -> 8.3 us; 333 of 32: 9.0 -> 6.8; 9350 of 256, bf16, top-8: 22.8 -> 16.2, four launches
 // before; 32768 of 256, top-8: 52 -> 36.)
 template <int DT, int L, int EPL, int TH>
 __global__ __launch_bounds__(TH) void topk_hist_kernel(const void *__restrict__ x, int64_t x_stride, int n_rows, int E,
@@ -1120,8 +1120,8 @@ __global__ __launch_bounds__(1024) void meta_fused_kernel(const void *__restrict
 // rows as they hold and set the rows' bits per expert (`members`, as above); six waves sum and scan those bits into the
 // ragged tables, each the row of one block size, and write their entries of the block schedule from the scan's registers;
 // then every entry is placed by the lane that picked it.  What such a workgroup is made of is the length of its chains, not its work:
-// with a histogram per 64 entries, prefix sums over them and a search per schedule entry one row of 128 logits took 14 500
-// cycles (6.4 us; 64 rows 9.5), now @@.
+// with a histogram per 64 entries, prefix sums over them and a search per schedule entry one row of 128 logits took 6.4 us
+// (14 500 cycles; 64 rows 9.5), now 3.4 and 5.2.
 template <int DT, int L, int EPL>
 __global__ __launch_bounds__(1024) void routing_fused_kernel(const void *__restrict__ x, int64_t x_stride, int n_rows,
                                                              int E, int k, int W, void *__restrict__ y_vals,
@@ -1412,7 +1412,7 @@ extern "C" int tamd_routing_gates(const void *logits, int dtype, int64_t stride,
     const int L = lanes_per_row(n_cols, k);
     const int64_t n = (int64_t)n_rows * k;
     hipStream_t st = (hipStream_t)stream;
-    // One launch where 1024 threads hold the rows: also at the line it is the faster (64 rows of 128: 5.9 us against 7.5 in
+    // One launch where 1024 threads hold the rows: also at the line it is the faster (64 rows of 128: 5.6 us against 7.5 in
     // two launches, which take 2.8 us longer to launch; 128 of 32: 4.7 and 6.5).
     if (n_rows <= 1024 / L) {
       const int W = (n_rows + 31) / 32;

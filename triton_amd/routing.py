@@ -2,7 +2,8 @@
 tests/test_distributed.py:201-208 (topk -> histogram / ordering -> ragged
 metadata; gather = col_sorted // k, scatter = col_sorted).
 
-One foreign call (`tamd_routing`: one launch at decode sizes, two up to 65535 rows, else four) writes into
+One foreign call (`tamd_routing`: one launch at decode sizes, two up to 65535 rows of up to 512 experts where these fill
+the chip, else the top-k and one to three launches for the metadata) writes into
 one int32 arena that holds every output and the kernels' workspace; its layout is computed once per shape and the
 tensors of the result are views of that arena, built when they are first asked for (the index arrays and ragged tables
 together, in one call): at these sizes the host time of this function is what a step waits for."""
