@@ -651,15 +651,16 @@ __global__ __launch_bounds__(256) void upcast_cols_tile_kernel(
 // Up to how many tiles of 8 groups a tensor whose quantised axis is strided goes to the kernels of one column per thread instead of the tile
 // kernels, given for 256 CUs.  Tiles of 32 groups (float32) and 16 left most of a last round empty on all but the largest tensors: 160
 // of [1 .. 8, 512 .. 2880, 512 .. 5760], time with tiles of 8 over the time before: quantising float32 0.927, bf16 0.911, dequantising to
-// float32 0.87, to bf16 0.855.  If rows start on lines the larger tiles, whose runs are longer, are as fast or faster again from some rounds over
-// the CUs on (kWideFrom*, in quarters): quantising float32 from four (8 x 2880 x 5760: 109.5 us in tiles of 32, 109.8 of 8), 16-bit types
-// from one and a quarter (8 x 2336 x 2688: 29 us, 37 in tiles of 8), dequantising from two and a half (0.94 to 1.0 of the time in tiles
-// of 32 and 16, 1.05 in those of 8).  With the merged halves below, float32 and back to bf16: 8 x 2304 x 3032 55.9 + 43.2 -> 48.9 + 24.1 us,
+// float32 0.87, to bf16 0.855.  If rows start on lines the larger tiles, whose runs are longer, are as fast or faster again above some rounds over
+// the CUs (kWideAbove*, in quarters): quantising float32 and dequantising to 16 bits from four (8 x 2880 x 5760: 109.5 us in tiles of 32,
+// 109.8 of 8), quantising 16-bit types above one and a quarter (8 x 2336 x 2688 29 us, 37 in tiles of 8; 8 x 2400 x 5760 72 and 79, but where the
+// larger ones end in half a round, 8 x 2048 x 5120, 49 and 44), dequantising to float32 above two and a half (0.94 to 1.0 of the time in tiles
+// of 32, 1.05 in those of 8).  With the merged halves below, float32 and back to bf16: 8 x 2304 x 3032 55.9 + 43.2 -> 48.9 + 24.1 us,
 // 8 x 2432 x 1432 39.9 + 23.3 -> 24.5 + 14.7; 200 others 0.86 and 0.82 over the same memory again and again, 0.87 and 0.87 into memory that no cache
 // holds (the worst 1.09 and 1.19).  Just above the lines columns and tiles take about as long: quantising 7.5 us and 7.8 at 130 tiles
 // (float32), 8.6 and 8.7 at 105 (bf16), dequantising 4.9 and 5.7 at 33, 5.3 and 5.6 at 45.
 constexpr int64_t kColumnsUpToDown = 96, kColumnsUpToUp = 40;
-constexpr int kWideFromDown32 = 16, kWideFromDown16 = 5, kWideFromUp = 10;
+constexpr int kWideAboveDown32 = 15, kWideAboveDown16 = 5, kWideAboveUp32 = 10, kWideAboveUp16 = 15;
 // Rows that do not start on a line of 128 bytes: a line that two tiles share is read, or written in part, by both.  Non-temporal loads fetch
 // it from memory for each (plain loads 0.86 to 0.98 of the time); non-temporal stores send it out in halves.  Plain ones let the caches
 // merge these, which pays if they hold the destination's lines from an earlier use: dequantising over the same memory, time with plain
@@ -700,7 +701,7 @@ int launch_downcast(const void *src, int64_t nb, int64_t L, int64_t nr, int64_t 
   if (int rc = cu_count(cus)) return rc;
   if (vec && tiles * 256 > kColumnsUpToDown * cus) {
     const bool lines = aligned(src, 128) && (ssb * ES) % 128 == 0 && (ssl * ES) % 128 == 0;
-    const bool wide = lines && 4 * cols * ((G + WIDE - 1) / WIDE) >= (ES == 4 ? kWideFromDown32 : kWideFromDown16) * (int64_t)cus;
+    const bool wide = lines && 4 * cols * ((G + WIDE - 1) / WIDE) > (ES == 4 ? kWideAboveDown32 : kWideAboveDown16) * (int64_t)cus;
     const int64_t blocks = wide ? cols * ((G + WIDE - 1) / WIDE) : tiles;
     if (blocks > 0x7FFFFFFF) return TAMD_E_UNSUPPORTED;
     auto kern = wide ? downcast_cols_tile_kernel<DT, WIDE, true> : (lines ? downcast_cols_tile_kernel<DT, 8, true> : downcast_cols_tile_kernel<DT, 8, false>);
@@ -742,7 +743,7 @@ int launch_upcast(const uint8_t *vals, int64_t vsb, int64_t vsr, const uint8_t *
   if (int rc = cu_count(cus)) return rc;
   if (vec && tiles * 256 > kColumnsUpToUp * cus) {
     const bool lines = aligned(dst, 128) && (dsb * ES) % 128 == 0 && (dsl * ES) % 128 == 0;
-    const bool wide = lines && 4 * cols * ((G + 15) / 16) >= kWideFromUp * (int64_t)cus;
+    const bool wide = lines && 4 * cols * ((G + 15) / 16) > (ES == 4 ? kWideAboveUp32 : kWideAboveUp16) * (int64_t)cus;
     const int64_t blocks = wide ? cols * ((G + 15) / 16) : tiles;
     if (blocks > 0x7FFFFFFF) return TAMD_E_UNSUPPORTED;
     auto kern = wide ? upcast_cols_tile_kernel<DT, 16, true>
