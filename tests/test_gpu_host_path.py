@@ -340,3 +340,28 @@ def test_native_matmul_fills_in_the_output_block_size(device, monkeypatch):
         return [y, ys]
 
     assert BothPaths(monkeypatch, "matmul")(call)
+
+
+def test_routing_in_threads(device):
+    """Four threads that meet more shapes than are kept, and one that all of them come back to: every call is answered, each with its own tables."""
+    import threading
+    logits = torch.randn(900, 16, generator=torch.Generator().manual_seed(1)).to(device)
+    want = {T: RR.routing_ref(logits[:T].cpu(), 2)["col_sum"] for T in (3, 333)}
+    errors = []
+
+    def work(first):
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                for T in range(first, 900, 4):
+                    r, again = routing(logits[:T], 2), routing(logits[:3], 2)
+                    assert r.col_sum.sum().item() == 2 * T and torch.equal(again.col_sum.cpu(), want[3])
+                assert torch.equal(routing(logits[:333], 2).col_sum.cpu(), want[333])
+        except Exception as e:
+            errors.append(e)
+    torch.cuda.synchronize()
+    threads = [threading.Thread(target=work, args=(i + 1,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors
