@@ -20,7 +20,7 @@
 // kernels do, up to ten stages in the same two sums to the bit, beyond in four, one for each quarter of K, which are those of the narrow
 // tiles to the bit.  Results that are not the 64-bit sum rounded, f16, tiled kernels / one sum / now: 8 slices of 55 rows, 576 -> 2152, of
 // 951184 743 / 761 / 743; 8 of 12, 3784 -> 2560, of 238080 347 / 446 / 347 (narrow tiles); 8 of 60, 2544 -> 1856, of 885312 1406 / 1451 / 1195.  Of 100 products
-// of 3 to 200 rows per slice, K 256 to 5600, 9 of 19 below the line had more than the tiled kernels with one sum, none now.  The second set costs up to 3 %
+// of 3 to 200 rows per slice, K 256 to 5600, 16 of the 19 below the line had more than the tiled kernels with one sum, none now.  The second set costs up to 3 %
 // of a short tile.
 // Blocks of 160 rows, the most that three stages have LDS for (128: 1021 tokens 225, 2000 tokens 357 where 160 take 311; 96: 266 and 393);
 // of 64 where slices are smaller, whose copies of rows that are not there cost 2 to 4 % (300 tokens: 170 -> 165; blocks of 32 with a ring

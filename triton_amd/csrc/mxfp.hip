@@ -652,7 +652,7 @@ __global__ __launch_bounds__(256) void upcast_cols_tile_kernel(
 // kernels, given for 256 CUs.  Tiles of 32 groups (float32) and 16 left most of a last round empty on all but the largest tensors: 160
 // of [1 .. 8, 512 .. 2880, 512 .. 5760], time with tiles of 8 over the time before: quantising float32 0.927, bf16 0.911, dequantising to
 // float32 0.87, to bf16 0.855.  If rows start on lines the larger tiles, whose runs are longer, are as fast or faster again above some rounds over
-// the CUs (kWideAbove*, in quarters): quantising float32 and dequantising to 16 bits from four (8 x 2880 x 5760: 109.5 us in tiles of 32,
+// the CUs (kWideAbove*, in quarters): quantising float32 and dequantising to 16 bits about four (8 x 2880 x 5760: 109.5 us in tiles of 32,
 // 109.8 of 8), quantising 16-bit types above one and a quarter (8 x 2336 x 2688 29 us, 37 in tiles of 8; 8 x 2400 x 5760 72 and 79, but where the
 // larger ones end in half a round, 8 x 2048 x 5120, 49 and 44), dequantising to float32 above two and a half (0.94 to 1.0 of the time in tiles
 // of 32, 1.05 in those of 8).  With the merged halves below, float32 and back to bf16: 8 x 2304 x 3032 55.9 + 43.2 -> 48.9 + 24.1 us,
